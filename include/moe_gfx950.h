@@ -331,6 +331,80 @@ int moe_ffn_forward(const void* x, int x_dtype, const void* logits, int logits_d
                     int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out, int out_dtype,
                     void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Router weight gradient (autograd of the product at mlp.py:100): dw [E,H] = dlogits^T x for bf16
+ * dlogits [T,E] and x [T,H]; E a multiple of 8.  Slices of the tokens are contracted side by side and
+ * their fp32 sums added in a fixed order. */
+int64_t moe_router_wgrad_workspace_bytes(int64_t T, int64_t H, int64_t E);
+int moe_router_wgrad(const uint16_t* dlogits, const uint16_t* x, int64_t T, int64_t H, int64_t E, void* dw,
+                     int dw_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* ---- training: the layer body in one call per direction ---------------------------------
+ * mlp.py:101-167 and its backward with what the backward pass needs kept in buffers of the
+ * caller's: the launches of the entry points above, in their order, enqueued from one call.
+ * The arguments travel in a structure (every member 8 bytes); a pointer documented "or NULL" may
+ * be NULL, and members a call does not use may be 0. */
+typedef struct {
+  int64_t T, H, E, I, k;
+  const void* x;          /* [T,H] rows the experts see */
+  int64_t x_dtype;
+  const void* logits;     /* [T,E], or NULL: ids (and gates) are given */
+  int64_t logits_dtype;
+  const float* bias;      /* [E] or NULL */
+  const int64_t* ids64;   /* without logits: [R] expert ids to be written to `ids` first, or NULL (ids holds them) */
+  const uint16_t *w1, *w3, *w2;
+  const void* residual;   /* [T,H] of out's dtype added to the result, or NULL */
+  void* out;              /* [T,H] */
+  int64_t out_dtype;
+  int32_t* ids;           /* [R]; written from the logits or ids64 */
+  float* gates;           /* [R]; written from the logits; NULL without them: all ones */
+  int32_t *counts, *offs, *pos_to_row, *row_to_pos;
+  int32_t* bad_ids;       /* [1] or NULL */
+  uint16_t* xp;           /* [R,H] kept */
+  void* gu;               /* moe_gu_blocked_bytes(R, E, I) kept, or NULL: g and u are not written */
+  uint16_t* act;          /* [R,I] kept */
+  void* scratch;          /* moe_layer_scratch_bytes(T, H, E, I, k, 0), 256-byte aligned */
+  int64_t scratch_bytes;
+} moe_layer_forward_args;
+
+typedef struct {
+  int64_t T, H, E, I, k;
+  const void* dout;       /* [T,H] */
+  int64_t dout_dtype;
+  const float* gates;     /* as the forward call left them, from here to w2 (bf16) */
+  const int32_t *ids, *offs, *pos_to_row, *row_to_pos;
+  const uint16_t* xp;
+  const void* gu;
+  const uint16_t* act;
+  const uint16_t *w1, *w3, *w2;
+  void* dw[3];            /* gradients of w1, w3, w2; NULL: not wanted */
+  int64_t dw_dtype[3];
+  int64_t dw_accumulate[3];
+  void* dlogits;          /* [T,E] or NULL */
+  int64_t dlogits_dtype;
+  float* dgates;          /* [R] or NULL; if given, the gate gradients are left here and nothing below is done
+                             but dx without the router's share */
+  const uint16_t* wr;     /* [E,H] bf16 if the router product belongs to the layer, else NULL */
+  const uint16_t* xn;     /* [T,H] bf16 rows it read (with dwr) */
+  void* dwr;              /* [E,H] or NULL; not together with dlogits */
+  int64_t dwr_dtype;
+  void* dx;               /* [T,H] or NULL */
+  int64_t dx_dtype;
+  uint16_t* dxp;          /* [R,H] or NULL: where the gradients of the expert-ordered rows are left */
+  void* scratch;          /* moe_layer_scratch_bytes(T, H, E, I, k, 1), 256-byte aligned */
+  int64_t scratch_bytes;
+} moe_layer_backward_args;
+
+int64_t moe_layer_scratch_bytes(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int backward);
+int moe_layer_forward(const moe_layer_forward_args* args, void* stream);
+int moe_layer_backward(const moe_layer_backward_args* args, void* stream);
+
+/* A profiling aid: `fn` is called before (after = 0) and after (1) every launch that the calls which
+ * enqueue several make (these two and moe_ffn_forward), with the name of the entry point that enqueues
+ * it alone.  NULL removes it.  Process-wide, not synchronised. */
+typedef void (*moe_launch_observer_fn)(const char* name, int after);
+void moe_set_launch_observer(moe_launch_observer_fn fn);
+
+
 /* ---- the path in fp32 ---------------------------------------------------------------
  * For a layer that runs without autocast on fp32 tensors: the reference then keeps every
  * step of mlp.py:104-169 in fp32 (the three bmm's of :154-157 included) and so do these

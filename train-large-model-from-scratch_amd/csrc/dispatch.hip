@@ -14,6 +14,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "internal.h"
 
 namespace {
 
@@ -350,12 +351,19 @@ __global__ __launch_bounds__(256) void permute_fwd_scatter_kernel(const XT* __re
 }
 
 // out[t,:] = sum_j gates[t*k+j] * y[row_to_pos[t*k+j],:]  (+ addend[t,:]); fp32, slot order.
-template <typename OT, typename AT>
+// ROUTER: + bf16(sum_j dsel[t*k+j] * wr[ids[t*k+j],:]), the router path's input gradient: a row of
+// dlogits has k nonzero entries, so that product is k rows of the router weight per token, which sit in
+// every XCD's L2 (at most 512 rows) -- instead of a library product over all E columns, its result in
+// memory and another read of it here.
+template <typename OT, typename AT, bool ROUTER>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __restrict__ y,
                                                          const float* __restrict__ gates,
                                                          const int32_t* __restrict__ row_to_pos,
                                                          const AT* __restrict__ addend, int T,
-                                                         int H8, int k, OT* __restrict__ out) {
+                                                         int H8, int k, OT* __restrict__ out,
+                                                         const float* __restrict__ dsel,
+                                                         const int32_t* __restrict__ ids,
+                                                         const uint16_t* __restrict__ wr) {
   const int H = H8 * 8;
   for (long long blk = blockIdx.x; blk * ROWS_PER_BLOCK < T; blk += gridDim.x) {
     const int row0 = (int)(blk * ROWS_PER_BLOCK);
@@ -409,6 +417,19 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
         const Row8 a = load8(addend + (size_t)t * H + col);
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc.v[i] += a.v[i];
+      }
+      if constexpr (ROUTER) {
+        Row8 d2;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) d2.v[i] = 0.f;
+        for (int q = 0; q < k; ++q) {
+          const float ds = dsel[(size_t)t * k + q];
+          const Row8 w = load8(wr + (size_t)ids[(size_t)t * k + q] * H + col);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) d2.v[i] += ds * w.v[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc.v[i] += bf16_to_f32(f32_to_bf16(d2.v[i]));
       }
       store8(out + (size_t)t * H + col, acc);
     }
@@ -731,14 +752,14 @@ static int combine_like(const uint16_t* y, const float* gates, const int32_t* ro
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
   if (out_dtype == MOE_DT_BF16 && addend_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t>), grid, block, 0, s, y, gates, row_to_pos,
-                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (uint16_t*)out);
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false>), grid, block, 0, s, y, gates, row_to_pos,
+                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (uint16_t*)out, nullptr, nullptr, nullptr);
   else if (out_dtype == MOE_DT_F32 && addend_dtype == MOE_DT_F32)
-    hipLaunchKernelGGL((combine_fwd_kernel<float, float>), grid, block, 0, s, y, gates, row_to_pos,
-                       (const float*)addend, (int)T, (int)(H / 8), (int)k, (float*)out);
+    hipLaunchKernelGGL((combine_fwd_kernel<float, float, false>), grid, block, 0, s, y, gates, row_to_pos,
+                       (const float*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
   else if (out_dtype == MOE_DT_F32 && addend_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t>), grid, block, 0, s, y, gates, row_to_pos,
-                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (float*)out);
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false>), grid, block, 0, s, y, gates, row_to_pos,
+                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
   else
     return MOE_ERR_DTYPE;
   return moe_launch_status();
@@ -1019,5 +1040,67 @@ extern "C" int moe_cast_f32_bf16(const float* src, uint16_t* dst, int64_t n, voi
   if (blocks > 256 * 16) blocks = 256 * 16;
   hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, src,
                      dst, n8, (long long)n);
+  return moe_launch_status();
+}
+
+int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const float* dsel, const int32_t* ids,
+                           const uint16_t* wr, int64_t T, int64_t H, int64_t k, void* dx, int dx_dtype,
+                           hipStream_t s) {
+  const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
+  if (dx_dtype == MOE_DT_BF16)
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, true>), grid, block, 0, s, dxp, nullptr, row_to_pos,
+                       nullptr, (int)T, (int)(H / 8), (int)k, (uint16_t*)dx, dsel, ids, wr);
+  else
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, true>), grid, block, 0, s, dxp, nullptr, row_to_pos,
+                       nullptr, (int)T, (int)(H / 8), (int)k, (float*)dx, dsel, ids, wr);
+  return moe_launch_status();
+}
+
+namespace {
+
+// 8 elements per thread; the slices of an element are read a fixed ascending order: reproducible
+template <typename OutT>
+__global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, int slices,
+                                                        long long stride8, long long n8,
+                                                        OutT* __restrict__ dw) {
+  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (i >= n8) return;
+  Row8 acc;
+#pragma unroll
+  for (int v = 0; v < 8; ++v) acc.v[v] = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < slices; ++s) {
+    const Row8 r = load8(part + (s * stride8 + i) * 8);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) acc.v[v] += r.v[v];
+  }
+  store8(dw + i * 8, acc);
+}
+
+__global__ __launch_bounds__(256) void narrow_ids_kernel(const int64_t* __restrict__ ids, int R,
+                                                        int32_t* __restrict__ out) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= R) return;
+  const int64_t v = ids[r];
+  out[r] = (v < 0 || v > 0x7fffffffll) ? -1 : (int32_t)v;
+}
+
+}  // namespace
+
+int moe_sum_slices(const float* part, int64_t slices, int64_t Mp, int64_t M, int64_t N, void* dw, int dw_dtype,
+                   hipStream_t s) {
+  const long long n8 = M * N / 8;
+  const dim3 grid((unsigned)((n8 + 255) / 256)), block(256);
+  if (dw_dtype == MOE_DT_F32)
+    hipLaunchKernelGGL(sum_slices_kernel<float>, grid, block, 0, s, part, (int)slices, (long long)(Mp * N / 8), n8,
+                       (float*)dw);
+  else
+    hipLaunchKernelGGL(sum_slices_kernel<uint16_t>, grid, block, 0, s, part, (int)slices, (long long)(Mp * N / 8), n8,
+                       (uint16_t*)dw);
+  return moe_launch_status();
+}
+
+int moe_narrow_ids(const int64_t* ids, int64_t R, int32_t* out, hipStream_t s) {
+  hipLaunchKernelGGL(narrow_ids_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, s, ids, (int)R, out);
   return moe_launch_status();
 }

@@ -29,6 +29,7 @@
 // Workgroups are numbered so that each XCD (own L2) works on a contiguous range of tiles,
 // i.e. on its own experts' weights.
 #include "common.h"
+#include "internal.h"
 
 namespace {
 
@@ -56,6 +57,7 @@ struct GemmArgs {
   int ld_a;     // row stride of A0/A1 in elements when it is not the contraction length (0: K)
   int ld_c;     // row stride of the outputs C0/C1 in elements when it is not N (0: N)
   int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
+  int slice;    // WGRAD without offsets: "expert" e is rows e*slice .. (e+1)*slice of the R rows; 0: offs
 };
 
 template <int BM_, int BN_, int BK_, int WM_, int WN_>
@@ -292,7 +294,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
       lo = x * wgs;
       t_hi = p.E * TP;
       t_step = nb;
-      if (p.E <= MOE_WAVE && TP % wgs == 0 && p.E * (TP / wgs) <= MAX_GROUPS) {
+      if (!p.slice && p.E <= MOE_WAVE && TP % wgs == 0 && p.E * (TP / wgs) <= MAX_GROUPS) {
         if (threadIdx.x < MOE_WAVE) {
           const int gpe = TP / wgs;  // groups per expert
           constexpr long long FIXED = 4 * BK;  // fill, tile switch and epilogue, in rows' worth
@@ -383,8 +385,13 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
     if constexpr (MODE == WGRAD) {
       t.e = slot / p.m_slots;
       t.m0 = (slot % p.m_slots) * BM;
-      t.row0 = p.offs[t.e];
-      t.row_end = p.offs[t.e + 1];
+      if (p.slice) {
+        t.row0 = t.e * p.slice;
+        t.row_end = t.row0 + p.slice < p.R ? t.row0 + p.slice : p.R;
+      } else {
+        t.row0 = p.offs[t.e];
+        t.row_end = p.offs[t.e + 1];
+      }
     } else {
       if (slot >= tile_start[p.E]) return false;
       int lo = 0, hi = p.E;  // largest e with tile_start[e] <= slot (skips empty experts)
@@ -1037,7 +1044,9 @@ using CfgMain = TileCfg<MOE_BM, MOE_BN, MOE_BK, MOE_WM, MOE_WN>;
 // large tile's cost, spread such a launch over twice the compute units.
 using CfgSmall = TileCfg<MOE_BM / 2, MOE_BN, MOE_BK, MOE_WM, MOE_WN>;
 
-int compute_units() {
+}  // namespace
+
+int moe_compute_units() {
   static int cus[MOE_MAX_DEVICES];  // per GPU; 0 = not asked yet
   const int dev = moe_current_device();
   if (cus[dev] == 0) {
@@ -1047,6 +1056,9 @@ int compute_units() {
   }
   return cus[dev];
 }
+
+namespace {
+
 
 // `ntiles` is the number of tile slots; the grid is as many workgroups as are resident at
 // once (one or two per compute unit, by LDS footprint), or fewer when there are fewer tiles.
@@ -1063,7 +1075,7 @@ int launch(const GemmArgs& a, long long ntiles, hipStream_t s) {
     attr_done[dev] = true;
   }
   // as many workgroups as can be resident at once: the LDS footprint decides how many share a CU
-  const long long slots = (long long)compute_units() * ((160 * 1024) / LDS >= Cfg::WGS_PER_CU ? Cfg::WGS_PER_CU : 1);
+  const long long slots = (long long)moe_compute_units() * ((160 * 1024) / LDS >= Cfg::WGS_PER_CU ? Cfg::WGS_PER_CU : 1);
   const unsigned grid = (unsigned)(ntiles < slots ? ntiles : slots);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(Cfg::NT), LDS, s, a);
   return moe_launch_status();
@@ -1095,7 +1107,7 @@ int forced_row_tile = 0;
 bool small_row_tiles(int64_t R, int64_t E, int64_t cols) {
   if (forced_row_tile) return forced_row_tile == CfgSmall::BM;
   const int64_t tiles = (int64_t)row_slots<CfgMain>(R, E) * ((cols + CfgMain::BN - 1) / CfgMain::BN);
-  return 2 * tiles < (int64_t)compute_units();
+  return 2 * tiles < (int64_t)moe_compute_units();
 }
 template <typename F>
 int with_row_tile(bool small, F&& f) {
@@ -1314,4 +1326,15 @@ extern "C" int moe_gemm_wgrad(const uint16_t* a_, const uint16_t* b_, const int3
   if (dw_dtype == MOE_DT_F32)
     return launch<WGRAD, Cfg, float>(a, nblocks, (hipStream_t)stream);
   return launch<WGRAD, Cfg, uint16_t>(a, nblocks, (hipStream_t)stream);
+}
+
+int moe_wgrad_slices(const uint16_t* a_, const uint16_t* b_, int64_t T, int64_t M, int64_t N, int64_t slices,
+                     int64_t slice_rows, float* part, hipStream_t s) {
+  using Cfg = CfgMain;
+  GemmArgs a{};
+  a.A0 = a_; a.B0 = b_; a.C0 = part; a.slice = (int)slice_rows;
+  a.E = (int)slices; a.R = (int)T; a.M = (int)M; a.N = (int)N;
+  a.n_tiles = (int)((N + Cfg::BN - 1) / Cfg::BN);
+  a.m_slots = (int)((M + Cfg::BM - 1) / Cfg::BM);
+  return launch<WGRAD, Cfg, float>(a, (long long)a.n_tiles * a.m_slots * slices, s);
 }

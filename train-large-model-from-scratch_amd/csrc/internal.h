@@ -1,0 +1,32 @@
+// Launchers the library's own files share (the C ABI is in include/moe_gfx950.h).  Arguments are
+// checked by the entry points that reach them.
+#pragma once
+#include "common.h"
+
+// Compute units of the current GPU (asked of the runtime once).
+int moe_compute_units();
+
+// part[s] = a[rows of slice s]^T b[rows of slice s], fp32 [slices][M][N]: a [T,M], b [T,N] bf16, slice s
+// = rows s*slice_rows .. of T (gemm.hip).
+int moe_wgrad_slices(const uint16_t* a, const uint16_t* b, int64_t T, int64_t M, int64_t N, int64_t slices,
+                     int64_t slice_rows, float* part, hipStream_t s);
+
+// dw[m][n] = sum over s, ascending, of part[s][m][n] for m < M; part has Mp >= M rows per slice (dispatch.hip).
+int moe_sum_slices(const float* part, int64_t slices, int64_t Mp, int64_t M, int64_t N, void* dw, int dw_dtype,
+                   hipStream_t s);
+
+// Gate gradients from the dgrad-down kernel's block sums, softmax Jacobian and scatter to the logits in
+// one kernel (route.hip).  dlogits [T, ld] with columns E..ld-1 zero; dsel fp32 [T*k] (may be NULL): the k
+// nonzero entries per token, rounded to dlogits' type.
+int moe_router_bwd_from_blocks(const float* part, int64_t P, const float* gates, const int32_t* ids,
+                               const int32_t* row_to_pos, int64_t T, int64_t E, int64_t k, int64_t ld,
+                               void* dlogits, int dlogits_dtype, float* dsel, hipStream_t s);
+
+// moe_permute_bwd with the router path's input gradient in the same pass: dx[t] = sum_j dxp[pos(t,j)]
+// + bf16(sum_j dsel[t,j] * wr[ids[t,j]]) (dispatch.hip).
+int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const float* dsel, const int32_t* ids,
+                           const uint16_t* wr, int64_t T, int64_t H, int64_t k, void* dx, int dx_dtype,
+                           hipStream_t s);
+
+// int64 expert ids to int32, values outside int32 to -1 (dispatch.hip).
+int moe_narrow_ids(const int64_t* ids, int64_t R, int32_t* out, hipStream_t s);

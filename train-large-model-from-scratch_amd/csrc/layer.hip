@@ -1,13 +1,32 @@
-// The whole forward pass of the layer body behind one call: routing, dispatch, row gather, the two
+// The layer body behind single calls.
+//
+// Forward only: the whole pass behind one call: routing, dispatch, row gather, the two
 // grouped GEMMs and the combine (model/modules/mlp.py:101-167) enqueued back to back on the
 // caller's stream, with every intermediate in a workspace the caller provides.  For callers that
 // only want the output (inference, evaluation, a forward under no_grad): one crossing of the FFI
 // boundary and two buffers instead of six crossings and a dozen.  Nothing here touches the GPU
 // itself: the kernels are the ones the separate entry points launch, in the same order, so the
 // output holds the same bits.
+//
+// Training: moe_layer_forward / moe_layer_backward enqueue one direction each (two dozen kernels
+// between them).  What they replace is host work: a step of 512 tokens of a narrow layer has 0.1 ms of
+// kernels, and took the host 0.42 ms when every launch was its own call from Python with its own
+// allocations.
 #include "common.h"
+#include "internal.h"
 
 namespace {
+
+moe_launch_observer_fn g_observer = nullptr;
+
+// Enqueues one step and tells the observer about it; leaves the calling function on an error.
+#define MOE_STEP(name, call)              \
+  do {                                    \
+    if (g_observer) g_observer(name, 0);  \
+    const int rc_ = (call);               \
+    if (g_observer) g_observer(name, 1);  \
+    if (rc_) return rc_;                  \
+  } while (0)
 
 constexpr int64_t ALIGN = 256;
 int64_t up(int64_t n) { return (n + ALIGN - 1) / ALIGN * ALIGN; }
@@ -81,17 +100,306 @@ extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, i
   uint16_t* xp = (uint16_t*)(ws + c.xp);
   uint16_t* act = (uint16_t*)(ws + c.act);
   uint16_t* y = (uint16_t*)(ws + c.y);
-  int rc = moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream);
-  if (rc) return rc;
-  rc = moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
-                          moe_dispatch_workspace_bytes(R, E), stream);
-  if (rc) return rc;
-  rc = k > 1 ? moe_permute_fwd_scatter(x, x_dtype, row_to_pos, T, H, k, xp, stream)
-             : moe_permute_fwd(x, x_dtype, pos_to_row, R, H, k, xp, stream);
-  if (rc) return rc;
-  rc = moe_gemm_gateup_swiglu_fwd(xp, w1, w3, offs, E, R, H, I, nullptr, nullptr, act, stream);
-  if (rc) return rc;
-  rc = moe_gemm_down_fwd(act, w2, offs, E, R, H, I, y, stream);
-  if (rc) return rc;
-  return moe_combine_fwd(y, gates, row_to_pos, T, H, k, out, out_dtype, stream);
+  MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream));
+  MOE_STEP("moe_histogram_scan_checked",
+           moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
+                              moe_dispatch_workspace_bytes(R, E), stream));
+  MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
+           k > 1 ? moe_permute_fwd_scatter(x, x_dtype, row_to_pos, T, H, k, xp, stream)
+                 : moe_permute_fwd(x, x_dtype, pos_to_row, R, H, k, xp, stream));
+  MOE_STEP("moe_gemm_gateup_swiglu_fwd",
+           moe_gemm_gateup_swiglu_fwd(xp, w1, w3, offs, E, R, H, I, nullptr, nullptr, act, stream));
+  MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_fwd(act, w2, offs, E, R, H, I, y, stream));
+  MOE_STEP("moe_combine_fwd", moe_combine_fwd(y, gates, row_to_pos, T, H, k, out, out_dtype, stream));
+  return 0;
+}
+
+extern "C" void moe_set_launch_observer(moe_launch_observer_fn fn) { g_observer = fn; }
+
+// ---- training: one call per direction -------------------------------------------------------------
+
+namespace {
+
+struct Scratch {
+  char* base;
+  int64_t at, have;
+  void* take(int64_t bytes) {
+    void* p = base ? base + at : nullptr;
+    at += up(bytes > 0 ? bytes : 1);
+    return p;
+  }
+  bool fits() const { return at <= have; }
+};
+
+struct FwdScratch {
+  uint16_t* y;
+  void* dispatch;
+  FwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t k) {
+    y = (uint16_t*)s.take(T * k * H * 2);
+    dispatch = s.take(moe_dispatch_workspace_bytes(T * k, E));
+  }
+};
+
+// Weight gradients of one stack: how the contraction over an expert's rows is cut.  The kernel makes
+// one workgroup per 256 x 256 tile of the result and expert; with few experts and small matrices that
+// is a fraction of the chip, and under skewed routing the tiles of the largest expert set the time.
+// Below half a round of the compute units every expert is cut into ceil(n_e / L) equal segments, L such
+// that the (ceil(R/L) + E) x tiles jobs about fill the chip once (at most 1024 segments); their fp32
+// partial sums are added per expert in a fixed order.  Decided from shapes alone: no look at the counts.
+constexpr int64_t WTILE = 256;
+struct Segments {
+  int64_t L = 0, S_max = 0;
+};
+Segments wgrad_segments(int64_t E, int64_t M, int64_t N, int64_t R) {
+  Segments g;
+  const int64_t cus = moe_compute_units();
+  const int64_t tiles = ((M + WTILE - 1) / WTILE) * ((N + WTILE - 1) / WTILE);
+  if (R == 0 || cus / (E * tiles) < 2) return g;
+  const int64_t free_cus = cus - E * tiles > tiles ? cus - E * tiles : tiles;
+  int64_t L = (R * tiles + free_cus - 1) / free_cus;
+  L = (L + 63) / 64 * 64;
+  if (L < 256) L = 256;
+  while ((R + L - 1) / L + E > 1024) L *= 2;
+  g.L = L;
+  g.S_max = moe_segments_by_length_max(R, E, L);
+  return g;
+}
+
+// Router weight gradient: slices of the tokens play the experts of the weight-gradient kernel; as many as
+// give every compute unit a job, of at least 64 tokens, at most 32 (their partial sums are written and
+// read once more).
+struct RouterSlices {
+  int64_t slices, rows, Ep;
+};
+RouterSlices router_slices(int64_t T, int64_t H, int64_t E) {
+  const int64_t tiles = (H + WTILE - 1) / WTILE;
+  int64_t S = moe_compute_units() / tiles;
+  if (S > 32) S = 32;
+  if (S > (T + 63) / 64) S = (T + 63) / 64;
+  if (S < 1) S = 1;
+  RouterSlices r;
+  r.rows = T > 0 ? ((T + S - 1) / S + 63) / 64 * 64 : 64;
+  r.slices = T > 0 ? (T + r.rows - 1) / r.rows : 1;
+  r.Ep = (E + 7) / 8 * 8;
+  return r;
+}
+
+struct BwdScratch {
+  uint16_t *dyp, *dg, *dxp;
+  float *part, *dsel, *wpart, *rpart;
+  uint16_t* dlogits;
+  int32_t *seg, *seg_start;
+  BwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
+    const int64_t R = T * k;
+    dyp = (uint16_t*)s.take(R * H * 2);
+    dg = (uint16_t*)s.take(R * I * 4);
+    dxp = (uint16_t*)s.take(R * H * 2);
+    part = (float*)s.take(moe_dgate_blocks(I) * R * 4);
+    dsel = (float*)s.take(R * 4);
+    const RouterSlices rs = router_slices(T, H, E);
+    dlogits = (uint16_t*)s.take(T * rs.Ep * 4);
+    rpart = (float*)s.take(rs.slices * rs.Ep * H * 4);
+    const Segments g = wgrad_segments(E, I, H, R);
+    seg = (int32_t*)s.take((g.S_max + 1) * 4);
+    seg_start = (int32_t*)s.take((E + 1) * 4);
+    wpart = (float*)s.take(g.L ? g.S_max * I * H * 4 : 0);
+  }
+};
+
+bool dtype_ok(int64_t d) { return d == MOE_DT_BF16 || d == MOE_DT_F32; }
+
+}  // namespace
+
+extern "C" int64_t moe_router_wgrad_workspace_bytes(int64_t T, int64_t H, int64_t E) {
+  if (T < 0 || H <= 0 || E <= 0 || T > (int64_t)1 << 30 || H > 65536 || E > MOE_MAX_EXPERTS) return 0;
+  const RouterSlices r = router_slices(T, H, E);
+  return r.slices * r.Ep * H * 4;
+}
+
+extern "C" int moe_router_wgrad(const uint16_t* dlogits, const uint16_t* x, int64_t T, int64_t H, int64_t E,
+                                void* dw, int dw_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (T < 0 || H <= 0 || E <= 0 || H % 8 != 0 || E % 8 != 0) return MOE_ERR_SHAPE;
+  if (T > (int64_t)1 << 30 || H > 65536 || E > MOE_MAX_EXPERTS) return MOE_ERR_LIMIT;
+  if (!dtype_ok(dw_dtype)) return MOE_ERR_DTYPE;
+  MOE_CHECK_PTR(dw);
+  MOE_CHECK_PTR(workspace);
+  MOE_CHECK_PTR(dlogits);
+  MOE_CHECK_PTR(x);
+  if (workspace_bytes < moe_router_wgrad_workspace_bytes(T, H, E)) return MOE_ERR_WORKSPACE;
+  const RouterSlices r = router_slices(T, H, E);
+  if (int rc = moe_wgrad_slices(dlogits, x, T, E, H, r.slices, r.rows, (float*)workspace, (hipStream_t)stream)) return rc;
+  return moe_sum_slices((const float*)workspace, r.slices, E, E, H, dw, dw_dtype, (hipStream_t)stream);
+}
+
+extern "C" int64_t moe_layer_scratch_bytes(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int backward) {
+  if (!sizes_ok(T, H, E, I, k)) return 0;
+  Scratch s{nullptr, 0, 0};
+  if (backward) BwdScratch(s, T, H, E, I, k);
+  else FwdScratch(s, T, H, E, k);
+  return s.at;
+}
+
+extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) {
+  if (!a) return MOE_ERR_NULL;
+  const int64_t T = a->T, H = a->H, E = a->E, I = a->I, k = a->k, R = T * k;
+  if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
+  if (!sizes_ok(T, H, E, I, k)) return MOE_ERR_LIMIT;
+  if (!dtype_ok(a->x_dtype) || !dtype_ok(a->out_dtype) || (a->logits && !dtype_ok(a->logits_dtype)))
+    return MOE_ERR_DTYPE;
+  MOE_CHECK_PTR(a->counts);
+  MOE_CHECK_PTR(a->offs);
+  MOE_CHECK_PTR(a->scratch);
+  if (T > 0) {
+    MOE_CHECK_PTR(a->x);
+    MOE_CHECK_PTR(a->w1);
+    MOE_CHECK_PTR(a->w3);
+    MOE_CHECK_PTR(a->w2);
+    MOE_CHECK_PTR(a->out);
+    MOE_CHECK_PTR(a->ids);
+    MOE_CHECK_PTR(a->pos_to_row);
+    MOE_CHECK_PTR(a->row_to_pos);
+    MOE_CHECK_PTR(a->xp);
+    MOE_CHECK_PTR(a->act);
+  }
+  if (a->logits && !a->gates) return MOE_ERR_NULL;
+  Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
+  const FwdScratch ws(s, T, H, E, k);
+  if (!s.fits()) return MOE_ERR_WORKSPACE;
+  if (a->logits)
+    MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids,
+                                                        a->gates, stream));
+  else if (a->ids64 && R > 0)
+    MOE_STEP("moe_narrow_ids", moe_narrow_ids(a->ids64, R, a->ids, (hipStream_t)stream));
+  MOE_STEP("moe_histogram_scan_checked",
+           moe_histogram_scan_checked(a->ids, R, E, a->counts, a->offs, a->pos_to_row, a->row_to_pos, a->bad_ids,
+                                      ws.dispatch, moe_dispatch_workspace_bytes(R, E), stream));
+  if (T == 0) return 0;
+  MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
+           k > 1 ? moe_permute_fwd_scatter(a->x, (int)a->x_dtype, a->row_to_pos, T, H, k, a->xp, stream)
+                 : moe_permute_fwd(a->x, (int)a->x_dtype, a->pos_to_row, R, H, k, a->xp, stream));
+  if (a->gu)
+    MOE_STEP("moe_gemm_gateup_swiglu_fwd_blocked",
+             moe_gemm_gateup_swiglu_fwd_blocked(a->xp, a->w1, a->w3, a->offs, E, R, H, I, a->gu, a->act, stream));
+  else
+    MOE_STEP("moe_gemm_gateup_swiglu_fwd",
+             moe_gemm_gateup_swiglu_fwd(a->xp, a->w1, a->w3, a->offs, E, R, H, I, nullptr, nullptr, a->act, stream));
+  MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_fwd(a->act, a->w2, a->offs, E, R, H, I, ws.y, stream));
+  if (a->residual)
+    MOE_STEP("moe_combine_fwd_residual",
+             moe_combine_fwd_residual(ws.y, a->gates, a->row_to_pos, a->residual, T, H, k, a->out,
+                                      (int)a->out_dtype, stream));
+  else
+    MOE_STEP("moe_combine_fwd", moe_combine_fwd(ws.y, a->gates, a->row_to_pos, T, H, k, a->out, (int)a->out_dtype,
+                                                stream));
+  return 0;
+}
+
+extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream) {
+  if (!a) return MOE_ERR_NULL;
+  const int64_t T = a->T, H = a->H, E = a->E, I = a->I, k = a->k, R = T * k;
+  if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
+  if (!sizes_ok(T, H, E, I, k)) return MOE_ERR_LIMIT;
+  if (!dtype_ok(a->dout_dtype) || !dtype_ok(a->dx_dtype) || !dtype_ok(a->dlogits_dtype) || !dtype_ok(a->dwr_dtype))
+    return MOE_ERR_DTYPE;
+  for (int i = 0; i < 3; ++i)
+    if (!dtype_ok(a->dw_dtype[i])) return MOE_ERR_DTYPE;
+  MOE_CHECK_PTR(a->offs);
+  MOE_CHECK_PTR(a->scratch);
+  const bool router = a->wr != nullptr;                               // the router product is part of the layer
+  const bool to_logits = !a->dgates && (a->dlogits || router);        // ... and the gradient goes through it here
+  if (T > 0) {
+    MOE_CHECK_PTR(a->dout);
+    MOE_CHECK_PTR(a->pos_to_row);
+    MOE_CHECK_PTR(a->row_to_pos);
+    MOE_CHECK_PTR(a->xp);
+    MOE_CHECK_PTR(a->gu);
+    MOE_CHECK_PTR(a->act);
+    MOE_CHECK_PTR(a->w1);
+    MOE_CHECK_PTR(a->w3);
+    MOE_CHECK_PTR(a->w2);
+    if ((to_logits || a->dgates) && (!a->gates || !a->ids)) return MOE_ERR_NULL;
+    if (a->dwr && (!router || !a->xn)) return MOE_ERR_NULL;
+  }
+  Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
+  const BwdScratch ws(s, T, H, E, I, k);
+  if (!s.fits()) return MOE_ERR_WORKSPACE;
+  hipStream_t st = (hipStream_t)stream;
+  uint16_t* dxp = a->dxp ? a->dxp : ws.dxp;
+  if (R > 0) {
+    if (k > 1 && H <= 2048)
+      MOE_STEP("moe_combine_bwd_by_token", moe_combine_bwd_by_token(a->dout, (int)a->dout_dtype, nullptr, a->gates,
+                                                                    a->row_to_pos, T, H, k, ws.dyp, nullptr, stream));
+    else
+      MOE_STEP("moe_combine_bwd", moe_combine_bwd(a->dout, (int)a->dout_dtype, nullptr, a->gates, a->pos_to_row, R, H,
+                                                  k, ws.dyp, nullptr, stream));
+  }
+  const Segments g = wgrad_segments(E, I, H, R);
+  // dg and du side by side where their two weight gradients can come out of one launch: both wanted into
+  // results of one kind, no 256-row tile of the stacked result across the halves, no row segments
+  const bool pair = R > 0 && a->dw[0] && a->dw[1] && I % WTILE == 0 && !g.L && a->dw_dtype[0] == a->dw_dtype[1] &&
+                    a->dw_accumulate[0] == a->dw_accumulate[1];
+  uint16_t* dg = ws.dg;
+  uint16_t* du = pair ? ws.dg + I : ws.dg + R * I;
+  float* part = (to_logits || a->dgates) ? ws.part : nullptr;
+  MOE_STEP("moe_gemm_dgrad_down_swiglu_bwd_blocked",
+           moe_gemm_dgrad_down_swiglu_bwd_blocked(ws.dyp, a->w2, a->gu, a->offs, E, R, H, I, dg, du, pair ? 2 * I : 0,
+                                                  part, stream));
+  if (a->dx || a->dxp) {
+    if (pair)
+      MOE_STEP("moe_gemm_dgrad_gateup_packed",
+               moe_gemm_dgrad_gateup_packed(dg, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
+    else
+      MOE_STEP("moe_gemm_dgrad_gateup", moe_gemm_dgrad_gateup(dg, du, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
+  }
+  // weight gradients, down projection first: [dyp | act], [dg | xp], [du | xp]
+  if (g.L && (a->dw[0] || a->dw[1] || a->dw[2]))
+    MOE_STEP("moe_segment_offsets_by_length",
+             moe_segment_offsets_by_length(a->offs, E, g.L, g.S_max, ws.seg, ws.seg_start, stream));
+  const int order[3] = {2, 0, 1};
+  for (int n = 0; n < 3; ++n) {
+    const int w = order[n];
+    if (!a->dw[w]) continue;
+    if (pair && w == 1) continue;  // came with the gate stack's
+    const uint16_t* lhs = w == 2 ? ws.dyp : w == 0 ? dg : du;
+    const uint16_t* rhs = w == 2 ? a->act : a->xp;
+    const int64_t M = w == 2 ? H : I, N = w == 2 ? I : H;
+    const int dt = (int)a->dw_dtype[w], acc = a->dw_accumulate[w] ? 1 : 0;
+    if (pair && w == 0) {
+      MOE_STEP("moe_gemm_wgrad_pair",
+               moe_gemm_wgrad_pair(dg, a->xp, a->offs, E, R, I, H, a->dw[0], a->dw[1], dt, acc, stream));
+    } else if (g.L) {
+      MOE_STEP("moe_gemm_wgrad", moe_gemm_wgrad(lhs, rhs, ws.seg, g.S_max, R, M, N, ws.wpart, MOE_DT_F32, 0, stream));
+      MOE_STEP("moe_wgrad_reduce_segments",
+               moe_wgrad_reduce_segments(ws.wpart, ws.seg_start, E, M, N, a->dw[w], dt, acc, stream));
+    } else {
+      MOE_STEP("moe_gemm_wgrad", moe_gemm_wgrad(lhs, rhs, a->offs, E, R, M, N, a->dw[w], dt, acc, stream));
+    }
+  }
+  if (a->dgates && R > 0)
+    MOE_STEP("moe_dgates_from_blocks_by_pos", moe_dgates_from_blocks_by_pos(part, moe_dgate_blocks(I), a->gates,
+                                                                            a->pos_to_row, R, a->dgates, stream));
+  const RouterSlices rs = router_slices(T, H, E);
+  if (to_logits && R > 0) {
+    // (for the router's weight gradient the rows of dlogits are padded to a multiple of 8 columns)
+    const bool own = !a->dlogits;
+    MOE_STEP("moe_router_bwd_from_blocks",
+             moe_router_bwd_from_blocks(part, moe_dgate_blocks(I), a->gates, a->ids, a->row_to_pos, T, E, k,
+                                        own ? rs.Ep : E, own ? ws.dlogits : a->dlogits,
+                                        own ? MOE_DT_BF16 : (int)a->dlogits_dtype, router ? ws.dsel : nullptr, st));
+  }
+  if (router && to_logits && a->dwr) {
+    if (a->dlogits) return MOE_ERR_SHAPE;  // one or the other: the caller's dlogits are not padded
+    MOE_STEP("moe_wgrad_slices",
+             moe_wgrad_slices(ws.dlogits, a->xn, T, rs.Ep, H, rs.slices, rs.rows, ws.rpart, st));
+    MOE_STEP("moe_sum_slices", moe_sum_slices(ws.rpart, rs.slices, rs.Ep, E, H, a->dwr, (int)a->dwr_dtype, st));
+  }
+  if (a->dx && T > 0) {
+    if (router && to_logits)
+      MOE_STEP("moe_permute_bwd_router",
+               moe_permute_bwd_router(dxp, a->row_to_pos, ws.dsel, a->ids, a->wr, T, H, k, a->dx, (int)a->dx_dtype, st));
+    else
+      MOE_STEP("moe_permute_bwd",
+               moe_permute_bwd(dxp, a->row_to_pos, nullptr, T, H, k, a->dx, (int)a->dx_dtype, stream));
+  }
+  return 0;
 }

@@ -5,6 +5,7 @@
 // max-reduction over 64-bit keys, and the softmax over the k winners is a wave reduction.
 // HBM-bound: reads T*E logits, writes T*k ids and gates.
 #include "common.h"
+#include "internal.h"
 #include "topk_core.h"
 
 namespace {
@@ -78,6 +79,57 @@ __global__ __launch_bounds__(256) void router_topk_bwd_kernel(const float* __res
   }
 }
 
+// The router's backward from the block sums the dgrad-down kernel leaves (part [P][R], by position:
+// gate * <dy, y> split over 64-column blocks): gate gradient, softmax Jacobian over the k winners and the
+// row of dlogits in one kernel, TB tokens per block.  The block sums of a row are gathered (P reads of
+// 4 bytes at the row's position: they were written just before and come from L2), everything after
+// that stays in LDS.  Same arithmetic as moe_dgates_from_blocks + moe_router_topk_bwd up to the order
+// of the k-term sum (ascending here).
+constexpr int RB_PAIRS = 512;  // (token, slot) pairs per block at most
+template <typename DT>
+__global__ __launch_bounds__(256) void router_bwd_from_blocks_kernel(
+    const float* __restrict__ part, int P, const float* __restrict__ gates, const int32_t* __restrict__ ids,
+    const int32_t* __restrict__ row_to_pos, int T, int E, int k, int TB, int ld, DT* __restrict__ dlogits,
+    float* __restrict__ dsel_out) {
+  __shared__ float sg[RB_PAIRS], sdg[RB_PAIRS], ssel[RB_PAIRS];
+  __shared__ int sid[RB_PAIRS];
+  const int t0 = blockIdx.x * TB, nt = T - t0 < TB ? T - t0 : TB, n = nt * k;
+  const size_t R = (size_t)T * k, r0 = (size_t)t0 * k;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const float* src = part + row_to_pos[r0 + i];
+    float s = 0.f;
+    int b = 0;
+    for (; b + 4 <= P; b += 4) {  // (four gathers in flight, added in ascending order)
+      const float v0 = src[(size_t)b * R], v1 = src[(size_t)(b + 1) * R], v2 = src[(size_t)(b + 2) * R],
+                  v3 = src[(size_t)(b + 3) * R];
+      s = (((s + v0) + v1) + v2) + v3;
+    }
+    for (; b < P; ++b) s += src[(size_t)b * R];
+    const float g = gates[r0 + i];
+    sg[i] = g;
+    sdg[i] = g != 0.f ? s / g : 0.f;
+    sid[i] = ids[r0 + i];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const int first = i / k * k;
+    float dot = 0.f;
+    for (int j = 0; j < k; ++j) dot += sg[first + j] * sdg[first + j];
+    float v = sg[i] * (sdg[i] - dot);
+    if constexpr (sizeof(DT) == 2) v = bf16_to_f32(f32_to_bf16(v));
+    ssel[i] = v;
+    if (dsel_out) dsel_out[r0 + i] = v;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < nt * ld; i += blockDim.x) {
+    const int t = i / ld, e = i - t * ld;
+    float v = 0.f;
+    for (int j = 0; j < k; ++j) v = sid[t * k + j] == e ? ssel[t * k + j] : v;
+    if constexpr (sizeof(DT) == 2) ((uint16_t*)dlogits)[(size_t)t0 * ld + i] = f32_to_bf16(v);
+    else ((float*)dlogits)[(size_t)t0 * ld + i] = v;
+  }
+}
+
 template <typename F>
 int dispatch_vpl(int64_t E, F&& f) {
   if (E <= 64) return f(std::integral_constant<int, 1>{});
@@ -130,4 +182,21 @@ extern "C" int moe_router_topk_bwd(const float* gates, const float* dgates, cons
                          (int)T, (int)E, (int)k, (float*)dlogits);
     return moe_launch_status();
   });
+}
+
+int moe_router_bwd_from_blocks(const float* part, int64_t P, const float* gates, const int32_t* ids,
+                               const int32_t* row_to_pos, int64_t T, int64_t E, int64_t k, int64_t ld,
+                               void* dlogits, int dlogits_dtype, float* dsel, hipStream_t s) {
+  // tokens per block: about a pair per thread, and enough blocks for the chip
+  int64_t TB = 256 / k;
+  if (TB < 1) TB = 1;
+  while (TB > 4 && (T + TB - 1) / TB < 512) TB /= 2;
+  const dim3 grid((unsigned)((T + TB - 1) / TB)), block(256);
+  if (dlogits_dtype == MOE_DT_BF16)
+    hipLaunchKernelGGL(router_bwd_from_blocks_kernel<uint16_t>, grid, block, 0, s, part, (int)P, gates, ids,
+                       row_to_pos, (int)T, (int)E, (int)k, (int)TB, (int)ld, (uint16_t*)dlogits, dsel);
+  else
+    hipLaunchKernelGGL(router_bwd_from_blocks_kernel<float>, grid, block, 0, s, part, (int)P, gates, ids, row_to_pos,
+                       (int)T, (int)E, (int)k, (int)TB, (int)ld, (float*)dlogits, dsel);
+  return moe_launch_status();
 }

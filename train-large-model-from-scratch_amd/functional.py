@@ -50,10 +50,6 @@ def _first_order_only():
                            "without create_graph=True")
 
 
-_SPLIT_ROWS = 512  # tokens per partial sum of the router weight gradient
-_split_offsets = {}  # (tokens, slices, device) -> int32 slice bounds
-
-
 class _RouterLinear(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
@@ -82,21 +78,9 @@ def _router_wgrad(dlogits, x, w_dtype):
             and E % 8 == 0 and H % 8 == 0 and T > 0)
     if not fast:
         return (dlogits.t() @ x).to(w_dtype)
-    # contraction over the tokens: slices of _SPLIT_ROWS tokens play the experts of the ragged
-    # weight-gradient kernel, fp32 partials are summed in a fixed order (deterministic)
-    S = min(128, (T + _SPLIT_ROWS - 1) // _SPLIT_ROWS)
-    key = (T, S, x.device)
-    offs = _split_offsets.get(key)
-    if offs is None:  # constant for a given token count: made once
-        step = (T + S - 1) // S
-        offs = torch.clamp(torch.arange(S + 1, device=x.device, dtype=torch.int32) * step, max=T).to(torch.int32)
-        # (not kept when made under graph capture: such a tensor lives in the graph's memory and is
-        # only filled when the graph runs)
-        # (entries are never dropped: a captured graph may be reading one; each is at most 129 ints)
-        if not torch.cuda.is_current_stream_capturing() and len(_split_offsets) < 4096:
-            _split_offsets[key] = offs
-    part = ops.gemm_wgrad(_dense(dlogits), _dense(x), offs, S, torch.float32)
-    return part.sum(0).to(w_dtype)
+    if w_dtype not in (torch.bfloat16, torch.float32):
+        return ops.router_wgrad(_dense(dlogits), _dense(x), torch.float32).to(w_dtype)
+    return ops.router_wgrad(_dense(dlogits), _dense(x), w_dtype)
 
 
 def router_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -109,209 +93,101 @@ def router_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return out.reshape(*lead, weight.shape[0])
 
 
-_WGRAD_TILE = 256   # output tile edge of the weight-gradient kernel
-_cu_count = {}
+def _weight_gradients(needed, params, weights, wdtype):
+    """Where the gradients of the three stacks go, given which are `needed`, the parameters whose `.grad`
+    the kernel may write (or None each) and the stacks themselves: -> (tensors or None, whether each is
+    added to, what autograd receives, [(parameter, its new .grad)])."""
+    out, acc, ret, fresh = [], [], [], []
+    for need, param, w in zip(needed, params or (None, None, None), weights):
+        into, add, give = None, False, None
+        if need:
+            held = None if param is None else param.grad
+            if param is not None and held is None:
+                into = torch.empty(w.shape, dtype=param.dtype, device=w.device)
+                fresh.append((param, into))
+            elif (param is not None and held.dtype in (torch.float32, torch.bfloat16) and held.is_contiguous()
+                  and held.shape == w.shape and held.device == w.device):
+                into, add = held, True
+            else:  # autograd takes the gradient (and sums it with a .grad the kernel cannot add to)
+                into = give = torch.empty(w.shape, dtype=wdtype, device=w.device)
+        out.append(into)
+        acc.append(add)
+        ret.append(give)
+    return out, acc, ret, fresh
 
 
-def _compute_units(device) -> int:
-    n = _cu_count.get(device)
-    if n is None:
-        n = _cu_count[device] = torch.cuda.get_device_properties(device).multi_processor_count
-    return n
+def _expert_gradients(ctx, dout, needed, routing, xp, gu, act, w1b, w3b, w2b, k, **results):
+    """The layer body's backward call with the weight gradients put where they belong; -> what autograd
+    receives for the three stacks."""
+    dw, acc, ret, fresh = _weight_gradients(needed, ctx.grad_params, (w1b, w3b, w2b), ctx.w_dtype)
+    ids, gates, _, offs, pos_to_row, row_to_pos, _ = routing
+    ops.layer_backward(dout, dout.shape[0], k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b,
+                       dw, acc, **results)
+    for param, grad in fresh:
+        param.grad = grad
+    return ret
 
 
-def _wgrad_split(E: int, M: int, N: int, device) -> int:
-    """Compute units per output tile of the weight-gradient launch for [E, M, N] (at least 1).
-    The kernel makes one workgroup per 256 x 256 output tile and expert; with few experts and
-    small matrices that is a fraction of the chip, and under skewed routing the tiles of the
-    largest expert set the time: from 2 on, the contraction is cut into row segments.  Decided
-    from shapes alone (no look at the counts, no host synchronisation)."""
-    tiles = E * -(-M // _WGRAD_TILE) * -(-N // _WGRAD_TILE)
-    return max(1, _compute_units(device) // max(tiles, 1))
-
-
-def _segment_rows(E: int, M: int, N: int, R: int, device) -> int:
-    """Row segment length L for a small launch: every expert's contraction is cut into
-    ceil(n_e / L) equal parts, so that the (ceil(R/L) + E) x tiles jobs about fill the compute
-    units once and none contracts over more than L rows, however skewed the routing."""
-    tiles = -(-M // _WGRAD_TILE) * -(-N // _WGRAD_TILE)   # per expert
-    free = max(_compute_units(device) - E * tiles, tiles)
-    L = -(-R * tiles // free)
-    L = max(256, -(-L // 64) * 64)
-    while -(-R // L) + E > 1024:   # the launch takes at most 1024 segments
-        L *= 2
-    return L
-
-
-def _gemm_wgrad(a, b, offs, E, dtype, out=None, segs=None):
-    """dw[e] (+)= a[rows of e]^T b[rows of e], cut along the rows when the launch would otherwise
-    leave most of the chip idle: the segments are the "experts" of one launch with fp32 results,
-    which a second kernel adds per expert in a fixed order (reproducible).  `segs` (a dict that
-    lives as long as one backward pass) keeps the segments of these `offs` per length, so that the
-    three stacks share them."""
-    R, M = a.shape
-    N = b.shape[1]
-    if R == 0 or _wgrad_split(E, M, N, a.device) < 2:
-        return ops.gemm_wgrad(a, b, offs, E, dtype, out=out)
-    L = _segment_rows(E, M, N, R, a.device)
-    held = None if segs is None else segs.get(L)
-    if held is None:
-        held = ops.segment_offsets_by_length(offs, E, L, R)
-        if segs is not None:
-            segs[L] = held
-    seg, seg_start, S_max = held
-    part = ops.gemm_wgrad(a, b, seg, S_max, torch.float32)
-    return ops.wgrad_reduce_segments(part, seg_start, E, dtype, out=out)
-
-
-def _wgrad(a, b, offs, E, wdtype, needed, param, segs=None):
-    """One stack's weight gradient.  With `param` given the result goes into `param.grad`
-    (added to it when it exists) and None is returned for autograd."""
-    if not needed:
-        return None
-    if param is None:
-        return _gemm_wgrad(a, b, offs, E, wdtype, segs=segs)
-    held = param.grad
-    if held is None:
-        param.grad = _gemm_wgrad(a, b, offs, E, param.dtype, segs=segs)
-        return None
-    if (held.dtype in (torch.float32, torch.bfloat16) and held.is_contiguous()
-            and held.shape == (E, a.shape[1], b.shape[1]) and held.device == a.device):
-        _gemm_wgrad(a, b, offs, E, held.dtype, out=held, segs=segs)
-        return None
-    return _gemm_wgrad(a, b, offs, E, wdtype)  # a .grad the kernel cannot add to: autograd sums
-
-
-def _grad_slot_ok(param, shape, device):
-    held = param.grad
-    return held is None or (held.dtype in (torch.float32, torch.bfloat16) and held.is_contiguous()
-                            and tuple(held.shape) == tuple(shape) and held.device == device)
-
-
-def _pair_ok(E, I, H, need_w, into, device):
-    """Whether the gate and up weight gradients can come out of one launch on the side-by-side
-    [dg | du] buffer: both wanted, 256-row tiles of the stacked result do not straddle the halves,
-    the launch fills the chip without a row split, and (when the kernel is to add into `.grad`)
-    both slots are in the same state."""
-    if not (need_w[0] and need_w[1]) or I % _WGRAD_TILE != 0 or _wgrad_split(E, I, H, device) >= 2:
-        return False
-    p1, p3 = into[0], into[1]
-    if p1 is None and p3 is None:
-        return True
-    if p1 is None or p3 is None:
-        return False
-    shape = (E, I, H)
-    if not (_grad_slot_ok(p1, shape, device) and _grad_slot_ok(p3, shape, device)):
-        return False
-    g1, g3 = p1.grad, p3.grad
-    return (g1 is None) == (g3 is None) and (g1 is None or g1.dtype == g3.dtype) and p1.dtype == p3.dtype
-
-
-def _gateup(xp, w1b, w3b, offs, train: bool):
-    """Gate/up product and SwiGLU of the forward pass: -> (gu, act).  When a backward pass will
-    follow, g and u are saved in the library's blocked layout (read by nothing but the SwiGLU
-    backward); otherwise they are not written at all and `gu` is None."""
-    if train:
-        return ops.gemm_gateup_blocked(xp, w1b, w3b, offs)
-    return None, ops.gemm_gateup(xp, w1b, w3b, offs, save_gu=False)[2]
-
-
-def _expert_backward(dyp, xp, gu, act, w1b, w3b, w2b, offs, wdtype, need_w=(True, True, True),
-                     into=None, gate_blocks=False):
-    """Shared backward of the expert FFN over expert-contiguous rows.  `gu` is the forward's g and
-    u in the library's blocked layout (ops.gemm_gateup_blocked).  `need_w` and `into` are per
-    stack in the order gate, up, down.  With `gate_blocks` the fifth result holds the per-row block
-    sums of <dact, act> (the gate gradients are made from them), else None."""
-    E, I, H = w1b.shape
-    into = into or (None, None, None)
-    part = None
-    if dyp.shape[0] > 0 and _pair_ok(E, I, H, need_w, into, dyp.device):
-        # dg and du side by side: their two weight gradients are one grouped product
-        dgu, part = ops.gemm_dgrad_down_blocked(dyp, w2b, gu, offs, gate_blocks, packed=True)
-        dxp = ops.gemm_dgrad_gateup_packed(dgu, w1b, w3b, offs)
-        dw2 = _wgrad(dyp, act, offs, E, wdtype, need_w[2], into[2])
-        p1, p3 = into[0], into[1]
-        if p1 is None:
-            dw1, dw3 = ops.gemm_wgrad_pair(dgu, xp, offs, E, wdtype)
-        elif p1.grad is None:
-            p1.grad, p3.grad = ops.gemm_wgrad_pair(dgu, xp, offs, E, p1.dtype)
-            dw1 = dw3 = None
-        else:
-            ops.gemm_wgrad_pair(dgu, xp, offs, E, p1.grad.dtype, out1=p1.grad, out3=p3.grad)
-            dw1 = dw3 = None
-        return dxp, dw1, dw3, dw2, part
-    dg, du, part = ops.gemm_dgrad_down_blocked(dyp, w2b, gu, offs, gate_blocks)
-    dxp = ops.gemm_dgrad_gateup(dg, du, w1b, w3b, offs)
-    segs = {}
-    dw2 = _wgrad(dyp, act, offs, E, wdtype, need_w[2], into[2], segs)
-    dw1 = _wgrad(dg, xp, offs, E, wdtype, need_w[0], into[0], segs)
-    dw3 = _wgrad(du, xp, offs, E, wdtype, need_w[1], into[1], segs)
-    return dxp, dw1, dw3, dw2, part
+def _routing_dict(r):
+    return {"ids": r.ids, "gates": r.gates, "counts": r.counts, "offs": r.offs, "pos_to_row": r.pos_to_row,
+            "row_to_pos": r.row_to_pos}
 
 
 class _MoEFFN(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, logits, w1, w3, w2, k, bias, shadows, grad_params):
+    def forward(ctx, x, logits, w1, w3, w2, k, bias, shadows, grad_params, routing_out):
         T, H = x.shape
-        E = logits.shape[1]
+        E, I = logits.shape[1], w1.shape[1]
         x = _dense(x)
         logits = _dense(logits)
-        shadows = shadows or (None, None, None)
-        w1b, w3b, w2b = (sh if sh is not None else ops.cast_bf16(_dense(w))
-                         for w, sh in zip((w1, w3, w2), shadows))
-        ids, gates = ops.router_topk(logits, k, bias)
-        counts, offs, pos_to_row, row_to_pos = ops.histogram_scan(ids, E)
-        xp = ops.permute_fwd(x, pos_to_row, k, row_to_pos)
+        w1b, w3b, w2b = _weights_bf16(w1, w3, w2, shadows)
+        routing = ops.new_routing(T, H, E, I, k, x.device)
         train = any(ctx.needs_input_grad)
-        gu, act = _gateup(xp, w1b, w3b, offs, train)
-        y = ops.gemm_down(act, w2b, offs)
-        out = ops.combine_fwd(y, gates, row_to_pos, T, k, x.dtype)
+        out, xp, gu, act = ops.layer_forward(x, w1b, w3b, w2b, k, routing, x.dtype, logits=logits, bias=bias,
+                                             train=train)
         if train:  # (y is not kept: the gate gradients come out of the dgrad-down kernel)
-            ctx.save_for_backward(xp, gu, act, gates, ids, offs, pos_to_row, row_to_pos,
-                                  w1b, w3b, w2b)
+            ctx.save_for_backward(xp, gu, act, routing.buf, w1b, w3b, w2b)
         ctx.k, ctx.E = k, E
         ctx.grad_params = grad_params
         ctx.x_dtype, ctx.logits_dtype, ctx.w_dtype = x.dtype, logits.dtype, w1.dtype
-        ctx.mark_non_differentiable(ids, gates, counts, offs, pos_to_row, row_to_pos)
-        ctx.set_materialize_grads(False)  # no zero tensors made up for the routing outputs
+        ctx.set_materialize_grads(False)
         ctx.out_shape = out.shape
-        return out, ids, gates, counts, offs, pos_to_row, row_to_pos
+        if routing_out is not None:
+            routing_out.append(routing)
+        return out
 
     @staticmethod
-    def backward(ctx, dout, *unused):
+    def backward(ctx, dout):
         _first_order_only()
-        xp, gu, act, gates, ids, offs, pos_to_row, row_to_pos, w1b, w3b, w2b = ctx.saved_tensors
+        xp, gu, act, buf, w1b, w3b, w2b = ctx.saved_tensors
         k, E = ctx.k, ctx.E
+        dev = xp.device
         if dout is None:
-            dout = torch.zeros(ctx.out_shape, dtype=ctx.x_dtype, device=xp.device)
-        T = dout.shape[0]
+            dout = torch.zeros(ctx.out_shape, dtype=ctx.x_dtype, device=dev)
+        T, H = dout.shape
         dout = _dense(dout)
         if dout.dtype not in (torch.bfloat16, torch.float32):
             dout = dout.float()
-        dyp, _ = ops.combine_bwd(dout, None, gates, pos_to_row, k, row_to_pos)
-        dxp, dw1, dw3, dw2, part = _expert_backward(dyp, xp, gu, act, w1b, w3b, w2b, offs, ctx.w_dtype,
-                                                    ctx.needs_input_grad[2:5], ctx.grad_params,
-                                                    ctx.needs_input_grad[1] or ctx.needs_input_grad[6])
-        dx = ops.permute_bwd(dxp, row_to_pos, T, k, ctx.x_dtype) if ctx.needs_input_grad[0] else None
-        dlogits = dbias = None
-        if ctx.needs_input_grad[1] or ctx.needs_input_grad[6]:
-            dgates = ops.dgates_from_blocks(part, gates, row_to_pos, pos_to_row)
-            if ctx.needs_input_grad[6]:  # column sum of the logits' gradient, before any rounding
-                dl32 = ops.router_topk_bwd(gates, dgates, ids, T, E, k, torch.float32)
-                dbias = dl32.sum(0)
-                dlogits = dl32.to(ctx.logits_dtype) if ctx.needs_input_grad[1] else None
-            else:
-                dlogits = ops.router_topk_bwd(gates, dgates, ids, T, E, k, ctx.logits_dtype)
-        return dx, dlogits, dw1, dw3, dw2, None, dbias, None, None
+        need = ctx.needs_input_grad
+        routing = ops.new_routing(T, H, E, w1b.shape[1], k, dev, buf)
+        dx = torch.empty((T, H), dtype=ctx.x_dtype, device=dev) if need[0] else None
+        dlogits = dgates = dbias = None
+        if need[6]:
+            dgates = torch.empty(T * k, dtype=torch.float32, device=dev)
+        elif need[1]:
+            dlogits = torch.empty((T, E), dtype=ctx.logits_dtype, device=dev)
+        dw1, dw3, dw2 = _expert_gradients(ctx, dout, need[2:5], routing.pointers(), xp, gu, act, w1b, w3b, w2b, k,
+                                          dlogits=dlogits, dgates=dgates, dx=dx)
+        if need[6]:  # column sum of the logits' gradient, before any rounding
+            dl32 = ops.router_topk_bwd(routing.gates, dgates, routing.ids, T, E, k, torch.float32)
+            dbias = dl32.sum(0)
+            dlogits = dl32.to(ctx.logits_dtype) if need[1] else None
+        return dx, dlogits, dw1, dw3, dw2, None, dbias, None, None, None
 
 
 def _forward_only(*tensors) -> bool:
-    """Whether a call needs nothing kept for a backward pass: then the whole forward goes to the
-    library as one call (`ops.ffn_forward`).  Not while a launch observer is installed: it wants
-    to see the launches one by one."""
-    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
-        return False
-    return ops.launch_observer() is None
+    """Whether a call needs nothing kept for a backward pass: then nothing is (`ops.ffn_forward`)."""
+    return not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors))
 
 
 def _weights_bf16(w1, w3, w2, shadows):
@@ -337,12 +213,9 @@ def moe_ffn(x: torch.Tensor, logits: torch.Tensor, w1: torch.Tensor, w3: torch.T
     grad_params = None
     if accumulate_into_grad:
         grad_params = tuple(w if (w.requires_grad and w.is_leaf) else None for w in (w1, w3, w2))
-    out, ids, gates, counts, offs, pos_to_row, row_to_pos = _MoEFFN.apply(
-        x, logits, w1, w3, w2, k, bias, bf16_weights, grad_params)
-    if return_routing:
-        return out, {"ids": ids, "gates": gates, "counts": counts, "offs": offs,
-                     "pos_to_row": pos_to_row, "row_to_pos": row_to_pos}
-    return out
+    routing = [] if return_routing else None
+    out = _MoEFFN.apply(x, logits, w1, w3, w2, k, bias, bf16_weights, grad_params, routing)
+    return (out, _routing_dict(routing[0])) if return_routing else out
 
 
 class _MoEFFNf32(torch.autograd.Function):
@@ -415,9 +288,6 @@ def moe_ffn_f32(x: torch.Tensor, logits: torch.Tensor, w1: torch.Tensor, w3: tor
     return out
 
 
-_ROUTING_NAMES = ("ids", "gates", "counts", "offs", "pos_to_row", "row_to_pos")
-
-
 class _PreNormMoE(torch.autograd.Function):
     """Router product, routing, experts and combine as one node, optionally with the caller's
     RMSNorm in front (norm_w) and residual add behind.  Without the norm, xn is x itself
@@ -425,97 +295,103 @@ class _PreNormMoE(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, norm_w, wr, w1, w3, w2, eps, k, bias, shadows, grad_params, add_residual,
-                fused_router):
+                fused_router, routing_out):
         T, H = x.shape
-        E = wr.shape[0]
+        E, I = wr.shape[0], w1.shape[1]
         x = _dense(x)
-        shadows = shadows or (None, None, None)
-        w1b, w3b, w2b = (sh if sh is not None else ops.cast_bf16(_dense(w))
-                         for w, sh in zip((w1, w3, w2), shadows))
-        wrb = wr.detach().to(torch.bfloat16)
+        w1b, w3b, w2b = _weights_bf16(w1, w3, w2, shadows)
+        wrb = _dense(wr.detach().to(torch.bfloat16))
+        routing = ops.new_routing(T, H, E, I, k, x.device)
+        nw = rstd = None
+        if norm_w is not None:
+            nw = norm_w.detach().float().contiguous()
         if (fused_router and norm_w is not None and bias is None and T > 0
                 and ops.rmsnorm_router_supported(H, E, k)):
             # norm, router product and selection in one kernel: the normalised rows are not read
             # a second time for the router, the logits are selected on before they leave the chip
-            nw = norm_w.detach().float().contiguous()
-            xn, rstd, logits, ids, gates = ops.rmsnorm_router_fwd(x, nw, eps, _dense(wrb), k)
+            xn, rstd, logits, _, _ = ops.rmsnorm_router_fwd(x, nw, eps, wrb, k, routing)
+            selected = True
         else:
             if norm_w is not None:
-                nw = norm_w.detach().float().contiguous()
                 xn, rstd = ops.rmsnorm_fwd(x, nw, eps)
             else:
-                nw = rstd = None
                 xn = ops.cast_bf16(x)
             with torch.autocast("cuda", enabled=False):
                 logits = xn @ wrb.t()
-            ids, gates = ops.router_topk(logits, k, bias)
-        counts, offs, pos_to_row, row_to_pos = ops.histogram_scan(ids, E)
-        xp = ops.permute_fwd(xn, pos_to_row, k, row_to_pos)
+            selected = False
         train = any(ctx.needs_input_grad)
-        gu, act = _gateup(xp, w1b, w3b, offs, train)
-        y = ops.gemm_down(act, w2b, offs)
-        if add_residual:
-            out = ops.combine_fwd_residual(y, gates, row_to_pos, x, k)
-        else:
-            out = ops.combine_fwd(y, gates, row_to_pos, T, k, x.dtype)
+        out, xp, gu, act = ops.layer_forward(xn, w1b, w3b, w2b, k, routing, x.dtype,
+                                             logits=None if selected else logits, bias=bias,
+                                             residual=x if add_residual else None, train=train)
         ctx.has_norm = norm_w is not None
         if train:
-            ctx.save_for_backward(x if ctx.has_norm else None, nw, rstd, xn, wrb, xp, gu, act, gates, ids,
-                                  offs, pos_to_row, row_to_pos, w1b, w3b, w2b)
+            ctx.save_for_backward(x if ctx.has_norm else None, nw, rstd, xn, wrb, xp, gu, act, routing.buf,
+                                  w1b, w3b, w2b)
         ctx.k, ctx.E, ctx.add_residual = k, E, add_residual
         ctx.grad_params = grad_params
         ctx.x_dtype, ctx.x_shape = x.dtype, x.shape
         ctx.nw_dtype = norm_w.dtype if ctx.has_norm else None
         ctx.wr_dtype, ctx.w_dtype = wr.dtype, w1.dtype
-        ctx.mark_non_differentiable(ids, gates, counts, offs, pos_to_row, row_to_pos)
         ctx.set_materialize_grads(False)
-        return out, logits, ids, gates, counts, offs, pos_to_row, row_to_pos
+        if routing_out is not None:
+            routing_out.append(routing)
+        return out, logits
 
     @staticmethod
-    def backward(ctx, dout, dlogits_ext, *unused):
+    def backward(ctx, dout, dlogits_ext):
         _first_order_only()
-        (x, nw, rstd, xn, wrb, xp, gu, act, gates, ids, offs, pos_to_row, row_to_pos,
-         w1b, w3b, w2b) = ctx.saved_tensors
+        x, nw, rstd, xn, wrb, xp, gu, act, buf, w1b, w3b, w2b = ctx.saved_tensors
         k, E = ctx.k, ctx.E
-        T = ctx.x_shape[0]
+        T, H = ctx.x_shape
+        dev = xn.device
         if dout is None:
-            dout = torch.zeros(ctx.x_shape, dtype=ctx.x_dtype, device=xn.device)
+            dout = torch.zeros(ctx.x_shape, dtype=ctx.x_dtype, device=dev)
         dout = _dense(dout)
         if dout.dtype != ctx.x_dtype:
             dout = dout.to(ctx.x_dtype)
-        dyp, _ = ops.combine_bwd(dout, None, gates, pos_to_row, k, row_to_pos)
-        dxp, dw1, dw3, dw2, part = _expert_backward(dyp, xp, gu, act, w1b, w3b, w2b, offs, ctx.w_dtype,
-                                                    ctx.needs_input_grad[3:6], ctx.grad_params, True)
-        dgates = ops.dgates_from_blocks(part, gates, row_to_pos, pos_to_row)
-        dbias = None
-        if ctx.needs_input_grad[8]:
-            # the bias is a per-expert constant added to the logits (in fp32): its gradient is the
-            # column sum of the logits' gradient, taken before that is rounded to bf16
-            dl32 = ops.router_topk_bwd(gates, dgates, ids, T, E, k, torch.float32)
-            if dlogits_ext is not None:
-                dl32 = dl32 + dlogits_ext.float()
-            dbias = dl32.sum(0)
-            dlogits = dl32.to(torch.bfloat16)
+        need = ctx.needs_input_grad
+        routing = ops.new_routing(T, H, E, w1b.shape[1], k, dev, buf)
+        want_dx = need[0] or (ctx.has_norm and need[1])
+        dx = torch.empty((T, H), dtype=ctx.x_dtype, device=dev) if want_dx else None
+        dwr = torch.empty((E, H), dtype=ctx.wr_dtype, device=dev) if need[2] else None
+        dbias = dnw = d2 = None
+        if not need[8] and dlogits_ext is None:
+            # the gradients of the rows' two paths (experts, router) meet inside the k-row sum
+            dw1, dw3, dw2 = _expert_gradients(ctx, dout, need[3:6], routing.pointers(), xp, gu, act, w1b, w3b, w2b, k,
+                                              wr=wrb, xn=xn, dwr=dwr, dx=dx)
         else:
-            dlogits = ops.router_topk_bwd(gates, dgates, ids, T, E, k, torch.bfloat16)
-            if dlogits_ext is not None:
+            # the logits' gradient is wanted by itself (for the bias), or has a share from outside
+            dgates = torch.empty(T * k, dtype=torch.float32, device=dev)
+            dxp = torch.empty((T * k, H), dtype=torch.bfloat16, device=dev) if want_dx else None
+            dw1, dw3, dw2 = _expert_gradients(ctx, dout, need[3:6], routing.pointers(), xp, gu, act, w1b, w3b, w2b, k,
+                                              dgates=dgates, dxp=dxp)
+            if need[8]:
+                # the bias is a per-expert constant added to the logits (in fp32): its gradient is the
+                # column sum of the logits' gradient, taken before that is rounded to bf16
+                dl32 = ops.router_topk_bwd(routing.gates, dgates, routing.ids, T, E, k, torch.float32)
+                if dlogits_ext is not None:
+                    dl32 = dl32 + dlogits_ext.float()
+                dbias = dl32.sum(0)
+                dlogits = dl32.to(torch.bfloat16)
+            else:
+                dlogits = ops.router_topk_bwd(routing.gates, dgates, routing.ids, T, E, k, torch.bfloat16)
                 dlogits = dlogits + dlogits_ext.to(dlogits.dtype)
-        dwr = _router_wgrad(dlogits, xn, ctx.wr_dtype) if ctx.needs_input_grad[2] else None
-        dx = dnw = None
-        if ctx.needs_input_grad[0] or (ctx.has_norm and ctx.needs_input_grad[1]):
-            with torch.autocast("cuda", enabled=False):
-                d2 = dlogits @ wrb
+            if need[2]:
+                dwr = _router_wgrad(dlogits, xn, ctx.wr_dtype)
+            if want_dx:
+                with torch.autocast("cuda", enabled=False):
+                    d2 = dlogits @ wrb
+                # (with the norm, the router's share joins inside the norm's backward kernel)
+                dx = ops.permute_bwd(dxp, routing.row_to_pos, T, k, ctx.x_dtype, addend=None if ctx.has_norm else d2)
+        if want_dx:
             if ctx.has_norm:
-                d1 = ops.permute_bwd(dxp, row_to_pos, T, k, ctx.x_dtype)
-                dx, dnw = ops.rmsnorm_bwd(x, nw, rstd, d1, d2, dout if ctx.add_residual else None)
-                dnw = dnw.to(ctx.nw_dtype) if ctx.needs_input_grad[1] else None
-            else:  # the router path's gradient joins the k-row sum in the same pass
-                dx = ops.permute_bwd(dxp, row_to_pos, T, k, ctx.x_dtype, addend=d2)
-                if ctx.add_residual:
-                    dx = dx + dout
-            if not ctx.needs_input_grad[0]:
+                dx, dnw = ops.rmsnorm_bwd(x, nw, rstd, dx, d2, dout if ctx.add_residual else None)
+                dnw = dnw.to(ctx.nw_dtype) if need[1] else None
+            elif ctx.add_residual:
+                dx = dx + dout
+            if not need[0]:
                 dx = None
-        return dx, dnw, dwr, dw1, dw3, dw2, None, None, dbias, None, None, None, None
+        return dx, dnw, dwr, dw1, dw3, dw2, None, None, dbias, None, None, None, None, None
 
 
 def prenorm_moe(x: torch.Tensor, norm_weight: torch.Tensor, router_weight: torch.Tensor,
@@ -532,11 +408,10 @@ def prenorm_moe(x: torch.Tensor, norm_weight: torch.Tensor, router_weight: torch
     grad_params = None
     if accumulate_into_grad:
         grad_params = tuple(w if (w.requires_grad and w.is_leaf) else None for w in (w1, w3, w2))
+    routing = [] if return_routing else None
     res = _PreNormMoE.apply(x, norm_weight, router_weight, w1, w3, w2, float(eps), k, None, bf16_weights,
-                            grad_params, add_residual, fused_router)
-    if return_routing:
-        return res[0], res[1], dict(zip(_ROUTING_NAMES, res[2:]))
-    return res[0], res[1]
+                            grad_params, add_residual, fused_router, routing)
+    return (*res, _routing_dict(routing[0])) if return_routing else res
 
 
 def routed_moe(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor,
@@ -558,51 +433,51 @@ def routed_moe(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tensor, w
     grad_params = None
     if accumulate_into_grad:
         grad_params = tuple(w if (w.requires_grad and w.is_leaf) else None for w in (w1, w3, w2))
+    routing = [] if return_routing else None
     res = _PreNormMoE.apply(x, None, router_weight, w1, w3, w2, 0.0, k, bias, bf16_weights, grad_params,
-                            False, True)
-    if return_routing:
-        return res[0], res[1], dict(zip(_ROUTING_NAMES, res[2:]))
-    return res[0], res[1]
+                            False, True, routing)
+    return (*res, _routing_dict(routing[0])) if return_routing else res
 
 
 class _ExpertsRows(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, rows, ids, w1, w3, w2, grad_params):
+    def forward(ctx, rows, ids, w1, w3, w2, grad_params, routing_out):
         R, H = rows.shape
-        E = w1.shape[0]
+        E, I = w1.shape[0], w1.shape[1]
         rows = _dense(rows)
-        ids32 = _dense(ids.to(torch.int32))
-        w1b, w3b, w2b = (ops.cast_bf16(_dense(w)) for w in (w1, w3, w2))
-        counts, offs, pos_to_row, row_to_pos, bad = ops.histogram_scan(ids32, E, return_bad=True)
-        xp = ops.permute_fwd(rows, pos_to_row, 1)
+        if ids.dtype != torch.int64:
+            ids = ids.to(torch.int32)
+        w1b, w3b, w2b = _weights_bf16(w1, w3, w2, None)
+        routing = ops.new_routing(R, H, E, I, 1, rows.device)
         train = any(ctx.needs_input_grad)
-        gu, act = _gateup(xp, w1b, w3b, offs, train)
-        y = ops.gemm_down(act, w2b, offs)
-        out = ops.combine_fwd(y, None, row_to_pos, R, 1, rows.dtype)
+        out, xp, gu, act = ops.layer_forward(rows, w1b, w3b, w2b, 1, routing, rows.dtype, ids=_dense(ids), train=train)
         if train:
-            ctx.save_for_backward(xp, gu, act, offs, pos_to_row, row_to_pos, w1b, w3b, w2b)
+            ctx.save_for_backward(xp, gu, act, routing.buf, w1b, w3b, w2b)
         ctx.x_dtype, ctx.w_dtype = rows.dtype, w1.dtype
         ctx.grad_params = grad_params
-        ctx.mark_non_differentiable(counts, offs, pos_to_row, row_to_pos, bad)
         ctx.set_materialize_grads(False)
         ctx.out_shape = out.shape
-        return out, counts, offs, pos_to_row, row_to_pos, bad
+        if routing_out is not None:
+            routing_out.append(routing)
+        return out
 
     @staticmethod
-    def backward(ctx, dout, *unused):
+    def backward(ctx, dout):
         _first_order_only()
-        xp, gu, act, offs, pos_to_row, row_to_pos, w1b, w3b, w2b = ctx.saved_tensors
+        xp, gu, act, buf, w1b, w3b, w2b = ctx.saved_tensors
         if dout is None:
             dout = torch.zeros(ctx.out_shape, dtype=ctx.x_dtype, device=xp.device)
-        R = dout.shape[0]
+        R, H = dout.shape
         dout = _dense(dout)
         if dout.dtype not in (torch.bfloat16, torch.float32):
             dout = dout.float()
-        dyp, _ = ops.combine_bwd(dout, None, None, pos_to_row, 1)
-        dxp, dw1, dw3, dw2, _ = _expert_backward(dyp, xp, gu, act, w1b, w3b, w2b, offs,
-                                                 ctx.w_dtype, ctx.needs_input_grad[2:5], ctx.grad_params)
-        drows = ops.permute_bwd(dxp, row_to_pos, R, 1, ctx.x_dtype) if ctx.needs_input_grad[0] else None
-        return drows, None, dw1, dw3, dw2, None
+        need = ctx.needs_input_grad
+        ids, _, counts, offs, p2r, r2p, bad = ops.new_routing(R, H, w1b.shape[0], w1b.shape[1], 1, xp.device,
+                                                              buf).pointers()
+        drows = torch.empty((R, H), dtype=ctx.x_dtype, device=xp.device) if need[0] else None
+        dw1, dw3, dw2 = _expert_gradients(ctx, dout, need[2:5], (0, 0, counts, offs, p2r, r2p, bad), xp, gu, act,
+                                          w1b, w3b, w2b, 1, dx=drows)
+        return drows, None, dw1, dw3, dw2, None, None
 
 
 class _ExpertsRowsF32(torch.autograd.Function):
@@ -676,12 +551,14 @@ def experts_rows(rows: torch.Tensor, ids: torch.Tensor, w1, w3, w2, return_routi
     grad_params = None
     if accumulate_into_grad:
         grad_params = tuple(w if (w.requires_grad and w.is_leaf) else None for w in (w1, w3, w2))
-    out, counts, offs, pos_to_row, row_to_pos, bad = _ExpertsRows.apply(rows, ids, w1, w3, w2, grad_params)
+    routing = [] if (check_ids or return_routing) else None
+    out = _ExpertsRows.apply(rows, ids, w1, w3, w2, grad_params, routing)
     if check_ids:
-        n = int(bad.item())
+        n = int(routing[0].bad_ids.item())
         if n:
             raise ValueError(f"experts_rows: {n} of {ids.numel()} expert ids lie outside [0, {w1.shape[0]})")
     if return_routing:
-        return out, {"counts": counts, "offs": offs, "pos_to_row": pos_to_row, "row_to_pos": row_to_pos,
-                     "bad_ids": bad}
+        r = routing[0]
+        return out, {"counts": r.counts, "offs": r.offs, "pos_to_row": r.pos_to_row, "row_to_pos": r.row_to_pos,
+                     "bad_ids": r.bad_ids}
     return out

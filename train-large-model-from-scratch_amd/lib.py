@@ -8,6 +8,8 @@ import threading
 from .build import LIB_PATH
 
 _vp, _i64, _int = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
+_args = ctypes.c_char_p                                       # an argument structure, packed
+_observer_fn = ctypes.CFUNCTYPE(None, ctypes.c_char_p, _int)  # moe_launch_observer_fn
 
 # name -> (restype, argtypes); mirrors include/moe_gfx950.h one to one
 SIGNATURES = {
@@ -61,6 +63,12 @@ SIGNATURES = {
     "moe_ffn_forward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64]),
     "moe_ffn_forward": (_int, [_vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _int,
                                 _vp, _i64, _vp]),
+    "moe_router_wgrad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "moe_router_wgrad": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _int, _vp, _i64, _vp]),
+    "moe_layer_scratch_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _int]),
+    "moe_layer_forward": (_int, [_args, _vp]),
+    "moe_layer_backward": (_int, [_args, _vp]),
+    "moe_set_launch_observer": (None, [_observer_fn]),
     "moe_f32_gather_rows": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp]),
     "moe_f32_combine_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp]),
     "moe_f32_combine_bwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp]),
@@ -90,20 +98,45 @@ class MoELib:
             fn = getattr(self.cdll, name)  # AttributeError if the symbol is missing
             fn.restype, fn.argtypes = res, args
         self.abi_version = self.cdll.moe_abi_version()
-        # Optional observer of the launches (a profiling aid): an object with before(name) and
-        # after(name), called around every entry point, e.g. to record events on the stream.
-        self.observer = None
+        self._observer = self._observer_callback = None
+
+    @property
+    def observer(self):
+        """Optional observer of the launches (a profiling aid): an object with before(name) and
+        after(name), called around every entry point, and around every launch inside those that
+        make several, e.g. to record events on the stream."""
+        return self._observer
+
+    @observer.setter
+    def observer(self, obs):
+        def forward(name, after):
+            (obs.after if after else obs.before)(name.decode())
+
+        self._observer = obs
+        callback = _observer_fn(forward) if obs is not None else _observer_fn()
+        self.cdll.moe_set_launch_observer(callback)
+        self._observer_callback = callback  # (the library holds a bare pointer to it)
 
     def call(self, name: str, *args):
-        obs = self.observer
+        obs = self._observer
         if obs is not None:
             obs.before(name)
         rc = getattr(self.cdll, name)(*args)
         if obs is not None:
             obs.after(name)
         if rc != 0:
-            what = ERRORS.get(rc, f"hipError_t {rc}" if rc > 0 else f"code {rc}")
-            raise MoELibError(f"{name} failed: {what}")
+            self.failed(name, rc)
+
+    def call_layer(self, name: str, *args):
+        """An entry point that enqueues many launches: its launches are observed, not the call."""
+        rc = getattr(self.cdll, name)(*args)
+        if rc != 0:
+            self.failed(name, rc)
+
+    @staticmethod
+    def failed(name: str, rc: int):
+        what = ERRORS.get(rc, f"hipError_t {rc}" if rc > 0 else f"code {rc}")
+        raise MoELibError(f"{name} failed: {what}")
 
 
 _lock = threading.Lock()

@@ -26,7 +26,7 @@ import torch
 from torch import Tensor
 
 from . import ops
-from .functional import _expert_backward, _router_wgrad
+from .functional import _router_wgrad
 
 _BF16 = torch.bfloat16
 
@@ -54,17 +54,11 @@ def ffn_fwd(x: Tensor, logits: Tensor, w1: Tensor, w3: Tensor, w2: Tensor, k: in
     E = logits.shape[1]
     x, logits = ops.dense(x), ops.dense(logits)
     wb = [ops.dense(w) if w.dtype == _BF16 else ops.cast_bf16(ops.dense(w)) for w in (w1, w3, w2)]
-    ids, gates = ops.router_topk(logits, k, None)
-    _, offs, pos_to_row, row_to_pos = ops.histogram_scan(ids, E)
-    xp = ops.permute_fwd(x, pos_to_row, k, row_to_pos)
-    if train:
-        gu, act = ops.gemm_gateup_blocked(xp, wb[0], wb[1], offs)
-    else:
-        gu, act = _empty(x, torch.uint8), ops.gemm_gateup(xp, wb[0], wb[1], offs, save_gu=False)[2]
-    y = ops.gemm_down(act, wb[2], offs)
-    out = ops.combine_fwd(y, gates, row_to_pos, T, k, x.dtype)
+    r = ops.RoutingTensors(T, E, k, x.device)
+    out, xp, gu, act = ops.layer_forward(x, *wb, k, r, x.dtype, logits=logits, train=train)
     copies = [b if w.dtype != _BF16 else _empty(x) for w, b in zip((w1, w3, w2), wb)]
-    return (out, ids, gates, offs, pos_to_row, row_to_pos, xp, gu, act, *copies)
+    return (out, r.ids, r.gates, r.offs, r.pos_to_row, r.row_to_pos, xp, gu if train else _empty(x, torch.uint8), act,
+            *copies)
 
 
 @ffn_fwd.register_fake
@@ -85,21 +79,19 @@ def ffn_bwd(dout: Tensor, xp: Tensor, gu: Tensor, act: Tensor, gates: Tensor,
             ids: Tensor, offs: Tensor, pos_to_row: Tensor, row_to_pos: Tensor, w1b: Tensor,
             w3b: Tensor, w2b: Tensor, k: int, x_is_f32: bool, logits_is_f32: bool,
             w_is_f32: bool) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
-    """-> dx, dlogits, dw1, dw3, dw2.  The kernels of the eager backward pass
-    (`functional._expert_backward`)."""
-    T = dout.shape[0]
+    """-> dx, dlogits, dw1, dw3, dw2.  The call of the eager backward pass."""
+    T, H = dout.shape
     E = offs.numel() - 1
     f32 = torch.float32
     dout = ops.dense(dout)
     if dout.dtype not in (_BF16, f32):
         dout = dout.float()
-    dyp, _ = ops.combine_bwd(dout, None, gates, pos_to_row, k, row_to_pos)
-    wdt = f32 if w_is_f32 else _BF16
-    dxp, dw1, dw3, dw2, part = _expert_backward(dyp, xp, gu, act, w1b, w3b, w2b, offs, wdt, gate_blocks=True)
-    dgates = ops.dgates_from_blocks(part, gates, row_to_pos, pos_to_row)
-    dx = ops.permute_bwd(dxp, row_to_pos, T, k, f32 if x_is_f32 else _BF16)
-    dlogits = ops.router_topk_bwd(gates, dgates, ids, T, E, k, f32 if logits_is_f32 else _BF16)
-    return dx, dlogits, dw1, dw3, dw2
+    dx = dout.new_empty(T, H, dtype=f32 if x_is_f32 else _BF16)
+    dlogits = dout.new_empty(T, E, dtype=f32 if logits_is_f32 else _BF16)
+    dw = [torch.empty_like(w, dtype=f32 if w_is_f32 else _BF16) for w in (w1b, w3b, w2b)]
+    ops.layer_backward(dout, T, k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b, dw,
+                       dlogits=dlogits, dx=dx)
+    return dx, dlogits, *dw
 
 
 @ffn_bwd.register_fake
@@ -161,20 +153,13 @@ def routed_fwd(x: Tensor, wr: Tensor, w1: Tensor, w3: Tensor, w2: Tensor, k: int
     wrb = ops.dense(wr.detach().to(_BF16))
     with torch.autocast("cuda", enabled=False):
         logits = xn @ wrb.t()
-    ids, gates = ops.router_topk(logits, k, None)
-    _, offs, pos_to_row, row_to_pos = ops.histogram_scan(ids, E)
-    xp = ops.permute_fwd(xn, pos_to_row, k, row_to_pos)
-    if train:
-        gu, act = ops.gemm_gateup_blocked(xp, wb[0], wb[1], offs)
-    else:
-        gu, act = _empty(x, torch.uint8), ops.gemm_gateup(xp, wb[0], wb[1], offs, save_gu=False)[2]
-    y = ops.gemm_down(act, wb[2], offs)
-    out = ops.combine_fwd(y, gates, row_to_pos, T, k, x.dtype)
+    r = ops.RoutingTensors(T, E, k, x.device)
+    out, xp, gu, act = ops.layer_forward(xn, *wb, k, r, x.dtype, logits=logits, train=train)
     copies = [b if w.dtype != _BF16 else _empty(x) for w, b in zip((w1, w3, w2), wb)]
     if not train:
-        return (out, logits, ids, gates, offs, pos_to_row, row_to_pos, _empty(x), _empty(x), _empty(x), gu,
-                _empty(x), *copies)
-    return (out, logits, ids, gates, offs, pos_to_row, row_to_pos, xn if x.dtype != _BF16 else _empty(x),
+        return (out, logits, r.ids, r.gates, r.offs, r.pos_to_row, r.row_to_pos, _empty(x), _empty(x), _empty(x),
+                _empty(x, torch.uint8), _empty(x), *copies)
+    return (out, logits, r.ids, r.gates, r.offs, r.pos_to_row, r.row_to_pos, xn if x.dtype != _BF16 else _empty(x),
             wrb if wr.dtype != _BF16 else _empty(x), xp, gu, act, *copies)
 
 
@@ -201,25 +186,28 @@ def routed_bwd(dout: Tensor, dlogits_ext: Tensor | None, xn: Tensor, wrb: Tensor
     """-> dx, dwr, dw1, dw3, dw2.  The backward of `functional.routed_moe`: `dlogits_ext` is the
     gradient that reaches the returned logits from outside (an auxiliary loss) or None; the router
     path's input gradient joins the k-row sum inside the permute-backward kernel."""
-    T = dout.shape[0]
+    T, H = dout.shape
     E = offs.numel() - 1
     f32 = torch.float32
     xdt = f32 if x_is_f32 else _BF16
     dout = ops.dense(dout)
     if dout.dtype != xdt:
         dout = dout.to(xdt)
-    dyp, _ = ops.combine_bwd(dout, None, gates, pos_to_row, k, row_to_pos)
-    dxp, dw1, dw3, dw2, part = _expert_backward(dyp, xp, gu, act, w1b, w3b, w2b, offs,
-                                                f32 if w_is_f32 else _BF16, gate_blocks=True)
-    dgates = ops.dgates_from_blocks(part, gates, row_to_pos, pos_to_row)
-    dlogits = ops.router_topk_bwd(gates, dgates, ids, T, E, k, _BF16)
-    if dlogits_ext is not None:
-        dlogits = dlogits + dlogits_ext.to(_BF16)
+    dw = [torch.empty_like(w, dtype=f32 if w_is_f32 else _BF16) for w in (w1b, w3b, w2b)]
+    saved = (dout, T, k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b, dw)
+    if dlogits_ext is None:
+        dx = dout.new_empty(T, H)
+        dwr = torch.empty_like(wrb, dtype=f32 if wr_is_f32 else _BF16)
+        ops.layer_backward(*saved, wr=wrb, xn=xn, dwr=dwr, dx=dx)
+        return dx, dwr, *dw
+    dgates, dxp = torch.empty_like(gates), torch.empty_like(xp)
+    ops.layer_backward(*saved, dgates=dgates, dxp=dxp)
+    dlogits = ops.router_topk_bwd(gates, dgates, ids, T, E, k, _BF16) + dlogits_ext.to(_BF16)
     dwr = _router_wgrad(dlogits, xn, f32 if wr_is_f32 else _BF16)
     with torch.autocast("cuda", enabled=False):
         d2 = dlogits @ wrb
     dx = ops.permute_bwd(dxp, row_to_pos, T, k, xdt, addend=d2)
-    return dx, dwr, dw1, dw3, dw2
+    return dx, dwr, *dw
 
 
 @routed_bwd.register_fake
