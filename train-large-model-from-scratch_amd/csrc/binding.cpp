@@ -1,0 +1,665 @@
+// The differentiable entry points as autograd nodes in C++: what `functional.py` calls.
+//
+// A small step is bound by the host (a step of 512 tokens of a narrow layer has 0.1 ms of kernels), and
+// most of that host time was Python: argument handling, a dozen allocations and the node itself, in both
+// directions.  The nodes below do the same with three allocations per direction besides the results, and
+// the backward pass runs on the engine's thread without taking the interpreter's lock.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/extension.h>
+
+#include <stdexcept>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include "moe_gfx950.h"
+
+void moe_observe(const char* name, int after);  // (internal.h, which only device code can include)
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+typedef std::optional<Tensor> OptTensor;
+
+namespace {
+
+// Raised as lib.MoELibError.
+struct LibError : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
+void check(int rc, const char* name) {
+  if (rc == 0) return;
+  static const char* const names[] = {"MOE_ERR_NULL", "MOE_ERR_SHAPE", "MOE_ERR_LIMIT",
+                                      "MOE_ERR_DTYPE", "MOE_ERR_WORKSPACE", "MOE_ERR_ALIGN"};
+  const std::string what = rc < 0 && rc >= -6 ? std::string(names[-rc - 1])
+                                              : (rc > 0 ? "hipError_t " : "code ") + std::to_string(rc);
+  throw LibError(std::string(name) + " failed: " + what);
+}
+
+#define CALL(fn, ...)                \
+  do {                               \
+    moe_observe(#fn, 0);             \
+    const int rc_ = fn(__VA_ARGS__); \
+    moe_observe(#fn, 1);             \
+    check(rc_, #fn);                 \
+  } while (0)
+
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+int64_t dt(at::ScalarType t) {
+  if (t == at::kBFloat16) return MOE_DT_BF16;
+  if (t == at::kFloat) return MOE_DT_F32;
+  throw py::type_error("unsupported dtype: the MoE kernels take bf16 or fp32");
+}
+int64_t dt(const Tensor& t) { return dt(t.scalar_type()); }
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+void need_gpu(const Tensor& t) {
+  TORCH_CHECK(!t.defined() || t.is_cuda(), "the MoE kernels need GPU tensors (no CPU path exists)");
+}
+
+// Contiguous and 16-byte aligned, as the kernels need their buffers.
+Tensor dense(const Tensor& t) {
+  need_gpu(t);
+  Tensor c = t.is_contiguous() ? t : t.contiguous();
+  return (reinterpret_cast<uintptr_t>(c.data_ptr()) & 15) == 0 ? c : c.clone();
+}
+
+Tensor empty(at::IntArrayRef size, at::ScalarType type, const Tensor& like) {
+  return at::empty(size, at::TensorOptions().dtype(type).device(like.device()));
+}
+
+Tensor cast_bf16(const Tensor& t) {
+  if (t.scalar_type() == at::kBFloat16) return t;
+  if (t.scalar_type() != at::kFloat) return t.to(at::kBFloat16);
+  Tensor out = empty(t.sizes(), at::kBFloat16, t);
+  CALL(moe_cast_f32_bf16, t.data_ptr<float>(), (uint16_t*)out.data_ptr(), t.numel(), stream_of(t));
+  return out;
+}
+
+const uint16_t* bf(const Tensor& t) { return (const uint16_t*)ptr(t); }
+
+// The bf16 product is a bf16 product whatever autocast the caller is in.
+struct NoAutocast {
+  c10::impl::ExcludeDispatchKeyGuard guard{c10::DispatchKey::AutocastCUDA};
+};
+
+int64_t up(int64_t n, int64_t to) { return (n + to - 1) / to * to; }
+
+// What a forward pass leaves for the backward pass besides its inputs: the routing (int32 words, parts in
+// this order: ids, gates, counts, offs, pos_to_row, row_to_pos, bad ids) and the expert-ordered rows xp
+// with gu and act behind them.
+struct Routing {
+  enum Part { IDS, GATES, COUNTS, OFFS, POS_TO_ROW, ROW_TO_POS, BAD, PARTS };
+  int64_t at[PARTS + 1];
+  Routing(int64_t R, int64_t E) {
+    const int64_t n[PARTS] = {R, R, E, E + 1, R, R, 1};
+    at[0] = 0;
+    for (int i = 0; i < PARTS; ++i) at[i + 1] = at[i] + up(n[i], 64);
+  }
+  int32_t* part(const Tensor& buf, Part p) const { return buf.data_ptr<int32_t>() + at[p]; }
+};
+
+struct Kept {
+  int64_t gu, act, total;
+  Kept(int64_t R, int64_t H, int64_t E, int64_t I, bool with_gu) {
+    gu = up(R * H * 2, 256);
+    act = gu + (with_gu ? up(moe_gu_blocked_bytes(R, E, I), 256) : 0);
+    total = act + up(R * I * 2, 256);
+    if (total == 0) total = 256;
+  }
+};
+
+struct Weights {
+  Tensor w1, w3, w2;
+};
+
+Weights bf16_weights(const Tensor& w1, const Tensor& w3, const Tensor& w2, const OptTensor& s1, const OptTensor& s3,
+                     const OptTensor& s2) {
+  const auto one = [](const Tensor& w, const OptTensor& s) { return s && s->defined() ? *s : cast_bf16(dense(w)); };
+  return {one(w1, s1), one(w3, s3), one(w2, s2)};
+}
+
+const Tensor& value(const OptTensor& t) {
+  static const Tensor none;
+  return t ? *t : none;
+}
+
+// Autograd counts a node's inputs without the tensors that were not given.
+struct Present {
+  int64_t mask = 0;
+  Present() = default;
+  Present(std::initializer_list<bool> given) {
+    int i = 0;
+    for (bool g : given) mask |= (int64_t)g << i++;
+  }
+  bool wants_gradient(AutogradContext* ctx, int input) const {
+    return (mask >> input & 1) && ctx->needs_input_grad(__builtin_popcountll(mask & ((1ll << input) - 1)));
+  }
+};
+
+struct Layer {  // the arguments of one call
+  int64_t k = 1;
+  double eps = 0;
+  bool add_residual = false, fused_router = false, accumulate = false, train = false;
+  OptTensor s1, s3, s2;           // bf16 copies of the weights
+  Tensor* routing_out = nullptr;  // where the caller wants the routing left
+};
+
+struct Outputs {
+  Tensor out, logits, routing, kept, xn, wrb, nw, rstd;
+  Weights w;
+};
+
+Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Tensor& wr, const Tensor& logits_,
+                const Tensor& w1, const Tensor& w3, const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
+  Outputs f;
+  need_gpu(x_);
+  const c10::DeviceGuard guard(x_.device());
+  const Tensor x = dense(x_);
+  TORCH_CHECK(x.dim() == 2 && w1.dim() == 3, "the layer takes x [tokens, hidden] and weights [experts, ., .]");
+  const int64_t T = x.size(0), H = x.size(1), I = w1.size(1), k = o.k, R = T * k;
+  const int64_t E = wr.defined() ? wr.size(0) : logits_.defined() ? logits_.size(1) : w1.size(0);
+  TORCH_CHECK(w1.size(0) == E && w3.size(0) == E && w2.size(0) == E && w1.size(2) == H && w3.size(2) == H &&
+                  w3.size(1) == I && w2.size(1) == H && w2.size(2) == I,
+              "the weights' shapes do not belong together");
+  (void)dt(x);
+  const at::ScalarType x_type = x.scalar_type();
+  f.w = bf16_weights(w1, w3, w2, o.s1, o.s3, o.s2);
+  void* s = stream_of(x);
+  const Routing r(R, E);
+  Tensor rows = x;
+  Tensor logits;
+  bool selected = false;
+  if (o.train || o.routing_out || !(wr.defined() || logits_.defined()) || norm_w.defined() || T == 0)
+    f.routing = empty({r.at[Routing::PARTS]}, at::kInt, x);
+  if (wr.defined()) {
+    f.wrb = dense(cast_bf16(dense(wr.detach())));
+    if (norm_w.defined()) {
+      f.nw = norm_w.detach().to(at::kFloat).contiguous();
+      f.xn = empty({T, H}, at::kBFloat16, x);
+      f.rstd = empty({T}, at::kFloat, x);
+      if (o.fused_router && !bias.defined() && T > 0 && moe_rmsnorm_router_supported(H, E, k)) {
+        // norm, router product and selection in one kernel: the normalised rows are not read a second
+        // time for the router, the logits are selected on before they leave the chip
+        logits = empty({T, E}, at::kBFloat16, x);
+        CALL(moe_rmsnorm_router_fwd, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, bf(f.wrb), T, H,
+             E, k, (uint16_t*)f.xn.data_ptr(), f.rstd.data_ptr<float>(), (uint16_t*)logits.data_ptr(),
+             r.part(f.routing, Routing::IDS), (float*)r.part(f.routing, Routing::GATES), s);
+        selected = true;
+      } else {
+        CALL(moe_rmsnorm_fwd, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, T, H,
+             (uint16_t*)f.xn.data_ptr(), f.rstd.data_ptr<float>(), s);
+      }
+    } else {
+      f.xn = cast_bf16(x);
+    }
+    rows = f.xn;
+    if (!selected) {
+      const NoAutocast off;
+      logits = at::mm(f.xn, f.wrb.t());
+    }
+  } else if (logits_.defined()) {
+    logits = dense(logits_);
+  }
+  f.logits = logits;
+  const Tensor b = bias.defined() ? dense(bias) : Tensor();
+  if (!f.routing.defined()) {  // nothing is kept and nobody asks for the routing
+    f.out = empty({T, H}, x_type, x);
+    const int64_t bytes = moe_ffn_forward_workspace_bytes(T, H, E, I, k);
+    const Tensor ws = empty({std::max<int64_t>(bytes, 256)}, at::kByte, x);
+    // (it tells the observer about its launches itself, as do the two calls of a training step)
+    check(moe_ffn_forward(rows.data_ptr(), (int)dt(rows), logits.data_ptr(), (int)dt(logits), (const float*)ptr(b),
+                          bf(f.w.w1), bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(), (int)dt(x_type),
+                          ws.data_ptr(), ws.numel(), s),
+          "moe_ffn_forward");
+    return f;
+  }
+  f.out = empty({T, H}, x_type, x);
+  const Kept kept(R, H, E, I, o.train);
+  f.kept = empty({kept.total}, at::kByte, x);
+  char* base = (char*)f.kept.data_ptr();
+  const int64_t bytes = std::max<int64_t>(moe_layer_scratch_bytes(T, H, E, I, k, 0), 256);
+  const Tensor scratch = empty({bytes}, at::kByte, x);
+  Tensor ids = ids_;
+  moe_layer_forward_args a{};
+  a.T = T, a.H = H, a.E = E, a.I = I, a.k = k;
+  a.x = rows.data_ptr(), a.x_dtype = dt(rows);
+  a.ids = r.part(f.routing, Routing::IDS);
+  a.gates = (float*)r.part(f.routing, Routing::GATES);
+  if (logits.defined() && !selected) {
+    a.logits = logits.data_ptr(), a.logits_dtype = dt(logits), a.bias = (const float*)ptr(b);
+  } else if (!logits.defined()) {  // rows already dispatched: their experts are given
+    ids = dense(ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt ? ids : ids.to(at::kInt));
+    TORCH_CHECK(ids.numel() == R, "one expert id per row is needed");
+    a.gates = nullptr;
+    if (ids.scalar_type() == at::kLong) a.ids64 = ids.data_ptr<int64_t>();
+    else a.ids = ids.data_ptr<int32_t>();
+    a.bad_ids = r.part(f.routing, Routing::BAD);
+  }
+  a.counts = r.part(f.routing, Routing::COUNTS), a.offs = r.part(f.routing, Routing::OFFS);
+  a.pos_to_row = r.part(f.routing, Routing::POS_TO_ROW), a.row_to_pos = r.part(f.routing, Routing::ROW_TO_POS);
+  a.w1 = bf(f.w.w1), a.w3 = bf(f.w.w3), a.w2 = bf(f.w.w2);
+  a.residual = o.add_residual ? x.data_ptr() : nullptr;
+  a.out = f.out.data_ptr(), a.out_dtype = dt(x_type);
+  a.xp = (uint16_t*)base;
+  a.gu = o.train ? base + kept.gu : nullptr;
+  a.act = (uint16_t*)(base + kept.act);
+  a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
+  check(moe_layer_forward(&a, s), "moe_layer_forward");
+  if (o.routing_out) *o.routing_out = f.routing;
+  return f;
+}
+
+void first_order_only() {
+  // Called at the top of every backward here.  The backward passes run kernels autograd cannot see
+  // through, so a gradient of a gradient would silently lack their terms (grad mode is on inside a
+  // backward pass only under create_graph).
+  TORCH_CHECK(!at::GradMode::is_enabled(),
+              "the MoE kernels' backward pass is not differentiable: call backward()/grad() without create_graph=True");
+}
+
+// Where the gradients of the three stacks go: tensors of their own that autograd receives, or (with
+// `params`: the masters whose .grad the kernel may write) the existing .grad, added to, or a new one.
+struct WeightGradients {
+  Tensor into[3], give[3], fresh[3];
+  bool add[3] = {false, false, false};
+  WeightGradients(const bool (&need)[3], const std::vector<Tensor>& params, const Tensor (&w)[3], at::ScalarType type) {
+    for (int i = 0; i < 3; ++i) {
+      if (!need[i]) continue;
+      const Tensor param = params.empty() ? Tensor() : params[i];
+      const Tensor held = param.defined() ? param.grad() : Tensor();
+      if (param.defined() && !held.defined()) {
+        into[i] = fresh[i] = empty(w[i].sizes(), param.scalar_type(), w[i]);
+      } else if (held.defined() && (held.scalar_type() == at::kFloat || held.scalar_type() == at::kBFloat16) &&
+                 held.is_contiguous() && held.sizes() == w[i].sizes() && held.device() == w[i].device()) {
+        into[i] = held;
+        add[i] = true;
+      } else {  // autograd takes the gradient (and sums it with a .grad the kernel cannot add to)
+        into[i] = give[i] = empty(w[i].sizes(), type, w[i]);
+      }
+    }
+  }
+};
+
+Tensor router_wgrad(const Tensor& dlogits, const Tensor& xn, at::ScalarType type) {
+  const int64_t T = xn.size(0), H = xn.size(1), E = dlogits.size(1);
+  if (T == 0 || E % 8 != 0 || H % 8 != 0) return at::mm(dlogits.t(), xn).to(type);
+  const bool direct = type == at::kFloat || type == at::kBFloat16;
+  Tensor dw = empty({E, H}, direct ? type : at::kFloat, xn);
+  const int64_t bytes = moe_router_wgrad_workspace_bytes(T, H, E);
+  const Tensor ws = empty({std::max<int64_t>(bytes, 16)}, at::kByte, xn);
+  CALL(moe_router_wgrad, bf(dlogits), bf(xn), T, H, E, dw.data_ptr(), (int)dt(dw), ws.data_ptr(), ws.numel(),
+       stream_of(xn));
+  return direct ? dw : dw.to(type);
+}
+
+// Router product (or given logits, or given expert ids), routing, experts and combine as one node,
+// optionally with the caller's RMSNorm in front and residual add behind.
+struct LayerNode : torch::autograd::Function<LayerNode> {
+  enum Input { X, NORM, WR, LOGITS, W1, W3, W2, BIAS, IDS, OPTIONS, INPUTS };
+
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& norm_w_, const OptTensor& wr_,
+                               const OptTensor& logits_, const Tensor& w1, const Tensor& w3, const Tensor& w2,
+                               const OptTensor& bias_, const OptTensor& ids_, const Layer& o) {
+    const Tensor &norm_w = value(norm_w_), &wr = value(wr_), &logits = value(logits_), &bias = value(bias_),
+                 &ids = value(ids_);
+    const Outputs f = ::forward(o, x, norm_w, wr, logits, w1, w3, w2, bias, ids);
+    // (y is not kept: the gate gradients come out of the dgrad-down kernel)
+    ctx->save_for_backward({norm_w.defined() ? dense(x) : Tensor(), f.nw, f.rstd, f.xn, f.wrb, f.kept, f.routing, f.w.w1,
+                            f.w.w3, f.w.w2});
+    const auto type = [](const Tensor& t) { return t.defined() ? (int64_t)t.scalar_type() : -1; };
+    ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), x.size(1), o.k, o.add_residual, type(x), type(norm_w),
+                                                type(wr), type(logits), type(w1),
+                                                Present{true, norm_w.defined(), wr.defined(), logits.defined(), true, true,
+                                                        true, bias.defined(), ids.defined()}.mask};
+    if (o.accumulate) {
+      std::vector<Tensor> params;
+      for (const Tensor* w : {&w1, &w3, &w2}) params.push_back(w->requires_grad() && w->is_leaf() ? *w : Tensor());
+      ctx->saved_data["params"] = params;
+    }
+    ctx->set_materialize_grads(false);
+    if (wr.defined()) return {f.out, f.logits};
+    return {f.out};
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    first_order_only();
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &nw = saved[1], &rstd = saved[2], &xn = saved[3], &wrb = saved[4], &kept_buf = saved[5],
+                 &routing = saved[6];
+    const Tensor w[3] = {saved[7], saved[8], saved[9]};
+    const std::vector<int64_t> ints = ctx->saved_data["i"].toIntVector();
+    const int64_t T = ints[0], H = ints[1], k = ints[2], R = T * k, E = w[0].size(0), I = w[0].size(1);
+    const bool add_residual = ints[3], has_norm = ints[5] >= 0, has_router = ints[6] >= 0, has_logits = ints[7] >= 0;
+    const auto type = [&](int i) { return (at::ScalarType)ints[i]; };
+    const at::ScalarType x_type = type(4);
+    std::vector<Tensor> params;
+    const auto held = ctx->saved_data.find("params");
+    if (held != ctx->saved_data.end()) params = held->second.toTensorVector();
+    const c10::DeviceGuard guard(kept_buf.device());
+    Present present;
+    present.mask = ints[9];
+    const auto need = [&](Input i) { return present.wants_gradient(ctx, i); };
+
+    Tensor dout = grads[0].defined() ? grads[0] : at::zeros({T, H}, kept_buf.options().dtype(x_type));
+    dout = dense(dout);
+    if (has_router ? dout.scalar_type() != x_type : dout.scalar_type() != at::kBFloat16 && dout.scalar_type() != at::kFloat)
+      dout = dout.to(has_router ? x_type : at::kFloat);
+    const Tensor ext = has_router && grads.size() > 1 ? grads[1] : Tensor();
+
+    const bool need_w[3] = {need(W1), need(W3), need(W2)};
+    const bool want_dx = need(X) || (has_norm && need(NORM)), want_bias = need(BIAS);
+    const bool want_logits = has_logits && need(LOGITS), want_wr = has_router && need(WR);
+    // the logits' gradient is wanted by itself (for the bias) or has a share from outside: the router's
+    // side is then worked out below from the gate gradients
+    const bool by_hand = want_bias || ext.defined();
+    WeightGradients wg(need_w, params, w, type(8));
+    Tensor dx, dxp, dwr, dlogits, dgates, dbias, dnw, d2;
+    const bool rows_out = by_hand && has_router;  // the router's share joins below
+    if (want_dx && !rows_out) dx = empty({T, H}, x_type, kept_buf);
+    if (want_dx && rows_out) dxp = empty({R, H}, at::kBFloat16, kept_buf);
+    if (by_hand) dgates = empty({R}, at::kFloat, kept_buf);
+    const bool wr_direct = has_router && (type(6) == at::kFloat || type(6) == at::kBFloat16);
+    if (!by_hand && want_wr) dwr = empty({E, H}, wr_direct ? type(6) : at::kFloat, kept_buf);
+    if (!by_hand && want_logits) dlogits = empty({T, E}, type(7), kept_buf);
+
+    const Routing r(R, E);
+    const Kept kept(R, H, E, I, true);
+    const char* base = (const char*)kept_buf.data_ptr();
+    const int64_t bytes = std::max<int64_t>(moe_layer_scratch_bytes(T, H, E, I, k, 1), 256);
+    const Tensor scratch = empty({bytes}, at::kByte, kept_buf);
+    void* s = stream_of(kept_buf);
+    moe_layer_backward_args a{};
+    a.T = T, a.H = H, a.E = E, a.I = I, a.k = k;
+    a.dout = dout.data_ptr(), a.dout_dtype = dt(dout);
+    const float* gates = has_router || has_logits ? (const float*)r.part(routing, Routing::GATES) : nullptr;
+    const int32_t* ids = r.part(routing, Routing::IDS);
+    a.gates = gates, a.ids = ids;
+    a.offs = r.part(routing, Routing::OFFS);
+    a.pos_to_row = r.part(routing, Routing::POS_TO_ROW), a.row_to_pos = r.part(routing, Routing::ROW_TO_POS);
+    a.xp = (const uint16_t*)base, a.gu = base + kept.gu, a.act = (const uint16_t*)(base + kept.act);
+    a.w1 = bf(w[0]), a.w3 = bf(w[1]), a.w2 = bf(w[2]);
+    for (int i = 0; i < 3; ++i) {
+      a.dw[i] = ptr(wg.into[i]);
+      a.dw_dtype[i] = wg.into[i].defined() ? dt(wg.into[i]) : 0;
+      a.dw_accumulate[i] = wg.add[i];
+    }
+    if (dlogits.defined()) a.dlogits = dlogits.data_ptr(), a.dlogits_dtype = dt(dlogits);
+    a.dgates = (float*)ptr(dgates);
+    a.wr = bf(wrb), a.xn = bf(xn);
+    if (dwr.defined()) a.dwr = dwr.data_ptr(), a.dwr_dtype = dt(dwr);
+    if (dx.defined()) a.dx = dx.data_ptr(), a.dx_dtype = dt(dx);
+    a.dxp = (uint16_t*)ptr(dxp);
+    a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
+    check(moe_layer_backward(&a, s), "moe_layer_backward");
+    for (int i = 0; i < 3; ++i)
+      if (wg.fresh[i].defined()) params[i].mutable_grad() = wg.fresh[i];
+    if (dwr.defined() && !wr_direct) dwr = dwr.to(type(6));
+
+    if (by_hand) {
+      const NoAutocast off;
+      const auto logit_gradient = [&](at::ScalarType t) {
+        Tensor d = empty({T, E}, t, kept_buf);
+        CALL(moe_router_topk_bwd, gates, (const float*)ptr(dgates), ids, T, E, k, ptr(d), (int)dt(t), s);
+        return d;
+      };
+      const at::ScalarType logit_type = has_logits ? type(7) : at::kBFloat16;
+      if (want_bias) {
+        // the bias is a per-expert constant added to the logits (in fp32): its gradient is the column
+        // sum of the logits' gradient, taken before that is rounded
+        Tensor d32 = logit_gradient(at::kFloat);
+        if (ext.defined()) d32 = d32 + ext.to(at::kFloat);
+        dbias = d32.sum(0);
+        dlogits = d32.to(logit_type);
+      } else {
+        dlogits = logit_gradient(logit_type);
+        dlogits = dlogits + ext.to(logit_type);
+      }
+      if (has_router) {
+        if (want_wr) dwr = router_wgrad(dlogits, xn, type(6));
+        if (want_dx) {
+          d2 = at::mm(dlogits, wrb);
+          dx = empty({T, H}, x_type, kept_buf);
+          // (with the norm, the router's share joins inside the norm's backward kernel)
+          if (has_norm || T == 0)
+            CALL(moe_permute_bwd, bf(dxp), r.part(routing, Routing::ROW_TO_POS), nullptr, T, H, k, ptr(dx), (int)dt(dx), s);
+          else
+            CALL(moe_permute_bwd_addend, bf(dxp), r.part(routing, Routing::ROW_TO_POS), d2.data_ptr(), (int)dt(d2), T, H, k,
+                 ptr(dx), (int)dt(dx), s);
+        }
+      }
+      if (!want_logits) dlogits = Tensor();
+    }
+    if (want_dx && has_norm) {
+      const int64_t nb = std::max<int64_t>(moe_rmsnorm_bwd_workspace_bytes(T, H), 16);
+      const Tensor ws = empty({nb}, at::kByte, kept_buf);
+      const Tensor d1 = dx;
+      dx = empty({T, H}, x_type, kept_buf);
+      dnw = empty({H}, at::kFloat, kept_buf);
+      CALL(moe_rmsnorm_bwd, x.data_ptr(), (int)dt(x), nw.data_ptr<float>(), rstd.data_ptr<float>(), d1.data_ptr(),
+           (int)dt(d1), bf(d2), add_residual ? dout.data_ptr() : nullptr, T, H, dx.data_ptr(), dnw.data_ptr<float>(),
+           ws.data_ptr(), nb, s);
+      dnw = need(NORM) ? dnw.to(type(5)) : Tensor();
+    } else if (want_dx && add_residual) {
+      dx = dx + dout;
+    }
+    if (!need(X)) dx = Tensor();
+    variable_list out(INPUTS);
+    out[X] = dx, out[NORM] = dnw, out[WR] = dwr, out[LOGITS] = dlogits, out[BIAS] = dbias;
+    out[W1] = wg.give[0], out[W3] = wg.give[1], out[W2] = wg.give[2];
+    return out;
+  }
+};
+
+// -> (out, logits if the router product is inside, routing words if asked for)
+std::tuple<Tensor, OptTensor, OptTensor> layer(const Tensor& x, const OptTensor& norm_w, const OptTensor& wr,
+                                               const OptTensor& logits, const OptTensor& ids, const Tensor& w1,
+                                               const Tensor& w3, const Tensor& w2, const OptTensor& bias,
+                                               const OptTensor& s1, const OptTensor& s3, const OptTensor& s2, int64_t k,
+                                               double eps, bool add_residual, bool fused_router, bool accumulate,
+                                               bool want_routing) {
+  const Tensor &n = value(norm_w), &r = value(wr), &l = value(logits), &b = value(bias), &i = value(ids);
+  Layer o;
+  o.k = k, o.eps = eps, o.add_residual = add_residual, o.fused_router = fused_router, o.accumulate = accumulate;
+  o.s1 = s1, o.s3 = s3, o.s2 = s2;
+  Tensor routing;
+  if (want_routing) o.routing_out = &routing;
+  if (at::GradMode::is_enabled())
+    for (const Tensor* p : {&x, &n, &r, &l, &w1, &w3, &w2, &b}) o.train = o.train || (p->defined() && p->requires_grad());
+  Tensor out, lg;
+  if (o.train) {
+    const variable_list v = LayerNode::apply(x, norm_w, wr, logits, w1, w3, w2, bias, ids, o);
+    out = v[0];
+    if (v.size() > 1) lg = v[1];
+  } else {
+    const at::NoGradGuard off;
+    const Outputs f = forward(o, x, n, r, l, w1, w3, w2, b, i);
+    out = f.out;
+    if (r.defined()) lg = f.logits;
+  }
+  return {out, lg.defined() ? OptTensor(lg) : std::nullopt, want_routing ? OptTensor(routing) : std::nullopt};
+}
+
+
+// ---- the layer in fp32 (model/modules/mlp.py:101-167 with fp32 operands and no autocast) --------------
+
+// Kept for the backward pass: xp [R,H], g, u, act [R,I], y [R,H] (y with logits only: the gate gradient
+// reads it), all fp32.
+struct KeptF32 {
+  int64_t g, u, act, y, total;
+  KeptF32(int64_t R, int64_t H, int64_t I) {
+    const int64_t rh = up(R * H, 64), ri = up(R * I, 64);
+    g = rh, u = g + ri, act = u + ri, y = act + ri, total = y + rh;
+    if (total == 0) total = 64;
+  }
+};
+
+struct OutputsF32 {
+  Tensor out, routing, kept, w[3];
+};
+
+OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, const Tensor& w1, const Tensor& w3,
+                       const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
+  OutputsF32 f;
+  const Tensor x = dense(x_);
+  const c10::DeviceGuard guard(x.device());
+  const int64_t T = x.size(0), H = x.size(1), E = w1.size(0), I = w1.size(1), k = o.k, R = T * k;
+  TORCH_CHECK(w3.size(0) == E && w2.size(0) == E && w1.size(2) == H && w3.size(2) == H && w3.size(1) == I &&
+                  w2.size(1) == H && w2.size(2) == I && (!logits_.defined() || logits_.size(1) == E),
+              "the weights' shapes do not belong together");
+  f.w[0] = dense(w1), f.w[1] = dense(w3), f.w[2] = dense(w2);
+  void* s = stream_of(x);
+  const Routing r(R, E);
+  f.routing = empty({r.at[Routing::PARTS]}, at::kInt, x);
+  f.out = empty({T, H}, at::kFloat, x);
+  const KeptF32 kept(R, H, I);
+  f.kept = empty({kept.total}, at::kFloat, x);
+  float* base = f.kept.data_ptr<float>();
+  float *xp = base, *g = base + kept.g, *u = base + kept.u, *act = base + kept.act, *y = base + kept.y;
+  float* gates = nullptr;
+  const int32_t* ids = r.part(f.routing, Routing::IDS);
+  int32_t* bad = nullptr;
+  Tensor given;
+  if (logits_.defined()) {
+    const Tensor logits = dense(logits_), b = bias.defined() ? dense(bias) : Tensor();
+    gates = (float*)r.part(f.routing, Routing::GATES);
+    CALL(moe_router_topk_fwd, logits.data_ptr(), (int)dt(logits), (const float*)ptr(b), T, E, k,
+         r.part(f.routing, Routing::IDS), gates, s);
+  } else {
+    given = dense(ids_.to(at::kInt));
+    TORCH_CHECK(given.numel() == R, "one expert id per row is needed");
+    ids = given.data_ptr<int32_t>();
+    bad = r.part(f.routing, Routing::BAD);
+  }
+  const int64_t wsb = std::max<int64_t>(moe_dispatch_workspace_bytes(R, E), 16);
+  const Tensor ws = empty({wsb}, at::kByte, x);
+  const int32_t* offs = r.part(f.routing, Routing::OFFS);
+  const int32_t* p2r = r.part(f.routing, Routing::POS_TO_ROW);
+  const int32_t* r2p = r.part(f.routing, Routing::ROW_TO_POS);
+  CALL(moe_histogram_scan_checked, ids, R, E, r.part(f.routing, Routing::COUNTS), r.part(f.routing, Routing::OFFS),
+       r.part(f.routing, Routing::POS_TO_ROW), r.part(f.routing, Routing::ROW_TO_POS), bad, ws.data_ptr(), wsb, s);
+  CALL(moe_f32_gather_rows, x.data_ptr<float>(), p2r, T, R, H, k, xp, s);
+  CALL(moe_f32_gemm_rows, xp, f.w[0].data_ptr<float>(), offs, E, R, I, H, 1, g, 0, s);
+  CALL(moe_f32_gemm_rows, xp, f.w[1].data_ptr<float>(), offs, E, R, I, H, 1, u, 0, s);
+  CALL(moe_f32_swiglu_fwd, g, u, R * I, act, s);
+  CALL(moe_f32_gemm_rows, act, f.w[2].data_ptr<float>(), offs, E, R, H, I, 1, y, 0, s);
+  CALL(moe_f32_combine_fwd, y, gates, r2p, T, H, k, f.out.data_ptr<float>(), s);
+  if (o.routing_out) *o.routing_out = f.routing;
+  return f;
+}
+
+struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
+  enum Input { X, LOGITS, W1, W3, W2, BIAS, IDS, OPTIONS, INPUTS };
+
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& logits_, const Tensor& w1,
+                               const Tensor& w3, const Tensor& w2, const OptTensor& bias_, const OptTensor& ids_,
+                               const Layer& o) {
+    const Tensor &logits = value(logits_), &bias = value(bias_), &ids = value(ids_);
+    const OutputsF32 f = forward_f32(o, x, logits, w1, w3, w2, bias, ids);
+    ctx->save_for_backward({f.kept, f.routing, f.w[0], f.w[1], f.w[2]});
+    ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), o.k, logits.defined(),
+                                                Present{true, logits.defined(), true, true, true, bias.defined(),
+                                                        ids.defined()}.mask};
+    ctx->set_materialize_grads(false);
+    return {f.out};
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    first_order_only();
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &kept_buf = saved[0], &routing = saved[1], &w1 = saved[2], &w3 = saved[3], &w2 = saved[4];
+    const std::vector<int64_t> ints = ctx->saved_data["i"].toIntVector();
+    const int64_t T = ints[0], k = ints[1], R = T * k, E = w1.size(0), I = w1.size(1), H = w1.size(2);
+    const bool routed = ints[2];
+    const c10::DeviceGuard guard(kept_buf.device());
+    Present present;
+    present.mask = ints[3];
+    const auto need = [&](Input i) { return present.wants_gradient(ctx, i); };
+    const bool want_gates = routed && (need(LOGITS) || need(BIAS));
+    const Tensor dout = grads[0].defined() ? dense(grads[0].to(at::kFloat)) : at::zeros({T, H}, kept_buf.options());
+    const Routing r(R, E);
+    const KeptF32 kept(R, H, I);
+    const float* base = kept_buf.data_ptr<float>();
+    const float *xp = base, *g = base + kept.g, *u = base + kept.u, *act = base + kept.act, *y = base + kept.y;
+    const float* gates = routed ? (const float*)r.part(routing, Routing::GATES) : nullptr;
+    const int32_t* offs = r.part(routing, Routing::OFFS);
+    const int32_t* p2r = r.part(routing, Routing::POS_TO_ROW);
+    const int32_t* r2p = r.part(routing, Routing::ROW_TO_POS);
+    void* s = stream_of(kept_buf);
+    const int64_t rh = up(R * H, 64), ri = up(R * I, 64);
+    const Tensor scratch = empty({2 * rh + 3 * ri + up(R, 64) + 64}, at::kFloat, kept_buf);
+    float* dyp = scratch.data_ptr<float>();
+    float *dxp = dyp + rh, *dact = dxp + rh, *dg = dact + ri, *du = dg + ri, *dgates = du + ri;
+    CALL(moe_f32_combine_bwd, dout.data_ptr<float>(), want_gates ? y : nullptr, gates, p2r, T, R, H, k, dyp,
+         want_gates ? dgates : nullptr, s);
+    CALL(moe_f32_gemm_rows, dyp, w2.data_ptr<float>(), offs, E, R, I, H, 0, dact, 0, s);
+    CALL(moe_f32_swiglu_bwd, dact, g, u, R * I, dg, du, s);
+    Tensor dx, dw1, dw3, dw2, dlogits, dbias;
+    if (need(X)) {
+      dx = empty({T, H}, at::kFloat, kept_buf);
+      CALL(moe_f32_gemm_rows, dg, w1.data_ptr<float>(), offs, E, R, H, I, 0, dxp, 0, s);
+      CALL(moe_f32_gemm_rows, du, w3.data_ptr<float>(), offs, E, R, H, I, 0, dxp, 1, s);
+      CALL(moe_f32_permute_bwd, dxp, r2p, T, H, k, dx.data_ptr<float>(), s);
+    }
+    const auto wgrad = [&](const float* a, const float* b, int64_t M, int64_t N) {
+      Tensor dw = empty({E, M, N}, at::kFloat, kept_buf);
+      CALL(moe_f32_gemm_wgrad, a, b, offs, E, R, M, N, dw.data_ptr<float>(), 0, s);
+      return dw;
+    };
+    if (need(W1)) dw1 = wgrad(dg, xp, I, H);
+    if (need(W3)) dw3 = wgrad(du, xp, I, H);
+    if (need(W2)) dw2 = wgrad(dyp, act, H, I);
+    if (want_gates) {
+      dlogits = empty({T, E}, at::kFloat, kept_buf);
+      CALL(moe_router_topk_bwd, gates, dgates, r.part(routing, Routing::IDS), T, E, k, dlogits.data_ptr(), MOE_DT_F32, s);
+      if (need(BIAS)) dbias = dlogits.sum(0);
+      if (!need(LOGITS)) dlogits = Tensor();
+    }
+    variable_list out(INPUTS);
+    out[X] = dx, out[LOGITS] = dlogits, out[W1] = dw1, out[W3] = dw3, out[W2] = dw2, out[BIAS] = dbias;
+    return out;
+  }
+};
+
+// -> (out, routing words if asked for)
+std::tuple<Tensor, OptTensor> layer_f32(const Tensor& x, const OptTensor& logits, const OptTensor& ids, const Tensor& w1,
+                                        const Tensor& w3, const Tensor& w2, const OptTensor& bias, int64_t k,
+                                        bool want_routing) {
+  const Tensor &l = value(logits), &b = value(bias), &i = value(ids);
+  Layer o;
+  o.k = k;
+  Tensor routing;
+  if (want_routing) o.routing_out = &routing;
+  if (at::GradMode::is_enabled())
+    for (const Tensor* p : {&x, &l, &w1, &w3, &w2, &b}) o.train = o.train || (p->defined() && p->requires_grad());
+  Tensor out;
+  if (o.train) {
+    out = LayerF32Node::apply(x, logits, w1, w3, w2, bias, ids, o)[0];
+  } else {
+    const at::NoGradGuard off;
+    out = forward_f32(o, x, l, w1, w3, w2, b, i).out;
+  }
+  return {out, want_routing ? OptTensor(routing) : std::nullopt};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  static py::object error_type;
+  m.def("set_error_type", [](py::object t) { error_type = std::move(t); });
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const LibError& e) {
+      PyErr_SetString(error_type ? error_type.ptr() : PyExc_RuntimeError, e.what());
+    }
+  });
+  m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
+  m.def("layer_f32", &layer_f32, py::call_guard<py::gil_scoped_release>());
+}

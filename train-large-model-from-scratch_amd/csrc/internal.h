@@ -3,6 +3,9 @@
 #pragma once
 #include "common.h"
 
+// Tells the installed launch observer, if any, about one launch (layer.hip).
+void moe_observe(const char* name, int after);
+
 // Compute units of the current GPU (asked of the runtime once).
 int moe_compute_units();
 

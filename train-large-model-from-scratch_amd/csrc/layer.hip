@@ -20,12 +20,12 @@ namespace {
 moe_launch_observer_fn g_observer = nullptr;
 
 // Enqueues one step and tells the observer about it; leaves the calling function on an error.
-#define MOE_STEP(name, call)              \
-  do {                                    \
-    if (g_observer) g_observer(name, 0);  \
-    const int rc_ = (call);               \
-    if (g_observer) g_observer(name, 1);  \
-    if (rc_) return rc_;                  \
+#define MOE_STEP(name, call)    \
+  do {                          \
+    moe_observe(name, 0);       \
+    const int rc_ = (call);     \
+    moe_observe(name, 1);       \
+    if (rc_) return rc_;        \
   } while (0)
 
 constexpr int64_t ALIGN = 256;
@@ -112,6 +112,10 @@ extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, i
   MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_fwd(act, w2, offs, E, R, H, I, y, stream));
   MOE_STEP("moe_combine_fwd", moe_combine_fwd(y, gates, row_to_pos, T, H, k, out, out_dtype, stream));
   return 0;
+}
+
+void moe_observe(const char* name, int after) {
+  if (g_observer) g_observer(name, after);
 }
 
 extern "C" void moe_set_launch_observer(moe_launch_observer_fn fn) { g_observer = fn; }

@@ -2,10 +2,11 @@
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
-from .build import LIB_PATH
+from .build import LIB_PATH, NATIVE_PATH
 
 _vp, _i64, _int = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
 _args = ctypes.c_char_p                                       # an argument structure, packed
@@ -141,6 +142,7 @@ class MoELib:
 
 _lock = threading.Lock()
 _lib: MoELib | None = None
+_native = None
 
 
 def load() -> MoELib:
@@ -157,3 +159,21 @@ def load() -> MoELib:
             import torch  # noqa: F401  -- makes sure torch's HIP runtime is the one in the process
             _lib = MoELib(LIB_PATH)
         return _lib
+
+
+def native():
+    """The module with the autograd nodes (_native.so), on top of the library."""
+    global _native
+    if _native is not None:
+        return _native
+    load()
+    with _lock:
+        if _native is None:
+            if not os.path.exists(NATIVE_PATH):
+                raise MoELibError(f"{NATIVE_PATH} is not built; run `python __graft_entry__.py` first")
+            spec = importlib.util.spec_from_file_location("_native", NATIVE_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            module.set_error_type(MoELibError)
+            _native = module
+        return _native

@@ -5,7 +5,6 @@ Every function requires CUDA(HIP) tensors; nothing here computes on the host.
 """
 from __future__ import annotations
 
-import functools
 import struct
 
 import torch
@@ -325,22 +324,18 @@ def rmsnorm_router_supported(H: int, E: int, k: int) -> bool:
     return bool(_lib.load().cdll.moe_rmsnorm_router_supported(H, E, k))
 
 
-def rmsnorm_router_fwd(x: torch.Tensor, weight: torch.Tensor, eps: float, router_weight: torch.Tensor, k: int,
-                       routing=None):
+def rmsnorm_router_fwd(x: torch.Tensor, weight: torch.Tensor, eps: float, router_weight: torch.Tensor, k: int):
     """RMSNorm, router product and top-k in one kernel: x [T,H], norm weight fp32 [H], router
     weight bf16 [E,H] -> xn bf16 [T,H], rstd fp32 [T], logits bf16 [T,E], ids int32 [T*k],
-    gates fp32 [T*k] (both in `routing` if that is given)."""
+    gates fp32 [T*k]."""
     T, H = x.shape
     E = router_weight.shape[0]
     dev = x.device
     xn = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
     rstd = torch.empty(T, dtype=torch.float32, device=dev)
     logits = torch.empty(T, E, dtype=torch.bfloat16, device=dev)
-    if routing is not None:
-        ids, gates = routing.ids, routing.gates
-    else:
-        ids = torch.empty(T * k, dtype=torch.int32, device=dev)
-        gates = torch.empty(T * k, dtype=torch.float32, device=dev)
+    ids = torch.empty(T * k, dtype=torch.int32, device=dev)
+    gates = torch.empty(T * k, dtype=torch.float32, device=dev)
     _lib.load().call("moe_rmsnorm_router_fwd", _p(x), _dt(x), _p(weight), float(eps), _p(router_weight), T, H, E, k,
                      _p(xn), _p(rstd), _p(logits), _p(ids), _p(gates), _stream())
     return xn, rstd, logits, ids, gates
@@ -385,21 +380,6 @@ def cast_bf16(w: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def ffn_forward(x: torch.Tensor, logits: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor, w2: torch.Tensor,
-                k: int, bias: torch.Tensor | None = None, out_dtype: torch.dtype | None = None) -> torch.Tensor:
-    """The layer body's forward pass in one call of the library (no intermediate is kept): x [T,H]
-    bf16/fp32, logits [T,E] bf16/fp32, bf16 weights -> out [T,H] of `out_dtype` (default: x's)."""
-    T, H = x.shape
-    E, I = w1.shape[0], w1.shape[1]
-    L = _lib.load()
-    out = torch.empty(T, H, dtype=out_dtype or x.dtype, device=x.device)
-    nbytes = L.cdll.moe_ffn_forward_workspace_bytes(T, H, E, I, k)
-    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=x.device)
-    L.call_layer("moe_ffn_forward", _p(x), _dt(x), _p(logits), _dt(logits), _p(bias), _p(w1), _p(w3), _p(w2),
-           T, H, E, I, k, _p(out), _dt(out), _p(ws), ws.numel(), _stream())
-    return out
-
-
 def router_wgrad(dlogits: torch.Tensor, x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """dlogits^T x for bf16 dlogits [T,E], x [T,H] (E and H multiples of 8) -> [E,H]."""
     T, H = x.shape
@@ -417,20 +397,6 @@ _FORWARD_ARGS = struct.Struct("<29q")
 _BACKWARD_ARGS = struct.Struct("<39q")
 
 
-@functools.lru_cache(maxsize=512)
-def _layer_sizes(T: int, H: int, E: int, I: int, k: int, device_index: int):
-    """Bytes of (forward scratch, backward scratch, blocked g/u) and the int32 offsets of the routing
-    buffer's parts: ids, gates, counts, offs, pos_to_row, row_to_pos, bad, total."""
-    c = _lib.load().cdll
-    R = T * k
-    at, offsets = 0, []
-    for n in (R, R, E, E + 1, R, R, 1):
-        offsets.append(at)
-        at += (n + 63) // 64 * 64
-    return (max(c.moe_layer_scratch_bytes(T, H, E, I, k, 0), 256), max(c.moe_layer_scratch_bytes(T, H, E, I, k, 1), 256),
-            max(c.moe_gu_blocked_bytes(R, E, I), 16), (*offsets, at))
-
-
 class RoutingTensors:
     """The integer tensors (and gates) of one routed batch as tensors of their own."""
 
@@ -439,104 +405,62 @@ class RoutingTensors:
         R = T * k
         self.ids, self.counts, self.offs = i32(R), i32(E), i32(E + 1)
         self.gates = torch.empty(R, dtype=torch.float32, device=device)
-        self.pos_to_row, self.row_to_pos, self.bad_ids = i32(R), i32(R), i32(1)
-
-    def pointers(self):
-        return [t.data_ptr() for t in (self.ids, self.gates, self.counts, self.offs, self.pos_to_row,
-                                       self.row_to_pos, self.bad_ids)]
+        self.pos_to_row, self.row_to_pos = i32(R), i32(R)
 
 
 class Routing:
-    """The integer tensors (and gates) of one routed batch, in one allocation."""
-    __slots__ = ("buf", "R", "E", "offsets")
+    """The same as parts of one buffer of 32-bit words, each beginning at a multiple of 64 words: how a
+    call of the layer leaves them (csrc/binding.cpp)."""
 
-    def __init__(self, buf, R, E, offsets):
-        self.buf, self.R, self.E, self.offsets = buf, R, E, offsets
-
-    def part(self, i, n):
-        return self.buf.narrow(0, self.offsets[i], n)
-
-    def pointers(self):
-        base = self.buf.data_ptr()
-        return [base + 4 * o for o in self.offsets[:7]]
-
-    ids = property(lambda s: s.part(0, s.R))
-    gates = property(lambda s: s.part(1, s.R).view(torch.float32))
-    counts = property(lambda s: s.part(2, s.E))
-    offs = property(lambda s: s.part(3, s.E + 1))
-    pos_to_row = property(lambda s: s.part(4, s.R))
-    row_to_pos = property(lambda s: s.part(5, s.R))
-    bad_ids = property(lambda s: s.part(6, 1))
+    def __init__(self, buf: torch.Tensor, R: int, E: int):
+        at, parts = 0, []
+        for n in (R, R, E, E + 1, R, R, 1):
+            parts.append(buf.narrow(0, at, n))
+            at += (n + 63) // 64 * 64
+        self.ids, gates, self.counts, self.offs, self.pos_to_row, self.row_to_pos, self.bad_ids = parts
+        self.gates = gates.view(torch.float32)
 
 
-def new_routing(T: int, H: int, E: int, I: int, k: int, device, buf: torch.Tensor | None = None) -> Routing:
-    """A fresh one, or (`buf`) the one that lives in a buffer made here earlier for the same sizes."""
-    offsets = _layer_sizes(T, H, E, I, k, device.index)[3]
-    if buf is None:
-        buf = torch.empty(offsets[7], dtype=torch.int32, device=device)
-    return Routing(buf, T * k, E, offsets)
-
-
-def layer_forward(x, w1, w3, w2, k: int, routing, out_dtype, logits=None, bias=None, ids=None,
-                  residual=None, train: bool = True):
-    """The layer body (routing to combine) in one call -> (out [T,H], xp, gu, act).  With `logits` the
-    routing is worked out from them; with `ids` (k = 1, rows already dispatched) only their order is, and
-    all gates are 1; with neither, `routing` already holds ids and gates.  g and u are kept (`gu`) when a
-    backward pass will follow (`train`)."""
+def layer_forward(x, logits, w1, w3, w2, k: int, train: bool, out_dtype: torch.dtype | None = None):
+    """The layer body (routing to combine) in one call -> (out [T,H], routing, xp, gu, act).  g and u are
+    kept (`gu`, else None) when a backward pass will follow."""
     T, H = x.shape
     E, I, _ = w1.shape
-    dev = x.device
-    scratch_bytes, _, gu_bytes, _ = _layer_sizes(T, H, E, I, k, dev.index)
-    bf16 = torch.bfloat16
-    out = torch.empty((T, H), dtype=out_dtype, device=dev)
+    dev, bf16 = x.device, torch.bfloat16
+    L = _lib.load()
+    r = RoutingTensors(T, E, k, dev)
+    out = torch.empty((T, H), dtype=out_dtype or x.dtype, device=dev)
     xp = torch.empty((T * k, H), dtype=bf16, device=dev)
     act = torch.empty((T * k, I), dtype=bf16, device=dev)
-    gu = torch.empty(gu_bytes, dtype=torch.uint8, device=dev) if train else None
-    scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=dev)
-    pids, pgates, pcounts, poffs, pp2r, pr2p, pbad = routing.pointers()
-    ids64 = 0
-    if ids is not None:
-        pgates = 0
-        if ids.dtype == torch.int64:
-            ids64 = _p(ids)
-        else:
-            pids = _p(ids)
-    args = _FORWARD_ARGS.pack(
-        T, H, E, I, k, _p(x), _dt(x), _p(logits) or 0, _dt(logits) if logits is not None else 0, _p(bias) or 0,
-        ids64, _p(w1), _p(w3), _p(w2), _p(residual) or 0, out.data_ptr(), DT_BF16 if out_dtype == bf16 else DT_F32,
-        pids, pgates, pcounts, poffs, pp2r, pr2p, pbad if ids is not None else 0, xp.data_ptr(),
-        gu.data_ptr() if train else 0, act.data_ptr(), scratch.data_ptr(), scratch_bytes)
-    _lib.load().call_layer("moe_layer_forward", args, _stream())
-    return out, xp, gu, act
-
-
-def layer_backward(dout, T: int, k: int, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1, w3, w2,
-                   dw=(None, None, None), dw_accumulate=(False, False, False), dlogits=None, dgates=None, wr=None,
-                   xn=None, dwr=None, dx=None, dxp=None):
-    """The backward of layer_forward in one call.  The routing arguments are pointers or tensors; `gates` and
-    `ids` may be None where there are none.  Every result goes into the tensor given for it and is left out
-    where None is: dw (gradients of w1, w3, w2, bf16 or fp32, added to if dw_accumulate), dlogits [T,E],
-    dgates [R] (instead of everything further down the router), dwr with xn (router weight), dx [T,H] (with
-    `wr` the router's share included, unless dgates is asked for), dxp [T*k,H]."""
-    R, H = xp.shape
-    E, I, _ = w1.shape
-    dev = xp.device
-    nbytes = _layer_sizes(T, H, E, I, k, dev.index)[1]
+    gu = torch.empty(max(L.cdll.moe_gu_blocked_bytes(T * k, E, I), 16), dtype=torch.uint8, device=dev) if train else None
+    nbytes = max(L.cdll.moe_layer_scratch_bytes(T, H, E, I, k, 0), 256)
     scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    args = _FORWARD_ARGS.pack(
+        T, H, E, I, k, _p(x), _dt(x), _p(logits), _dt(logits), 0, 0, _p(w1), _p(w3), _p(w2), 0, _p(out), _dt(out),
+        _p(r.ids), _p(r.gates), _p(r.counts), _p(r.offs), _p(r.pos_to_row), _p(r.row_to_pos), 0, _p(xp), _p(gu) or 0,
+        _p(act), _p(scratch), nbytes)
+    L.call_layer("moe_layer_forward", args, _stream())
+    return out, r, xp, gu, act
 
-    def ptr(t):
-        return t if isinstance(t, int) else _p(t) or 0
 
-    def dt(t):
-        return 0 if t is None else _dt(t)
-
-    d1, d3, d2 = dw
+def layer_backward(dout, k: int, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1, w3, w2, dw, dlogits=None,
+                   dgates=None, wr=None, xn=None, dwr=None, dx=None, dxp=None):
+    """The backward of layer_forward in one call.  Every result goes into the tensor given for it and is left
+    out where None is: dw (gradients of w1, w3, w2), dlogits [T,E], dgates [R] (instead of everything further
+    down the router), dwr with xn (router weight), dx [T,H] (with `wr` the router's share included, unless
+    dgates is asked for), dxp [T*k,H]."""
+    T, H = dout.shape
+    E, I, _ = w1.shape
+    L = _lib.load()
+    nbytes = max(L.cdll.moe_layer_scratch_bytes(T, H, E, I, k, 1), 256)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=xp.device)
+    ptr = lambda t: _p(t) or 0
+    dt = lambda t: 0 if t is None else _dt(t)
     args = _BACKWARD_ARGS.pack(
-        T, H, E, I, k, _p(dout), _dt(dout), ptr(gates), ptr(ids), ptr(offs), ptr(pos_to_row), ptr(row_to_pos),
-        xp.data_ptr(), gu.data_ptr(), act.data_ptr(), _p(w1), _p(w3), _p(w2), ptr(d1), ptr(d3), ptr(d2),
-        dt(d1), dt(d3), dt(d2), *(1 if a else 0 for a in dw_accumulate), ptr(dlogits), dt(dlogits), ptr(dgates),
-        ptr(wr), ptr(xn), ptr(dwr), dt(dwr), ptr(dx), dt(dx), ptr(dxp), scratch.data_ptr(), nbytes)
-    _lib.load().call_layer("moe_layer_backward", args, _stream())
+        T, H, E, I, k, _p(dout), _dt(dout), *map(ptr, (gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1, w3, w2)),
+        *map(ptr, dw), *map(dt, dw), 0, 0, 0, ptr(dlogits), dt(dlogits), ptr(dgates), ptr(wr), ptr(xn), ptr(dwr),
+        dt(dwr), ptr(dx), dt(dx), ptr(dxp), _p(scratch), nbytes)
+    L.call_layer("moe_layer_backward", args, _stream())
 
 
 # ---- the path in fp32 (layer called without autocast on fp32 tensors) ---------------------------

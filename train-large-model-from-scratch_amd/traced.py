@@ -54,8 +54,7 @@ def ffn_fwd(x: Tensor, logits: Tensor, w1: Tensor, w3: Tensor, w2: Tensor, k: in
     E = logits.shape[1]
     x, logits = ops.dense(x), ops.dense(logits)
     wb = [ops.dense(w) if w.dtype == _BF16 else ops.cast_bf16(ops.dense(w)) for w in (w1, w3, w2)]
-    r = ops.RoutingTensors(T, E, k, x.device)
-    out, xp, gu, act = ops.layer_forward(x, *wb, k, r, x.dtype, logits=logits, train=train)
+    out, r, xp, gu, act = ops.layer_forward(x, logits, *wb, k, train)
     copies = [b if w.dtype != _BF16 else _empty(x) for w, b in zip((w1, w3, w2), wb)]
     return (out, r.ids, r.gates, r.offs, r.pos_to_row, r.row_to_pos, xp, gu if train else _empty(x, torch.uint8), act,
             *copies)
@@ -89,7 +88,7 @@ def ffn_bwd(dout: Tensor, xp: Tensor, gu: Tensor, act: Tensor, gates: Tensor,
     dx = dout.new_empty(T, H, dtype=f32 if x_is_f32 else _BF16)
     dlogits = dout.new_empty(T, E, dtype=f32 if logits_is_f32 else _BF16)
     dw = [torch.empty_like(w, dtype=f32 if w_is_f32 else _BF16) for w in (w1b, w3b, w2b)]
-    ops.layer_backward(dout, T, k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b, dw,
+    ops.layer_backward(dout, k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b, dw,
                        dlogits=dlogits, dx=dx)
     return dx, dlogits, *dw
 
@@ -153,8 +152,7 @@ def routed_fwd(x: Tensor, wr: Tensor, w1: Tensor, w3: Tensor, w2: Tensor, k: int
     wrb = ops.dense(wr.detach().to(_BF16))
     with torch.autocast("cuda", enabled=False):
         logits = xn @ wrb.t()
-    r = ops.RoutingTensors(T, E, k, x.device)
-    out, xp, gu, act = ops.layer_forward(xn, *wb, k, r, x.dtype, logits=logits, train=train)
+    out, r, xp, gu, act = ops.layer_forward(xn, logits, *wb, k, train, x.dtype)
     copies = [b if w.dtype != _BF16 else _empty(x) for w, b in zip((w1, w3, w2), wb)]
     if not train:
         return (out, logits, r.ids, r.gates, r.offs, r.pos_to_row, r.row_to_pos, _empty(x), _empty(x), _empty(x),
@@ -194,7 +192,7 @@ def routed_bwd(dout: Tensor, dlogits_ext: Tensor | None, xn: Tensor, wrb: Tensor
     if dout.dtype != xdt:
         dout = dout.to(xdt)
     dw = [torch.empty_like(w, dtype=f32 if w_is_f32 else _BF16) for w in (w1b, w3b, w2b)]
-    saved = (dout, T, k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b, dw)
+    saved = (dout, k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b, dw)
     if dlogits_ext is None:
         dx = dout.new_empty(T, H)
         dwr = torch.empty_like(wrb, dtype=f32 if wr_is_f32 else _BF16)
