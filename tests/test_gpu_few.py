@@ -1,0 +1,40 @@
+"""The kernels for few tokens (a forward without gradients of at most 64): against the oracle at the edges
+of their blocks of 16 rows, 16 columns and 32-deep steps, and at the ends of their range."""
+import pytest
+import torch
+
+from _tol import check
+from oracle import moe_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,E,k,H,I,x_dt", [
+    (1, 64, 8, 256, 136, torch.bfloat16),    # one token: the kernel that also combines
+    (1, 4, 3, 2056, 1032, torch.float32),    # ... contractions that end inside a step, experts' shares split
+    (1, 40, 33, 64, 64, torch.bfloat16),     # ... more experts a token than that kernel takes
+    (2, 128, 1, 520, 8, torch.float32),
+    (16, 4, 4, 136, 248, torch.bfloat16),    # every expert has 16 rows
+    (17, 4, 4, 136, 248, torch.bfloat16),    # ... 17
+    (33, 3, 3, 1032, 72, torch.float32),     # ... 33
+    (64, 2, 2, 4104, 40, torch.bfloat16),    # ... 64; shares of the contraction too long for registers
+    (48, 130, 8, 264, 520, torch.bfloat16),  # more experts than the router kernel takes
+])
+def test_forward_of_few_tokens_matches_the_oracle(pkg, lib, T, E, k, H, I, x_dt):
+    print("few tokens", T, E, k, H, I, x_dt, flush=True)
+    g = torch.Generator().manual_seed(T * 1000 + E)
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(torch.bfloat16)
+    x, wr, w1, w3, w2 = r(T, H), r(E, H, std=0.3), r(E, I, H, std=0.05), r(E, I, H, std=0.05), r(E, H, I, std=0.05)
+    xd = x.cuda().to(x_dt)
+    ws = [w.cuda() for w in (w1, w3, w2)]
+    bias = torch.randn(E, generator=g) if T % 2 else None
+    with torch.no_grad():
+        out, logits = pkg.routed_moe(xd, wr.cuda(), *ws, k, bias=None if bias is None else bias.cuda())
+        given = pkg.moe_ffn(xd, logits, *ws, k, bias=None if bias is None else bias.cuda())
+    assert out.dtype == x_dt and torch.equal(out, given)
+    lg = logits.cpu()
+    check("logits", lg, x.float() @ wr.float().t(), (x.float() @ wr.float().t()).bfloat16().float())
+    sel = lg.float() + bias if bias is not None else lg
+    f = O.moe_forward(x, wr, w1, w3, w2, k, logits=sel)
+    fe = O.moe_forward(x, wr, w1, w3, w2, k, logits=sel, emulate_bf16=True)
+    check("out", out, f["out"], fe["out"])

@@ -17,7 +17,14 @@
 
 #include "moe_gfx950.h"
 
-void moe_observe(const char* name, int after);  // (internal.h, which only device code can include)
+// (from internal.h and layer.hip, which only device code can include)
+void moe_observe(const char* name, int after);
+bool moe_router_few_ok(int64_t T, int64_t H, int64_t E, int64_t k);
+int moe_router_logits(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
+                      void* stream);
+int moe_routed_forward(const uint16_t* x, const uint16_t* wr, uint16_t* logits, const float* bias, const uint16_t* w1,
+                       const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k,
+                       void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
 using at::Tensor;
 using torch::autograd::AutogradContext;
@@ -175,7 +182,8 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   const Routing r(R, E);
   Tensor rows = x;
   Tensor logits;
-  bool selected = false;
+  bool selected = false, inside = false;  // selection done; the forward-only call makes the logits itself
+  const Tensor b = bias.defined() ? dense(bias) : Tensor();
   if (o.train || o.routing_out || !(wr.defined() || logits_.defined()) || norm_w.defined() || T == 0)
     f.routing = empty({r.at[Routing::PARTS]}, at::kInt, x);
   if (wr.defined()) {
@@ -200,7 +208,12 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
       f.xn = cast_bf16(x);
     }
     rows = f.xn;
-    if (!selected) {
+    if (!selected && moe_router_few_ok(T, H, E, k)) {
+      logits = empty({T, E}, at::kBFloat16, x);
+      inside = !f.routing.defined();
+      if (!inside)
+        check(moe_router_logits(bf(f.xn), bf(f.wrb), T, H, E, (uint16_t*)logits.data_ptr(), s), "moe_router_few");
+    } else if (!selected) {
       const NoAutocast off;
       logits = at::mm(f.xn, f.wrb.t());
     }
@@ -208,13 +221,17 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
     logits = dense(logits_);
   }
   f.logits = logits;
-  const Tensor b = bias.defined() ? dense(bias) : Tensor();
   if (!f.routing.defined()) {  // nothing is kept and nobody asks for the routing
     f.out = empty({T, H}, x_type, x);
     const int64_t bytes = moe_ffn_forward_workspace_bytes(T, H, E, I, k);
     const Tensor ws = empty({std::max<int64_t>(bytes, 256)}, at::kByte, x);
     // (it tells the observer about its launches itself, as do the two calls of a training step)
-    check(moe_ffn_forward(rows.data_ptr(), (int)dt(rows), logits.data_ptr(), (int)dt(logits), (const float*)ptr(b),
+    if (inside)
+      check(moe_routed_forward(bf(rows), bf(f.wrb), (uint16_t*)logits.data_ptr(), (const float*)ptr(b), bf(f.w.w1),
+                               bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(), (int)dt(x_type), ws.data_ptr(),
+                               ws.numel(), s),
+            "moe_routed_forward");
+    else check(moe_ffn_forward(rows.data_ptr(), (int)dt(rows), logits.data_ptr(), (int)dt(logits), (const float*)ptr(b),
                           bf(f.w.w1), bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(), (int)dt(x_type),
                           ws.data_ptr(), ws.numel(), s),
           "moe_ffn_forward");
@@ -457,6 +474,21 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
   }
 };
 
+// The router product alone: bf16 x [T,H] and wr [E,H] -> bf16 logits, the bits the layer selects on.
+Tensor router_logits(const Tensor& x, const Tensor& wr) {
+  const at::NoGradGuard off;
+  const NoAutocast no_autocast;
+  const int64_t T = x.size(0), H = x.size(1), E = wr.size(0);
+  if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || wr.scalar_type() != at::kBFloat16 || H % 8 != 0 ||
+      !moe_router_few_ok(T, H, E, 1))
+    return at::mm(x, wr.t());
+  const c10::DeviceGuard guard(x.device());
+  const Tensor xd = dense(x), wd = dense(wr);
+  Tensor logits = empty({T, E}, at::kBFloat16, x);
+  check(moe_router_logits(bf(xd), bf(wd), T, H, E, (uint16_t*)logits.data_ptr(), stream_of(x)), "moe_router_few");
+  return logits;
+}
+
 // -> (out, logits if the router product is inside, routing words if asked for)
 std::tuple<Tensor, OptTensor, OptTensor> layer(const Tensor& x, const OptTensor& norm_w, const OptTensor& wr,
                                                const OptTensor& logits, const OptTensor& ids, const Tensor& w1,
@@ -661,5 +693,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     }
   });
   m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
+  m.def("router_logits", &router_logits, py::call_guard<py::gil_scoped_release>());
   m.def("layer_f32", &layer_f32, py::call_guard<py::gil_scoped_release>());
 }

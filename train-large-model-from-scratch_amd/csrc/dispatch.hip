@@ -350,7 +350,8 @@ __global__ __launch_bounds__(256) void permute_fwd_scatter_kernel(const XT* __re
   }
 }
 
-// out[t,:] = sum_j gates[t*k+j] * y[row_to_pos[t*k+j],:]  (+ addend[t,:]); fp32, slot order.
+// out[t,:] = sum_j gates[t*k+j] * y[row_to_pos[t*k+j],:]  (+ addend[t,:]); fp32, slot order.  row_to_pos NULL:
+// the rows of y are in routed order.
 // ROUTER: + bf16(sum_j dsel[t*k+j] * wr[ids[t*k+j],:]), the router path's input gradient: a row of
 // dlogits has k nonzero entries, so that product is k rows of the router weight per token, which sit in
 // every XCD's L2 (at most 512 rows) -- instead of a library product over all E columns, its result in
@@ -380,7 +381,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
         Row8 v[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          pos[q] = row_to_pos[(size_t)t * k + j + q];
+          pos[q] = row_to_pos ? row_to_pos[(size_t)t * k + j + q] : t * k + j + q;
           gt[q] = gates ? gates[(size_t)t * k + j + q] : 1.f;
         }
 #pragma unroll
@@ -396,7 +397,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
         Row8 v[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          pos[q] = row_to_pos[(size_t)t * k + j + q];
+          pos[q] = row_to_pos ? row_to_pos[(size_t)t * k + j + q] : t * k + j + q;
           gt[q] = gates ? gates[(size_t)t * k + j + q] : 1.f;
         }
 #pragma unroll
@@ -407,7 +408,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
           for (int i = 0; i < 8; ++i) acc.v[i] += gt[q] * v[q].v[i];
       }
       for (; j < k; ++j) {
-        const int pos = row_to_pos[(size_t)t * k + j];
+        const int pos = row_to_pos ? row_to_pos[(size_t)t * k + j] : t * k + j;
         const float gt = gates ? gates[(size_t)t * k + j] : 1.f;
         const Row8 v = load8_nt(y + (size_t)pos * H + col);
 #pragma unroll
@@ -1040,6 +1041,19 @@ extern "C" int moe_cast_f32_bf16(const float* src, uint16_t* dst, int64_t n, voi
   if (blocks > 256 * 16) blocks = 256 * 16;
   hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, src,
                      dst, n8, (long long)n);
+  return moe_launch_status();
+}
+
+int moe_combine_in_order(const uint16_t* y, const float* gates, int64_t T, int64_t H, int64_t k, void* out,
+                         int out_dtype, hipStream_t s) {
+  const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
+  const uint16_t* none = nullptr;
+  if (out_dtype == MOE_DT_BF16)
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
+                       (int)(H / 8), (int)k, (uint16_t*)out, nullptr, nullptr, nullptr);
+  else
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
+                       (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
   return moe_launch_status();
 }
 

@@ -1,0 +1,410 @@
+// Few tokens: the router with its selection, and the whole layer body for at most 64 tokens.
+//
+// Generation asks for the experts of one token, or of one token from each sequence of a batch.  What
+// such a call cannot do without is one pass over the weights of the experts it asks for (one token of
+// the 64-expert layer: 100 MB; 48 tokens: 800 MB, nearly all of them), and next to that a kernel's
+// start and end are what costs.  So there are three kernels, none of which waits for another launch to
+// sort rows: every workgroup finds the rows of its expert in the (at most 512) expert ids itself, rows
+// stay in routed order, and the combine is part of the down kernel.  The products run on
+// v_mfma_f32_16x16x32_bf16, whose 16 rows are the tokens of an expert: weights go from memory straight to
+// the operand registers, every byte once, with a wave's whole share of the contraction requested before
+// the first product where it fits.
+#include "common.h"
+#include "internal.h"
+
+namespace {
+
+constexpr int DOWN_ONE_MAX_K = 32;
+constexpr unsigned OUTSIDE = 0xfffffff0u;  // a byte offset past every resource: reads as zero
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, long long bytes) {
+  if (bytes > 0xffffffe0ll) bytes = 0xffffffe0ll;
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(unsigned)bytes, 0x00020000);
+}
+__device__ __forceinline__ bf16x8 load_frag(__amdgpu_buffer_rsrc_t rs, unsigned off) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+}
+__device__ __forceinline__ float silu_mul(float g, float u) {
+  return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * u;
+}
+
+// ---- router product ---------------------------------------------------------------------------------
+// logits[t][e] = bf16(sum_h x[t][h] wr[e][h]) for 16 tokens and 16 experts a block; its 16 waves share the
+// contraction (a contiguous sixteenth each, requested at once) and their sums are added in order.  What
+// bounds it is one trip to memory; the library's product took 8-11 us and 18 us on the host.
+constexpr int RT_WAVES = 16;
+__global__ __launch_bounds__(RT_WAVES* MOE_WAVE) void router_few_kernel(const uint16_t* __restrict__ x,
+                                                                       const uint16_t* __restrict__ wr, int T, int H,
+                                                                       int E, uint16_t* __restrict__ logits) {
+  constexpr int KC = 8;
+  __shared__ float part[RT_WAVES][16][17];
+  const int lane = lane_id(), wv = threadIdx.x / MOE_WAVE, l16 = lane & 15, lq = lane >> 4;
+  const int e0 = blockIdx.x * 16, t0 = blockIdx.y * 16;
+  const int steps = (H + 31) / 32, per = (steps + RT_WAVES - 1) / RT_WAVES;
+  const int s_lo = wv * per, s_hi = s_lo + per < steps ? s_lo + per : steps;
+  const __amdgpu_buffer_rsrc_t rx = rsrc(x + (size_t)t0 * H, (long long)(T - t0) * H * 2);
+  const __amdgpu_buffer_rsrc_t rw = rsrc(wr + (size_t)e0 * H, (long long)(E - e0) * H * 2);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s = s_lo; s < s_hi; s += KC) {
+    bf16x8 a[KC], b[KC];
+#pragma unroll
+    for (int d = 0; d < KC; ++d) {
+      const int kk = (s + d) * 32 + lq * 8;
+      const unsigned off = s + d < s_hi && kk < H ? (unsigned)(l16 * H + kk) * 2 : OUTSIDE;
+      a[d] = load_frag(rx, off);  // (rows past T, experts past E: past the resource's end)
+      b[d] = load_frag(rw, off);
+    }
+#pragma unroll
+    for (int d = 0; d < KC; ++d) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], b[d], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[wv][lq * 4 + i][l16] = acc[i];
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    const int m = threadIdx.x >> 4, e = threadIdx.x & 15;
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < RT_WAVES; ++q) v += part[q][m][e];
+    if (t0 + m < T && e0 + e < E) logits[(size_t)(t0 + m) * E + e0 + e] = f32_to_bf16(v);
+  }
+}
+
+// ---- rows of one expert times its weights' columns ----------------------------------------------------
+// Columns: KC 32-deep k-steps of 16 columns of NB weight stacks; rows: the same steps of MF blocks of 16 rows.
+template <int NB, int KC>
+struct Columns {
+  bf16x8 v[NB][KC];
+};
+template <int MF, int KC>
+struct Rows {
+  bf16x8 v[MF][KC];
+};
+// Request steps s .. s + KC - 1 (those below s_end; the rest reads as zero).
+template <int NB, int KC>
+__device__ __forceinline__ void request(Columns<NB, KC>& c, const __amdgpu_buffer_rsrc_t (&w)[NB], bool live_col, int K,
+                                        int s, int s_end) {
+  const int lane = lane_id(), l16 = lane & 15, lq = lane >> 4;
+#pragma unroll
+  for (int d = 0; d < KC; ++d) {
+    const int kk = (s + d) * 32 + lq * 8;
+    const unsigned off = s + d < s_end && kk < K && live_col ? (unsigned)(l16 * K + kk) * 2 : OUTSIDE;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) c.v[n][d] = load_frag(w[n], off);
+  }
+}
+template <typename AT, int MF, int KC>
+__device__ __forceinline__ void request(Rows<MF, KC>& r, const AT* const (&row)[MF] /* NULL: no such row */, int K, int s,
+                                        int s_end) {
+  const int lq = lane_id() >> 4;
+#pragma unroll
+  for (int d = 0; d < KC; ++d) {
+    const int kk = (s + d) * 32 + lq * 8;
+    const bool in = s + d < s_end && kk < K;
+#pragma unroll
+    for (int m = 0; m < MF; ++m) {
+      u32x4 v = {0, 0, 0, 0};
+      if (in && row[m]) {
+        if constexpr (sizeof(AT) == 2) {
+          v = *reinterpret_cast<const u32x4*>(row[m] + kk);
+        } else {
+          const Row8 f = load8(row[m] + kk);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = pack_bf16x2(f.v[2 * i], f.v[2 * i + 1]);
+        }
+      }
+      r.v[m][d] = __builtin_bit_cast(bf16x8, v);
+    }
+  }
+}
+template <int NB, int MF, int KC>
+__device__ __forceinline__ void multiply(const Rows<MF, KC>& r, const Columns<NB, KC>& c, f32x4 (&acc)[NB][MF]) {
+#pragma unroll
+  for (int d = 0; d < KC; ++d)
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+        acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.v[m][d], c.v[n][d], acc[n][m], 0, 0, 0);
+}
+
+// The routed rows of expert e, listed in LDS by the whole workgroup (the order is left to chance: a row's
+// result does not depend on its place in the list); their number comes back.
+__device__ __forceinline__ int list_rows(const int32_t* __restrict__ ids, int R, int E, int e, int* rows, int* count) {
+  if (threadIdx.x == 0) *count = 0;
+  __syncthreads();
+  for (int r = threadIdx.x; r < R; r += blockDim.x) {
+    int id = ids[r];
+    id = id < 0 ? 0 : (id >= E ? E - 1 : id);
+    if (id == e) {
+      const int at = atomicAdd(count, 1);
+      if (at < FEW_MAX_TOKENS) rows[at] = r;
+    }
+  }
+  __syncthreads();
+  return *count < FEW_MAX_TOKENS ? *count : FEW_MAX_TOKENS;
+}
+
+// One expert's rows times `nblk` blocks of 16 columns of NB weight stacks [E,N,K], the four waves a contiguous
+// quarter of the contraction each.  NB = 2: gate and up, C = silu(g) u; NB = 1: down, C = y.  Rows of A are
+// tokens (a routed row's token is row / div) or routed rows (div = 1); rows of C are routed rows.
+// The blocks' chunks (KC k-steps) are one stream: while a chunk is multiplied (or a block's partial sums are
+// added through LDS) the next one is on its way, so that a workgroup never stops asking for weights.
+// KEEP > 0: a wave's share of the contraction is KEEP chunks, and its rows stay in registers for all blocks
+// (asked for again with every block they cost an eighth of the time: 48 tokens of the 64-expert layer,
+// gate and up 0.54 GB, 109 -> 97 us, 5.5 TB/s; a plain read loop over as much runs at 6.2-6.9).
+template <typename AT, int NB, int MF, int KC, int KEEP>
+__device__ __forceinline__ void few_columns(const AT* __restrict__ A, int div, const uint16_t* const (&w)[NB], int e,
+                                            int n0, int nblk, int N, int K, const int* rows, int n, float* part,
+                                            uint16_t* __restrict__ C) {
+  const int lane = lane_id(), wv = threadIdx.x / MOE_WAVE, l16 = lane & 15, lq = lane >> 4;
+  const int steps = (K + 31) / 32, per = ((steps + 3) / 4 + 1) & ~1;
+  const int s_lo = wv * per, s_hi = s_lo + per < steps ? s_lo + per : steps;
+  const int chunks = KEEP ? KEEP : (per + KC - 1) / KC;  // per block, the same for every wave
+  const AT* row[MF];
+#pragma unroll
+  for (int m = 0; m < MF; ++m) row[m] = m * 16 + l16 < n ? A + (size_t)(rows[m * 16 + l16] / div) * K : nullptr;
+  f32x4 acc[NB][MF];
+  const auto clear = [&]() {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int m = 0; m < MF; ++m) acc[b][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  int rb = 0, rc = 0;  // block and chunk of the next request
+  const auto ask = [&](Columns<NB, KC>& c) {
+    const int col = n0 + rb * 16;
+    __amdgpu_buffer_rsrc_t rs[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) rs[b] = rsrc(w[b] + ((size_t)e * N + col) * K, (long long)(N - col) * K * 2);
+    request<NB, KC>(c, rs, col + l16 < N, K, s_lo + rc * KC, s_hi);
+    if (++rc == chunks) rc = 0, ++rb;
+  };
+  int mb = 0;  // block of the current product
+  const auto finish = [&]() {
+    // part [2][4][NB][MF][4][64]: the four waves' sums of this block (two buffers: a wave that runs ahead
+    // writes the other one)
+    float* buf = part + (mb & 1) * (4 * NB * MF * 256);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int m = 0; m < MF; ++m)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) buf[((wv * NB + b) * MF + m) * 256 + q * MOE_WAVE + lane] = acc[b][m][q];
+    clear();
+    __syncthreads();
+    const int col = n0 + mb * 16 + l16;
+#pragma unroll
+    for (int m = 0; m < MF; ++m) {  // wave q: rows 16 m + 4 lq + q
+      float v[NB];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        v[b] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[b] += buf[((i * NB + b) * MF + m) * 256 + wv * MOE_WAVE + lane];
+      }
+      const int at = m * 16 + lq * 4 + wv;
+      if (at < n && col < N) C[(size_t)rows[at] * N + col] = f32_to_bf16(NB == 2 ? silu_mul(v[0], v[NB - 1]) : v[0]);
+    }
+    ++mb;
+  };
+  Columns<NB, KC> c0, c1;
+  clear();
+  ask(c0);
+  const int total = nblk * chunks;
+  if constexpr (KEEP > 0) {
+    Rows<MF, KC> r[KEEP];
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) request<AT, MF, KC>(r[i], row, K, s_lo + i * KC, s_hi);
+    for (int i = 0; i < total; i += 2) {
+      if (i + 1 < total) ask(c1);
+      multiply<NB, MF, KC>(r[0], c0, acc);
+      if (KEEP == 1) finish();
+      if (i + 1 >= total) break;
+      if (i + 2 < total) ask(c0);
+      multiply<NB, MF, KC>(r[KEEP - 1], c1, acc);
+      finish();
+    }
+  } else {
+    Rows<MF, KC> r0, r1;
+    int mc = 0;
+    request<AT, MF, KC>(r0, row, K, s_lo, s_hi);
+    const auto next_rows = [&](Rows<MF, KC>& r, int i) { request<AT, MF, KC>(r, row, K, s_lo + i % chunks * KC, s_hi); };
+    for (int i = 0; i < total; i += 2) {
+      if (i + 1 < total) ask(c1), next_rows(r1, i + 1);
+      multiply<NB, MF, KC>(r0, c0, acc);
+      if (++mc == chunks) mc = 0, finish();
+      if (i + 1 >= total) break;
+      if (i + 2 < total) ask(c0), next_rows(r0, i + 2);
+      multiply<NB, MF, KC>(r1, c1, acc);
+      if (++mc == chunks) mc = 0, finish();
+    }
+  }
+}
+
+// At most 16 rows: they stay in registers where a wave's share of the contraction is at most 16 steps.
+template <typename AT, int NB>
+__device__ __forceinline__ void few_columns_16(const AT* __restrict__ A, int div, const uint16_t* const (&w)[NB], int e,
+                                               int n0, int nblk, int N, int K, const int* rows, int n, float* part,
+                                               uint16_t* __restrict__ C) {
+  const int per = ((((K + 31) / 32) + 3) / 4 + 1) & ~1;
+  if (per <= 8) few_columns<AT, NB, 1, 8, 1>(A, div, w, e, n0, nblk, N, K, rows, n, part, C);
+  else if (per <= 16) few_columns<AT, NB, 1, 8, 2>(A, div, w, e, n0, nblk, N, K, rows, n, part, C);
+  else few_columns<AT, NB, 1, 8, 0>(A, div, w, e, n0, nblk, N, K, rows, n, part, C);
+}
+
+// ONE: a single token; block row j takes its j-th expert and no list is needed.
+template <typename AT, int NB, bool ONE>
+__global__ __launch_bounds__(256, 2) void few_kernel(const AT* __restrict__ A, int div, const int32_t* __restrict__ ids,
+                                                    int R, const uint16_t* __restrict__ w0,
+                                                    const uint16_t* __restrict__ w1, int E, int N, int K, int nblk,
+                                                    uint16_t* __restrict__ C) {
+  __shared__ int rows[FEW_MAX_TOKENS], count;
+  __shared__ float part[2 * 4 * NB * (ONE ? 1 : 4) * 256];
+  const uint16_t* w[NB];
+  w[0] = w0;
+  if constexpr (NB == 2) w[1] = w1;
+  const int n0 = blockIdx.x * nblk * 16, left = (N - n0 + 15) / 16;
+  const int nb = left < nblk ? left : nblk;
+  if constexpr (ONE) {
+    const int j = blockIdx.y;
+    int e = ids[j];
+    e = e < 0 ? 0 : (e >= E ? E - 1 : e);
+    if (threadIdx.x == 0) rows[0] = j;
+    __syncthreads();
+    few_columns_16<AT, NB>(A, div, w, e, n0, nb, N, K, rows, 1, part, C);
+  } else {
+    const int e = blockIdx.y;
+    const int n = list_rows(ids, R, E, e, rows, &count);
+    if (n == 0) return;
+    if (n <= 16) few_columns_16<AT, NB>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
+    else if (n <= 32) few_columns<AT, NB, 2, 4, 0>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
+    else few_columns<AT, NB, 4, 2, 0>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
+  }
+}
+
+// ---- down projection and combine of one token -----------------------------------------------------------------
+// out[h] = sum_j gate[j] bf16(y[j][h]) for the 16 columns h of this block: the block's eight waves take the
+// token's experts in turn (or shares of their contractions, where fewer than eight are asked for) and leave
+// their sums in LDS, where they are added up in slot order, as the combine kernel does.
+constexpr int DOWN_WAVES = 8;
+template <typename OT>
+__global__ __launch_bounds__(DOWN_WAVES* MOE_WAVE) void down_one_kernel(const uint16_t* __restrict__ act,
+                                                                       const int32_t* __restrict__ ids,
+                                                                       const float* __restrict__ gates, int k,
+                                                                       const uint16_t* __restrict__ w2, int E, int H,
+                                                                       int I, OT* __restrict__ out) {
+  constexpr int KC = 32;                                             // k-steps requested at once
+  __shared__ float y[DOWN_WAVES + DOWN_ONE_MAX_K][16];               // [splits][k]
+  __shared__ __align__(16) uint16_t arow[DOWN_WAVES][KC * 32];       // a wave's piece of its row of act
+  const int lane = lane_id(), wv = threadIdx.x / MOE_WAVE, l16 = lane & 15, lq = lane >> 4;
+  const int h0 = blockIdx.x * 16;
+  const int splits = k >= DOWN_WAVES ? 1 : DOWN_WAVES / k;
+  const int steps = (I + 31) / 32, per = ((steps + splits - 1) / splits + 1) & ~1;
+  for (int item = wv; item < k * splits; item += DOWN_WAVES) {
+    const int j = item / splits, sp = item - j * splits;
+    int e = ids[j];
+    e = e < 0 ? 0 : (e >= E ? E - 1 : e);
+    const int s_lo = sp * per, s_hi = s_lo + per < steps ? s_lo + per : steps;
+    const __amdgpu_buffer_rsrc_t rs[1] = {rsrc(w2 + ((size_t)e * H + h0) * I, (long long)(H - h0) * I * 2)};
+    const __amdgpu_buffer_rsrc_t ra = rsrc(act + (size_t)j * I, (long long)I * 2);
+    f32x4 acc[1][1] = {{f32x4{0.f, 0.f, 0.f, 0.f}}};
+    for (int s = s_lo; s < s_hi; s += KC) {
+      Columns<1, KC> c;
+      request<1, KC>(c, rs, h0 + l16 < H, I, s, s_hi);
+      // (a single row: in operand layout 15 of 16 lanes would carry zeros, so it comes through LDS)
+#pragma unroll
+      for (int i = 0; i < KC * 32 / (MOE_WAVE * 8); ++i) {
+        const int at = (i * MOE_WAVE + lane) * 8;
+        *reinterpret_cast<bf16x8*>(&arow[wv][at]) = load_frag(ra, (unsigned)(s * 32 + at) * 2);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int d = 0; d < KC; ++d) {
+        bf16x8 a = *reinterpret_cast<const bf16x8*>(&arow[wv][d * 32 + lq * 8]);
+        if (l16 != 0) a = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
+        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, c.v[0][d], acc[0][0], 0, 0, 0);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (lq == 0) y[sp * k + j][l16] = acc[0][0][0];  // row 0 of the product
+  }
+  __syncthreads();
+  if (threadIdx.x < 16 && h0 + threadIdx.x < H) {
+    const int c = threadIdx.x;
+    float acc = 0.f;
+    for (int j = 0; j < k; ++j) {
+      float v = y[j][c];
+      for (int sp = 1; sp < splits; ++sp) v += y[sp * k + j][c];
+      acc += gates[j] * bf16_to_f32(f32_to_bf16(v));
+    }
+    if constexpr (sizeof(OT) == 2) out[h0 + c] = f32_to_bf16(acc);
+    else out[h0 + c] = acc;
+  }
+}
+
+}  // namespace
+
+bool moe_router_few_ok(int64_t T, int64_t H, int64_t E, int64_t k) {
+  // (a large batch takes the library's product: there the few logits that round the other way would now
+  // and then select another expert than a caller's own product of the same tensors)
+  return T > 0 && T <= FEW_MAX_TOKENS && H <= 65536 && E <= FEW_MAX_EXPERTS && k <= E && k <= MOE_MAX_TOPK;
+}
+
+int moe_router_few(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
+                   hipStream_t s) {
+  const dim3 grid((unsigned)((E + 15) / 16), (unsigned)((T + 15) / 16));
+  hipLaunchKernelGGL(router_few_kernel, grid, dim3(RT_WAVES * MOE_WAVE), 0, s, x, wr, (int)T, (int)H, (int)E, logits);
+  return moe_launch_status();
+}
+
+// At most 64 tokens: an expert's rows then fit four blocks of 16, and all of them the lists.  (The tiled
+// kernels take 256 rows at a time, of which 1 to 64 are there.)
+bool moe_few_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
+  return T > 0 && T <= FEW_MAX_TOKENS && E <= 65535 && H <= 65536 && I <= 65536;
+}
+
+namespace {
+// 16-column blocks per workgroup: as many as leave two workgroups for every compute unit (two are resident)
+// if `busy` experts are asked for.
+int few_blocks(int64_t N, int64_t busy) {
+  const int64_t blocks = (N + 15) / 16, fit = blocks * busy / (4 * (int64_t)moe_compute_units());
+  return (int)(fit < 1 ? 1 : (fit > 8 ? 8 : fit));
+}
+}  // namespace
+
+int moe_gateup_few(const void* x, int x_dtype, const int32_t* ids, const uint16_t* w1, const uint16_t* w3, int64_t T,
+                   int64_t H, int64_t E, int64_t I, int64_t k, uint16_t* act, hipStream_t s) {
+  const int nblk = few_blocks(I, T * k < E ? T * k : E);
+  const dim3 grid((unsigned)(((I + 15) / 16 + nblk - 1) / nblk), (unsigned)(T == 1 ? k : E)), block(256);
+  const auto go = [&](auto one, auto xt) {
+    using XT = decltype(xt);
+    hipLaunchKernelGGL((few_kernel<XT, 2, decltype(one)::value>), grid, block, 0, s, (const XT*)x, (int)k, ids, (int)(T * k),
+                       w1, w3, (int)E, (int)I, (int)H, nblk, act);
+    return moe_launch_status();
+  };
+  if (x_dtype == MOE_DT_BF16) return T == 1 ? go(std::true_type{}, uint16_t{}) : go(std::false_type{}, uint16_t{});
+  return T == 1 ? go(std::true_type{}, float{}) : go(std::false_type{}, float{});
+}
+
+int moe_down_few(const uint16_t* act, const int32_t* ids, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I,
+                 int64_t k, uint16_t* y, hipStream_t s) {
+  const int nblk = few_blocks(H, T * k < E ? T * k : E);
+  const dim3 grid((unsigned)(((H + 15) / 16 + nblk - 1) / nblk), (unsigned)E), block(256);
+  hipLaunchKernelGGL((few_kernel<uint16_t, 1, false>), grid, block, 0, s, act, 1, ids, (int)(T * k), w2, nullptr, (int)E,
+                     (int)H, (int)I, nblk, y);
+  return moe_launch_status();
+}
+
+bool moe_down_one_ok(int64_t T, int64_t k) { return T == 1 && k <= DOWN_ONE_MAX_K; }
+
+int moe_down_one(const uint16_t* act, const int32_t* ids, const float* gates, const uint16_t* w2, int64_t H, int64_t E,
+                 int64_t I, int64_t k, void* out, int out_dtype, hipStream_t s) {
+  const dim3 grid((unsigned)((H + 15) / 16)), block(DOWN_WAVES * MOE_WAVE);
+  if (out_dtype == MOE_DT_BF16)
+    hipLaunchKernelGGL(down_one_kernel<uint16_t>, grid, block, 0, s, act, ids, gates, (int)k, w2, (int)E, (int)H, (int)I,
+                       (uint16_t*)out);
+  else
+    hipLaunchKernelGGL(down_one_kernel<float>, grid, block, 0, s, act, ids, gates, (int)k, w2, (int)E, (int)H, (int)I,
+                       (float*)out);
+  return moe_launch_status();
+}

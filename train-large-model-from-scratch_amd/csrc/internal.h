@@ -33,3 +33,25 @@ int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const
 
 // int64 expert ids to int32, values outside int32 to -1 (dispatch.hip).
 int moe_narrow_ids(const int64_t* ids, int64_t R, int32_t* out, hipStream_t s);
+
+// ---- few tokens (few.hip) ----
+constexpr int FEW_MAX_TOKENS = 64;
+constexpr int FEW_MAX_EXPERTS = 128;
+
+// Router product rounded to bf16: shapes it takes, and the launch.
+bool moe_router_few_ok(int64_t T, int64_t H, int64_t E, int64_t k);
+int moe_router_few(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
+                   hipStream_t s);
+// The experts on at most 64 tokens, rows in routed order: act [T*k, I] from x and the expert ids, y [T*k, H]
+// from act, and for one token the combined output from act.
+bool moe_few_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k);
+int moe_gateup_few(const void* x, int x_dtype, const int32_t* ids, const uint16_t* w1, const uint16_t* w3, int64_t T,
+                   int64_t H, int64_t E, int64_t I, int64_t k, uint16_t* act, hipStream_t s);
+int moe_down_few(const uint16_t* act, const int32_t* ids, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I,
+                 int64_t k, uint16_t* y, hipStream_t s);
+bool moe_down_one_ok(int64_t T, int64_t k);
+int moe_down_one(const uint16_t* act, const int32_t* ids, const float* gates, const uint16_t* w2, int64_t H, int64_t E,
+                 int64_t I, int64_t k, void* out, int out_dtype, hipStream_t s);
+// moe_combine_fwd with the rows of y in routed order (dispatch.hip).
+int moe_combine_in_order(const uint16_t* y, const float* gates, int64_t T, int64_t H, int64_t k, void* out,
+                         int out_dtype, hipStream_t s);

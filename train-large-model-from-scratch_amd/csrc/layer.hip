@@ -70,10 +70,12 @@ extern "C" int64_t moe_ffn_forward_workspace_bytes(int64_t T, int64_t H, int64_t
   return carve(T, H, E, I, k).total;
 }
 
-extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, int logits_dtype,
-                               const float* bias, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
-                               int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
-                               int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+// The pass itself.  With `wr` the router product is part of it (logits are written to logits_out; shapes
+// that moe_router_few_ok takes), without it the logits are given.
+static int forward_only(const void* x, int x_dtype, const void* logits, int logits_dtype, const uint16_t* wr,
+                        uint16_t* logits_out, const float* bias, const uint16_t* w1, const uint16_t* w3,
+                        const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
+                        int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
   if (!sizes_ok(T, H, E, I, k)) return MOE_ERR_LIMIT;
   if (x_dtype != MOE_DT_BF16 && x_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
@@ -81,7 +83,14 @@ extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, i
   if (out_dtype != MOE_DT_BF16 && out_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
   if (T == 0) return 0;
   MOE_CHECK_PTR(x);
-  MOE_CHECK_PTR(logits);
+  if (wr) {
+    MOE_CHECK_PTR(wr);
+    MOE_CHECK_PTR(logits_out);
+    if (x_dtype != MOE_DT_BF16) return MOE_ERR_DTYPE;
+    if (!moe_router_few_ok(T, H, E, k)) return MOE_ERR_LIMIT;
+  } else {
+    MOE_CHECK_PTR(logits);
+  }
   MOE_CHECK_PTR(w1);
   MOE_CHECK_PTR(w3);
   MOE_CHECK_PTR(w2);
@@ -100,7 +109,23 @@ extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, i
   uint16_t* xp = (uint16_t*)(ws + c.xp);
   uint16_t* act = (uint16_t*)(ws + c.act);
   uint16_t* y = (uint16_t*)(ws + c.y);
+  hipStream_t st = (hipStream_t)stream;
+  if (wr) {
+    MOE_STEP("moe_router_few", moe_router_few((const uint16_t*)x, wr, T, H, E, logits_out, st));
+    logits = logits_out;
+    logits_dtype = MOE_DT_BF16;
+  }
   MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream));
+  if (moe_few_ok(T, H, E, I, k)) {  // rows stay in routed order: no dispatch, no gather
+    MOE_STEP("moe_gateup_few", moe_gateup_few(x, x_dtype, ids, w1, w3, T, H, E, I, k, act, st));
+    if (moe_down_one_ok(T, k)) {
+      MOE_STEP("moe_down_one", moe_down_one(act, ids, gates, w2, H, E, I, k, out, out_dtype, st));
+      return 0;
+    }
+    MOE_STEP("moe_down_few", moe_down_few(act, ids, w2, T, H, E, I, k, y, st));
+    MOE_STEP("moe_combine_in_order", moe_combine_in_order(y, gates, T, H, k, out, out_dtype, st));
+    return 0;
+  }
   MOE_STEP("moe_histogram_scan_checked",
            moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
                               moe_dispatch_workspace_bytes(R, E), stream));
@@ -111,6 +136,28 @@ extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, i
            moe_gemm_gateup_swiglu_fwd(xp, w1, w3, offs, E, R, H, I, nullptr, nullptr, act, stream));
   MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_fwd(act, w2, offs, E, R, H, I, y, stream));
   MOE_STEP("moe_combine_fwd", moe_combine_fwd(y, gates, row_to_pos, T, H, k, out, out_dtype, stream));
+  return 0;
+}
+
+extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, int logits_dtype,
+                               const float* bias, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
+                               int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
+                               int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  return forward_only(x, x_dtype, logits, logits_dtype, nullptr, nullptr, bias, w1, w3, w2, T, H, E, I, k, out,
+                      out_dtype, workspace, workspace_bytes, stream);
+}
+
+int moe_routed_forward(const uint16_t* x, const uint16_t* wr, uint16_t* logits, const float* bias, const uint16_t* w1,
+                       const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k,
+                       void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!wr) return MOE_ERR_NULL;
+  return forward_only(x, MOE_DT_BF16, nullptr, MOE_DT_BF16, wr, logits, bias, w1, w3, w2, T, H, E, I, k, out, out_dtype,
+                      workspace, workspace_bytes, stream);
+}
+
+int moe_router_logits(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
+                      void* stream) {
+  MOE_STEP("moe_router_few", moe_router_few(x, wr, T, H, E, logits, (hipStream_t)stream));
   return 0;
 }
 

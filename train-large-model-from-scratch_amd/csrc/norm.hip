@@ -99,56 +99,68 @@ __global__ __launch_bounds__(NT) void rmsnorm_router_fwd_kernel(
     const uint16_t* __restrict__ wr, int E, int k, uint16_t* __restrict__ xn, float* __restrict__ rstd,
     uint16_t* __restrict__ logits, int32_t* __restrict__ ids, float* __restrict__ gates) {
   extern __shared__ __attribute__((aligned(16))) uint16_t rows[];  // [RB][H + 8]; later fp32 partials
-  __shared__ float red[NW];
   __shared__ uint16_t lg16[RB * RMAX_EB * 16];
   const int H = H8 * 8, LDT = H + 8;
   const int lane = lane_id(), wv = threadIdx.x / MOE_WAVE;
   const int t0 = blockIdx.x * RB;
-  Row8 wv8[NV];
+  // normalisation: a wave per row, its next row requested before this one is reduced (a block-wide
+  // reduction per row, 16 in a row, left the kernel waiting: 62 us for 8192 rows of 2048, now 55)
+  Row8 xv[NV], nx[NV];
+  const auto request = [&](int rr, Row8(&to)[NV]) {
+    if (t0 + rr >= T) return;
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int c = threadIdx.x + i * NT;
-    if (c < H8) wv8[i] = load8(w + c * 8);
-  }
-  for (int rr = 0; rr < RB; ++rr) {
-    const int t = t0 + rr;
-    if (t >= T) {  // block-uniform: rows past the end are zero rows for the product
+    for (int i = 0; i < NV; ++i) {
+      const int c = lane + i * MOE_WAVE;
+      if (c < H8) to[i] = load8(x + (size_t)(t0 + rr) * H + c * 8);
+    }
+  };
+  request(wv, xv);
+#pragma unroll
+  for (int q = 0; q < RB / NW; ++q) {
+    const int rr = wv + q * NW, t = t0 + rr;
+    if (q + 1 < RB / NW) request(rr + NW, nx);
+    if (t >= T) {  // wave-uniform: rows past the end are zero rows for the product
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const int c = threadIdx.x + i * NT;
+        const int c = lane + i * MOE_WAVE;
         if (c < H8) *reinterpret_cast<u32x4*>(rows + rr * LDT + c * 8) = u32x4{0, 0, 0, 0};
       }
       continue;
     }
-    Row8 xv[NV];
-    float ss = 0.f;
+    // (four partial sums, as the block of rmsnorm_fwd_kernel forms them: the same bits)
+    float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int c = threadIdx.x + i * NT;
-      if (c < H8) {
-        xv[i] = load8(x + (size_t)t * H + c * 8);
+    for (int g = 0; g < NW && g < NV; ++g) {
+      float ss = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ss += xv[i].v[j] * xv[i].v[j];
+      for (int i = g; i < NV; i += NW) {
+        if (lane + i * MOE_WAVE < H8) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ss += xv[i].v[j] * xv[i].v[j];
+        }
       }
+      sum += moe_wave_sum_f32(ss);
     }
-    ss = block_sum(ss, red);
-    const float r = rsqrtf(ss / (float)H + eps);
-    if (threadIdx.x == 0) rstd[t] = r;
+    const float r = rsqrtf(sum / (float)H + eps);
+    if (lane == 0) rstd[t] = r;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = threadIdx.x + i * NT;
+      const int c = lane + i * MOE_WAVE;
       if (c < H8) {
+        const Row8 wn = load8(w + c * 8);
         Row8 o;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           float v = xv[i].v[j] * r;
           if (is_bf16<XT>::value) v = bf16_to_f32(f32_to_bf16(v));  // `.to(input_dtype)`, norm.py:19
-          o.v[j] = wv8[i].v[j] * v;
+          o.v[j] = wn.v[j] * v;
         }
         store8(xn + (size_t)t * H + c * 8, o);
         store8(rows + rr * LDT + c * 8, o);
       }
     }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) xv[i] = nx[i];
   }
   __syncthreads();
   // logits[m][e] = sum_h rows[m][h] * wr[e][h]: lane l holds A row l % 16 (token) and B row
@@ -158,16 +170,37 @@ __global__ __launch_bounds__(NT) void rmsnorm_router_fwd_kernel(
 #pragma unroll
   for (int nb = 0; nb < RMAX_EB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int l16 = lane & 15, lq = lane >> 4;
-  for (int ks = wv; ks < H / 32; ks += NW) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(rows + l16 * LDT + ks * 32 + lq * 8);
+  // (the router's rows come from L2: a step's are requested while the step before is multiplied)
+  const auto product = [&](auto eb_c) {
+    constexpr int EBT = decltype(eb_c)::value;  // column blocks, EB rounded up: the surplus repeats the last
+    bf16x8 b[2][EBT];
+    const auto request = [&](int ks, bf16x8(&to)[EBT]) {
 #pragma unroll
-    for (int nb = 0; nb < RMAX_EB; ++nb) {
-      if (nb < EB) {
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(wr + (size_t)(nb * 16 + l16) * H + ks * 32 + lq * 8);
-        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nb], 0, 0, 0);
+      for (int nb = 0; nb < EBT; ++nb) {
+        const int n = nb < EB ? nb : EB - 1;
+        to[nb] = *reinterpret_cast<const bf16x8*>(wr + (size_t)(n * 16 + l16) * H + ks * 32 + lq * 8);
       }
+    };
+    const auto step = [&](int ks, const bf16x8(&from)[EBT]) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(rows + l16 * LDT + ks * 32 + lq * 8);
+#pragma unroll
+      for (int nb = 0; nb < EBT; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, from[nb], acc[nb], 0, 0, 0);
+    };
+    const int n = H / 32;
+    int ks = wv;
+    if (ks < n) request(ks, b[0]);
+    for (; ks < n; ks += 2 * NW) {
+      if (ks + NW < n) request(ks + NW, b[1]);
+      step(ks, b[0]);
+      if (ks + NW >= n) break;
+      if (ks + 2 * NW < n) request(ks + 2 * NW, b[0]);
+      step(ks + NW, b[1]);
     }
-  }
+  };
+  if (EB <= 1) product(std::integral_constant<int, 1>{});
+  else if (EB <= 2) product(std::integral_constant<int, 2>{});
+  else if (EB <= 4) product(std::integral_constant<int, 4>{});
+  else product(std::integral_constant<int, 8>{});
   __syncthreads();  // every wave is done with the rows: their memory takes the partial products
   float* part = reinterpret_cast<float*>(rows);  // [NW][RB][E]
   // accumulator layout: lane l holds column l % 16 (expert) of rows 4 * (l / 16) .. + 3 (tokens)
@@ -277,22 +310,35 @@ __global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(
   }
 }
 
-// dw[c] = sum_b part[b][c], b ascending within each of the block's NW row groups, groups
-// combined in ascending order: one fixed order whatever the launch.
-__global__ __launch_bounds__(NT) void colsum_kernel(const float* __restrict__ part, int nb, int H,
-                                                   float* __restrict__ dw) {
-  __shared__ float red[NW][MOE_WAVE];
+// dw[c] = sum_b part[b][c], b ascending within each of CG row groups, groups combined in ascending order:
+// one fixed order whatever the launch.  A block owns 64 columns, a wave a group of rows: the launch has
+// few blocks (32 at H = 2048), so what bounds it is the length of a wave's chain of loads; with 16 groups
+// and eight loads in flight it takes 6 us where 4 groups with one took 64 (1024 partial rows of 2048).
+constexpr int CG = 16;
+__global__ __launch_bounds__(CG* MOE_WAVE) void colsum_kernel(const float* __restrict__ part, int nb, int H,
+                                                             float* __restrict__ dw) {
+  __shared__ float red[CG][MOE_WAVE];
   const int c = blockIdx.x * MOE_WAVE + lane_id(), g = threadIdx.x / MOE_WAVE;
-  const int per = (nb + NW - 1) / NW;
+  const int per = (nb + CG - 1) / CG;
+  const int lo = g * per, hi = lo + per < nb ? lo + per : nb;
   float s = 0.f;
-  if (c < H)
-    for (int b = g * per; b < nb && b < (g + 1) * per; ++b) s += part[(size_t)b * H + c];
+  if (c < H) {
+    int b = lo;
+    for (; b + 8 <= hi; b += 8) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = part[(size_t)(b + i) * H + c];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s += v[i];
+    }
+    for (; b < hi; ++b) s += part[(size_t)b * H + c];
+  }
   red[g][lane_id()] = s;
   __syncthreads();
   if (g == 0 && c < H) {
     float tot = 0.f;
 #pragma unroll
-    for (int i = 0; i < NW; ++i) tot += red[i][lane_id()];
+    for (int i = 0; i < CG; ++i) tot += red[i][lane_id()];
     dw[c] = tot;
   }
 }
@@ -398,11 +444,15 @@ extern "C" int moe_rmsnorm_router_fwd(const void* x, int x_dtype, const float* w
     hipLaunchKernelGGL(kern, grid, block, lds, s, (const XT*)x, weight, eps, (int)T, (int)(H / 8),       \
                        router_weight, (int)E, (int)k, xn, rstd, logits, ids, gates);                     \
   } while (0)
-  const int nv = pick_nv(H);
+  const int64_t groups = (H / 8 + MOE_WAVE - 1) / MOE_WAVE;  // 16-byte column groups per lane (H <= 4096: at most 8)
   if (x_dtype == MOE_DT_BF16) {
-    if (nv == 1) MOE_NORM_ROUTER(uint16_t, 1); else MOE_NORM_ROUTER(uint16_t, 2);
+    if (groups <= 2) MOE_NORM_ROUTER(uint16_t, 2);
+    else if (groups <= 4) MOE_NORM_ROUTER(uint16_t, 4);
+    else MOE_NORM_ROUTER(uint16_t, 8);
   } else if (x_dtype == MOE_DT_F32) {
-    if (nv == 1) MOE_NORM_ROUTER(float, 1); else MOE_NORM_ROUTER(float, 2);
+    if (groups <= 2) MOE_NORM_ROUTER(float, 2);
+    else if (groups <= 4) MOE_NORM_ROUTER(float, 4);
+    else MOE_NORM_ROUTER(float, 8);
   } else {
     return MOE_ERR_DTYPE;
   }
@@ -423,7 +473,7 @@ extern "C" int moe_rmsnorm_bwd(const void* x, int x_dtype, const float* weight, 
   MOE_CHECK_PTR(dweight);
   hipStream_t s = (hipStream_t)stream;
   if (T == 0) {  // no rows: the weight gradient is zero
-    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + MOE_WAVE - 1) / MOE_WAVE)), dim3(NT), 0, s,
+    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + MOE_WAVE - 1) / MOE_WAVE)), dim3(CG * MOE_WAVE), 0, s,
                        (const float*)dweight, 0, (int)H, dweight);
     return moe_launch_status();
   }
@@ -449,7 +499,7 @@ extern "C" int moe_rmsnorm_bwd(const void* x, int x_dtype, const float* weight, 
   else
     return MOE_ERR_DTYPE;
   if (rc) return rc;
-  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + MOE_WAVE - 1) / MOE_WAVE)), dim3(NT), 0, s,
+  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + MOE_WAVE - 1) / MOE_WAVE)), dim3(CG * MOE_WAVE), 0, s,
                      (const float*)part, bwd_blocks(T), (int)H, dweight);
   return moe_launch_status();
 }

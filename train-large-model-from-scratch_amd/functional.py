@@ -55,7 +55,7 @@ class _RouterLinear(torch.autograd.Function):
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx, x, w):
         ctx.save_for_backward(x, w)
-        return torch.nn.functional.linear(x, w)
+        return _lib.native().router_logits(x, w)
 
     @staticmethod
     @torch.amp.custom_bwd(device_type="cuda")

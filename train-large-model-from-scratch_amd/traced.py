@@ -25,7 +25,7 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from . import ops
+from . import lib as _lib, ops
 from .functional import _router_wgrad
 
 _BF16 = torch.bfloat16
@@ -150,8 +150,7 @@ def routed_fwd(x: Tensor, wr: Tensor, w1: Tensor, w3: Tensor, w2: Tensor, k: int
     wb = [ops.cast_bf16(ops.dense(w)) for w in (w1, w3, w2)]
     xn = ops.cast_bf16(x)
     wrb = ops.dense(wr.detach().to(_BF16))
-    with torch.autocast("cuda", enabled=False):
-        logits = xn @ wrb.t()
+    logits = _lib.native().router_logits(xn, wrb)
     out, r, xp, gu, act = ops.layer_forward(xn, logits, *wb, k, train, x.dtype)
     copies = [b if w.dtype != _BF16 else _empty(x) for w, b in zip((w1, w3, w2), wb)]
     if not train:
