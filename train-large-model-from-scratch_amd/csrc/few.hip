@@ -296,13 +296,14 @@ __global__ __launch_bounds__(DOWN_WAVES* MOE_WAVE) void down_one_kernel(const ui
   constexpr int KC = 32;                                             // k-steps requested at once
   __shared__ float y[DOWN_WAVES + DOWN_ONE_MAX_K][16];               // [splits][k]
   __shared__ __align__(16) uint16_t arow[DOWN_WAVES][KC * 32];       // a wave's piece of its row of act
-  const int lane = lane_id(), wv = threadIdx.x / MOE_WAVE, l16 = lane & 15, lq = lane >> 4;
+  const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MOE_WAVE)), l16 = lane & 15,
+            lq = lane >> 4;
   const int h0 = blockIdx.x * 16;
   const int splits = k >= DOWN_WAVES ? 1 : DOWN_WAVES / k;
   const int steps = (I + 31) / 32, per = ((steps + splits - 1) / splits + 1) & ~1;
   for (int item = wv; item < k * splits; item += DOWN_WAVES) {
     const int j = item / splits, sp = item - j * splits;
-    int e = ids[j];
+    int e = __builtin_amdgcn_readfirstlane(ids[j]);
     e = e < 0 ? 0 : (e >= E ? E - 1 : e);
     const int s_lo = sp * per, s_hi = s_lo + per < steps ? s_lo + per : steps;
     const __amdgpu_buffer_rsrc_t rs[1] = {rsrc(w2 + ((size_t)e * H + h0) * I, (long long)(H - h0) * I * 2)};

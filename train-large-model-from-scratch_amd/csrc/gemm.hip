@@ -28,8 +28,8 @@
 // as they lie in memory and read through the transposing LDS read of gfx950.
 // Workgroups are numbered so that each XCD (own L2) works on a contiguous range of tiles,
 // i.e. on its own experts' weights.
-#include "common.h"
 #include "internal.h"
+#include "tile_ops.h"
 
 namespace {
 
@@ -77,122 +77,6 @@ struct TileCfg {
 // the epilogues are VALU-bound, and an IEEE division would triple their cost.
 __device__ __forceinline__ float sigmoidf_(float x) {
   return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
-
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-
-// A window of global memory read through a buffer resource: reads at or past `bytes`
-// return zero.  Only the per-lane offset takes part in the hardware bounds check (a scalar
-// offset does not), so a window is advanced along k by moving its base and shrinking its
-// size, both scalar operations.
-struct View {
-  const uint16_t* base;
-  long long bytes;
-};
-__device__ __forceinline__ View make_view(const uint16_t* base, long long valid_elems) {
-  return View{base, valid_elems > 0 ? valid_elems * 2 : 0};
-}
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t view_rsrc(const View& w, long long byte_off) {
-  long long left = w.bytes - byte_off;
-  if (left < 0) left = 0;
-  if (left > 0xffffffffll) left = 0xffffffffll;
-  return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)w.base + byte_off), 0,
-                                           (int)(unsigned)left, 0x00020000);
-}
-
-// ---- operand staging ----------------------------------------------------------------------
-// Two LDS layouts, one per memory order of the operand, each with the fragment read that
-// hands an MFMA lane its 8 consecutive k values for row (lane % 32):
-//
-// OpInner  source is k-contiguous: element (r, kk) at view[r * ld + k0 + kk].
-//          LDS holds [ROWS][BK + 8] (16 bytes of padding per row); a fragment is one
-//          16-byte LDS read.
-// OpOuter  source is row-contiguous: element (r, kk) at view[(k0 + kk) * ld + r].
-//          LDS holds the tile as it lies in memory, [BK][ROWS + 32] (64 bytes of padding
-//          per k line); a fragment is two ds_read_b64_tr_b16, the gfx950 transposing LDS
-//          read: a group of 16 lanes addresses a block of 4 k lines x 16 columns (lane i
-//          points at line i/4, columns 4*(i%4)..+3) and lane i gets back column i of that
-//          block, i.e. 4 consecutive k of its own row.
-template <int ROWS_, int BK, int NT>
-struct OpInner {
-  static constexpr int ROWS = ROWS_;
-  static constexpr int LDK = BK + 8;
-  static constexpr int LDS_ELEMS = ROWS * LDK;
-  static constexpr int CPR = BK / 8;          // 16-byte chunks per row
-  static constexpr int CH = ROWS * CPR / NT;  // chunks per thread
-  static constexpr int RSTEP = NT / CPR;      // rows between a thread's consecutive chunks
-  static_assert((ROWS * CPR) % NT == 0 && NT % CPR == 0, "loader shape");
-  int voff[CH];  // byte offsets of this thread's chunks inside the view at k0 = 0
-  int lds_w;     // element offset of its first chunk in the LDS tile
-  int kc;        // first k of its chunks inside the tile
-  __device__ __forceinline__ void init(int ld) {
-    const int r = threadIdx.x / CPR;
-    kc = (threadIdx.x % CPR) * 8;
-#pragma unroll
-    for (int i = 0; i < CH; ++i) voff[i] = ((r + i * RSTEP) * ld + kc) * 2;
-    lds_w = r * LDK + kc;
-  }
-  static __device__ __forceinline__ long long k_bytes(int k0, int /*ld*/) { return (long long)k0 * 2; }
-  __device__ __forceinline__ u32x4 load_one(int i, __amdgpu_buffer_rsrc_t rs) const {
-    return __builtin_amdgcn_raw_buffer_load_b128(rs, voff[i], 0, 0);
-  }
-  // k beyond the end of the contraction lies in the next row of a k-contiguous source, so
-  // the hardware bound cannot catch it: such chunks are cleared by hand (k_left = valid k)
-  __device__ __forceinline__ bool past_k(int k_left) const { return kc >= k_left; }
-  __device__ __forceinline__ void store_one(int i, uint16_t* lds, u32x4 v) const {
-    *reinterpret_cast<u32x4*>(lds + lds_w + i * RSTEP * LDK) = v;
-  }
-  static __device__ __forceinline__ int lane_off(int lane) { return (lane & 31) * LDK + (lane >> 5) * 8; }
-  static __device__ __forceinline__ bf16x8 frag(const uint16_t* lds, int lane_offset, int row_base, int ks) {
-    return *reinterpret_cast<const bf16x8*>(lds + lane_offset + row_base * LDK + ks * 16);
-  }
-};
-
-template <int ROWS_, int BK, int NT>
-struct OpOuter {
-  static constexpr int ROWS = ROWS_;
-  static constexpr int LDN = ROWS + 32;
-  static constexpr int LDS_ELEMS = BK * LDN;
-  static constexpr int CPK = ROWS / 8;        // 16-byte chunks per k line
-  static constexpr int CH = BK * CPK / NT;
-  static constexpr int KSTEP = NT / CPK;      // k lines between a thread's consecutive chunks
-  static_assert((BK * CPK) % NT == 0 && NT % CPK == 0, "loader shape");
-  int voff[CH];
-  int lds_w;
-  __device__ __forceinline__ void init(int ld) {
-    const int kk = threadIdx.x / CPK, rc = (threadIdx.x % CPK) * 8;
-#pragma unroll
-    for (int i = 0; i < CH; ++i) voff[i] = ((kk + i * KSTEP) * ld + rc) * 2;
-    lds_w = kk * LDN + rc;
-  }
-  static __device__ __forceinline__ long long k_bytes(int k0, int ld) { return (long long)k0 * ld * 2; }
-  __device__ __forceinline__ u32x4 load_one(int i, __amdgpu_buffer_rsrc_t rs) const {
-    return __builtin_amdgcn_raw_buffer_load_b128(rs, voff[i], 0, 0);
-  }
-  // the k bound of this layout is the end of the view: the hardware zero-fills
-  __device__ __forceinline__ bool past_k(int) const { return false; }
-  __device__ __forceinline__ void store_one(int i, uint16_t* lds, u32x4 v) const {
-    *reinterpret_cast<u32x4*>(lds + lds_w + i * KSTEP * LDN) = v;
-  }
-  // lane l = 16*b + i: k line (b/2)*8 + i/4, columns 16*(b%2) + 4*(i%4) .. +3
-  static __device__ __forceinline__ int lane_off(int lane) {
-    const int i = lane & 15, b = lane >> 4;
-    return ((b >> 1) * 8 + (i >> 2)) * LDN + (b & 1) * 16 + (i & 3) * 4;
-  }
-  static __device__ __forceinline__ bf16x8 frag(const uint16_t* lds, int lane_offset, int row_base, int ks) {
-    const uint16_t* p = lds + lane_offset + ks * 16 * LDN + row_base;
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * LDN));
-    typedef __attribute__((ext_vector_type(8))) short s16x8;
-    const s16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return __builtin_bit_cast(bf16x8, r);
-  }
-};
-
-// Wait for this wave's LDS traffic, then meet the other waves.  Global loads stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 template <int MODE, typename Cfg>

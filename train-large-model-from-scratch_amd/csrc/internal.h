@@ -34,6 +34,23 @@ int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const
 // int64 expert ids to int32, values outside int32 to -1 (dispatch.hip).
 int moe_narrow_ids(const int64_t* ids, int64_t R, int32_t* out, hipStream_t s);
 
+// ---- weight gradients of small launches (wgrad.hip) ----
+// out [E,M,N] (+)= a^T b per expert, a [R,M] and b [R,N] with row strides lda and ldb; part: room for partial sums.
+struct MoeWgradStack {
+  const uint16_t *a, *b;
+  void* out;
+  float* part;
+  int64_t lda, ldb, M, N;
+  int dtype, accumulate;
+};
+// Bytes of each stack's part for R rows.
+int64_t moe_wgrad_multi_part_bytes(int64_t R, int64_t H, int64_t I);
+// The stacks (the first n_stacks, all of the size I x H or H x I) and, unless NULL, the router: a [T, M >= E] and b
+// [T,N] contracted in router_slices slices of router_rows rows (part [slices][M][N]), out [E,N].
+int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgradStack* router, const int32_t* offs,
+                    int64_t E, int64_t R, int64_t H, int64_t I, int64_t T, int64_t router_slices,
+                    int64_t router_rows, hipStream_t s);
+
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;
 constexpr int FEW_MAX_EXPERTS = 128;

@@ -191,29 +191,14 @@ struct FwdScratch {
   }
 };
 
-// Weight gradients of one stack: how the contraction over an expert's rows is cut.  The kernel makes
-// one workgroup per 256 x 256 tile of the result and expert; with few experts and small matrices that
-// is a fraction of the chip, and under skewed routing the tiles of the largest expert set the time.
-// Below half a round of the compute units every expert is cut into ceil(n_e / L) equal segments, L such
-// that the (ceil(R/L) + E) x tiles jobs about fill the chip once (at most 1024 segments); their fp32
-// partial sums are added per expert in a fixed order.  Decided from shapes alone: no look at the counts.
+// Whether the weight gradients go to the kernel that takes all stacks at once (wgrad.hip): where one stack's
+// 256 x 256 tiles are at most MULTI_ROUNDS for every compute unit.  Decided from shapes alone.  (64 tiles, Zipf: a
+// step of 8192 tokens 406 -> 362 us; 216 tiles: 401 -> 395; 512 tiles: 494 -> 514, so not there.)
 constexpr int64_t WTILE = 256;
-struct Segments {
-  int64_t L = 0, S_max = 0;
-};
-Segments wgrad_segments(int64_t E, int64_t M, int64_t N, int64_t R) {
-  Segments g;
-  const int64_t cus = moe_compute_units();
+constexpr int64_t MULTI_ROUNDS = 1;
+bool wgrad_multi(int64_t E, int64_t M, int64_t N, int64_t R) {
   const int64_t tiles = ((M + WTILE - 1) / WTILE) * ((N + WTILE - 1) / WTILE);
-  if (R == 0 || cus / (E * tiles) < 2) return g;
-  const int64_t free_cus = cus - E * tiles > tiles ? cus - E * tiles : tiles;
-  int64_t L = (R * tiles + free_cus - 1) / free_cus;
-  L = (L + 63) / 64 * 64;
-  if (L < 256) L = 256;
-  while ((R + L - 1) / L + E > 1024) L *= 2;
-  g.L = L;
-  g.S_max = moe_segments_by_length_max(R, E, L);
-  return g;
+  return R > 0 && E * tiles <= MULTI_ROUNDS * moe_compute_units();
 }
 
 // Router weight gradient: slices of the tokens play the experts of the weight-gradient kernel; as many as
@@ -237,9 +222,8 @@ RouterSlices router_slices(int64_t T, int64_t H, int64_t E) {
 
 struct BwdScratch {
   uint16_t *dyp, *dg, *dxp;
-  float *part, *dsel, *wpart, *rpart;
+  float *part, *dsel, *wpart[3], *rpart;
   uint16_t* dlogits;
-  int32_t *seg, *seg_start;
   BwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
     const int64_t R = T * k;
     dyp = (uint16_t*)s.take(R * H * 2);
@@ -250,10 +234,7 @@ struct BwdScratch {
     const RouterSlices rs = router_slices(T, H, E);
     dlogits = (uint16_t*)s.take(T * rs.Ep * 4);
     rpart = (float*)s.take(rs.slices * rs.Ep * H * 4);
-    const Segments g = wgrad_segments(E, I, H, R);
-    seg = (int32_t*)s.take((g.S_max + 1) * 4);
-    seg_start = (int32_t*)s.take((E + 1) * 4);
-    wpart = (float*)s.take(g.L ? g.S_max * I * H * 4 : 0);
+    for (float*& w : wpart) w = (float*)s.take(wgrad_multi(E, I, H, R) ? moe_wgrad_multi_part_bytes(R, H, I) : 0);
   }
 };
 
@@ -384,10 +365,10 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
       MOE_STEP("moe_combine_bwd", moe_combine_bwd(a->dout, (int)a->dout_dtype, nullptr, a->gates, a->pos_to_row, R, H,
                                                   k, ws.dyp, nullptr, stream));
   }
-  const Segments g = wgrad_segments(E, I, H, R);
-  // dg and du side by side where their two weight gradients can come out of one launch: both wanted into
-  // results of one kind, no 256-row tile of the stacked result across the halves, no row segments
-  const bool pair = R > 0 && a->dw[0] && a->dw[1] && I % WTILE == 0 && !g.L && a->dw_dtype[0] == a->dw_dtype[1] &&
+  const bool multi = wgrad_multi(E, I, H, R);
+  // dg and du side by side where their two weight gradients can come out of one launch of the tiled kernel: both
+  // wanted into results of one kind, no 256-row tile of the stacked result across the halves
+  const bool pair = R > 0 && a->dw[0] && a->dw[1] && I % WTILE == 0 && !multi && a->dw_dtype[0] == a->dw_dtype[1] &&
                     a->dw_accumulate[0] == a->dw_accumulate[1];
   uint16_t* dg = ws.dg;
   uint16_t* du = pair ? ws.dg + I : ws.dg + R * I;
@@ -395,37 +376,6 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
   MOE_STEP("moe_gemm_dgrad_down_swiglu_bwd_blocked",
            moe_gemm_dgrad_down_swiglu_bwd_blocked(ws.dyp, a->w2, a->gu, a->offs, E, R, H, I, dg, du, pair ? 2 * I : 0,
                                                   part, stream));
-  if (a->dx || a->dxp) {
-    if (pair)
-      MOE_STEP("moe_gemm_dgrad_gateup_packed",
-               moe_gemm_dgrad_gateup_packed(dg, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
-    else
-      MOE_STEP("moe_gemm_dgrad_gateup", moe_gemm_dgrad_gateup(dg, du, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
-  }
-  // weight gradients, down projection first: [dyp | act], [dg | xp], [du | xp]
-  if (g.L && (a->dw[0] || a->dw[1] || a->dw[2]))
-    MOE_STEP("moe_segment_offsets_by_length",
-             moe_segment_offsets_by_length(a->offs, E, g.L, g.S_max, ws.seg, ws.seg_start, stream));
-  const int order[3] = {2, 0, 1};
-  for (int n = 0; n < 3; ++n) {
-    const int w = order[n];
-    if (!a->dw[w]) continue;
-    if (pair && w == 1) continue;  // came with the gate stack's
-    const uint16_t* lhs = w == 2 ? ws.dyp : w == 0 ? dg : du;
-    const uint16_t* rhs = w == 2 ? a->act : a->xp;
-    const int64_t M = w == 2 ? H : I, N = w == 2 ? I : H;
-    const int dt = (int)a->dw_dtype[w], acc = a->dw_accumulate[w] ? 1 : 0;
-    if (pair && w == 0) {
-      MOE_STEP("moe_gemm_wgrad_pair",
-               moe_gemm_wgrad_pair(dg, a->xp, a->offs, E, R, I, H, a->dw[0], a->dw[1], dt, acc, stream));
-    } else if (g.L) {
-      MOE_STEP("moe_gemm_wgrad", moe_gemm_wgrad(lhs, rhs, ws.seg, g.S_max, R, M, N, ws.wpart, MOE_DT_F32, 0, stream));
-      MOE_STEP("moe_wgrad_reduce_segments",
-               moe_wgrad_reduce_segments(ws.wpart, ws.seg_start, E, M, N, a->dw[w], dt, acc, stream));
-    } else {
-      MOE_STEP("moe_gemm_wgrad", moe_gemm_wgrad(lhs, rhs, a->offs, E, R, M, N, a->dw[w], dt, acc, stream));
-    }
-  }
   if (a->dgates && R > 0)
     MOE_STEP("moe_dgates_from_blocks_by_pos", moe_dgates_from_blocks_by_pos(part, moe_dgate_blocks(I), a->gates,
                                                                             a->pos_to_row, R, a->dgates, stream));
@@ -438,11 +388,56 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
                                         own ? rs.Ep : E, own ? ws.dlogits : a->dlogits,
                                         own ? MOE_DT_BF16 : (int)a->dlogits_dtype, router ? ws.dsel : nullptr, st));
   }
-  if (router && to_logits && a->dwr) {
-    if (a->dlogits) return MOE_ERR_SHAPE;  // one or the other: the caller's dlogits are not padded
-    MOE_STEP("moe_wgrad_slices",
-             moe_wgrad_slices(ws.dlogits, a->xn, T, rs.Ep, H, rs.slices, rs.rows, ws.rpart, st));
-    MOE_STEP("moe_sum_slices", moe_sum_slices(ws.rpart, rs.slices, rs.Ep, E, H, a->dwr, (int)a->dwr_dtype, st));
+  if (a->dx || a->dxp) {
+    if (pair)
+      MOE_STEP("moe_gemm_dgrad_gateup_packed",
+               moe_gemm_dgrad_gateup_packed(dg, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
+    else
+      MOE_STEP("moe_gemm_dgrad_gateup", moe_gemm_dgrad_gateup(dg, du, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
+  }
+  const bool router_dw = router && to_logits && a->dwr;
+  if (router_dw && a->dlogits) return MOE_ERR_SHAPE;  // one or the other: the caller's dlogits are not padded
+  // weight gradients, down projection first: [dyp | act], [dg | xp], [du | xp]
+  MoeWgradStack stacks[3], rstack{};
+  int n_stacks = 0;
+  for (int w : {2, 0, 1}) {
+    if (!a->dw[w]) continue;
+    MoeWgradStack& m = stacks[n_stacks++];
+    m.a = w == 2 ? ws.dyp : w == 0 ? dg : du;
+    m.b = w == 2 ? a->act : a->xp;
+    m.M = w == 2 ? H : I;
+    m.N = w == 2 ? I : H;
+    m.lda = m.M, m.ldb = m.N;
+    m.out = a->dw[w];
+    m.part = ws.wpart[w];
+    m.dtype = (int)a->dw_dtype[w];
+    m.accumulate = a->dw_accumulate[w] ? 1 : 0;
+  }
+  if (router_dw) {
+    rstack.a = ws.dlogits, rstack.b = a->xn, rstack.out = a->dwr, rstack.part = ws.rpart;
+    rstack.M = rstack.lda = rs.Ep, rstack.N = rstack.ldb = H;
+    rstack.dtype = (int)a->dwr_dtype;
+  }
+  if (multi) {
+    if (n_stacks || router_dw)
+      MOE_STEP("moe_wgrad_multi", moe_wgrad_multi(stacks, n_stacks, router_dw ? &rstack : nullptr, a->offs, E, R, H, I, T,
+                                                  rs.slices, rs.rows, st));
+  } else {
+    for (int i = 0; i < n_stacks; ++i) {
+      const MoeWgradStack& m = stacks[i];
+      if (pair && m.out == a->dw[0]) {
+        MOE_STEP("moe_gemm_wgrad_pair", moe_gemm_wgrad_pair(dg, a->xp, a->offs, E, R, I, H, a->dw[0], a->dw[1], m.dtype,
+                                                            m.accumulate, stream));
+        ++i;  // the up stack's came with it
+        continue;
+      }
+      MOE_STEP("moe_gemm_wgrad", moe_gemm_wgrad(m.a, m.b, a->offs, E, R, m.M, m.N, m.out, m.dtype, m.accumulate, stream));
+    }
+    if (router_dw) {
+      MOE_STEP("moe_wgrad_slices",
+               moe_wgrad_slices(ws.dlogits, a->xn, T, rs.Ep, H, rs.slices, rs.rows, ws.rpart, st));
+      MOE_STEP("moe_sum_slices", moe_sum_slices(ws.rpart, rs.slices, rs.Ep, E, H, a->dwr, (int)a->dwr_dtype, st));
+    }
   }
   if (a->dx && T > 0) {
     if (router && to_logits)
