@@ -463,7 +463,8 @@ def fp32_config3(P, torch, dev, steps=3, warmup=1):
         torch.cuda.synchronize()
     finally:
         P.lib.load().observer = None
-    per = {"moe_f32_gemm_rows": 2, "moe_f32_gemm_wgrad": 2}  # flops per launch in units of R*H*I
+    per = {"moe_f32_gateup": 4, "moe_f32_gemm_rows": 2, "moe_f32_gemm_down_swiglu_bwd": 2,
+           "moe_f32_gemm_gateup_bwd": 4, "moe_f32_wgrads": 6}  # flops per launch in units of R*H*I
     recs, g_ms = [], 0.0
     for name, kms in watch.per_launch_ms(1):
         rec = {"entry": name, "ms": round(kms, 4)}

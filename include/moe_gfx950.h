@@ -444,7 +444,22 @@ int moe_f32_gemm_rows(const float* a, const float* b, const int32_t* offs, int64
  * Experts without rows get exact zeros (are left untouched when accumulating). */
 int moe_f32_gemm_wgrad(const float* a, const float* b, const int32_t* offs, int64_t E, int64_t R,
                        int64_t M, int64_t N, float* dw, int accumulate, void* stream);
-/* Test hook (no counterpart in the reference): the two fp32 GEMM entries choose 64 x 64 or
+/* The same products with what follows them fused in: g = xp W1^T, u = xp W3^T, act = silu(g) u; dg, du from dact = dyp W2 and the g and u of the forward; dxp = dg W1 + du W3;
+ * dw1 = dg^T xp, dw3 = du^T xp, dw2 = dyp^T act.  xp, dyp, dxp [R,H], g, u,
+ * act, dg, du [R,I], w1, w3, dw1, dw3 [E,I,H], w2, dw2 [E,H,I]. */
+int moe_f32_gemm_gateup_swiglu(const float* xp, const float* w1, const float* w3, const int32_t* offs,
+                               int64_t E, int64_t R, int64_t H, int64_t I, float* g, float* u, float* act,
+                               void* stream);
+int moe_f32_gemm_down_swiglu_bwd(const float* dyp, const float* w2, const float* g, const float* u,
+                                 const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I,
+                                 float* dg, float* du, void* stream);
+int moe_f32_gemm_gateup_bwd(const float* dg, const float* du, const float* w1, const float* w3,
+                            const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, float* dxp,
+                            void* stream);
+int moe_f32_gemm_wgrads(const float* dg, const float* du, const float* dyp, const float* xp,
+                        const float* act, const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I,
+                        float* dw1, float* dw3, float* dw2, void* stream);
+/* Test hook (no counterpart in the reference): the fp32 GEMM entries choose 64 x 64 or
  * 128 x 128 output tiles from the shapes; 64 or 128 forces one, 0 restores the choice.  Returns
  * the previous setting.  Process-wide, not synchronised. */
 int moe_f32_gemm_force_tile(int t);

@@ -22,6 +22,10 @@ void moe_observe(const char* name, int after);
 bool moe_router_few_ok(int64_t T, int64_t H, int64_t E, int64_t k);
 int moe_router_logits(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
                       void* stream);
+int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
+                   int64_t I, float* g, float* u, float* act, void* stream);
+int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
+                   int64_t E, int64_t R, int64_t H, int64_t I, float* dw1, float* dw3, float* dw2, void* stream);
 int moe_routed_forward(const uint16_t* x, const uint16_t* wr, uint16_t* logits, const float* bias, const uint16_t* w1,
                        const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k,
                        void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
@@ -577,9 +581,8 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
   CALL(moe_histogram_scan_checked, ids, R, E, r.part(f.routing, Routing::COUNTS), r.part(f.routing, Routing::OFFS),
        r.part(f.routing, Routing::POS_TO_ROW), r.part(f.routing, Routing::ROW_TO_POS), bad, ws.data_ptr(), wsb, s);
   CALL(moe_f32_gather_rows, x.data_ptr<float>(), p2r, T, R, H, k, xp, s);
-  CALL(moe_f32_gemm_rows, xp, f.w[0].data_ptr<float>(), offs, E, R, I, H, 1, g, 0, s);
-  CALL(moe_f32_gemm_rows, xp, f.w[1].data_ptr<float>(), offs, E, R, I, H, 1, u, 0, s);
-  CALL(moe_f32_swiglu_fwd, g, u, R * I, act, s);
+  CALL(moe_f32_gateup, xp, f.w[0].data_ptr<float>(), f.w[1].data_ptr<float>(), offs, E, R, H, I,
+       o.train ? g : nullptr, o.train ? u : nullptr, act, s);
   CALL(moe_f32_gemm_rows, act, f.w[2].data_ptr<float>(), offs, E, R, H, I, 1, y, 0, s);
   CALL(moe_f32_combine_fwd, y, gates, r2p, T, H, k, f.out.data_ptr<float>(), s);
   if (o.routing_out) *o.routing_out = f.routing;
@@ -625,28 +628,23 @@ struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
     const int32_t* r2p = r.part(routing, Routing::ROW_TO_POS);
     void* s = stream_of(kept_buf);
     const int64_t rh = up(R * H, 64), ri = up(R * I, 64);
-    const Tensor scratch = empty({2 * rh + 3 * ri + up(R, 64) + 64}, at::kFloat, kept_buf);
+    const Tensor scratch = empty({2 * rh + 2 * ri + up(R, 64) + 64}, at::kFloat, kept_buf);
     float* dyp = scratch.data_ptr<float>();
-    float *dxp = dyp + rh, *dact = dxp + rh, *dg = dact + ri, *du = dg + ri, *dgates = du + ri;
+    float *dxp = dyp + rh, *dg = dxp + rh, *du = dg + ri, *dgates = du + ri;
     CALL(moe_f32_combine_bwd, dout.data_ptr<float>(), want_gates ? y : nullptr, gates, p2r, T, R, H, k, dyp,
          want_gates ? dgates : nullptr, s);
-    CALL(moe_f32_gemm_rows, dyp, w2.data_ptr<float>(), offs, E, R, I, H, 0, dact, 0, s);
-    CALL(moe_f32_swiglu_bwd, dact, g, u, R * I, dg, du, s);
+    CALL(moe_f32_gemm_down_swiglu_bwd, dyp, w2.data_ptr<float>(), g, u, offs, E, R, H, I, dg, du, s);
     Tensor dx, dw1, dw3, dw2, dlogits, dbias;
     if (need(X)) {
       dx = empty({T, H}, at::kFloat, kept_buf);
-      CALL(moe_f32_gemm_rows, dg, w1.data_ptr<float>(), offs, E, R, H, I, 0, dxp, 0, s);
-      CALL(moe_f32_gemm_rows, du, w3.data_ptr<float>(), offs, E, R, H, I, 0, dxp, 1, s);
+      CALL(moe_f32_gemm_gateup_bwd, dg, du, w1.data_ptr<float>(), w3.data_ptr<float>(), offs, E, R, H, I, dxp, s);
       CALL(moe_f32_permute_bwd, dxp, r2p, T, H, k, dx.data_ptr<float>(), s);
     }
-    const auto wgrad = [&](const float* a, const float* b, int64_t M, int64_t N) {
-      Tensor dw = empty({E, M, N}, at::kFloat, kept_buf);
-      CALL(moe_f32_gemm_wgrad, a, b, offs, E, R, M, N, dw.data_ptr<float>(), 0, s);
-      return dw;
-    };
-    if (need(W1)) dw1 = wgrad(dg, xp, I, H);
-    if (need(W3)) dw3 = wgrad(du, xp, I, H);
-    if (need(W2)) dw2 = wgrad(dyp, act, H, I);
+    if (need(W1)) dw1 = empty({E, I, H}, at::kFloat, kept_buf);
+    if (need(W3)) dw3 = empty({E, I, H}, at::kFloat, kept_buf);
+    if (need(W2)) dw2 = empty({E, H, I}, at::kFloat, kept_buf);
+    CALL(moe_f32_wgrads, dg, du, dyp, xp, act, offs, E, R, H, I, (float*)ptr(dw1), (float*)ptr(dw3),
+         (float*)ptr(dw2), s);
     if (want_gates) {
       dlogits = empty({T, E}, at::kFloat, kept_buf);
       CALL(moe_router_topk_bwd, gates, dgates, r.part(routing, Routing::IDS), T, E, k, dlogits.data_ptr(), MOE_DT_F32, s);

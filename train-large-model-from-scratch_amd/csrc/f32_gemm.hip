@@ -1,0 +1,663 @@
+// Grouped (per-expert, ragged) GEMMs of the fp32 path on the matrix cores (v_mfma_f32_32x32x2_f32: fp32
+// operands, fp32 accumulation), and what is fused into them.
+//
+// An fp32 MFMA takes 64 cycles for 2048 multiply-adds, sixteen times as long per flop as a bf16 one, so
+// that neither LDS nor HBM bounds these kernels: what does is how evenly the chip's matrix pipes are
+// loaded and how much of the time they wait for a wave's own loads, barriers and address arithmetic.
+// Hence small workgroups (four waves), several of them on a compute unit, k-tiles requested at least two
+// iterations before their use, one barrier per iteration that leaves global loads in flight, output tiles of a quarter
+// of the size where the last round of tiles would leave compute units empty, and few launches: gate and up share
+// one (and with it their tiles), the two halves of the input gradient another, the three weight gradients a third.
+#include "internal.h"
+#include "tile_ops.h"
+
+namespace {
+
+constexpr int NT = 256;                    // threads
+constexpr unsigned OUTSIDE = 0xfffffff0u;  // a byte offset that no window reaches: reads as zero
+
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Operand chunks of 16 bytes are read through buffer resources, whose hardware bounds check makes an out-of-range
+// chunk a zero without a branch: chunks past the tile's rows or past the end of the contraction get the offset OUTSIDE.
+// A window is moved along k by its base, a scalar addition.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t window(const float* base, long long elems) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(base + elems), 0, 0x7fffffff, 0x00020000);
+}
+__device__ __forceinline__ f32x4 window_load(__amdgpu_buffer_rsrc_t rs, unsigned off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+}
+
+// Operand tiles of ROWS x TK.  Of each group of eight k values the lower half of a wave multiplies the first
+// four and the upper half the others (MFMA j takes k = j and j + 4; any pairing will do as long as both operands use
+// the same), so that an operand that lies k-contiguous in LDS is read 16 bytes at a time.
+//
+// KCont: element (r, k) at base[r * ld + k]; LDS [ROWS][TK + 4], the padding keeps 16-byte reads of 32 rows
+//        free of bank conflicts.
+// RCont: element (r, k) at base[k * ld + r]; LDS [TK][ROWS + 4], read a value at a time.
+template <int ROWS, int TK>
+struct KCont {
+  static constexpr int LD = TK + 4, ELEMS = ROWS * LD;
+  static constexpr int CPR = TK / 4, STEP = NT / CPR, CH = ROWS * CPR / NT;
+  static_assert(ROWS * CPR % NT == 0, "loader shape");
+  unsigned voff[CH];
+  int kc, at;
+  // Row of the tile that this thread's chunk i is of.  (TK = 16: a group of eight lanes writes two rows, which lie
+  // half the banks apart when they are four rows apart.)
+  static __device__ __forceinline__ int row(int i) {
+    const int q = threadIdx.x / CPR;
+    return (CPR == 4 ? (q & ~7) | (q & 1) << 2 | (q >> 1 & 3) : q) + i * STEP;
+  }
+  __device__ __forceinline__ void init(int ld, int rows) {  // rows: of the tile that exist
+    const int r = row(0);
+    kc = threadIdx.x % CPR * 4;
+    at = r * LD + kc;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) voff[i] = r + i * STEP < rows ? (unsigned)((r + i * STEP) * ld + kc) * 4u : OUTSIDE;
+  }
+  static __device__ __forceinline__ long long k_elems(int k0, int) { return k0; }
+  __device__ __forceinline__ f32x4 load(int i, __amdgpu_buffer_rsrc_t rs, int k_left) const {
+    return window_load(rs, kc < k_left ? voff[i] : OUTSIDE);  // (K % 4 == 0)
+  }
+  __device__ __forceinline__ void store(int i, float* lds, f32x4 v) const {
+    *reinterpret_cast<f32x4*>(lds + at + i * STEP * LD) = v;
+  }
+  static __device__ __forceinline__ f32x4 frag(const float* lds, int row0, int c) {
+    const int lane = threadIdx.x & 63;
+    return *reinterpret_cast<const f32x4*>(lds + (row0 + (lane & 31)) * LD + c * 8 + (lane >> 5) * 4);
+  }
+};
+template <int ROWS, int TK>
+struct RCont {
+  static constexpr int LD = ROWS + 4, ELEMS = TK * LD;
+  static constexpr int CPK = ROWS / 4, STEP = NT / CPK, CH = TK * CPK / NT;
+  static_assert(TK * CPK % NT == 0, "loader shape");
+  unsigned voff[CH];
+  int kk, at;
+  __device__ __forceinline__ void init(int ld, int rows) {
+    const int r = threadIdx.x % CPK * 4;
+    kk = threadIdx.x / CPK;
+    at = kk * LD + r;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) voff[i] = r < rows ? (unsigned)((kk + i * STEP) * ld + r) * 4u : OUTSIDE;  // (rows % 4 == 0)
+  }
+  static __device__ __forceinline__ long long k_elems(int k0, int ld) { return (long long)k0 * ld; }
+  __device__ __forceinline__ f32x4 load(int i, __amdgpu_buffer_rsrc_t rs, int k_left) const {
+    return window_load(rs, kk + i * STEP < k_left ? voff[i] : OUTSIDE);
+  }
+  __device__ __forceinline__ void store(int i, float* lds, f32x4 v) const {
+    *reinterpret_cast<f32x4*>(lds + at + i * STEP * LD) = v;
+  }
+  static __device__ __forceinline__ f32x4 frag(const float* lds, int row0, int c) {
+    const int lane = threadIdx.x & 63;
+    const float* p = lds + (c * 8 + (lane >> 5) * 4) * LD + row0 + (lane & 31);
+    return f32x4{p[0], p[LD], p[2 * LD], p[3 * LD]};
+  }
+};
+
+// An output tile of BM x BN over k-tiles of TK.  The four waves are WM x WN x WK: each has BM/WM x BN/WN of it as
+// NM x NN blocks of 32 x 32, and one of WK equal shares of every k-tile (WK > 1: fold() adds the shares up).
+// PF: k-tiles held in registers on their way to LDS.
+template <int BM_, int BN_, int TK_, int WM_, int WN_, int PF_>
+struct Shape {
+  static constexpr int BM = BM_, BN = BN_, TK = TK_, WM = WM_, WN = WN_, WK = 4 / (WM * WN), PF = PF_;
+  static constexpr int NM = BM / WM / 32, NN = BN / WN / 32, CK = TK / 8 / WK;  // CK: groups of eight k values per wave
+  static constexpr int WAVES = NM * NN > 1 ? 3 : 4;  // per SIMD, at least
+  static_assert(WM * WN * WK == 4 && NM > 0 && NN > 0 && CK > 0 && PF % 2 == 0, "shape");
+};
+
+// The k loop: acc = A-tile x B-tile over `n` > 0 k-tiles.  k-tile t is requested (`load`) while t - 1 - PF is
+// multiplied, written to LDS (two stages) while t - 1 is.  The operands go into the MFMA swapped: a lane ends up with row
+// lane % 32 of a block and four consecutive columns per group of four registers (columns 8g + 4*(lane/32) .. +3).
+template <typename S, typename OpA, typename OpB>
+struct Loop {
+  static constexpr int CH = OpA::CH + OpB::CH, STAGES = 2 * (OpA::ELEMS + OpB::ELEMS);
+  static constexpr int LDS_FLOATS = S::WK > 1 && STAGES < 4 * 1024 ? 4 * 1024 : STAGES;
+  typedef f32x16 Acc[S::NM][S::NN];
+  struct Stage {
+    f32x4 v[CH];
+  };
+  template <typename Load>
+  static __device__ __forceinline__ void run(float* lds, const OpA& opA, const OpB& opB, int n, bool idle, int wv, Acc& acc,
+                                             Load&& load) {
+    if (idle) loop(std::true_type{}, lds, opA, opB, n, wv, acc, load);
+    else loop(std::false_type{}, lds, opA, opB, n, wv, acc, load);
+  }
+  // Idle: a wave without rows only moves its share of the operands and meets the barriers
+  template <typename Idle, typename Load>
+  static __device__ __forceinline__ void loop(Idle, float* lds, const OpA& opA, const OpB& opB, int n, int wv, Acc& acc,
+                                              Load& load) {
+    const int wk = wv / (S::WM * S::WN), wm = wv / S::WN % S::WM, wn = wv % S::WN;
+#pragma unroll
+    for (int i = 0; i < S::NM; ++i)
+#pragma unroll
+      for (int j = 0; j < S::NN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    const auto stage_a = [&](int b) { return lds + b * OpA::ELEMS; };
+    const auto stage_b = [&](int b) { return lds + 2 * OpA::ELEMS + b * OpB::ELEMS; };
+    const auto put = [&](const Stage& s, int b) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        if (c < OpA::CH) opA.store(c, stage_a(b), s.v[c]);
+        else opB.store(c - OpA::CH, stage_b(b), s.v[c]);
+      }
+    };
+    Stage st[S::PF];
+    const auto step = [&](int t, auto at) {  // at: t modulo PF
+      constexpr int b = decltype(at)::value & 1, next = (decltype(at)::value + 1) % S::PF;
+      f32x4 fa[S::CK][S::NM], fb[S::CK][S::NN];
+      if constexpr (!Idle::value) {
+#pragma unroll
+        for (int c = 0; c < S::CK; ++c) {
+#pragma unroll
+          for (int x = 0; x < S::NM; ++x) fa[c][x] = OpA::frag(stage_a(b), (wm * S::NM + x) * 32, wk * S::CK + c);
+#pragma unroll
+          for (int x = 0; x < S::NN; ++x) fb[c][x] = OpB::frag(stage_b(b), (wn * S::NN + x) * 32, wk * S::CK + c);
+        }
+      }
+      put(st[next], b ^ 1);
+      load(t + 1 + S::PF, st[next]);
+      if constexpr (!Idle::value) {
+#pragma unroll
+        for (int c = 0; c < S::CK; ++c)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int x = 0; x < S::NM; ++x)
+#pragma unroll
+              for (int y = 0; y < S::NN; ++y)
+                acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[c][y][j], fa[c][x][j], acc[x][y], 0, 0, 0);
+      }
+      lds_barrier();
+    };
+    const auto steps = [&](int t, int count, auto... at) { ((decltype(at)::value < count ? step(t + decltype(at)::value, at) : void()), ...); };
+    const auto round = [&](int t, int count) {
+      if constexpr (S::PF == 2) steps(t, count, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
+      else steps(t, count, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{},
+                 std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
+    };
+    static_assert(S::PF == 2 || S::PF == 4, "rounds of two or four");
+#pragma unroll
+    for (int i = 0; i < S::PF; ++i) load(i, st[i]);
+    put(st[0], 0);
+    load(S::PF, st[0]);
+    lds_barrier();
+    int t = 0;
+    for (; t + S::PF <= n; t += S::PF) round(t, S::PF);
+    if (t < n) round(t, n - t);
+  }
+  // WK > 1 (one block per wave): wave w gets the sum, in the order of the shares, of group `g` of the block
+  static __device__ __forceinline__ void give(float* lds, int wv, const Acc& acc) {
+    static_assert(S::WK == 4 && S::NM == 1 && S::NN == 1, "one block, four shares");
+    f32x4* x = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) x[(wv * 4 + g) * 64 + (threadIdx.x & 63)] = quad(acc[0][0], g);
+    lds_barrier();
+  }
+  static __device__ __forceinline__ f32x4 taken(const float* lds, int g) {
+    const f32x4* x = reinterpret_cast<const f32x4*>(lds) + g * 64 + (threadIdx.x & 63);
+    return ((x[0] + x[4 * 64]) + x[8 * 64]) + x[12 * 64];
+  }
+  static __device__ __forceinline__ f32x4 quad(const f32x16& a, int g) {
+    return f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+  }
+};
+
+struct RowsArgs {
+  const float *A0, *A1, *B0, *B1;  // A [R, K], B one stack of [E][N][K] or [E][K][N]; the second of each: see the modes
+  const float *X0, *X1;            // SwiGLU backward: g and u [R, N]
+  float *C0, *C1, *C2;             // [R, N]
+  const int32_t* offs;
+  int E, R, N, K, accumulate;
+};
+
+// PLAIN_T  C0 (+)= A0 B0^T, B0 [N][K]
+// PLAIN_N  C0 (+)= A0 B0, B0 [K][N]
+// GATEUP   g = A0 B0^T, u = A0 B1^T, both [N][K], half a tile of columns each: two waves hold g, two u of the same
+//          columns; C2 = silu(g) * u, and C0 = g, C1 = u unless they are null
+// DOWN_BWD d = A0 B0 as PLAIN_N; C0 = dg = d * u * silu'(g), C1 = du = d * silu(g)
+// GATEUP_BWD C0 = A0 B0 + A1 B1 as PLAIN_N, one after the other
+enum Mode { PLAIN_T, PLAIN_N, GATEUP, DOWN_BWD, GATEUP_BWD };
+
+__device__ __forceinline__ int expert_rows(const RowsArgs& p, int e, int& first) {
+  first = 0;
+  if (e >= p.E) return 0;
+  const int b = p.offs[e], n = p.offs[e + 1] - b;
+  first = b;
+  return n <= 0 || b < 0 || n > p.R - b ? 0 : n;  // (empty, or offsets that no dispatch would produce)
+}
+__device__ __forceinline__ int wave_inclusive(int v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < MOE_WAVE; o <<= 1) {
+    const int u = __shfl_up(v, o, MOE_WAVE);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+
+
+__device__ __forceinline__ float sigmoid_f32(float x) { return 1.f / (1.f + expf(-x)); }
+
+// Which tile a workgroup computes.  The hardware hands workgroup b to XCD b % 8, each with an L2 of its own: XCD x takes
+// the x-th contiguous eighth of the list, whose workgroups share a few row tiles and one or two experts' weights
+// there.  The tiles after the last full round of one per compute unit are cut into four each, unless they nearly fill
+// another round: 4.25 rounds of tiles then take the time of about 4.25 and not of 5.  (4096 rows of 8 experts, 1024 <-> 512:
+// 89 us in whole tiles, 79 with the last quarter round cut; a chip's worth of small tiles keeps more launches of fewer
+// tiles than compute units busy, too.)
+struct Job {
+  int tile, part;  // part: 0..3 of the tile, -1: all of it; tile < 0: none
+};
+__device__ __forceinline__ Job job_of(int tiles, int cus) {
+  const int rest = tiles % cus, cut = rest * 4 <= cus * 3 ? rest : 0, whole = tiles - cut;
+  const int x = blockIdx.x & 7;
+  int j = blockIdx.x >> 3;
+  const int q = whole / 8, r = whole % 8, mine = q + (x < r ? 1 : 0);
+  if (j < mine) return Job{x * q + (x < r ? x : r) + j, -1};
+  j -= mine;
+  const int q4 = cut * 4 / 8, r4 = cut * 4 % 8;
+  if (j >= q4 + (x < r4 ? 1 : 0)) return Job{-1, 0};  // (the grid is sized for the most there can be)
+  const int at = x * q4 + (x < r4 ? x : r4) + j;
+  return Job{whole + at / 4, at % 4};
+}
+// Workgroups for at most `tiles` tiles: each XCD may round its two shares up.
+unsigned grid_of(int64_t tiles, int64_t cus) { return (unsigned)((tiles + 3 * (cus * 3 / 4) + 7) / 8 * 8 + 16); }
+
+template <int MODE>
+constexpr bool b_kcont = MODE == PLAIN_T || MODE == GATEUP;
+template <int MODE, typename S>
+using RowsB = typename std::conditional<b_kcont<MODE>, KCont<S::BN, S::TK>, RCont<S::BN, S::TK>>::type;
+template <int MODE, typename S>
+using RowsLoop = Loop<S, KCont<S::BM, S::TK>, RowsB<MODE, S>>;
+constexpr int larger(int a, int b) { return a > b ? a : b; }
+
+// The tile of Shape S at rows row0.. (of the expert's up to row_end), columns n0..
+template <int MODE, typename S>
+__device__ __forceinline__ void rows_tile(const RowsArgs& p, float* lds, int e, int row0, int row_end, int n0) {
+  constexpr bool B_KCONT = b_kcont<MODE>, DUAL = MODE == GATEUP;
+  using OpA = KCont<S::BM, S::TK>;
+  using OpB = RowsB<MODE, S>;
+  using L = RowsLoop<MODE, S>;
+  const int lane = threadIdx.x & 63, wv = uniform((int)(threadIdx.x >> 6));
+  const int ldb = B_KCONT ? p.K : p.N;
+  OpA opA;
+  OpB opB;
+  opA.init(p.K, row_end - row0);
+  opB.init(ldb, p.N - n0);
+  // GATEUP: each 32 columns of the product are 16 of g and 16 of u, so that a lane holds both of a place
+  const auto is_up = [&](int c) {  // (the same for a whole wave)
+    if constexpr (DUAL) {
+      static_assert(16 % (64 / OpB::CPR) == 0, "a wave's chunks lie in 16 rows");
+      return ((wv * (64 / OpB::CPR) + c * OpB::STEP) & 16) != 0;
+    }
+    return false;
+  };
+  if constexpr (DUAL) {
+#pragma unroll
+    for (int i = 0; i < OpB::CH; ++i) {
+      const int rr = OpB::row(i), r = rr / 32 * 16 + (rr & 15);
+      opB.voff[i] = r < p.N - n0 ? (unsigned)(r * p.K + opB.kc) * 4u : OUTSIDE;
+    }
+  }
+  const long long wofs = (long long)e * p.N * p.K + (long long)n0 * (B_KCONT ? p.K : 1);
+  const float *A0 = p.A0 + (long long)row0 * p.K, *B0 = p.B0 + wofs;
+  const float *A1 = p.A1 + (long long)row0 * p.K, *B1 = p.B1 + wofs;  // (null and unused outside the two-operand modes)
+  const int per_seg = (p.K + S::TK - 1) / S::TK;
+  auto load = [&](int t, typename L::Stage& s) {
+    int k0 = t * S::TK;
+    const bool second = MODE == GATEUP_BWD && t >= per_seg;
+    if (second) k0 -= per_seg * S::TK;
+    const __amdgpu_buffer_rsrc_t ra = window(second ? A1 : A0, OpA::k_elems(k0, p.K));
+#pragma unroll
+    for (int c = 0; c < OpA::CH; ++c) s.v[c] = opA.load(c, ra, p.K - k0);
+#pragma unroll
+    for (int c = 0; c < OpB::CH; ++c)
+      s.v[OpA::CH + c] = opB.load(c, window(second || is_up(c) ? B1 : B0, OpB::k_elems(k0, ldb)), p.K - k0);
+  };
+  typename L::Acc acc;
+  const int wm = wv / S::WN % S::WM, wn = wv % S::WN;
+  const bool idle = uniform((int)(row0 + wm * S::NM * 32 >= row_end)) != 0;
+  L::run(lds, opA, opB, MODE == GATEUP_BWD ? 2 * per_seg : per_seg, idle, wv, acc, load);
+
+  // ---- results: a lane holds four consecutive columns of one row at a time
+  const auto emit = [&](int m, int n, f32x4 v, f32x4 u) {
+    if (m >= row_end || n >= p.N) return;  // (N % 4 == 0: the four columns are inside or outside together)
+    const long long at = (long long)m * p.N + n;
+    if constexpr (DUAL) {
+      f32x4 a;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) a[c] = v[c] * sigmoid_f32(v[c]) * u[c];
+      if (p.C0) {
+        *reinterpret_cast<f32x4*>(p.C0 + at) = v;
+        *reinterpret_cast<f32x4*>(p.C1 + at) = u;
+      }
+      *reinterpret_cast<f32x4*>(p.C2 + at) = a;
+    } else if constexpr (MODE == DOWN_BWD) {  // silu'(g) = s * (1 + g * (1 - s)), s = sigmoid(g)
+      const f32x4 gv = *reinterpret_cast<const f32x4*>(p.X0 + at), uv = *reinterpret_cast<const f32x4*>(p.X1 + at);
+      f32x4 dg, du;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float s = sigmoid_f32(gv[c]);
+        dg[c] = v[c] * uv[c] * (s * (1.f + gv[c] * (1.f - s)));
+        du[c] = v[c] * (gv[c] * s);
+      }
+      *reinterpret_cast<f32x4*>(p.C0 + at) = dg;
+      *reinterpret_cast<f32x4*>(p.C1 + at) = du;
+    } else {
+      if (p.accumulate) v += *reinterpret_cast<const f32x4*>(p.C0 + at);
+      *reinterpret_cast<f32x4*>(p.C0 + at) = v;
+    }
+  };
+  const int l32 = lane & 31, lh = lane >> 5;
+  if constexpr (S::WK > 1) {
+    L::give(lds, wv, acc);
+    if (DUAL && wv >= 2) return;
+    const f32x4 v = L::taken(lds, wv), u = DUAL ? L::taken(lds, wv + 2) : v;
+    emit(row0 + l32, n0 + 8 * wv + 4 * lh, v, u);
+  } else if (!idle) {
+#pragma unroll
+    for (int bi = 0; bi < S::NM; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < S::NN; ++bj)
+#pragma unroll
+        for (int g = 0; g < (DUAL ? 2 : 4); ++g)
+          emit(row0 + (wm * S::NM + bi) * 32 + l32, n0 + (wn * S::NN + bj) * (DUAL ? 16 : 32) + 8 * g + 4 * lh,
+               L::quad(acc[bi][bj], g), L::quad(acc[bi][bj], DUAL ? g + 2 : g));
+  }
+}
+
+// Tiles are numbered row tile by row tile (an expert's last one may be short), column tiles fastest; S is a whole
+// tile, Q a quarter of one.
+template <int MODE, typename S, typename Q>
+__global__ __launch_bounds__(NT, S::WAVES) void f32_rows_kernel(const RowsArgs p, int cus) {
+  static_assert(S::BM == 2 * Q::BM && S::BN == 2 * Q::BN, "a quarter");
+  constexpr int TN = MODE == GATEUP ? S::BN / 2 : S::BN;  // columns of a tile
+  __shared__ __align__(16) float lds[larger(RowsLoop<MODE, S>::LDS_FLOATS, RowsLoop<MODE, Q>::LDS_FLOATS)];
+  const int lane = threadIdx.x & 63, n_col = (p.N + TN - 1) / TN;
+  int tiles = 0;
+  for (int e0 = 0; e0 < p.E; e0 += MOE_WAVE) {
+    int first;
+    const int nt = (expert_rows(p, e0 + lane, first) + S::BM - 1) / S::BM;
+    tiles += uniform(__shfl(wave_inclusive(nt), MOE_WAVE - 1, MOE_WAVE));
+  }
+  const Job job = job_of(tiles * n_col, cus);
+  if (job.tile < 0) return;
+  const int row_tile = job.tile / n_col;
+  int n0 = job.tile % n_col * TN, e = 0, row0 = 0, row_end = 0;
+  for (int e0 = 0, seen = 0; e0 < p.E; e0 += MOE_WAVE) {
+    int first;
+    const int n = expert_rows(p, e0 + lane, first), nt = (n + S::BM - 1) / S::BM, incl = seen + wave_inclusive(nt);
+    const unsigned long long past = __ballot(incl > row_tile);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      e = e0 + l;
+      row0 = uniform(__shfl(first + (row_tile - (incl - nt)) * S::BM, l, MOE_WAVE));
+      row_end = uniform(__shfl(first + n, l, MOE_WAVE));
+      break;
+    }
+    seen = uniform(__shfl(incl, MOE_WAVE - 1, MOE_WAVE));
+  }
+  if (job.part < 0) {
+    rows_tile<MODE, S>(p, lds, e, row0, row_end, n0);
+  } else {
+    row0 += (job.part >> 1) * Q::BM;
+    n0 += (job.part & 1) * (TN / 2);
+    if (row0 < row_end && n0 < p.N) rows_tile<MODE, Q>(p, lds, e, row0, row_end, n0);
+  }
+}
+
+// Weight gradients: per stack C_e[m, n] (+)= sum over the rows r of expert e of A[r, m] * B[r, n], up to three stacks in
+// one launch.  Tiles are numbered stack by stack and expert by expert: the workgroups that an XCD runs side by side walk
+// the rows of one or two experts together and find them in its L2.  An expert without rows gets zeros (or is
+// left alone when accumulating).
+struct F32Stack {
+  const float *a, *b;  // [R, M], [R, N]
+  float* c;            // [E, M, N]
+  int M, N, accumulate;
+};
+struct WgradArgs {
+  F32Stack s[3];
+  const int32_t* offs;
+  int n, E, R;
+};
+
+template <typename S>
+using WgradLoop = Loop<S, RCont<S::BM, S::TK>, RCont<S::BN, S::TK>>;
+template <typename S>
+__device__ __forceinline__ void wgrad_tile(const F32Stack& s, float* lds, int e, int b, int end, int m0, int n0) {
+  using OpA = RCont<S::BM, S::TK>;
+  using OpB = RCont<S::BN, S::TK>;
+  using L = WgradLoop<S>;
+  const int lane = threadIdx.x & 63, wv = uniform((int)(threadIdx.x >> 6));
+  OpA opA;
+  OpB opB;
+  opA.init(s.M, s.M - m0);
+  opB.init(s.N, s.N - n0);
+  const float *A = s.a + (long long)b * s.M + m0, *B = s.b + (long long)b * s.N + n0;
+  auto load = [&](int t, typename L::Stage& st) {
+    const int left = end - b - t * S::TK;
+    const __amdgpu_buffer_rsrc_t ra = window(A, OpA::k_elems(t * S::TK, s.M)), rb = window(B, OpB::k_elems(t * S::TK, s.N));
+#pragma unroll
+    for (int c = 0; c < OpA::CH; ++c) st.v[c] = opA.load(c, ra, left);
+#pragma unroll
+    for (int c = 0; c < OpB::CH; ++c) st.v[OpA::CH + c] = opB.load(c, rb, left);
+  };
+  typename L::Acc acc;
+  const int n = (end - b + S::TK - 1) / S::TK;  // (without rows: one k-tile of zeros)
+  L::run(lds, opA, opB, n > 0 ? n : 1, false, wv, acc, load);
+  if (end == b && s.accumulate) return;
+  float* C = s.c + (long long)e * s.M * s.N;
+  const auto emit = [&](int m, int n, f32x4 v) {
+    if (m >= s.M || n >= s.N) return;
+    f32x4* dst = reinterpret_cast<f32x4*>(C + (long long)m * s.N + n);
+    if (s.accumulate) v += *dst;
+    *dst = v;
+  };
+  const int l32 = lane & 31, lh = lane >> 5, wm = wv / S::WN % S::WM, wn = wv % S::WN;
+  if constexpr (S::WK > 1) {
+    L::give(lds, wv, acc);
+    emit(m0 + l32, n0 + 8 * wv + 4 * lh, L::taken(lds, wv));
+  } else {
+#pragma unroll
+    for (int bi = 0; bi < S::NM; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < S::NN; ++bj)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          emit(m0 + (wm * S::NM + bi) * 32 + l32, n0 + (wn * S::NN + bj) * 32 + 8 * g + 4 * lh, L::quad(acc[bi][bj], g));
+  }
+}
+
+template <typename S, typename Q>
+__global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs p, int cus) {
+  __shared__ __align__(16) float lds[larger(WgradLoop<S>::LDS_FLOATS, WgradLoop<Q>::LDS_FLOATS)];
+  int per_e[3], n_col[3], tiles = 0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    n_col[i] = i < p.n ? (p.s[i].N + S::BN - 1) / S::BN : 0;
+    per_e[i] = i < p.n ? n_col[i] * ((p.s[i].M + S::BM - 1) / S::BM) : 0;
+    tiles += per_e[i] * p.E;
+  }
+  Job job = job_of(tiles, cus);
+  if (job.tile < 0) return;
+  int w = 0, pe = per_e[0], nc = n_col[0];
+#pragma unroll
+  for (int i = 1; i < 3; ++i)
+    if (w == i - 1 && job.tile >= per_e[i - 1] * p.E) {
+      job.tile -= per_e[i - 1] * p.E;
+      w = i, pe = per_e[i], nc = n_col[i];
+    }
+  const F32Stack s = p.s[w];
+  const int e = job.tile / pe;
+  int m0 = job.tile % pe / nc * S::BM, n0 = job.tile % pe % nc * S::BN;
+  int b = p.offs[e], end = p.offs[e + 1];
+  if (b < 0 || end > p.R || end < b) b = end = 0;
+  if (job.part < 0) {
+    wgrad_tile<S>(s, lds, e, b, end, m0, n0);
+  } else {
+    m0 += (job.part >> 1) * Q::BM;
+    n0 += (job.part & 1) * Q::BN;
+    if (m0 < s.M && n0 < s.N) wgrad_tile<Q>(s, lds, e, b, end, m0, n0);
+  }
+}
+
+using Small = Shape<64, 64, 32, 2, 2, 2>;    // four of them on a compute unit by their LDS
+using Quarter = Shape<32, 32, 32, 1, 1, 4>;  // of Small: the four waves share the contraction
+using Large = Shape<128, 128, 16, 2, 2, 2>;  // three by their registers
+using LargeQuarter = Shape<64, 64, 16, 2, 2, 2>;
+
+int forced_tile = 0;
+// The large tile has half the operand traffic and LDS reads per flop (32768 rows of 8 experts, 2048 <-> 1024, gate and up: 1.99
+// against 2.17 ms, 138 TFLOP/s), but few of them share a compute unit less evenly (8192 rows of 16 experts, 1024 <-> 1024, five
+// rounds of large tiles: 335 against 295 us; three rounds: equal): from eight rounds on.
+bool large_tiles(int64_t tiles128) {
+  if (forced_tile) return forced_tile == 128;
+  return tiles128 >= 8 * (int64_t)moe_compute_units();
+}
+
+int check_rows(int64_t E, int64_t R, int64_t N, int64_t K) {
+  for (int64_t width : {N, K})
+    if (width <= 0 || width % 4 != 0) return MOE_ERR_SHAPE;
+  if (E <= 0 || R < 0) return MOE_ERR_SHAPE;
+  if (E > 1024 || R > (int64_t)1 << 30 || N > 65536 || K > 65536) return MOE_ERR_LIMIT;
+  if ((R / 64 + E) * ((N + 31) / 32) > 0x70000000ll) return MOE_ERR_LIMIT;
+  return 0;
+}
+
+template <int MODE>
+int launch_rows(RowsArgs a, int64_t E, int64_t R, int64_t N, int64_t K, hipStream_t s) {
+  a.E = (int)E, a.R = (int)R, a.N = (int)N, a.K = (int)K;
+  const int cus = moe_compute_units();
+  const auto tiles = [&](int64_t t) { return (R / t + E) * ((N * (MODE == GATEUP ? 2 : 1) + t - 1) / t); };  // at most
+  if (large_tiles(tiles(128)))
+    hipLaunchKernelGGL((f32_rows_kernel<MODE, Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, s, a, cus);
+  else
+    hipLaunchKernelGGL((f32_rows_kernel<MODE, Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, s, a, cus);
+  return moe_launch_status();
+}
+
+}  // namespace
+
+extern "C" int moe_f32_gemm_rows(const float* a, const float* b, const int32_t* offs, int64_t E, int64_t R, int64_t N,
+                                 int64_t K, int b_k_contiguous, float* c, int accumulate, void* stream) {
+  if (int rc = check_rows(E, R, N, K)) return rc;
+  if (R == 0) return 0;
+  MOE_CHECK_PTR(a);
+  MOE_CHECK_PTR(b);
+  MOE_CHECK_PTR(c);
+  if (!offs) return MOE_ERR_NULL;
+  RowsArgs p{};
+  p.A0 = a, p.B0 = b, p.C0 = c, p.offs = offs, p.accumulate = accumulate;
+  return b_k_contiguous ? launch_rows<PLAIN_T>(p, E, R, N, K, (hipStream_t)stream)
+                        : launch_rows<PLAIN_N>(p, E, R, N, K, (hipStream_t)stream);
+}
+
+// (g and u null: not stored)
+int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
+                   int64_t I, float* g, float* u, float* act, void* stream) {
+  if (int rc = check_rows(E, R, I, H)) return rc;
+  if (R == 0) return 0;
+  for (const float* q : {xp, w1, w3, (const float*)act}) MOE_CHECK_PTR(q);
+  if (!offs) return MOE_ERR_NULL;
+  RowsArgs p{};
+  p.A0 = xp, p.B0 = w1, p.B1 = w3, p.C0 = g, p.C1 = u, p.C2 = act, p.offs = offs;
+  return launch_rows<GATEUP>(p, E, R, I, H, (hipStream_t)stream);
+}
+
+extern "C" int moe_f32_gemm_gateup_swiglu(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E,
+                                          int64_t R, int64_t H, int64_t I, float* g, float* u, float* act, void* stream) {
+  if (R > 0) {
+    MOE_CHECK_PTR(g);
+    MOE_CHECK_PTR(u);
+  }
+  return moe_f32_gateup(xp, w1, w3, offs, E, R, H, I, g, u, act, stream);
+}
+
+extern "C" int moe_f32_gemm_down_swiglu_bwd(const float* dyp, const float* w2, const float* g, const float* u,
+                                            const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, float* dg,
+                                            float* du, void* stream) {
+  if (int rc = check_rows(E, R, I, H)) return rc;
+  if (R == 0) return 0;
+  for (const float* q : {dyp, w2, g, u, (const float*)dg, (const float*)du}) MOE_CHECK_PTR(q);
+  if (!offs) return MOE_ERR_NULL;
+  RowsArgs p{};
+  p.A0 = dyp, p.B0 = w2, p.X0 = g, p.X1 = u, p.C0 = dg, p.C1 = du, p.offs = offs;
+  return launch_rows<DOWN_BWD>(p, E, R, I, H, (hipStream_t)stream);
+}
+
+extern "C" int moe_f32_gemm_gateup_bwd(const float* dg, const float* du, const float* w1, const float* w3,
+                                       const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, float* dxp,
+                                       void* stream) {
+  if (int rc = check_rows(E, R, H, I)) return rc;
+  if (R == 0) return 0;
+  for (const float* q : {dg, du, w1, w3, (const float*)dxp}) MOE_CHECK_PTR(q);
+  if (!offs) return MOE_ERR_NULL;
+  RowsArgs p{};
+  p.A0 = dg, p.A1 = du, p.B0 = w1, p.B1 = w3, p.C0 = dxp, p.offs = offs;
+  return launch_rows<GATEUP_BWD>(p, E, R, H, I, (hipStream_t)stream);
+}
+
+static int wgrads(const F32Stack* s, int n, const int32_t* offs, int64_t E, int64_t R, hipStream_t st) {
+  if (n < 0 || n > 3) return MOE_ERR_SHAPE;
+  if (n == 0) return 0;
+  if (!offs) return MOE_ERR_NULL;
+  WgradArgs p{};
+  p.offs = offs, p.n = n, p.E = (int)E, p.R = (int)R;
+  const auto tiles = [&](int64_t t) {
+    int64_t b = 0;
+    for (int i = 0; i < n; ++i) b += E * ((s[i].M + t - 1) / t) * ((s[i].N + t - 1) / t);
+    return b;
+  };
+  for (int i = 0; i < n; ++i) {
+    if (int rc = check_rows(E, R, s[i].M, s[i].N)) return rc;
+    MOE_CHECK_PTR(s[i].c);
+    if (R > 0) {
+      MOE_CHECK_PTR(s[i].a);
+      MOE_CHECK_PTR(s[i].b);
+    }
+    p.s[i] = s[i];
+  }
+  if (tiles(64) > 0x70000000ll) return MOE_ERR_LIMIT;
+  const int cus = moe_compute_units();
+  if (large_tiles(tiles(128)))
+    hipLaunchKernelGGL((f32_wgrad_kernel<Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, st, p, cus);
+  else
+    hipLaunchKernelGGL((f32_wgrad_kernel<Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, st, p, cus);
+  return moe_launch_status();
+}
+
+// (a null result is not computed)
+int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
+                   int64_t E, int64_t R, int64_t H, int64_t I, float* dw1, float* dw3, float* dw2, void* stream) {
+  if (H > 65536 || I > 65536) return MOE_ERR_LIMIT;
+  const F32Stack all[3] = {{dg, xp, dw1, (int)I, (int)H, 0}, {du, xp, dw3, (int)I, (int)H, 0}, {dyp, act, dw2, (int)H, (int)I, 0}};
+  F32Stack wanted[3];
+  int n = 0;
+  for (const F32Stack& s : all)
+    if (s.c) wanted[n++] = s;
+  return wgrads(wanted, n, offs, E, R, (hipStream_t)stream);
+}
+
+extern "C" int moe_f32_gemm_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act,
+                                   const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, float* dw1, float* dw3,
+                                   float* dw2, void* stream) {
+  for (const float* q : {dw1, dw3, dw2}) MOE_CHECK_PTR(q);
+  return moe_f32_wgrads(dg, du, dyp, xp, act, offs, E, R, H, I, dw1, dw3, dw2, stream);
+}
+
+extern "C" int moe_f32_gemm_wgrad(const float* a, const float* b, const int32_t* offs, int64_t E, int64_t R, int64_t M,
+                                  int64_t N, float* dw, int accumulate, void* stream) {
+  if (M > 65536 || N > 65536) return MOE_ERR_LIMIT;
+  const F32Stack s{a, b, dw, (int)M, (int)N, accumulate};
+  return wgrads(&s, 1, offs, E, R, (hipStream_t)stream);
+}
+
+// Test hook: 0 lets every fp32 GEMM launch choose its tile (the default), 64 or 128 forces it.
+// Process-wide and not synchronised: for tests, not for production callers.  Returns the previous
+// setting.
+extern "C" int moe_f32_gemm_force_tile(int t) {
+  const int before = forced_tile;
+  if (t == 0 || t == 64 || t == 128) forced_tile = t;
+  return before;
+}

@@ -78,6 +78,10 @@ SIGNATURES = {
     "moe_f32_swiglu_bwd": (_int, [_vp, _vp, _vp, _i64, _vp, _vp, _vp]),
     "moe_f32_gemm_rows": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _int, _vp]),
     "moe_f32_gemm_wgrad": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _int, _vp]),
+    "moe_f32_gemm_gateup_swiglu": (_int, [_vp] * 4 + [_i64] * 4 + [_vp] * 4),
+    "moe_f32_gemm_down_swiglu_bwd": (_int, [_vp] * 5 + [_i64] * 4 + [_vp] * 3),
+    "moe_f32_gemm_gateup_bwd": (_int, [_vp] * 5 + [_i64] * 4 + [_vp] * 2),
+    "moe_f32_gemm_wgrads": (_int, [_vp] * 6 + [_i64] * 4 + [_vp] * 4),
     "moe_f32_gemm_force_tile": (_int, [_int]),
 }
 

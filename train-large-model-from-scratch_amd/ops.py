@@ -562,3 +562,56 @@ def f32_gemm_wgrad(a: torch.Tensor, b: torch.Tensor, offs: torch.Tensor, E: int,
     _lib.load().call("moe_f32_gemm_wgrad", _p(a), _p(b), _p(offs), E, R, M, N, _p(dw), int(out is not None),
                      _stream())
     return dw
+
+
+def f32_gateup_swiglu(xp, w1, w3, offs):
+    """-> g, u, act fp32 [R,I]: g = xp @ w1[e].T, u = xp @ w3[e].T, act = silu(g) * u."""
+    _f32(xp, w1, w3)
+    (R, H), (E, I) = xp.shape, w1.shape[:2]
+    _check_offs(offs, E)
+    if w1.shape != w3.shape or w1.shape[2] != H:
+        raise ValueError(f"shape mismatch: xp {tuple(xp.shape)}, w1 {tuple(w1.shape)}, w3 {tuple(w3.shape)}")
+    g, u, act = (torch.empty(R, I, dtype=torch.float32, device=xp.device) for _ in range(3))
+    _lib.load().call("moe_f32_gemm_gateup_swiglu", _p(xp), _p(w1), _p(w3), _p(offs), E, R, H, I, _p(g), _p(u),
+                     _p(act), _stream())
+    return g, u, act
+
+
+def f32_down_swiglu_bwd(dyp, w2, g, u, offs):
+    """-> dg, du fp32 [R,I] from dact = dyp @ w2[e] and the g and u of the forward pass."""
+    _f32(dyp, w2, g, u)
+    (R, H), (E, _, I) = dyp.shape, w2.shape
+    _check_offs(offs, E)
+    if w2.shape[1] != H or tuple(g.shape) != (R, I) or tuple(u.shape) != (R, I):
+        raise ValueError(f"shape mismatch: dyp {tuple(dyp.shape)}, w2 {tuple(w2.shape)}, g {tuple(g.shape)}")
+    dg, du = torch.empty_like(g), torch.empty_like(g)
+    _lib.load().call("moe_f32_gemm_down_swiglu_bwd", _p(dyp), _p(w2), _p(g), _p(u), _p(offs), E, R, H, I, _p(dg),
+                     _p(du), _stream())
+    return dg, du
+
+
+def f32_gateup_bwd(dg, du, w1, w3, offs):
+    """-> dxp fp32 [R,H] = dg @ w1[e] + du @ w3[e]."""
+    _f32(dg, du, w1, w3)
+    (R, I), (E, _, H) = dg.shape, w1.shape
+    _check_offs(offs, E)
+    if w1.shape != w3.shape or w1.shape[1] != I or du.shape != dg.shape:
+        raise ValueError(f"shape mismatch: dg {tuple(dg.shape)}, w1 {tuple(w1.shape)}, w3 {tuple(w3.shape)}")
+    dxp = torch.empty(R, H, dtype=torch.float32, device=dg.device)
+    _lib.load().call("moe_f32_gemm_gateup_bwd", _p(dg), _p(du), _p(w1), _p(w3), _p(offs), E, R, H, I, _p(dxp),
+                     _stream())
+    return dxp
+
+
+def f32_wgrads(dg, du, dyp, xp, act, offs):
+    """-> dw1, dw3 fp32 [E,I,H], dw2 fp32 [E,H,I]."""
+    _f32(dg, du, dyp, xp, act)
+    (R, I), H, E = dg.shape, xp.shape[1], offs.numel() - 1
+    _check_offs(offs, E)
+    if any(tuple(t.shape) != s for t, s in ((du, (R, I)), (act, (R, I)), (dyp, (R, H)), (xp, (R, H)))):
+        raise ValueError("f32_wgrads: the rows' shapes do not belong together")
+    dw1, dw3 = (torch.empty(E, I, H, dtype=torch.float32, device=dg.device) for _ in range(2))
+    dw2 = torch.empty(E, H, I, dtype=torch.float32, device=dg.device)
+    _lib.load().call("moe_f32_gemm_wgrads", _p(dg), _p(du), _p(dyp), _p(xp), _p(act), _p(offs), E, R, H, I,
+                     _p(dw1), _p(dw3), _p(dw2), _stream())
+    return dw1, dw3, dw2

@@ -267,9 +267,7 @@ def ffn_f32_fwd(x: Tensor, logits: Tensor, w1: Tensor, w3: Tensor, w2: Tensor, k
     ids, gates = ops.router_topk(logits, k, None)
     _, offs, pos_to_row, row_to_pos = ops.histogram_scan(ids, E)
     xp = ops.f32_gather_rows(x, pos_to_row, k)
-    g = ops.f32_gemm_rows(xp, w1, offs, True)
-    u = ops.f32_gemm_rows(xp, w3, offs, True)
-    act = ops.f32_swiglu(g, u)
+    g, u, act = ops.f32_gateup_swiglu(xp, w1, w3, offs)
     y = ops.f32_gemm_rows(act, w2, offs, True)
     out = ops.f32_combine_fwd(y, gates, row_to_pos, T, k)
     if not train:
@@ -299,13 +297,10 @@ def ffn_f32_bwd(dout: Tensor, xp: Tensor, g: Tensor, u: Tensor, act: Tensor, y: 
     E = offs.numel() - 1
     w1, w3, w2 = ops.dense(w1), ops.dense(w3), ops.dense(w2)
     dyp, dgates = ops.f32_combine_bwd(ops.dense(dout.float()), y, gates, pos_to_row, k)
-    dg, du = ops.f32_swiglu_bwd(ops.f32_gemm_rows(dyp, w2, offs, False), g, u)
-    dxp = ops.f32_gemm_rows(dg, w1, offs, False)
-    ops.f32_gemm_rows(du, w3, offs, False, out=dxp)
+    dg, du = ops.f32_down_swiglu_bwd(dyp, w2, g, u, offs)
+    dxp = ops.f32_gateup_bwd(dg, du, w1, w3, offs)
     dx = ops.f32_permute_bwd(dxp, row_to_pos, T, k)
-    dw1 = ops.f32_gemm_wgrad(dg, xp, offs, E)
-    dw3 = ops.f32_gemm_wgrad(du, xp, offs, E)
-    dw2 = ops.f32_gemm_wgrad(dyp, act, offs, E)
+    dw1, dw3, dw2 = ops.f32_wgrads(dg, du, dyp, xp, act, offs)
     dlogits = ops.router_topk_bwd(gates, dgates, ids, T, E, k, torch.float32)
     return dx, dlogits, dw1, dw3, dw2
 
