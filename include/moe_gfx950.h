@@ -173,13 +173,13 @@ int moe_dgates_from_blocks_by_pos(const float* dgate_part, int64_t blocks, const
                                   const int32_t* pos_to_row, int64_t R, float* dgates, void* stream);
 /* g and u in a layout private to the library.  Nothing but the SwiGLU backward reads the two
  * pre-activation planes the forward saves (mlp.py:154-156 under autograd keeps them as [R, I]
- * tensors), so they need not be rows: gu_blocked holds one 4 KB record per 32 x 32 block of every
- * 256-row tile of the expert-contiguous rows, g and u of the block together, each in the order in
+ * tensors), so they need not be rows: gu_blocked holds one 4 KB record per 32 x 32 block of each
+ * expert's rows (row block b of expert e is block offs[e]/32 + e + b), g and u of the block together, each in the order in
  * which a wavefront's matrix-core accumulators hold it.  The forward kernel stores the records
  * straight from its registers and the backward kernel loads them straight into the layout it
  * computes in; act, dg, du and dgate_part are the same bits as from the row-major entry points.
  * The buffer is opaque to the caller: moe_gu_blocked_bytes(R, E, I) bytes (it depends on R, E and
- * I only, never on the routing: (ceil(R/256) + E) * 256 rows are provided for), 16-byte aligned,
+ * I only, never on the routing: R/32 + E row blocks are provided for), 16-byte aligned,
  * written by moe_gemm_gateup_swiglu_fwd_blocked and valid for moe_gemm_dgrad_down_swiglu_bwd_blocked
  * with the same offs, E, R and I.  dg and du [R, ld_out] rows (ld_out = 0 means I; 2*I with
  * du = dg + I gives the side-by-side buffer of moe_gemm_wgrad_pair); dgate_part may be NULL. */
@@ -193,9 +193,9 @@ int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const uint16_t* 
                                            uint16_t* du, int64_t ld_out, float* dgate_part,
                                            void* stream);
 /* Test hook (no counterpart in the reference).  The four row-ragged products (gate/up, down and
- * their two input gradients) run on 256-row tiles, or on 128-row tiles when the launch has too few
- * large tiles for half of the compute units; the choice is made from R, E and the
- * output width alone.  moe_gemm_force_row_tile(128 or 256) forces one of them for every later
+ * their two input gradients) run on 256-row tiles, what is left after whole rounds of them on
+ * 128-row tiles where that is shorter, and launches of few tiles on 128-row tiles throughout.
+ * moe_gemm_force_row_tile(128 or 256) forces one of them for every later
  * call, 0 restores the automatic choice; the previous setting is returned.  Process-wide and not
  * synchronised with calls in flight on other host threads.  No result depends on the choice:
  * every output element is accumulated over k in the same order on both tile heights, so all

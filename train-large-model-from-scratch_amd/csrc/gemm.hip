@@ -57,6 +57,7 @@ struct GemmArgs {
   int ld_a;     // row stride of A0/A1 in elements when it is not the contraction length (0: K)
   int ld_c;     // row stride of the outputs C0/C1 in elements when it is not N (0: N)
   int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
+  int whole_only;  // row-ragged modes: no half tiles (test hook)
   int slice;    // WGRAD without offsets: "expert" e is rows e*slice .. (e+1)*slice of the R rows; 0: offs
 };
 
@@ -89,6 +90,7 @@ constexpr int lds_bytes() {
 }
 
 constexpr int GEMM_MAX_E = 1024;  // per-expert tile prefix lives in LDS
+constexpr int ROW_TILE = 256;     // rows of a tile of the row-ragged modes
 
 // BLK (GATEUP and DGRAD_DOWN only): g and u, which nothing but the SwiGLU backward reads, are kept
 // in a layout private to the library instead of as [R, I] rows: one 4 KB record per 32 x 32 block
@@ -96,8 +98,13 @@ constexpr int GEMM_MAX_E = 1024;  // per-expert tile prefix lives in LDS
 // (see gu_block below).  The forward kernel then stores them straight from its registers and the
 // backward kernel loads them straight into the layout it computes in: neither passes them
 // through LDS.
-template <int MODE, typename Cfg, typename OutT, bool BLK = false>
-__global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_kernel(const GemmArgs p) {
+//
+// The kernel's tile walk: the tiles at positions t_next, t_next + t_step, .. below t_hi of the launch's tile
+// list, or of `list` where one is given.  The rows of a row-ragged launch are numbered in tiles of UNIT rows; where
+// the configuration's are half as high, a list entry is 2 * tile + half.  (tile_start and, there, offs: in LDS.)
+template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE>
+__device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, const int* tile_start, const int* offs,
+                                           const uint32_t* list, int t_next, const int t_hi, const int t_step) {
   static_assert(!BLK || MODE == GATEUP || MODE == DGRAD_DOWN, "only g and u have the blocked layout");
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, KS = Cfg::KS;
   constexpr int FM = Cfg::FM, FN = Cfg::FN, WTM = Cfg::WTM, WTN = Cfg::WTN;
@@ -114,8 +121,6 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
   using StBh = OpInner<BN / 2, BK, NT>;  // dual mode: the W1 half and the W3 half of the B tile
   static_assert(!DUAL || !B_OUTER, "dual mode stages k-contiguous weights");
 
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  __shared__ int tile_start[(MODE == WGRAD) ? 1 : GEMM_MAX_E + 1];
   uint16_t* sA = smem;                       // [2][StA::LDS_ELEMS]
   uint16_t* sB = smem + 2 * StA::LDS_ELEMS;  // [2][StB::LDS_ELEMS]
 
@@ -124,132 +129,11 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int wm = wv / Cfg::WN, wn = wv % Cfg::WN;
 
-  // ---- which tiles this workgroup computes
-  // The kernel is persistent: the grid has one workgroup per compute unit and each walks a
-  // list of tiles.  Hardware hands workgroup b to XCD b % 8 (each XCD has its own L2), so
-  // XCD x takes the x-th contiguous eighth of the tile list and its workgroups sweep that
-  // range side by side: at any time they share a few experts' weights and row blocks in L2.
-  if constexpr (MODE != WGRAD) {
-    // tile_start[e] = number of row tiles of the experts before e (wave 0 scans)
-    if (threadIdx.x < MOE_WAVE) {
-      int carry = 0;
-      for (int b = 0; b < p.E; b += MOE_WAVE) {
-        const int e = b + lane;
-        const int nt = e < p.E ? (p.offs[e + 1] - p.offs[e] + BM - 1) / BM : 0;
-        int incl = nt;
-#pragma unroll
-        for (int off = 1; off < MOE_WAVE; off <<= 1) {
-          const int o = __shfl_up(incl, off, MOE_WAVE);
-          if (lane >= off) incl += o;
-        }
-        if (e < p.E) tile_start[e] = carry + incl - nt;
-        carry += __shfl(incl, MOE_WAVE - 1, MOE_WAVE);
-      }
-      if (lane == 0) tile_start[p.E] = carry;
-    }
-    __syncthreads();
-  }
-  // The XCDs that have workgroups (all 8 unless the grid is tiny) share out the tile list.
-  // Row-ragged modes: every tile costs about the same; XCD x takes the x-th contiguous eighth of
-  // the list (equal counts of real tiles) and its workgroups sweep it side by side.
-  // WGRAD with more tiles than workgroups: a tile of expert e contracts over that expert's rows,
-  // so under skewed routing tiles differ in cost by orders of magnitude and a contiguous range is
-  // all heavy or all light.  The (expert-major) list is dealt in groups of as many consecutive
-  // tiles as an XCD has workgroups, group g to XCD g % 8, one tile to each of its workgroups: the
-  // workgroups of an XCD stay on one expert (or two) and walk its rows together, and every XCD
-  // sees every part of the list.  With at most 64 experts, whole groups per expert and skewed
-  // routing (the largest expert above 1.25 times the mean) the groups are not dealt round-robin
-  // but longest first: experts in descending order of their rows, each group to the XCD with the
-  // least work so far; every workgroup works that out for itself from the offsets, the same way,
-  // and keeps its own tiles' numbers in LDS.  (A generated power-law skew over 16 experts: 10-12 %
-  // faster dealt in groups than with contiguous ranges of equal work, another 9-10 % longest
-  // first; near-uniform routing: the same in all three.)
-  constexpr int MAX_GROUPS = 512;
-  __shared__ int glist[(MODE == WGRAD) ? MAX_GROUPS : 1];
-  __shared__ int gcount;
-  int t_next, t_hi, t_step;  // (t_step == 0: positions in glist, else tile numbers)
-  {
-    const int nb = gridDim.x, x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int nx = nb < 8 ? nb : 8;
-    t_step = (nb >> 3) + (x < (nb & 7) ? 1 : 0);
-    int lo;
-    if (MODE == WGRAD && p.E * p.m_slots * p.n_tiles > nb && (nb & 7) == 0) {
-      const int wgs = nb >> 3, TP = p.m_slots * p.n_tiles;
-      lo = x * wgs;
-      t_hi = p.E * TP;
-      t_step = nb;
-      if (!p.slice && p.E <= MOE_WAVE && TP % wgs == 0 && p.E * (TP / wgs) <= MAX_GROUPS) {
-        if (threadIdx.x < MOE_WAVE) {
-          const int gpe = TP / wgs;  // groups per expert
-          constexpr long long FIXED = 4 * BK;  // fill, tile switch and epilogue, in rows' worth
-          int rows = 0;
-          if (lane < p.E) {
-            rows = p.offs[lane + 1] - p.offs[lane];
-            rows = rows < 0 ? 0 : rows;
-          }
-          const long long cost = rows + FIXED;
-          // (only worth it when the routing is skewed: with near-equal experts the plain dealing is
-          // as balanced and keeps neighbouring experts on neighbouring XCDs)
-          int mx = rows, sum = rows;
-#pragma unroll
-          for (int off = MOE_WAVE / 2; off > 0; off >>= 1) {
-            const int om = __shfl_xor(mx, off, MOE_WAVE);
-            mx = om > mx ? om : mx;
-            sum += __shfl_xor(sum, off, MOE_WAVE);
-          }
-          const bool skewed = 4ll * mx * p.E > 5ll * sum;
-          int rank = 0;  // position of expert `lane` in descending order of cost (ties: lower index first)
-          for (int o = 0; o < p.E; ++o) {
-            const long long co = __shfl(cost, o, MOE_WAVE);
-            rank += (co > cost || (co == cost && o < lane)) ? 1 : 0;
-          }
-          if (lane >= p.E) rank = -1;
-          // lanes 0..7 carry the XCDs' loads, packed with the XCD index for the arg-min
-          long long load = 0;
-          int cnt = 0;
-          for (int s_ = 0; skewed && s_ < p.E; ++s_) {
-            const int e = __builtin_ctzll(__ballot(rank == s_));
-            const long long ce = __shfl(cost, e, MOE_WAVE);
-            for (int gi = 0; gi < gpe; ++gi) {
-              long long key = lane < 8 ? ((load << 3) | lane) : 0x7fffffffffffffffll;
-#pragma unroll
-              for (int off = 1; off < 8; off <<= 1) {
-                const long long other = __shfl_xor(key, off, MOE_WAVE);
-                key = other < key ? other : key;
-              }
-              const int xmin = (int)(__shfl(key, 0, MOE_WAVE) & 7);
-              if (lane == xmin) load += ce;
-              if (xmin == x) {
-                if (lane == 0) glist[cnt] = (e * gpe + gi) * wgs + j;
-                ++cnt;
-              }
-            }
-          }
-          if (lane == 0) gcount = skewed ? cnt : -1;
-        }
-        __syncthreads();
-        const int cnt = gcount;
-        if (cnt >= 0) {
-          t_hi = cnt;  // (positions in the list)
-          lo = -j;
-          t_step = 0;
-        }
-      }
-    } else {
-      int total;  // real tiles
-      if constexpr (MODE == WGRAD) total = p.E * p.m_slots * p.n_tiles;
-      else total = tile_start[p.E] * p.n_tiles;
-      const int q = total / nx, r = total % nx;
-      lo = x * q + (x < r ? x : r);
-      t_hi = lo + q + (x < r ? 1 : 0);
-    }
-    t_next = lo + j;
-  }
-  // the tile behind position `pos` of this workgroup's walk
-  auto tile_at = [&](int pos) { return t_step == 0 ? __builtin_amdgcn_readfirstlane(glist[pos]) : pos; };
+  auto tile_at = [&](int pos) { return list ? (uint32_t)__builtin_amdgcn_readfirstlane((int)list[pos]) : (uint32_t)pos; };
 
   struct Tile {
-    int e, row0, row_end, n0, m0, slot;
+    int e, row0, row_end, n0, m0;
+    int block0;  // first of its 32-row blocks in the blocked g/u layout
     int Kseg, kt_per_seg, nkt;
     bool need_mask;
     View vA0, vA1, vB0, vB1;
@@ -261,11 +145,12 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
 
   // Fills `t` for tile slot `logical`; false when the slot lies past the last real tile.
   // Every lane computes the same thing from the same LDS words / scalar loads.
-  auto locate = [&](int logical, Tile& t) -> bool {
-    const int n_tile = logical % p.n_tiles;
-    const int slot = logical / p.n_tiles;
+  auto locate = [&](uint32_t entry, Tile& t) -> bool {
+    constexpr bool HALF = MODE != WGRAD && BM < UNIT;
+    const uint32_t logical = HALF ? entry >> 1 : entry;
+    const int n_tile = (int)(logical % (uint32_t)p.n_tiles);
+    const int slot = (int)(logical / (uint32_t)p.n_tiles);
     t.m0 = 0;
-    t.slot = slot;
     if constexpr (MODE == WGRAD) {
       t.e = slot / p.m_slots;
       t.m0 = (slot % p.m_slots) * BM;
@@ -273,8 +158,8 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
         t.row0 = t.e * p.slice;
         t.row_end = t.row0 + p.slice < p.R ? t.row0 + p.slice : p.R;
       } else {
-        t.row0 = p.offs[t.e];
-        t.row_end = p.offs[t.e + 1];
+        t.row0 = offs[t.e];
+        t.row_end = offs[t.e + 1];
       }
     } else {
       if (slot >= tile_start[p.E]) return false;
@@ -285,8 +170,13 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
         else hi = mid;
       }
       t.e = __builtin_amdgcn_readfirstlane(lo);
-      t.row0 = p.offs[t.e] + (slot - __builtin_amdgcn_readfirstlane(tile_start[lo])) * BM;
-      t.row_end = p.offs[t.e + 1];
+      const int off = __builtin_amdgcn_readfirstlane(offs[t.e]);
+      int in_expert = (slot - __builtin_amdgcn_readfirstlane(tile_start[lo])) * UNIT;
+      if (HALF) in_expert += (int)(entry & 1) * BM;
+      t.row0 = off + in_expert;
+      t.row_end = __builtin_amdgcn_readfirstlane(offs[t.e + 1]);
+      // (off / 32 + e grows from one expert to the next by at least the expert's blocks, whatever the tile height)
+      t.block0 = off / 32 + t.e + in_expert / 32;
     }
     t.n0 = n_tile * BNC;
     t.Kseg = (MODE == WGRAD) ? (t.row_end - t.row0) : p.K;
@@ -523,17 +413,17 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
   };
-  // Blocked g/u (BLK): record of the 32 x 32 block (row block rb of row-tile slot `slot`, column
+  // Blocked g/u (BLK): record of the 32 x 32 block (row block rb of the tile, column
   // block cb = column / 32), GU_BLOCK_BYTES each: [g: q0q1 of lanes 0..63 | g: q2q3 | u: q0q1 |
   // u: q2q3], 16 bytes per lane and part, where lane l of the wave that owns the block holds row
   // l % 32 and columns 8*q + 4*(l/32) .. +3 of it for q = 0..3 (the accumulator layout above).
-  // A wave-wide 16-byte access to one part covers 1 KB of consecutive addresses.  Row tiles are
-  // numbered as the tile list numbers them (expert by expert, BM rows each), so that the forward
-  // and the backward kernel agree on `slot` from the offsets alone.
+  // A wave-wide 16-byte access to one part covers 1 KB of consecutive addresses.  Row blocks are
+  // numbered expert by expert from the offsets alone (Tile::block0), so that the forward and the backward
+  // kernel agree on them whatever tiles either of them takes.
   constexpr int GU_BLOCK_BYTES = 4096;
   const int n_cb = (p.N + 31) / 32;
   auto gu_block = [&](const void* base, const Tile& t, int rb, int cb, int ln) {
-    return (char*)base + (((long long)t.slot * (BM / 32) + rb) * n_cb + cb) * GU_BLOCK_BYTES + ln * 16;
+    return (char*)base + (((long long)t.block0 + rb) * n_cb + cb) * GU_BLOCK_BYTES + ln * 16;
   };
   // `halfway` runs once, after the second of the FM strips; `last_rows_in` once the SwiGLU-backward
   // epilogue has taken the last g/u rows out of their registers
@@ -833,7 +723,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
     // where the next tile lies is worked out now (a binary search in LDS and some address
     // arithmetic), in the shadow of this tile's first MFMAs, not between the tiles
     Tile nxt;
-    t_next += t_step ? t_step : 1;
+    t_next += t_step;
     const bool more = t_next < t_hi && locate(tile_at(t_next), nxt);
     const int nkt = cur.nkt;
     if (nkt > 0) {
@@ -921,18 +811,239 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WAVES_PER_SIMD) void grouped_gemm_ker
   }
 }
 
-#ifndef MOE_BM
-#define MOE_BM 256
-#define MOE_BN 256
-#define MOE_BK 64
-#define MOE_WM 2
-#define MOE_WN 4
-#endif
-using CfgMain = TileCfg<MOE_BM, MOE_BN, MOE_BK, MOE_WM, MOE_WN>;
-// Row tiles of half the height (the eight waves 64 x 64 each) for launches too small to give even
-// half of the compute units one of the large tiles: twice the tiles, each at about 0.7 of the
-// large tile's cost, spread such a launch over twice the compute units.
-using CfgSmall = TileCfg<MOE_BM / 2, MOE_BN, MOE_BK, MOE_WM, MOE_WN>;
+using CfgMain = TileCfg<ROW_TILE, 256, 64, 2, 4>;
+// Row tiles of half the height (the eight waves 64 x 64 each), at 0.65 to 0.7 of a tile's cost.
+using CfgHalf = TileCfg<ROW_TILE / 2, 256, 64, 2, 4>;
+
+// tile_start[e] = number of tiles of UNIT rows of the experts before e, offs = p.offs, both in LDS (wave 0 scans).
+template <int UNIT>
+__device__ __forceinline__ void number_tiles(const GemmArgs& p, int* tile_start, int* offs) {
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < MOE_WAVE) {
+    int carry = 0;
+    for (int b = 0; b < p.E; b += MOE_WAVE) {
+      const int e = b + lane;
+      const int first = e < p.E ? p.offs[e] : 0, end = e < p.E ? p.offs[e + 1] : 0;
+      const int nt = (end - first + UNIT - 1) / UNIT;
+      int incl = nt;
+#pragma unroll
+      for (int off = 1; off < MOE_WAVE; off <<= 1) {
+        const int o = __shfl_up(incl, off, MOE_WAVE);
+        if (lane >= off) incl += o;
+      }
+      if (e < p.E) {
+        tile_start[e] = carry + incl - nt;
+        offs[e] = first;
+        if (e == p.E - 1) offs[p.E] = end;
+      }
+      carry += __shfl(incl, MOE_WAVE - 1, MOE_WAVE);
+    }
+    if (lane == 0) tile_start[p.E] = carry;
+  }
+  __syncthreads();
+}
+
+// Every tile of a row-ragged launch costs about the same.  Of the XCDs that have workgroups (all 8 unless the
+// grid is tiny) XCD x takes the x-th contiguous eighth of the n positions of the list and its workgroups
+// sweep it side by side: at any time they share a few experts' weights and row blocks in L2.
+struct Sweep {
+  int first, end, step;
+};
+__device__ __forceinline__ Sweep sweep_of(int n) {
+  const int nb = gridDim.x, x = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int nx = nb < 8 ? nb : 8;
+  const int q = n / nx, r = n % nx;
+  const int lo = x * q + (x < r ? x : r);
+  return {lo + j, lo + q + (x < r ? 1 : 0), (nb >> 3) + (x < (nb & 7) ? 1 : 0)};
+}
+
+// The last round is mostly partial.  What is left after the whole rounds is done in half tiles where that is at most
+// one to every workgroup, and the round before with it where that is at most two (at 0.65 of a tile two are less
+// than a whole one and a half one).  Which halves have rows follows from the offsets; every workgroup works it
+// out for itself, a tile a thread.  Whole tiles -> this, gate/up, down, dgrad-down and dgrad-gate/up in us:
+//   16384 rows of 8 experts, 1024 <-> 512    54 -> 48, 32 -> 29, 40 (0.53 rounds, 264 halves), 53 -> 48
+//   9999 rows of 12 experts, 1416 <-> 568    40 (0.9), 36 -> 29, 49 -> 36 (0.53 rounds, 252 halves), 61 -> 47
+// From some ten rounds on it makes no difference.
+template <int MODE, typename OutT, bool BLK>
+__global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gemm_kernel(const GemmArgs p) {
+  static_assert(CfgHalf::NT == CfgMain::NT, "one workgroup runs both");
+  constexpr int WAVES = CfgMain::NT / MOE_WAVE;
+  constexpr int MAX_LISTED = CfgMain::NT;
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  __shared__ int tile_start[GEMM_MAX_E + 1], offs[GEMM_MAX_E + 1];
+  __shared__ uint32_t half_list[MAX_LISTED];
+  __shared__ int wave_halves[2][WAVES];
+  number_tiles<ROW_TILE>(p, tile_start, offs);
+  const int nb = gridDim.x;
+  const int total = __builtin_amdgcn_readfirstlane(tile_start[p.E]) * p.n_tiles;
+  int whole = total;  // tiles 0 .. whole are done whole
+  int halves = 0;     // halves with rows of the others
+  const int left = total % nb;
+  if (!p.whole_only && left > 0 && nb <= MAX_LISTED) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int round = total > nb && 2 * nb <= MAX_LISTED ? nb : 0;  // (of whole tiles that may be halved too)
+    const int tile = total - left - round + (int)threadIdx.x;
+    const bool last = tile >= total - left;
+    int n = 0;
+    if (tile < total) {
+      const int slot = tile / p.n_tiles;
+      int e = 0, hi = p.E;
+      while (hi - e > 1) {
+        const int mid = (e + hi) >> 1;
+        if (tile_start[mid] <= slot) e = mid;
+        else hi = mid;
+      }
+      n = offs[e + 1] - offs[e] - (slot - tile_start[e]) * ROW_TILE > CfgHalf::BM ? 2 : 1;
+    }
+    const unsigned long long some = __ballot(n > 0), both = __ballot(n > 1), in_last = __ballot(last);
+    const unsigned long long below = (1ull << lane) - 1;
+    if (lane == 0) {
+      wave_halves[0][wv] = __popcll(some) + __popcll(both);
+      wave_halves[1][wv] = __popcll(some & in_last) + __popcll(both & in_last);
+    }
+    __syncthreads();
+    int at = __popcll(some & below) + __popcll(both & below), all = 0, in_left = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const int c = __builtin_amdgcn_readfirstlane(wave_halves[0][w]);
+      at += w < wv ? c : 0;
+      all += c;
+      in_left += __builtin_amdgcn_readfirstlane(wave_halves[1][w]);
+    }
+    int skip = 0;  // halves of the round before, when that stays whole
+    if (round > 0 && all <= 2 * nb) {
+      halves = all;
+      whole = total - left - round;
+    } else if (in_left <= nb) {
+      halves = in_left;
+      whole = total - left;
+      skip = all - in_left;
+    }
+    if (tile >= whole)
+      for (int h = 0; h < n; ++h) half_list[at + h - skip] = 2u * (uint32_t)tile + h;
+  }
+  const Sweep s = sweep_of(whole);
+  walk_tiles<MODE, CfgMain, OutT, BLK>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
+  if (halves == 0) return;
+  __syncthreads();  // (the operand stages are free, the list is complete)
+  const Sweep h = sweep_of(halves);
+  walk_tiles<MODE, CfgHalf, OutT, BLK>(p, smem, tile_start, offs, half_list, h.first, h.end, h.step);
+}
+
+// All in half tiles: launches of so few tiles that there is nothing to decide (4096 rows of 8 experts, 1024 <-> 512,
+// gate/up and down 17.4 and 11.6 us; through the kernel above 18.6 and 12.5).
+template <int MODE, typename OutT, bool BLK>
+__global__ __launch_bounds__(CfgHalf::NT, CfgHalf::WAVES_PER_SIMD) void small_rows_gemm_kernel(const GemmArgs p) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  __shared__ int tile_start[GEMM_MAX_E + 1], offs[GEMM_MAX_E + 1];
+  number_tiles<CfgHalf::BM>(p, tile_start, offs);
+  const Sweep s = sweep_of(__builtin_amdgcn_readfirstlane(tile_start[p.E]) * p.n_tiles);
+  walk_tiles<MODE, CfgHalf, OutT, BLK, CfgHalf::BM>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
+}
+
+// Weight gradients.
+template <typename OutT>
+__global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_gemm_kernel(const GemmArgs p) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  const int lane = threadIdx.x & 63;
+  // ---- which tiles this workgroup computes
+  // The kernel is persistent: the grid has one workgroup per compute unit and each walks a
+  // list of tiles.  Hardware hands workgroup b to XCD b % 8 (each XCD has its own L2).
+  // With more tiles than workgroups: a tile of expert e contracts over that expert's rows,
+  // so under skewed routing tiles differ in cost by orders of magnitude and a contiguous range is
+  // all heavy or all light.  The (expert-major) list is dealt in groups of as many consecutive
+  // tiles as an XCD has workgroups, group g to XCD g % 8, one tile to each of its workgroups: the
+  // workgroups of an XCD stay on one expert (or two) and walk its rows together, and every XCD
+  // sees every part of the list.  With at most 64 experts, whole groups per expert and skewed
+  // routing (the largest expert above 1.25 times the mean) the groups are not dealt round-robin
+  // but longest first: experts in descending order of their rows, each group to the XCD with the
+  // least work so far; every workgroup works that out for itself from the offsets, the same way,
+  // and keeps its own tiles' numbers in LDS.  (A generated power-law skew over 16 experts: 10-12 %
+  // faster dealt in groups than with contiguous ranges of equal work, another 9-10 % longest
+  // first; near-uniform routing: the same in all three.)
+  constexpr int MAX_GROUPS = 512;
+  __shared__ uint32_t glist[MAX_GROUPS];
+  __shared__ int gcount;
+  int t_next, t_hi, t_step;
+  const uint32_t* list = nullptr;  // (given: positions in it, else tile numbers)
+  {
+    const int nb = gridDim.x, x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int nx = nb < 8 ? nb : 8;
+    t_step = (nb >> 3) + (x < (nb & 7) ? 1 : 0);
+    int lo;
+    if (p.E * p.m_slots * p.n_tiles > nb && (nb & 7) == 0) {
+      const int wgs = nb >> 3, TP = p.m_slots * p.n_tiles;
+      lo = x * wgs;
+      t_hi = p.E * TP;
+      t_step = nb;
+      if (!p.slice && p.E <= MOE_WAVE && TP % wgs == 0 && p.E * (TP / wgs) <= MAX_GROUPS) {
+        if (threadIdx.x < MOE_WAVE) {
+          const int gpe = TP / wgs;  // groups per expert
+          constexpr long long FIXED = 4 * CfgMain::BK;  // fill, tile switch and epilogue, in rows' worth
+          int rows = 0;
+          if (lane < p.E) {
+            rows = p.offs[lane + 1] - p.offs[lane];
+            rows = rows < 0 ? 0 : rows;
+          }
+          const long long cost = rows + FIXED;
+          // (only worth it when the routing is skewed: with near-equal experts the plain dealing is
+          // as balanced and keeps neighbouring experts on neighbouring XCDs)
+          int mx = rows, sum = rows;
+#pragma unroll
+          for (int off = MOE_WAVE / 2; off > 0; off >>= 1) {
+            const int om = __shfl_xor(mx, off, MOE_WAVE);
+            mx = om > mx ? om : mx;
+            sum += __shfl_xor(sum, off, MOE_WAVE);
+          }
+          const bool skewed = 4ll * mx * p.E > 5ll * sum;
+          int rank = 0;  // position of expert `lane` in descending order of cost (ties: lower index first)
+          for (int o = 0; o < p.E; ++o) {
+            const long long co = __shfl(cost, o, MOE_WAVE);
+            rank += (co > cost || (co == cost && o < lane)) ? 1 : 0;
+          }
+          if (lane >= p.E) rank = -1;
+          // lanes 0..7 carry the XCDs' loads, packed with the XCD index for the arg-min
+          long long load = 0;
+          int cnt = 0;
+          for (int s_ = 0; skewed && s_ < p.E; ++s_) {
+            const int e = __builtin_ctzll(__ballot(rank == s_));
+            const long long ce = __shfl(cost, e, MOE_WAVE);
+            for (int gi = 0; gi < gpe; ++gi) {
+              long long key = lane < 8 ? ((load << 3) | lane) : 0x7fffffffffffffffll;
+#pragma unroll
+              for (int off = 1; off < 8; off <<= 1) {
+                const long long other = __shfl_xor(key, off, MOE_WAVE);
+                key = other < key ? other : key;
+              }
+              const int xmin = (int)(__shfl(key, 0, MOE_WAVE) & 7);
+              if (lane == xmin) load += ce;
+              if (xmin == x) {
+                if (lane == 0) glist[cnt] = (e * gpe + gi) * wgs + j;
+                ++cnt;
+              }
+            }
+          }
+          if (lane == 0) gcount = skewed ? cnt : -1;
+        }
+        __syncthreads();
+        const int cnt = gcount;
+        if (cnt >= 0) {
+          t_hi = cnt;
+          lo = -j;
+          t_step = 1;
+          list = glist;
+        }
+      }
+    } else {
+      const int total = p.E * p.m_slots * p.n_tiles;
+      const int q = total / nx, r = total % nx;
+      lo = x * q + (x < r ? x : r);
+      t_hi = lo + q + (x < r ? 1 : 0);
+    }
+    t_next = lo + j;
+  }
+  walk_tiles<WGRAD, CfgMain, OutT, false>(p, smem, nullptr, p.offs, list, t_next, t_hi, t_step);
+}
 
 }  // namespace
 
@@ -950,25 +1061,51 @@ int moe_compute_units() {
 namespace {
 
 
-// `ntiles` is the number of tile slots; the grid is as many workgroups as are resident at
-// once (one or two per compute unit, by LDS footprint), or fewer when there are fewer tiles.
-template <int MODE, typename Cfg, typename OutT, bool BLK = false>
-int launch(const GemmArgs& a, long long ntiles, hipStream_t s) {
-  if (ntiles <= 0) return 0;
-  auto kern = grouped_gemm_kernel<MODE, Cfg, OutT, BLK>;
+// As many workgroups as are resident at once (one per compute unit), or as there are jobs.
+template <int MODE, typename Cfg>
+int launch(void (*kern)(GemmArgs), bool (&attr_done)[MOE_MAX_DEVICES], const GemmArgs& a, long long jobs, hipStream_t s) {
+  if (jobs <= 0) return 0;
   constexpr int LDS = lds_bytes<MODE, Cfg>();
-  static bool attr_done[MOE_MAX_DEVICES];  // per GPU and instantiation
   const int dev = moe_current_device();
   if (!attr_done[dev]) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return (int)e;
     attr_done[dev] = true;
   }
-  // as many workgroups as can be resident at once: the LDS footprint decides how many share a CU
-  const long long slots = (long long)moe_compute_units() * ((160 * 1024) / LDS >= Cfg::WGS_PER_CU ? Cfg::WGS_PER_CU : 1);
-  const unsigned grid = (unsigned)(ntiles < slots ? ntiles : slots);
+  const long long slots = moe_compute_units();
+  const unsigned grid = (unsigned)(jobs < slots ? jobs : slots);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(Cfg::NT), LDS, s, a);
   return moe_launch_status();
+}
+
+long long row_slots(int64_t R, int64_t E, int tile) { return (R + tile - 1) / tile + E; }
+
+// Which kernel a row-ragged launch takes: decided from the shapes alone (never from the routing: no host
+// synchronisation).  With fewer tiles than half the compute units, by the bound on their number, every one of them can be
+// halved.  `forced_row_tile` (0: automatic) is a test hook.
+int forced_row_tile = 0;
+
+// A row-ragged launch with `cols` output columns to a tile.
+template <int MODE, bool BLK = false>
+int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
+  static_assert(lds_bytes<MODE, CfgHalf>() <= lds_bytes<MODE, CfgMain>(), "both row tiles fit");
+  static bool attr_done[2][MOE_MAX_DEVICES];  // per GPU and instantiation
+  a.n_tiles = (a.N + cols - 1) / cols;
+  const long long tiles = row_slots(a.R, a.E, ROW_TILE) * ((a.N + CfgMain::BN - 1) / CfgMain::BN);
+  const bool small = forced_row_tile ? forced_row_tile == CfgHalf::BM : 2 * tiles < moe_compute_units();
+  if (small)
+    return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK>, attr_done[0], a,
+                                 a.n_tiles * row_slots(a.R, a.E, CfgHalf::BM), s);
+  a.whole_only = forced_row_tile == ROW_TILE;
+  return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK>, attr_done[1], a,
+                               2 * a.n_tiles * row_slots(a.R, a.E, ROW_TILE), s);
+}
+template <typename OutT>
+int launch_wgrad(GemmArgs& a, hipStream_t s) {
+  a.n_tiles = (a.N + CfgMain::BN - 1) / CfgMain::BN;
+  a.m_slots = (a.M + CfgMain::BM - 1) / CfgMain::BM;
+  static bool attr_done[MOE_MAX_DEVICES];
+  return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT>, attr_done, a, (long long)a.n_tiles * a.m_slots * a.E, s);
 }
 
 int check_common(const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I) {
@@ -983,27 +1120,6 @@ int check_common(const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I
   return 0;
 }
 
-template <typename Cfg>
-int row_slots(int64_t R, int64_t E) {
-  return (int)((R + Cfg::BM - 1) / Cfg::BM + E);
-}
-
-// Which row-tile height a row-ragged launch uses: decided from the shapes alone (never from the
-// routing: no host synchronisation), the same way for the forward kernel that writes blocked g/u
-// and the backward kernel that reads it (both pass I as `cols`).  Measured on the two small
-// benchmark configurations: 4096 rows of 8 experts (48 large tiles by this count) run 24 % faster
-// on the small tiles, 16384 rows (144) no faster.  `forced_row_tile` (0: automatic) is a test hook.
-int forced_row_tile = 0;
-bool small_row_tiles(int64_t R, int64_t E, int64_t cols) {
-  if (forced_row_tile) return forced_row_tile == CfgSmall::BM;
-  const int64_t tiles = (int64_t)row_slots<CfgMain>(R, E) * ((cols + CfgMain::BN - 1) / CfgMain::BN);
-  return 2 * tiles < (int64_t)moe_compute_units();
-}
-template <typename F>
-int with_row_tile(bool small, F&& f) {
-  return small ? f(CfgSmall{}) : f(CfgMain{});
-}
-
 }  // namespace
 
 extern "C" int moe_gemm_gateup_swiglu_fwd(const uint16_t* xp, const uint16_t* w1, const uint16_t* w3,
@@ -1014,23 +1130,17 @@ extern "C" int moe_gemm_gateup_swiglu_fwd(const uint16_t* xp, const uint16_t* w1
   if (R == 0) return 0;
   MOE_CHECK_PTR(xp); MOE_CHECK_PTR(w1); MOE_CHECK_PTR(w3); MOE_CHECK_PTR(act);
   if ((g == nullptr) != (u == nullptr)) return MOE_ERR_NULL;
-  return with_row_tile(small_row_tiles(R, E, I), [&](auto cfg) {
-    using Cfg = decltype(cfg);
-    GemmArgs a{};
-    a.A0 = xp; a.B0 = w1; a.B1 = w3; a.C0 = g; a.C1 = u; a.C2 = act; a.offs = offs;
-    a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H;
-    a.n_tiles = (int)((I + Cfg::BN / 2 - 1) / (Cfg::BN / 2));
-    a.m_slots = row_slots<Cfg>(R, E);
-    return launch<GATEUP, Cfg, uint16_t>(a, (long long)a.n_tiles * a.m_slots, (hipStream_t)stream);
-  });
+  GemmArgs a{};
+  a.A0 = xp; a.B0 = w1; a.B1 = w3; a.C0 = g; a.C1 = u; a.C2 = act; a.offs = offs;
+  a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H;
+  return launch_rows<GATEUP>(a, CfgMain::BN / 2, (hipStream_t)stream);
 }
 
-// Bytes of the blocked g/u buffer: one 4 KB record per 32 x 32 block of every row-tile slot the
-// tile list can have (ceil(R/256) + E bounds their number whatever the routing).
+// Bytes of the blocked g/u buffer: one 4 KB record per 32 x 32 block (R/32 + E bounds the number of row
+// blocks whatever the routing).
 extern "C" int64_t moe_gu_blocked_bytes(int64_t R, int64_t E, int64_t I) {
   if (R <= 0 || E <= 0 || I <= 0) return 0;
-  using Cfg = CfgMain;
-  return (int64_t)row_slots<Cfg>(R, E) * (Cfg::BM / 32) * ((I + 31) / 32) * 4096;
+  return (R / 32 + E) * ((I + 31) / 32) * 4096;
 }
 
 extern "C" int moe_gemm_gateup_swiglu_fwd_blocked(const uint16_t* xp, const uint16_t* w1, const uint16_t* w3,
@@ -1039,15 +1149,10 @@ extern "C" int moe_gemm_gateup_swiglu_fwd_blocked(const uint16_t* xp, const uint
   if (int rc = check_common(offs, E, R, H, I)) return rc;
   if (R == 0) return 0;
   MOE_CHECK_PTR(xp); MOE_CHECK_PTR(w1); MOE_CHECK_PTR(w3); MOE_CHECK_PTR(act); MOE_CHECK_PTR(gu_blocked);
-  return with_row_tile(small_row_tiles(R, E, I), [&](auto cfg) {
-    using Cfg = decltype(cfg);
-    GemmArgs a{};
-    a.A0 = xp; a.B0 = w1; a.B1 = w3; a.C0 = gu_blocked; a.C2 = act; a.offs = offs;
-    a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H;
-    a.n_tiles = (int)((I + Cfg::BN / 2 - 1) / (Cfg::BN / 2));
-    a.m_slots = row_slots<Cfg>(R, E);
-    return launch<GATEUP, Cfg, uint16_t, true>(a, (long long)a.n_tiles * a.m_slots, (hipStream_t)stream);
-  });
+  GemmArgs a{};
+  a.A0 = xp; a.B0 = w1; a.B1 = w3; a.C0 = gu_blocked; a.C2 = act; a.offs = offs;
+  a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H;
+  return launch_rows<GATEUP, true>(a, CfgMain::BN / 2, (hipStream_t)stream);
 }
 
 extern "C" int moe_gemm_down_fwd(const uint16_t* act, const uint16_t* w2, const int32_t* offs,
@@ -1056,15 +1161,10 @@ extern "C" int moe_gemm_down_fwd(const uint16_t* act, const uint16_t* w2, const 
   if (int rc = check_common(offs, E, R, H, I)) return rc;
   if (R == 0) return 0;
   MOE_CHECK_PTR(act); MOE_CHECK_PTR(w2); MOE_CHECK_PTR(y);
-  return with_row_tile(small_row_tiles(R, E, H), [&](auto cfg) {
-    using Cfg = decltype(cfg);
-    GemmArgs a{};
-    a.A0 = act; a.B0 = w2; a.C0 = y; a.offs = offs;
-    a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I;
-    a.n_tiles = (int)((H + Cfg::BN - 1) / Cfg::BN);
-    a.m_slots = row_slots<Cfg>(R, E);
-    return launch<DOWN, Cfg, uint16_t>(a, (long long)a.n_tiles * a.m_slots, (hipStream_t)stream);
-  });
+  GemmArgs a{};
+  a.A0 = act; a.B0 = w2; a.C0 = y; a.offs = offs;
+  a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I;
+  return launch_rows<DOWN>(a, CfgMain::BN, (hipStream_t)stream);
 }
 
 // Test hook: 0 lets every row-ragged launch choose its row-tile height (the default), 128 or 256
@@ -1072,7 +1172,7 @@ extern "C" int moe_gemm_down_fwd(const uint16_t* act, const uint16_t* w2, const 
 // configuration, not for production callers.  Returns the previous setting.
 extern "C" int moe_gemm_force_row_tile(int rows) {
   const int before = forced_row_tile;
-  if (rows == 0 || rows == CfgSmall::BM || rows == CfgMain::BM) forced_row_tile = rows;
+  if (rows == 0 || rows == CfgHalf::BM || rows == CfgMain::BM) forced_row_tile = rows;
   return before;
 }
 
@@ -1088,16 +1188,11 @@ static int dgrad_down_impl(const uint16_t* dyp, const uint16_t* w2, const uint16
   if (R == 0) return 0;
   MOE_CHECK_PTR(dyp); MOE_CHECK_PTR(w2); MOE_CHECK_PTR(g); MOE_CHECK_PTR(u);
   MOE_CHECK_PTR(dg); MOE_CHECK_PTR(du);
-  return with_row_tile(small_row_tiles(R, E, I), [&](auto cfg) {
-    using Cfg = decltype(cfg);
-    GemmArgs a{};
-    a.C2 = dgate_part;
-    a.A0 = dyp; a.B0 = w2; a.X0 = g; a.X1 = u; a.C0 = dg; a.C1 = du; a.offs = offs;
-    a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H; a.ld_c = (int)ld_out;
-    a.n_tiles = (int)((I + Cfg::BN - 1) / Cfg::BN);
-    a.m_slots = row_slots<Cfg>(R, E);
-    return launch<DGRAD_DOWN, Cfg, uint16_t>(a, (long long)a.n_tiles * a.m_slots, (hipStream_t)stream);
-  });
+  GemmArgs a{};
+  a.C2 = dgate_part;
+  a.A0 = dyp; a.B0 = w2; a.X0 = g; a.X1 = u; a.C0 = dg; a.C1 = du; a.offs = offs;
+  a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H; a.ld_c = (int)ld_out;
+  return launch_rows<DGRAD_DOWN>(a, CfgMain::BN, (hipStream_t)stream);
 }
 
 extern "C" int moe_gemm_dgrad_down_swiglu_bwd(const uint16_t* dyp, const uint16_t* w2,
@@ -1125,16 +1220,11 @@ extern "C" int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const
   if (R == 0) return 0;
   MOE_CHECK_PTR(dyp); MOE_CHECK_PTR(w2); MOE_CHECK_PTR(gu_blocked); MOE_CHECK_PTR(dg); MOE_CHECK_PTR(du);
   if (ld_out != 0 && (ld_out < I || (ld_out % 8) != 0 || ld_out > (1 << 17))) return MOE_ERR_SHAPE;
-  return with_row_tile(small_row_tiles(R, E, I), [&](auto cfg) {
-    using Cfg = decltype(cfg);
-    GemmArgs a{};
-    a.C2 = dgate_part;
-    a.A0 = dyp; a.B0 = w2; a.X0 = (const uint16_t*)gu_blocked; a.C0 = dg; a.C1 = du; a.offs = offs;
-    a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H; a.ld_c = (int)ld_out;
-    a.n_tiles = (int)((I + Cfg::BN - 1) / Cfg::BN);
-    a.m_slots = row_slots<Cfg>(R, E);
-    return launch<DGRAD_DOWN, Cfg, uint16_t, true>(a, (long long)a.n_tiles * a.m_slots, (hipStream_t)stream);
-  });
+  GemmArgs a{};
+  a.C2 = dgate_part;
+  a.A0 = dyp; a.B0 = w2; a.X0 = (const uint16_t*)gu_blocked; a.C0 = dg; a.C1 = du; a.offs = offs;
+  a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H; a.ld_c = (int)ld_out;
+  return launch_rows<DGRAD_DOWN, true>(a, CfgMain::BN, (hipStream_t)stream);
 }
 
 // The two row gradients side by side in one buffer: dgu [R, 2I], row = [dg row | du row].  The
@@ -1155,15 +1245,10 @@ static int dgrad_gateup_impl(const uint16_t* dg, const uint16_t* du, int64_t ld_
   if (int rc = check_common(offs, E, R, H, I)) return rc;
   if (R == 0) return 0;
   MOE_CHECK_PTR(dg); MOE_CHECK_PTR(du); MOE_CHECK_PTR(w1); MOE_CHECK_PTR(w3); MOE_CHECK_PTR(dxp);
-  return with_row_tile(small_row_tiles(R, E, H), [&](auto cfg) {
-    using Cfg = decltype(cfg);
-    GemmArgs a{};
-    a.A0 = dg; a.A1 = du; a.B0 = w1; a.B1 = w3; a.C0 = dxp; a.offs = offs; a.ld_a = (int)ld_in;
-    a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I;
-    a.n_tiles = (int)((H + Cfg::BN - 1) / Cfg::BN);
-    a.m_slots = row_slots<Cfg>(R, E);
-    return launch<DGRAD_GATEUP, Cfg, uint16_t>(a, (long long)a.n_tiles * a.m_slots, (hipStream_t)stream);
-  });
+  GemmArgs a{};
+  a.A0 = dg; a.A1 = du; a.B0 = w1; a.B1 = w3; a.C0 = dxp; a.offs = offs; a.ld_a = (int)ld_in;
+  a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I;
+  return launch_rows<DGRAD_GATEUP>(a, CfgMain::BN, (hipStream_t)stream);
 }
 
 extern "C" int moe_gemm_dgrad_gateup_packed(const uint16_t* dgu, const uint16_t* w1, const uint16_t* w3,
@@ -1182,15 +1267,11 @@ extern "C" int moe_gemm_wgrad_pair(const uint16_t* dgu, const uint16_t* xp, cons
   MOE_CHECK_PTR(dw1); MOE_CHECK_PTR(dw3);
   if (R > 0) { MOE_CHECK_PTR(dgu); MOE_CHECK_PTR(xp); }
   if (dw_dtype != MOE_DT_BF16 && dw_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
-  using Cfg = CfgMain;
   GemmArgs a{};
   a.A0 = dgu; a.B0 = xp; a.C0 = dw1; a.C1 = dw3; a.offs = offs; a.m_split = (int)I;
   a.E = (int)E; a.R = (int)R; a.M = (int)(2 * I); a.N = (int)H; a.accumulate = accumulate;
-  a.n_tiles = (int)((H + Cfg::BN - 1) / Cfg::BN);
-  a.m_slots = (int)((2 * I + Cfg::BM - 1) / Cfg::BM);
-  const long long nblocks = (long long)a.n_tiles * a.m_slots * E;
-  if (dw_dtype == MOE_DT_F32) return launch<WGRAD, Cfg, float>(a, nblocks, (hipStream_t)stream);
-  return launch<WGRAD, Cfg, uint16_t>(a, nblocks, (hipStream_t)stream);
+  return dw_dtype == MOE_DT_F32 ? launch_wgrad<float>(a, (hipStream_t)stream)
+                                : launch_wgrad<uint16_t>(a, (hipStream_t)stream);
 }
 
 extern "C" int moe_gemm_dgrad_gateup(const uint16_t* dg, const uint16_t* du, const uint16_t* w1,
@@ -1206,25 +1287,17 @@ extern "C" int moe_gemm_wgrad(const uint16_t* a_, const uint16_t* b_, const int3
   MOE_CHECK_PTR(dw);
   if (R > 0) { MOE_CHECK_PTR(a_); MOE_CHECK_PTR(b_); }
   if (dw_dtype != MOE_DT_BF16 && dw_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
-  using Cfg = CfgMain;
   GemmArgs a{};
   a.A0 = a_; a.B0 = b_; a.C0 = dw; a.offs = offs;
   a.E = (int)E; a.R = (int)R; a.M = (int)M; a.N = (int)N; a.accumulate = accumulate;
-  a.n_tiles = (int)((N + Cfg::BN - 1) / Cfg::BN);
-  a.m_slots = (int)((M + Cfg::BM - 1) / Cfg::BM);
-  const long long nblocks = (long long)a.n_tiles * a.m_slots * E;
-  if (dw_dtype == MOE_DT_F32)
-    return launch<WGRAD, Cfg, float>(a, nblocks, (hipStream_t)stream);
-  return launch<WGRAD, Cfg, uint16_t>(a, nblocks, (hipStream_t)stream);
+  return dw_dtype == MOE_DT_F32 ? launch_wgrad<float>(a, (hipStream_t)stream)
+                                : launch_wgrad<uint16_t>(a, (hipStream_t)stream);
 }
 
 int moe_wgrad_slices(const uint16_t* a_, const uint16_t* b_, int64_t T, int64_t M, int64_t N, int64_t slices,
                      int64_t slice_rows, float* part, hipStream_t s) {
-  using Cfg = CfgMain;
   GemmArgs a{};
   a.A0 = a_; a.B0 = b_; a.C0 = part; a.slice = (int)slice_rows;
   a.E = (int)slices; a.R = (int)T; a.M = (int)M; a.N = (int)N;
-  a.n_tiles = (int)((N + Cfg::BN - 1) / Cfg::BN);
-  a.m_slots = (int)((M + Cfg::BM - 1) / Cfg::BM);
-  return launch<WGRAD, Cfg, float>(a, (long long)a.n_tiles * a.m_slots * slices, s);
+  return launch_wgrad<float>(a, s);
 }

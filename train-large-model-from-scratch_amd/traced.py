@@ -37,9 +37,9 @@ def _empty(ref: Tensor, dtype=_BF16) -> Tensor:
 
 def gu_blocked_bytes(R, E: int, I: int):
     """Size of ops.gemm_gateup_blocked's buffer, as arithmetic a symbolic row count passes through:
-    moe_gu_blocked_bytes (4 KB per 32 x 32 block of ceil(R/256) + E row tiles of 256 rows), with
-    the wrapper's floor of 16 bytes."""
-    return (((R + 255) // 256 + E) * 8 * ((I + 31) // 32) * 4096) if R > 0 else 16
+    moe_gu_blocked_bytes (4 KB per 32 x 32 block of at most R/32 + E row blocks), with the
+    wrapper's floor of 16 bytes."""
+    return ((R // 32 + E) * ((I + 31) // 32) * 4096) if R > 0 else 16
 
 
 @torch.library.custom_op("moe_gfx950::ffn_fwd", mutates_args=(), device_types="cuda")
