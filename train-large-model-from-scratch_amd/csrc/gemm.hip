@@ -135,6 +135,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     int e, row0, row_end, n0, m0;
     int block0;  // first of its 32-row blocks in the blocked g/u layout
     int Kseg, kt_per_seg, nkt;
+    int kt0;  // k-tile it starts with (it goes round)
     bool need_mask;
     View vA0, vA1, vB0, vB1;
   };
@@ -186,6 +187,16 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     // last k-tile cleared by hand (outside the static schedule)
     t.need_mask = ((t.Kseg % BK) != 0) && (!A_OUTER || !B_OUTER);
     const long long rows = t.row_end - t.row0;
+    // With few rows an expert is bound by its weights, each line of which is read once.  Where their rows are a
+    // multiple of 4 KB long, experts that sweep k side by side ask for the same lines of every page, which lie on few
+    // of the memory channels; started at different k-tiles they do not (all tiles of an expert at the same one, so
+    // that they go on sharing the operands in L2).  Gate/up of 64 experts, 2048 <-> 1024, rows per expert and us: 64,
+    // 130 -> 98; 128, 134 -> 107; 191, 147 -> 131; 256, 152 -> 144; from 384 on no difference.  Down, 1024 <-> 2048, 128
+    // rows: 78 -> 60.  With rows of 2 KB there is nothing to gain.
+    t.kt0 = 0;
+    if constexpr (MODE == GATEUP || MODE == DOWN) {
+      if (p.K % 2048 == 0) t.kt0 = (t.e * 13) & 31;  // (32 k-tiles to 4 KB)
+    }
     if constexpr (MODE == GATEUP) {
       t.vA0 = make_view(p.A0 + (long long)t.row0 * lda, rows * lda);
       const long long wofs = ((long long)t.e * p.N + t.n0) * p.K;
@@ -235,7 +246,11 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   };
   auto tile_src = [&](const Tile& t, int kt) {
     const int seg = (NSEG == 2) ? kt / t.kt_per_seg : 0;
-    const int k0 = (kt - seg * t.kt_per_seg) * BK;
+    int k0 = (kt - seg * t.kt_per_seg) * BK;
+    if constexpr (MODE == GATEUP || MODE == DOWN) {
+      const int at = kt + t.kt0;
+      k0 = (at >= t.nkt ? at - t.nkt : at) * BK;
+    }
     TileSrc ts;
     ts.a = view_rsrc((NSEG == 2 && seg) ? t.vA1 : t.vA0, StA::k_bytes(k0, lda));
     if constexpr (DUAL) {
