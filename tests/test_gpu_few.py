@@ -13,6 +13,9 @@ pytestmark = pytest.mark.gpu
     (1, 64, 8, 256, 136, torch.bfloat16),    # one token: the kernel that also combines
     (1, 4, 3, 2056, 1032, torch.float32),    # ... contractions that end inside a step, experts' shares split
     (1, 40, 33, 64, 64, torch.bfloat16),     # ... more experts a token than that kernel takes
+    (1, 128, 8, 264, 520, torch.bfloat16),   # ... selected from two logits a lane
+    (1, 65, 32, 72, 136, torch.float32),     # ... the most experts a token that the combining kernel takes
+    (1, 130, 8, 264, 24, torch.bfloat16),    # ... selected by the router kernel
     (2, 128, 1, 520, 8, torch.float32),
     (16, 4, 4, 136, 248, torch.bfloat16),    # every expert has 16 rows
     (17, 4, 4, 136, 248, torch.bfloat16),    # ... 17

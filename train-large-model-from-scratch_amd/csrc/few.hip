@@ -11,6 +11,7 @@
 // the first product where it fits.
 #include "common.h"
 #include "internal.h"
+#include "topk_core.h"
 
 namespace {
 
@@ -252,12 +253,24 @@ __device__ __forceinline__ void few_columns_16(const AT* __restrict__ A, int div
   else few_columns<AT, NB, 1, 8, 0>(A, div, w, e, n0, nblk, N, K, rows, n, part, C);
 }
 
-// ONE: a single token; block row j takes its j-th expert and no list is needed.
-template <typename AT, int NB, bool ONE>
+// The selection of a single token, made by every wave for itself (128 experts: in about the time its ids would take to
+// arrive, where a launch of its own costs more: 64 experts, 2048 <-> 1024, 33.5 -> 32.1 us a
+// token; 128 experts, 1024 <-> 256, 28.2 -> 25.0).
+struct Selection {
+  const void* logits;
+  const float* bias;
+  int32_t* ids;  // results, written by the first workgroup
+  float* gates;
+  int logits_f32, k;
+};
+
+// ONE: a single token; block row j takes its j-th expert and no list is needed.  VPL > 0: which one that is comes from
+// the logits of at most 64 * VPL experts, not from ids.
+template <typename AT, int NB, bool ONE, int VPL = 0>
 __global__ __launch_bounds__(256, 2) void few_kernel(const AT* __restrict__ A, int div, const int32_t* __restrict__ ids,
                                                     int R, const uint16_t* __restrict__ w0,
                                                     const uint16_t* __restrict__ w1, int E, int N, int K, int nblk,
-                                                    uint16_t* __restrict__ C) {
+                                                    uint16_t* __restrict__ C, const Selection sel) {
   __shared__ int rows[FEW_MAX_TOKENS], count;
   __shared__ float part[2 * 4 * NB * (ONE ? 1 : 4) * 256];
   const uint16_t* w[NB];
@@ -267,7 +280,23 @@ __global__ __launch_bounds__(256, 2) void few_kernel(const AT* __restrict__ A, i
   const int nb = left < nblk ? left : nblk;
   if constexpr (ONE) {
     const int j = blockIdx.y;
-    int e = ids[j];
+    int e;
+    if constexpr (VPL > 0) {
+      const int lane = lane_id();
+      uint64_t key[VPL];
+      if (sel.logits_f32) moe_topk_keys<VPL>((const float*)sel.logits, sel.bias, E, lane, key);
+      else moe_topk_keys<VPL>((const uint16_t*)sel.logits, sel.bias, E, lane, key);
+      int id;
+      float gate;
+      moe_topk_softmax_wave<VPL>(key, sel.k, lane, id, gate);
+      if (blockIdx.x == 0 && j == 0 && threadIdx.x < sel.k) {
+        sel.ids[lane] = id;
+        sel.gates[lane] = gate;
+      }
+      e = __builtin_amdgcn_readlane(id, j);
+    } else {
+      e = ids[j];
+    }
     e = e < 0 ? 0 : (e >= E ? E - 1 : e);
     if (threadIdx.x == 0) rows[0] = j;
     __syncthreads();
@@ -380,7 +409,7 @@ int moe_gateup_few(const void* x, int x_dtype, const int32_t* ids, const uint16_
   const auto go = [&](auto one, auto xt) {
     using XT = decltype(xt);
     hipLaunchKernelGGL((few_kernel<XT, 2, decltype(one)::value>), grid, block, 0, s, (const XT*)x, (int)k, ids, (int)(T * k),
-                       w1, w3, (int)E, (int)I, (int)H, nblk, act);
+                       w1, w3, (int)E, (int)I, (int)H, nblk, act, Selection{});
     return moe_launch_status();
   };
   if (x_dtype == MOE_DT_BF16) return T == 1 ? go(std::true_type{}, uint16_t{}) : go(std::false_type{}, uint16_t{});
@@ -392,8 +421,29 @@ int moe_down_few(const uint16_t* act, const int32_t* ids, const uint16_t* w2, in
   const int nblk = few_blocks(H, T * k < E ? T * k : E);
   const dim3 grid((unsigned)(((H + 15) / 16 + nblk - 1) / nblk), (unsigned)E), block(256);
   hipLaunchKernelGGL((few_kernel<uint16_t, 1, false>), grid, block, 0, s, act, 1, ids, (int)(T * k), w2, nullptr, (int)E,
-                     (int)H, (int)I, nblk, y);
+                     (int)H, (int)I, nblk, y, Selection{});
   return moe_launch_status();
+}
+
+// (64 threads of the first workgroup write the results)
+bool moe_gateup_one_ok(int64_t T, int64_t E, int64_t k) { return moe_down_one_ok(T, k) && E <= 2 * MOE_WAVE; }
+
+int moe_gateup_one(const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias, const uint16_t* w1,
+                   const uint16_t* w3, int64_t H, int64_t E, int64_t I, int64_t k, int32_t* ids, float* gates,
+                   uint16_t* act, hipStream_t s) {
+  const int nblk = few_blocks(I, k);
+  const dim3 grid((unsigned)(((I + 15) / 16 + nblk - 1) / nblk), (unsigned)k), block(256);
+  const Selection sel{logits, bias, ids, gates, logits_dtype == MOE_DT_F32, (int)k};
+  const auto go = [&](auto vpl, auto xt) {
+    using XT = decltype(xt);
+    hipLaunchKernelGGL((few_kernel<XT, 2, true, decltype(vpl)::value>), grid, block, 0, s, (const XT*)x, (int)k, nullptr,
+                       (int)k, w1, w3, (int)E, (int)I, (int)H, nblk, act, sel);
+    return moe_launch_status();
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  if (x_dtype == MOE_DT_BF16) return E <= MOE_WAVE ? go(One{}, uint16_t{}) : go(Two{}, uint16_t{});
+  return E <= MOE_WAVE ? go(One{}, float{}) : go(Two{}, float{});
 }
 
 bool moe_down_one_ok(int64_t T, int64_t k) { return T == 1 && k <= DOWN_ONE_MAX_K; }

@@ -20,18 +20,7 @@ __global__ __launch_bounds__(256) void router_topk_fwd_kernel(const LT* __restri
   const int t = blockIdx.x * (blockDim.x / MOE_WAVE) + (threadIdx.x / MOE_WAVE);
   if (t >= T) return;  // whole wave exits together
   uint64_t key[VPL];
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) {
-    const int e = i * MOE_WAVE + lane;
-    key[i] = 0;
-    if (e < E) {
-      float v;
-      if constexpr (sizeof(LT) == 2) v = bf16_to_f32(((const uint16_t*)logits)[(size_t)t * E + e]);
-      else v = ((const float*)logits)[(size_t)t * E + e];
-      if (bias) v += bias[e];
-      key[i] = moe_topk_key(v, e);
-    }
-  }
+  moe_topk_keys<VPL>(logits + (size_t)t * E, bias, E, lane, key);
   int my_id;
   float my_gate;
   moe_topk_softmax_wave<VPL>(key, k, lane, my_id, my_gate);

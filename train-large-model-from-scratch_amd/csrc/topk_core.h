@@ -53,6 +53,24 @@ __device__ __forceinline__ float moe_wave_sum_f32(float v) {
   return v;
 }
 
+// The keys of one token's E logits, plus the experts' biases unless NULL.
+template <int VPL, typename LT>
+__device__ __forceinline__ void moe_topk_keys(const LT* __restrict__ logits, const float* __restrict__ bias, int E, int lane,
+                                              uint64_t (&key)[VPL]) {
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int e = i * MOE_WAVE + lane;
+    key[i] = 0;
+    if (e < E) {
+      float v;
+      if constexpr (sizeof(LT) == 2) v = bf16_to_f32(((const uint16_t*)logits)[e]);
+      else v = ((const float*)logits)[e];
+      if (bias) v += bias[e];
+      key[i] = moe_topk_key(v, e);
+    }
+  }
+}
+
 // k rounds of a wave-wide maximum over the keys (consumed), then the softmax over the k selected
 // logits in fp32.  On return lane j < k holds slot j: expert id and gate.
 template <int VPL>
