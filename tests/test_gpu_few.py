@@ -12,6 +12,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T,E,k,H,I,x_dt", [
     (1, 64, 8, 256, 136, torch.bfloat16),    # one token: the kernel that also combines
     (1, 4, 3, 2056, 1032, torch.float32),    # ... contractions that end inside a step, experts' shares split
+    (1, 8, 2, 4104, 72, torch.bfloat16),     # ... that many columns that a workgroup takes 16
+    (1, 8, 3, 4096, 2120, torch.float32),    # ... and several requests for each share
+    (1, 16, 8, 2040, 2120, torch.bfloat16),  # ... 8
     (1, 40, 33, 64, 64, torch.bfloat16),     # ... more experts a token than that kernel takes
     (1, 128, 8, 264, 520, torch.bfloat16),   # ... selected from two logits a lane
     (1, 65, 32, 72, 136, torch.float32),     # ... the most experts a token that the combining kernel takes

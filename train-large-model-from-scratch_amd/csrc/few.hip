@@ -312,63 +312,82 @@ __global__ __launch_bounds__(256, 2) void few_kernel(const AT* __restrict__ A, i
 }
 
 // ---- down projection and combine of one token -----------------------------------------------------------------
-// out[h] = sum_j gate[j] bf16(y[j][h]) for the 16 columns h of this block: the block's eight waves take the
+// out[h] = sum_j gate[j] bf16(y[j][h]) for the COLS columns h of this block: the block's eight waves take the
 // token's experts in turn (or shares of their contractions, where fewer than eight are asked for) and leave
 // their sums in LDS, where they are added up in slot order, as the combine kernel does.
+// COLS = 8: the product's 16 columns are 8 columns twice, once for each half of the share (row 0 of the other operand is the
+// first half of the token's row, row 1 the second), so that twice the workgroups ask for weights.
+// (One token, 64 experts, 2048 <-> 1024, k = 8, the whole layer: 32.7 -> 31.0 us; k = 2 and 4: no difference.)
 constexpr int DOWN_WAVES = 8;
-template <typename OT>
+template <typename OT, int COLS>
 __global__ __launch_bounds__(DOWN_WAVES* MOE_WAVE) void down_one_kernel(const uint16_t* __restrict__ act,
                                                                        const int32_t* __restrict__ ids,
                                                                        const float* __restrict__ gates, int k,
                                                                        const uint16_t* __restrict__ w2, int E, int H,
                                                                        int I, OT* __restrict__ out) {
-  constexpr int KC = 32;                                             // k-steps requested at once
+  constexpr int PARTS = 16 / COLS;                                   // of a share
+  constexpr int KC = 32 / PARTS;                                     // k-steps of a part requested at once
   __shared__ float y[DOWN_WAVES + DOWN_ONE_MAX_K][16];               // [splits][k]
-  __shared__ __align__(16) uint16_t arow[DOWN_WAVES][KC * 32];       // a wave's piece of its row of act
+  __shared__ __align__(16) uint16_t arow[DOWN_WAVES][32 * 32];       // a wave's pieces of its row of act
   const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MOE_WAVE)), l16 = lane & 15,
             lq = lane >> 4;
-  const int h0 = blockIdx.x * 16;
+  const int h0 = blockIdx.x * COLS;
+  const int col = l16 % COLS, part = l16 / COLS;
   const int splits = k >= DOWN_WAVES ? 1 : DOWN_WAVES / k;
-  const int steps = (I + 31) / 32, per = ((steps + splits - 1) / splits + 1) & ~1;
+  const int steps = (I + 31) / 32, per = ((steps + splits * PARTS - 1) / (splits * PARTS) + 1) & ~1;  // of a part
   for (int item = wv; item < k * splits; item += DOWN_WAVES) {
     const int j = item / splits, sp = item - j * splits;
     int e = __builtin_amdgcn_readfirstlane(ids[j]);
     e = e < 0 ? 0 : (e >= E ? E - 1 : e);
-    const int s_lo = sp * per, s_hi = s_lo + per < steps ? s_lo + per : steps;
-    const __amdgpu_buffer_rsrc_t rs[1] = {rsrc(w2 + ((size_t)e * H + h0) * I, (long long)(H - h0) * I * 2)};
+    const int s_lo = sp * PARTS * per;                               // of the first part
+    const auto end_of = [&](int p) { return s_lo + (p + 1) * per < steps ? s_lo + (p + 1) * per : steps; };
+    const __amdgpu_buffer_rsrc_t rw = rsrc(w2 + ((size_t)e * H + h0) * I, (long long)(H - h0) * I * 2);
     const __amdgpu_buffer_rsrc_t ra = rsrc(act + (size_t)j * I, (long long)I * 2);
-    f32x4 acc[1][1] = {{f32x4{0.f, 0.f, 0.f, 0.f}}};
-    for (int s = s_lo; s < s_hi; s += KC) {
-      Columns<1, KC> c;
-      request<1, KC>(c, rs, h0 + l16 < H, I, s, s_hi);
-      // (a single row: in operand layout 15 of 16 lanes would carry zeros, so it comes through LDS)
-#pragma unroll
-      for (int i = 0; i < KC * 32 / (MOE_WAVE * 8); ++i) {
-        const int at = (i * MOE_WAVE + lane) * 8;
-        *reinterpret_cast<bf16x8*>(&arow[wv][at]) = load_frag(ra, (unsigned)(s * 32 + at) * 2);
-      }
-      __builtin_amdgcn_wave_barrier();
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < per; s += KC) {
+      const int first = s_lo + part * per + s, end = end_of(part);
+      bf16x8 w[KC];
 #pragma unroll
       for (int d = 0; d < KC; ++d) {
-        bf16x8 a = *reinterpret_cast<const bf16x8*>(&arow[wv][d * 32 + lq * 8]);
-        if (l16 != 0) a = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
-        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, c.v[0][d], acc[0][0], 0, 0, 0);
+        const int kk = (first + d) * 32 + lq * 8;
+        const bool in = (PARTS == 1 || s + d < per) && first + d < end && kk < I && h0 + col < H;
+        w[d] = load_frag(rw, in ? (unsigned)(col * I + kk) * 2 : OUTSIDE);
+      }
+      // (a single row: in operand layout 15 of 16 lanes would carry zeros, so it comes through LDS)
+#pragma unroll
+      for (int i = 0; i < 32 * 32 / (MOE_WAVE * 8); ++i) {
+        const int at = (i * MOE_WAVE + lane) * 8, p = at / (KC * 32), in_p = at % (KC * 32);
+        const int step = s + in_p / 32;
+        const bool in = PARTS == 1 || (step < per && s_lo + p * per + step < end_of(p));  // (the next part's must not count)
+        *reinterpret_cast<bf16x8*>(&arow[wv][at]) =
+            load_frag(ra, in ? (unsigned)((s_lo + p * per + s) * 32 + in_p) * 2 : OUTSIDE);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int d = 0; d < KC; ++d) {  // operand row p: part p
+        bf16x8 a = *reinterpret_cast<const bf16x8*>(&arow[wv][(l16 % PARTS) * KC * 32 + d * 32 + lq * 8]);
+        if (l16 >= PARTS) a = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[d], acc, 0, 0, 0);
       }
       __builtin_amdgcn_wave_barrier();
     }
-    if (lq == 0) y[sp * k + j][l16] = acc[0][0][0];  // row 0 of the product
+    if (lq == 0) y[sp * k + j][l16] = part == 0 ? acc[0] : acc[1];  // row `part` of the product
   }
   __syncthreads();
-  if (threadIdx.x < 16 && h0 + threadIdx.x < H) {
+  if (threadIdx.x < COLS && h0 + threadIdx.x < H) {
     const int c = threadIdx.x;
-    float acc = 0.f;
+    float sum = 0.f;
     for (int j = 0; j < k; ++j) {
       float v = y[j][c];
-      for (int sp = 1; sp < splits; ++sp) v += y[sp * k + j][c];
-      acc += gates[j] * bf16_to_f32(f32_to_bf16(v));
+      if constexpr (PARTS == 2) v += y[j][COLS + c];
+      for (int sp = 1; sp < splits; ++sp) {
+        v += y[sp * k + j][c];
+        if constexpr (PARTS == 2) v += y[sp * k + j][COLS + c];
+      }
+      sum += gates[j] * bf16_to_f32(f32_to_bf16(v));
     }
-    if constexpr (sizeof(OT) == 2) out[h0 + c] = f32_to_bf16(acc);
-    else out[h0 + c] = acc;
+    if constexpr (sizeof(OT) == 2) out[h0 + c] = f32_to_bf16(sum);
+    else out[h0 + c] = sum;
   }
 }
 
@@ -450,12 +469,17 @@ bool moe_down_one_ok(int64_t T, int64_t k) { return T == 1 && k <= DOWN_ONE_MAX_
 
 int moe_down_one(const uint16_t* act, const int32_t* ids, const float* gates, const uint16_t* w2, int64_t H, int64_t E,
                  int64_t I, int64_t k, void* out, int out_dtype, hipStream_t s) {
-  const dim3 grid((unsigned)((H + 15) / 16)), block(DOWN_WAVES * MOE_WAVE);
-  if (out_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL(down_one_kernel<uint16_t>, grid, block, 0, s, act, ids, gates, (int)k, w2, (int)E, (int)H, (int)I,
-                       (uint16_t*)out);
-  else
-    hipLaunchKernelGGL(down_one_kernel<float>, grid, block, 0, s, act, ids, gates, (int)k, w2, (int)E, (int)H, (int)I,
-                       (float*)out);
-  return moe_launch_status();
+  // (more workgroups than compute units of the narrow kind: 2880 columns, 32.3 -> 34.0 us a token)
+  const bool wide = (H + 7) / 8 > moe_compute_units();
+  const auto go = [&](auto cols, auto ot) {
+    using OT = decltype(ot);
+    constexpr int COLS = decltype(cols)::value;
+    hipLaunchKernelGGL((down_one_kernel<OT, COLS>), dim3((unsigned)((H + COLS - 1) / COLS)), dim3(DOWN_WAVES * MOE_WAVE), 0,
+                       s, act, ids, gates, (int)k, w2, (int)E, (int)H, (int)I, (OT*)out);
+    return moe_launch_status();
+  };
+  using Narrow = std::integral_constant<int, 8>;
+  using Wide = std::integral_constant<int, 16>;
+  if (out_dtype == MOE_DT_BF16) return wide ? go(Wide{}, uint16_t{}) : go(Narrow{}, uint16_t{});
+  return wide ? go(Wide{}, float{}) : go(Narrow{}, float{});
 }
