@@ -1,0 +1,38 @@
+"""What a call is refused for on the host, before anything is launched: on tensors that only claim to be on a
+GPU (no storage, no kernel runs), so that the checks are seen without one."""
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+from conftest import load_pkg
+
+BF16, F32 = torch.bfloat16, torch.float32
+T, H, E, I, K = 4, 64, 8, 32, 2
+
+
+def _gpu(*shape, dtype=BF16):
+    return torch.empty(*shape, device="cuda", dtype=dtype)
+
+
+def _weights(dtype=BF16):
+    return [_gpu(E, I, H, dtype=dtype), _gpu(E, I, H, dtype=dtype), _gpu(E, H, I, dtype=dtype)]
+
+
+@pytest.mark.parametrize("entry", ["moe_ffn", "routed_moe", "prenorm_moe"])
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("wrong,error,match", [
+    (lambda c: c.transpose(1, 2).contiguous().transpose(1, 2), RuntimeError, "contiguous"),
+    (lambda c: c.float(), TypeError, "bf16"),
+    (lambda c: c[:-1], RuntimeError, "shape"),
+    (lambda c: c.new_empty(E, c.shape[2], c.shape[1]), RuntimeError, "shape"),
+    (lambda c: torch.empty(c.shape, dtype=BF16, device="cpu"), RuntimeError, "GPU"),
+])
+def test_copies_of_the_weights_are_what_a_cast_would_give(entry, which, wrong, error, match):
+    pkg = load_pkg()
+    with FakeTensorMode():
+        x, wr = _gpu(T, H, dtype=F32), _gpu(E, H)
+        masters, copies = _weights(F32), _weights()
+        copies[which] = wrong(copies[which])
+        front = {"moe_ffn": (x, _gpu(T, E)), "routed_moe": (x, wr), "prenorm_moe": (x, _gpu(H, dtype=F32), wr)}[entry]
+        with pytest.raises(error, match=match):
+            getattr(pkg, entry)(*front, *masters, K, bf16_weights=copies)

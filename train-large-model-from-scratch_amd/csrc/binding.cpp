@@ -136,6 +136,16 @@ Weights bf16_weights(const Tensor& w1, const Tensor& w3, const Tensor& w2, const
   return {one(w1, s1), one(w3, s3), one(w2, s2)};
 }
 
+// A copy the caller made is read in place of its master: it has to be what cast_bf16(dense(master)) would be.
+void check_copy(const OptTensor& s, const Tensor& w, const Tensor& x) {
+  if (!s || !s->defined()) return;
+  need_gpu(*s);
+  TORCH_CHECK(s->device() == x.device(), "a bf16 copy of the weights is on ", s->device(), ", x on ", x.device());
+  TORCH_CHECK_TYPE(s->scalar_type() == at::kBFloat16, "the copies of the weights must be bf16, got ", s->scalar_type());
+  TORCH_CHECK(s->sizes() == w.sizes(), "a bf16 copy has shape ", s->sizes(), ", its weights ", w.sizes());
+  TORCH_CHECK(s->is_contiguous(), "the MoE kernels need contiguous tensors: a bf16 copy of the weights is strided");
+}
+
 const Tensor& value(const OptTensor& t) {
   static const Tensor none;
   return t ? *t : none;
@@ -171,16 +181,17 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
                 const Tensor& w1, const Tensor& w3, const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
   Outputs f;
   need_gpu(x_);
-  const c10::DeviceGuard guard(x_.device());
-  const Tensor x = dense(x_);
-  TORCH_CHECK(x.dim() == 2 && w1.dim() == 3, "the layer takes x [tokens, hidden] and weights [experts, ., .]");
-  const int64_t T = x.size(0), H = x.size(1), I = w1.size(1), k = o.k, R = T * k;
+  TORCH_CHECK(x_.dim() == 2 && w1.dim() == 3, "the layer takes x [tokens, hidden] and weights [experts, ., .]");
+  const int64_t T = x_.size(0), H = x_.size(1), I = w1.size(1), k = o.k, R = T * k;
   const int64_t E = wr.defined() ? wr.size(0) : logits_.defined() ? logits_.size(1) : w1.size(0);
   TORCH_CHECK(w1.size(0) == E && w3.size(0) == E && w2.size(0) == E && w1.size(2) == H && w3.size(2) == H &&
                   w3.size(1) == I && w2.size(1) == H && w2.size(2) == I,
               "the weights' shapes do not belong together");
-  (void)dt(x);
-  const at::ScalarType x_type = x.scalar_type();
+  check_copy(o.s1, w1, x_), check_copy(o.s3, w3, x_), check_copy(o.s2, w2, x_);
+  (void)dt(x_);
+  const at::ScalarType x_type = x_.scalar_type();
+  const c10::DeviceGuard guard(x_.device());
+  const Tensor x = dense(x_);
   f.w = bf16_weights(w1, w3, w2, o.s1, o.s3, o.s2);
   void* s = stream_of(x);
   const Routing r(R, E);
