@@ -36,3 +36,27 @@ def test_copies_of_the_weights_are_what_a_cast_would_give(entry, which, wrong, e
         front = {"moe_ffn": (x, _gpu(T, E)), "routed_moe": (x, wr), "prenorm_moe": (x, _gpu(H, dtype=F32), wr)}[entry]
         with pytest.raises(error, match=match):
             getattr(pkg, entry)(*front, *masters, K, bf16_weights=copies)
+
+
+@pytest.mark.parametrize("tokens", [T, 65])
+@pytest.mark.parametrize("shape", [(E, H - 8), (E, H + 8), (E, H, 1)])
+def test_router_weight_has_the_width_of_x(tokens, shape):
+    pkg = load_pkg()
+    with FakeTensorMode():
+        x, wr = _gpu(tokens, H), _gpu(*shape)
+        for call in (lambda: pkg.routed_moe(x, wr, *_weights(), K),
+                     lambda: pkg.prenorm_moe(x, _gpu(H, dtype=F32), wr, *_weights(), K)):
+            with pytest.raises(RuntimeError, match="router weight"):
+                call()
+        with pytest.raises(RuntimeError, match="mat1 and mat2|reduction dim|expects a tensor"):
+            pkg.router_linear(x, wr)
+
+
+def test_router_weight_is_where_x_is():
+    pkg = load_pkg()
+    with FakeTensorMode():
+        x, wr = _gpu(T, H), torch.empty(E, H, dtype=BF16, device="cpu")
+        with pytest.raises(RuntimeError, match="GPU"):
+            pkg.routed_moe(x, wr, *_weights(), K)
+        with pytest.raises(RuntimeError, match="device"):
+            pkg.router_linear(x, wr)

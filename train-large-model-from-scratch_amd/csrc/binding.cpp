@@ -187,6 +187,11 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   TORCH_CHECK(w1.size(0) == E && w3.size(0) == E && w2.size(0) == E && w1.size(2) == H && w3.size(2) == H &&
                   w3.size(1) == I && w2.size(1) == H && w2.size(2) == I,
               "the weights' shapes do not belong together");
+  if (wr.defined()) {
+    need_gpu(wr);
+    TORCH_CHECK(wr.dim() == 2 && wr.size(1) == H, "the router weight has shape ", wr.sizes(), ", x ", x_.sizes());
+    TORCH_CHECK(wr.device() == x_.device(), "the router weight is on ", wr.device(), ", x on ", x_.device());
+  }
   check_copy(o.s1, w1, x_), check_copy(o.s3, w3, x_), check_copy(o.s2, w2, x_);
   (void)dt(x_);
   const at::ScalarType x_type = x_.scalar_type();
@@ -495,8 +500,8 @@ Tensor router_logits(const Tensor& x, const Tensor& wr) {
   const NoAutocast no_autocast;
   const int64_t T = x.size(0), H = x.size(1), E = wr.size(0);
   if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || wr.scalar_type() != at::kBFloat16 || H % 8 != 0 ||
-      !moe_router_few_ok(T, H, E, 1))
-    return at::mm(x, wr.t());
+      !moe_router_few_ok(T, H, E, 1) || x.dim() != 2 || wr.dim() != 2 || wr.size(1) != H || wr.device() != x.device())
+    return at::mm(x, wr.t());  // (which also refuses what does not belong together)
   const c10::DeviceGuard guard(x.device());
   const Tensor xd = dense(x), wd = dense(wr);
   Tensor logits = empty({T, E}, at::kBFloat16, x);
