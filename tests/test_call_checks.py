@@ -60,3 +60,15 @@ def test_router_weight_is_where_x_is():
             pkg.routed_moe(x, wr, *_weights(), K)
         with pytest.raises(RuntimeError, match="device"):
             pkg.router_linear(x, wr)
+
+
+@pytest.mark.parametrize("weight,match", [
+    (lambda: torch.empty(H, device="cpu"), "GPU"),
+    (lambda: _gpu(H - 8, dtype=F32), "norm's weight"),
+    (lambda: _gpu(2 * H, dtype=F32), "norm's weight"),
+])
+def test_norm_weight_is_on_the_gpu_and_as_wide_as_x(weight, match):
+    pkg = load_pkg()
+    with FakeTensorMode():
+        with pytest.raises(RuntimeError, match=match):
+            pkg.prenorm_moe(_gpu(T, H), weight(), _gpu(E, H), *_weights(), K)

@@ -192,6 +192,11 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
     TORCH_CHECK(wr.dim() == 2 && wr.size(1) == H, "the router weight has shape ", wr.sizes(), ", x ", x_.sizes());
     TORCH_CHECK(wr.device() == x_.device(), "the router weight is on ", wr.device(), ", x on ", x_.device());
   }
+  if (norm_w.defined()) {
+    need_gpu(norm_w);
+    TORCH_CHECK(norm_w.numel() == H, "the norm's weight has ", norm_w.numel(), " elements, x is ", H, " wide");
+    TORCH_CHECK(norm_w.device() == x_.device(), "the norm's weight is on ", norm_w.device(), ", x on ", x_.device());
+  }
   check_copy(o.s1, w1, x_), check_copy(o.s3, w3, x_), check_copy(o.s2, w2, x_);
   (void)dt(x_);
   const at::ScalarType x_type = x_.scalar_type();
