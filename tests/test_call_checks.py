@@ -1,5 +1,7 @@
 """What a call is refused for on the host, before anything is launched: on tensors that only claim to be on a
 GPU (no storage, no kernel runs), so that the checks are seen without one."""
+import importlib
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -72,3 +74,27 @@ def test_norm_weight_is_on_the_gpu_and_as_wide_as_x(weight, match):
     with FakeTensorMode():
         with pytest.raises(RuntimeError, match=match):
             pkg.prenorm_moe(_gpu(T, H), weight(), _gpu(E, H), *_weights(), K)
+
+
+@pytest.mark.parametrize("dual", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("entry", ["moe_ffn", "moe_ffn_f32", "routed_moe", "prenorm_moe", "experts_rows",
+                                   "experts_rows_f32"])
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("return_routing", [False, True])
+def test_forward_mode_is_refused(entry, dual, grad, return_routing):
+    """... whether or not anything requires a gradient (plain host tensors: the refusal comes first)."""
+    pkg = load_pkg()
+    w = [torch.zeros(E, I, H, requires_grad=grad), torch.zeros(E, I, H), torch.zeros(E, H, I)]
+    x, wr, norm, logits, ids = torch.zeros(T, H), torch.zeros(E, H), torch.ones(H), torch.zeros(T, E), torch.zeros(T)
+    args = {"moe_ffn": [x, logits, *w, K], "moe_ffn_f32": [x, logits, *w, K], "routed_moe": [x, wr, *w, K],
+            "prenorm_moe": [x, norm, wr, *w, K], "experts_rows": [x, ids.long(), *w],
+            "experts_rows_f32": [x, ids.long(), *w]}[entry]
+    floats = [i for i, a in enumerate(args) if torch.is_tensor(a) and a.is_floating_point()]
+    at = floats[dual % len(floats)]
+    fn = getattr(importlib.import_module(pkg.__name__ + ".functional"), entry)
+    with torch.autograd.forward_ad.dual_level():
+        args[at] = torch.autograd.forward_ad.make_dual(args[at], torch.ones_like(args[at]))
+        with pytest.raises(NotImplementedError):
+            fn(*args, return_routing=return_routing)
+        with torch.no_grad(), pytest.raises(NotImplementedError):
+            fn(*args, return_routing=return_routing)

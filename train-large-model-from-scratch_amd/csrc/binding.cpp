@@ -74,6 +74,14 @@ void need_gpu(const Tensor& t) {
   TORCH_CHECK(!t.defined() || t.is_cuda(), "the MoE kernels need GPU tensors (no CPU path exists)");
 }
 
+// The kernels read pointers: a tangent that forward-mode differentiation hangs on an input would be lost without a
+// word, in the node (whose backward is all it has) and around it (where nothing requires a gradient).
+void no_tangents(std::initializer_list<const Tensor*> inputs) {
+  for (const Tensor* t : inputs)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(/*level=*/0).defined(),
+                                "the MoE kernels have no forward-mode derivative");
+}
+
 // Contiguous and 16-byte aligned, as the kernels need their buffers.
 Tensor dense(const Tensor& t) {
   need_gpu(t);
@@ -522,6 +530,7 @@ std::tuple<Tensor, OptTensor, OptTensor> layer(const Tensor& x, const OptTensor&
                                                double eps, bool add_residual, bool fused_router, bool accumulate,
                                                bool want_routing) {
   const Tensor &n = value(norm_w), &r = value(wr), &l = value(logits), &b = value(bias), &i = value(ids);
+  no_tangents({&x, &n, &r, &l, &w1, &w3, &w2, &b});
   Layer o;
   o.k = k, o.eps = eps, o.add_residual = add_residual, o.fused_router = fused_router, o.accumulate = accumulate;
   o.s1 = s1, o.s3 = s3, o.s2 = s2;
@@ -683,6 +692,7 @@ std::tuple<Tensor, OptTensor> layer_f32(const Tensor& x, const OptTensor& logits
                                         const Tensor& w3, const Tensor& w2, const OptTensor& bias, int64_t k,
                                         bool want_routing) {
   const Tensor &l = value(logits), &b = value(bias), &i = value(ids);
+  no_tangents({&x, &l, &w1, &w3, &w2, &b});
   Layer o;
   o.k = k;
   Tensor routing;
