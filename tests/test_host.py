@@ -315,3 +315,24 @@ def test_precision_rule_of_the_module_cpu():
     assert not mb._runs_in_fp32(x) and not mb._runs_in_fp32(x.to(torch.bfloat16))
     m.experts_up_weights.data = m.experts_up_weights.data.to(torch.bfloat16)   # mixed parameters
     assert not m._runs_in_fp32(x)
+
+
+def test_layer_backward_checks_the_alignment_of_every_result():
+    """moe_layer_backward with each result in turn (and the two operands of the router) 4 bytes past a 16-byte
+    boundary, at shapes that go to either weight-gradient kernel: refused before anything is launched.  Host
+    pointers: CPU only."""
+    if torch.cuda.is_available():
+        pytest.skip("hands host pointers to the entry point: CPU-only check")
+    pkg = load_pkg()
+    L, pack = pkg.lib.load(), pkg.ops._BACKWARD_ARGS.pack
+    host = ctypes.create_string_buffer(1 << 16)
+    base = (ctypes.addressof(host) + 255) & ~255
+    names = ("T H E I k dout dout_dtype gates ids offs pos_to_row row_to_pos xp gu act w1 w3 w2 dw0 dw1 dw2 dt0 dt1 dt2 "
+             "acc0 acc1 acc2 dlogits dlogits_dtype dgates wr xn dwr dwr_dtype dx dx_dtype dxp scratch scratch_bytes").split()
+    for E in (4, 512):  # one launch for all weight gradients; the tiled kernel (more tiles than compute units)
+        args = dict.fromkeys(names, base)
+        args.update(T=8, H=64, E=E, I=256, k=2, scratch_bytes=1 << 40, dlogits=0, dgates=0)
+        args.update({n: 0 for n in names if "dtype" in n or n[:2] == "dt" or n[:3] == "acc"})
+        for n in ("dw0", "dw1", "dw2", "dwr", "dx", "dxp", "wr", "xn"):
+            off = dict(args, **{n: base + 4})
+            assert L.cdll.moe_layer_backward(pack(*(off[m] for m in names)), None) == -6, (E, n)

@@ -340,6 +340,9 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     return MOE_ERR_DTYPE;
   for (int i = 0; i < 3; ++i)
     if (!dtype_ok(a->dw_dtype[i])) return MOE_ERR_DTYPE;
+  // (a result that is not asked for is NULL; here, so that it does not depend on which kernel the shapes pick)
+  for (const void* p : {a->dw[0], a->dw[1], a->dw[2], a->dwr, a->dx, (void*)a->dxp, (void*)a->wr, (void*)a->xn})
+    if (!aligned16(p)) return MOE_ERR_ALIGN;
   MOE_CHECK_PTR(a->offs);
   MOE_CHECK_PTR(a->scratch);
   const bool router = a->wr != nullptr;                               // the router product is part of the layer
