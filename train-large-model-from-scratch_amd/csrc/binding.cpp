@@ -7,10 +7,10 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/extension.h>
 
-#include <stdexcept>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -37,9 +37,13 @@ typedef std::optional<Tensor> OptTensor;
 
 namespace {
 
-// Raised as lib.MoELibError.
-struct LibError : std::runtime_error {
-  using std::runtime_error::runtime_error;
+PyObject* error_type = nullptr;  // lib.MoELibError
+
+// Raised as lib.MoELibError.  (torch's own kind of exception with a Python type: the autograd engine hands those
+// of a backward pass on as they are, any other becomes a plain RuntimeError.)
+struct LibError : torch::PyTorchError {
+  using torch::PyTorchError::PyTorchError;
+  PyObject* python_type() override { return error_type ? error_type : PyExc_RuntimeError; }
 };
 
 void check(int rc, const char* name) {
@@ -64,7 +68,7 @@ void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t
 int64_t dt(at::ScalarType t) {
   if (t == at::kBFloat16) return MOE_DT_BF16;
   if (t == at::kFloat) return MOE_DT_F32;
-  throw py::type_error("unsupported dtype: the MoE kernels take bf16 or fp32");
+  throw torch::TypeError("unsupported dtype: the MoE kernels take bf16 or fp32");
 }
 int64_t dt(const Tensor& t) { return dt(t.scalar_type()); }
 
@@ -712,13 +716,12 @@ std::tuple<Tensor, OptTensor> layer_f32(const Tensor& x, const OptTensor& logits
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  static py::object error_type;
-  m.def("set_error_type", [](py::object t) { error_type = std::move(t); });
+  m.def("set_error_type", [](py::object t) { error_type = t.release().ptr(); });  // (as long as the process)
   py::register_exception_translator([](std::exception_ptr p) {
     try {
       if (p) std::rethrow_exception(p);
-    } catch (const LibError& e) {
-      PyErr_SetString(error_type ? error_type.ptr() : PyExc_RuntimeError, e.what());
+    } catch (torch::PyTorchError& e) {
+      PyErr_SetString(e.python_type(), e.what());
     }
   });
   m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
