@@ -44,3 +44,23 @@ def test_forward_of_few_tokens_matches_the_oracle(pkg, lib, T, E, k, H, I, x_dt)
     f = O.moe_forward(x, wr, w1, w3, w2, k, logits=sel)
     fe = O.moe_forward(x, wr, w1, w3, w2, k, logits=sel, emulate_bf16=True)
     check("out", out, f["out"], fe["out"])
+
+
+@pytest.mark.parametrize("H", [2048, 4104])  # columns in workgroups of 8 and of 16
+@pytest.mark.parametrize("k,I", [(1, 264), (2, 72), (3, 1032), (8, 72)])
+def test_one_infinite_activation_makes_infinite_outputs(pkg, lib, H, k, I):
+    """One token, an activation that overflows: every output is infinite, none a NaN, wherever in its expert's
+    contraction that activation lies (in workgroups' shares other than its own it must not be there at all)."""
+    print("infinite activation", H, k, I, flush=True)
+    E = 2 * k
+    w1, w3, w2 = torch.zeros(E, I, H), torch.zeros(E, I, H), torch.full((E, H, I), 0.5)
+    x = torch.zeros(1, H)
+    x[0, 0] = 1.0
+    logits = torch.arange(E, 0, -1).float()[None].cuda()  # experts 0 .. k-1
+    bf = torch.bfloat16
+    for i in sorted({0, 31, I // 2, I - 1}):
+        w1[:, :, 0] = w3[:, :, 0] = 1e-3
+        w1[k - 1, i, 0] = w3[k - 1, i, 0] = 1e30
+        with torch.no_grad():
+            out = pkg.moe_ffn(x.cuda().to(bf), logits, *(w.cuda().to(bf) for w in (w1, w3, w2)), k)
+        assert torch.isposinf(out).all(), (i, out.isnan().sum().item(), out.isfinite().sum().item())

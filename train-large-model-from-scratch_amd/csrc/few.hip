@@ -342,7 +342,10 @@ __global__ __launch_bounds__(DOWN_WAVES* MOE_WAVE) void down_one_kernel(const ui
     const int s_lo = sp * PARTS * per;                               // of the first part
     const auto end_of = [&](int p) { return s_lo + (p + 1) * per < steps ? s_lo + (p + 1) * per : steps; };
     const __amdgpu_buffer_rsrc_t rw = rsrc(w2 + ((size_t)e * H + h0) * I, (long long)(H - h0) * I * 2);
-    const __amdgpu_buffer_rsrc_t ra = rsrc(act + (size_t)j * I, (long long)I * 2);
+    // (an undivided share's activations end where the share does: past it they must not count, not even times a weight
+    // of zero, since they may be infinite.  The resource's end costs nothing; a test a lane took 1-2 % of the call.)
+    const int a_end = PARTS == 1 && end_of(0) * 32 < I ? end_of(0) * 32 : I;
+    const __amdgpu_buffer_rsrc_t ra = rsrc(act + (size_t)j * I, (long long)a_end * 2);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < per; s += KC) {
       const int first = s_lo + part * per + s, end = end_of(part);
