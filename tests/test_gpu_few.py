@@ -46,6 +46,33 @@ def test_forward_of_few_tokens_matches_the_oracle(pkg, lib, T, E, k, H, I, x_dt)
     check("out", out, f["out"], fe["out"])
 
 
+@pytest.mark.parametrize("E,H,I,x_dt,few", [  # 64 tokens, every expert asked for by each
+    (9, 1032, 792, torch.bfloat16, True), (9, 1032, 808, torch.bfloat16, False),  # 2.47 and 2.52 GB past 8 rows each
+    (9, 1032, 400, torch.float32, True), (9, 1032, 408, torch.float32, False),    # ... of fp32 rows
+    (8, 1368, 1352, torch.bfloat16, True), (8, 1368, 1360, torch.bfloat16, False),  # 4.97 and 5.0009, at most 8 experts
+])
+def test_many_rows_an_expert_take_the_tiled_kernels(pkg, lib, E, H, I, x_dt, few):
+    print("few or tiled", E, H, I, x_dt, flush=True)
+    g = torch.Generator().manual_seed(H + I)
+    r = lambda *s, std=0.05: (torch.randn(*s, generator=g) * std).to(torch.bfloat16)
+    x, wr, w1, w3, w2, lg = r(64, H, std=1.0), r(E, H), r(E, I, H), r(E, I, H), r(E, H, I), r(64, E, std=1.0)
+    names = []
+
+    class Obs:
+        before = names.append
+        after = staticmethod(lambda name: None)
+
+    lib.observer = Obs()
+    try:
+        with torch.no_grad():
+            out = pkg.moe_ffn(x.cuda().to(x_dt), lg.cuda(), w1.cuda(), w3.cuda(), w2.cuda(), E)
+    finally:
+        lib.observer = None
+    assert ("moe_gateup_few" in names, "moe_gemm_gateup_swiglu_fwd" in names) == (few, not few), names
+    f = O.moe_forward(x, wr, w1, w3, w2, E, logits=lg)
+    check("out", out, f["out"], O.moe_forward(x, wr, w1, w3, w2, E, logits=lg, emulate_bf16=True)["out"])
+
+
 @pytest.mark.parametrize("H", [2048, 4104])  # columns in workgroups of 8 and of 16
 @pytest.mark.parametrize("k,I", [(1, 264), (2, 72), (3, 1032), (8, 72)])
 def test_one_infinite_activation_makes_infinite_outputs(pkg, lib, H, k, I):

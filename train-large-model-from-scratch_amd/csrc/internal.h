@@ -61,7 +61,7 @@ int moe_router_few(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, 
                    hipStream_t s);
 // The experts on at most 64 tokens, rows in routed order: act [T*k, I] from x and the expert ids, y [T*k, H]
 // from act, and for one token the combined output from act.
-bool moe_few_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k);
+bool moe_few_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int x_dtype);
 int moe_gateup_few(const void* x, int x_dtype, const int32_t* ids, const uint16_t* w1, const uint16_t* w3, int64_t T,
                    int64_t H, int64_t E, int64_t I, int64_t k, uint16_t* act, hipStream_t s);
 // The same for one token, its selection with it: ids and gates [k] are results.

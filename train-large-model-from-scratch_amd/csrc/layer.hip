@@ -121,7 +121,7 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
     return 0;
   }
   MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream));
-  if (moe_few_ok(T, H, E, I, k)) {  // rows stay in routed order: no dispatch, no gather
+  if (moe_few_ok(T, H, E, I, k, x_dtype)) {  // rows stay in routed order: no dispatch, no gather
     MOE_STEP("moe_gateup_few", moe_gateup_few(x, x_dtype, ids, w1, w3, T, H, E, I, k, act, st));
     if (moe_down_one_ok(T, k)) {
       MOE_STEP("moe_down_one", moe_down_one(act, ids, gates, w2, H, E, I, k, out, out_dtype, st));
