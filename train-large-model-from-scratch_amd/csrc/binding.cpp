@@ -341,9 +341,14 @@ struct WeightGradients {
   }
 };
 
-Tensor router_wgrad(const Tensor& dlogits, const Tensor& xn, at::ScalarType type) {
-  const int64_t T = xn.size(0), H = xn.size(1), E = dlogits.size(1);
-  if (T == 0 || E % 8 != 0 || H % 8 != 0) return at::mm(dlogits.t(), xn).to(type);
+// dWr = dlogits^T x for dlogits [T,E], x [T,H].
+Tensor router_wgrad(const Tensor& dlogits_, const Tensor& xn_, at::ScalarType type) {
+  const int64_t T = xn_.size(0), H = xn_.size(1), E = dlogits_.size(1);
+  if (T == 0 || E % 8 != 0 || H % 8 != 0 || !xn_.is_cuda() || xn_.scalar_type() != at::kBFloat16 ||
+      dlogits_.scalar_type() != at::kBFloat16)
+    return at::mm(dlogits_.t(), xn_).to(type);
+  const c10::DeviceGuard guard(xn_.device());
+  const Tensor dlogits = dense(dlogits_), xn = dense(xn_);
   const bool direct = type == at::kFloat || type == at::kBFloat16;
   Tensor dw = empty({E, H}, direct ? type : at::kFloat, xn);
   const int64_t bytes = moe_router_wgrad_workspace_bytes(T, H, E);
@@ -726,5 +731,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   });
   m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
   m.def("router_logits", &router_logits, py::call_guard<py::gil_scoped_release>());
+  m.def("router_wgrad",
+        [](const Tensor& dlogits, const Tensor& xn, py::object type) {
+          const at::ScalarType t = torch::python::detail::py_object_to_dtype(type);
+          const py::gil_scoped_release off;
+          return router_wgrad(dlogits, xn, t);
+        });
   m.def("layer_f32", &layer_f32, py::call_guard<py::gil_scoped_release>());
 }

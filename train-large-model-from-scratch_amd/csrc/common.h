@@ -121,6 +121,18 @@ __device__ __forceinline__ Row8 load8_nt(const uint16_t* p) {
 }
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (MOE_WAVE - 1); }
+// A value known to be the same in every lane, in a scalar register.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// Sum over the wave's lanes up to and including the own (by a whole wave).
+__device__ __forceinline__ int wave_inclusive(int v) {
+  const int lane = lane_id();
+#pragma unroll
+  for (int o = 1; o < MOE_WAVE; o <<= 1) {
+    const int u = __shfl_up(v, o, MOE_WAVE);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
 
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -16,8 +16,6 @@ namespace {
 constexpr int NT = 256;                    // threads
 constexpr unsigned OUTSIDE = 0xfffffff0u;  // a byte offset that no window reaches: reads as zero
 
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
 // Operand chunks of 16 bytes are read through buffer resources, whose hardware bounds check makes an out-of-range
 // chunk a zero without a branch: chunks past the tile's rows or past the end of the contraction get the offset OUTSIDE.
 // A window is moved along k by its base, a scalar addition.
@@ -226,15 +224,6 @@ __device__ __forceinline__ int expert_rows(const RowsArgs& p, int e, int& first)
   const int b = p.offs[e], n = p.offs[e + 1] - b;
   first = b;
   return n <= 0 || b < 0 || n > p.R - b ? 0 : n;  // (empty, or offsets that no dispatch would produce)
-}
-__device__ __forceinline__ int wave_inclusive(int v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < MOE_WAVE; o <<= 1) {
-    const int u = __shfl_up(v, o, MOE_WAVE);
-    if (lane >= o) v += u;
-  }
-  return v;
 }
 
 

@@ -40,15 +40,6 @@ struct MultiArgs {
 struct Segment {
   int e, row0, row_end, parts, slot;  // slot: of its partial sums, where the expert has several parts
 };
-__device__ __forceinline__ int wave_scan(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < MOE_WAVE; o <<= 1) {
-    const int u = __shfl_up(v, o, MOE_WAVE);
-    if (lane >= o) v += u;
-  }
-  return v;
-}
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ int expert_rows(const int32_t* offs, int e, int E) {
   const int n = e < E ? offs[e + 1] - offs[e] : 0;
   return n > 0 ? n : 0;
@@ -61,7 +52,7 @@ __device__ __forceinline__ int slots_before(const int32_t* offs, int E, int L, i
   int slots = 0;
   for (int b = 0; b < e; b += MOE_WAVE) {
     const int p = b + lane < e ? parts_of(expert_rows(offs, b + lane, E), L) : 1;
-    slots += uniform(__shfl(wave_scan(p > 1 ? p : 0, lane), MOE_WAVE - 1, MOE_WAVE));
+    slots += uniform(__shfl(wave_inclusive(p > 1 ? p : 0), MOE_WAVE - 1, MOE_WAVE));
   }
   return slots;
 }
@@ -73,7 +64,7 @@ __device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, 
       const int n = expert_rows(offs, b + lane, E);
       const bool mine = b + lane < E && (2 * n > L) == (pass == 0);
       const int p = mine ? parts_of(n, L) : 0;
-      const int incl = wave_scan(p, lane);
+      const int incl = wave_inclusive(p);
       const int total = uniform(__shfl(incl, MOE_WAVE - 1, MOE_WAVE));
       if (seg < carry + total) {
         const int f = __builtin_ctzll(__ballot(carry + incl > seg));
@@ -248,7 +239,7 @@ __global__ __launch_bounds__(256) void wgrad_multi_sum_kernel(const MultiArgs p)
       const int n = expert_rows(p.offs, b + lane, p.E);
       const int c = b + lane < p.E && n > p.L ? parts_of(n, p.L) : 0;
       const unsigned long long m = __ballot(c > 0);
-      const int incl = wave_scan(c, lane);
+      const int incl = wave_inclusive(c);
       const int want = (int)blockIdx.y - carry;
       if (want < __popcll(m)) {
         const bool me = c > 0 && __popcll(m & ((1ull << lane) - 1)) == want;

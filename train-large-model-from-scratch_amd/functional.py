@@ -38,7 +38,6 @@ from __future__ import annotations
 import torch
 
 from . import lib as _lib, ops
-from .ops import dense as _dense
 
 
 def _first_order_only():
@@ -66,21 +65,8 @@ class _RouterLinear(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dx = dlogits @ w
         if ctx.needs_input_grad[1]:
-            dw = _router_wgrad(dlogits, x, w.dtype)
+            dw = _lib.native().router_wgrad(dlogits, x, w.dtype)
         return dx, dw
-
-
-def _router_wgrad(dlogits, x, w_dtype):
-    """dWr = dlogits^T x for dlogits [T,E], x [T,H]."""
-    T, H = x.shape
-    E = dlogits.shape[1]
-    fast = (x.is_cuda and x.dtype == torch.bfloat16 and dlogits.dtype == torch.bfloat16
-            and E % 8 == 0 and H % 8 == 0 and T > 0)
-    if not fast:
-        return (dlogits.t() @ x).to(w_dtype)
-    if w_dtype not in (torch.bfloat16, torch.float32):
-        return ops.router_wgrad(_dense(dlogits), _dense(x), torch.float32).to(w_dtype)
-    return ops.router_wgrad(_dense(dlogits), _dense(x), w_dtype)
 
 
 def router_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

@@ -301,15 +301,6 @@ def combine_fwd(y, gates, row_to_pos, T: int, k: int, dtype: torch.dtype):
     return out
 
 
-def combine_fwd_residual(y, gates, row_to_pos, residual: torch.Tensor, k: int):
-    """residual [T,H] + the combined expert rows; same dtype as `residual`."""
-    T, H = residual.shape
-    out = torch.empty_like(residual)
-    _lib.load().call("moe_combine_fwd_residual", _p(y), _p(gates), _p(row_to_pos), _p(residual), T, H, k,
-                     _p(out), _dt(out), _stream())
-    return out
-
-
 def rmsnorm_fwd(x: torch.Tensor, weight: torch.Tensor, eps: float):
     """x [T,H] (bf16/fp32), weight fp32 [H] -> xn bf16 [T,H], rstd fp32 [T]."""
     T, H = x.shape
@@ -378,17 +369,6 @@ def cast_bf16(w: torch.Tensor) -> torch.Tensor:
     out = torch.empty(w.shape, dtype=torch.bfloat16, device=w.device)
     _lib.load().call("moe_cast_f32_bf16", _p(w), _p(out), w.numel(), _stream())
     return out
-
-
-def router_wgrad(dlogits: torch.Tensor, x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    """dlogits^T x for bf16 dlogits [T,E], x [T,H] (E and H multiples of 8) -> [E,H]."""
-    T, H = x.shape
-    E = dlogits.shape[1]
-    L = _lib.load()
-    dw = torch.empty((E, H), dtype=dtype, device=x.device)
-    ws = torch.empty(max(L.cdll.moe_router_wgrad_workspace_bytes(T, H, E), 16), dtype=torch.uint8, device=x.device)
-    L.call("moe_router_wgrad", _p(dlogits), _p(x), T, H, E, _p(dw), _dt(dw), _p(ws), ws.numel(), _stream())
-    return dw
 
 
 # ---- one call per direction of a training step ------------------------------------------------------

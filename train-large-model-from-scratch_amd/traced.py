@@ -26,7 +26,6 @@ import torch
 from torch import Tensor
 
 from . import lib as _lib, ops
-from .functional import _router_wgrad
 
 _BF16 = torch.bfloat16
 
@@ -200,7 +199,7 @@ def routed_bwd(dout: Tensor, dlogits_ext: Tensor | None, xn: Tensor, wrb: Tensor
     dgates, dxp = torch.empty_like(gates), torch.empty_like(xp)
     ops.layer_backward(*saved, dgates=dgates, dxp=dxp)
     dlogits = ops.router_topk_bwd(gates, dgates, ids, T, E, k, _BF16) + dlogits_ext.to(_BF16)
-    dwr = _router_wgrad(dlogits, xn, f32 if wr_is_f32 else _BF16)
+    dwr = _lib.native().router_wgrad(dlogits, xn, f32 if wr_is_f32 else _BF16)
     with torch.autocast("cuda", enabled=False):
         d2 = dlogits @ wrb
     dx = ops.permute_bwd(dxp, row_to_pos, T, k, xdt, addend=d2)
