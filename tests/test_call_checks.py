@@ -98,3 +98,26 @@ def test_forward_mode_is_refused(entry, dual, grad, return_routing):
             fn(*args, return_routing=return_routing)
         with torch.no_grad(), pytest.raises(NotImplementedError):
             fn(*args, return_routing=return_routing)
+
+
+@pytest.mark.parametrize("dtype,entry", [(BF16, "moe_ffn"), (F32, "moe_ffn_f32")])
+@pytest.mark.parametrize("logits,bias,error,match", [
+    (lambda d: _gpu(T - 1, E, dtype=d), lambda: None, RuntimeError, "logits"),
+    (lambda d: _gpu(1, T, E, dtype=d), lambda: None, RuntimeError, "logits|shapes"),
+    (lambda d: _gpu(T, E - 1, dtype=d), lambda: None, RuntimeError, "logits|shapes"),
+    (lambda d: _gpu(T, E, dtype=d), lambda: _gpu(E - 1, dtype=F32), RuntimeError, "bias"),
+    (lambda d: _gpu(T, E, dtype=d), lambda: _gpu(E), TypeError, "bias"),
+])
+def test_logits_and_bias_belong_to_x(dtype, entry, logits, bias, error, match):
+    pkg = load_pkg()
+    with FakeTensorMode():
+        with pytest.raises(error, match=match):
+            getattr(pkg, entry)(_gpu(T, H, dtype=dtype), logits(dtype), *_weights(dtype), K, bias=bias())
+
+
+def test_fp32_rows_are_a_matrix():
+    pkg = load_pkg()
+    with FakeTensorMode():
+        w = [_gpu(E, I, H, dtype=F32), _gpu(E, I, H, dtype=F32), _gpu(E, H, I, dtype=F32)]
+        with pytest.raises(RuntimeError, match="x .tokens, hidden."):
+            pkg.moe_ffn_f32(_gpu(T, H, 2, dtype=F32), _gpu(T, E, dtype=F32), *w, K)

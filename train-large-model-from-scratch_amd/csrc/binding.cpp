@@ -158,6 +158,15 @@ void check_copy(const OptTensor& s, const Tensor& w, const Tensor& x) {
   TORCH_CHECK(s->is_contiguous(), "the MoE kernels need contiguous tensors: a bf16 copy of the weights is strided");
 }
 
+// Logits [tokens, E] and the fp32 constant per expert that is added to them.
+void check_logits(const Tensor& logits, const Tensor& bias, const Tensor& x, int64_t E) {
+  TORCH_CHECK(!logits.defined() || (logits.dim() == 2 && logits.size(0) == x.size(0) && logits.size(1) == E),
+              "the logits have shape ", logits.sizes(), ", x ", x.sizes(), " and there are ", E, " experts");
+  if (!bias.defined()) return;
+  TORCH_CHECK_TYPE(bias.scalar_type() == at::kFloat, "the bias must be fp32, got ", bias.scalar_type());
+  TORCH_CHECK(bias.numel() == E, "the bias has ", bias.numel(), " elements, there are ", E, " experts");
+}
+
 const Tensor& value(const OptTensor& t) {
   static const Tensor none;
   return t ? *t : none;
@@ -209,6 +218,7 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
     TORCH_CHECK(norm_w.numel() == H, "the norm's weight has ", norm_w.numel(), " elements, x is ", H, " wide");
     TORCH_CHECK(norm_w.device() == x_.device(), "the norm's weight is on ", norm_w.device(), ", x on ", x_.device());
   }
+  check_logits(logits_, bias, x_, E);
   check_copy(o.s1, w1, x_), check_copy(o.s3, w3, x_), check_copy(o.s2, w2, x_);
   (void)dt(x_);
   const at::ScalarType x_type = x_.scalar_type();
@@ -582,12 +592,15 @@ struct OutputsF32 {
 OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, const Tensor& w1, const Tensor& w3,
                        const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
   OutputsF32 f;
-  const Tensor x = dense(x_);
-  const c10::DeviceGuard guard(x.device());
-  const int64_t T = x.size(0), H = x.size(1), E = w1.size(0), I = w1.size(1), k = o.k, R = T * k;
+  need_gpu(x_);
+  TORCH_CHECK(x_.dim() == 2 && w1.dim() == 3, "the layer takes x [tokens, hidden] and weights [experts, ., .]");
+  const int64_t T = x_.size(0), H = x_.size(1), E = w1.size(0), I = w1.size(1), k = o.k, R = T * k;
   TORCH_CHECK(w3.size(0) == E && w2.size(0) == E && w1.size(2) == H && w3.size(2) == H && w3.size(1) == I &&
-                  w2.size(1) == H && w2.size(2) == I && (!logits_.defined() || logits_.size(1) == E),
+                  w2.size(1) == H && w2.size(2) == I,
               "the weights' shapes do not belong together");
+  check_logits(logits_, bias, x_, E);
+  const c10::DeviceGuard guard(x_.device());
+  const Tensor x = dense(x_);
   f.w[0] = dense(w1), f.w[1] = dense(w3), f.w[2] = dense(w2);
   void* s = stream_of(x);
   const Routing r(R, E);
