@@ -350,13 +350,14 @@ __global__ __launch_bounds__(256) void permute_fwd_scatter_kernel(const XT* __re
   }
 }
 
-// out[t,:] = sum_j gates[t*k+j] * y[row_to_pos[t*k+j],:]  (+ addend[t,:]); fp32, slot order.  row_to_pos NULL:
-// the rows of y are in routed order.
+// out[t,:] = sum_j gates[t*k+j] * y[row_to_pos[t*k+j],:]  (+ addend[t,:]); fp32, slot order.  IN_ORDER: the rows of
+// y are in routed order, there is no map.  (A question at run time parts the loads of the positions from each
+// other: 1531 tokens, k = 8, 2048 wide, 11.6 -> 12.6 us.)
 // ROUTER: + bf16(sum_j dsel[t*k+j] * wr[ids[t*k+j],:]), the router path's input gradient: a row of
 // dlogits has k nonzero entries, so that product is k rows of the router weight per token, which sit in
 // every XCD's L2 (at most 512 rows) -- instead of a library product over all E columns, its result in
 // memory and another read of it here.
-template <typename OT, typename AT, bool ROUTER>
+template <typename OT, typename AT, bool ROUTER, bool IN_ORDER>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __restrict__ y,
                                                          const float* __restrict__ gates,
                                                          const int32_t* __restrict__ row_to_pos,
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
         Row8 v[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          pos[q] = row_to_pos ? row_to_pos[(size_t)t * k + j + q] : t * k + j + q;
+          pos[q] = IN_ORDER ? t * k + j + q : row_to_pos[(size_t)t * k + j + q];
           gt[q] = gates ? gates[(size_t)t * k + j + q] : 1.f;
         }
 #pragma unroll
@@ -397,7 +398,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
         Row8 v[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          pos[q] = row_to_pos ? row_to_pos[(size_t)t * k + j + q] : t * k + j + q;
+          pos[q] = IN_ORDER ? t * k + j + q : row_to_pos[(size_t)t * k + j + q];
           gt[q] = gates ? gates[(size_t)t * k + j + q] : 1.f;
         }
 #pragma unroll
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
           for (int i = 0; i < 8; ++i) acc.v[i] += gt[q] * v[q].v[i];
       }
       for (; j < k; ++j) {
-        const int pos = row_to_pos ? row_to_pos[(size_t)t * k + j] : t * k + j;
+        const int pos = IN_ORDER ? t * k + j : row_to_pos[(size_t)t * k + j];
         const float gt = gates ? gates[(size_t)t * k + j] : 1.f;
         const Row8 v = load8_nt(y + (size_t)pos * H + col);
 #pragma unroll
@@ -753,13 +754,13 @@ static int combine_like(const uint16_t* y, const float* gates, const int32_t* ro
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
   if (out_dtype == MOE_DT_BF16 && addend_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false>), grid, block, 0, s, y, gates, row_to_pos,
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false, false>), grid, block, 0, s, y, gates, row_to_pos,
                        (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (uint16_t*)out, nullptr, nullptr, nullptr);
   else if (out_dtype == MOE_DT_F32 && addend_dtype == MOE_DT_F32)
-    hipLaunchKernelGGL((combine_fwd_kernel<float, float, false>), grid, block, 0, s, y, gates, row_to_pos,
+    hipLaunchKernelGGL((combine_fwd_kernel<float, float, false, false>), grid, block, 0, s, y, gates, row_to_pos,
                        (const float*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
   else if (out_dtype == MOE_DT_F32 && addend_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false>), grid, block, 0, s, y, gates, row_to_pos,
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false, false>), grid, block, 0, s, y, gates, row_to_pos,
                        (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
   else
     return MOE_ERR_DTYPE;
@@ -1049,10 +1050,10 @@ int moe_combine_in_order(const uint16_t* y, const float* gates, int64_t T, int64
   const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
   const uint16_t* none = nullptr;
   if (out_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false, true>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
                        (int)(H / 8), (int)k, (uint16_t*)out, nullptr, nullptr, nullptr);
   else
-    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false, true>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
                        (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
   return moe_launch_status();
 }
@@ -1062,10 +1063,10 @@ int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const
                            hipStream_t s) {
   const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
   if (dx_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, true>), grid, block, 0, s, dxp, nullptr, row_to_pos,
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, true, false>), grid, block, 0, s, dxp, nullptr, row_to_pos,
                        nullptr, (int)T, (int)(H / 8), (int)k, (uint16_t*)dx, dsel, ids, wr);
   else
-    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, true>), grid, block, 0, s, dxp, nullptr, row_to_pos,
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, true, false>), grid, block, 0, s, dxp, nullptr, row_to_pos,
                        nullptr, (int)T, (int)(H / 8), (int)k, (float*)dx, dsel, ids, wr);
   return moe_launch_status();
 }
