@@ -246,7 +246,9 @@ int moe_segment_offsets(const int32_t* offs, int64_t E, int64_t S, int32_t* seg,
  * of the rows).  moe_gemm_wgrad over seg with S_max "experts" and fp32 output gives the partial
  * sums; moe_wgrad_reduce_segments adds each expert's partials in ascending order (reproducible)
  * into dw [E,M,N] of dw_dtype: dw[e] (+)= sum_s part[s], exact zeros for experts without rows
- * (left untouched when accumulate != 0).  S_max <= 1024.  (No counterpart in the reference.) */
+ * (left untouched when accumulate != 0).  S_max <= 1024.  (No counterpart in the reference.  The layer's
+ * own calls cut experts inside the kernel that makes all weight gradients: these three are for callers
+ * that put the pass together from the separate entry points.) */
 int64_t moe_segments_by_length_max(int64_t R, int64_t E, int64_t L);
 int moe_segment_offsets_by_length(const int32_t* offs, int64_t E, int64_t L, int64_t S_max,
                                   int32_t* seg, int32_t* seg_start, void* stream);
@@ -323,8 +325,10 @@ int moe_cast_f32_bf16(const float* src, uint16_t* dst, int64_t n, void* stream);
  * under no_grad): routing, dispatch, row gather, both grouped GEMMs and the combine enqueued
  * back to back, every intermediate in `workspace` (moe_ffn_forward_workspace_bytes, 256-byte
  * aligned pieces; contents unspecified afterwards).  x [T,H] and logits [T,E] bf16 or f32, bias
- * f32 [E] or NULL, weights bf16 as stored, out [T,H] of out_dtype.  The same kernels in the same
- * order as the separate entry points: the same bits. */
+ * f32 [E] or NULL, weights bf16 as stored, out [T,H] of out_dtype.  Above 64 tokens the same kernels
+ * in the same order as the separate entry points: the same bits.  At most 64 tokens (where an expert has
+ * few rows) run on kernels of their own, whose sums are formed in another order: same operands, same
+ * roundings, other last bits. */
 int64_t moe_ffn_forward_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k);
 int moe_ffn_forward(const void* x, int x_dtype, const void* logits, int logits_dtype,
                     const float* bias, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
@@ -430,7 +434,8 @@ int moe_f32_combine_bwd(const float* dy, const float* y, const float* gates, con
 int moe_f32_permute_bwd(const float* dxp, const int32_t* row_to_pos, int64_t T, int64_t H, int64_t k,
                         float* dx, void* stream);
 /* mlp.py:156: act = silu(g) * u over n elements (n a multiple of 4), and its backward
- * dg = dact * u * silu'(g), du = dact * silu(g). */
+ * dg = dact * u * silu'(g), du = dact * silu(g).  (These two and moe_f32_gemm_wgrad are the separate
+ * steps; the layer's own calls run the fused products further down.) */
 int moe_f32_swiglu_fwd(const float* g, const float* u, int64_t n, float* act, void* stream);
 int moe_f32_swiglu_bwd(const float* dact, const float* g, const float* u, int64_t n, float* dg,
                        float* du, void* stream);
@@ -444,8 +449,8 @@ int moe_f32_gemm_rows(const float* a, const float* b, const int32_t* offs, int64
  * Experts without rows get exact zeros (are left untouched when accumulating). */
 int moe_f32_gemm_wgrad(const float* a, const float* b, const int32_t* offs, int64_t E, int64_t R,
                        int64_t M, int64_t N, float* dw, int accumulate, void* stream);
-/* The same products with what follows them fused in: g = xp W1^T, u = xp W3^T, act = silu(g) u; dg, du from dact = dyp W2 and the g and u of the forward; dxp = dg W1 + du W3;
- * dw1 = dg^T xp, dw3 = du^T xp, dw2 = dyp^T act.  xp, dyp, dxp [R,H], g, u,
+/* The same products with what follows them fused in: g = xp W1^T, u = xp W3^T, act = silu(g) u;
+ * dg, du from dact = dyp W2 and the g and u of the forward; dxp = dg W1 + du W3; dw1 = dg^T xp, dw3 = du^T xp, dw2 = dyp^T act.  xp, dyp, dxp [R,H], g, u,
  * act, dg, du [R,I], w1, w3, dw1, dw3 [E,I,H], w2, dw2 [E,H,I]. */
 int moe_f32_gemm_gateup_swiglu(const float* xp, const float* w1, const float* w3, const int32_t* offs,
                                int64_t E, int64_t R, int64_t H, int64_t I, float* g, float* u, float* act,

@@ -1,11 +1,12 @@
-// Few tokens: the router with its selection, and the whole layer body for at most 64 tokens.
+// Few tokens: the router with its selection, and the whole layer body for at most 64 tokens (moe_few_ok
+// below has the line).
 //
 // Generation asks for the experts of one token, or of one token from each sequence of a batch.  What
 // such a call cannot do without is one pass over the weights of the experts it asks for (one token of
 // the 64-expert layer: 100 MB; 48 tokens: 800 MB, nearly all of them), and next to that a kernel's
-// start and end are what costs.  So there are three kernels, none of which waits for another launch to
-// sort rows: every workgroup finds the rows of its expert in the (at most 512) expert ids itself, rows
-// stay in routed order, and the combine is part of the down kernel.  The products run on
+// start and end are what costs.  So no kernel waits for another launch to sort rows: every workgroup finds
+// the rows of its expert in the expert ids itself, rows stay in routed order, and for one token the selection
+// is part of the gate/up kernel and the combine part of the down kernel.  The products run on
 // v_mfma_f32_16x16x32_bf16, whose 16 rows are the tokens of an expert: weights go from memory straight to
 // the operand registers, every byte once, with a wave's whole share of the contraction requested before
 // the first product where it fits.

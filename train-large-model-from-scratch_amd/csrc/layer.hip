@@ -5,8 +5,10 @@
 // caller's stream, with every intermediate in a workspace the caller provides.  For callers that
 // only want the output (inference, evaluation, a forward under no_grad): one crossing of the FFI
 // boundary and two buffers instead of six crossings and a dozen.  Nothing here touches the GPU
-// itself: the kernels are the ones the separate entry points launch, in the same order, so the
-// output holds the same bits.
+// itself.  Above 64 tokens the kernels are the ones the separate entry points launch, in the same
+// order, so the output holds the same bits; at most 64 tokens go to kernels of their own
+// (moe_few_ok), which add the same products in another order: a token's output then depends on
+// whether it came in a batch of 64 or of 65, by what another order of fp32 sums makes of it.
 //
 // Training: moe_layer_forward / moe_layer_backward enqueue one direction each (two dozen kernels
 // between them).  What they replace is host work: a step of 512 tokens of a narrow layer has 0.1 ms of

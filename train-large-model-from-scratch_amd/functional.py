@@ -72,8 +72,10 @@ class _RouterLinear(torch.autograd.Function):
 def router_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """Router logits `x @ weight^T` (mlp.py:100) for x [..., H], weight [E, H].  Forward and
     input gradient are the library products `nn.Linear` would run, under the same autocast
-    rule (bf16 operands and result inside a bf16 autocast region); the weight gradient is
-    computed here (see the module docstring)."""
+    rule (bf16 operands and result inside a bf16 autocast region), but for a bf16 forward of at
+    most 64 tokens and 128 experts: that is a kernel here, whose own summation order can move a
+    bf16 logit by one unit in the last place.  The weight gradient is computed here (see the
+    module docstring)."""
     lead = x.shape[:-1]
     out = _RouterLinear.apply(x.reshape(-1, x.shape[-1]), weight)
     return out.reshape(*lead, weight.shape[0])
@@ -140,10 +142,10 @@ def prenorm_moe(x: torch.Tensor, norm_weight: torch.Tensor, router_weight: torch
     """(x + MoE(RMSNorm(x)), router logits) for x [T,H]: model/gpt.py:32-33 with
     model/modules/norm.py:14-19 and model/modules/mlp.py:95-169 in one differentiable call.
     Router logits are bf16 (what the reference produces under its bf16 autocast); the output
-    has the dtype of x.  H <= 8192.  `fused_router=False` takes the logits from the library's
-    product (bit-identical to what `routed_moe` and `MoE.forward` select on) instead of the fused
-    norm+router kernel, whose own summation order can move a bf16 logit by one unit in the last
-    place."""
+    has the dtype of x.  H <= 8192.  `fused_router=False` takes the logits from the product that
+    `routed_moe` and `MoE.forward` run on the same rows (the same bits they select on) instead of the
+    fused norm+router kernel, whose own summation order can move a bf16 logit by one unit in the
+    last place."""
     out, logits, routing = _call(x, k, w1, w3, w2, norm_weight=norm_weight, router_weight=router_weight,
                                  bf16_weights=bf16_weights, eps=float(eps), add_residual=add_residual,
                                  fused_router=fused_router, accumulate=accumulate_into_grad, routing=return_routing)
@@ -155,9 +157,11 @@ def routed_moe(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tensor, w
                accumulate_into_grad: bool = False, return_routing: bool = False):
     """(MoE(x), router logits) for x [T,H]: `router_linear` and `moe_ffn` as one autograd node
     (mlp.py:100-167), so that the two gradient contributions to x (expert path, router path)
-    are summed inside the k-row-sum kernel.  The router product is a bf16 library product
-    whatever the dtypes (the reference's behaviour under its bf16 autocast); the output has
-    the dtype of x.  With `return_routing` a dict of the integer routing tensors and gates is
+    are summed inside the k-row-sum kernel.  The router product is a bf16 product whatever the
+    dtypes (the reference's behaviour under its bf16 autocast), the one of `router_linear`; the
+    output has the dtype of x.  With nothing to differentiate, at most 64 tokens run on kernels
+    whose sums are formed in another order, so their output can differ from the differentiable
+    call's, and from that of the same tokens in a larger batch, in its last bits.  With `return_routing` a dict of the integer routing tensors and gates is
     returned as a third value."""
     out, logits, routing = _call(x, k, w1, w3, w2, router_weight=router_weight, bias=bias, bf16_weights=bf16_weights,
                                  accumulate=accumulate_into_grad, routing=return_routing)

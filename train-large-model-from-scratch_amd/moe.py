@@ -72,8 +72,8 @@ class MoE(nn.Module):
         # instead of by autograd (saves a pass over them per gradient-accumulation micro-step;
         # hooks on these three parameters then do not run, see functional.py).
         self.accumulate_wgrad_into_grad = False
-        # False: `forward_prenorm` takes the router logits from the library's product (the one
-        # `forward` uses) instead of the fused norm+router kernel, whose summation order can move
+        # False: `forward_prenorm` takes the router logits from the product that `forward` uses
+        # instead of the fused norm+router kernel, whose summation order can move
         # a bf16 logit by one unit in the last place and with it the routing of a near-tie.
         self.fused_router = True
         # False (the reference's rule): a call without autocast on fp32 input and fp32 parameters

@@ -7,7 +7,8 @@ every MoE layer.  The two operators below, `moe_gfx950::ffn_fwd` and `moe_gfx950
 carry shape-and-dtype-only ("fake") implementations and an autograd formula, so the tracer
 can keep `MoE.forward` inside one graph, forward and backward: the kernels stay opaque calls,
 everything around them is traced.  `MoE.forward` takes this route only while it is being
-traced; eager calls use `functional.moe_ffn` (same kernels, plus the cached weight copies).
+traced; eager calls use `functional.moe_ffn` (same kernels, plus the cached weight copies, and
+kernels of their own for at most 64 tokens without gradients).
 
 A second pair, `moe_gfx950::routed_fwd` / `routed_bwd`, has the router product inside (the traced
 counterpart of `functional.routed_moe`, what the module's eager call runs under bf16 autocast), and
@@ -140,8 +141,8 @@ def routed_fwd(x: Tensor, wr: Tensor, w1: Tensor, w3: Tensor, w2: Tensor, k: int
                train: bool) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor,
                                      Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     """-> out, logits, ids, gates, offs, pos_to_row, row_to_pos, xn, wrb, xp, gu, act, w1b, w3b, w2b.
-    The forward of `functional.routed_moe`: the router logits are a bf16 library product on the
-    bf16 rows (`xn`) and the bf16 router weight (`wrb`); the rest as in `ffn_fwd`.  A bf16 copy of
+    The forward of `functional.routed_moe`: the router logits are its bf16 product of the bf16 rows
+    (`xn`) and the bf16 router weight (`wrb`); the rest as in `ffn_fwd`.  A bf16 copy of
     a tensor that already is bf16 is empty; without `train` so are xn, wrb, xp, gu and act."""
     T, H = x.shape
     E = wr.shape[0]
