@@ -190,9 +190,11 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     // With few rows an expert is bound by its weights, each line of which is read once.  Where their rows are a
     // multiple of 4 KB long, experts that sweep k side by side ask for the same lines of every page, which lie on few
     // of the memory channels; started at different k-tiles they do not (all tiles of an expert at the same one, so
-    // that they go on sharing the operands in L2).  Gate/up of 64 experts, 2048 <-> 1024, rows per expert and us: 64,
-    // 130 -> 98; 128, 134 -> 107; 191, 147 -> 131; 256, 152 -> 144; from 384 on no difference.  Down, 1024 <-> 2048, 128
-    // rows: 78 -> 60.  With rows of 2 KB there is nothing to gain.
+    // that they go on sharing the operands in L2).  Gate/up of 64 experts, 2048 <-> 1024, again and again on the same
+    // rows, rows per expert and us: 16, 128 -> 94; 64, 130 -> 100; 128, 138 -> 118; 191, 149 -> 141; 256, 186 -> 185.
+    // The whole forward: 100 / 257 / 1000 / 1531 / 2600 tokens (12 to 325 rows an expert) 198 -> 185, 213 -> 188, 237 ->
+    // 218, 269 -> 264, 389 -> 388; above that within 0.6 % either way.  16 experts, 4096 <-> 1536: 64 rows 168 -> 158, 175
+    // rows 196 -> 195.  With rows of 2 KB there is nothing to gain.
     t.kt0 = 0;
     if constexpr (MODE == GATEUP || MODE == DOWN) {
       if (p.K % 2048 == 0) t.kt0 = (t.e * 13) & 31;  // (32 k-tiles to 4 KB)
