@@ -419,8 +419,8 @@ int moe_router_few(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, 
 // 4.8 GB) 49 / 62 / 72 / 84 against 67 / 69 / 69 / 70; 12 experts, 4096 <-> 2048, at 8 / 12 / 20 / 32 (0 / 2.4 / 7.2 / 14)
 // 131 / 153 / 180 / 240 against 135 / 145 / 147 / 149; 8 experts, 4096 <-> 2048, at 16 / 24 / 32 (3.2 / 6.4 / 9.7) 109 / 126 /
 // 148 against 123 / 124 / 126, and 4096 <-> 1024 at 32 (4.8) 78 against 92; 8 experts, 4096 <-> 2048, fp32 rows, at 12 / 16
-// (3.2 / 6.4) 115 / 144 against 124.  At up to 8 rows each these kernels are between half the time (few or small
-// experts) and 1.08 times (64 experts of 50 MB).
+// (3.2 / 6.4) 115 / 144 against 124.  At up to 8 rows each these kernels take from a third of the time (few or
+// small experts) to 1.08 times (64 experts of 50 MB).
 bool moe_few_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int x_dtype) {
   if (T <= 0 || T > FEW_MAX_TOKENS || E > 65535 || H > 65536 || I > 65536) return false;
   const double again = (double)(T * k - 8 * E) * 6.0 * (double)H * (double)I * (x_dtype == MOE_DT_F32 ? 2 : 1);
