@@ -168,3 +168,28 @@ def test_compiled_fp32_call_takes_the_fp32_operators(pkg, lib):
         _say(f"  {n}: rel diff compiled vs eager {rel:.2e}")
         assert rel < 1e-5, (n, rel)
     assert torch.equal(eager[0], compiled[0])
+
+
+@pytest.mark.parametrize("loss_on_logits", [False, True])
+@pytest.mark.parametrize("T", [37, 192])
+def test_traced_layer_takes_views_of_bf16_tensors(pkg, T, loss_on_logits):
+    """x strided or beginning in the middle of an aligned block, the router weight transposed: the operators save
+    them as they are, and the backward pass gives the bits it gives for dense copies."""
+    _say("traced layer on views", T, loss_on_logits)
+    traced = importlib.import_module(pkg.__name__ + ".traced")
+    H, E, I, k = 256, 8, 64, 2
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    wide, flat, wr_t = r(T, H + 8), r(T * H + 1), r(H, E, std=0.3)
+    ws, dy, dl = [r(E, I, H, std=0.1), r(E, I, H, std=0.1), r(E, H, I, std=0.1)], r(T, H), r(T, E)
+
+    def grads(x, wr):
+        leaves = [t.detach().requires_grad_(True) for t in (x, wr, *ws)]
+        out, logits = traced.routed_moe(*leaves, k)
+        torch.autograd.backward([out, logits] if loss_on_logits else [out], [dy, dl] if loss_on_logits else [dy])
+        return [out, logits] + [t.grad for t in leaves]
+
+    for x in (wide[:, :H], flat[1:].view(T, H)):
+        for wr in (wr_t.t(), wr_t.t().contiguous()):
+            for a, b in zip(grads(x, wr), grads(x.contiguous().clone(), wr.contiguous())):
+                assert torch.equal(a, b)

@@ -190,6 +190,7 @@ def routed_bwd(dout: Tensor, dlogits_ext: Tensor | None, xn: Tensor, wrb: Tensor
     dout = ops.dense(dout)
     if dout.dtype != xdt:
         dout = dout.to(xdt)
+    xn, wrb = ops.dense(xn), ops.dense(wrb)  # (x and the router weight themselves where they are bf16: any view)
     dw = [torch.empty_like(w, dtype=f32 if w_is_f32 else _BF16) for w in (w1b, w3b, w2b)]
     saved = (dout, k, gates, ids, offs, pos_to_row, row_to_pos, xp, gu, act, w1b, w3b, w2b, dw)
     if dlogits_ext is None:
