@@ -52,3 +52,25 @@ def test_small_launch_weight_gradients(pkg, lib, T, E, k, H, I, shares, dtype):
     for w, a in zip(ws[1:], again[1:]):
         assert torch.allclose(a.grad.float(), 2 * w.grad.float(), rtol=2e-2 if dtype == torch.bfloat16 else 1e-5,
                               atol=1e-6 * float(w.grad.abs().max()))
+
+
+@pytest.mark.parametrize("H,I", [(128, 128), (136, 264)])
+def test_steps_and_stages(pkg, lib, H, I):
+    """Experts that end at and around every step (32 rows) of the ring of three stages, and one without rows: one
+    launch without and one with a second column tile."""
+    print("steps and stages", H, I, flush=True)
+    counts = [1, 31, 32, 33, 0, 63, 64, 65, 95, 96, 97, 128, 129]
+    g = torch.Generator().manual_seed(H)
+    E = len(counts)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ids = ids[torch.randperm(len(ids), generator=g)]
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(torch.bfloat16)
+    x, w1, w3, w2 = r(len(ids), H), r(E, I, H, std=0.08), r(E, I, H, std=0.08), r(E, H, I, std=0.08)
+    dy = r(len(ids), H, std=0.1)
+    ws = [w.cuda().requires_grad_(True) for w in (w1, w3, w2)]
+    pkg.experts_rows(x.cuda(), ids.cuda(), *ws).backward(dy.cuda())
+    b, be = (O.experts_rows_backward(O.experts_rows_forward(x, ids.numpy(), w1, w3, w2, emulate_bf16=e), dy.float(), w1, w3,
+                                     w2, emulate_bf16=e) for e in (False, True))
+    for name, w in zip(("dw1", "dw3", "dw2"), ws):
+        check(name, w.grad, b[name], be[name])
+        assert not w.grad[counts.index(0)].any()

@@ -123,16 +123,18 @@ __device__ __forceinline__ Row8 load8_nt(const uint16_t* p) {
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (MOE_WAVE - 1); }
 // A value known to be the same in every lane, in a scalar register.
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-// Sum over the wave's lanes up to and including the own (by a whole wave).
+// Sum over the wave's lanes up to and including the own (by a whole wave).  In the vector unit alone: through LDS
+// (six dependent shuffles) it takes some thousand cycles where other waves keep LDS busy.
 __device__ __forceinline__ int wave_inclusive(int v) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int o = 1; o < MOE_WAVE; o <<= 1) {
-    const int u = __shfl_up(v, o, MOE_WAVE);
-    if (lane >= o) v += u;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8: inside the rows of 16
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
   return v;
 }
+__device__ __forceinline__ int read_lane(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

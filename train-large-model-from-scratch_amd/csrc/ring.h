@@ -1,0 +1,78 @@
+// Operand tiles that go from memory straight into a ring of LDS stages (buffer_load .. lds), for workgroups of four
+// waves: no staging registers, no LDS stores, and as many steps on their way as the ring has stages.  A wave-wide load
+// fills 1 KB of consecutive LDS, so a stage has no padding; 16-byte chunks are permuted on the way instead, so that
+// the fragment reads find different banks (no conflicts by SQ_LDS_BANK_CONFLICT).
+#pragma once
+#include "tile_ops.h"
+
+namespace {
+
+// The window's resource from byte_off on; not `live`: empty, everything reads as zero.
+__device__ __forceinline__ u32x4 ring_rsrc(const View& w, long long byte_off, bool live) {
+  long long left = w.bytes - byte_off;
+  if (left < 0 || !live) left = 0;
+  if (left > 0xffffffffll) left = 0xffffffffll;
+  const uint64_t at = (uint64_t)((const char*)w.base + byte_off);
+  return u32x4{(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, (uint32_t)left, 0x00020000u};
+}
+// 16 bytes per lane from `off` into LDS at lds_byte + 16 * lane.  In assembly because the compiler would wait for every
+// such load before any LDS read that follows; the waits are ring_wait's.
+__device__ __forceinline__ void ring_load(uint32_t lds_byte, u32x4 rsrc, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds_byte));
+}
+// All but the wave's N youngest loads have arrived and its LDS reads are done; then meet the other waves, for whose loads
+// and reads the same holds.
+template <int N>
+__device__ __forceinline__ void ring_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const char* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}
+
+// Source is row-contiguous: element (r, kk) at view[(k0 + kk) * ld + r].  A stage holds BK lines of ROWS elements as they
+// lie in memory; fragments come through the transposing read (see OpOuter).
+template <int ROWS_, int BK>
+struct RingOuter {
+  static constexpr int ROWS = ROWS_;
+  static constexpr int CPL = ROWS / 8;  // 16-byte chunks per line
+  static constexpr int BYTES = ROWS * BK * 2;
+  static constexpr int LPP = 64 / CPL;  // lines per wave-wide load
+  static constexpr int PER_WAVE = BYTES / 4096;
+  static_assert(BYTES % 4096 == 0 && ROWS % 128 == 0 && ROWS <= 256, "four waves, lines of 16 or 32 chunks");
+  // Half a wave's transposing read covers 64 bytes of each of four lines: they lie in different quarters of the 64 banks.
+  static __device__ __forceinline__ int swizzle(int line) { return 4 * (line & 3); }
+  uint32_t off[PER_WAVE];  // byte offsets of this lane's chunks in the view
+  __device__ __forceinline__ void init(int ld, int wv) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) {
+      const int line = (i * 4 + wv) * LPP + lane / CPL;
+      off[i] = (uint32_t)(line * ld + ((lane % CPL) ^ swizzle(line)) * 8) * 2;
+    }
+  }
+  __device__ __forceinline__ void load(uint32_t stage, int wv, u32x4 rsrc) const {
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) ring_load(stage + (i * 4 + wv) * 1024, rsrc, off[i]);
+  }
+  // A lane's place in the fragments of rows row0 .. row0 + 31, + 32, ...
+  struct Place {
+    uint32_t at, chunk;
+  };
+  static __device__ __forceinline__ Place place(int row0) {
+    const int lane = lane_id(), i = lane & 15, b = lane >> 4;
+    return {(uint32_t)(((b >> 1) * 8 + (i >> 2)) * ROWS * 2 + (i & 1) * 8),
+            (uint32_t)((row0 / 8 + 2 * (b & 1) + ((i & 3) >> 1)) ^ swizzle(i >> 2))};
+  }
+  // (rows: 0, 32, .. past row0, in bits that row0 does not have)
+  static __device__ __forceinline__ bf16x8 frag(const char* stage, const Place& p, int rows, int ks) {
+    const char* at = stage + (p.at + ((p.chunk ^ (uint32_t)(rows / 8)) << 4) + ks * 16 * ROWS * 2);
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * ROWS * 2));
+    typedef __attribute__((ext_vector_type(8))) short s16x8;
+    const s16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8, r);
+  }
+};
+
+}  // namespace

@@ -8,24 +8,25 @@
 // of the results over at most L rows of an expert, in one launch: there are jobs enough for the chip at three
 // times the segment length, and only experts of more than L rows are cut at all (the others are written
 // straight to their result).  One more launch adds up what was cut.
-#include "tile_ops.h"
-
 #include "internal.h"
+#include "ring.h"
 
 namespace {
 
-constexpr int WBM = 128, WBN = 128;  // tile
-constexpr int WK = 64;               // rows per step
-constexpr int WNT = 256;             // threads: 2 x 2 waves
+constexpr int WBM = 128, WBN = 128;            // tile
+constexpr int WK = 32, WSTAGES = 3;            // rows per step, stages of the ring
+constexpr int WNT = 256;                       // threads: 2 x 2 waves
 constexpr int WFM = WBM / 64, WFN = WBN / 64;  // 32 x 32 blocks per wave
-using WOpA = OpOuter<WBM, WK, WNT>;
-using WOpB = OpOuter<WBN, WK, WNT>;
+using WOpA = RingOuter<WBM, WK>;
+using WOpB = RingOuter<WBN, WK>;
+constexpr int WSTAGE = WOpA::BYTES + WOpB::BYTES;
 
 struct Stack {
   const uint16_t *a, *b;  // [R, M] and [R, N] with row strides lda, ldb
   void* out;              // [E, M, N]
   float* part;            // partial sums [slot][M][N]
   int lda, ldb, M, N, n_tiles, tiles, out_f32, accumulate;
+  float per_n;            // 1 / n_tiles
 };
 struct MultiArgs {
   Stack s[3];
@@ -33,10 +34,18 @@ struct MultiArgs {
   const int32_t* offs;
   int E, L, n_stacks, tiles;   // tiles: of all stacks together
   int T, r_rows, r_slices;
+  int each, r_each;       // tiles of a segment to an XCD, router jobs to an XCD
+  float per_each, r_per_tiles;
 };
+// n / d of a wave-uniform n, 1 / d given (exact: n is far below 2^23)
+__device__ __forceinline__ int quotient(int n, int d, float per_d) {
+  int q = uniform((int)((float)n * per_d));
+  q -= q * d > n;
+  return q + ((q + 1) * d <= n);
+}
 
-// Segment `seg` of the experts' rows: experts of more than L / 2 rows come first (so that the short jobs fill
-// the end), each cut into ceil(n / L) equal parts, an empty one still being a part.
+// A segment of the experts' rows: experts of more than L / 2 rows come first (so that the short jobs fill
+// the end), each cut into ceil(n / L) parts, an empty one still being a part.
 struct Segment {
   int e, row0, row_end, parts, slot;  // slot: of its partial sums, where the expert has several parts
 };
@@ -44,7 +53,11 @@ __device__ __forceinline__ int expert_rows(const int32_t* offs, int e, int E) {
   const int n = e < E ? offs[e + 1] - offs[e] : 0;
   return n > 0 ? n : 0;
 }
-__device__ __forceinline__ int parts_of(int n, int L) { return n > L ? (n + L - 1) / L : 1; }
+__device__ __forceinline__ int parts_of(int n, int L) {
+  if (n <= L) return 1;
+  const int q = (int)((float)n * __builtin_amdgcn_rcpf((float)L));  // within one of n / L
+  return q + (q * L < n) + ((q + 1) * L < n);
+}
 
 // Number of partial-sum slots of the experts before e.
 __device__ __forceinline__ int slots_before(const int32_t* offs, int E, int L, int e) {
@@ -52,30 +65,54 @@ __device__ __forceinline__ int slots_before(const int32_t* offs, int E, int L, i
   int slots = 0;
   for (int b = 0; b < e; b += MOE_WAVE) {
     const int p = b + lane < e ? parts_of(expert_rows(offs, b + lane, E), L) : 1;
-    slots += uniform(__shfl(wave_inclusive(p > 1 ? p : 0), MOE_WAVE - 1, MOE_WAVE));
+    slots += read_lane(wave_inclusive(p > 1 ? p : 0), MOE_WAVE - 1);
   }
   return slots;
 }
-__device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, int seg, Segment& s) {
+// Part j of an expert's rows: equal multiples of 64, the last one what is left (maybe nothing).
+__device__ __forceinline__ void part_rows(int lo, int rows, int j, Segment& s) {
+  const int size = ((int)uniform((int)((float)rows * __builtin_amdgcn_rcpf((float)s.parts))) + 1 + 63) & ~63;
+  const int from = j * size < rows ? j * size : rows;
+  s.row0 = lo + from;
+  s.row_end = lo + (j + 1 < s.parts && from + size < rows ? from + size : rows);
+}
+// Segment `seg`; first and n: the first row and the number of rows of expert `lane`.
+__device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, int seg, int first, int n, Segment& s) {
   const int lane = lane_id();
   int carry = 0;
+  if (E <= MOE_WAVE) {
+    const int p = lane < E ? parts_of(n, L) : 0;
+    const bool big = 2 * n > L;
+    const int ib = wave_inclusive(big ? p : 0);
+    const int nbig = read_lane(ib, 63);
+    const int is = nbig + wave_inclusive(big ? 0 : p);
+    const int sl = wave_inclusive(p > 1 ? p : 0);
+    if (seg >= read_lane(is, 63)) return false;
+    const int f = __builtin_ctzll(__ballot(lane < E && big == (seg < nbig) && (big ? ib : is) > seg));
+    s.e = f;
+    s.parts = read_lane(p, f);
+    const int j = seg - (read_lane(seg < nbig ? ib : is, f) - s.parts);
+    const int lo = read_lane(first, f), rows = read_lane(n, f);
+    part_rows(lo, rows, j, s);
+    s.slot = s.parts > 1 ? read_lane(sl, f) - s.parts + j : 0;
+    return true;
+  }
   for (int pass = 0; pass < 2; ++pass)
     for (int b = 0; b < E; b += MOE_WAVE) {
       const int n = expert_rows(offs, b + lane, E);
       const bool mine = b + lane < E && (2 * n > L) == (pass == 0);
       const int p = mine ? parts_of(n, L) : 0;
       const int incl = wave_inclusive(p);
-      const int total = uniform(__shfl(incl, MOE_WAVE - 1, MOE_WAVE));
+      const int total = read_lane(incl, MOE_WAVE - 1);
       if (seg < carry + total) {
         const int f = __builtin_ctzll(__ballot(carry + incl > seg));
         // (read into scalar registers: everything derived from these is then known to be the same in every
         // lane, which the buffer resources of the operands need)
         s.e = uniform(b + f);
-        s.parts = uniform(__shfl(p, f, MOE_WAVE));
-        const int j = seg - (carry + uniform(__shfl(incl, f, MOE_WAVE)) - s.parts);
-        const int lo = uniform(offs[s.e]), rows = uniform(__shfl(n, f, MOE_WAVE));
-        s.row0 = lo + uniform((int)((long long)rows * j / s.parts));
-        s.row_end = lo + uniform((int)((long long)rows * (j + 1) / s.parts));
+        s.parts = read_lane(p, f);
+        const int j = seg - (carry + read_lane(incl, f) - s.parts);
+        const int lo = uniform(offs[s.e]), rows = read_lane(n, f);
+        part_rows(lo, rows, j, s);
         s.slot = s.parts > 1 ? slots_before(offs, E, L, s.e) + j : 0;
         return true;
       }
@@ -84,26 +121,34 @@ __device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, 
   return false;
 }
 
-// One job per workgroup; three workgroups share a compute unit (41 KB of LDS, four waves of 64 x 64) and hide
-// each other's barriers, loads and epilogues, so the loop is the plain one: the step's lines go from registers to
-// LDS, the next step's are requested, the products run.  Lines keep their memory order in LDS and are read
-// through the transposing read.
+// One job per workgroup; three workgroups share a compute unit (48 KB of LDS each, four waves of 64 x 64) and hide each
+// other's barriers, set-up and epilogues.  Lines come straight into a ring of three 32-row stages, two steps on
+// their way.  What bounds it: LDS (a step's fragments and lines take 1.5 times as long there as its products do), then
+// the jobs' ends (2.0 to 2.5 of 3 workgroups are there on average) and starts (some 6000 cycles until the first lines are
+// asked for, of 28000 and more in the loop).  8192 tokens of 8 experts, 1024 <-> 512, Zipf, and 3333 tokens of 12
+// experts, 1416 <-> 568: through staging registers, 41 KB of LDS, the tiles of a segment dealt to one XCD 99 and
+// 95 us; this one 79 and 81.  Two workgroups with two stages of 64 rows or four of 32: 84 and 92, 80 and 93; two
+// with 256 x 128 tiles and three stages: 99 and 103.
 __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) {
-  __shared__ __attribute__((aligned(16))) uint16_t sm[WOpA::LDS_ELEMS + WOpB::LDS_ELEMS];
+  constexpr int KS = WK / 16, LOADS = WOpA::PER_WAVE + WOpB::PER_WAVE;
+  __shared__ __attribute__((aligned(1024))) char sm[WSTAGES * WSTAGE];
   const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MOE_WAVE));
   const int wm = wv >> 1, wn = wv & 1;
-  // workgroup b runs on XCD b % 8: of 512 consecutive jobs each XCD takes 64 consecutive ones, which
-  // share an expert's rows
-  const int nb = gridDim.x, b = blockIdx.x;
-  int job = b;
-  if ((b | 511) < nb) job = (b & ~511) + (b & 7) * 64 + ((b & 511) >> 3);
+  // Workgroup b runs on XCD b % 8.  Every XCD takes an eighth of each segment's tiles (neighbours, which share operands
+  // in its L2), so that all of them have the same list of segments, long ones first.  (64 consecutive tiles to an
+  // XCD, Zipf: 1.30 workgroups a compute unit on average where it is 1.55 now, with two resident.)
+  const int b = blockIdx.x, x = b & 7;
+  int job = b >> 3;
   Stack st;
   Segment sg;
   int tile;
-  const int r_jobs = p.r_slices * p.router.tiles;
-  if (job < r_jobs) {
+  // (asked for first: on the way while the job's numbers are worked out)
+  const int first = lane < p.E ? p.offs[lane] : 0, count = lane < p.E ? max(p.offs[lane + 1] - first, 0) : 0;
+  if (job < p.r_each) {
+    job += x * p.r_each;
+    if (job >= p.r_slices * p.router.tiles) return;
     st = p.router;
-    const int sl = job / st.tiles;
+    const int sl = quotient(job, st.tiles, p.r_per_tiles);
     tile = job - sl * st.tiles;
     sg.e = 0;
     sg.row0 = sl * p.r_rows;
@@ -111,31 +156,36 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
     sg.parts = 2;  // (its sums always go through the second kernel, which may have fewer rows to write)
     sg.slot = sl;
   } else {
-    job -= r_jobs;
-    const int seg = job / p.tiles;
-    tile = job - seg * p.tiles;
-    if (!find_segment(p.offs, p.E, p.L, seg, sg)) return;
-    int k = 0;
-    while (k + 1 < p.n_stacks && tile >= p.s[k].tiles) tile -= p.s[k++].tiles;
-    st = p.s[k];
+    job -= p.r_each;
+    const int seg = quotient(job, p.each, p.per_each);
+    tile = x * p.each + job - seg * p.each;
+    if (tile >= p.tiles || !find_segment(p.offs, p.E, p.L, seg, first, count, sg)) return;
+    const int t0 = p.s[0].tiles, t1 = t0 + p.s[1].tiles;
+    st = tile < t0 ? p.s[0] : (tile < t1 ? p.s[1] : p.s[2]);
+    tile -= tile < t0 ? 0 : (tile < t1 ? t0 : t1);
   }
-  const int m0 = tile / st.n_tiles * WBM, n0 = tile % st.n_tiles * WBN;
+  const int tm = quotient(tile, st.n_tiles, st.per_n);
+  const int m0 = tm * WBM, n0 = (tile - tm * st.n_tiles) * WBN;
   const int rows = uniform(sg.row_end - sg.row0);
   WOpA opA;
   WOpB opB;
-  opA.init(st.lda);
-  opB.init(st.ldb);
+  opA.init(st.lda, wv);
+  opB.init(st.ldb, wv);
   const View vA = make_view(st.a + (long long)sg.row0 * st.lda + m0, (long long)rows * st.lda - m0);
   const View vB = make_view(st.b + (long long)sg.row0 * st.ldb + n0, (long long)rows * st.ldb - n0);
-  uint16_t *sA = sm, *sB = sm + WOpA::LDS_ELEMS;
-  u32x4 stage[WOpA::CH + WOpB::CH];
-  const auto request = [&](int k0) {
-    const __amdgpu_buffer_rsrc_t ra = view_rsrc(vA, WOpA::k_bytes(k0, st.lda)), rb = view_rsrc(vB, WOpB::k_bytes(k0, st.ldb));
-#pragma unroll
-    for (int c = 0; c < WOpA::CH; ++c) stage[c] = opA.load_one(c, ra);
-#pragma unroll
-    for (int c = 0; c < WOpB::CH; ++c) stage[WOpA::CH + c] = opB.load_one(c, rb);
+  const int steps = (rows + WK - 1) / WK;
+  const uint32_t stages = lds_address(sm);
+  long long askA = 0, askB = 0;
+  uint32_t ask_at = 0;
+  const auto ask = [&](bool live) {  // (past the last step: empty loads, which the counting of loads relies on)
+    opA.load(stages + ask_at, wv, ring_rsrc(vA, askA, live));
+    opB.load(stages + ask_at + WOpA::BYTES, wv, ring_rsrc(vB, askB, live));
+    askA += (long long)st.lda * (WK * 2);
+    askB += (long long)st.ldb * (WK * 2);
+    ask_at = ask_at == (WSTAGES - 1) * WSTAGE ? 0 : ask_at + WSTAGE;
   };
+#pragma unroll
+  for (int i = 0; i < WSTAGES - 1; ++i) ask(i < steps);
   f32x16 acc[WFM][WFN];
 #pragma unroll
   for (int i = 0; i < WFM; ++i)
@@ -143,42 +193,42 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
     for (int j = 0; j < WFN; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  const int offA = WOpA::lane_off(lane), offB = WOpB::lane_off(lane);
-  if (rows > 0) request(0);
-  for (int k0 = 0; k0 < rows; k0 += WK) {
-    lds_barrier();  // the step before is read
-#pragma unroll
-    for (int c = 0; c < WOpA::CH; ++c) opA.store_one(c, sA, stage[c]);
-#pragma unroll
-    for (int c = 0; c < WOpB::CH; ++c) opB.store_one(c, sB, stage[WOpA::CH + c]);
-    lds_barrier();
-    if (k0 + WK < rows) request(k0 + WK);
-    // (a step's fragments are read in the shadow of the products of the step before: the fences keep the
-    // compiler from clumping the reads in front of their use)
+  const WOpA::Place inA = WOpA::place(wm * (WBM / 2));
+  const WOpB::Place inB = WOpB::place(wn * (WBN / 2));
+  uint32_t at = 0;
+  for (int s = 0; s < steps; ++s) {
+    ring_wait<(WSTAGES - 2) * LOADS>();
+    const char *sA = sm + at, *sB = sA + WOpA::BYTES;
     bf16x8 fa[2][WFM], fb[2][WFN];
     const auto read_one = [&](int u, int ks) {  // in the order the products need them
-      if (u == 0) fa[ks & 1][0] = WOpA::frag(sA, offA, wm * (WBM / 2), ks);
-      else if (u <= WFN) fb[ks & 1][u - 1] = WOpB::frag(sB, offB, wn * (WBN / 2) + (u - 1) * 32, ks);
-      else fa[ks & 1][u - WFN] = WOpA::frag(sA, offA, wm * (WBM / 2) + (u - WFN) * 32, ks);
+      if (u == 0) fa[ks & 1][0] = WOpA::frag(sA, inA, 0, ks);
+      else if (u <= WFN) fb[ks & 1][u - 1] = WOpB::frag(sB, inB, (u - 1) * 32, ks);
+      else fa[ks & 1][u - WFN] = WOpA::frag(sA, inA, (u - WFN) * 32, ks);
     };
 #pragma unroll
     for (int u = 0; u < WFM + WFN; ++u) read_one(u, 0);
+    // (the stage of the step before is free; the requests go out while the first fragments are on their way, and the
+    // fences keep the compiler from clumping the other reads in front of their use)
+    __builtin_amdgcn_sched_barrier(0);
+    ask(s + WSTAGES - 1 < steps);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < WK / 16; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int n = 0; n < WFM * WFN; ++n) {
         const int i = n / WFN, j = (i & 1) ? WFN - 1 - n % WFN : n % WFN;  // neighbours share an operand
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks & 1][j], fa[ks & 1][i], acc[i][j], 0, 0, 0);
-        if (ks + 1 < WK / 16 && n < WFM + WFN) read_one(n, ks + 1);
+        if (ks + 1 < KS && n < WFM + WFN) read_one(n, ks + 1);
         __builtin_amdgcn_sched_barrier(0);
       }
+    at = at == (WSTAGES - 1) * WSTAGE ? 0 : at + WSTAGE;
   }
-  lds_barrier();
+  ring_wait<0>();
   // results leave through LDS in strips of 32 rows x 64 columns, fp32: a wave's accumulators hold row l % 32 and
   // columns 8 q + 4 (l / 32) .. + 3 of each block
   constexpr int SS = 64 + 4;  // words per strip row
   float* strip = reinterpret_cast<float*>(sm) + wv * 32 * SS;
-  static_assert(WBN == 128 && 4 * 32 * SS * 4 <= (WOpA::LDS_ELEMS + WOpB::LDS_ELEMS) * 2, "strips fit in the stage");
+  static_assert(WBN == 128 && 4 * 32 * SS * 4 <= WSTAGES * WSTAGE, "strips fit in the stages");
   const bool partial = sg.parts > 1;
   const bool wide = partial || st.out_f32;
   const long long MN = (long long)st.M * st.N;
@@ -304,7 +354,7 @@ int tiles_n(int64_t n) { return (int)((n + WBN - 1) / WBN); }
 int64_t segment_rows(int64_t R, int64_t H, int64_t I) {
   const int64_t tiles = (int64_t)tiles_m(H) * tiles_n(I) + 2 * (int64_t)tiles_m(I) * tiles_n(H);
   int64_t L = R * tiles / (2 * (int64_t)moe_compute_units());
-  L = (L + WK - 1) / WK * WK;
+  L = (L + 63) / 64 * 64;
   return L < 512 ? 512 : (L > (1 << 30) ? 1 << 30 : L);
 }
 
@@ -321,7 +371,7 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
   const auto fill = [](Stack& d, const MoeWgradStack& m) {
     d.a = m.a, d.b = m.b, d.out = m.out, d.part = m.part;
     d.lda = (int)m.lda, d.ldb = (int)m.ldb, d.M = (int)m.M, d.N = (int)m.N;
-    d.n_tiles = tiles_n(m.N), d.tiles = tiles_m(m.M) * d.n_tiles;
+    d.n_tiles = tiles_n(m.N), d.tiles = tiles_m(m.M) * d.n_tiles, d.per_n = 1.f / d.n_tiles;
     d.out_f32 = m.dtype == MOE_DT_F32, d.accumulate = m.accumulate;
   };
   for (int i = 0; i < n_stacks; ++i) {
@@ -339,8 +389,10 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
     a.r_rows = (int)router_rows;
     a.r_slices = (int)router_slices;
   }
+  a.each = a.tiles > 0 ? (a.tiles + 7) / 8 : 1, a.per_each = 1.f / a.each;
+  a.r_each = (a.r_slices * a.router.tiles + 7) / 8, a.r_per_tiles = a.router.tiles ? 1.f / a.router.tiles : 0.f;
   const long long segs = n_stacks ? R / a.L + E : 0;
-  const long long jobs = segs * a.tiles + (long long)a.r_slices * a.router.tiles;
+  const long long jobs = 8 * ((n_stacks ? segs * a.each : 0) + (long long)a.r_each);
   if (jobs <= 0) return 0;
   if (jobs > 0x7fffffffll) return MOE_ERR_LIMIT;
   hipLaunchKernelGGL(wgrad_multi_kernel, dim3((unsigned)jobs), dim3(WNT), 0, s, a);
