@@ -22,6 +22,13 @@ void moe_observe(const char* name, int after);
 bool moe_router_few_ok(int64_t T, int64_t H, int64_t E, int64_t k);
 int moe_router_logits(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
                       void* stream);
+bool moe_place_ok(int64_t T, int64_t E, int64_t k);
+int64_t moe_place_bytes(int64_t T, int64_t E);
+int moe_select_count(const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t E, int64_t k,
+                     int32_t* ids, float* gates, void* table, void* stream);
+int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
+                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, void* xp,
+                   int xp_dtype, void* stream);
 int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
                    int64_t I, float* g, float* u, float* act, void* stream);
 int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
@@ -611,28 +618,39 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
   float* base = f.kept.data_ptr<float>();
   float *xp = base, *g = base + kept.g, *u = base + kept.u, *act = base + kept.act, *y = base + kept.y;
   float* gates = nullptr;
-  const int32_t* ids = r.part(f.routing, Routing::IDS);
-  int32_t* bad = nullptr;
-  Tensor given;
-  if (logits_.defined()) {
-    const Tensor logits = dense(logits_), b = bias.defined() ? dense(bias) : Tensor();
-    gates = (float*)r.part(f.routing, Routing::GATES);
-    CALL(moe_router_topk_fwd, logits.data_ptr(), (int)dt(logits), (const float*)ptr(b), T, E, k,
-         r.part(f.routing, Routing::IDS), gates, s);
-  } else {
-    given = dense(ids_.to(at::kInt));
-    TORCH_CHECK(given.numel() == R, "one expert id per row is needed");
-    ids = given.data_ptr<int32_t>();
-    bad = r.part(f.routing, Routing::BAD);
-  }
-  const int64_t wsb = std::max<int64_t>(moe_dispatch_workspace_bytes(R, E), 16);
+  const bool place = logits_.defined() && H % 8 == 0 && moe_place_ok(T, E, k);
+  const int64_t wsb = std::max<int64_t>(place ? moe_place_bytes(T, E) : moe_dispatch_workspace_bytes(R, E), 16);
   const Tensor ws = empty({wsb}, at::kByte, x);
-  const int32_t* offs = r.part(f.routing, Routing::OFFS);
-  const int32_t* p2r = r.part(f.routing, Routing::POS_TO_ROW);
-  const int32_t* r2p = r.part(f.routing, Routing::ROW_TO_POS);
-  CALL(moe_histogram_scan_checked, ids, R, E, r.part(f.routing, Routing::COUNTS), r.part(f.routing, Routing::OFFS),
-       r.part(f.routing, Routing::POS_TO_ROW), r.part(f.routing, Routing::ROW_TO_POS), bad, ws.data_ptr(), wsb, s);
-  CALL(moe_f32_gather_rows, x.data_ptr<float>(), p2r, T, R, H, k, xp, s);
+  int32_t* counts = r.part(f.routing, Routing::COUNTS);
+  int32_t* offs = r.part(f.routing, Routing::OFFS);
+  int32_t* p2r = r.part(f.routing, Routing::POS_TO_ROW);
+  int32_t* r2p = r.part(f.routing, Routing::ROW_TO_POS);
+  int32_t* ids = r.part(f.routing, Routing::IDS);
+  Tensor logits, b;
+  if (logits_.defined()) {
+    logits = dense(logits_);
+    if (bias.defined()) b = dense(bias);
+    gates = (float*)r.part(f.routing, Routing::GATES);
+  }
+  if (place) {
+    CALL(moe_select_count, logits.data_ptr(), (int)dt(logits), (const float*)ptr(b), T, E, k, ids, gates, ws.data_ptr(), s);
+    CALL(moe_place_rows, x.data_ptr<float>(), MOE_DT_F32, ids, ws.data_ptr(), T, H, E, k, counts, offs, p2r, r2p, xp,
+         MOE_DT_F32, s);
+  } else {
+    int32_t* bad = nullptr;
+    Tensor given;
+    const int32_t* sorted = ids;
+    if (logits.defined()) {
+      CALL(moe_router_topk_fwd, logits.data_ptr(), (int)dt(logits), (const float*)ptr(b), T, E, k, ids, gates, s);
+    } else {
+      given = dense(ids_.to(at::kInt));
+      TORCH_CHECK(given.numel() == R, "one expert id per row is needed");
+      sorted = given.data_ptr<int32_t>();
+      bad = r.part(f.routing, Routing::BAD);
+    }
+    CALL(moe_histogram_scan_checked, sorted, R, E, counts, offs, p2r, r2p, bad, ws.data_ptr(), wsb, s);
+    CALL(moe_f32_gather_rows, x.data_ptr<float>(), p2r, T, R, H, k, xp, s);
+  }
   CALL(moe_f32_gateup, xp, f.w[0].data_ptr<float>(), f.w[1].data_ptr<float>(), offs, E, R, H, I,
        o.train ? g : nullptr, o.train ? u : nullptr, act, s);
   CALL(moe_f32_gemm_rows, act, f.w[2].data_ptr<float>(), offs, E, R, H, I, 1, y, 0, s);

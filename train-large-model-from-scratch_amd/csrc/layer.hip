@@ -37,6 +37,13 @@ struct Carve {
   int64_t ids, gates, counts, offs, pos_to_row, row_to_pos, xp, act, y, dispatch, total;
 };
 
+// Room for the counts that selection and places, or histograms and scans, work on.
+int64_t order_bytes(int64_t T, int64_t E, int64_t k) {
+  const int64_t general = moe_dispatch_workspace_bytes(T * k, E);
+  const int64_t place = moe_place_ok(T, E, k) ? moe_place_bytes(T, E) : 0;
+  return place > general ? place : general;
+}
+
 Carve carve(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
   const int64_t R = T * k;
   Carve c;
@@ -55,7 +62,7 @@ Carve carve(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
   c.xp = take(R * H * 2);
   c.act = take(R * I * 2);
   c.y = take(R * H * 2);
-  c.dispatch = take(moe_dispatch_workspace_bytes(R, E));
+  c.dispatch = take(order_bytes(T, E, k));
   c.total = at;
   return c;
 }
@@ -122,8 +129,12 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
     MOE_STEP("moe_down_one", moe_down_one(act, ids, gates, w2, H, E, I, k, out, out_dtype, st));
     return 0;
   }
-  MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream));
-  if (moe_few_ok(T, H, E, I, k, x_dtype)) {  // rows stay in routed order: no dispatch, no gather
+  const bool few = moe_few_ok(T, H, E, I, k, x_dtype), place = !few && moe_place_ok(T, E, k);
+  if (place)
+    MOE_STEP("moe_select_count", moe_select_count(logits, logits_dtype, bias, T, E, k, ids, gates, ws + c.dispatch, stream));
+  else
+    MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream));
+  if (few) {  // rows stay in routed order: no dispatch, no gather
     MOE_STEP("moe_gateup_few", moe_gateup_few(x, x_dtype, ids, w1, w3, T, H, E, I, k, act, st));
     if (moe_down_one_ok(T, k)) {
       MOE_STEP("moe_down_one", moe_down_one(act, ids, gates, w2, H, E, I, k, out, out_dtype, st));
@@ -133,12 +144,17 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
     MOE_STEP("moe_combine_in_order", moe_combine_in_order(y, gates, T, H, k, out, out_dtype, st));
     return 0;
   }
-  MOE_STEP("moe_histogram_scan_checked",
-           moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
-                              moe_dispatch_workspace_bytes(R, E), stream));
-  MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
-           k > 1 ? moe_permute_fwd_scatter(x, x_dtype, row_to_pos, T, H, k, xp, stream)
-                 : moe_permute_fwd(x, x_dtype, pos_to_row, R, H, k, xp, stream));
+  if (place) {
+    MOE_STEP("moe_place_rows", moe_place_rows(x, x_dtype, ids, ws + c.dispatch, T, H, E, k, counts, offs, pos_to_row,
+                                              row_to_pos, xp, MOE_DT_BF16, stream));
+  } else {
+    MOE_STEP("moe_histogram_scan_checked",
+             moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
+                                moe_dispatch_workspace_bytes(R, E), stream));
+    MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
+             k > 1 ? moe_permute_fwd_scatter(x, x_dtype, row_to_pos, T, H, k, xp, stream)
+                   : moe_permute_fwd(x, x_dtype, pos_to_row, R, H, k, xp, stream));
+  }
   MOE_STEP("moe_gemm_gateup_swiglu_fwd",
            moe_gemm_gateup_swiglu_fwd(xp, w1, w3, offs, E, R, H, I, nullptr, nullptr, act, stream));
   MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_fwd(act, w2, offs, E, R, H, I, y, stream));
@@ -194,7 +210,7 @@ struct FwdScratch {
   void* dispatch;
   FwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t k) {
     y = (uint16_t*)s.take(T * k * H * 2);
-    dispatch = s.take(moe_dispatch_workspace_bytes(T * k, E));
+    dispatch = s.take(order_bytes(T, E, k));
   }
 };
 
@@ -304,18 +320,25 @@ extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) 
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
   const FwdScratch ws(s, T, H, E, k);
   if (!s.fits()) return MOE_ERR_WORKSPACE;
-  if (a->logits)
-    MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids,
-                                                        a->gates, stream));
-  else if (a->ids64 && R > 0)
-    MOE_STEP("moe_narrow_ids", moe_narrow_ids(a->ids64, R, a->ids, (hipStream_t)stream));
-  MOE_STEP("moe_histogram_scan_checked",
-           moe_histogram_scan_checked(a->ids, R, E, a->counts, a->offs, a->pos_to_row, a->row_to_pos, a->bad_ids,
-                                      ws.dispatch, moe_dispatch_workspace_bytes(R, E), stream));
-  if (T == 0) return 0;
-  MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
-           k > 1 ? moe_permute_fwd_scatter(a->x, (int)a->x_dtype, a->row_to_pos, T, H, k, a->xp, stream)
-                 : moe_permute_fwd(a->x, (int)a->x_dtype, a->pos_to_row, R, H, k, a->xp, stream));
+  if (a->logits && moe_place_ok(T, E, k)) {
+    MOE_STEP("moe_select_count", moe_select_count(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids, a->gates,
+                                                  ws.dispatch, stream));
+    MOE_STEP("moe_place_rows", moe_place_rows(a->x, (int)a->x_dtype, a->ids, ws.dispatch, T, H, E, k, a->counts, a->offs,
+                                              a->pos_to_row, a->row_to_pos, a->xp, MOE_DT_BF16, stream));
+  } else {
+    if (a->logits)
+      MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids,
+                                                          a->gates, stream));
+    else if (a->ids64 && R > 0)
+      MOE_STEP("moe_narrow_ids", moe_narrow_ids(a->ids64, R, a->ids, (hipStream_t)stream));
+    MOE_STEP("moe_histogram_scan_checked",
+             moe_histogram_scan_checked(a->ids, R, E, a->counts, a->offs, a->pos_to_row, a->row_to_pos, a->bad_ids,
+                                        ws.dispatch, moe_dispatch_workspace_bytes(R, E), stream));
+    if (T == 0) return 0;
+    MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
+             k > 1 ? moe_permute_fwd_scatter(a->x, (int)a->x_dtype, a->row_to_pos, T, H, k, a->xp, stream)
+                   : moe_permute_fwd(a->x, (int)a->x_dtype, a->pos_to_row, R, H, k, a->xp, stream));
+  }
   if (a->gu)
     MOE_STEP("moe_gemm_gateup_swiglu_fwd_blocked",
              moe_gemm_gateup_swiglu_fwd_blocked(a->xp, a->w1, a->w3, a->offs, E, R, H, I, a->gu, a->act, stream));

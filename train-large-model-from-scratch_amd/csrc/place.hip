@@ -1,0 +1,213 @@
+// From logits to rows in expert order in two launches: selection with counts, then places and rows.
+//
+// The general path (route.hip, dispatch.hip) takes four or five: selection, histograms, their scan, positions, rows.
+// Each of the middle ones moves a few KB and lasts as long as a launch does, 4 to 7 us.  Here the selection's
+// workgroups count their own 16 tokens, a byte an expert, and every workgroup of the second launch adds up the
+// bytes in front of it for itself, while its rows are on their way from memory.  The permutation is the same one: a
+// token asks for an expert at most once, so rows of an expert in the order of their tokens is the stable order.
+// Selection to rows, us, before and now: 2048 tokens, 8 experts, 1024 wide 13.3, 8.3; 1531 tokens, 64 experts,
+// 8 a token, 2048 wide 31.6, 19.7; 8192 tokens, 8 experts 27.6, 16.2; 512 tokens, 256 wide 12.0, 7.3.
+#include "common.h"
+#include "internal.h"
+#include "topk_core.h"
+
+namespace {
+
+constexpr int PLACE_EXPERTS = 2 * MOE_WAVE;
+// Bytes of counts, all of which every placing workgroup reads.  At this many (4096 tokens, 128 experts, 8 a token, 1024
+// wide) the two launches take 26 us where the general path takes 38; past it there are more workgroups, too, and
+// a pass lasts so long that the difference no longer counts.
+constexpr int64_t PLACE_TABLE = 32 * 1024;
+
+int words_of(int64_t E) { return (int)((E + 3) / 4); }
+// Tokens counted together, one a wave.  8 where 16 would leave many compute units idle: 1531 tokens, 64 experts, 8 a token,
+// selection 5.7 us instead of 7.0 (places 14.0 and 13.0); 2048 tokens, 8 experts 3.5 and 4.1 (4.8 and 4.9).
+int chunk_of(int64_t T) { return T <= 2048 ? 8 : 16; }
+
+// One wave a token, as router_topk_fwd_kernel; table[chunk][e] = how many of the chunk's tokens ask for e.
+template <int VPL, typename LT, int CHUNK>
+__global__ __launch_bounds__(CHUNK* MOE_WAVE) void select_count_kernel(const LT* __restrict__ logits,
+                                                                      const float* __restrict__ bias, int T, int E, int k,
+                                                                      int32_t* __restrict__ ids, float* __restrict__ gates,
+                                                                      uint32_t* __restrict__ table) {
+  __shared__ uint32_t asked[PLACE_EXPERTS];  // bit t: token t of the chunk asks for the expert
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE));
+  if (threadIdx.x < PLACE_EXPERTS) asked[threadIdx.x] = 0;
+  __syncthreads();
+  const int t = blockIdx.x * CHUNK + wv;
+  if (t < T) {
+    uint64_t key[VPL];
+    moe_topk_keys<VPL>(logits + (size_t)t * E, bias, E, lane, key);
+    int id;
+    float gate;
+    moe_topk_softmax_wave<VPL>(key, k, lane, id, gate);
+    if (lane < k) {
+      ids[(size_t)t * k + lane] = id;
+      gates[(size_t)t * k + lane] = gate;
+      atomicOr(&asked[id], 1u << wv);
+    }
+  }
+  __syncthreads();
+  const int words = (E + 3) / 4;
+  if (threadIdx.x < words) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) w |= (uint32_t)__popc(asked[threadIdx.x * 4 + b]) << (8 * b);
+    table[(size_t)blockIdx.x * words + threadIdx.x] = w;
+  }
+}
+
+// WAVES tokens of a chunk, one a wave.  `shift`: 2^shift words hold a chunk's counts.
+template <typename XT, typename OT, int CHUNK, int WAVES>
+__global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
+    const XT* __restrict__ x, const int32_t* __restrict__ ids, const uint32_t* __restrict__ table, int T, int E, int k,
+    int H, int shift, int32_t* __restrict__ counts, int32_t* __restrict__ offs, int32_t* __restrict__ pos_to_row,
+    int32_t* __restrict__ row_to_pos, OT* __restrict__ xp) {
+  __shared__ int below[PLACE_EXPERTS], total[PLACE_EXPERTS];  // of earlier chunks, of all
+  __shared__ uint32_t asked[PLACE_EXPERTS];
+  constexpr int AHEAD = 4;  // 8-element pieces of the row requested at once
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE));
+  const int chunk = blockIdx.x / (CHUNK / WAVES), chunks = (T + CHUNK - 1) / CHUNK, words = (E + 3) / 4;
+  const int t = blockIdx.x * WAVES + wv;
+  const bool live = t < T;
+  typename std::conditional<sizeof(XT) == 2, u32x4, Row8>::type row[AHEAD];
+  const auto request = [&](int base) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int col = base + (i * MOE_WAVE + lane) * 8;
+      if (live && col < H) {
+        if constexpr (sizeof(XT) == 2) row[i] = *reinterpret_cast<const u32x4*>(x + (size_t)t * H + col);
+        else row[i] = load8(x + (size_t)t * H + col);
+      }
+    }
+  };
+  request(0);
+  const int my_id = live && lane < k ? ids[(size_t)t * k + lane] : 0;
+  static_assert(WAVES * MOE_WAVE >= PLACE_EXPERTS && CHUNK % WAVES == 0, "a thread an expert");
+  if (threadIdx.x < PLACE_EXPERTS) below[threadIdx.x] = total[threadIdx.x] = 0, asked[threadIdx.x] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < CHUNK * k; i += blockDim.x) {
+    const int r = chunk * CHUNK * k + i;
+    if (r < T * k) atomicOr(&asked[ids[r]], 1u << (i / k));
+  }
+  // two 16-bit sums a register: no expert has more rows than there are tokens
+  const int w = threadIdx.x & ((1 << shift) - 1), step = blockDim.x >> shift;
+  uint32_t all02 = 0, all13 = 0, low02 = 0, low13 = 0;
+  if (w < words) {
+#pragma unroll 4
+    for (int c = threadIdx.x >> shift; c < chunks; c += step) {
+      const uint32_t v = table[(size_t)c * words + w];
+      const uint32_t v02 = v & 0x00ff00ffu, v13 = (v >> 8) & 0x00ff00ffu;
+      all02 += v02;
+      all13 += v13;
+      low02 += c < chunk ? v02 : 0;
+      low13 += c < chunk ? v13 : 0;
+    }
+  }
+  for (int off = MOE_WAVE / 2; off >= 1 << shift; off >>= 1) {
+    all02 += __shfl_xor(all02, off, MOE_WAVE);
+    all13 += __shfl_xor(all13, off, MOE_WAVE);
+    low02 += __shfl_xor(low02, off, MOE_WAVE);
+    low13 += __shfl_xor(low13, off, MOE_WAVE);
+  }
+  if (w < words && lane < (1 << shift)) {
+    atomicAdd(&total[4 * w + 0], (int)(all02 & 0xffff));
+    atomicAdd(&total[4 * w + 1], (int)(all13 & 0xffff));
+    atomicAdd(&total[4 * w + 2], (int)(all02 >> 16));
+    atomicAdd(&total[4 * w + 3], (int)(all13 >> 16));
+    atomicAdd(&below[4 * w + 0], (int)(low02 & 0xffff));
+    atomicAdd(&below[4 * w + 1], (int)(low13 & 0xffff));
+    atomicAdd(&below[4 * w + 2], (int)(low02 >> 16));
+    atomicAdd(&below[4 * w + 3], (int)(low13 >> 16));
+  }
+  __syncthreads();
+  const int n0 = total[lane], n1 = total[MOE_WAVE + lane];
+  const int upto0 = wave_inclusive(n0), half = read_lane(upto0, MOE_WAVE - 1), upto1 = half + wave_inclusive(n1);
+  if (blockIdx.x == 0 && wv == 0) {
+    if (lane < E) counts[lane] = n0, offs[lane] = upto0 - n0;
+    if (MOE_WAVE + lane < E) counts[MOE_WAVE + lane] = n1, offs[MOE_WAVE + lane] = upto1 - n1;
+    if (lane == 0) offs[E] = T * k;
+  }
+  const int first0 = __shfl(upto0 - n0, my_id & 63, MOE_WAVE), first1 = __shfl(upto1 - n1, my_id & 63, MOE_WAVE);
+  int pos = 0;
+  if (live && lane < k) {
+    const uint32_t earlier = asked[my_id] & ((1u << (t % CHUNK)) - 1);
+    pos = (my_id < MOE_WAVE ? first0 : first1) + below[my_id] + __popc(earlier);
+    const int r = t * k + lane;
+    row_to_pos[r] = pos;
+    pos_to_row[pos] = r;
+  }
+  if (!live) return;
+  for (int base = 0; base < H; base += AHEAD * MOE_WAVE * 8) {
+    if (base > 0) request(base);
+    for (int j = 0; j < k; ++j) {
+      OT* dst = xp + (size_t)read_lane(pos, j) * H;
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) {
+        const int col = base + (i * MOE_WAVE + lane) * 8;
+        if (col < H) {
+          if constexpr (sizeof(XT) == 2) store_bits_nt(dst + col, row[i]);
+          else if constexpr (sizeof(OT) == 2) store8_nt(dst + col, row[i]);
+          else store8(dst + col, row[i]);
+        }
+      }
+    }
+  }
+}
+
+}  // namespace
+
+bool moe_place_ok(int64_t T, int64_t E, int64_t k) {
+  return T > 0 && T < 65536 && E <= PLACE_EXPERTS && k <= E && k <= MOE_MAX_TOPK && moe_place_bytes(T, E) <= PLACE_TABLE;
+}
+int64_t moe_place_bytes(int64_t T, int64_t E) { return (T + chunk_of(T) - 1) / chunk_of(T) * words_of(E) * 4; }
+
+int moe_select_count(const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t E, int64_t k,
+                     int32_t* ids, float* gates, void* table, void* stream) {
+  hipStream_t s = (hipStream_t)stream;
+  const auto go = [&](auto vpl, auto lt, auto chunk) {
+    using LT = decltype(lt);
+    constexpr int CHUNK = decltype(chunk)::value;
+    hipLaunchKernelGGL((select_count_kernel<decltype(vpl)::value, LT, CHUNK>), dim3((unsigned)((T + CHUNK - 1) / CHUNK)),
+                       dim3(CHUNK * MOE_WAVE), 0, s, (const LT*)logits, bias, (int)T, (int)E, (int)k, ids, gates,
+                       (uint32_t*)table);
+    return moe_launch_status();
+  };
+  const auto of = [&](auto chunk) {
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if (logits_dtype == MOE_DT_BF16) return E <= MOE_WAVE ? go(One{}, uint16_t{}, chunk) : go(Two{}, uint16_t{}, chunk);
+    return E <= MOE_WAVE ? go(One{}, float{}, chunk) : go(Two{}, float{}, chunk);
+  };
+  return chunk_of(T) == 8 ? of(std::integral_constant<int, 8>{}) : of(std::integral_constant<int, 16>{});
+}
+
+int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
+                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, void* xp,
+                   int xp_dtype, void* stream) {
+  if (H <= 0 || H % 8 != 0) return MOE_ERR_SHAPE;
+  if (H > 65536) return MOE_ERR_LIMIT;
+  if (x_dtype == MOE_DT_BF16 && xp_dtype != MOE_DT_BF16) return MOE_ERR_DTYPE;
+  hipStream_t s = (hipStream_t)stream;
+  int shift = 0;
+  while ((1 << shift) < words_of(E)) ++shift;
+  const auto go = [&](auto xt, auto ot, auto chunk, auto waves) {
+    using XT = decltype(xt);
+    using OT = decltype(ot);
+    constexpr int CHUNK = decltype(chunk)::value, WAVES = decltype(waves)::value;
+    hipLaunchKernelGGL((place_rows_kernel<XT, OT, CHUNK, WAVES>), dim3((unsigned)((T + WAVES - 1) / WAVES)),
+                       dim3(WAVES * MOE_WAVE), 0, s, (const XT*)x, ids, (const uint32_t*)table, (int)T, (int)E, (int)k,
+                       (int)H, shift, counts, offs, pos_to_row, row_to_pos, (OT*)xp);
+    return moe_launch_status();
+  };
+  const auto of = [&](auto chunk, auto waves) {
+    if (x_dtype == MOE_DT_BF16) return go(uint16_t{}, uint16_t{}, chunk, waves);
+    return xp_dtype == MOE_DT_BF16 ? go(float{}, uint16_t{}, chunk, waves) : go(float{}, float{}, chunk, waves);
+  };
+  using Eight = std::integral_constant<int, 8>;
+  using Sixteen = std::integral_constant<int, 16>;
+  if (chunk_of(T) == 8) return of(Eight{}, Eight{});
+  // (fewer workgroups to read a large table: 4096 tokens, 128 experts 18.1 us, with 8 waves 20.0; 8192 tokens, 8 experts,
+  // 4 KB 11.1 and 10.7)
+  return moe_place_bytes(T, E) > PLACE_TABLE / 2 ? of(Sixteen{}, Sixteen{}) : of(Sixteen{}, Eight{});
+}
