@@ -357,6 +357,10 @@ __global__ __launch_bounds__(256) void permute_fwd_scatter_kernel(const XT* __re
 // dlogits has k nonzero entries, so that product is k rows of the router weight per token, which sit in
 // every XCD's L2 (at most 512 rows) -- instead of a library product over all E columns, its result in
 // memory and another read of it here.
+// Bound by memory; on small calls by the two trips it takes, positions and then rows.  One wave a token: positions,
+// gates and ids are the same for all of its lanes and come as scalars, eight at a time, and the rows of y and of wr
+// are on their way together.  (A lane a piece of any of four tokens, wr after y: 8192 tokens, k = 2, 1024 wide,
+// both directions 31.2 -> 23.2 us; 3333 tokens, k = 3, 1416 wide 32.4 -> 21.2; 16384 tokens, k = 8, 2048 wide 250 -> 227.)
 template <typename OT, typename AT, bool ROUTER, bool IN_ORDER>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __restrict__ y,
                                                          const float* __restrict__ gates,
@@ -367,69 +371,54 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
                                                          const int32_t* __restrict__ ids,
                                                          const uint16_t* __restrict__ wr) {
   const int H = H8 * 8;
-  for (long long blk = blockIdx.x; blk * ROWS_PER_BLOCK < T; blk += gridDim.x) {
-    const int row0 = (int)(blk * ROWS_PER_BLOCK);
-    for (int c = threadIdx.x; c < ROWS_PER_BLOCK * H8; c += blockDim.x) {
-      const int t = row0 + c / H8, col = (c % H8) * 8;
-      if (t >= T) continue;
-      Row8 acc;
+  for (int t = blockIdx.x * ROWS_PER_BLOCK + uniform((int)(threadIdx.x / MOE_WAVE)); t < T;
+       t += gridDim.x * ROWS_PER_BLOCK) {
+    const int r0 = t * k;
+    for (int col = lane_id() * 8; col < H; col += MOE_WAVE * 8) {
+      Row8 acc, d2;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc.v[i] = 0.f;
+      for (int i = 0; i < 8; ++i) acc.v[i] = 0.f, d2.v[i] = 0.f;
+      // the next N rows, all in flight; summed in slot order
+      const auto add = [&](int j, auto n) {
+        constexpr int N = decltype(n)::value;
+        u32x4 v[N], w[ROUTER ? N : 1];
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+          const int pos = IN_ORDER ? r0 + j + q : row_to_pos[r0 + j + q];
+          v[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(y + (size_t)pos * H + col));
+        }
+        if constexpr (ROUTER) {
+#pragma unroll
+          for (int q = 0; q < N; ++q) w[q] = *reinterpret_cast<const u32x4*>(wr + (size_t)ids[r0 + j + q] * H + col);
+        }
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+          const float gt = gates ? gates[r0 + j + q] : 1.f;
+          const Row8 row = row8_from_bits(v[q]);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc.v[i] += gt * row.v[i];
+        }
+        if constexpr (ROUTER) {
+#pragma unroll
+          for (int q = 0; q < N; ++q) {
+            const float ds = dsel[r0 + j + q];
+            const Row8 row = row8_from_bits(w[q]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) d2.v[i] += ds * row.v[i];
+          }
+        }
+      };
       int j = 0;
-      for (; j + 8 <= k; j += 8) {  // eight rows in flight; summed in slot order all the same
-        int pos[8];
-        float gt[8];
-        Row8 v[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          pos[q] = IN_ORDER ? t * k + j + q : row_to_pos[(size_t)t * k + j + q];
-          gt[q] = gates ? gates[(size_t)t * k + j + q] : 1.f;
-        }
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = load8_nt(y + (size_t)pos[q] * H + col);
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc.v[i] += gt[q] * v[q].v[i];
-      }
-      for (; j + 4 <= k; j += 4) {  // four rows in flight; summed in slot order all the same
-        int pos[4];
-        float gt[4];
-        Row8 v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          pos[q] = IN_ORDER ? t * k + j + q : row_to_pos[(size_t)t * k + j + q];
-          gt[q] = gates ? gates[(size_t)t * k + j + q] : 1.f;
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = load8_nt(y + (size_t)pos[q] * H + col);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc.v[i] += gt[q] * v[q].v[i];
-      }
-      for (; j < k; ++j) {
-        const int pos = IN_ORDER ? t * k + j : row_to_pos[(size_t)t * k + j];
-        const float gt = gates ? gates[(size_t)t * k + j] : 1.f;
-        const Row8 v = load8_nt(y + (size_t)pos * H + col);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc.v[i] += gt * v.v[i];
-      }
+      for (; j + 8 <= k; j += 8) add(j, std::integral_constant<int, 8>{});
+      if (j + 4 <= k) add(j, std::integral_constant<int, 4>{}), j += 4;
+      if (j + 2 <= k) add(j, std::integral_constant<int, 2>{}), j += 2;
+      if (j < k) add(j, std::integral_constant<int, 1>{});
       if (addend) {
         const Row8 a = load8(addend + (size_t)t * H + col);
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc.v[i] += a.v[i];
       }
       if constexpr (ROUTER) {
-        Row8 d2;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) d2.v[i] = 0.f;
-        for (int q = 0; q < k; ++q) {
-          const float ds = dsel[(size_t)t * k + q];
-          const Row8 w = load8(wr + (size_t)ids[(size_t)t * k + q] * H + col);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) d2.v[i] += ds * w.v[i];
-        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc.v[i] += bf16_to_f32(f32_to_bf16(d2.v[i]));
       }
@@ -515,8 +504,7 @@ __global__ __launch_bounds__(256) void combine_bwd_token_kernel(
     float* __restrict__ dgates) {
   const int H = H8 * 8, lane = lane_id();
   const int wpb = blockDim.x / MOE_WAVE;
-  for (long long t = (long long)blockIdx.x * wpb + threadIdx.x / MOE_WAVE; t < T;
-       t += (long long)gridDim.x * wpb) {
+  for (int t = blockIdx.x * wpb + uniform((int)(threadIdx.x / MOE_WAVE)); t < T; t += gridDim.x * wpb) {
     Row8 d[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -524,7 +512,7 @@ __global__ __launch_bounds__(256) void combine_bwd_token_kernel(
       if (c < H8) d[i] = load8(dy + (size_t)t * H + c * 8);
     }
     for (int j = 0; j < k; ++j) {
-      const long long r = t * k + j;
+      const int r = t * k + j;
       const int pos = row_to_pos[r];
       const float gt = gates ? gates[r] : 1.f;
       float dot = 0.f;
