@@ -71,6 +71,37 @@ __global__ __launch_bounds__(RT_WAVES* MOE_WAVE) void router_few_kernel(const ui
   }
 }
 
+// One token: a wave an expert, all of its 16-byte pieces requested before the first product where the row is at most
+// 4096 wide.  As one column of 16 the matrix kernel above fills four workgroups of sixteen waves, whose start and sums
+// cost more than the trip to memory: 64 experts, 2048 wide 5.5 -> TODO us.
+constexpr int RO_WAVES = 4;
+__global__ __launch_bounds__(RO_WAVES* MOE_WAVE) void router_one_kernel(const uint16_t* __restrict__ x,
+                                                                       const uint16_t* __restrict__ wr, int H, int E,
+                                                                       uint16_t* __restrict__ logits) {
+  constexpr int KC = 8;
+  const int lane = lane_id(), e = blockIdx.x * RO_WAVES + uniform((int)(threadIdx.x / MOE_WAVE));
+  if (e >= E) return;
+  const __amdgpu_buffer_rsrc_t rx = rsrc(x, (long long)H * 2), rw = rsrc(wr + (size_t)e * H, (long long)H * 2);
+  float acc = 0.f;
+  for (int h = 0; h < H; h += KC * MOE_WAVE * 8) {
+    bf16x8 a[KC], b[KC];
+#pragma unroll
+    for (int d = 0; d < KC; ++d) {  // (past the row: zeros)
+      const unsigned off = (unsigned)(h + (d * MOE_WAVE + lane) * 8) * 2;
+      a[d] = load_frag(rx, off);
+      b[d] = load_frag(rw, off);
+    }
+#pragma unroll
+    for (int d = 0; d < KC; ++d) {
+      const Row8 u = row8_from_bits(__builtin_bit_cast(u32x4, a[d])), v = row8_from_bits(__builtin_bit_cast(u32x4, b[d]));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc += u.v[i] * v.v[i];
+    }
+  }
+  acc = moe_wave_sum_f32(acc);
+  if (lane == 0) logits[e] = f32_to_bf16(acc);
+}
+
 // ---- rows of one expert times its weights' columns ----------------------------------------------------
 // Columns: KC 32-deep k-steps of 16 columns of NB weight stacks; rows: the same steps of MF blocks of 16 rows.
 template <int NB, int KC>
@@ -405,6 +436,11 @@ bool moe_router_few_ok(int64_t T, int64_t H, int64_t E, int64_t k) {
 
 int moe_router_few(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
                    hipStream_t s) {
+  if (T == 1) {
+    hipLaunchKernelGGL(router_one_kernel, dim3((unsigned)((E + RO_WAVES - 1) / RO_WAVES)), dim3(RO_WAVES * MOE_WAVE), 0, s, x,
+                       wr, (int)H, (int)E, logits);
+    return moe_launch_status();
+  }
   const dim3 grid((unsigned)((E + 15) / 16), (unsigned)((T + 15) / 16));
   hipLaunchKernelGGL(router_few_kernel, grid, dim3(RT_WAVES * MOE_WAVE), 0, s, x, wr, (int)T, (int)H, (int)E, logits);
   return moe_launch_status();
