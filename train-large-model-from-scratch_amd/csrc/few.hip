@@ -73,7 +73,7 @@ __global__ __launch_bounds__(RT_WAVES* MOE_WAVE) void router_few_kernel(const ui
 
 // One token: a wave an expert, all of its 16-byte pieces requested before the first product where the row is at most
 // 4096 wide.  As one column of 16 the matrix kernel above fills four workgroups of sixteen waves, whose start and sums
-// cost more than the trip to memory: 64 experts, 2048 wide 5.5 -> TODO us.
+// cost more than the trip to memory: 64 experts, 2048 wide 5.4 -> 3.7 us (a token 30.5 -> 28.1).
 constexpr int RO_WAVES = 4;
 __global__ __launch_bounds__(RO_WAVES* MOE_WAVE) void router_one_kernel(const uint16_t* __restrict__ x,
                                                                        const uint16_t* __restrict__ wr, int H, int E,
