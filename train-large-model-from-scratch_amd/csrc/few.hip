@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void few_kernel(const AT* __restrict__ A, i
     int e;
     if constexpr (VPL > 0) {
       const int lane = lane_id();
-      uint64_t key[VPL];
+      uint32_t key[VPL];
       if (sel.logits_f32) moe_topk_keys<VPL>((const float*)sel.logits, sel.bias, E, lane, key);
       else moe_topk_keys<VPL>((const uint16_t*)sel.logits, sel.bias, E, lane, key);
       int id;

@@ -226,11 +226,11 @@ __global__ __launch_bounds__(NT) void rmsnorm_router_fwd_kernel(
   for (int m = wv; m < RB; m += NW) {
     const int t = t0 + m;
     if (t >= T) break;
-    uint64_t key[2];
+    uint32_t key[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int e = i * MOE_WAVE + lane;
-      key[i] = e < E ? moe_topk_key(bf16_to_f32(lg16[m * E + e]), e) : 0;
+      key[i] = e < E ? moe_orderable(bf16_to_f32(lg16[m * E + e])) : 0;
     }
     int my_id;
     float my_gate;

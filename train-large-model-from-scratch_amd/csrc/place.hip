@@ -36,7 +36,7 @@ __global__ __launch_bounds__(CHUNK* MOE_WAVE) void select_count_kernel(const LT*
   __syncthreads();
   const int t = blockIdx.x * CHUNK + wv;
   if (t < T) {
-    uint64_t key[VPL];
+    uint32_t key[VPL];
     moe_topk_keys<VPL>(logits + (size_t)t * E, bias, E, lane, key);
     int id;
     float gate;

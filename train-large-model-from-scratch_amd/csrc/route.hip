@@ -19,7 +19,7 @@ __global__ __launch_bounds__(256) void router_topk_fwd_kernel(const LT* __restri
   const int lane = lane_id();
   const int t = blockIdx.x * (blockDim.x / MOE_WAVE) + (threadIdx.x / MOE_WAVE);
   if (t >= T) return;  // whole wave exits together
-  uint64_t key[VPL];
+  uint32_t key[VPL];
   moe_topk_keys<VPL>(logits + (size_t)t * E, bias, E, lane, key);
   int my_id;
   float my_gate;

@@ -15,37 +15,22 @@ __device__ __forceinline__ float moe_from_orderable(uint32_t u) {
   u ^= ((u >> 31) ? 0x80000000u : 0xffffffffu);
   return __builtin_bit_cast(float, u);
 }
-// key = (orderable(logit) << 32) | (0xffffffff - expert): the maximum key is the largest logit
-// and, among equal logits, the smallest expert index.  0 marks "taken / absent".
-__device__ __forceinline__ uint64_t moe_topk_key(float logit, int expert) {
-  return ((uint64_t)moe_orderable(logit) << 32) | (uint64_t)(0xffffffffu - (uint32_t)expert);
-}
-
-// Wave-wide maximum of a 64-bit key, the same value in every lane.  Four exchange steps inside
-// each row of 16 lanes go through the DPP data path of the vector ALU (neighbour, pair, mirrored
-// half row, mirrored row: no LDS, no waits), then the four row maxima are read as scalars.
-template <int CTRL>
-__device__ __forceinline__ uint64_t moe_dpp_max_step(uint64_t v) {
-  const int lo = (int)(uint32_t)v, hi = (int)(uint32_t)(v >> 32);
-  const uint32_t lo2 = (uint32_t)__builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, false);
-  const uint32_t hi2 = (uint32_t)__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, false);
-  const uint64_t o = ((uint64_t)hi2 << 32) | lo2;
-  return o > v ? o : v;
-}
-__device__ __forceinline__ uint64_t moe_wave_max_u64(uint64_t v) {
-  v = moe_dpp_max_step<0xB1>(v);   // quad_perm [1,0,3,2]: lane ^ 1
-  v = moe_dpp_max_step<0x4E>(v);   // quad_perm [2,3,0,1]: lane ^ 2
-  v = moe_dpp_max_step<0x141>(v);  // row_half_mirror: the other quad of each 8 lanes
-  v = moe_dpp_max_step<0x140>(v);  // row_mirror: the other half of each 16 lanes
-  const int lo = (int)(uint32_t)v, hi = (int)(uint32_t)(v >> 32);
-  uint64_t best = 0;
-#pragma unroll
-  for (int row = 0; row < MOE_WAVE / 16; ++row) {
-    const uint64_t o = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, 16 * row) << 32) |
-                       (uint32_t)__builtin_amdgcn_readlane(lo, 16 * row);
-    best = o > best ? o : best;
+// Wave-wide maximum, the same value in every lane: a running maximum inside the rows of 16 lanes and then across them
+// on the DPP data path of the vector ALU (no LDS, no waits), read from the last lane.
+__device__ __forceinline__ uint32_t moe_wave_max_u32(uint32_t v) {
+#define MOE_MAX_STEP(ctrl, rows)                                                                            \
+  {                                                                                                         \
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, ctrl, rows, 0xf, false);       \
+    v = o > v ? o : v;                                                                                      \
   }
-  return best;
+  MOE_MAX_STEP(0x111, 0xf)  // row_shr:1, 2, 4, 8
+  MOE_MAX_STEP(0x112, 0xf)
+  MOE_MAX_STEP(0x114, 0xf)
+  MOE_MAX_STEP(0x118, 0xf)
+  MOE_MAX_STEP(0x142, 0xa)  // row_bcast:15 to rows 1 and 3
+  MOE_MAX_STEP(0x143, 0xc)  // row_bcast:31 to rows 2 and 3
+#undef MOE_MAX_STEP
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, MOE_WAVE - 1);
 }
 __device__ __forceinline__ float moe_wave_sum_f32(float v) {
 #pragma unroll
@@ -53,10 +38,11 @@ __device__ __forceinline__ float moe_wave_sum_f32(float v) {
   return v;
 }
 
-// The keys of one token's E logits, plus the experts' biases unless NULL.
+// The keys of one token's E logits, plus the experts' biases unless NULL: the larger the logit, the larger the key; 0
+// (which no logit maps to) marks what is taken or absent.
 template <int VPL, typename LT>
 __device__ __forceinline__ void moe_topk_keys(const LT* __restrict__ logits, const float* __restrict__ bias, int E, int lane,
-                                              uint64_t (&key)[VPL]) {
+                                              uint32_t (&key)[VPL]) {
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int e = i * MOE_WAVE + lane;
@@ -66,33 +52,42 @@ __device__ __forceinline__ void moe_topk_keys(const LT* __restrict__ logits, con
       if constexpr (sizeof(LT) == 2) v = bf16_to_f32(((const uint16_t*)logits)[e]);
       else v = ((const float*)logits)[e];
       if (bias) v += bias[e];
-      key[i] = moe_topk_key(v, e);
+      key[i] = moe_orderable(v);
     }
   }
 }
 
-// k rounds of a wave-wide maximum over the keys (consumed), then the softmax over the k selected
-// logits in fp32.  On return lane j < k holds slot j: expert id and gate.
+// k rounds of a wave-wide maximum over the keys (consumed), each won by the first expert that has it, then the
+// softmax over the k selected logits in fp32.  On return lane j < k holds slot j: expert id and gate.
+// What bounds it is the chain of k rounds: a 32-bit key, and the winner from a ballot, make a round a dozen
+// instructions.  (64-bit keys that held the expert too: 4096 tokens, 8 of 128 experts
+// 7.5 -> 5.6 us; norm, router and selection of 8192 tokens 52.1 -> 49.4; a single token, whose gate/up waits for it, 15.8 -> 15.1.)
 template <int VPL>
-__device__ __forceinline__ void moe_topk_softmax_wave(uint64_t (&key)[VPL], int k, int lane, int& my_id,
+__device__ __forceinline__ void moe_topk_softmax_wave(uint32_t (&key)[VPL], int k, int lane, int& my_id,
                                                       float& my_gate) {
   my_id = 0;
-  float my_val = 0.f;
+  float my_val = 0.f, vmax = 0.f;
   for (int j = 0; j < k; ++j) {
-    uint64_t best = key[0];
+    uint32_t best = key[0];
 #pragma unroll
     for (int i = 1; i < VPL; ++i) best = key[i] > best ? key[i] : best;
-    best = moe_wave_max_u64(best);
-    const uint32_t e = 0xffffffffu - (uint32_t)best;
+    best = moe_wave_max_u32(best);
+    int e = 0;
+#pragma unroll
+    for (int i = VPL - 1; i >= 0; --i) {  // (the first slot that has it, and there the first lane)
+      const unsigned long long here = __ballot(key[i] == best);
+      if (here) e = i * MOE_WAVE + __builtin_ctzll(here);
+    }
 #pragma unroll
     for (int i = 0; i < VPL; ++i)
-      if ((int)e == i * MOE_WAVE + lane) key[i] = 0;
+      if (e == i * MOE_WAVE + lane) key[i] = 0;
+    const float val = moe_from_orderable(best);
+    if (j == 0) vmax = val;
     if (lane == j) {
-      my_id = (int)e;
-      my_val = moe_from_orderable((uint32_t)(best >> 32));
+      my_id = e;
+      my_val = val;
     }
   }
-  const float vmax = __shfl(my_val, 0, MOE_WAVE);
   const float p = lane < k ? expf(my_val - vmax) : 0.f;
   const float s = moe_wave_sum_f32(p);
   my_gate = p / s;
