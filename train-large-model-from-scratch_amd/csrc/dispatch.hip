@@ -1061,25 +1061,6 @@ int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const
 
 namespace {
 
-// 8 elements per thread; the slices of an element are read a fixed ascending order: reproducible
-template <typename OutT>
-__global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, int slices,
-                                                        long long stride8, long long n8,
-                                                        OutT* __restrict__ dw) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= n8) return;
-  Row8 acc;
-#pragma unroll
-  for (int v = 0; v < 8; ++v) acc.v[v] = 0.f;
-#pragma unroll 4
-  for (int s = 0; s < slices; ++s) {
-    const Row8 r = load8(part + (s * stride8 + i) * 8);
-#pragma unroll
-    for (int v = 0; v < 8; ++v) acc.v[v] += r.v[v];
-  }
-  store8(dw + i * 8, acc);
-}
-
 __global__ __launch_bounds__(256) void narrow_ids_kernel(const int64_t* __restrict__ ids, int R,
                                                         int32_t* __restrict__ out) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1089,19 +1070,6 @@ __global__ __launch_bounds__(256) void narrow_ids_kernel(const int64_t* __restri
 }
 
 }  // namespace
-
-int moe_sum_slices(const float* part, int64_t slices, int64_t Mp, int64_t M, int64_t N, void* dw, int dw_dtype,
-                   hipStream_t s) {
-  const long long n8 = M * N / 8;
-  const dim3 grid((unsigned)((n8 + 255) / 256)), block(256);
-  if (dw_dtype == MOE_DT_F32)
-    hipLaunchKernelGGL(sum_slices_kernel<float>, grid, block, 0, s, part, (int)slices, (long long)(Mp * N / 8), n8,
-                       (float*)dw);
-  else
-    hipLaunchKernelGGL(sum_slices_kernel<uint16_t>, grid, block, 0, s, part, (int)slices, (long long)(Mp * N / 8), n8,
-                       (uint16_t*)dw);
-  return moe_launch_status();
-}
 
 int moe_narrow_ids(const int64_t* ids, int64_t R, int32_t* out, hipStream_t s) {
   hipLaunchKernelGGL(narrow_ids_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, s, ids, (int)R, out);

@@ -58,7 +58,6 @@ struct GemmArgs {
   int ld_c;     // row stride of the outputs C0/C1 in elements when it is not N (0: N)
   int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
   int whole_only;  // row-ragged modes: no half tiles (test hook)
-  int slice;    // WGRAD without offsets: "expert" e is rows e*slice .. (e+1)*slice of the R rows; 0: offs
 };
 
 template <int BM_, int BN_, int BK_, int WM_, int WN_>
@@ -155,13 +154,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     if constexpr (MODE == WGRAD) {
       t.e = slot / p.m_slots;
       t.m0 = (slot % p.m_slots) * BM;
-      if (p.slice) {
-        t.row0 = t.e * p.slice;
-        t.row_end = t.row0 + p.slice < p.R ? t.row0 + p.slice : p.R;
-      } else {
-        t.row0 = offs[t.e];
-        t.row_end = offs[t.e + 1];
-      }
+      t.row0 = offs[t.e];
+      t.row_end = offs[t.e + 1];
     } else {
       if (slot >= tile_start[p.E]) return false;
       int lo = 0, hi = p.E;  // largest e with tile_start[e] <= slot (skips empty experts)
@@ -993,7 +987,7 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_ge
       lo = x * wgs;
       t_hi = p.E * TP;
       t_step = nb;
-      if (!p.slice && p.E <= MOE_WAVE && TP % wgs == 0 && p.E * (TP / wgs) <= MAX_GROUPS) {
+      if (p.E <= MOE_WAVE && TP % wgs == 0 && p.E * (TP / wgs) <= MAX_GROUPS) {
         if (threadIdx.x < MOE_WAVE) {
           const int gpe = TP / wgs;  // groups per expert
           constexpr long long FIXED = 4 * CfgMain::BK;  // fill, tile switch and epilogue, in rows' worth
@@ -1309,12 +1303,4 @@ extern "C" int moe_gemm_wgrad(const uint16_t* a_, const uint16_t* b_, const int3
   a.E = (int)E; a.R = (int)R; a.M = (int)M; a.N = (int)N; a.accumulate = accumulate;
   return dw_dtype == MOE_DT_F32 ? launch_wgrad<float>(a, (hipStream_t)stream)
                                 : launch_wgrad<uint16_t>(a, (hipStream_t)stream);
-}
-
-int moe_wgrad_slices(const uint16_t* a_, const uint16_t* b_, int64_t T, int64_t M, int64_t N, int64_t slices,
-                     int64_t slice_rows, float* part, hipStream_t s) {
-  GemmArgs a{};
-  a.A0 = a_; a.B0 = b_; a.C0 = part; a.slice = (int)slice_rows;
-  a.E = (int)slices; a.R = (int)T; a.M = (int)M; a.N = (int)N;
-  return launch_wgrad<float>(a, s);
 }

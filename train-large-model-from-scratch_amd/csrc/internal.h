@@ -9,15 +9,6 @@ void moe_observe(const char* name, int after);
 // Compute units of the current GPU (asked of the runtime once).
 int moe_compute_units();
 
-// part[s] = a[rows of slice s]^T b[rows of slice s], fp32 [slices][M][N]: a [T,M], b [T,N] bf16, slice s
-// = rows s*slice_rows .. of T (gemm.hip).
-int moe_wgrad_slices(const uint16_t* a, const uint16_t* b, int64_t T, int64_t M, int64_t N, int64_t slices,
-                     int64_t slice_rows, float* part, hipStream_t s);
-
-// dw[m][n] = sum over s, ascending, of part[s][m][n] for m < M; part has Mp >= M rows per slice (dispatch.hip).
-int moe_sum_slices(const float* part, int64_t slices, int64_t Mp, int64_t M, int64_t N, void* dw, int dw_dtype,
-                   hipStream_t s);
-
 // Gate gradients from the dgrad-down kernel's block sums, softmax Jacobian and scatter to the logits in
 // one kernel (route.hip).  dlogits [T, ld] with columns E..ld-1 zero; dsel fp32 [T*k] (may be NULL): the k
 // nonzero entries per token, rounded to dlogits' type.
@@ -45,7 +36,7 @@ struct MoeWgradStack {
 };
 // Bytes of each stack's part for R rows.
 int64_t moe_wgrad_multi_part_bytes(int64_t R, int64_t H, int64_t I);
-// The stacks (the first n_stacks, all of the size I x H or H x I) and, unless NULL, the router: a [T, M >= E] and b
+// The stacks (the first n_stacks, all of the size I x H or H x I; without any, offs may be NULL) and, unless NULL, the router: a [T, M >= E] and b
 // [T,N] contracted in router_slices slices of router_rows rows (part [slices][M][N]), out [E,N].
 int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgradStack* router, const int32_t* offs,
                     int64_t E, int64_t R, int64_t H, int64_t I, int64_t T, int64_t router_slices,

@@ -34,7 +34,7 @@ struct MultiArgs {
   const int32_t* offs;
   int E, L, n_stacks, tiles;   // tiles: of all stacks together
   int T, r_rows, r_slices;
-  int each, r_each;       // tiles of a segment to an XCD, router jobs to an XCD
+  int each, e_each, r_each;  // tiles of a segment to an XCD, its jobs of all segments, its router jobs (which come last)
   float per_each, r_per_tiles;
 };
 // n / d of a wave-uniform n, 1 / d given (exact: n is far below 2^23)
@@ -127,8 +127,9 @@ __device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, 
 // the jobs' ends (2.0 to 2.5 of 3 workgroups are there on average) and starts (some 6000 cycles until the first lines are
 // asked for, of 28000 and more in the loop).  8192 tokens of 8 experts, 1024 <-> 512, Zipf, and 3333 tokens of 12
 // experts, 1416 <-> 568: through staging registers, 41 KB of LDS, the tiles of a segment dealt to one XCD 99 and
-// 95 us; this one 79 and 81.  Two workgroups with two stages of 64 rows or four of 32: 84 and 92, 80 and 93; two
-// with 256 x 128 tiles and three stages: 99 and 103.
+// 95 us; this one 79 and 81, and with 16 slices of the router's tokens, at the end of the list, instead of 32 at its start
+// 72 and 82.  Two workgroups with two stages of 64 rows or four of 32: 84 and 92, 80 and 93; two with 256 x 128 tiles
+// and three stages: 99 and 103; four with two stages of 32 rows 77 and 85 where this one takes 72 and 82.
 __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) {
   constexpr int KS = WK / 16, LOADS = WOpA::PER_WAVE + WOpB::PER_WAVE;
   __shared__ __attribute__((aligned(1024))) char sm[WSTAGES * WSTAGE];
@@ -143,9 +144,10 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   Segment sg;
   int tile;
   // (asked for first: on the way while the job's numbers are worked out)
-  const int first = lane < p.E ? p.offs[lane] : 0, count = lane < p.E ? max(p.offs[lane + 1] - first, 0) : 0;
-  if (job < p.r_each) {
-    job += x * p.r_each;
+  const bool experts = job < p.e_each && lane < p.E;
+  const int first = experts ? p.offs[lane] : 0, count = experts ? max(p.offs[lane + 1] - first, 0) : 0;
+  if (job >= p.e_each) {
+    job += x * p.r_each - p.e_each;
     if (job >= p.r_slices * p.router.tiles) return;
     st = p.router;
     const int sl = quotient(job, st.tiles, p.r_per_tiles);
@@ -156,7 +158,6 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
     sg.parts = 2;  // (its sums always go through the second kernel, which may have fewer rows to write)
     sg.slot = sl;
   } else {
-    job -= p.r_each;
     const int seg = quotient(job, p.each, p.per_each);
     tile = x * p.each + job - seg * p.each;
     if (tile >= p.tiles || !find_segment(p.offs, p.E, p.L, seg, first, count, sg)) return;
@@ -392,9 +393,10 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
   a.each = a.tiles > 0 ? (a.tiles + 7) / 8 : 1, a.per_each = 1.f / a.each;
   a.r_each = (a.r_slices * a.router.tiles + 7) / 8, a.r_per_tiles = a.router.tiles ? 1.f / a.router.tiles : 0.f;
   const long long segs = n_stacks ? R / a.L + E : 0;
-  const long long jobs = 8 * ((n_stacks ? segs * a.each : 0) + (long long)a.r_each);
+  const long long e_each = n_stacks ? segs * a.each : 0, jobs = 8 * (e_each + (long long)a.r_each);
   if (jobs <= 0) return 0;
   if (jobs > 0x7fffffffll) return MOE_ERR_LIMIT;
+  a.e_each = (int)e_each;
   hipLaunchKernelGGL(wgrad_multi_kernel, dim3((unsigned)jobs), dim3(WNT), 0, s, a);
   const long long cut = n_stacks ? R / a.L : 0;  // experts of more than L rows, at most
   const long long ys = (cut < E ? cut : E) + (router ? 1 : 0);
