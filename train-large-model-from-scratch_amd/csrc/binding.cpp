@@ -22,6 +22,7 @@ void moe_observe(const char* name, int after);
 bool moe_router_few_ok(int64_t T, int64_t H, int64_t E, int64_t k);
 int moe_router_logits(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,
                       void* stream);
+int moe_cast_two(const float* a, uint16_t* to_a, int64_t na, const float* b, uint16_t* to_b, int64_t nb, void* stream);
 bool moe_place_ok(int64_t T, int64_t E, int64_t k);
 int64_t moe_place_bytes(int64_t T, int64_t E);
 int moe_select_count(const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t E, int64_t k,
@@ -241,7 +242,16 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   if (o.train || o.routing_out || !(wr.defined() || logits_.defined()) || norm_w.defined() || T == 0)
     f.routing = empty({r.at[Routing::PARTS]}, at::kInt, x);
   if (wr.defined()) {
-    f.wrb = dense(cast_bf16(dense(wr.detach())));
+    const Tensor wrd = dense(wr.detach());
+    const bool both = !norm_w.defined() && x_type == at::kFloat && wrd.scalar_type() == at::kFloat && H % 8 == 0 && T > 0;
+    if (both) {  // (a launch each took 4.7 us for the router's weight and 7.7 for 4096 tokens, 1024 wide; together 8.8)
+      f.wrb = empty(wrd.sizes(), at::kBFloat16, x);
+      f.xn = empty(x.sizes(), at::kBFloat16, x);
+      CALL(moe_cast_two, x.data_ptr<float>(), (uint16_t*)f.xn.data_ptr(), x.numel(), wrd.data_ptr<float>(),
+           (uint16_t*)f.wrb.data_ptr(), wrd.numel(), s);
+    } else {
+      f.wrb = dense(cast_bf16(wrd));
+    }
     if (norm_w.defined()) {
       f.nw = norm_w.detach().to(at::kFloat).contiguous();
       f.xn = empty({T, H}, at::kBFloat16, x);
@@ -258,7 +268,7 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
         CALL(moe_rmsnorm_fwd, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, T, H,
              (uint16_t*)f.xn.data_ptr(), f.rstd.data_ptr<float>(), s);
       }
-    } else {
+    } else if (!both) {
       f.xn = cast_bf16(x);
     }
     rows = f.xn;

@@ -550,6 +550,17 @@ __global__ __launch_bounds__(256) void cast_kernel(const float* __restrict__ src
     dst[n8 * 8 + threadIdx.x] = f32_to_bf16(src[n8 * 8 + threadIdx.x]);
 }
 
+// Two tensors of multiples of 8 elements in one launch.
+__global__ __launch_bounds__(256) void cast_two_kernel(const float* __restrict__ a, uint16_t* __restrict__ to_a,
+                                                      long long a8, const float* __restrict__ b,
+                                                      uint16_t* __restrict__ to_b, long long b8) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < a8 + b8;
+       i += (long long)gridDim.x * blockDim.x) {
+    if (i < a8) store8(to_a + i * 8, load8(a + i * 8));
+    else store8(to_b + (i - a8) * 8, load8(b + (i - a8) * 8));
+  }
+}
+
 inline unsigned mover_grid(int64_t rows, int per_block) {
   int64_t b = (rows + per_block - 1) / per_block;
   const int64_t cap = 256 * 16;  // 16 resident 256-thread blocks per CU is plenty for a copy
@@ -1030,6 +1041,17 @@ extern "C" int moe_cast_f32_bf16(const float* src, uint16_t* dst, int64_t n, voi
   if (blocks > 256 * 16) blocks = 256 * 16;
   hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, src,
                      dst, n8, (long long)n);
+  return moe_launch_status();
+}
+
+int moe_cast_two(const float* a, uint16_t* to_a, int64_t na, const float* b, uint16_t* to_b, int64_t nb, void* stream) {
+  if (na < 0 || nb < 0 || na % 8 != 0 || nb % 8 != 0) return MOE_ERR_SHAPE;
+  for (const void* q : {(const void*)a, (const void*)to_a, (const void*)b, (const void*)to_b}) MOE_CHECK_PTR(q);
+  long long blocks = ((na + nb) / 8 + 255) / 256;
+  if (blocks < 1) blocks = 1;
+  if (blocks > 256 * 16) blocks = 256 * 16;
+  hipLaunchKernelGGL(cast_two_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a, to_a,
+                     (long long)(na / 8), b, to_b, (long long)(nb / 8));
   return moe_launch_status();
 }
 

@@ -22,6 +22,9 @@ int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const
                            const uint16_t* wr, int64_t T, int64_t H, int64_t k, void* dx, int dx_dtype,
                            hipStream_t s);
 
+// fp32 to bf16, two tensors of multiples of 8 elements in one launch (dispatch.hip).
+int moe_cast_two(const float* a, uint16_t* to_a, int64_t na, const float* b, uint16_t* to_b, int64_t nb, void* stream);
+
 // int64 expert ids to int32, values outside int32 to -1 (dispatch.hip).
 int moe_narrow_ids(const int64_t* ids, int64_t R, int32_t* out, hipStream_t s);
 
