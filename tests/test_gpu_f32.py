@@ -107,6 +107,33 @@ def _gemm_case(P, counts, N, K):
             assert torch.equal(acc_w[e].cpu(), prev[e])
 
 
+@pytest.mark.parametrize("counts", [
+    [7] * 63 + [900],                                # 64 experts, all but one tied, the largest last
+    [0, 5, 0, 5, 600, 5, 0, 1],                      # ties, empty experts
+    [(37 * i) % 90 for i in range(65)],              # one more than are sorted
+    [400] + [3] * 129,                               # three words of experts, dealt
+    [130] * 5,                                       # even: not dealt
+], ids=["64", "8", "65", "130", "even"])
+@pytest.mark.parametrize("tile", [64, 128])
+def test_f32_weight_gradients_of_uneven_experts(P, counts, tile):
+    """Three stacks in one launch, the largest experts' tiles first and dealt to all XCDs: every tile of every
+    expert once.  Sums of at most 900 products in fp32: the bar of this file."""
+    E, R, H, I = len(counts), int(sum(counts)), 260, 132
+    _say("f32 wgrads", E, R, "tile", tile)
+    offs = _offsets(counts)
+    g = torch.Generator().manual_seed(E + R)
+    dg, du, act = (torch.randn(R, I, generator=g) for _ in range(3))
+    dyp, xp = (torch.randn(R, H, generator=g) for _ in range(2))
+    before = P.lib.load().cdll.moe_f32_gemm_force_tile(tile)
+    try:
+        got = P.ops.f32_wgrads(*(t.cuda() for t in (dg, du, dyp, xp, act)), torch.from_numpy(offs).cuda())
+    finally:
+        P.lib.load().cdll.moe_f32_gemm_force_tile(before)
+    for name, w, a, b in zip(("dw1", "dw3", "dw2"), got, (dg, du, dyp), (xp, xp, act)):
+        ref = torch.stack([a[s:t].double().t() @ b[s:t].double() for s, t in zip(offs[:-1], offs[1:])])
+        _close(name, w, ref)
+
+
 @pytest.mark.parametrize("T,H,E,k", [(300, 64, 8, 2), (1000, 132, 64, 8), (5, 4, 3, 1), (64, 2048, 16, 4)])
 def test_f32_row_movers(P, T, H, E, k):
     _say("f32 movers", T, H, E, k)

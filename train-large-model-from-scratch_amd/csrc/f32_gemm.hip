@@ -238,10 +238,17 @@ __device__ __forceinline__ float sigmoid_f32(float x) { return 1.f / (1.f + expf
 struct Job {
   int tile, part;  // part: 0..3 of the tile, -1: all of it; tile < 0: none
 };
-__device__ __forceinline__ Job job_of(int tiles, int cus) {
+// chunk > 0: the list is dealt to the XCDs by so many tiles instead (what is left after the last full deal one by one).
+__device__ __forceinline__ Job job_of(int tiles, int cus, int chunk = 0) {
   const int rest = tiles % cus, cut = rest * 4 <= cus * 3 ? rest : 0, whole = tiles - cut;
   const int x = blockIdx.x & 7;
   int j = blockIdx.x >> 3;
+  if (chunk > 0) {
+    const int b = blockIdx.x, at = b - (whole + 7) / 8 * 8;
+    if (j < whole / (8 * chunk) * chunk) return Job{(j / chunk * 8 + x) * chunk + j % chunk, -1};
+    if (b < whole) return Job{b, -1};
+    return at >= 0 && at < cut * 4 ? Job{whole + at / 4, at % 4} : Job{-1, 0};
+  }
   const int q = whole / 8, r = whole % 8, mine = q + (x < r ? 1 : 0);
   if (j < mine) return Job{x * q + (x < r ? x : r) + j, -1};
   j -= mine;
@@ -259,7 +266,7 @@ template <int MODE, typename S>
 using RowsB = typename std::conditional<b_kcont<MODE>, KCont<S::BN, S::TK>, RCont<S::BN, S::TK>>::type;
 template <int MODE, typename S>
 using RowsLoop = Loop<S, KCont<S::BM, S::TK>, RowsB<MODE, S>>;
-constexpr int larger(int a, int b) { return a > b ? a : b; }
+constexpr __host__ __device__ int larger(int a, int b) { return a > b ? a : b; }
 
 // The tile of Shape S at rows row0.. (of the expert's up to row_end), columns n0..
 template <int MODE, typename S>
@@ -397,9 +404,8 @@ __global__ __launch_bounds__(NT, S::WAVES) void f32_rows_kernel(const RowsArgs p
 }
 
 // Weight gradients: per stack C_e[m, n] (+)= sum over the rows r of expert e of A[r, m] * B[r, n], up to three stacks in
-// one launch.  Tiles are numbered stack by stack and expert by expert: the workgroups that an XCD runs side by side walk
-// the rows of one or two experts together and find them in its L2.  An expert without rows gets zeros (or is
-// left alone when accumulating).
+// one launch: the workgroups that an XCD runs side by side walk the rows of a few experts together and find them in its
+// L2.  An expert without rows gets zeros (or is left alone when accumulating).
 struct F32Stack {
   const float *a, *b;  // [R, M], [R, N]
   float* c;            // [E, M, N]
@@ -458,30 +464,65 @@ __device__ __forceinline__ void wgrad_tile(const F32Stack& s, float* lds, int e,
   }
 }
 
+// The e-th largest of up to 64 values >= 0, each lane's own (a lane without one has -1), equal ones in the order of the
+// lanes: its lane.  The value bit by bit from the top, by how many are at least as large.  (Every ballot is of all lanes.)
+__device__ __forceinline__ int lane_of_rank(int n, int largest, int e) {
+  int value = 0;
+  for (int bit = 1 << (31 - __builtin_clz(largest | 1)); bit; bit >>= 1)
+    if (__builtin_popcountll(__ballot(n >= (value | bit))) > e) value |= bit;
+  const unsigned long long same = __ballot(n == value);
+  const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)same, 0));
+  const int place = e - __builtin_popcountll(__ballot(n > value));
+  return __builtin_ctzll(__ballot(n == value & before == place));
+}
+
+// A tile costs what its expert has rows.  Tiles go stack by stack and expert by expert, an eighth of the list for each XCD, which
+// gives it parts of three different experts; but where one expert has more than 5/4 of the mean they go expert by expert, up to
+// 64 experts the largest first, and are dealt to all XCDs, an eighth of a stack's at a time.  (4096 rows of 8 experts, three
+// stacks of 1024 x 512, half the rows in one expert: 205 us the first way, 167 dealt; 8192 rows of 24 experts: 135 and 82;
+// even experts: 120 and 122.)
 template <typename S, typename Q>
 __global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs p, int cus) {
   __shared__ __align__(16) float lds[larger(WgradLoop<S>::LDS_FLOATS, WgradLoop<Q>::LDS_FLOATS)];
-  int per_e[3], n_col[3], tiles = 0;
+  int per_e[3], n_col[3], per = 0;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     n_col[i] = i < p.n ? (p.s[i].N + S::BN - 1) / S::BN : 0;
     per_e[i] = i < p.n ? n_col[i] * ((p.s[i].M + S::BM - 1) / S::BM) : 0;
-    tiles += per_e[i] * p.E;
+    per += per_e[i];
   }
-  Job job = job_of(tiles, cus);
+  const auto rows_of = [&](int e, int& first) {  // 0: none, or offsets that no dispatch would produce; -1: no such expert
+    first = 0;
+    if (e >= p.E) return -1;
+    const int b = p.offs[e], end = p.offs[e + 1];
+    if (b < 0 || end > p.R || end <= b) return 0;
+    first = b;
+    return end - b;
+  };
+  const int lane = threadIdx.x & 63;
+  int first, rows = rows_of(lane, first);
+  bool uneven = false;
+  for (int e0 = 0; e0 < p.E; e0 += MOE_WAVE) {
+    int at;
+    uneven |= __ballot(4ll * p.E * rows_of(e0 + lane, at) > 5ll * p.R) != 0;
+  }
+  const Job job = job_of(per * p.E, cus, uneven ? larger(per_e[0] / 8, 1) : 0);
   if (job.tile < 0) return;
-  int w = 0, pe = per_e[0], nc = n_col[0];
+  int w = 0, nc = n_col[0], pe = per_e[0], tile = uneven ? job.tile % per : job.tile;
+  const int share = uneven ? 1 : p.E;  // experts whose tiles of a stack follow each other
 #pragma unroll
   for (int i = 1; i < 3; ++i)
-    if (w == i - 1 && job.tile >= per_e[i - 1] * p.E) {
-      job.tile -= per_e[i - 1] * p.E;
-      w = i, pe = per_e[i], nc = n_col[i];
+    if (w == i - 1 && tile >= per_e[i - 1] * share) {
+      tile -= per_e[i - 1] * share;
+      w = i, nc = n_col[i], pe = per_e[i];
     }
+  int e = uneven ? job.tile / per : tile / pe;
+  tile %= pe;
+  if (uneven && p.E <= MOE_WAVE) e = lane_of_rank(rows, p.R, e);
+  rows = rows_of(e, first);
+  const int b = uniform(first), end = b + uniform(rows);
   const F32Stack s = p.s[w];
-  const int e = job.tile / pe;
-  int m0 = job.tile % pe / nc * S::BM, n0 = job.tile % pe % nc * S::BN;
-  int b = p.offs[e], end = p.offs[e + 1];
-  if (b < 0 || end > p.R || end < b) b = end = 0;
+  int m0 = tile / nc * S::BM, n0 = tile % nc * S::BN;
   if (job.part < 0) {
     wgrad_tile<S>(s, lds, e, b, end, m0, n0);
   } else {
@@ -499,10 +540,14 @@ using LargeQuarter = Shape<64, 64, 16, 2, 2, 2>;
 int forced_tile = 0;
 // The large tile has half the operand traffic and LDS reads per flop (32768 rows of 8 experts, 2048 <-> 1024, gate and up: 1.99
 // against 2.17 ms, 138 TFLOP/s), but few of them share a compute unit less evenly (8192 rows of 16 experts, 1024 <-> 1024, five
-// rounds of large tiles: 335 against 295 us; three rounds: equal): from eight rounds on.
-bool large_tiles(int64_t tiles128) {
+// rounds of large tiles: 335 against 295 us; three rounds: equal): from eight rounds on.  A weight gradient's operands are
+// both read from LDS a value at a time, which the large tile halves (three stacks of 1024 x 512, 4096 rows of 8 experts, three
+// rounds: 120 against 126 us; 4096 rows of 16 experts, six rounds: 123 against 134; 1.5 rounds of 512 x 512: 60
+// against 58): from three rounds on.
+constexpr int ROW_ROUNDS = 8, WGRAD_ROUNDS = 3;
+bool large_tiles(int64_t tiles128, int rounds) {
   if (forced_tile) return forced_tile == 128;
-  return tiles128 >= 8 * (int64_t)moe_compute_units();
+  return tiles128 >= rounds * (int64_t)moe_compute_units();
 }
 
 int check_rows(int64_t E, int64_t R, int64_t N, int64_t K) {
@@ -519,7 +564,7 @@ int launch_rows(RowsArgs a, int64_t E, int64_t R, int64_t N, int64_t K, hipStrea
   a.E = (int)E, a.R = (int)R, a.N = (int)N, a.K = (int)K;
   const int cus = moe_compute_units();
   const auto tiles = [&](int64_t t) { return (R / t + E) * ((N * (MODE == GATEUP ? 2 : 1) + t - 1) / t); };  // at most
-  if (large_tiles(tiles(128)))
+  if (large_tiles(tiles(128), ROW_ROUNDS))
     hipLaunchKernelGGL((f32_rows_kernel<MODE, Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, s, a, cus);
   else
     hipLaunchKernelGGL((f32_rows_kernel<MODE, Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, s, a, cus);
@@ -609,7 +654,7 @@ static int wgrads(const F32Stack* s, int n, const int32_t* offs, int64_t E, int6
   }
   if (tiles(64) > 0x70000000ll) return MOE_ERR_LIMIT;
   const int cus = moe_compute_units();
-  if (large_tiles(tiles(128)))
+  if (large_tiles(tiles(128), WGRAD_ROUNDS))
     hipLaunchKernelGGL((f32_wgrad_kernel<Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, st, p, cus);
   else
     hipLaunchKernelGGL((f32_wgrad_kernel<Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, st, p, cus);
