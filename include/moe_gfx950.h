@@ -194,11 +194,12 @@ int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const uint16_t* 
                                            void* stream);
 /* Test hook (no counterpart in the reference).  The four row-ragged products (gate/up, down and
  * their two input gradients) run on 256-row tiles, what is left after whole rounds of them on
- * 128-row tiles where that is shorter, and launches of few tiles on 128-row tiles throughout.
- * moe_gemm_force_row_tile(128 or 256) forces one of them for every later
- * call, 0 restores the automatic choice; the previous setting is returned.  Process-wide and not
+ * 128-row tiles where that is shorter, and launches of few tiles on 128-row tiles or 64-row tiles (up to
+ * 128 experts, g and u blocked or not kept) throughout.
+ * moe_gemm_force_row_tile(64, 128 or 256) forces one of them for every later
+ * call (64: where there is such a tile), 0 restores the automatic choice; the previous setting is returned.  Process-wide and not
  * synchronised with calls in flight on other host threads.  No result depends on the choice:
- * every output element is accumulated over k in the same order on both tile heights, so all
+ * every output element is accumulated over k in the same order on all tile heights, so all
  * outputs (the gate gradients' block sums included) are the same bits either way. */
 int moe_gemm_force_row_tile(int rows);
 /* Backward of gate/up w.r.t. the rows (autograd of mlp.py:154-155): dxp = dg*W1 + du*W3. */

@@ -28,37 +28,10 @@
 // as they lie in memory and read through the transposing LDS read of gfx950.
 // Workgroups are numbered so that each XCD (own L2) works on a contiguous range of tiles,
 // i.e. on its own experts' weights.
-#include "internal.h"
+#include "gemm_args.h"
 #include "tile_ops.h"
 
 namespace {
-
-enum Mode { GATEUP = 0, DOWN = 1, DGRAD_DOWN = 2, DGRAD_GATEUP = 3, WGRAD = 4 };
-
-struct GemmArgs {
-  const uint16_t* A0;
-  const uint16_t* A1;
-  const uint16_t* B0;
-  const uint16_t* B1;
-  void* C0;
-  void* C1;
-  void* C2;
-  const uint16_t* X0;
-  const uint16_t* X1;
-  const int32_t* offs;
-  int E;        // experts
-  int R;        // total rows of the row-ragged operand(s)
-  int M;        // WGRAD only: rows of dw[e]
-  int N;        // output columns
-  int K;        // contraction length per segment (not used by WGRAD)
-  int n_tiles;  // tiles along N
-  int m_slots;  // row-tile slots (ragged modes) or tiles along M (WGRAD)
-  int accumulate;
-  int ld_a;     // row stride of A0/A1 in elements when it is not the contraction length (0: K)
-  int ld_c;     // row stride of the outputs C0/C1 in elements when it is not N (0: N)
-  int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
-  int whole_only;  // row-ragged modes: no half tiles (test hook)
-};
 
 template <int BM_, int BN_, int BK_, int WM_, int WN_>
 struct TileCfg {
@@ -72,12 +45,6 @@ struct TileCfg {
   static constexpr int WAVES_PER_SIMD = NT / 256 * WGS_PER_CU;
   static_assert(WTM % 32 == 0 && WTN % 32 == 0 && BK % 32 == 0, "tile shape");
 };
-
-// sigmoid from the two hardware transcendentals (v_exp_f32, v_rcp_f32; about 1 ulp each):
-// the epilogues are VALU-bound, and an IEEE division would triple their cost.
-__device__ __forceinline__ float sigmoidf_(float x) {
-  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
 
 template <int MODE, typename Cfg>
 constexpr int lds_bytes() {
@@ -1093,7 +1060,8 @@ long long row_slots(int64_t R, int64_t E, int tile) { return (R + tile - 1) / ti
 
 // Which kernel a row-ragged launch takes: decided from the shapes alone (never from the routing: no host
 // synchronisation).  With fewer tiles than half the compute units, by the bound on their number, every one of them can be
-// halved.  `forced_row_tile` (0: automatic) is a test hook.
+// halved; what csrc/row_ring.hip takes is done there.  `forced_row_tile` (0: automatic) is a test hook.
+constexpr int RING_TILE = 64;
 int forced_row_tile = 0;
 
 // A row-ragged launch with `cols` output columns to a tile.
@@ -1101,9 +1069,13 @@ template <int MODE, bool BLK = false>
 int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   static_assert(lds_bytes<MODE, CfgHalf>() <= lds_bytes<MODE, CfgMain>(), "both row tiles fit");
   static bool attr_done[2][MOE_MAX_DEVICES];  // per GPU and instantiation
+  int rc = 0;
+  if ((!forced_row_tile || forced_row_tile == RING_TILE) &&
+      moe_ring_rows((Mode)MODE, BLK, a, forced_row_tile == RING_TILE, s, &rc))
+    return rc;
   a.n_tiles = (a.N + cols - 1) / cols;
   const long long tiles = row_slots(a.R, a.E, ROW_TILE) * ((a.N + CfgMain::BN - 1) / CfgMain::BN);
-  const bool small = forced_row_tile ? forced_row_tile == CfgHalf::BM : 2 * tiles < moe_compute_units();
+  const bool small = forced_row_tile > RING_TILE ? forced_row_tile == CfgHalf::BM : 2 * tiles < moe_compute_units();
   if (small)
     return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK>, attr_done[0], a,
                                  a.n_tiles * row_slots(a.R, a.E, CfgHalf::BM), s);
@@ -1178,12 +1150,12 @@ extern "C" int moe_gemm_down_fwd(const uint16_t* act, const uint16_t* w2, const 
   return launch_rows<DOWN>(a, CfgMain::BN, (hipStream_t)stream);
 }
 
-// Test hook: 0 lets every row-ragged launch choose its row-tile height (the default), 128 or 256
-// forces it.  Process-wide and not synchronised: for tests that want every shape on every tile
-// configuration, not for production callers.  Returns the previous setting.
+// Test hook: 0 lets every row-ragged launch choose its row-tile height (the default), 64, 128 or 256 forces it (64: of
+// the launches that have such tiles).  Process-wide and not synchronised: for tests that want every shape on every
+// tile configuration, not for production callers.  Returns the previous setting.
 extern "C" int moe_gemm_force_row_tile(int rows) {
   const int before = forced_row_tile;
-  if (rows == 0 || rows == CfgHalf::BM || rows == CfgMain::BM) forced_row_tile = rows;
+  if (rows == 0 || rows == RING_TILE || rows == CfgHalf::BM || rows == CfgMain::BM) forced_row_tile = rows;
   return before;
 }
 

@@ -1,0 +1,39 @@
+// What the kernels of the grouped bf16 products share: the modes, a launch's arguments, the gate's sigmoid.
+#pragma once
+#include "internal.h"
+
+enum Mode { GATEUP = 0, DOWN = 1, DGRAD_DOWN = 2, DGRAD_GATEUP = 3, WGRAD = 4 };
+
+struct GemmArgs {
+  const uint16_t* A0;
+  const uint16_t* A1;
+  const uint16_t* B0;
+  const uint16_t* B1;
+  void* C0;
+  void* C1;
+  void* C2;
+  const uint16_t* X0;
+  const uint16_t* X1;
+  const int32_t* offs;
+  int E;        // experts
+  int R;        // total rows of the row-ragged operand(s)
+  int M;        // WGRAD only: rows of dw[e]
+  int N;        // output columns
+  int K;        // contraction length per segment (not used by WGRAD)
+  int n_tiles;  // tiles along N
+  int m_slots;  // row-tile slots (ragged modes) or tiles along M (WGRAD)
+  int accumulate;
+  int ld_a;     // row stride of A0/A1 in elements when it is not the contraction length (0: K)
+  int ld_c;     // row stride of the outputs C0/C1 in elements when it is not N (0: N)
+  int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
+  int whole_only;  // row-ragged modes: no half tiles (test hook)
+};
+
+// sigmoid from the two hardware transcendentals (v_exp_f32, v_rcp_f32; about 1 ulp each):
+// the epilogues are VALU-bound, and an IEEE division would triple their cost.
+__device__ __forceinline__ float sigmoidf_(float x) {
+  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+}
+
+// Takes a row-ragged launch of few tiles (csrc/row_ring.hip): false where it does not.
+bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, bool forced, hipStream_t s, int* rc);

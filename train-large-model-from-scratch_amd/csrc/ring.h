@@ -30,6 +30,43 @@ __device__ __forceinline__ uint32_t lds_address(const char* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
 
+// Source is k-contiguous: element (r, kk) at view[r * ld + k0 + kk].  A stage holds ROWS rows of BK elements; fragments are
+// 16-byte reads.
+template <int ROWS_, int BK>
+struct RingInner {
+  static constexpr int ROWS = ROWS_;
+  static constexpr int CPR = BK / 8;  // 16-byte chunks per row
+  static constexpr int BYTES = ROWS * BK * 2;
+  static constexpr int RPP = 64 / CPR;  // rows per wave-wide load
+  static constexpr int PER_WAVE = BYTES / 4096;
+  static_assert(BYTES % 4096 == 0 && CPR == 8, "four waves, rows of 128 bytes");
+  static __device__ __forceinline__ int swizzle(int row) { return (row >> 1) & 7; }
+  uint32_t off[PER_WAVE];  // byte offsets of this lane's chunks in the view
+  int kc;                  // first k of its chunks
+  __device__ __forceinline__ void init(int ld, int wv) {
+    const int lane = lane_id(), r = lane / CPR;
+    kc = ((lane % CPR) ^ swizzle(wv * RPP + r)) * 8;
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) off[i] = (uint32_t)(((i * 4 + wv) * RPP + r) * ld + kc) * 2;
+  }
+  // k past the end of the contraction lies in the next row: such chunks get an offset past any view (k_left: valid k)
+  __device__ __forceinline__ void load(uint32_t stage, int wv, u32x4 rsrc, int k_left) const {
+    const uint32_t past = kc >= k_left ? 0xffffffffu : 0u;
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) ring_load(stage + (i * 4 + wv) * 1024, rsrc, off[i] | past);
+  }
+  struct Place {
+    uint32_t at, chunk;
+  };
+  static __device__ __forceinline__ Place place(int row0) {
+    const int lane = lane_id(), r = row0 + (lane & 31);
+    return {(uint32_t)(r * BK * 2), (uint32_t)((lane >> 5) ^ swizzle(r))};
+  }
+  static __device__ __forceinline__ bf16x8 frag(const char* stage, const Place& p, int rows, int ks) {
+    return *reinterpret_cast<const bf16x8*>(stage + (p.at + rows * BK * 2 + ((p.chunk ^ (uint32_t)(ks * 2)) << 4)));
+  }
+};
+
 // Source is row-contiguous: element (r, kk) at view[(k0 + kk) * ld + r].  A stage holds BK lines of ROWS elements as they
 // lie in memory; fragments come through the transposing read (see OpOuter).
 template <int ROWS_, int BK>
