@@ -265,11 +265,12 @@ bool launch(GemmArgs a, bool forced, hipStream_t s, int* rc) {
   const long long tiles = ((a.R + BM - 1) / BM + (long long)a.E) * a.n_tiles;  // at most
   // Up to two for each compute unit, all resident at once.  (Tiles, this and the kernels of larger tiles in us: gate/up
   // 320, 14.8 and 19.2; 512, 18.0 and 19.2; 576, 23.3 and 20.5; dgrad-down 288, 18.1 and 23.8; 404, 19.7 and 24.8; 544, 29.2
-  // and 25.3.)  With mostly one tile to an expert the weights bound a launch of any size, and larger tiles are padding
-  // (gate/up, down, dgrad-down and dgrad-gate/up, larger tiles -> this: 64 experts, 2048 <-> 1024, 31 rows each 148, 55, 52,
-  // 101 -> 150, 49, 50, 99, 63 rows each 152, 58, 53, 107 -> 167, 60, 69, 118; 24 experts, 3000 <-> 1200, 50 rows 131, 63,
-  // 45, 98 -> 129, 50, 32, 85; 128 experts, 1024 <-> 256, 31 rows 35, 27, 22, 28 -> 32, 27, 15, 24).
-  const bool few = tiles <= 2ll * moe_compute_units() || a.R <= 48ll * a.E;
+  // and 25.3.)  With one tile to an expert the weights bound a launch of any size, and larger tiles are padding (gate/up,
+  // down, dgrad-down and dgrad-gate/up, larger tiles -> this: 64 experts, 2048 <-> 1024, 31 rows each 148, 55, 52, 101 ->
+  // 150, 49, 50, 99; 37 rows 153, 56, 52, 104 -> 152, 51, 51, 101; 50 rows 154, 56, 52, 107 -> 164, 57, 63, 116, as one expert
+  // or the other then has a second tile; 96 experts, 1536 <-> 640, 42 rows 126, 52, 56, 86 -> 121, 43, 43, 81; 128 experts,
+  // 1024 <-> 256, 31 rows 35, 27, 22, 28 -> 32, 27, 15, 24).
+  const bool few = tiles <= 2ll * moe_compute_units() || a.R <= 40ll * a.E;
   if (!(few || forced) || tiles > 0x7fffff00ll) return false;
   const auto kern = ring_rows_kernel<MODE, BLK>;
   static bool attr_done[MOE_MAX_DEVICES];
