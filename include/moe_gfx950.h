@@ -194,8 +194,8 @@ int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const uint16_t* 
                                            void* stream);
 /* Test hook (no counterpart in the reference).  The four row-ragged products (gate/up, down and
  * their two input gradients) run on 256-row tiles, what is left after whole rounds of them on
- * 128-row tiles where that is shorter, and launches of few tiles on 128-row tiles or 64-row tiles (up to
- * 128 experts, g and u blocked or not kept) throughout.
+ * 128-row tiles where that is shorter, and launches of few tiles on narrower 128-row or on 64-row tiles
+ * (up to 128 experts, g and u blocked or not kept) throughout.
  * moe_gemm_force_row_tile(64, 128 or 256) forces one of them for every later
  * call (64: where there is such a tile), 0 restores the automatic choice; the previous setting is returned.  Process-wide and not
  * synchronised with calls in flight on other host threads.  No result depends on the choice:

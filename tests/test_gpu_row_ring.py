@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
     ([3] * 64 + [100], 72, 264),                   # 65
     ([2, 0, 7, 1] * 32, 128, 64),                  # 128, columns of half a tile
     ([300, 2, 900], 1000, 512),                    # more row tiles than an XCD's share
-], ids=["whole", "least", "edges", "64", "65", "128", "long"])
+    ([513, 511, 0, 900, 1, 640, 384, 513], 1000, 520),   # down and dgrad-gate/up in tiles of 128 rows by themselves
+], ids=["whole", "least", "edges", "64", "65", "128", "long", "tall"])
 def test_row_ring_bits(pkg, lib, counts, H, I):
     print("row ring", len(counts), sum(counts), H, I, flush=True)
     ops = pkg.ops

@@ -3,12 +3,12 @@
 // With a tile or two to a compute unit nothing but a tile's own length counts: a trip to memory for the offsets, one for the
 // first k-tile, the contraction, the epilogue.  Hence small tiles of 64 x 128 (gate and up: 64 columns of each), four waves
 // of 32 rows x 64 columns, and k-tiles of 64 that go straight into a ring of three LDS stages, two on their way;
-// two such workgroups share a compute unit.  A k-tile takes 600 to 700 cycles of mostly LDS traffic (24 KB arriving, 48
-// KB read), where the eight waves of a 128 x 256 tile take 1400 and have their loads one k-tile ahead.
+// two such workgroups share a compute unit.  A k-tile takes 1050 cycles alone and 700 shared (576 of LDS traffic: 24 KB
+// arriving, 48 KB read), where the eight waves of a 128 x 256 tile take 2000 and have their loads one k-tile ahead.
 // 1024 rows of 8 experts, 1024 <-> 512, gate/up, down, dgrad-down and dgrad-gate/up: 18.6, 10.6, 22.0, 17.0 us in
 // tiles of 128 x 256, 11.8, 6.0, 13.3, 10.7 here; 768 rows of 12 experts, 1416 <-> 568: 25.8, 12.8, 29.7, 20.5 and 17.6,
 // 10.6, 18.5, 15.2.  (64 x 128 in five stages, one workgroup to a compute unit: 12.6, 6.7, 13.9, 11.9; 128 x 128 in
-// three: 14.2, 7.9, 17.5, 13.7.)
+// three: 14.2, 7.9, 17.5, 13.7; the next k-tile's first fragments read before the last products: 12.2, 6.5, 13.6, 11.0.)
 #include <type_traits>
 
 #include "gemm_args.h"
@@ -16,10 +16,12 @@
 
 namespace {
 
-constexpr int BM = 64, BN = 128, BK = 64, STAGES = 3, KS = BK / 16, MAX_E = 2 * MOE_WAVE;
+constexpr int BN = 128, BK = 64, KS = BK / 16, MAX_E = 2 * MOE_WAVE;
 
-template <int MODE>
+// FM: a wave's rows / 32
+template <int MODE, int FM>
 struct Operands {
+  static constexpr int BM = 64 * FM, STAGES = FM == 1 ? 3 : 2;
   static constexpr bool DUAL = MODE == GATEUP, B_OUTER = MODE == DGRAD_DOWN || MODE == DGRAD_GATEUP;
   static constexpr int BNC = DUAL ? BN / 2 : BN;  // output columns of a tile
   using OpA = RingInner<BM, BK>;
@@ -32,7 +34,7 @@ struct Operands {
 // A lane's experts `lane` and `lane + 64`: their rows, and the row tiles up to and including theirs.
 struct Experts {
   int first[2], end[2], upto[2], total;
-  __device__ __forceinline__ void init(const int32_t* offs, int E) {
+  __device__ __forceinline__ void init(const int32_t* offs, int E, int bm) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int e = h * MOE_WAVE + lane_id();
@@ -42,19 +44,19 @@ struct Experts {
     total = 0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      upto[h] = total + wave_inclusive((end[h] - first[h] + BM - 1) / BM);
+      upto[h] = total + wave_inclusive((end[h] - first[h] + bm - 1) / bm);
       total = read_lane(upto[h], MOE_WAVE - 1);
     }
   }
 };
 
 // BLK: g and u are kept in blocks, as the other kernels keep them (see there).
-template <int MODE, bool BLK>
+template <int MODE, bool BLK, int FM>
 __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
-  using O = Operands<MODE>;
+  using O = Operands<MODE, FM>;
   using OpA = typename O::OpA;
   using OpB = typename O::OpB;
-  constexpr int BNC = O::BNC, NSEG = MODE == DGRAD_GATEUP ? 2 : 1;
+  constexpr int BM = O::BM, STAGES = O::STAGES, BNC = O::BNC, NSEG = MODE == DGRAD_GATEUP ? 2 : 1;
   constexpr bool DUAL = O::DUAL, B_OUTER = O::B_OUTER;
   extern __shared__ __attribute__((aligned(1024))) char ring[];
   const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE)), wm = wv >> 1, wn = wv & 1;
@@ -62,7 +64,7 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
   // ---- this workgroup's tile: XCD x takes the x-th contiguous eighth of the list, in which the row tiles of an expert
   // over the same columns follow each other
   Experts ex;
-  ex.init(p.offs, p.E);
+  ex.init(p.offs, p.E, BM);
   const int total = ex.total * p.n_tiles, x = blockIdx.x & 7, j = blockIdx.x >> 3, q = total >> 3, r = total & 7;
   if (j >= q + (x < r ? 1 : 0)) return;
   const int tile = x * q + (x < r ? x : r) + j;
@@ -114,14 +116,16 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
   };
 #pragma unroll
   for (int i = 0; i < STAGES - 1; ++i) ask(i < steps);
-  const auto placeA = OpA::place(wm * 32);
+  const auto placeA = OpA::place(wm * 32 * FM);
   const auto placeB = OpB::place(wn * (DUAL ? 32 : 64));
-  f32x16 acc[2];  // 32 rows x 32 columns each: two neighbours, or of gate and up
+  f32x16 acc[FM][2];  // 32 rows x 32 columns each: two neighbours, or of gate and up
 #pragma unroll
-  for (int c = 0; c < 2; ++c)
+  for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[c][v] = 0.f;
-  const bool idle = wm * 32 >= row_end - row0;  // (such a wave only moves its share of the operands)
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][c][v] = 0.f;
+  const bool idle = wm * 32 * FM >= row_end - row0;  // (such a wave only moves its share of the operands)
   for (int s = 0; s < steps; ++s) {
     ring_wait<(STAGES - 2) * O::LOADS>();
     const char *sa = ring + at, *sb = sa + OpA::BYTES;
@@ -130,25 +134,26 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
       ask(s + STAGES - 1 < steps);
       continue;
     }
-    bf16x8 fa[2], fb[2][2];
+    bf16x8 fa[2][FM], fb[2][2];
     const auto read = [&](int u, int ks) {
-      if (u == 2) fa[ks & 1] = OpA::frag(sa, placeA, 0, ks);
+      if (u >= 2) fa[ks & 1][u - 2] = OpA::frag(sa, placeA, (u - 2) * 32, ks);
       else if (DUAL) fb[ks & 1][u] = OpB::frag(sb + u * OpB::BYTES, placeB, 0, ks);
       else fb[ks & 1][u] = OpB::frag(sb, placeB, u * 32, ks);
     };
 #pragma unroll
-    for (int u = 0; u < 3; ++u) read(u, 0);
+    for (int u = 0; u < 2 + FM; ++u) read(u, 0);
     __builtin_amdgcn_sched_barrier(0);
     ask(s + STAGES - 1 < steps);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks & 1][c], fa[ks & 1], acc[c], 0, 0, 0);
+      for (int n = 0; n < 2 * FM; ++n) {
+        const int i = n / 2, c = (i & 1) ? 1 - n % 2 : n % 2;
+        acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks & 1][c], fa[ks & 1][i], acc[i][c], 0, 0, 0);
         if (ks + 1 < KS) {
-          read(c, ks + 1);
-          if (c == 1) read(2, ks + 1);
+          read(n, ks + 1);
+          if (FM == 1 && n == 1) read(2, ks + 1);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -157,7 +162,8 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
   // ---- the epilogue, as in the other kernels: through a strip of the wave's own LDS
   constexpr int WTNC = DUAL ? 32 : 64;
   const int col_w0 = n0 + wn * WTNC, n_cb = (p.N + 31) / 32;
-  const int rows = row_end - row0 - wm * 32;  // the wave's, from its first on
+  const int row_w0 = row0 + wm * 32 * FM, rows = row_end - row_w0;
+  static_assert(FM == 1 || MODE == DOWN || MODE == DGRAD_GATEUP, "one strip of the fused modes");
   const auto gu_block = [&](const void* base, int cb) {
     return (char*)base + ((long long)(first / 32 + e + row / 32 + wm) * n_cb + cb) * 4096 + lane * 16;
   };
@@ -184,13 +190,13 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
     *reinterpret_cast<u32x2*>(strip + l32 * STRIDE + perm(l32, c * 4 + g4) * 16 + lh * 8) = v;
   };
   const auto pack4 = [](float v0, float v1, float v2, float v3) { return u32x2{pack_bf16x2(v0, v1), pack_bf16x2(v2, v3)}; };
-  const auto store_rows = [&](void* base) {
+  const auto store_rows = [&](void* base, int strip_row) {
 #pragma unroll
     for (int it = 0; it < 32 / RPS; ++it) {
       const int rr = it * RPS + lane / CPS, ch = lane % CPS, col = col_w0 + ch * 8;
       const u32x4 v = *reinterpret_cast<const u32x4*>(strip + rr * STRIDE + perm(rr, ch) * 16);
-      if (rr < rows && col < p.N)
-        *reinterpret_cast<u32x4*>((char*)base + ((long long)(row0 + wm * 32 + rr) * ldc + col) * 2) = v;
+      if (strip_row + rr < rows && col < p.N)
+        *reinterpret_cast<u32x4*>((char*)base + ((long long)(row_w0 + strip_row + rr) * ldc + col) * 2) = v;
     }
   };
   if constexpr (MODE == GATEUP) {
@@ -202,8 +208,8 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
       float g[4], u[4], a[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        g[v] = acc[0][4 * g4 + v];
-        u[v] = acc[1][4 * g4 + v];
+        g[v] = acc[0][0][4 * g4 + v];
+        u[v] = acc[0][1][4 * g4 + v];
         a[v] = g[v] * sigmoidf_(g[v]) * u[v];
       }
       put4(0, g4, pack4(a[0], a[1], a[2], a[3]));
@@ -214,7 +220,7 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
         __builtin_nontemporal_store(u32x4{uq[0][0], uq[0][1], uq[1][0], uq[1][1]}, rec + 128 + 64 * (g4 >> 1));
       }
     }
-    store_rows(p.C2);
+    store_rows(p.C2, 0);
   } else if constexpr (MODE == DGRAD_DOWN) {
     float rowdot = 0.f;  // this lane's share of <dact[row,:], act[row,:]>
     u32x2 du4[2][4];
@@ -229,7 +235,7 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
         float dg[4], du[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const float dact = acc[c][4 * g4 + v], sg = sigmoidf_(g[v]), gs = g[v] * sg;  // gs: silu(g)
+          const float dact = acc[0][c][4 * g4 + v], sg = sigmoidf_(g[v]), gs = g[v] * sg;  // gs: silu(g)
           du[v] = dact * gs;
           dg[v] = (dact * u[v]) * (sg + (gs - gs * sg));  // silu'(g) = s + g*s*(1-s)
           rowdot += du[v] * u[v];                         // dact * act
@@ -240,39 +246,35 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
     // one partial per 64 columns and row, every one of them written
     rowdot += __shfl_xor(rowdot, 32, MOE_WAVE);
     if (lh == 0 && l32 < rows && p.C2)
-      reinterpret_cast<float*>(p.C2)[(long long)(col_w0 / 64) * p.R + row0 + wm * 32 + l32] = rowdot;
-    store_rows(p.C0);
+      reinterpret_cast<float*>(p.C2)[(long long)(col_w0 / 64) * p.R + row_w0 + l32] = rowdot;
+    store_rows(p.C0, 0);
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) put4(c, g4, du4[c][g4]);
-    store_rows(p.C1);
+    store_rows(p.C1, 0);
   } else {
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int i = 0; i < FM; ++i) {
+      const f32x16* r = acc[i];
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4)
-        put4(c, g4, pack4(acc[c][4 * g4], acc[c][4 * g4 + 1], acc[c][4 * g4 + 2], acc[c][4 * g4 + 3]));
-    store_rows(p.C0);
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) put4(c, g4, pack4(r[c][4 * g4], r[c][4 * g4 + 1], r[c][4 * g4 + 2], r[c][4 * g4 + 3]));
+      store_rows(p.C0, i * 32);
+    }
   }
 }
 
-template <int MODE, bool BLK>
-bool launch(GemmArgs a, bool forced, hipStream_t s, int* rc) {
-  using O = Operands<MODE>;
+// Launches of at most `most` tiles (by the bound that R and E give), or of any number.
+template <int MODE, bool BLK, int FM>
+bool launch(GemmArgs a, long long most, bool any, hipStream_t s, int* rc) {
+  using O = Operands<MODE, FM>;
   // (dgrad-down's sums cover the columns in steps of 256)
   a.n_tiles = MODE == DGRAD_DOWN ? (a.N + 255) / 256 * 2 : (a.N + O::BNC - 1) / O::BNC;
-  const long long tiles = ((a.R + BM - 1) / BM + (long long)a.E) * a.n_tiles;  // at most
-  // Up to two for each compute unit, all resident at once.  (Tiles, this and the kernels of larger tiles in us: gate/up
-  // 320, 14.8 and 19.2; 512, 18.0 and 19.2; 576, 23.3 and 20.5; dgrad-down 288, 18.1 and 23.8; 404, 19.7 and 24.8; 544, 29.2
-  // and 25.3.)  With one tile to an expert the weights bound a launch of any size, and larger tiles are padding (gate/up,
-  // down, dgrad-down and dgrad-gate/up, larger tiles -> this: 64 experts, 2048 <-> 1024, 31 rows each 148, 55, 52, 101 ->
-  // 150, 49, 50, 99; 37 rows 153, 56, 52, 104 -> 152, 51, 51, 101; 50 rows 154, 56, 52, 107 -> 164, 57, 63, 116, as one expert
-  // or the other then has a second tile; 96 experts, 1536 <-> 640, 42 rows 126, 52, 56, 86 -> 121, 43, 43, 81; 128 experts,
-  // 1024 <-> 256, 31 rows 35, 27, 22, 28 -> 32, 27, 15, 24).
-  const bool few = tiles <= 2ll * moe_compute_units() || a.R <= 40ll * a.E;
-  if (!(few || forced) || tiles > 0x7fffff00ll) return false;
-  const auto kern = ring_rows_kernel<MODE, BLK>;
+  const long long tiles = ((a.R + O::BM - 1) / O::BM + (long long)a.E) * a.n_tiles;
+  if (tiles > (any ? 0x7fffff00ll : most)) return false;
+  const auto kern = ring_rows_kernel<MODE, BLK, FM>;
   static bool attr_done[MOE_MAX_DEVICES];
   const int dev = moe_current_device();
   if (!attr_done[dev]) {
@@ -284,16 +286,34 @@ bool launch(GemmArgs a, bool forced, hipStream_t s, int* rc) {
   return *rc = moe_launch_status(), true;
 }
 
+// Up to two tiles for each compute unit, all resident at once.  (Tiles of 64 rows, this and the kernels of larger tiles in
+// us: gate/up 320, 14.8 and 19.2; 512, 18.0 and 19.2; 576, 23.3 and 20.5; dgrad-down 288, 18.1 and 23.8; 404, 19.7 and
+// 24.8; 544, 29.2 and 25.3.)  With one tile to an expert the weights bound a launch of any size, and larger tiles are
+// padding (gate/up, down, dgrad-down and dgrad-gate/up, larger tiles -> this: 64 experts, 2048 <-> 1024, 31 rows each
+// 148, 55, 52, 101 -> 150, 49, 50, 99; 37 rows 153, 56, 52, 104 -> 152, 51, 51, 101; 50 rows 154, 56, 52, 107 -> 164, 57, 63,
+// 116, as one expert or the other then has a second tile; 96 experts, 1536 <-> 640, 42 rows 126, 52, 56, 86 -> 121, 43, 43,
+// 81; 128 experts, 1024 <-> 256, 31 rows 35, 27, 22, 28 -> 32, 27, 15, 24).
+// Down and dgrad-gate/up, whose epilogues are short, have tiles of 128 rows and two stages for what is too much for 64
+// rows (tiles of 128 rows; down and dgrad-gate/up us: 320 12.4, 19.8 -> 11.2, 17.6; 440 14.5, 22.6 -> 12.5, 19.6; 576
+// 19.0, 29.2 -> 19.5, 31.8).
+template <int MODE, bool BLK>
+bool choose(const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
+  const long long slots = 2ll * moe_compute_units();
+  if (launch<MODE, BLK, 1>(a, slots, forced || a.R <= 40ll * a.E, s, rc)) return true;
+  if constexpr (MODE == DOWN || MODE == DGRAD_GATEUP) return launch<MODE, BLK, 2>(a, slots, false, s, rc);
+  else return false;
+}
+
 }  // namespace
 
 bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
   if (a.E > MAX_E) return false;
   switch (mode) {
     case GATEUP:
-      if (blocked) return launch<GATEUP, true>(a, forced, s, rc);
-      return !a.C0 && launch<GATEUP, false>(a, forced, s, rc);  // (g and u in rows: not here)
-    case DOWN: return launch<DOWN, false>(a, forced, s, rc);
-    case DGRAD_DOWN: return blocked && launch<DGRAD_DOWN, true>(a, forced, s, rc);
-    default: return launch<DGRAD_GATEUP, false>(a, forced, s, rc);
+      if (blocked) return choose<GATEUP, true>(a, forced, s, rc);
+      return !a.C0 && choose<GATEUP, false>(a, forced, s, rc);  // (g and u in rows: not here)
+    case DOWN: return choose<DOWN, false>(a, forced, s, rc);
+    case DGRAD_DOWN: return blocked && choose<DGRAD_DOWN, true>(a, forced, s, rc);
+    default: return choose<DGRAD_GATEUP, false>(a, forced, s, rc);
   }
 }
