@@ -28,7 +28,7 @@
 // as they lie in memory and read through the transposing LDS read of gfx950.
 // Workgroups are numbered so that each XCD (own L2) works on a contiguous range of tiles,
 // i.e. on its own experts' weights.
-#include "gemm_args.h"
+#include "row_ring.h"
 #include "tile_ops.h"
 
 namespace {
@@ -842,6 +842,11 @@ __device__ __forceinline__ Sweep sweep_of(int n) {
 //   16384 rows of 8 experts, 1024 <-> 512    54 -> 48, 32 -> 29, 40 (0.53 rounds, 264 halves), 53 -> 48
 //   9999 rows of 12 experts, 1416 <-> 568    40 (0.9), 36 -> 29, 49 -> 36 (0.53 rounds, 252 halves), 61 -> 47
 // From some ten rounds on it makes no difference.
+// Up to a quarter of a round left is done in quarters of 64 x 256 instead, at most one to a workgroup, through the ring of
+// direct loads (csrc/row_ring.h): a short round waits for memory k-tile by k-tile, and the ring has two of them
+// on their way.  16384 rows of 8 experts as above: 55, 32, 45, 52 -> 52, 30, 44, 48 us; 18000 rows of 4, 1024 <-> 1024,
+// gate/up 55 -> 52; 14000 rows of 12, 1536 <-> 640, gate/up 77 -> 72.  (The same quarters with the staging registers of
+// the other tiles: two thirds of that.)
 template <int MODE, typename OutT, bool BLK>
 __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gemm_kernel(const GemmArgs p) {
   static_assert(CfgHalf::NT == CfgMain::NT, "one workgroup runs both");
@@ -850,19 +855,21 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   __shared__ int tile_start[GEMM_MAX_E + 1], offs[GEMM_MAX_E + 1];
   __shared__ uint32_t half_list[MAX_LISTED];
-  __shared__ int wave_halves[2][WAVES];
+  __shared__ int wave_halves[3][WAVES];
   number_tiles<ROW_TILE>(p, tile_start, offs);
   const int nb = gridDim.x;
   const int total = __builtin_amdgcn_readfirstlane(tile_start[p.E]) * p.n_tiles;
   int whole = total;  // tiles 0 .. whole are done whole
-  int halves = 0;     // halves with rows of the others
+  int halves = 0;     // halves with rows of the others, or quarters
+  bool quarters = false;
   const int left = total % nb;
+  const bool can_quarter = BLK || MODE == DOWN || MODE == DGRAD_GATEUP || (MODE == GATEUP && !p.C0);  // (g and u in rows: not)
   if (!p.whole_only && left > 0 && nb <= MAX_LISTED) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int round = total > nb && 2 * nb <= MAX_LISTED ? nb : 0;  // (of whole tiles that may be halved too)
     const int tile = total - left - round + (int)threadIdx.x;
     const bool last = tile >= total - left;
-    int n = 0;
+    int n = 0, n4 = 0;  // this tile's halves and quarters with rows
     if (tile < total) {
       const int slot = tile / p.n_tiles;
       int e = 0, hi = p.E;
@@ -871,33 +878,51 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
         if (tile_start[mid] <= slot) e = mid;
         else hi = mid;
       }
-      n = offs[e + 1] - offs[e] - (slot - tile_start[e]) * ROW_TILE > CfgHalf::BM ? 2 : 1;
+      const int rows = offs[e + 1] - offs[e] - (slot - tile_start[e]) * ROW_TILE;
+      n = rows > CfgHalf::BM ? 2 : 1;
+      n4 = last && can_quarter ? ((rows < ROW_TILE ? rows : ROW_TILE) + 63) / 64 : 0;
     }
     const unsigned long long some = __ballot(n > 0), both = __ballot(n > 1), in_last = __ballot(last);
     const unsigned long long below = (1ull << lane) - 1;
+    int at4 = 0, all4 = 0;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const unsigned long long b = __ballot(n4 > h);
+      at4 += __popcll(b & below), all4 += __popcll(b);
+    }
     if (lane == 0) {
       wave_halves[0][wv] = __popcll(some) + __popcll(both);
       wave_halves[1][wv] = __popcll(some & in_last) + __popcll(both & in_last);
+      wave_halves[2][wv] = all4;
     }
     __syncthreads();
     int at = __popcll(some & below) + __popcll(both & below), all = 0, in_left = 0;
+    all4 = 0;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       const int c = __builtin_amdgcn_readfirstlane(wave_halves[0][w]);
       at += w < wv ? c : 0;
       all += c;
       in_left += __builtin_amdgcn_readfirstlane(wave_halves[1][w]);
+      const int c4 = __builtin_amdgcn_readfirstlane(wave_halves[2][w]);
+      at4 += w < wv ? c4 : 0;
+      all4 += c4;
     }
     int skip = 0;  // halves of the round before, when that stays whole
     if (round > 0 && all <= 2 * nb) {
       halves = all;
       whole = total - left - round;
+    } else if (can_quarter && all4 <= nb) {
+      halves = all4;
+      whole = total - left;
+      quarters = true;
+      for (int h = 0; h < n4; ++h) half_list[at4 + h] = 4u * (uint32_t)tile + h;
     } else if (in_left <= nb) {
       halves = in_left;
       whole = total - left;
       skip = all - in_left;
     }
-    if (tile >= whole)
+    if (tile >= whole && !quarters)
       for (int h = 0; h < n; ++h) half_list[at + h - skip] = 2u * (uint32_t)tile + h;
   }
   const Sweep s = sweep_of(whole);
@@ -905,6 +930,27 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
   if (halves == 0) return;
   __syncthreads();  // (the operand stages are free, the list is complete)
   const Sweep h = sweep_of(halves);
+  if constexpr (BLK || MODE != DGRAD_DOWN) {
+    if (quarters) {
+      using Quarter = RingTile<MODE, 1, CfgMain::NT / MOE_WAVE>;
+      static_assert(Quarter::LDS <= lds_bytes<MODE, CfgMain>() && Quarter::BM * 4 == ROW_TILE, "fits");
+      for (int at = h.first; at < h.end; at += h.step) {
+        const int entry = __builtin_amdgcn_readfirstlane((int)half_list[at]), tile = entry >> 2, slot = tile / p.n_tiles;
+        int e = 0, hi = p.E;
+        while (hi - e > 1) {
+          const int mid = (e + hi) >> 1;
+          if (tile_start[mid] <= slot) e = mid;
+          else hi = mid;
+        }
+        e = __builtin_amdgcn_readfirstlane(e);
+        const int first = __builtin_amdgcn_readfirstlane(offs[e]), end = __builtin_amdgcn_readfirstlane(offs[e + 1]);
+        const int row = (slot - __builtin_amdgcn_readfirstlane(tile_start[e])) * ROW_TILE + (entry & 3) * Quarter::BM;
+        ring_tile<MODE, BLK, 1, WAVES>(p, (char*)smem, e, first, end, row, tile % p.n_tiles * Quarter::BNC);
+        __syncthreads();
+      }
+      return;
+    }
+  }
   walk_tiles<MODE, CfgHalf, OutT, BLK>(p, smem, tile_start, offs, half_list, h.first, h.end, h.step);
 }
 

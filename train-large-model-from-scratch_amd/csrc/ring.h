@@ -1,4 +1,4 @@
-// Operand tiles that go from memory straight into a ring of LDS stages (buffer_load .. lds), for workgroups of four
+// Operand tiles that go from memory straight into a ring of LDS stages (buffer_load .. lds), for workgroups of WAVES
 // waves: no staging registers, no LDS stores, and as many steps on their way as the ring has stages.  A wave-wide load
 // fills 1 KB of consecutive LDS, so a stage has no padding; 16-byte chunks are permuted on the way instead, so that
 // the fragment reads find different banks (no conflicts by SQ_LDS_BANK_CONFLICT).
@@ -32,14 +32,14 @@ __device__ __forceinline__ uint32_t lds_address(const char* p) {
 
 // Source is k-contiguous: element (r, kk) at view[r * ld + k0 + kk].  A stage holds ROWS rows of BK elements; fragments are
 // 16-byte reads.
-template <int ROWS_, int BK>
+template <int ROWS_, int BK, int WAVES = 4>
 struct RingInner {
   static constexpr int ROWS = ROWS_;
   static constexpr int CPR = BK / 8;  // 16-byte chunks per row
   static constexpr int BYTES = ROWS * BK * 2;
   static constexpr int RPP = 64 / CPR;  // rows per wave-wide load
-  static constexpr int PER_WAVE = BYTES / 4096;
-  static_assert(BYTES % 4096 == 0 && CPR == 8, "four waves, rows of 128 bytes");
+  static constexpr int PER_WAVE = BYTES / (WAVES * 1024);
+  static_assert(BYTES % (WAVES * 1024) == 0 && CPR == 8, "whole loads, rows of 128 bytes");
   static __device__ __forceinline__ int swizzle(int row) { return (row >> 1) & 7; }
   uint32_t off[PER_WAVE];  // byte offsets of this lane's chunks in the view
   int kc;                  // first k of its chunks
@@ -47,13 +47,13 @@ struct RingInner {
     const int lane = lane_id(), r = lane / CPR;
     kc = ((lane % CPR) ^ swizzle(wv * RPP + r)) * 8;
 #pragma unroll
-    for (int i = 0; i < PER_WAVE; ++i) off[i] = (uint32_t)(((i * 4 + wv) * RPP + r) * ld + kc) * 2;
+    for (int i = 0; i < PER_WAVE; ++i) off[i] = (uint32_t)(((i * WAVES + wv) * RPP + r) * ld + kc) * 2;
   }
   // k past the end of the contraction lies in the next row: such chunks get an offset past any view (k_left: valid k)
   __device__ __forceinline__ void load(uint32_t stage, int wv, u32x4 rsrc, int k_left) const {
     const uint32_t past = kc >= k_left ? 0xffffffffu : 0u;
 #pragma unroll
-    for (int i = 0; i < PER_WAVE; ++i) ring_load(stage + (i * 4 + wv) * 1024, rsrc, off[i] | past);
+    for (int i = 0; i < PER_WAVE; ++i) ring_load(stage + (i * WAVES + wv) * 1024, rsrc, off[i] | past);
   }
   struct Place {
     uint32_t at, chunk;
@@ -69,14 +69,14 @@ struct RingInner {
 
 // Source is row-contiguous: element (r, kk) at view[(k0 + kk) * ld + r].  A stage holds BK lines of ROWS elements as they
 // lie in memory; fragments come through the transposing read (see OpOuter).
-template <int ROWS_, int BK>
+template <int ROWS_, int BK, int WAVES = 4>
 struct RingOuter {
   static constexpr int ROWS = ROWS_;
   static constexpr int CPL = ROWS / 8;  // 16-byte chunks per line
   static constexpr int BYTES = ROWS * BK * 2;
   static constexpr int LPP = 64 / CPL;  // lines per wave-wide load
-  static constexpr int PER_WAVE = BYTES / 4096;
-  static_assert(BYTES % 4096 == 0 && ROWS % 128 == 0 && ROWS <= 256, "four waves, lines of 16 or 32 chunks");
+  static constexpr int PER_WAVE = BYTES / (WAVES * 1024);
+  static_assert(BYTES % (WAVES * 1024) == 0 && ROWS % 128 == 0 && ROWS <= 256, "whole loads, lines of 16 or 32 chunks");
   // Half a wave's transposing read covers 64 bytes of each of four lines: they lie in different quarters of the 64 banks.
   static __device__ __forceinline__ int swizzle(int line) { return 4 * (line & 3); }
   uint32_t off[PER_WAVE];  // byte offsets of this lane's chunks in the view
@@ -84,13 +84,13 @@ struct RingOuter {
     const int lane = lane_id();
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) {
-      const int line = (i * 4 + wv) * LPP + lane / CPL;
+      const int line = (i * WAVES + wv) * LPP + lane / CPL;
       off[i] = (uint32_t)(line * ld + ((lane % CPL) ^ swizzle(line)) * 8) * 2;
     }
   }
   __device__ __forceinline__ void load(uint32_t stage, int wv, u32x4 rsrc) const {
 #pragma unroll
-    for (int i = 0; i < PER_WAVE; ++i) ring_load(stage + (i * 4 + wv) * 1024, rsrc, off[i]);
+    for (int i = 0; i < PER_WAVE; ++i) ring_load(stage + (i * WAVES + wv) * 1024, rsrc, off[i]);
   }
   // A lane's place in the fragments of rows row0 .. row0 + 31, + 32, ...
   struct Place {
