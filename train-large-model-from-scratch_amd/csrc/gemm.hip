@@ -954,8 +954,8 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
   walk_tiles<MODE, CfgHalf, OutT, BLK>(p, smem, tile_start, offs, half_list, h.first, h.end, h.step);
 }
 
-// All in half tiles: launches of so few tiles that there is nothing to decide (4096 rows of 8 experts, 1024 <-> 512,
-// gate/up and down 17.4 and 11.6 us; through the kernel above 18.6 and 12.5).
+// All in half tiles: launches of so few tiles that there is nothing to decide and that csrc/row_ring.hip does not take (4096 rows
+// of 8 experts, 1024 <-> 512, gate/up 19.5 us; in ring tiles of 64 rows, a few more than fit at once, 23.3).
 template <int MODE, typename OutT, bool BLK>
 __global__ __launch_bounds__(CfgHalf::NT, CfgHalf::WAVES_PER_SIMD) void small_rows_gemm_kernel(const GemmArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
