@@ -363,7 +363,7 @@ typedef struct {
   int32_t* ids;           /* [R]; written from the logits or ids64 */
   float* gates;           /* [R]; written from the logits; NULL without them: all ones */
   int32_t *counts, *offs, *pos_to_row, *row_to_pos;
-  int32_t* bad_ids;       /* [1] or NULL */
+  int32_t* bad_ids;       /* [1] or NULL: receives the number of ids outside [0,E), 0 where the logits decide */
   uint16_t* xp;           /* [R,H] kept */
   void* gu;               /* moe_gu_blocked_bytes(R, E, I) kept, or NULL: g and u are not written */
   uint16_t* act;          /* [R,I] kept */

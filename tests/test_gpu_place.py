@@ -54,3 +54,25 @@ def test_places(pkg, lib, T, E, k, H, dtype):
     nan = torch.isnan(want)
     assert torch.equal(nan, torch.isnan(out))
     assert ((out.float() - want)[~nan].abs() <= rel * (want[~nan].abs() + 1e-3)).all()
+
+
+# (two launches, chunks of 8 and of 16 tokens; more experts than they take: the general path; no tokens)
+@pytest.mark.parametrize("T,E", [(100, 8), (2100, 8), (100, 136), (0, 8)])
+def test_the_count_of_bad_ids_is_written_with_logits(pkg, lib, T, E):
+    """The C entry, which takes the pointer also where the experts come from the logits: 0, whichever launches run."""
+    print("bad ids", T, E, flush=True)
+    ops, H, I, k = pkg.ops, 64, 32, 2
+    r = lambda *s: torch.randn(*s, device="cuda").to(torch.bfloat16)
+    i32 = lambda n: torch.empty(n, dtype=torch.int32, device="cuda")
+    n = max(T, 1)  # (no tokens: pointers all the same)
+    x, logits, w1, w3, w2, out = r(n, H), r(n, E), r(E, I, H), r(E, I, H), r(E, H, I), r(n, H)
+    ids, gates, counts, offs, p2r, r2p = i32(n * k), i32(n * k), i32(E), i32(E + 1), i32(n * k), i32(n * k)
+    bad = torch.full((1,), 7, dtype=torch.int32, device="cuda")
+    xp, act = r(n * k, H), r(n * k, I)
+    scratch = torch.empty(max(lib.cdll.moe_layer_scratch_bytes(T, H, E, I, k, 0), 256), dtype=torch.uint8, device="cuda")
+    p = lambda t: t.data_ptr()
+    bf16 = pkg.lib.DT_BF16
+    lib.call_layer("moe_layer_forward", ops._FORWARD_ARGS.pack(
+        T, H, E, I, k, p(x), bf16, p(logits), bf16, 0, 0, p(w1), p(w3), p(w2), 0, p(out), bf16, p(ids), p(gates),
+        p(counts), p(offs), p(p2r), p(r2p), p(bad), p(xp), 0, p(act), p(scratch), scratch.numel()), ops._stream())
+    assert bad.item() == 0 and counts.sum().item() == T * k

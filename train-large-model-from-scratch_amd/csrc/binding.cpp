@@ -28,8 +28,8 @@ int64_t moe_place_bytes(int64_t T, int64_t E);
 int moe_select_count(const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t E, int64_t k,
                      int32_t* ids, float* gates, void* table, void* stream);
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
-                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, void* xp,
-                   int xp_dtype, void* stream);
+                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
+                   void* xp, int xp_dtype, void* stream);
 int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
                    int64_t I, float* g, float* u, float* act, void* stream);
 int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
@@ -644,8 +644,8 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
   }
   if (place) {
     CALL(moe_select_count, logits.data_ptr(), (int)dt(logits), (const float*)ptr(b), T, E, k, ids, gates, ws.data_ptr(), s);
-    CALL(moe_place_rows, x.data_ptr<float>(), MOE_DT_F32, ids, ws.data_ptr(), T, H, E, k, counts, offs, p2r, r2p, xp,
-         MOE_DT_F32, s);
+    CALL(moe_place_rows, x.data_ptr<float>(), MOE_DT_F32, ids, ws.data_ptr(), T, H, E, k, counts, offs, p2r, r2p,
+         nullptr, xp, MOE_DT_F32, s);
   } else {
     int32_t* bad = nullptr;
     Tensor given;

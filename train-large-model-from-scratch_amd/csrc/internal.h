@@ -50,12 +50,12 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
 bool moe_place_ok(int64_t T, int64_t E, int64_t k);
 int64_t moe_place_bytes(int64_t T, int64_t E);
 // moe_router_topk_fwd that leaves the table, and from it the results of moe_histogram_scan and moe_permute_fwd (fp32 rows
-// where x is fp32 and xp_dtype says so).
+// where x is fp32 and xp_dtype says so); *bad_ids, unless NULL, becomes 0.
 int moe_select_count(const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t E, int64_t k,
                      int32_t* ids, float* gates, void* table, void* stream);
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
-                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, void* xp,
-                   int xp_dtype, void* stream);
+                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
+                   void* xp, int xp_dtype, void* stream);
 
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;

@@ -146,7 +146,7 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   }
   if (place) {
     MOE_STEP("moe_place_rows", moe_place_rows(x, x_dtype, ids, ws + c.dispatch, T, H, E, k, counts, offs, pos_to_row,
-                                              row_to_pos, xp, MOE_DT_BF16, stream));
+                                              row_to_pos, nullptr, xp, MOE_DT_BF16, stream));
   } else {
     MOE_STEP("moe_histogram_scan_checked",
              moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
@@ -327,7 +327,7 @@ extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) 
     MOE_STEP("moe_select_count", moe_select_count(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids, a->gates,
                                                   ws.dispatch, stream));
     MOE_STEP("moe_place_rows", moe_place_rows(a->x, (int)a->x_dtype, a->ids, ws.dispatch, T, H, E, k, a->counts, a->offs,
-                                              a->pos_to_row, a->row_to_pos, a->xp, MOE_DT_BF16, stream));
+                                              a->pos_to_row, a->row_to_pos, a->bad_ids, a->xp, MOE_DT_BF16, stream));
   } else {
     if (a->logits)
       MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids,

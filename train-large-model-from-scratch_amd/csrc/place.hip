@@ -62,7 +62,7 @@ template <typename XT, typename OT, int CHUNK, int WAVES>
 __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     const XT* __restrict__ x, const int32_t* __restrict__ ids, const uint32_t* __restrict__ table, int T, int E, int k,
     int H, int shift, int32_t* __restrict__ counts, int32_t* __restrict__ offs, int32_t* __restrict__ pos_to_row,
-    int32_t* __restrict__ row_to_pos, OT* __restrict__ xp) {
+    int32_t* __restrict__ row_to_pos, int32_t* __restrict__ bad_ids, OT* __restrict__ xp) {
   __shared__ int below[PLACE_EXPERTS], total[PLACE_EXPERTS];  // of earlier chunks, of all
   __shared__ uint32_t asked[PLACE_EXPERTS];
   constexpr int AHEAD = 4;  // 8-element pieces of the row requested at once
@@ -127,6 +127,7 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     if (lane < E) counts[lane] = n0, offs[lane] = upto0 - n0;
     if (MOE_WAVE + lane < E) counts[MOE_WAVE + lane] = n1, offs[MOE_WAVE + lane] = upto1 - n1;
     if (lane == 0) offs[E] = T * k;
+    if (lane == 0 && bad_ids) *bad_ids = 0;  // (a selection asks for no other experts)
   }
   const int first0 = __shfl(upto0 - n0, my_id & 63, MOE_WAVE), first1 = __shfl(upto1 - n1, my_id & 63, MOE_WAVE);
   int pos = 0;
@@ -183,8 +184,8 @@ int moe_select_count(const void* logits, int logits_dtype, const float* bias, in
 }
 
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
-                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, void* xp,
-                   int xp_dtype, void* stream) {
+                   int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
+                   void* xp, int xp_dtype, void* stream) {
   if (H <= 0 || H % 8 != 0) return MOE_ERR_SHAPE;
   if (H > 65536) return MOE_ERR_LIMIT;
   if (x_dtype == MOE_DT_BF16 && xp_dtype != MOE_DT_BF16) return MOE_ERR_DTYPE;
@@ -197,7 +198,7 @@ int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* t
     constexpr int CHUNK = decltype(chunk)::value, WAVES = decltype(waves)::value;
     hipLaunchKernelGGL((place_rows_kernel<XT, OT, CHUNK, WAVES>), dim3((unsigned)((T + WAVES - 1) / WAVES)),
                        dim3(WAVES * MOE_WAVE), 0, s, (const XT*)x, ids, (const uint32_t*)table, (int)T, (int)E, (int)k,
-                       (int)H, shift, counts, offs, pos_to_row, row_to_pos, (OT*)xp);
+                       (int)H, shift, counts, offs, pos_to_row, row_to_pos, bad_ids, (OT*)xp);
     return moe_launch_status();
   };
   const auto of = [&](auto chunk, auto waves) {
