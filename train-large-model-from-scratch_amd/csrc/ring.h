@@ -16,10 +16,15 @@ __device__ __forceinline__ u32x4 ring_rsrc(const View& w, long long byte_off, bo
   return u32x4{(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, (uint32_t)left, 0x00020000u};
 }
 // 16 bytes per lane from `off` into LDS at lds_byte + 16 * lane.  In assembly because the compiler would wait for every
-// such load before any LDS read that follows; the waits are ring_wait's.
+// such load before any LDS read that follows; the waits are ring_wait's.  The load takes its LDS address from m0, which is
+// written here and declared so: the compiler, which reserves m0, writes it anew for an instruction of its own that reads it.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (a reserved register on the list, which is the point)
 __device__ __forceinline__ void ring_load(uint32_t lds_byte, u32x4 rsrc, uint32_t off) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds_byte));
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds_byte)
+               : "m0");
 }
+#pragma clang diagnostic pop
 // All but the wave's N youngest loads have arrived and its LDS reads are done; then meet the other waves, for whose loads
 // and reads the same holds.
 template <int N>
