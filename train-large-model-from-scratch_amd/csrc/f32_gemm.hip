@@ -540,14 +540,15 @@ using LargeQuarter = Shape<64, 64, 16, 2, 2, 2>;
 int forced_tile = 0;
 // The large tile has half the operand traffic and LDS reads per flop (32768 rows of 8 experts, 2048 <-> 1024, gate and up: 1.99
 // against 2.17 ms, 138 TFLOP/s), but few of them share a compute unit less evenly (8192 rows of 16 experts, 1024 <-> 1024, five
-// rounds of large tiles: 335 against 295 us; three rounds: equal): from eight rounds on.  A weight gradient's operands are
-// both read from LDS a value at a time, which the large tile halves (three stacks of 1024 x 512, 4096 rows of 8 experts, three
-// rounds: 120 against 126 us; 4096 rows of 16 experts, six rounds: 123 against 134; 1.5 rounds of 512 x 512: 60
-// against 58): from three rounds on.
-constexpr int ROW_ROUNDS = 8, WGRAD_ROUNDS = 3;
-bool large_tiles(int64_t tiles128, int rounds) {
+// rounds of large tiles: 335 against 295 us; three rounds: equal): from eight rounds on.  So, too, for weight gradients,
+// where a tile takes as long as its expert has rows.  From three to eight rounds the large one is faster by a tenth
+// where a router with random weights deals the rows (4096 rows of 8 experts, three stacks of 1024 x 512, three rounds: 120 us
+// against 126), and slower where it does not: with logits off by 0.3 from expert to expert by 0.90 to 1.03 on average and down to 0.42
+// (16384 rows of 128 experts, 256 x 128: 220 us against 92), with Zipf's shares by 0.67 to 0.81 and down to 0.31.  From eight rounds
+// on: 1.04, 1.08 and 1.03 times as fast.
+bool large_tiles(int64_t tiles128) {
   if (forced_tile) return forced_tile == 128;
-  return tiles128 >= rounds * (int64_t)moe_compute_units();
+  return tiles128 >= 8 * (int64_t)moe_compute_units();
 }
 
 int check_rows(int64_t E, int64_t R, int64_t N, int64_t K) {
@@ -564,7 +565,7 @@ int launch_rows(RowsArgs a, int64_t E, int64_t R, int64_t N, int64_t K, hipStrea
   a.E = (int)E, a.R = (int)R, a.N = (int)N, a.K = (int)K;
   const int cus = moe_compute_units();
   const auto tiles = [&](int64_t t) { return (R / t + E) * ((N * (MODE == GATEUP ? 2 : 1) + t - 1) / t); };  // at most
-  if (large_tiles(tiles(128), ROW_ROUNDS))
+  if (large_tiles(tiles(128)))
     hipLaunchKernelGGL((f32_rows_kernel<MODE, Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, s, a, cus);
   else
     hipLaunchKernelGGL((f32_rows_kernel<MODE, Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, s, a, cus);
@@ -654,7 +655,7 @@ static int wgrads(const F32Stack* s, int n, const int32_t* offs, int64_t E, int6
   }
   if (tiles(64) > 0x70000000ll) return MOE_ERR_LIMIT;
   const int cus = moe_compute_units();
-  if (large_tiles(tiles(128), WGRAD_ROUNDS))
+  if (large_tiles(tiles(128)))
     hipLaunchKernelGGL((f32_wgrad_kernel<Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, st, p, cus);
   else
     hipLaunchKernelGGL((f32_wgrad_kernel<Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, st, p, cus);
