@@ -113,11 +113,17 @@ def _gemm_case(P, counts, N, K):
     [(37 * i) % 90 for i in range(65)],              # one more than are sorted
     [400] + [3] * 129,                               # three words of experts, dealt
     [130] * 5,                                       # even: not dealt
-], ids=["64", "8", "65", "130", "even"])
+    # as many rows an expert that the kernel looks at the offsets:
+    [7] * 63 + [16000],                              # 64 experts, all but one tied, the largest last
+    [0, 300, 0, 300, 2000, 300, 0, 1],               # ties, empty experts
+    [9000] + [(53 * i) % 300 for i in range(64)],    # one more than are sorted
+    [9000] + [190] * 129,                            # three words of experts
+    [700, 650, 500],                                 # even enough: not dealt
+], ids=["64", "8", "65", "130", "even", "64 dealt", "8 dealt", "65 dealt", "130 dealt", "3 even"])
 @pytest.mark.parametrize("tile", [64, 128])
 def test_f32_weight_gradients_of_uneven_experts(P, counts, tile):
     """Three stacks in one launch, the largest experts' tiles first and dealt to all XCDs: every tile of every
-    expert once.  Sums of at most 900 products in fp32: the bar of this file."""
+    expert once.  Sums of at most 16000 products in fp32: the bar of this file."""
     E, R, H, I = len(counts), int(sum(counts)), 260, 132
     _say("f32 wgrads", E, R, "tile", tile)
     offs = _offsets(counts)

@@ -476,12 +476,15 @@ __device__ __forceinline__ int lane_of_rank(int n, int largest, int e) {
   return __builtin_ctzll(__ballot(n == value & before == place));
 }
 
-// A tile costs what its expert has rows.  Tiles go stack by stack and expert by expert, an eighth of the list for each XCD, which
-// gives it parts of three different experts; but where one expert has more than 5/4 of the mean they go expert by expert, up to
-// 64 experts the largest first, and are dealt to all XCDs, an eighth of a stack's at a time.  (4096 rows of 8 experts, three
-// stacks of 1024 x 512, half the rows in one expert: 205 us the first way, 167 dealt; 8192 rows of 24 experts: 135 and 82;
-// even experts: 120 and 122.)
-template <typename S, typename Q>
+// Tiles go stack by stack and expert by expert, an eighth of the list for each XCD, which gives it the tiles of 3/8 of the
+// experts.  A tile costs what its expert has rows, so that an XCD with a heavy expert keeps the others waiting: where
+// it gets more by that than 1/8 of its share, the tiles go expert by expert, up to 64 experts the largest first,
+// and are dealt to all XCDs, an eighth of a stack's at a time.  (Shares with a heavy expert from there on gain: 1/8
+// to 3/8 more 1.09 to 1.12 times as fast, more 1.2 to 1.6; below it what dealing costs the L2s is more than it gives,
+// 0.93 to 0.98.  4096 rows of 8 experts by Zipf's shares, three stacks of 1024 x 512: 221 -> 111 us; even 107 and 107.)
+// DEAL: without it the offsets of all experts are not looked at, which costs a workgroup a trip to memory before it
+// can begin (2000 rows of 128 experts, 256 x 256: 32 us without and 40 with).
+template <typename S, typename Q, bool DEAL>
 __global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs p, int cus) {
   __shared__ __align__(16) float lds[larger(WgradLoop<S>::LDS_FLOATS, WgradLoop<Q>::LDS_FLOATS)];
   int per_e[3], n_col[3], per = 0;
@@ -499,12 +502,17 @@ __global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs
     first = b;
     return end - b;
   };
-  const int lane = threadIdx.x & 63;
-  int first, rows = rows_of(lane, first);
+  int first = 0, rows = 0;  // DEAL: of the lane's expert
   bool uneven = false;
-  for (int e0 = 0; e0 < p.E; e0 += MOE_WAVE) {
-    int at;
-    uneven |= __ballot(4ll * p.E * rows_of(e0 + lane, at) > 5ll * p.R) != 0;
+  if constexpr (DEAL) {
+    const int lane = threadIdx.x & 63;
+    const auto heavy = [&](int n) { return 64ll * ((long long)n * p.E - p.R) > (long long)p.n * p.E * p.R; };
+    rows = rows_of(lane, first);
+    uneven = __ballot(heavy(rows)) != 0;
+    for (int e0 = MOE_WAVE; e0 < p.E; e0 += MOE_WAVE) {
+      int at;
+      uneven |= __ballot(heavy(rows_of(e0 + lane, at))) != 0;
+    }
   }
   const Job job = job_of(per * p.E, cus, uneven ? larger(per_e[0] / 8, 1) : 0);
   if (job.tile < 0) return;
@@ -518,8 +526,13 @@ __global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs
     }
   int e = uneven ? job.tile / per : tile / pe;
   tile %= pe;
-  if (uneven && p.E <= MOE_WAVE) e = lane_of_rank(rows, p.R, e);
-  rows = rows_of(e, first);
+  if (DEAL && p.E <= MOE_WAVE) {
+    if (uneven) e = lane_of_rank(rows, p.R, e);
+    first = read_lane(first, e);
+    rows = read_lane(rows, e);
+  } else {
+    rows = rows_of(e, first);
+  }
   const int b = uniform(first), end = b + uniform(rows);
   const F32Stack s = p.s[w];
   int m0 = tile / nc * S::BM, n0 = tile % nc * S::BN;
@@ -655,10 +668,20 @@ static int wgrads(const F32Stack* s, int n, const int32_t* offs, int64_t E, int6
   }
   if (tiles(64) > 0x70000000ll) return MOE_ERR_LIMIT;
   const int cus = moe_compute_units();
-  if (large_tiles(tiles(128)))
-    hipLaunchKernelGGL((f32_wgrad_kernel<Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, st, p, cus);
-  else
-    hipLaunchKernelGGL((f32_wgrad_kernel<Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, st, p, cus);
+  const bool large = large_tiles(tiles(128));
+  const auto go = [&](auto deal) {
+    constexpr bool DEAL = decltype(deal)::value;
+    if (large)
+      hipLaunchKernelGGL((f32_wgrad_kernel<Large, LargeQuarter, DEAL>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, st, p, cus);
+    else
+      hipLaunchKernelGGL((f32_wgrad_kernel<Small, Quarter, DEAL>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, st, p, cus);
+  };
+  // Times as fast with a look at the offsets as without, up to 64 experts, even loads and loads with a heavy expert: tiles of
+  // 64, below 32 rows an expert 0.86 to 0.91, 0.87 to 1.0;
+  // 64 to 128 rows 0.94, 1.25; 128 to 256 rows 0.98, 1.35; more 0.99, 1.45.  Tiles of 128: below 64 rows 0.91 to 0.97, 1.03 to
+  // 1.13; 64 to 128 rows 0.98, 1.19; more 0.99, 1.3.  Of 128 experts, which are not sorted, 128 rows each: 0.95, 1.1.
+  if (R >= (E > MOE_WAVE ? 256 : large ? 64 : 128) * E) go(std::true_type{});
+  else go(std::false_type{});
   return moe_launch_status();
 }
 
