@@ -842,11 +842,14 @@ __device__ __forceinline__ Sweep sweep_of(int n) {
 //   16384 rows of 8 experts, 1024 <-> 512    54 -> 48, 32 -> 29, 40 (0.53 rounds, 264 halves), 53 -> 48
 //   9999 rows of 12 experts, 1416 <-> 568    40 (0.9), 36 -> 29, 49 -> 36 (0.53 rounds, 252 halves), 61 -> 47
 // From some ten rounds on it makes no difference.
-// Up to a quarter of a round left is done in quarters of 64 x 256 instead, at most one to a workgroup, through the ring of
-// direct loads (csrc/row_ring.h): a short round waits for memory k-tile by k-tile, and the ring has two of them
-// on their way.  16384 rows of 8 experts as above: 55, 32, 45, 52 -> 52, 30, 44, 48 us; 18000 rows of 4, 1024 <-> 1024,
-// gate/up 55 -> 52; 14000 rows of 12, 1536 <-> 640, gate/up 77 -> 72.  (The same quarters with the staging registers of
-// the other tiles: two thirds of that.)
+// Except in dgrad-down, what is left is done in quarters of 64 x 256 instead where that is at most one with rows to every
+// workgroup (a quarter of a round, or a round of tiles with up to 64 rows), through the ring of direct loads
+// (csrc/row_ring.h): a short round waits for memory k-tile by k-tile, and the ring has two of them on their way.  Halves ->
+// quarters, gate/up, down and dgrad-gate/up: 16384 rows of 8 experts as above 55, 32, 52 -> 52, 30, 48 us; 4321 rows of 24, 2880
+// <-> 1440, 123, 81, 130 -> 113, 74, 120; over 8 layers, 4 to 64 experts and 12 to 1500 rows an expert 1.05, 1.04, 1.07 times as
+// fast, 0.94 to 1.25.  (The same quarters with the staging registers of the other tiles: two thirds of that.)  Dgrad-down is
+// 0.79 times as fast in quarters where they are all there is, and 0.94 after whole rounds (577 rows of 24 experts, 4096 <->
+// 1536, 60 -> 96 us; 8641 rows of 48 193 -> 225), never more than 1.05.
 template <int MODE, typename OutT, bool BLK>
 __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gemm_kernel(const GemmArgs p) {
   static_assert(CfgHalf::NT == CfgMain::NT, "one workgroup runs both");
@@ -863,7 +866,7 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
   int halves = 0;     // halves with rows of the others, or quarters
   bool quarters = false;
   const int left = total % nb;
-  const bool can_quarter = BLK || MODE == DOWN || MODE == DGRAD_GATEUP || (MODE == GATEUP && !p.C0);  // (g and u in rows: not)
+  const bool can_quarter = MODE == DOWN || MODE == DGRAD_GATEUP || (MODE == GATEUP && (BLK || !p.C0));  // (g and u in rows: not)
   if (!p.whole_only && left > 0 && nb <= MAX_LISTED) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int round = total > nb && 2 * nb <= MAX_LISTED ? nb : 0;  // (of whole tiles that may be halved too)
@@ -930,7 +933,7 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
   if (halves == 0) return;
   __syncthreads();  // (the operand stages are free, the list is complete)
   const Sweep h = sweep_of(halves);
-  if constexpr (BLK || MODE != DGRAD_DOWN) {
+  if constexpr (MODE != DGRAD_DOWN) {
     if (quarters) {
       using Quarter = RingTile<MODE, 1, CfgMain::NT / MOE_WAVE>;
       static_assert(Quarter::LDS <= lds_bytes<MODE, CfgMain>() && Quarter::BM * 4 == ROW_TILE, "fits");
