@@ -556,9 +556,9 @@ int forced_tile = 0;
 // rounds of large tiles: 335 against 295 us; three rounds: equal): from eight rounds on.  So, too, for weight gradients,
 // where a tile takes as long as its expert has rows.  From three to eight rounds the large one is faster by a tenth
 // where a router with random weights deals the rows (4096 rows of 8 experts, three stacks of 1024 x 512, three rounds: 120 us
-// against 126), and slower where it does not: with logits off by 0.3 from expert to expert by 0.90 to 1.03 on average and down to 0.42
-// (16384 rows of 128 experts, 256 x 128: 220 us against 92), with Zipf's shares by 0.67 to 0.81 and down to 0.31.  From eight rounds
-// on: 1.04, 1.08 and 1.03 times as fast.
+// against 126), and slower where it does not: with logits off by 0.3 from expert to expert 0.90 to 1.03 times as fast on
+// average and down to 0.42 (16384 rows of 128 experts, 256 x 128: 220 us against 92), with Zipf's shares 0.67 to 0.81 and
+// down to 0.31.  From eight rounds on: 1.04, 1.08 and 1.03 times as fast.
 bool large_tiles(int64_t tiles128) {
   if (forced_tile) return forced_tile == 128;
   return tiles128 >= 8 * (int64_t)moe_compute_units();
@@ -677,9 +677,9 @@ static int wgrads(const F32Stack* s, int n, const int32_t* offs, int64_t E, int6
       hipLaunchKernelGGL((f32_wgrad_kernel<Small, Quarter, DEAL>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, st, p, cus);
   };
   // Times as fast with a look at the offsets as without, up to 64 experts, even loads and loads with a heavy expert: tiles of
-  // 64, below 32 rows an expert 0.86 to 0.91, 0.87 to 1.0;
-  // 64 to 128 rows 0.94, 1.25; 128 to 256 rows 0.98, 1.35; more 0.99, 1.45.  Tiles of 128: below 64 rows 0.91 to 0.97, 1.03 to
-  // 1.13; 64 to 128 rows 0.98, 1.19; more 0.99, 1.3.  Of 128 experts, which are not sorted, 128 rows each: 0.95, 1.1.
+  // 64, below 32 rows an expert 0.86 to 0.91, 0.87 to 1.0; 64 to 128 rows 0.94, 1.25; 128 to 256 rows 0.98, 1.35; more 0.99,
+  // 1.45.  Tiles of 128: below 64 rows 0.91 to 0.97, 1.03 to 1.13; 64 to 128 rows 0.98, 1.19; more 0.99, 1.3.  Of 128 experts,
+  // which are not sorted, 128 rows each: 0.95, 1.1.
   if (R >= (E > MOE_WAVE ? 256 : large ? 64 : 128) * E) go(std::true_type{});
   else go(std::false_type{});
   return moe_launch_status();
