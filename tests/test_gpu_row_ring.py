@@ -16,11 +16,15 @@ pytestmark = pytest.mark.gpu
     ([2, 0, 7, 1] * 32, 128, 64),                  # 128, columns of half a tile
     ([300, 2, 900], 1000, 512),                    # more row tiles than an XCD's share
     ([513, 511, 0, 900, 1, 640, 384, 513], 1000, 520),   # down and dgrad-gate/up in tiles of 128 rows by themselves
-    # a little more than a round of tiles of 256 rows (gate/up and dgrad-gate/up, then dgrad-down): the rest in quarters
+    # more small tiles than run at once: taken for down, dgrad-down and dgrad-gate/up; for down (dgrad-down has fewer) alone
+    ([50] * 46 + [70, 64], 1536, 640),
+    ([24] * 16, 4096, 2048),
+    # a little more than a round of tiles of 256 rows (gate/up and dgrad-gate/up, then dgrad-down): the rest in quarters (in
+    # dgrad-down in halves)
     ([8193], 2048, 1016),
     ([8200, 0, 70, 190], 1992, 1032),
     ([4100, 4300], 520, 2048),
-], ids=["whole", "least", "edges", "64", "65", "128", "long", "tall", "quarter of one row", "quarters", "quarters down"])
+], ids=["whole", "least", "edges", "64", "65", "128", "long", "tall", "by rounds", "whole rounds", "quarter of one row", "quarters", "quarters down"])
 def test_row_ring_bits(pkg, lib, counts, H, I):
     print("row ring", len(counts), sum(counts), H, I, flush=True)
     ops = pkg.ops

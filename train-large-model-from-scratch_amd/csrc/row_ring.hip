@@ -9,6 +9,8 @@
 // tiles of 128 x 256, 11.8, 6.0, 13.3, 10.7 here; 768 rows of 12 experts, 1416 <-> 568: 25.8, 12.8, 29.7, 20.5 and 17.6,
 // 10.6, 18.5, 15.2.  (64 x 128 in five stages, one workgroup to a compute unit: 12.6, 6.7, 13.9, 11.9; 128 x 128 in
 // three: 14.2, 7.9, 17.5, 13.7; the next k-tile's first fragments read before the last products: 12.2, 6.5, 13.6, 11.0.)
+#include <cmath>
+
 #include "row_ring.h"
 
 namespace {
@@ -76,22 +78,41 @@ bool launch(GemmArgs a, long long most, bool any, hipStream_t s, int* rc) {
   return *rc = moe_launch_status(), true;
 }
 
+// Whether tiles of 64 rows are the faster ones where there are more of them than run at once.  With few rows an expert the
+// weights bound a launch, larger tiles are padding and an expert has one of them: their launch lasts as many whole rounds
+// of one to a compute unit as E experts' tiles fill.  Tiles of 64 rows, two to a compute unit, are dealt out as they end
+// and take their share of a round each, about 0.8 of it where the contraction is short and 1 at 4096, and from some 30
+// rows an expert on more and more experts have two (by chance and by the router).  Over 11 layers, 4 to 128 experts,
+// 8 to 500 rows an expert dealt evenly and unevenly, this takes 2.2 % longer than the faster one everywhere, 40 rows an
+// expert as the line 3.3 %.  Larger tiles -> this, us: 24 experts, 3000 <-> 1200, 50 rows each (1.1 rounds) down 61 -> 48,
+// dgrad-gate/up 99 -> 84; 48 experts, 1536 <-> 640, 50 rows (1.1) 30 -> 22, 50 -> 40; 64 experts, 2048 <-> 1024 (2 rounds) 31 rows
+// down 55 -> 49, 50 rows, not taken, gate/up 154 -> 164, dgrad-gate/up 107 -> 116; 16 experts, 4096 <-> 2048, 37 rows (1
+// round), not taken, gate/up 89 -> 95, dgrad-gate/up 92 -> 99.  What it gets wrong: 16 experts, 2880 <-> 1440, 32 rows, gate/up
+// 45 -> 48; 32 experts, 2048 <-> 1024, 50 rows, down takes 33 and could take 28; 128 experts, 1024 <-> 256, 50 rows dealt
+// unevenly, gate/up takes 40 and could take 27.
+template <int MODE>
+bool small_tiles_pay(const GemmArgs& a) {
+  constexpr int LARGE = MODE == GATEUP ? 128 : 256, SMALL = MODE == GATEUP ? 64 : 128;  // columns of a tile
+  const double cus = moe_compute_units(), rows = (double)a.R / a.E, k = (double)a.K * (MODE == DGRAD_GATEUP ? 2 : 1);
+  if (rows > 80) return false;
+  const double second = rows > 30 ? (rows - 30) / 40 : 0;
+  const double large = std::ceil(a.E * (double)((a.N + LARGE - 1) / LARGE) / cus);
+  return a.E * (double)((a.N + SMALL - 1) / SMALL) / (2 * cus) * (1 + second) * (0.75 + 0.07 * k / 1024) < large;
+}
+
 // Up to two tiles for each compute unit, all resident at once.  (Tiles of 64 rows, this and the kernels of larger tiles in
 // us: gate/up 320, 14.8 and 19.2; 512, 18.0 and 19.2; 576, 23.3 and 20.5; dgrad-down 288, 18.1 and 23.8; 404, 19.7 and
-// 24.8; 544, 29.2 and 25.3.)  With one tile to an expert the weights bound a launch of any size, and larger tiles are
-// padding (gate/up, down, dgrad-down and dgrad-gate/up, larger tiles -> this: 64 experts, 2048 <-> 1024, 31 rows each
-// 148, 55, 52, 101 -> 150, 49, 50, 99; 37 rows 153, 56, 52, 104 -> 152, 51, 51, 101; 50 rows 154, 56, 52, 107 -> 164, 57, 63,
-// 116, as one expert or the other then has a second tile; 96 experts, 1536 <-> 640, 42 rows 126, 52, 56, 86 -> 121, 43, 43,
-// 81; 128 experts, 1024 <-> 256, 31 rows 35, 27, 22, 28 -> 32, 27, 15, 24).
+// 24.8; 544, 29.2 and 25.3.)
 // Down and dgrad-gate/up, whose epilogues are short, have tiles of 128 rows and two stages for what is too much for 64
 // rows (tiles of 128 rows; down and dgrad-gate/up us: 320 12.4, 19.8 -> 11.2, 17.6; 440 14.5, 22.6 -> 12.5, 19.6; 576
 // 19.0, 29.2 -> 19.5, 31.8).
 template <int MODE, bool BLK>
 bool choose(const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
   const long long slots = 2ll * moe_compute_units();
-  if (launch<MODE, BLK, 1>(a, slots, forced || a.R <= 40ll * a.E, s, rc)) return true;
-  if constexpr (MODE == DOWN || MODE == DGRAD_GATEUP) return launch<MODE, BLK, 2>(a, slots, false, s, rc);
-  else return false;
+  if (launch<MODE, BLK, 1>(a, slots, forced, s, rc)) return true;
+  if constexpr (MODE == DOWN || MODE == DGRAD_GATEUP)
+    if (launch<MODE, BLK, 2>(a, slots, false, s, rc)) return true;
+  return small_tiles_pay<MODE>(a) && launch<MODE, BLK, 1>(a, slots, true, s, rc);
 }
 
 }  // namespace
