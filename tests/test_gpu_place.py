@@ -11,11 +11,13 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("T,E,k,H", [
     (65, 4, 1, 8),           # a token past the kernels for few tokens, one piece of a row
-    (2047, 8, 2, 136),       # chunks of 8 tokens, the last one short
+    (2047, 8, 2, 136),       # the last chunk of 16 tokens one short
     (2048, 128, 8, 64),      # ... all full, as many experts as are taken
-    (2049, 65, 64, 16),      # chunks of 16; more than a wave of experts, as many a token as are taken
-    (4096, 128, 3, 64),      # the largest table, one workgroup a chunk
-    (4097, 128, 3, 64),      # one token more: the general path
+    (2049, 65, 64, 16),      # more than a wave of experts, as many a token as are taken
+    (4096, 128, 3, 64),      # a table of which one workgroup a chunk reads
+    (4097, 128, 3, 64),
+    (12288, 128, 2, 16),     # the largest table
+    (12289, 128, 2, 16),     # one token more: the general path
     (5000, 1, 1, 2056),      # one expert; more than four pieces a lane
     (8001, 31, 5, 24),       # a last word with one count missing
     (300, 8, 2, 12),         # rows that only the fp32 layer takes, which the general path moves
@@ -56,7 +58,7 @@ def test_places(pkg, lib, T, E, k, H, dtype):
     assert ((out.float() - want)[~nan].abs() <= rel * (want[~nan].abs() + 1e-3)).all()
 
 
-# (two launches, chunks of 8 and of 16 tokens; more experts than they take: the general path; no tokens)
+# (two launches; more experts than they take: the general path; no tokens)
 @pytest.mark.parametrize("T,E", [(100, 8), (2100, 8), (100, 136), (0, 8)])
 def test_the_count_of_bad_ids_is_written_with_logits(pkg, lib, T, E):
     """The C entry, which takes the pointer also where the experts come from the logits: 0, whichever launches run."""

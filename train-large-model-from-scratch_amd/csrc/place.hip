@@ -5,8 +5,8 @@
 // workgroups count their own 16 tokens, a byte an expert, and every workgroup of the second launch adds up the
 // bytes in front of it for itself, while its rows are on their way from memory.  The permutation is the same one: a
 // token asks for an expert at most once, so rows of an expert in the order of their tokens is the stable order.
-// Selection to rows, us, before and now: 2048 tokens, 8 experts, 1024 wide 13.3, 8.3; 1531 tokens, 64 experts,
-// 8 a token, 2048 wide 31.6, 19.7; 8192 tokens, 8 experts 27.6, 16.2; 512 tokens, 256 wide 12.0, 7.3.
+// From the selection's start to the rows' end, us, the general path and here: 2048 tokens, 8 experts, 1024 wide 16.9, 10.6;
+// 1531 tokens, 64 experts, 8 a token, 2048 wide 35.9, 17.4; 8192 tokens, 8 experts 32.9, 17.2; 512 tokens 15.6, 9.6.
 #include "common.h"
 #include "internal.h"
 #include "topk_core.h"
@@ -14,18 +14,20 @@
 namespace {
 
 constexpr int PLACE_EXPERTS = 2 * MOE_WAVE;
-// Bytes of counts, all of which every placing workgroup reads.  At this many (4096 tokens, 128 experts, 8 a token, 1024
-// wide) the two launches take 26 us where the general path takes 38; past it there are more workgroups, too, and
-// a pass lasts so long that the difference no longer counts.
-constexpr int64_t PLACE_TABLE = 32 * 1024;
+constexpr int CHUNK = 16;  // tokens counted together, one a wave of a selection's workgroup
+
+// Bytes of counts, all of which every placing workgroup reads: their number times the tokens is what makes the two launches
+// the slower ones in the end.  General path -> these, from the selection's start to the rows' end, us: 128 experts, 8 a
+// token, 1024 wide, 4096 tokens (32 KB) 37 -> 23, 8192 (64 KB) 55 -> 42, 16384 (128 KB) 93 -> 81; 1 a token, where there is least
+// else to do, 8192 28 -> 19, 12000 (94 KB) 31 -> 30, 16384 36 -> 39; 64 experts, 8 a token, 512 wide, 24000 (94 KB) 77 -> 69; 8
+// experts, 2 a token, 1024 wide, 60000 (30 KB) 113 -> 105.  (Chunks of 8 tokens, a table of twice the size: 30 of the first;
+// 1531 tokens of 64 experts, 2048 wide, 18.3 where 16 take 17.4; 256 tokens of 128 experts 10.0 and 10.3.)
+constexpr int64_t PLACE_TABLE = 96 * 1024;
 
 int words_of(int64_t E) { return (int)((E + 3) / 4); }
-// Tokens counted together, one a wave.  8 where 16 would leave many compute units idle: 1531 tokens, 64 experts, 8 a token,
-// selection 5.7 us instead of 7.0 (places 14.0 and 13.0); 2048 tokens, 8 experts 3.5 and 4.1 (4.8 and 4.9).
-int chunk_of(int64_t T) { return T <= 2048 ? 8 : 16; }
 
 // One wave a token, as router_topk_fwd_kernel; table[chunk][e] = how many of the chunk's tokens ask for e.
-template <int VPL, typename LT, int CHUNK>
+template <int VPL, typename LT>
 __global__ __launch_bounds__(CHUNK* MOE_WAVE) void select_count_kernel(const LT* __restrict__ logits,
                                                                       const float* __restrict__ bias, int T, int E, int k,
                                                                       int32_t* __restrict__ ids, float* __restrict__ gates,
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(CHUNK* MOE_WAVE) void select_count_kernel(const LT*
 }
 
 // WAVES tokens of a chunk, one a wave.  `shift`: 2^shift words hold a chunk's counts.
-template <typename XT, typename OT, int CHUNK, int WAVES>
+template <typename XT, typename OT, int WAVES>
 __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     const XT* __restrict__ x, const int32_t* __restrict__ ids, const uint32_t* __restrict__ table, int T, int E, int k,
     int H, int shift, int32_t* __restrict__ counts, int32_t* __restrict__ offs, int32_t* __restrict__ pos_to_row,
@@ -161,26 +163,22 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
 bool moe_place_ok(int64_t T, int64_t E, int64_t k) {
   return T > 0 && T < 65536 && E <= PLACE_EXPERTS && k <= E && k <= MOE_MAX_TOPK && moe_place_bytes(T, E) <= PLACE_TABLE;
 }
-int64_t moe_place_bytes(int64_t T, int64_t E) { return (T + chunk_of(T) - 1) / chunk_of(T) * words_of(E) * 4; }
+int64_t moe_place_bytes(int64_t T, int64_t E) { return (T + CHUNK - 1) / CHUNK * words_of(E) * 4; }
 
 int moe_select_count(const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t E, int64_t k,
                      int32_t* ids, float* gates, void* table, void* stream) {
   hipStream_t s = (hipStream_t)stream;
-  const auto go = [&](auto vpl, auto lt, auto chunk) {
+  const auto go = [&](auto vpl, auto lt) {
     using LT = decltype(lt);
-    constexpr int CHUNK = decltype(chunk)::value;
-    hipLaunchKernelGGL((select_count_kernel<decltype(vpl)::value, LT, CHUNK>), dim3((unsigned)((T + CHUNK - 1) / CHUNK)),
+    hipLaunchKernelGGL((select_count_kernel<decltype(vpl)::value, LT>), dim3((unsigned)((T + CHUNK - 1) / CHUNK)),
                        dim3(CHUNK * MOE_WAVE), 0, s, (const LT*)logits, bias, (int)T, (int)E, (int)k, ids, gates,
                        (uint32_t*)table);
     return moe_launch_status();
   };
-  const auto of = [&](auto chunk) {
-    using One = std::integral_constant<int, 1>;
-    using Two = std::integral_constant<int, 2>;
-    if (logits_dtype == MOE_DT_BF16) return E <= MOE_WAVE ? go(One{}, uint16_t{}, chunk) : go(Two{}, uint16_t{}, chunk);
-    return E <= MOE_WAVE ? go(One{}, float{}, chunk) : go(Two{}, float{}, chunk);
-  };
-  return chunk_of(T) == 8 ? of(std::integral_constant<int, 8>{}) : of(std::integral_constant<int, 16>{});
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  if (logits_dtype == MOE_DT_BF16) return E <= MOE_WAVE ? go(One{}, uint16_t{}) : go(Two{}, uint16_t{});
+  return E <= MOE_WAVE ? go(One{}, float{}) : go(Two{}, float{});
 }
 
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
@@ -192,23 +190,20 @@ int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* t
   hipStream_t s = (hipStream_t)stream;
   int shift = 0;
   while ((1 << shift) < words_of(E)) ++shift;
-  const auto go = [&](auto xt, auto ot, auto chunk, auto waves) {
+  const auto go = [&](auto xt, auto ot, auto waves) {
     using XT = decltype(xt);
     using OT = decltype(ot);
-    constexpr int CHUNK = decltype(chunk)::value, WAVES = decltype(waves)::value;
-    hipLaunchKernelGGL((place_rows_kernel<XT, OT, CHUNK, WAVES>), dim3((unsigned)((T + WAVES - 1) / WAVES)),
+    constexpr int WAVES = decltype(waves)::value;
+    hipLaunchKernelGGL((place_rows_kernel<XT, OT, WAVES>), dim3((unsigned)((T + WAVES - 1) / WAVES)),
                        dim3(WAVES * MOE_WAVE), 0, s, (const XT*)x, ids, (const uint32_t*)table, (int)T, (int)E, (int)k,
                        (int)H, shift, counts, offs, pos_to_row, row_to_pos, bad_ids, (OT*)xp);
     return moe_launch_status();
   };
-  const auto of = [&](auto chunk, auto waves) {
-    if (x_dtype == MOE_DT_BF16) return go(uint16_t{}, uint16_t{}, chunk, waves);
-    return xp_dtype == MOE_DT_BF16 ? go(float{}, uint16_t{}, chunk, waves) : go(float{}, float{}, chunk, waves);
+  const auto of = [&](auto waves) {
+    if (x_dtype == MOE_DT_BF16) return go(uint16_t{}, uint16_t{}, waves);
+    return xp_dtype == MOE_DT_BF16 ? go(float{}, uint16_t{}, waves) : go(float{}, float{}, waves);
   };
-  using Eight = std::integral_constant<int, 8>;
-  using Sixteen = std::integral_constant<int, 16>;
-  if (chunk_of(T) == 8) return of(Eight{}, Eight{});
   // (fewer workgroups to read a large table: 4096 tokens, 128 experts 18.1 us, with 8 waves 20.0; 8192 tokens, 8 experts,
   // 4 KB 11.1 and 10.7)
-  return moe_place_bytes(T, E) > PLACE_TABLE / 2 ? of(Sixteen{}, Sixteen{}) : of(Sixteen{}, Eight{});
+  return moe_place_bytes(T, E) > 16 * 1024 ? of(std::integral_constant<int, 16>{}) : of(std::integral_constant<int, 8>{});
 }
