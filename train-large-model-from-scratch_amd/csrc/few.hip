@@ -11,7 +11,7 @@
 // the operand registers, every byte once, with a wave's whole share of the contraction requested before
 // the first product where it fits.
 #include "common.h"
-#include "internal.h"
+#include "gemm_args.h"
 #include "topk_core.h"
 
 namespace {
@@ -25,9 +25,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, long lo
 }
 __device__ __forceinline__ bf16x8 load_frag(__amdgpu_buffer_rsrc_t rs, unsigned off) {
   return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
-}
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f)) * u;
 }
 
 // ---- router product ---------------------------------------------------------------------------------
@@ -236,7 +233,7 @@ __device__ __forceinline__ void few_columns(const AT* __restrict__ A, int div, c
         for (int i = 0; i < 4; ++i) v[b] += buf[((i * NB + b) * MF + m) * 256 + wv * MOE_WAVE + lane];
       }
       const int at = m * 16 + lq * 4 + wv;
-      if (at < n && col < N) C[(size_t)rows[at] * N + col] = f32_to_bf16(NB == 2 ? silu_mul(v[0], v[NB - 1]) : v[0]);
+      if (at < n && col < N) C[(size_t)rows[at] * N + col] = f32_to_bf16(NB == 2 ? swiglu(v[0], v[NB - 1]) : v[0]);
     }
     ++mb;
   };

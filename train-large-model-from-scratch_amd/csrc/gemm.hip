@@ -534,7 +534,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
             for (int x = 0; x < 4; ++x) {
               g[x] = acc[i][j][4 * q + x];
               u[x] = acc[i][j + FNC][4 * q + x];
-              a[x] = g[x] * sigmoidf_(g[x]) * u[x];
+              a[x] = swiglu(g[x], u[x]);
             }
             put4(0, j, q, a[0], a[1], a[2], a[3]);
             if constexpr (BLK) {
@@ -579,14 +579,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
             const float u[4] = {bf16lo(u01), bf16hi(u01), bf16lo(u23), bf16hi(u23)};
             float dg[4], du[4];
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              const float dact = acc[i][j][4 * q + x];
-              const float sg = sigmoidf_(g[x]);
-              const float gs = g[x] * sg;                     // silu(g)
-              du[x] = dact * gs;
-              dg[x] = (dact * u[x]) * (sg + (gs - gs * sg));  // silu'(g) = s + g*s*(1-s)
-              rowdot += du[x] * u[x];                         // dact * act
-            }
+            for (int x = 0; x < 4; ++x) swiglu_bwd(acc[i][j][4 * q + x], g[x], u[x], dg[x], du[x], rowdot);
             put4(0, j, q, dg[0], dg[1], dg[2], dg[3]);
             put4(1, j, q, du[0], du[1], du[2], du[3]);
             // (the running sum is wanted here, not at the end of the strip: left alone the compiler
@@ -622,14 +615,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
             const float u[4] = {bf16lo(uw[0]), bf16hi(uw[0]), bf16lo(uw[1]), bf16hi(uw[1])};
             float dg[4], du[4];
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              const float dact = acc[i][j][4 * q + x];
-              const float sg = sigmoidf_(g[x]);
-              const float gs = g[x] * sg;                     // silu(g)
-              du[x] = dact * gs;
-              dg[x] = (dact * u[x]) * (sg + (gs - gs * sg));  // silu'(g) = s + g*s*(1-s)
-              rowdot += du[x] * u[x];                         // dact * act
-            }
+            for (int x = 0; x < 4; ++x) swiglu_bwd(acc[i][j][4 * q + x], g[x], u[x], dg[x], du[x], rowdot);
             put4(0, j, q, dg[0], dg[1], dg[2], dg[3]);
             put4(1, j, q, du[0], du[1], du[2], du[3]);
             asm volatile("" : "+v"(rowdot));  // (summed here: see the blocked variant above)

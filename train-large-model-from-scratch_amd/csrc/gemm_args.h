@@ -35,5 +35,15 @@ __device__ __forceinline__ float sigmoidf_(float x) {
   return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
 }
 
+// What the fused epilogues do with an element, the same operations whatever the tile, so that the bits do not depend on it:
+// silu(g) * u, and backwards, with `dot` summing up dact * act.
+__device__ __forceinline__ float swiglu(float g, float u) { return g * sigmoidf_(g) * u; }
+__device__ __forceinline__ void swiglu_bwd(float dact, float g, float u, float& dg, float& du, float& dot) {
+  const float sg = sigmoidf_(g), gs = g * sg;  // gs: silu(g)
+  du = dact * gs;
+  dg = (dact * u) * (sg + (gs - gs * sg));     // silu'(g) = s + g*s*(1-s)
+  dot += du * u;
+}
+
 // Takes a row-ragged launch of few tiles (csrc/row_ring.hip): false where it does not.
 bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, bool forced, hipStream_t s, int* rc);

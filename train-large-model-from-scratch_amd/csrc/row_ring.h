@@ -165,7 +165,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
       for (int v = 0; v < 4; ++v) {
         g[v] = acc[0][0][4 * g4 + v];
         u[v] = acc[0][1][4 * g4 + v];
-        a[v] = g[v] * sigmoidf_(g[v]) * u[v];
+        a[v] = swiglu(g[v], u[v]);
       }
       put4(0, g4, pack4(a[0], a[1], a[2], a[3]));
       gq[g4 & 1] = pack4(g[0], g[1], g[2], g[3]);
@@ -189,12 +189,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
         const float u[4] = {bf16lo(u01), bf16hi(u01), bf16lo(u23), bf16hi(u23)};
         float dg[4], du[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const float dact = acc[0][c][4 * g4 + v], sg = sigmoidf_(g[v]), gs = g[v] * sg;  // gs: silu(g)
-          du[v] = dact * gs;
-          dg[v] = (dact * u[v]) * (sg + (gs - gs * sg));  // silu'(g) = s + g*s*(1-s)
-          rowdot += du[v] * u[v];                         // dact * act
-        }
+        for (int v = 0; v < 4; ++v) swiglu_bwd(acc[0][c][4 * g4 + v], g[v], u[v], dg[v], du[v], rowdot);
         put4(c, g4, pack4(dg[0], dg[1], dg[2], dg[3]));
         du4[c][g4] = pack4(du[0], du[1], du[2], du[3]);
       }
