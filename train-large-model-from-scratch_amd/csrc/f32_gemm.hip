@@ -1,5 +1,5 @@
-// Grouped (per-expert, ragged) GEMMs of the fp32 path on the matrix cores (v_mfma_f32_32x32x2_f32: fp32
-// operands, fp32 accumulation), and what is fused into them.
+// Grouped (per-expert, ragged) GEMMs of the fp32 path on the matrix cores, and what is fused into them: large ones in
+// three fp16 products for one of fp32 (f32_split.h), the others with v_mfma_f32_32x32x2_f32 (fp32 operands, fp32 accumulation).
 //
 // An fp32 MFMA takes 64 cycles for 2048 multiply-adds, sixteen times as long per flop as a bf16 one, so
 // that neither LDS nor HBM bounds these kernels: what does is how evenly the chip's matrix pipes are
@@ -8,24 +8,11 @@
 // iterations before their use, one barrier per iteration that leaves global loads in flight, output tiles of a quarter
 // of the size where the last round of tiles would leave compute units empty, and few launches: gate and up share
 // one (and with it their tiles), the two halves of the input gradient another, the three weight gradients a third.
-#include "internal.h"
-#include "tile_ops.h"
+#include "f32_split.h"
 
 namespace {
 
 constexpr int NT = 256;                    // threads
-constexpr unsigned OUTSIDE = 0xfffffff0u;  // a byte offset that no window reaches: reads as zero
-
-// Operand chunks of 16 bytes are read through buffer resources, whose hardware bounds check makes an out-of-range
-// chunk a zero without a branch: chunks past the tile's rows or past the end of the contraction get the offset OUTSIDE.
-// A window is moved along k by its base, a scalar addition.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t window(const float* base, long long elems) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)(base + elems), 0, 0x7fffffff, 0x00020000);
-}
-__device__ __forceinline__ f32x4 window_load(__amdgpu_buffer_rsrc_t rs, unsigned off) {
-  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
-}
-
 // Operand tiles of ROWS x TK.  Of each group of eight k values the lower half of a wave multiplies the first
 // four and the upper half the others (MFMA j takes k = j and j + 4; any pairing will do as long as both operands use
 // the same), so that an operand that lies k-contiguous in LDS is read 16 bytes at a time.
@@ -239,8 +226,8 @@ struct Job {
   int tile, part;  // part: 0..3 of the tile, -1: all of it; tile < 0: none
 };
 // chunk > 0: the list is dealt to the XCDs by so many tiles instead (what is left after the last full deal one by one).
-__device__ __forceinline__ Job job_of(int tiles, int cus, int chunk = 0) {
-  const int rest = tiles % cus, cut = rest * 4 <= cus * 3 ? rest : 0, whole = tiles - cut;
+__device__ __forceinline__ Job job_of(int tiles, int cus, int most, int chunk = 0) {
+  const int rest = tiles % cus, cut = rest * 4 <= most ? rest : 0, whole = tiles - cut;
   const int x = blockIdx.x & 7;
   int j = blockIdx.x >> 3;
   if (chunk > 0) {
@@ -260,6 +247,10 @@ __device__ __forceinline__ Job job_of(int tiles, int cus, int chunk = 0) {
 // Workgroups for at most `tiles` tiles: each XCD may round its two shares up.
 unsigned grid_of(int64_t tiles, int64_t cus) { return (unsigned)((tiles + 3 * (cus * 3 / 4) + 7) / 8 * 8 + 16); }
 
+// How many quarters the split tiles' last round may be cut into: one workgroup is resident on a compute unit, a whole tile takes
+// 9 + 0.03 k us and a quarter 9 + 0.009 k (k: length of the contraction), so that two rounds of quarters pay from 700 on.
+__device__ __forceinline__ int split_cut(int k, int cus) { return k > 700 ? 2 * cus : cus; }
+
 template <int MODE>
 constexpr bool b_kcont = MODE == PLAIN_T || MODE == GATEUP;
 template <int MODE, typename S>
@@ -267,6 +258,38 @@ using RowsB = typename std::conditional<b_kcont<MODE>, KCont<S::BN, S::TK>, RCon
 template <int MODE, typename S>
 using RowsLoop = Loop<S, KCont<S::BM, S::TK>, RowsB<MODE, S>>;
 constexpr __host__ __device__ int larger(int a, int b) { return a > b ? a : b; }
+
+// What becomes of four consecutive columns of one row (GATEUP: v of g and u of u; else u is not used)
+template <int MODE>
+__device__ __forceinline__ void rows_result(const RowsArgs& p, int m, int row_end, int n, f32x4 v, f32x4 u) {
+  constexpr bool DUAL = MODE == GATEUP;
+  if (m >= row_end || n >= p.N) return;  // (N % 4 == 0: the four columns are inside or outside together)
+  const long long at = (long long)m * p.N + n;
+  if constexpr (DUAL) {
+    f32x4 a;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) a[c] = v[c] * sigmoid_f32(v[c]) * u[c];
+    if (p.C0) {
+      *reinterpret_cast<f32x4*>(p.C0 + at) = v;
+      *reinterpret_cast<f32x4*>(p.C1 + at) = u;
+    }
+    *reinterpret_cast<f32x4*>(p.C2 + at) = a;
+  } else if constexpr (MODE == DOWN_BWD) {  // silu'(g) = s * (1 + g * (1 - s)), s = sigmoid(g)
+    const f32x4 gv = *reinterpret_cast<const f32x4*>(p.X0 + at), uv = *reinterpret_cast<const f32x4*>(p.X1 + at);
+    f32x4 dg, du;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float s = sigmoid_f32(gv[c]);
+      dg[c] = v[c] * uv[c] * (s * (1.f + gv[c] * (1.f - s)));
+      du[c] = v[c] * (gv[c] * s);
+    }
+    *reinterpret_cast<f32x4*>(p.C0 + at) = dg;
+    *reinterpret_cast<f32x4*>(p.C1 + at) = du;
+  } else {
+    if (p.accumulate) v += *reinterpret_cast<const f32x4*>(p.C0 + at);
+    *reinterpret_cast<f32x4*>(p.C0 + at) = v;
+  }
+}
 
 // The tile of Shape S at rows row0.. (of the expert's up to row_end), columns n0..
 template <int MODE, typename S>
@@ -316,35 +339,7 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& p, float* lds, int e, 
   const bool idle = uniform((int)(row0 + wm * S::NM * 32 >= row_end)) != 0;
   L::run(lds, opA, opB, MODE == GATEUP_BWD ? 2 * per_seg : per_seg, idle, wv, acc, load);
 
-  // ---- results: a lane holds four consecutive columns of one row at a time
-  const auto emit = [&](int m, int n, f32x4 v, f32x4 u) {
-    if (m >= row_end || n >= p.N) return;  // (N % 4 == 0: the four columns are inside or outside together)
-    const long long at = (long long)m * p.N + n;
-    if constexpr (DUAL) {
-      f32x4 a;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) a[c] = v[c] * sigmoid_f32(v[c]) * u[c];
-      if (p.C0) {
-        *reinterpret_cast<f32x4*>(p.C0 + at) = v;
-        *reinterpret_cast<f32x4*>(p.C1 + at) = u;
-      }
-      *reinterpret_cast<f32x4*>(p.C2 + at) = a;
-    } else if constexpr (MODE == DOWN_BWD) {  // silu'(g) = s * (1 + g * (1 - s)), s = sigmoid(g)
-      const f32x4 gv = *reinterpret_cast<const f32x4*>(p.X0 + at), uv = *reinterpret_cast<const f32x4*>(p.X1 + at);
-      f32x4 dg, du;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float s = sigmoid_f32(gv[c]);
-        dg[c] = v[c] * uv[c] * (s * (1.f + gv[c] * (1.f - s)));
-        du[c] = v[c] * (gv[c] * s);
-      }
-      *reinterpret_cast<f32x4*>(p.C0 + at) = dg;
-      *reinterpret_cast<f32x4*>(p.C1 + at) = du;
-    } else {
-      if (p.accumulate) v += *reinterpret_cast<const f32x4*>(p.C0 + at);
-      *reinterpret_cast<f32x4*>(p.C0 + at) = v;
-    }
-  };
+  const auto emit = [&](int m, int n, f32x4 v, f32x4 u) { rows_result<MODE>(p, m, row_end, n, v, u); };
   const int l32 = lane & 31, lh = lane >> 5;
   if constexpr (S::WK > 1) {
     L::give(lds, wv, acc);
@@ -363,43 +358,144 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& p, float* lds, int e, 
   }
 }
 
-// Tiles are numbered row tile by row tile (an expert's last one may be short), column tiles fastest; S is a whole
-// tile, Q a quarter of one.
-template <int MODE, typename S, typename Q>
-__global__ __launch_bounds__(NT, S::WAVES) void f32_rows_kernel(const RowsArgs p, int cus) {
-  static_assert(S::BM == 2 * Q::BM && S::BN == 2 * Q::BN, "a quarter");
-  constexpr int TN = MODE == GATEUP ? S::BN / 2 : S::BN;  // columns of a tile
-  __shared__ __align__(16) float lds[larger(RowsLoop<MODE, S>::LDS_FLOATS, RowsLoop<MODE, Q>::LDS_FLOATS)];
+// The same on the fp16 matrix cores (f32_split.h)
+template <int MODE, typename S>
+using SplitB = typename std::conditional<b_kcont<MODE>, SplitInner<S::BN, S::TK, S::NT>, SplitOuter<S::BN, S::TK, S::NT>>::type;
+template <int MODE, typename S>
+using SplitRowsLoop = SplitLoop<S, SplitInner<S::BM, S::TK, S::NT>, SplitB<MODE, S>>;
+
+template <int MODE, typename S>
+__device__ __forceinline__ void split_rows_tile(const RowsArgs& p, char* lds, int e, int row0, int row_end, int n0) {
+  constexpr bool B_KCONT = b_kcont<MODE>, DUAL = MODE == GATEUP;
+  using OpA = SplitInner<S::BM, S::TK, S::NT>;
+  using OpB = SplitB<MODE, S>;
+  using L = SplitRowsLoop<MODE, S>;
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x >> 6));
+  const int ldb = B_KCONT ? p.K : p.N;
+  OpA opA;
+  OpB opB;
+  opA.init(p.K, row_end - row0);
+  opB.init(ldb, p.N - n0);
+  bool up[OpB::CH];  // GATEUP: each 32 columns of the product are 16 of g and 16 of u (the same for a whole wave)
+#pragma unroll
+  for (int i = 0; i < OpB::CH; ++i) up[i] = false;
+  if constexpr (DUAL) {
+    static_assert(16 % (64 / OpB::CPR) == 0, "a wave's chunks lie in 16 rows");
+#pragma unroll
+    for (int i = 0; i < OpB::CH; ++i) {
+      const int rr = OpB::row(i), r = rr / 32 * 16 + (rr & 15);
+      opB.voff[i] = r < p.N - n0 ? (unsigned)(r * p.K + opB.kc) * 4u : OUTSIDE;
+      up[i] = ((wv * (64 / OpB::CPR) + i * OpB::STEP) & 16) != 0;
+    }
+  }
+  const long long wofs = (long long)e * p.N * p.K + (long long)n0 * (B_KCONT ? p.K : 1);
+  const float *A0 = p.A0 + (long long)row0 * p.K, *B0 = p.B0 + wofs;
+  const float *A1 = p.A1 + (long long)row0 * p.K, *B1 = p.B1 + wofs;  // (null and unused outside the two-operand modes)
+  const int per_seg = (p.K + S::TK - 1) / S::TK;
+  const auto load = [&](int t, typename L::Stage& s) __attribute__((always_inline)) {
+    int k0 = t * S::TK;
+    const bool second = MODE == GATEUP_BWD && t >= per_seg;
+    if (second) k0 -= per_seg * S::TK;
+    const __amdgpu_buffer_rsrc_t ra = window(second ? A1 : A0, OpA::k_elems(k0, p.K));
+#pragma unroll
+    for (int c = 0; c < OpA::CH; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) s.v[c][h] = opA.load(c, h, ra, p.K - k0);
+#pragma unroll
+    for (int c = 0; c < OpB::CH; ++c) {
+      const __amdgpu_buffer_rsrc_t rb = window(second || up[c] ? B1 : B0, OpB::k_elems(k0, ldb));
+#pragma unroll
+      for (int h = 0; h < 2; ++h) s.v[OpA::CH + c][h] = opB.load(c, h, rb, p.K - k0);
+    }
+  };
+  const int l32 = lane & 31, lh = lane >> 5;
+  const auto again = [&](int r0, int c0, f32x16& acc) {  // the block of rows r0.., columns c0.. of the tile
+    const int c = c0 + l32, col = DUAL ? c / 32 * 16 + (c & 15) : c;
+    for (int seg = 0; seg < (MODE == GATEUP_BWD ? 2 : 1); ++seg) {
+      const float *A = seg ? A1 : A0, *B = seg || (DUAL && (c & 16)) ? B1 : B0;
+      for (int k = 0; k < p.K; k += 2)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(OpB::value(B, ldb, p.N - n0, p.K, col, k + lh),
+                                                   OpA::value(A, p.K, row_end - row0, p.K, r0 + l32, k + lh), acc, 0, 0, 0);
+    }
+  };
+  typename L::Out out;
+  L::run(lds, MODE == GATEUP_BWD ? 2 * per_seg : per_seg, wv, out, load, again);
+
+  const int wn = wv % S::WN, wm = wv / S::WN % S::WM, wk = wv / (S::WN * S::WM);
+#pragma unroll
+  for (int o = 0; o < S::OWN; ++o) {
+    const int item = wk * S::OWN + o, block = item / 2, g = item & 1;
+    const int m = row0 + (wm * S::NM + block / S::NN) * 32 + l32, at = wn * S::NN + block % S::NN;
+    if constexpr (DUAL) {
+      rows_result<MODE>(p, m, row_end, n0 + at * 16 + 8 * g + 4 * lh, out.lo[o], out.hi[o]);
+    } else {
+      rows_result<MODE>(p, m, row_end, n0 + at * 32 + 8 * g + 4 * lh, out.lo[o], out.lo[o]);
+      rows_result<MODE>(p, m, row_end, n0 + at * 32 + 8 * g + 16 + 4 * lh, out.hi[o], out.hi[o]);
+    }
+  }
+}
+
+// Tiles of BM x TN are numbered row tile by row tile (an expert's last one may be short), column tiles fastest.  The
+// workgroup's: false if it has none.
+template <int BM, int TN>
+__device__ __forceinline__ bool rows_job(const RowsArgs& p, int cus, int most, int& e, int& row0, int& row_end, int& n0, int& part) {
   const int lane = threadIdx.x & 63, n_col = (p.N + TN - 1) / TN;
   int tiles = 0;
   for (int e0 = 0; e0 < p.E; e0 += MOE_WAVE) {
     int first;
-    const int nt = (expert_rows(p, e0 + lane, first) + S::BM - 1) / S::BM;
+    const int nt = (expert_rows(p, e0 + lane, first) + BM - 1) / BM;
     tiles += uniform(__shfl(wave_inclusive(nt), MOE_WAVE - 1, MOE_WAVE));
   }
-  const Job job = job_of(tiles * n_col, cus);
-  if (job.tile < 0) return;
+  const Job job = job_of(tiles * n_col, cus, most);
+  if (job.tile < 0) return false;
   const int row_tile = job.tile / n_col;
-  int n0 = job.tile % n_col * TN, e = 0, row0 = 0, row_end = 0;
+  n0 = job.tile % n_col * TN, e = 0, row0 = 0, row_end = 0, part = job.part;
   for (int e0 = 0, seen = 0; e0 < p.E; e0 += MOE_WAVE) {
     int first;
-    const int n = expert_rows(p, e0 + lane, first), nt = (n + S::BM - 1) / S::BM, incl = seen + wave_inclusive(nt);
+    const int n = expert_rows(p, e0 + lane, first), nt = (n + BM - 1) / BM, incl = seen + wave_inclusive(nt);
     const unsigned long long past = __ballot(incl > row_tile);
     if (past) {
       const int l = __builtin_ctzll(past);
       e = e0 + l;
-      row0 = uniform(__shfl(first + (row_tile - (incl - nt)) * S::BM, l, MOE_WAVE));
+      row0 = uniform(__shfl(first + (row_tile - (incl - nt)) * BM, l, MOE_WAVE));
       row_end = uniform(__shfl(first + n, l, MOE_WAVE));
       break;
     }
     seen = uniform(__shfl(incl, MOE_WAVE - 1, MOE_WAVE));
   }
-  if (job.part < 0) {
+  return true;
+}
+
+// S is a whole tile, Q a quarter of one.
+template <int MODE, typename S, typename Q>
+__global__ __launch_bounds__(NT, S::WAVES) void f32_rows_kernel(const RowsArgs p, int cus) {
+  static_assert(S::BM == 2 * Q::BM && S::BN == 2 * Q::BN, "a quarter");
+  constexpr int TN = MODE == GATEUP ? S::BN / 2 : S::BN;  // columns of a tile
+  __shared__ __align__(16) float lds[larger(RowsLoop<MODE, S>::LDS_FLOATS, RowsLoop<MODE, Q>::LDS_FLOATS)];
+  int e, row0, row_end, n0, part;
+  if (!rows_job<S::BM, TN>(p, cus, cus * 3, e, row0, row_end, n0, part)) return;
+  if (part < 0) {
     rows_tile<MODE, S>(p, lds, e, row0, row_end, n0);
   } else {
-    row0 += (job.part >> 1) * Q::BM;
-    n0 += (job.part & 1) * (TN / 2);
+    row0 += (part >> 1) * Q::BM;
+    n0 += (part & 1) * (TN / 2);
     if (row0 < row_end && n0 < p.N) rows_tile<MODE, Q>(p, lds, e, row0, row_end, n0);
+  }
+}
+
+template <int MODE, typename S, typename Q>
+__global__ __launch_bounds__(S::NT, S::NT / 256) void f32_split_rows_kernel(const RowsArgs p, int cus) {
+  static_assert(S::BM == 2 * Q::BM && S::BN == 2 * Q::BN && S::NT == Q::NT, "a quarter");
+  constexpr int TN = MODE == GATEUP ? S::BN / 2 : S::BN;  // columns of a tile
+  extern __shared__ __align__(16) char split_lds[];
+  int e, row0, row_end, n0, part;
+  if (!rows_job<S::BM, TN>(p, cus, split_cut(MODE == GATEUP_BWD ? 2 * p.K : p.K, cus), e, row0, row_end, n0, part)) return;
+  if (part < 0) {
+    split_rows_tile<MODE, S>(p, split_lds, e, row0, row_end, n0);
+  } else {
+    row0 += (part >> 1) * Q::BM;
+    n0 += (part & 1) * (TN / 2);
+    if (row0 < row_end && n0 < p.N) split_rows_tile<MODE, Q>(p, split_lds, e, row0, row_end, n0);
   }
 }
 
@@ -416,6 +512,13 @@ struct WgradArgs {
   const int32_t* offs;
   int n, E, R;
 };
+
+__device__ __forceinline__ void wgrad_result(const F32Stack& s, float* C, int m, int n, f32x4 v) {
+  if (m >= s.M || n >= s.N) return;
+  f32x4* dst = reinterpret_cast<f32x4*>(C + (long long)m * s.N + n);
+  if (s.accumulate) v += *dst;
+  *dst = v;
+}
 
 template <typename S>
 using WgradLoop = Loop<S, RCont<S::BM, S::TK>, RCont<S::BN, S::TK>>;
@@ -443,12 +546,7 @@ __device__ __forceinline__ void wgrad_tile(const F32Stack& s, float* lds, int e,
   L::run(lds, opA, opB, n > 0 ? n : 1, false, wv, acc, load);
   if (end == b && s.accumulate) return;
   float* C = s.c + (long long)e * s.M * s.N;
-  const auto emit = [&](int m, int n, f32x4 v) {
-    if (m >= s.M || n >= s.N) return;
-    f32x4* dst = reinterpret_cast<f32x4*>(C + (long long)m * s.N + n);
-    if (s.accumulate) v += *dst;
-    *dst = v;
-  };
+  const auto emit = [&](int m, int n, f32x4 v) { wgrad_result(s, C, m, n, v); };
   const int l32 = lane & 31, lh = lane >> 5, wm = wv / S::WN % S::WM, wn = wv % S::WN;
   if constexpr (S::WK > 1) {
     L::give(lds, wv, acc);
@@ -461,6 +559,52 @@ __device__ __forceinline__ void wgrad_tile(const F32Stack& s, float* lds, int e,
 #pragma unroll
         for (int g = 0; g < 4; ++g)
           emit(m0 + (wm * S::NM + bi) * 32 + l32, n0 + (wn * S::NN + bj) * 32 + 8 * g + 4 * lh, L::quad(acc[bi][bj], g));
+  }
+}
+
+template <typename S>
+using SplitWgradLoop = SplitLoop<S, SplitOuter<S::BM, S::TK, S::NT>, SplitOuter<S::BN, S::TK, S::NT>>;
+template <typename S>
+__device__ __forceinline__ void split_wgrad_tile(const F32Stack& s, char* lds, int e, int b, int end, int m0, int n0) {
+  using OpA = SplitOuter<S::BM, S::TK, S::NT>;
+  using OpB = SplitOuter<S::BN, S::TK, S::NT>;
+  using L = SplitWgradLoop<S>;
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x >> 6));
+  OpA opA;
+  OpB opB;
+  opA.init(s.M, s.M - m0);
+  opB.init(s.N, s.N - n0);
+  const float *A = s.a + (long long)b * s.M + m0, *B = s.b + (long long)b * s.N + n0;
+  const auto load = [&](int t, typename L::Stage& st) __attribute__((always_inline)) {
+    const int left = end - b - t * S::TK;
+    const __amdgpu_buffer_rsrc_t ra = window(A, OpA::k_elems(t * S::TK, s.M)), rb = window(B, OpB::k_elems(t * S::TK, s.N));
+#pragma unroll
+    for (int c = 0; c < OpA::CH; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) st.v[c][h] = opA.load(c, h, ra, left);
+#pragma unroll
+    for (int c = 0; c < OpB::CH; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) st.v[OpA::CH + c][h] = opB.load(c, h, rb, left);
+  };
+  const int l32 = lane & 31, lh = lane >> 5;
+  const auto again = [&](int r0, int c0, f32x16& acc) {
+    for (int k = 0; k < end - b; k += 2)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(OpB::value(B, s.N, s.N - n0, end - b, c0 + l32, k + lh),
+                                                 OpA::value(A, s.M, s.M - m0, end - b, r0 + l32, k + lh), acc, 0, 0, 0);
+  };
+  typename L::Out out;
+  const int n = (end - b + S::TK - 1) / S::TK;  // (without rows: one k-tile of zeros)
+  L::run(lds, n > 0 ? n : 1, wv, out, load, again);
+  if (end == b && s.accumulate) return;
+  float* C = s.c + (long long)e * s.M * s.N;
+  const int wn = wv % S::WN, wm = wv / S::WN % S::WM, wk = wv / (S::WN * S::WM);
+#pragma unroll
+  for (int o = 0; o < S::OWN; ++o) {
+    const int item = wk * S::OWN + o, block = item / 2, g = item & 1;
+    const int m = m0 + (wm * S::NM + block / S::NN) * 32 + l32, n = n0 + (wn * S::NN + block % S::NN) * 32 + 8 * g + 4 * lh;
+    wgrad_result(s, C, m, n, out.lo[o]);
+    wgrad_result(s, C, m, n + 16, out.hi[o]);
   }
 }
 
@@ -484,14 +628,16 @@ __device__ __forceinline__ int lane_of_rank(int n, int largest, int e) {
 // 0.93 to 0.98.  4096 rows of 8 experts by Zipf's shares, three stacks of 1024 x 512: 221 -> 111 us; even 107 and 107.)
 // DEAL: without it the offsets of all experts are not looked at, which costs a workgroup a trip to memory before it
 // can begin (2000 rows of 128 experts, 256 x 256: 32 us without and 40 with).
-template <typename S, typename Q, bool DEAL>
-__global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs p, int cus) {
-  __shared__ __align__(16) float lds[larger(WgradLoop<S>::LDS_FLOATS, WgradLoop<Q>::LDS_FLOATS)];
+struct WgradJob {
+  int w, e, b, end, m0, n0, part;  // stack w, rows b .. end of expert e; part as in Job
+};
+template <int BM, int BN, bool DEAL>
+__device__ __forceinline__ bool wgrad_job(const WgradArgs& p, int cus, int most, WgradJob& out) {
   int per_e[3], n_col[3], per = 0;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    n_col[i] = i < p.n ? (p.s[i].N + S::BN - 1) / S::BN : 0;
-    per_e[i] = i < p.n ? n_col[i] * ((p.s[i].M + S::BM - 1) / S::BM) : 0;
+    n_col[i] = i < p.n ? (p.s[i].N + BN - 1) / BN : 0;
+    per_e[i] = i < p.n ? n_col[i] * ((p.s[i].M + BM - 1) / BM) : 0;
     per += per_e[i];
   }
   const auto rows_of = [&](int e, int& first) {  // 0: none, or offsets that no dispatch would produce; -1: no such expert
@@ -514,8 +660,8 @@ __global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs
       uneven |= __ballot(heavy(rows_of(e0 + lane, at))) != 0;
     }
   }
-  const Job job = job_of(per * p.E, cus, uneven ? larger(per_e[0] / 8, 1) : 0);
-  if (job.tile < 0) return;
+  const Job job = job_of(per * p.E, cus, most, uneven ? larger(per_e[0] / 8, 1) : 0);
+  if (job.tile < 0) return false;
   int w = 0, nc = n_col[0], pe = per_e[0], tile = uneven ? job.tile % per : job.tile;
   const int share = uneven ? 1 : p.E;  // experts whose tiles of a stack follow each other
 #pragma unroll
@@ -533,15 +679,37 @@ __global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs
   } else {
     rows = rows_of(e, first);
   }
-  const int b = uniform(first), end = b + uniform(rows);
-  const F32Stack s = p.s[w];
-  int m0 = tile / nc * S::BM, n0 = tile % nc * S::BN;
-  if (job.part < 0) {
-    wgrad_tile<S>(s, lds, e, b, end, m0, n0);
+  const int b = uniform(first);
+  out = WgradJob{w, e, b, b + uniform(rows), tile / nc * BM, tile % nc * BN, job.part};
+  return true;
+}
+
+template <typename S, typename Q, bool DEAL>
+__global__ __launch_bounds__(NT, S::WAVES) void f32_wgrad_kernel(const WgradArgs p, int cus) {
+  __shared__ __align__(16) float lds[larger(WgradLoop<S>::LDS_FLOATS, WgradLoop<Q>::LDS_FLOATS)];
+  WgradJob j;
+  if (!wgrad_job<S::BM, S::BN, DEAL>(p, cus, cus * 3, j)) return;
+  const F32Stack s = p.s[j.w];
+  if (j.part < 0) {
+    wgrad_tile<S>(s, lds, j.e, j.b, j.end, j.m0, j.n0);
   } else {
-    m0 += (job.part >> 1) * Q::BM;
-    n0 += (job.part & 1) * Q::BN;
-    if (m0 < s.M && n0 < s.N) wgrad_tile<Q>(s, lds, e, b, end, m0, n0);
+    j.m0 += (j.part >> 1) * Q::BM;
+    j.n0 += (j.part & 1) * Q::BN;
+    if (j.m0 < s.M && j.n0 < s.N) wgrad_tile<Q>(s, lds, j.e, j.b, j.end, j.m0, j.n0);
+  }
+}
+template <typename S, typename Q, bool DEAL>
+__global__ __launch_bounds__(S::NT, S::NT / 256) void f32_split_wgrad_kernel(const WgradArgs p, int cus) {
+  extern __shared__ __align__(16) char split_lds[];
+  WgradJob j;
+  if (!wgrad_job<S::BM, S::BN, DEAL>(p, cus, split_cut(p.R / p.E, cus), j)) return;
+  const F32Stack s = p.s[j.w];
+  if (j.part < 0) {
+    split_wgrad_tile<S>(s, split_lds, j.e, j.b, j.end, j.m0, j.n0);
+  } else {
+    j.m0 += (j.part >> 1) * Q::BM;
+    j.n0 += (j.part & 1) * Q::BN;
+    if (j.m0 < s.M && j.n0 < s.N) split_wgrad_tile<Q>(s, split_lds, j.e, j.b, j.end, j.m0, j.n0);
   }
 }
 
@@ -550,7 +718,20 @@ using Quarter = Shape<32, 32, 32, 1, 1, 4>;  // of Small: the four waves share t
 using Large = Shape<128, 128, 16, 2, 2, 2>;  // three by their registers
 using LargeQuarter = Shape<64, 64, 16, 2, 2, 2>;
 
+using SplitTile = SplitShape<128, 128, 32, 2, 2, 2>;   // eight waves
+using SplitQuarter = SplitShape<64, 64, 64, 1, 2, 4>;
+
 int forced_tile = 0;
+template <typename K>
+int set_lds(K kern, bool (&done)[MOE_MAX_DEVICES], int bytes) {
+  const int dev = moe_current_device();
+  if (!done[dev]) {
+    const hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (err != hipSuccess) return (int)err;
+    done[dev] = true;
+  }
+  return 0;
+}
 // The large tile has half the operand traffic and LDS reads per flop (32768 rows of 8 experts, 2048 <-> 1024, gate and up: 1.99
 // against 2.17 ms, 138 TFLOP/s), but few of them share a compute unit less evenly (8192 rows of 16 experts, 1024 <-> 1024, five
 // rounds of large tiles: 335 against 295 us; three rounds: equal): from eight rounds on.  So, too, for weight gradients,
@@ -562,6 +743,21 @@ int forced_tile = 0;
 bool large_tiles(int64_t tiles128) {
   if (forced_tile) return forced_tile == 128;
   return tiles128 >= 8 * (int64_t)moe_compute_units();
+}
+
+// Split tiles (f32_split.h) keep a whole compute unit busy for 9 us and 0.03 us for each of the contraction's values: they take
+// launches with work for the chip and experts that fill a tile at least half (weight gradients: that have some length).  The
+// rules below are within 1.2 % (weight gradients 0.4 %) of the better side in the mean over 160 launches of each kind, 4 to
+// 128 experts, 64 to 32768 rows, 256 <-> 128 to 2048 <-> 1024.  4096 rows of 8 experts, 1024 <-> 512, the five
+// launches, fp32 tiles and these: 77, 43, 46, 76, 108 and 56, 34, 40, 54, 71 us; 256 rows: 67 and 85 us in all.
+constexpr int SPLIT = 1;
+bool split_rows(int64_t E, int64_t R, int64_t N, int64_t K) {
+  if (forced_tile) return forced_tile == SPLIT;
+  return R >= 64 * E && K >= 384 && R * N >= ((int64_t)1 << 30) / K;
+}
+bool split_wgrad(int64_t E, int64_t R, int64_t elements) {
+  if (forced_tile) return forced_tile == SPLIT;
+  return R >= 192 * E && elements >= ((int64_t)1 << 30) / R;
 }
 
 int check_rows(int64_t E, int64_t R, int64_t N, int64_t K) {
@@ -578,6 +774,14 @@ int launch_rows(RowsArgs a, int64_t E, int64_t R, int64_t N, int64_t K, hipStrea
   a.E = (int)E, a.R = (int)R, a.N = (int)N, a.K = (int)K;
   const int cus = moe_compute_units();
   const auto tiles = [&](int64_t t) { return (R / t + E) * ((N * (MODE == GATEUP ? 2 : 1) + t - 1) / t); };  // at most
+  if (split_rows(E, R, N * (MODE == GATEUP ? 2 : 1), K * (MODE == GATEUP_BWD ? 2 : 1))) {
+    constexpr int LDS = larger(SplitRowsLoop<MODE, SplitTile>::LDS_BYTES, SplitRowsLoop<MODE, SplitQuarter>::LDS_BYTES);
+    static bool done[MOE_MAX_DEVICES];
+    const auto kern = f32_split_rows_kernel<MODE, SplitTile, SplitQuarter>;
+    if (int rc = set_lds(kern, done, LDS)) return rc;
+    hipLaunchKernelGGL(kern, dim3(grid_of(tiles(128), cus)), dim3(SplitTile::NT), LDS, s, a, cus);
+    return moe_launch_status();
+  }
   if (large_tiles(tiles(128)))
     hipLaunchKernelGGL((f32_rows_kernel<MODE, Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, s, a, cus);
   else
@@ -668,20 +872,34 @@ static int wgrads(const F32Stack* s, int n, const int32_t* offs, int64_t E, int6
   }
   if (tiles(64) > 0x70000000ll) return MOE_ERR_LIMIT;
   const int cus = moe_compute_units();
-  const bool large = large_tiles(tiles(128));
+  int64_t elements = 0;
+  for (int i = 0; i < n; ++i) elements += s[i].M * (int64_t)s[i].N;
+  const bool large = large_tiles(tiles(128)), split = R > 0 && split_wgrad(E, R, elements);
   const auto go = [&](auto deal) {
     constexpr bool DEAL = decltype(deal)::value;
+    if (split) {
+      constexpr int LDS = larger(SplitWgradLoop<SplitTile>::LDS_BYTES, SplitWgradLoop<SplitQuarter>::LDS_BYTES);
+      static bool done[MOE_MAX_DEVICES];
+      const auto kern = f32_split_wgrad_kernel<SplitTile, SplitQuarter, DEAL>;
+      if (int rc = set_lds(kern, done, LDS)) return rc;
+      hipLaunchKernelGGL(kern, dim3(grid_of(tiles(128), cus)), dim3(SplitTile::NT), LDS, st, p, cus);
+      return 0;
+    }
     if (large)
       hipLaunchKernelGGL((f32_wgrad_kernel<Large, LargeQuarter, DEAL>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, st, p, cus);
     else
       hipLaunchKernelGGL((f32_wgrad_kernel<Small, Quarter, DEAL>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, st, p, cus);
+    return 0;
   };
   // Times as fast with a look at the offsets as without, up to 64 experts, even loads and loads with a heavy expert: tiles of
   // 64, below 32 rows an expert 0.86 to 0.91, 0.87 to 1.0; 64 to 128 rows 0.94, 1.25; 128 to 256 rows 0.98, 1.35; more 0.99,
   // 1.45.  Tiles of 128: below 64 rows 0.91 to 0.97, 1.03 to 1.13; 64 to 128 rows 0.98, 1.19; more 0.99, 1.3.  Of 128 experts,
   // which are not sorted, 128 rows each: 0.95, 1.1.
-  if (R >= (E > MOE_WAVE ? 256 : large ? 64 : 128) * E) go(std::true_type{});
-  else go(std::false_type{});
+  if (R >= (E > MOE_WAVE ? 256 : large || split ? 64 : 128) * E) {
+    if (int rc = go(std::true_type{})) return rc;
+  } else if (int rc = go(std::false_type{})) {
+    return rc;
+  }
   return moe_launch_status();
 }
 
@@ -711,11 +929,11 @@ extern "C" int moe_f32_gemm_wgrad(const float* a, const float* b, const int32_t*
   return wgrads(&s, 1, offs, E, R, (hipStream_t)stream);
 }
 
-// Test hook: 0 lets every fp32 GEMM launch choose its tile (the default), 64 or 128 forces it.
+// Test hook: 0 lets every fp32 GEMM launch choose its tile (the default), 64 or 128 forces it, 1 the split tiles.
 // Process-wide and not synchronised: for tests, not for production callers.  Returns the previous
 // setting.
 extern "C" int moe_f32_gemm_force_tile(int t) {
   const int before = forced_tile;
-  if (t == 0 || t == 64 || t == 128) forced_tile = t;
+  if (t == 0 || t == SPLIT || t == 64 || t == 128) forced_tile = t;
   return before;
 }
