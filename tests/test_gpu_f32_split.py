@@ -163,3 +163,23 @@ def test_two_runs_give_the_same_bits(pkg, lib, forced):
     old = torch.randn(4, I, H, generator=g).cuda()
     acc = pkg.ops.f32_gemm_wgrad(one[0], x, o, 4, out=old.clone())
     assert torch.equal(acc, torch.where(torch.tensor(counts, device="cuda").view(4, 1, 1) > 0, dw[0] + old, old))
+
+
+@pytest.mark.parametrize("E,R,N,K", [
+    (4, 2176, 2048, 256),    # the shortest contraction the split tiles take where there is work enough
+    (4, 2176, 2048, 252),    # shorter: fp32 products
+    (32, 2048, 2048, 260),   # experts that fill half a tile
+    (32, 2047, 2048, 260),   # ... a row less
+    (128, 1020, 2584, 36),   # many large tiles by the bound, of few rows: small ones
+])
+def test_at_the_lines_of_the_rule(pkg, lib, forced, E, R, N, K):
+    forced(0)
+    g = torch.Generator().manual_seed(R + K)
+    counts = [R // E + (e < R % E) for e in range(E)]
+    a, b = torch.randn(R, K, generator=g), torch.randn(E, N, K, generator=g)
+    got = pkg.ops.f32_gemm_rows(a.cuda(), b.cuda(), _offs(counts).cuda(), True)
+    parts, sizes = a.double().split(counts), a.double().abs().split(counts)
+    ref = torch.cat([p @ w.double().t() for p, w in zip(parts, b)])
+    size = torch.cat([p @ w.double().abs().t() for p, w in zip(sizes, b)])
+    # (either tile: at most a rounding for every product of the contraction, and the parts that the split leaves out)
+    assert ((got.cpu().double() - ref).abs() <= (K * 2.0 ** -24 + 2.0 ** -22) * size + 2.0 ** -37 * size.max()).all()

@@ -739,7 +739,9 @@ int set_lds(K kern, bool (&done)[MOE_MAX_DEVICES], int bytes) {
 // where a router with random weights deals the rows (4096 rows of 8 experts, three stacks of 1024 x 512, three rounds: 120 us
 // against 126), and slower where it does not: with logits off by 0.3 from expert to expert 0.90 to 1.03 times as fast on
 // average and down to 0.42 (16384 rows of 128 experts, 256 x 128: 220 us against 92), with Zipf's shares 0.67 to 0.81 and
-// down to 0.31.  From eight rounds on: 1.04, 1.08 and 1.03 times as fast.
+// down to 0.31.  From eight rounds on: 1.04, 1.08 and 1.03 times as fast.  Rounds by the bound, which has a tile for every
+// expert: row launches whose experts do not fill half of one stay with the small tile (1020 rows of 128 experts, 2584 <-> 288, down and
+// dgrad-gate/up 173, 315 us in large tiles, 105 and 171 in small ones).
 bool large_tiles(int64_t tiles128) {
   if (forced_tile) return forced_tile == 128;
   return tiles128 >= 8 * (int64_t)moe_compute_units();
@@ -747,13 +749,17 @@ bool large_tiles(int64_t tiles128) {
 
 // Split tiles (f32_split.h) keep a whole compute unit busy for 9 us and 0.03 us for each of the contraction's values: they take
 // launches with work for the chip and experts that fill a tile at least half (weight gradients: that have some length).  The
-// rules below are within 1.2 % (weight gradients 0.4 %) of the better side in the mean over 160 launches of each kind, 4 to
-// 128 experts, 64 to 32768 rows, 256 <-> 128 to 2048 <-> 1024.  4096 rows of 8 experts, 1024 <-> 512, the five
-// launches, fp32 tiles and these: 77, 43, 46, 76, 108 and 56, 34, 40, 54, 71 us; 256 rows: 67 and 85 us in all.
+// fused launches, where the second operand or the epilogue takes a tile longer, also need tiles for most compute units, by the
+// bound on their number.  The rules below are within 1.1 % (weight gradients 2.1 %) of the best of the three tiles in the mean
+// over 1040 row launches and 260 of weight gradients: 4 to 128 experts, 64 to 32768 rows, widths 256 to 4096 and 128 to 2048.
+// 4096 rows of 8 experts, 1024 <-> 512, the five launches, fp32 tiles and these: 77, 43, 46, 76, 108 and 56, 34, 40,
+// 54, 71 us; 256 rows: 67 and 85 us in all.  Contractions of 256 to 384 (taken) gain less: 13992 rows of 12 experts, 2368 <-> 256,
+// down 164 -> 132; 21996 of 32, 768 <-> 256, 84 -> 72.  Few tiles (not taken): 1492 rows of 12, 1920 <-> 448, dgrad-down, 48 to 92
+// tiles, 45 and 62.
 constexpr int SPLIT = 1;
-bool split_rows(int64_t E, int64_t R, int64_t N, int64_t K) {
+bool split_rows(int64_t E, int64_t R, int64_t N, int64_t K, int64_t tiles128, bool fused) {
   if (forced_tile) return forced_tile == SPLIT;
-  return R >= 64 * E && K >= 384 && R * N >= ((int64_t)1 << 30) / K;
+  return R >= 64 * E && K >= 256 && R * N >= ((int64_t)1 << 30) / K && (!fused || tiles128 * 8 >= 5 * (int64_t)moe_compute_units());
 }
 bool split_wgrad(int64_t E, int64_t R, int64_t elements) {
   if (forced_tile) return forced_tile == SPLIT;
@@ -774,7 +780,8 @@ int launch_rows(RowsArgs a, int64_t E, int64_t R, int64_t N, int64_t K, hipStrea
   a.E = (int)E, a.R = (int)R, a.N = (int)N, a.K = (int)K;
   const int cus = moe_compute_units();
   const auto tiles = [&](int64_t t) { return (R / t + E) * ((N * (MODE == GATEUP ? 2 : 1) + t - 1) / t); };  // at most
-  if (split_rows(E, R, N * (MODE == GATEUP ? 2 : 1), K * (MODE == GATEUP_BWD ? 2 : 1))) {
+  constexpr bool FUSED = MODE == GATEUP || MODE == DOWN_BWD || MODE == GATEUP_BWD;
+  if (split_rows(E, R, N * (MODE == GATEUP ? 2 : 1), K * (MODE == GATEUP_BWD ? 2 : 1), tiles(128), FUSED)) {
     constexpr int LDS = larger(SplitRowsLoop<MODE, SplitTile>::LDS_BYTES, SplitRowsLoop<MODE, SplitQuarter>::LDS_BYTES);
     static bool done[MOE_MAX_DEVICES];
     const auto kern = f32_split_rows_kernel<MODE, SplitTile, SplitQuarter>;
@@ -782,7 +789,7 @@ int launch_rows(RowsArgs a, int64_t E, int64_t R, int64_t N, int64_t K, hipStrea
     hipLaunchKernelGGL(kern, dim3(grid_of(tiles(128), cus)), dim3(SplitTile::NT), LDS, s, a, cus);
     return moe_launch_status();
   }
-  if (large_tiles(tiles(128)))
+  if (large_tiles(tiles(128)) && (R >= 64 * E || forced_tile))
     hipLaunchKernelGGL((f32_rows_kernel<MODE, Large, LargeQuarter>), dim3(grid_of(tiles(128), cus)), dim3(NT), 0, s, a, cus);
   else
     hipLaunchKernelGGL((f32_rows_kernel<MODE, Small, Quarter>), dim3(grid_of(tiles(64), cus)), dim3(NT), 0, s, a, cus);
