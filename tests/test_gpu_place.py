@@ -78,3 +78,36 @@ def test_the_count_of_bad_ids_is_written_with_logits(pkg, lib, T, E):
         T, H, E, I, k, p(x), bf16, p(logits), bf16, 0, 0, p(w1), p(w3), p(w2), 0, p(out), bf16, p(ids), p(gates),
         p(counts), p(offs), p(p2r), p(r2p), p(bad), p(xp), 0, p(act), p(scratch), scratch.numel()), ops._stream())
     assert bad.item() == 0 and counts.sum().item() == T * k
+
+
+@pytest.mark.parametrize("T,E,k,H,x_dt", [
+    (1, 16, 1, 32, torch.float32),         # one token, one wave of experts' product
+    (15, 16, 16, 64, torch.bfloat16),      # a chunk one token short, every expert asked for
+    (16, 48, 3, 544, torch.float32),       # a full one; column blocks that not every wave has
+    (17, 128, 64, 1056, torch.float32),    # one more; as many experts as are taken
+    (300, 80, 2, 2080, torch.bfloat16),    # rows that leave LDS for one block
+    (2049, 112, 8, 128, torch.float32),
+    (12288, 128, 2, 32, torch.float32),    # the largest table
+    (12289, 128, 2, 32, torch.float32),    # one token more: the general path
+])
+def test_places_behind_the_norm(pkg, lib, T, E, k, H, x_dt):
+    """Norm, router and selection in one kernel, which leaves the counts: the routing against numpy on its logits, the output
+    against the layer on the normalised rows with those logits."""
+    print("places behind the norm", T, E, k, H, x_dt, flush=True)
+    g = torch.Generator().manual_seed(T + E)
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).cuda()
+    x, nw, wr = r(T, H).to(x_dt), 1.0 + r(H, std=0.1), r(E, H, std=0.05).to(torch.bfloat16)
+    ws = [r(*s, std=0.1).to(torch.bfloat16) for s in ((E, 8, H), (E, 8, H), (E, H, 8))]
+    out, logits, rt = pkg.prenorm_moe(x, nw, wr, *ws, k, eps=1e-6, add_residual=False, return_routing=True)
+    flat = O.topk_select(logits.float().cpu(), k)[0].reshape(-1)
+    order = np.argsort(flat, kind="stable")
+    counts = np.bincount(flat, minlength=E)
+    inverse = np.empty_like(order)
+    inverse[order] = np.arange(T * k)
+    for name, want in (("ids", flat), ("counts", counts), ("offs", np.concatenate([[0], counts.cumsum()])),
+                       ("pos_to_row", order), ("row_to_pos", inverse)):
+        assert np.array_equal(rt[name].cpu().numpy(), want.astype(np.int32)), name
+    xn, _ = pkg.ops.rmsnorm_fwd(x, nw, 1e-6)
+    y, rows = pkg.moe_ffn(xn, logits, *ws, k, return_routing=True)
+    assert torch.equal(rt["gates"], rows["gates"])
+    assert torch.equal(out.to(torch.bfloat16), y)  # (the same kernels from the rows on; fp32 x: an fp32 result, rounded here)

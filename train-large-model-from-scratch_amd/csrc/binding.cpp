@@ -30,6 +30,10 @@ int moe_select_count(const void* logits, int logits_dtype, const float* bias, in
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
                    int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
                    void* xp, int xp_dtype, void* stream);
+int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, float eps, const uint16_t* router_weight,
+                             int64_t T, int64_t H, int64_t E, int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
+                             int32_t* ids, float* gates, void* table, void* stream);
+int moe_selected_layer_forward(const moe_layer_forward_args* a, const void* table, void* stream);
 int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
                    int64_t I, float* g, float* u, float* act, void* stream);
 int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
@@ -237,6 +241,7 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   const Routing r(R, E);
   Tensor rows = x;
   Tensor logits;
+  Tensor table;  // of the selection's counts, where it is done and they are wanted
   bool selected = false, inside = false;  // selection done; the forward-only call makes the logits itself
   const Tensor b = bias.defined() ? dense(bias) : Tensor();
   if (o.train || o.routing_out || !(wr.defined() || logits_.defined()) || norm_w.defined() || T == 0)
@@ -260,9 +265,10 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
         // norm, router product and selection in one kernel: the normalised rows are not read a second
         // time for the router, the logits are selected on before they leave the chip
         logits = empty({T, E}, at::kBFloat16, x);
-        CALL(moe_rmsnorm_router_fwd, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, bf(f.wrb), T, H,
+        if (moe_place_ok(T, E, k)) table = empty({moe_place_bytes(T, E)}, at::kByte, x);
+        CALL(moe_rmsnorm_router_count, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, bf(f.wrb), T, H,
              E, k, (uint16_t*)f.xn.data_ptr(), f.rstd.data_ptr<float>(), (uint16_t*)logits.data_ptr(),
-             r.part(f.routing, Routing::IDS), (float*)r.part(f.routing, Routing::GATES), s);
+             r.part(f.routing, Routing::IDS), (float*)r.part(f.routing, Routing::GATES), ptr(table), s);
         selected = true;
       } else {
         CALL(moe_rmsnorm_fwd, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, T, H,
@@ -332,7 +338,7 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   a.gu = o.train ? base + kept.gu : nullptr;
   a.act = (uint16_t*)(base + kept.act);
   a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
-  check(moe_layer_forward(&a, s), "moe_layer_forward");
+  check(moe_selected_layer_forward(&a, ptr(table), s), "moe_layer_forward");
   if (o.routing_out) *o.routing_out = f.routing;
   return f;
 }

@@ -46,7 +46,8 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
                     int64_t router_rows, hipStream_t s);
 
 // ---- selection, places and rows in two launches (place.hip) ----
-// Sizes it takes, and the bytes of its table of counts.
+// Sizes it takes, and the bytes of its table of counts: (E + 3) / 4 words for every so many tokens, a byte an expert.
+constexpr int MOE_PLACE_CHUNK = 16;
 bool moe_place_ok(int64_t T, int64_t E, int64_t k);
 int64_t moe_place_bytes(int64_t T, int64_t E);
 // moe_router_topk_fwd that leaves the table, and from it the results of moe_histogram_scan and moe_permute_fwd (fp32 rows
@@ -56,6 +57,11 @@ int moe_select_count(const void* logits, int logits_dtype, const float* bias, in
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
                    int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
                    void* xp, int xp_dtype, void* stream);
+
+// moe_rmsnorm_router_fwd that leaves the table too, unless it is NULL (norm.hip).
+int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, float eps, const uint16_t* router_weight,
+                             int64_t T, int64_t H, int64_t E, int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
+                             int32_t* ids, float* gates, void* table, void* stream);
 
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;

@@ -297,7 +297,8 @@ extern "C" int64_t moe_layer_scratch_bytes(int64_t T, int64_t H, int64_t E, int6
   return s.at;
 }
 
-extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) {
+// With `table` the selection is done, ids and gates are there, and so are its counts (moe_rmsnorm_router_count).
+static int layer_forward(const moe_layer_forward_args* a, const void* table, void* stream) {
   if (!a) return MOE_ERR_NULL;
   const int64_t T = a->T, H = a->H, E = a->E, I = a->I, k = a->k, R = T * k;
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
@@ -323,10 +324,11 @@ extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) 
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
   const FwdScratch ws(s, T, H, E, k);
   if (!s.fits()) return MOE_ERR_WORKSPACE;
-  if (a->logits && moe_place_ok(T, E, k)) {
-    MOE_STEP("moe_select_count", moe_select_count(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids, a->gates,
-                                                  ws.dispatch, stream));
-    MOE_STEP("moe_place_rows", moe_place_rows(a->x, (int)a->x_dtype, a->ids, ws.dispatch, T, H, E, k, a->counts, a->offs,
+  if ((a->logits || table) && moe_place_ok(T, E, k)) {
+    if (!table)
+      MOE_STEP("moe_select_count", moe_select_count(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids, a->gates,
+                                                    ws.dispatch, stream));
+    MOE_STEP("moe_place_rows", moe_place_rows(a->x, (int)a->x_dtype, a->ids, table ? table : ws.dispatch, T, H, E, k, a->counts, a->offs,
                                               a->pos_to_row, a->row_to_pos, a->bad_ids, a->xp, MOE_DT_BF16, stream));
   } else {
     if (a->logits)
@@ -357,6 +359,12 @@ extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) 
     MOE_STEP("moe_combine_fwd", moe_combine_fwd(ws.y, a->gates, a->row_to_pos, T, H, k, a->out, (int)a->out_dtype,
                                                 stream));
   return 0;
+}
+
+extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) { return layer_forward(a, nullptr, stream); }
+
+int moe_selected_layer_forward(const moe_layer_forward_args* a, const void* table, void* stream) {
+  return layer_forward(a, table, stream);
 }
 
 extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream) {

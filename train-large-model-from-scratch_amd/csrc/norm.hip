@@ -12,6 +12,7 @@
 // is reproducible run to run.  Both kernels are HBM-bound: each row is read once and written
 // once.
 #include "common.h"
+#include "internal.h"
 #include "topk_core.h"
 
 namespace {
@@ -86,39 +87,52 @@ __global__ __launch_bounds__(NT) void rmsnorm_fwd_kernel(const XT* __restrict__ 
 // The normalisation with the router behind it (model/gpt.py:32 into model/modules/mlp.py:100-103
 // in one pass): a block normalises RB rows, keeps their bf16 form in LDS besides writing it out,
 // multiplies them with the router weight on the matrix cores (v_mfma_f32_16x16x32_bf16: rows =
-// tokens from LDS, columns = experts straight from L2, the four waves split the contraction and
-// add their partial products through LDS), rounds the logits to bf16 (what the layer returns and
+// tokens from LDS, columns = experts straight from L2, the contraction split in four and the
+// partial products added through LDS), rounds the logits to bf16 (what the layer returns and
 // selects on) and runs the wave-level top-k + softmax on them.  The normalised rows are not read
-// again for the router, and the logits never leave the chip before selection.
+// again for the router, and the logits never leave the chip before selection.  Where place.hip takes the
+// tokens, the block also leaves its experts' counts in that table, which takes three launches away from behind it.
 constexpr int RB = 16;       // rows (tokens) per block
 constexpr int RMAX_EB = 8;   // 16-expert column blocks: E <= 128
+constexpr int ROUTER_WAVES = 16;
+// Waves a SIMD that two blocks on a compute unit make (rows past 2048 wide leave LDS for one)
+template <int NV, int WAVES>
+constexpr int ROUTER_EU = (NV <= 4 ? 2 : 1) * WAVES / 4;
 
-template <typename XT, int NV>
-__global__ __launch_bounds__(NT) void rmsnorm_router_fwd_kernel(
+// What bounds it: all blocks of a launch of 8192 tokens are resident at once and go through load, product and selection
+// together, each of them a chain of trips to memory or L2.  Sixteen waves, a row and a token's selection each, make the chains
+// as short as they get; two such blocks fill a compute unit's wave slots (54 registers).  8192 rows of 2048 in fp32, 64 experts,
+// 8 a token: 50.9 us with four waves of four rows, 39.9 here (100 MB: 19); with the launches up to the rows in expert
+// order 123 -> 100.  A whole training pass of 24 drawn layers with it 1.00 to 1.10 times as fast where the GPU bounds it.
+template <typename XT, int NV, int WAVES>
+__global__ __launch_bounds__(WAVES* MOE_WAVE, (ROUTER_EU<NV, WAVES>)) void rmsnorm_router_fwd_kernel(
     const XT* __restrict__ x, const float* __restrict__ w, float eps, int T, int H8,
     const uint16_t* __restrict__ wr, int E, int k, uint16_t* __restrict__ xn, float* __restrict__ rstd,
-    uint16_t* __restrict__ logits, int32_t* __restrict__ ids, float* __restrict__ gates) {
+    uint16_t* __restrict__ logits, int32_t* __restrict__ ids, float* __restrict__ gates, uint32_t* __restrict__ table) {
+  static_assert(RB == MOE_PLACE_CHUNK && WAVES % NW == 0 && RB % WAVES == 0, "a block counts a chunk's tokens");
   extern __shared__ __attribute__((aligned(16))) uint16_t rows[];  // [RB][H + 8]; later fp32 partials
   __shared__ uint16_t lg16[RB * RMAX_EB * 16];
+  __shared__ uint32_t asked[RMAX_EB * 16];  // bit t: token t of the block asks for the expert
   const int H = H8 * 8, LDT = H + 8;
-  const int lane = lane_id(), wv = threadIdx.x / MOE_WAVE;
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE));
   const int t0 = blockIdx.x * RB;
-  // normalisation: a wave per row, its next row requested before this one is reduced (a block-wide
-  // reduction per row, 16 in a row, left the kernel waiting: 62 us for 8192 rows of 2048, now 55)
-  Row8 xv[NV], nx[NV];
-  const auto request = [&](int rr, Row8(&to)[NV]) {
-    if (t0 + rr >= T) return;
+  if (threadIdx.x < RMAX_EB * 16) asked[threadIdx.x] = 0;
+  // normalisation: a wave per row, all of a wave's rows requested before the first is reduced
+  constexpr int OWN = RB / WAVES;
+  Row8 xs[OWN][NV];
+#pragma unroll
+  for (int q = 0; q < OWN; ++q) {
+    const int rr = wv + q * WAVES;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int c = lane + i * MOE_WAVE;
-      if (c < H8) to[i] = load8(x + (size_t)(t0 + rr) * H + c * 8);
+      if (t0 + rr < T && c < H8) xs[q][i] = load8(x + (size_t)(t0 + rr) * H + c * 8);
     }
-  };
-  request(wv, xv);
+  }
 #pragma unroll
-  for (int q = 0; q < RB / NW; ++q) {
-    const int rr = wv + q * NW, t = t0 + rr;
-    if (q + 1 < RB / NW) request(rr + NW, nx);
+  for (int q = 0; q < OWN; ++q) {
+    const int rr = wv + q * WAVES, t = t0 + rr;
+    const Row8(&xv)[NV] = xs[q];
     if (t >= T) {  // wave-uniform: rows past the end are zero rows for the product
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
@@ -159,60 +173,72 @@ __global__ __launch_bounds__(NT) void rmsnorm_router_fwd_kernel(
         store8(rows + rr * LDT + c * 8, o);
       }
     }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) xv[i] = nx[i];
   }
   __syncthreads();
   // logits[m][e] = sum_h rows[m][h] * wr[e][h]: lane l holds A row l % 16 (token) and B row
-  // l % 16 of the column block (expert), 8 consecutive h at (l / 16) * 8 of the 32-wide k-step
-  const int EB = E / 16;
-  f32x4 acc[RMAX_EB];
+  // l % 16 of the column block (expert), 8 consecutive h at (l / 16) * 8 of the 32-wide k-step.
+  // Wave wv has every NW-th k-step from wv % NW on, and of the column blocks every GROUPS-th from wv / NW on: the sums do not depend on
+  // the number of waves.
+  constexpr int GROUPS = WAVES / NW, MINE = RMAX_EB / GROUPS;
+  const int EB = E / 16, kg = wv % NW, cg = wv / NW;
+  f32x4 acc[MINE];
 #pragma unroll
-  for (int nb = 0; nb < RMAX_EB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int nb = 0; nb < MINE; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int l16 = lane & 15, lq = lane >> 4;
-  // (the router's rows come from L2: a step's are requested while the step before is multiplied)
+  // (the router's rows come from L2: so many k-steps' are requested while as many before are multiplied)
   const auto product = [&](auto eb_c) {
-    constexpr int EBT = decltype(eb_c)::value;  // column blocks, EB rounded up: the surplus repeats the last
-    bf16x8 b[2][EBT];
-    const auto request = [&](int ks, bf16x8(&to)[EBT]) {
+    constexpr int EBT = decltype(eb_c)::value;  // column blocks, rounded up: the surplus repeats the last
+    constexpr int AHEAD = EBT <= 2 ? 4 / EBT : 1;
+    bf16x8 b[2][AHEAD][EBT];
+    const int n = (H / 32 - kg + NW - 1) / NW;  // this wave's k-steps
+    const auto request = [&](int s, bf16x8(&to)[AHEAD][EBT]) {
 #pragma unroll
-      for (int nb = 0; nb < EBT; ++nb) {
-        const int n = nb < EB ? nb : EB - 1;
-        to[nb] = *reinterpret_cast<const bf16x8*>(wr + (size_t)(n * 16 + l16) * H + ks * 32 + lq * 8);
+      for (int d = 0; d < AHEAD; ++d) {
+        if (s + d >= n) break;
+        const int ks = kg + (s + d) * NW;
+#pragma unroll
+        for (int nb = 0; nb < EBT; ++nb) {
+          const int c = cg + nb * GROUPS < EB ? cg + nb * GROUPS : EB - 1;
+          to[d][nb] = *reinterpret_cast<const bf16x8*>(wr + (size_t)(c * 16 + l16) * H + ks * 32 + lq * 8);
+        }
       }
     };
-    const auto step = [&](int ks, const bf16x8(&from)[EBT]) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(rows + l16 * LDT + ks * 32 + lq * 8);
+    const auto multiply = [&](int s, const bf16x8(&from)[AHEAD][EBT]) {
 #pragma unroll
-      for (int nb = 0; nb < EBT; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, from[nb], acc[nb], 0, 0, 0);
+      for (int d = 0; d < AHEAD; ++d) {
+        if (s + d >= n) break;
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(rows + l16 * LDT + (kg + (s + d) * NW) * 32 + lq * 8);
+#pragma unroll
+        for (int nb = 0; nb < EBT; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, from[d][nb], acc[nb], 0, 0, 0);
+      }
     };
-    const int n = H / 32;
-    int ks = wv;
-    if (ks < n) request(ks, b[0]);
-    for (; ks < n; ks += 2 * NW) {
-      if (ks + NW < n) request(ks + NW, b[1]);
-      step(ks, b[0]);
-      if (ks + NW >= n) break;
-      if (ks + 2 * NW < n) request(ks + 2 * NW, b[0]);
-      step(ks + NW, b[1]);
+    request(0, b[0]);
+    for (int s = 0; s < n; s += 2 * AHEAD) {
+      request(s + AHEAD, b[1]);
+      multiply(s, b[0]);
+      request(s + 2 * AHEAD, b[0]);
+      multiply(s + AHEAD, b[1]);
     }
   };
-  if (EB <= 1) product(std::integral_constant<int, 1>{});
-  else if (EB <= 2) product(std::integral_constant<int, 2>{});
-  else if (EB <= 4) product(std::integral_constant<int, 4>{});
-  else product(std::integral_constant<int, 8>{});
+  if (cg < EB) {
+    const int mine = (EB - cg + GROUPS - 1) / GROUPS;
+    if (mine <= 1) product(std::integral_constant<int, 1>{});
+    else if (MINE <= 2 || mine <= 2) product(std::integral_constant<int, 2>{});
+    else product(std::integral_constant<int, MINE>{});
+  }
   __syncthreads();  // every wave is done with the rows: their memory takes the partial products
   float* part = reinterpret_cast<float*>(rows);  // [NW][RB][E]
   // accumulator layout: lane l holds column l % 16 (expert) of rows 4 * (l / 16) .. + 3 (tokens)
 #pragma unroll
-  for (int nb = 0; nb < RMAX_EB; ++nb) {
-    if (nb < EB) {
+  for (int nb = 0; nb < MINE; ++nb) {
+    const int c = cg + nb * GROUPS;
+    if (c < EB) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) part[(wv * RB + lq * 4 + i) * E + nb * 16 + l16] = acc[nb][i];
+      for (int i = 0; i < 4; ++i) part[(kg * RB + lq * 4 + i) * E + c * 16 + l16] = acc[nb][i];
     }
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < RB * E; idx += NT) {
+  for (int idx = threadIdx.x; idx < RB * E; idx += WAVES * MOE_WAVE) {
     float v = 0.f;
 #pragma unroll
     for (int q = 0; q < NW; ++q) v += part[q * RB * E + idx];  // fixed order: reproducible
@@ -223,8 +249,9 @@ __global__ __launch_bounds__(NT) void rmsnorm_router_fwd_kernel(
   }
   __syncthreads();
   // selection: one wave per token
-  for (int m = wv; m < RB; m += NW) {
-    const int t = t0 + m;
+#pragma unroll
+  for (int q = 0; q < OWN; ++q) {
+    const int m = wv + q * WAVES, t = t0 + m;
     if (t >= T) break;
     uint32_t key[2];
 #pragma unroll
@@ -234,11 +261,26 @@ __global__ __launch_bounds__(NT) void rmsnorm_router_fwd_kernel(
     }
     int my_id;
     float my_gate;
-    moe_topk_softmax_wave<2>(key, k, lane, my_id, my_gate);
+    if (E <= MOE_WAVE) {
+      uint32_t one[1] = {key[0]};
+      moe_topk_softmax_wave<1>(one, k, lane, my_id, my_gate);
+    } else {
+      moe_topk_softmax_wave<2>(key, k, lane, my_id, my_gate);
+    }
     if (lane < k) {
       ids[(size_t)t * k + lane] = my_id;
       gates[(size_t)t * k + lane] = my_gate;
+      if (table) atomicOr(&asked[my_id], 1u << m);
     }
+  }
+  if (!table) return;
+  __syncthreads();
+  const int words = (E + 3) / 4;  // (a row of place.hip's table)
+  if (threadIdx.x < words) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) c |= (uint32_t)__popc(asked[threadIdx.x * 4 + b]) << (8 * b);
+    table[(size_t)blockIdx.x * words + threadIdx.x] = c;
   }
 }
 
@@ -412,10 +454,9 @@ extern "C" int moe_rmsnorm_router_supported(int64_t H, int64_t E, int64_t k) {
              ? 1 : 0;
 }
 
-extern "C" int moe_rmsnorm_router_fwd(const void* x, int x_dtype, const float* weight, float eps,
-                                      const uint16_t* router_weight, int64_t T, int64_t H, int64_t E,
-                                      int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
-                                      int32_t* ids, float* gates, void* stream) {
+int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, float eps, const uint16_t* router_weight,
+                             int64_t T, int64_t H, int64_t E, int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
+                             int32_t* ids, float* gates, void* table, void* stream) {
   if (int rc = check_norm(T, H)) return rc;
   if (E <= 0 || k <= 0 || k > E) return MOE_ERR_SHAPE;
   if (!moe_rmsnorm_router_supported(H, E, k)) return MOE_ERR_LIMIT;
@@ -426,13 +467,13 @@ extern "C" int moe_rmsnorm_router_fwd(const void* x, int x_dtype, const float* w
   MOE_CHECK_PTR(xn);
   if (!rstd || !logits || !ids || !gates) return MOE_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)((T + RB - 1) / RB)), block(NT);
+  const dim3 grid((unsigned)((T + RB - 1) / RB)), block(ROUTER_WAVES * MOE_WAVE);
   const size_t lds = (size_t)RB * (H + 8) * 2 > (size_t)NW * RB * E * 4 ? (size_t)RB * (H + 8) * 2 : (size_t)NW * RB * E * 4;
   constexpr int MAX_ROUTER_LDS = RB * (4096 + 8) * 2 > NW * RB * 16 * RMAX_EB * 4 ? RB * (4096 + 8) * 2 : NW * RB * 16 * RMAX_EB * 4;
   if (lds > (size_t)MAX_ROUTER_LDS) return MOE_ERR_LIMIT;
 #define MOE_NORM_ROUTER(XT, NV)                                                                          \
   do {                                                                                                   \
-    auto kern = rmsnorm_router_fwd_kernel<XT, NV>;                                                       \
+    auto kern = rmsnorm_router_fwd_kernel<XT, NV, ROUTER_WAVES>;                                                     \
     static bool attr_done[MOE_MAX_DEVICES]; /* per GPU and instantiation: set once, to the largest */    \
     const int dev = moe_current_device();   /* footprint any supported shape asks for              */    \
     if (!attr_done[dev]) {                                                                               \
@@ -442,7 +483,7 @@ extern "C" int moe_rmsnorm_router_fwd(const void* x, int x_dtype, const float* w
       attr_done[dev] = true;                                                                             \
     }                                                                                                    \
     hipLaunchKernelGGL(kern, grid, block, lds, s, (const XT*)x, weight, eps, (int)T, (int)(H / 8),       \
-                       router_weight, (int)E, (int)k, xn, rstd, logits, ids, gates);                     \
+                       router_weight, (int)E, (int)k, xn, rstd, logits, ids, gates, (uint32_t*)table);   \
   } while (0)
   const int64_t groups = (H / 8 + MOE_WAVE - 1) / MOE_WAVE;  // 16-byte column groups per lane (H <= 4096: at most 8)
   if (x_dtype == MOE_DT_BF16) {
@@ -458,6 +499,14 @@ extern "C" int moe_rmsnorm_router_fwd(const void* x, int x_dtype, const float* w
   }
 #undef MOE_NORM_ROUTER
   return moe_launch_status();
+}
+
+extern "C" int moe_rmsnorm_router_fwd(const void* x, int x_dtype, const float* weight, float eps,
+                                      const uint16_t* router_weight, int64_t T, int64_t H, int64_t E,
+                                      int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
+                                      int32_t* ids, float* gates, void* stream) {
+  return moe_rmsnorm_router_count(x, x_dtype, weight, eps, router_weight, T, H, E, k, xn, rstd, logits, ids, gates, nullptr,
+                                  stream);
 }
 
 extern "C" int64_t moe_rmsnorm_bwd_workspace_bytes(int64_t T, int64_t H) {

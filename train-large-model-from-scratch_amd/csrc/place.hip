@@ -14,7 +14,7 @@
 namespace {
 
 constexpr int PLACE_EXPERTS = 2 * MOE_WAVE;
-constexpr int CHUNK = 16;  // tokens counted together, one a wave of a selection's workgroup
+constexpr int CHUNK = MOE_PLACE_CHUNK;  // tokens counted together, one a wave of a selection's workgroup
 
 // Bytes of counts, all of which every placing workgroup reads: their number times the tokens is what makes the two launches
 // the slower ones in the end.  General path -> these, from the selection's start to the rows' end, us: 128 experts, 8 a
