@@ -1095,7 +1095,8 @@ long long row_slots(int64_t R, int64_t E, int tile) { return (R + tile - 1) / ti
 
 // Which kernel a row-ragged launch takes: decided from the shapes alone (never from the routing: no host
 // synchronisation).  With fewer tiles than half the compute units, by the bound on their number, every one of them can be
-// halved; what csrc/row_ring.hip takes is done there.  `forced_row_tile` (0: automatic) is a test hook.
+// halved, as long as the halves are one round (gate/up has twice the tiles for its columns; 10842 rows of 8 experts, 2496 <-> 320, 266
+// halves 69 us, whole tiles and quarters 50; 13653 of 12, 1984 <-> 192, 225 halves, 34 and 35.5); what csrc/row_ring.hip takes is done there.  `forced_row_tile` (0: automatic) is a test hook.
 constexpr int RING_TILE = 64;
 int forced_row_tile = 0;
 
@@ -1110,7 +1111,9 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
     return rc;
   a.n_tiles = (a.N + cols - 1) / cols;
   const long long tiles = row_slots(a.R, a.E, ROW_TILE) * ((a.N + CfgMain::BN - 1) / CfgMain::BN);
-  const bool small = forced_row_tile > RING_TILE ? forced_row_tile == CfgHalf::BM : 2 * tiles < moe_compute_units();
+  const bool small = forced_row_tile > RING_TILE ? forced_row_tile == CfgHalf::BM
+                                                 : 2 * tiles < moe_compute_units() &&
+                                                       expected_tiles(a, CfgHalf::BM) * a.n_tiles <= moe_compute_units();
   if (small)
     return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK>, attr_done[0], a,
                                  a.n_tiles * row_slots(a.R, a.E, CfgHalf::BM), s);

@@ -118,23 +118,23 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
   constexpr int WTNC = DUAL ? 32 : 64;
   const int col_w0 = n0 + wn * WTNC, n_cb = (p.N + 31) / 32;
   const int row_w0 = row0 + wm * 32 * FM, rows = row_end - row_w0;
-  static_assert(FM == 1 || MODE == DOWN || MODE == DGRAD_GATEUP, "one strip of the fused modes");
-  const auto gu_block = [&](const void* base, int cb) {
-    return (char*)base + ((long long)(first / 32 + e + row / 32 + wm) * n_cb + cb) * 4096 + lane * 16;
+  const auto gu_block = [&](const void* base, int i, int cb) {
+    return (char*)base + ((long long)(first / 32 + e + row / 32 + wm * FM + i) * n_cb + cb) * 4096 + lane * 16;
   };
   u32x4 gu[2][4];
-  if constexpr (MODE == DGRAD_DOWN) {
+  const auto load_gu = [&](int i) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) gu[c][v] = u32x4{0, 0, 0, 0};
-      if (rows > 0 && col_w0 / 32 + c < n_cb) {
-        const u32x4* rec = reinterpret_cast<const u32x4*>(gu_block(p.X0, col_w0 / 32 + c));
+      if (rows > i * 32 && col_w0 / 32 + c < n_cb) {
+        const u32x4* rec = reinterpret_cast<const u32x4*>(gu_block(p.X0, i, col_w0 / 32 + c));
 #pragma unroll
         for (int v = 0; v < 4; ++v) gu[c][v] = __builtin_nontemporal_load(rec + 64 * v);
       }
     }
-  }
+  };
+  if constexpr (MODE == DGRAD_DOWN) load_gu(0);
   ring_wait<0>();  // the strips lie in the stages
   if (idle) return;
   constexpr int STRIDE = WTNC * 2, CPS = STRIDE / 16, RPS = 64 / CPS;
@@ -155,54 +155,61 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
     }
   };
   if constexpr (MODE == GATEUP) {
-    const bool keep = BLK && col_w0 / 32 < n_cb;
-    u32x4* rec = keep ? reinterpret_cast<u32x4*>(gu_block(p.C0, col_w0 / 32)) : nullptr;
-    u32x2 gq[2], uq[2];
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      float g[4], u[4], a[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        g[v] = acc[0][0][4 * g4 + v];
-        u[v] = acc[0][1][4 * g4 + v];
-        a[v] = swiglu(g[v], u[v]);
-      }
-      put4(0, g4, pack4(a[0], a[1], a[2], a[3]));
-      gq[g4 & 1] = pack4(g[0], g[1], g[2], g[3]);
-      uq[g4 & 1] = pack4(u[0], u[1], u[2], u[3]);
-      if (keep && (g4 & 1)) {
-        __builtin_nontemporal_store(u32x4{gq[0][0], gq[0][1], gq[1][0], gq[1][1]}, rec + 64 * (g4 >> 1));
-        __builtin_nontemporal_store(u32x4{uq[0][0], uq[0][1], uq[1][0], uq[1][1]}, rec + 128 + 64 * (g4 >> 1));
-      }
-    }
-    store_rows(p.C2, 0);
-  } else if constexpr (MODE == DGRAD_DOWN) {
-    float rowdot = 0.f;  // this lane's share of <dact[row,:], act[row,:]>
-    u32x2 du4[2][4];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int i = 0; i < FM; ++i) {
+      const bool keep = BLK && col_w0 / 32 < n_cb && rows > i * 32;
+      u32x4* rec = keep ? reinterpret_cast<u32x4*>(gu_block(p.C0, i, col_w0 / 32)) : nullptr;
+      u32x2 gq[2], uq[2];
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
-        const u32x4 gv = gu[c][g4 >> 1], uv = gu[c][2 + (g4 >> 1)];
-        const uint32_t g01 = gv[2 * (g4 & 1)], g23 = gv[2 * (g4 & 1) + 1], u01 = uv[2 * (g4 & 1)], u23 = uv[2 * (g4 & 1) + 1];
-        const float g[4] = {bf16lo(g01), bf16hi(g01), bf16lo(g23), bf16hi(g23)};
-        const float u[4] = {bf16lo(u01), bf16hi(u01), bf16lo(u23), bf16hi(u23)};
-        float dg[4], du[4];
+        float g[4], u[4], a[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) swiglu_bwd(acc[0][c][4 * g4 + v], g[v], u[v], dg[v], du[v], rowdot);
-        put4(c, g4, pack4(dg[0], dg[1], dg[2], dg[3]));
-        du4[c][g4] = pack4(du[0], du[1], du[2], du[3]);
+        for (int v = 0; v < 4; ++v) {
+          g[v] = acc[i][0][4 * g4 + v];
+          u[v] = acc[i][1][4 * g4 + v];
+          a[v] = swiglu(g[v], u[v]);
+        }
+        put4(0, g4, pack4(a[0], a[1], a[2], a[3]));
+        gq[g4 & 1] = pack4(g[0], g[1], g[2], g[3]);
+        uq[g4 & 1] = pack4(u[0], u[1], u[2], u[3]);
+        if (keep && (g4 & 1)) {
+          __builtin_nontemporal_store(u32x4{gq[0][0], gq[0][1], gq[1][0], gq[1][1]}, rec + 64 * (g4 >> 1));
+          __builtin_nontemporal_store(u32x4{uq[0][0], uq[0][1], uq[1][0], uq[1][1]}, rec + 128 + 64 * (g4 >> 1));
+        }
       }
-    // one partial per 64 columns and row, every one of them written
-    rowdot += __shfl_xor(rowdot, 32, MOE_WAVE);
-    if (lh == 0 && l32 < rows && p.C2)
-      reinterpret_cast<float*>(p.C2)[(long long)(col_w0 / 64) * p.R + row_w0 + l32] = rowdot;
-    store_rows(p.C0, 0);
+      store_rows(p.C2, i * 32);
+    }
+  } else if constexpr (MODE == DGRAD_DOWN) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int i = 0; i < FM; ++i) {
+      float rowdot = 0.f;  // this lane's share of <dact[row,:], act[row,:]>
+      u32x2 du4[2][4];
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) put4(c, g4, du4[c][g4]);
-    store_rows(p.C1, 0);
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const u32x4 gv = gu[c][g4 >> 1], uv = gu[c][2 + (g4 >> 1)];
+          const uint32_t g01 = gv[2 * (g4 & 1)], g23 = gv[2 * (g4 & 1) + 1], u01 = uv[2 * (g4 & 1)], u23 = uv[2 * (g4 & 1) + 1];
+          const float g[4] = {bf16lo(g01), bf16hi(g01), bf16lo(g23), bf16hi(g23)};
+          const float u[4] = {bf16lo(u01), bf16hi(u01), bf16lo(u23), bf16hi(u23)};
+          float dg[4], du[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) swiglu_bwd(acc[i][c][4 * g4 + v], g[v], u[v], dg[v], du[v], rowdot);
+          put4(c, g4, pack4(dg[0], dg[1], dg[2], dg[3]));
+          du4[c][g4] = pack4(du[0], du[1], du[2], du[3]);
+        }
+      if (i + 1 < FM) load_gu(i + 1);
+      // one partial per 64 columns and row, every one of them written
+      rowdot += __shfl_xor(rowdot, 32, MOE_WAVE);
+      if (lh == 0 && i * 32 + l32 < rows && p.C2)
+        reinterpret_cast<float*>(p.C2)[(long long)(col_w0 / 64) * p.R + row_w0 + i * 32 + l32] = rowdot;
+      store_rows(p.C0, i * 32);
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) put4(c, g4, du4[c][g4]);
+      store_rows(p.C1, i * 32);
+    }
   } else {
 #pragma unroll
     for (int i = 0; i < FM; ++i) {

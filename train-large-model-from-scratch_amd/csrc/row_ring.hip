@@ -106,10 +106,24 @@ bool small_tiles_pay(const GemmArgs& a) {
 // Down and dgrad-gate/up, whose epilogues are short, have tiles of 128 rows and two stages for what is too much for 64
 // rows (tiles of 128 rows; down and dgrad-gate/up us: 320 12.4, 19.8 -> 11.2, 17.6; 440 14.5, 22.6 -> 12.5, 19.6; 576
 // 19.0, 29.2 -> 19.5, 31.8).
+// The bound has a tile too many for every other expert.  Past it, launches that are expected to fit are taken all the same, and
+// in tiles of 128 rows where the contraction is at most 1280 (gate/up 640: longer ones are bound by LDS, where the larger kernels'
+// tiles of 128 x 256 have less traffic; 1024: 18.6 -> 16.8 us by itself, but a forward pass of 2048 tokens of 8 experts 45.3 -> 46.2),
+// or at most 320 and two rounds: there a tile's end is as long as its contraction, and two workgroups to a compute unit cover
+// each other's.  Before -> this, us: 6492 rows of 8 experts, 256 <-> 576, gate/up 16.2 -> 9.8; 18388 of 64, 576 <-> 192, down 18.4 ->
+// 12.1; 3784 of 16, 384 <-> 896, dgrad-down 16.3 -> 12.0 (in tiles of 64).  Of 2000 launches of 500 drawn layers 220 go
+// elsewhere, 7 % faster in the mean, 34 of them slower by more than 3 %.  Whole passes of 96 more layers: 0.99 to 1.16 times as
+// fast.  What it gets wrong: 15407 rows of 96, 576 <-> 192, gate/up 23.8 -> 26.6; 30411 of 12, 1408 <-> 320, down, not taken.
 template <int MODE, bool BLK>
 bool choose(const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
   const long long slots = 2ll * moe_compute_units();
   if (launch<MODE, BLK, 1>(a, slots, forced, s, rc)) return true;
+  constexpr int COLS = RingTile<MODE, 1, 4>::BNC;
+  const double cols = (a.N + COLS - 1) / COLS, k = (double)a.K * (MODE == DGRAD_GATEUP ? 2 : 1);
+  if (expected_tiles(a, 64) * cols <= slots) return launch<MODE, BLK, 1>(a, slots, true, s, rc);
+  const double half = expected_tiles(a, 128) * cols;
+  if ((half <= slots && k <= (MODE == GATEUP ? 640 : 1280)) || (half <= 2 * slots && k <= 320 && MODE != DGRAD_GATEUP))
+    return launch<MODE, BLK, 2>(a, slots, true, s, rc);
   if constexpr (MODE == DOWN || MODE == DGRAD_GATEUP)
     if (launch<MODE, BLK, 2>(a, slots, false, s, rc)) return true;
   return small_tiles_pay<MODE>(a) && launch<MODE, BLK, 1>(a, slots, true, s, rc);
