@@ -74,3 +74,13 @@ def test_steps_and_stages(pkg, lib, H, I):
     for name, w in zip(("dw1", "dw3", "dw2"), ws):
         check(name, w.grad, b[name], be[name])
         assert not w.grad[counts.index(0)].any()
+
+
+@pytest.mark.parametrize("T,E,k,H,I", [
+    (1100, 70, 2, 520, 264),   # 420 tiles of 256 x 256, six rounds against 4.1 of small tiles: taken
+    (600, 65, 2, 512, 512),    # 260, five rounds (two of the launches one) against 4.1: taken
+    (300, 66, 1, 512, 1024),   # 528, eight rounds against 8.25: not taken
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_weight_gradients_past_a_round_of_tiles(pkg, lib, T, E, k, H, I, dtype):
+    test_small_launch_weight_gradients(pkg, lib, T, E, k, H, I, None, dtype)

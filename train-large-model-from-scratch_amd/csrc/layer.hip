@@ -214,14 +214,22 @@ struct FwdScratch {
   }
 };
 
-// Whether the weight gradients go to the kernel that takes all stacks at once (wgrad.hip): where one stack's
-// 256 x 256 tiles are at most MULTI_ROUNDS for every compute unit.  Decided from shapes alone.  (64 tiles, Zipf: a
-// step of 8192 tokens 406 -> 362 us; 216 tiles: 401 -> 395; 512 tiles: 494 -> 514, so not there.)
+// Whether the weight gradients go to the kernel that takes all stacks at once (wgrad.hip).  Decided from shapes alone: where
+// one stack's 256 x 256 tiles are at most one for every compute unit, and up to four where its launch of 128 x 128 tiles, three to
+// a compute unit, comes to no more rounds than the tiled kernel's launches do (one for w2's stack, one or two for the others),
+// each of which ends in a partial round and pads the matrices to 256.  A round of either takes about as long: 4 us and 0.03 for each row
+// of an expert, another 4.4 with fp32 results.  (64 tiles, Zipf: a step of 8192 tokens 406 -> 362 us; 216 tiles: 401 -> 395; 512
+// tiles, 6 rounds against 8: 494 -> 514, not taken.  2006 tokens of 8 experts, 3136 <-> 704, 312 tiles, 6 rounds against 4.7: 326 -> 289;
+// 3959 tokens, 4 of 128 by Zipf's shares, 384 <-> 448, 6 against 6, 378 -> 223; 3390 of 64, 360 <-> 768, 5 against 4.5, 301 ->
+// 227.  150 drawn layers of one to eight rounds: 68 taken, steps 1.03 times as fast in the mean, four slower by 2 to 5 % (969
+// tokens, 6 of 128, 768 <-> 384, 9 against 9: 316 -> 331).)
 constexpr int64_t WTILE = 256;
-constexpr int64_t MULTI_ROUNDS = 1;
+constexpr int64_t MULTI_ROUNDS = 4;
 bool wgrad_multi(int64_t E, int64_t M, int64_t N, int64_t R) {
-  const int64_t tiles = ((M + WTILE - 1) / WTILE) * ((N + WTILE - 1) / WTILE);
-  return R > 0 && E * tiles <= MULTI_ROUNDS * moe_compute_units();
+  const int64_t cus = moe_compute_units();
+  const int64_t tiles = E * ((M + WTILE - 1) / WTILE) * ((N + WTILE - 1) / WTILE);
+  const int64_t rounds = (tiles + cus - 1) / cus + (M % WTILE == 0 ? (2 * tiles + cus - 1) / cus : 2 * ((tiles + cus - 1) / cus));
+  return R > 0 && (tiles <= cus || (tiles <= MULTI_ROUNDS * cus && rounds * cus >= E * ((M + 127) / 128) * ((N + 127) / 128)));
 }
 
 // Router weight gradient: the tokens are cut into slices, as many as give every compute unit a job, of at least 64
