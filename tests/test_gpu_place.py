@@ -111,3 +111,40 @@ def test_places_behind_the_norm(pkg, lib, T, E, k, H, x_dt):
     y, rows = pkg.moe_ffn(xn, logits, *ws, k, return_routing=True)
     assert torch.equal(rt["gates"], rows["gates"])
     assert torch.equal(out.to(torch.bfloat16), y)  # (the same kernels from the rows on; fp32 x: an fp32 result, rounded here)
+
+
+@pytest.mark.parametrize("T,E,H", [
+    (1, 1, 8),
+    (15, 4, 16),          # a chunk one row short
+    (257, 31, 2056),      # a row past a workgroup's 16 chunks; a last word with one count missing
+    (4097, 128, 64),      # the most experts
+    (12288, 128, 16),     # the largest table
+    (12289, 128, 16),     # one row more: the general path
+    (16384, 8, 8),        # the most rows
+    (16385, 8, 8),
+])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_places_of_given_experts(pkg, lib, T, E, H, dtype):
+    """Rows whose experts are given, some of them outside [0, E): placed with the nearest expert, and counted."""
+    print("places of given experts", T, E, H, dtype, flush=True)
+    rng = np.random.default_rng(T + E)
+    ids = rng.integers(0, E, T)
+    outside = rng.choice(T, T // 5, replace=False)
+    ids[outside] = rng.choice([-1, -7, E, E + 3, 2 ** 31 - 1], len(outside))
+    if dtype == torch.int64 and len(outside) > 1:
+        ids[outside[:2]] = [2 ** 31 + 1, -2 ** 40]
+    # (in 32 bits whatever does not fit, like anything below 0 of 64, is -1)
+    narrow = np.where((ids < 0) | (ids > 2 ** 31 - 1), -1, ids) if dtype == torch.int64 else ids
+    flat = np.clip(narrow, 0, E - 1)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16).cuda()
+    ws = [torch.randn(*s, device="cuda").to(torch.bfloat16) for s in ((E, 8, H), (E, 8, H), (E, H, 8))]
+    out, rt = pkg.experts_rows(x, torch.tensor(ids, dtype=dtype, device="cuda"), *ws, return_routing=True)
+    order = np.argsort(flat, kind="stable")
+    inverse = np.empty_like(order)
+    inverse[order] = np.arange(T)
+    counts = np.bincount(flat, minlength=E)
+    for name, want in (("counts", counts), ("offs", np.concatenate([[0], counts.cumsum()])), ("pos_to_row", order),
+                       ("row_to_pos", inverse), ("bad_ids", np.array([(narrow < 0).sum() + (narrow >= E).sum()]))):
+        assert np.array_equal(rt[name].cpu().numpy().reshape(-1), want.astype(np.int32)), name
+    sorted_out = pkg.experts_rows(x[torch.tensor(order, device="cuda")], torch.tensor(flat[order], device="cuda"), *ws)
+    assert torch.equal(out[torch.tensor(order, device="cuda")], sorted_out)

@@ -40,7 +40,7 @@ struct Carve {
 // Room for the counts that selection and places, or histograms and scans, work on.
 int64_t order_bytes(int64_t T, int64_t E, int64_t k) {
   const int64_t general = moe_dispatch_workspace_bytes(T * k, E);
-  const int64_t place = moe_place_ok(T, E, k) ? moe_place_bytes(T, E) : 0;
+  const int64_t place = moe_place_ok(T, E, k) ? moe_count_bytes(T, E) : 0;
   return place > general ? place : general;
 }
 
@@ -146,7 +146,7 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   }
   if (place) {
     MOE_STEP("moe_place_rows", moe_place_rows(x, x_dtype, ids, ws + c.dispatch, T, H, E, k, counts, offs, pos_to_row,
-                                              row_to_pos, nullptr, xp, MOE_DT_BF16, stream));
+                                              row_to_pos, nullptr, xp, MOE_DT_BF16, false, stream));
   } else {
     MOE_STEP("moe_histogram_scan_checked",
              moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
@@ -336,8 +336,13 @@ static int layer_forward(const moe_layer_forward_args* a, const void* table, voi
     if (!table)
       MOE_STEP("moe_select_count", moe_select_count(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids, a->gates,
                                                     ws.dispatch, stream));
-    MOE_STEP("moe_place_rows", moe_place_rows(a->x, (int)a->x_dtype, a->ids, table ? table : ws.dispatch, T, H, E, k, a->counts, a->offs,
-                                              a->pos_to_row, a->row_to_pos, a->bad_ids, a->xp, MOE_DT_BF16, stream));
+    MOE_STEP("moe_place_rows", moe_place_rows(a->x, (int)a->x_dtype, a->ids, table ? table : ws.dispatch, T, H, E, k, a->counts,
+                                              a->offs, a->pos_to_row, a->row_to_pos, a->bad_ids, a->xp, MOE_DT_BF16, false,
+                                              stream));
+  } else if (!a->logits && !table && moe_count_ok(T, E, k)) {
+    MOE_STEP("moe_count_ids", moe_count_ids(a->ids64, a->ids, T, E, ws.dispatch, stream));
+    MOE_STEP("moe_place_rows", moe_place_rows(a->x, (int)a->x_dtype, a->ids, ws.dispatch, T, H, E, k, a->counts, a->offs,
+                                              a->pos_to_row, a->row_to_pos, a->bad_ids, a->xp, MOE_DT_BF16, true, stream));
   } else {
     if (a->logits)
       MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids,

@@ -59,12 +59,39 @@ __global__ __launch_bounds__(CHUNK* MOE_WAVE) void select_count_kernel(const LT*
   }
 }
 
+// The table where the experts are given, one a row: an id outside [0, E) counts for the nearest expert, as in dispatch.hip, and
+// bad[chunk] is how many of the chunk's are.  With `narrowed` the ids are also left there in 32 bits.
+template <typename IT>
+__global__ __launch_bounds__(256) void count_ids_kernel(const IT* __restrict__ ids, int T, int E, int32_t* __restrict__ narrowed,
+                                                        uint32_t* __restrict__ table, uint32_t* __restrict__ bad) {
+  constexpr int CHUNKS = 256 / CHUNK;
+  __shared__ uint32_t counts[CHUNKS][PLACE_EXPERTS / 4];  // a byte an expert: a chunk has 16 rows
+  const int t = blockIdx.x * 256 + threadIdx.x, lane = lane_id(), words = (E + 3) / 4;
+  for (int i = threadIdx.x; i < CHUNKS * PLACE_EXPERTS / 4; i += 256) counts[0][i] = 0;
+  __syncthreads();
+  bool outside = false;
+  if (t < T) {
+    const IT v = ids[t];
+    const int id = v < 0 || (int64_t)v > 0x7fffffffll ? -1 : (int)v;
+    if (narrowed) narrowed[t] = id;
+    const int e = id < 0 ? 0 : id >= E ? E - 1 : id;
+    outside = e != id;
+    atomicAdd(&counts[threadIdx.x / CHUNK][e >> 2], 1u << (8 * (e & 3)));
+  }
+  const unsigned long long who = __ballot(outside);
+  if (t < T && lane % CHUNK == 0) bad[t / CHUNK] = __popcll((who >> lane) & ((1ull << CHUNK) - 1));
+  __syncthreads();
+  const int chunks = (T + CHUNK - 1) / CHUNK - blockIdx.x * CHUNKS, n = (chunks < CHUNKS ? chunks : CHUNKS) * words;
+  for (int i = threadIdx.x; i < n; i += 256) table[(size_t)blockIdx.x * CHUNKS * words + i] = counts[i / words][i % words];
+}
+
 // WAVES tokens of a chunk, one a wave.  `shift`: 2^shift words hold a chunk's counts.
-template <typename XT, typename OT, int WAVES>
+// GIVEN: the experts are, and may lie outside [0, E).
+template <typename XT, typename OT, int WAVES, bool GIVEN>
 __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     const XT* __restrict__ x, const int32_t* __restrict__ ids, const uint32_t* __restrict__ table, int T, int E, int k,
     int H, int shift, int32_t* __restrict__ counts, int32_t* __restrict__ offs, int32_t* __restrict__ pos_to_row,
-    int32_t* __restrict__ row_to_pos, int32_t* __restrict__ bad_ids, OT* __restrict__ xp) {
+    int32_t* __restrict__ row_to_pos, int32_t* __restrict__ bad_ids, OT* __restrict__ xp, const uint32_t* __restrict__ bad) {
   __shared__ int below[PLACE_EXPERTS], total[PLACE_EXPERTS];  // of earlier chunks, of all
   __shared__ uint32_t asked[PLACE_EXPERTS];
   constexpr int AHEAD = 4;  // 8-element pieces of the row requested at once
@@ -84,13 +111,24 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     }
   };
   request(0);
-  const int my_id = live && lane < k ? ids[(size_t)t * k + lane] : 0;
+  const auto expert_of = [&](int r) {
+    const int e = ids[r];
+    return !GIVEN ? e : e < 0 ? 0 : e >= E ? E - 1 : e;
+  };
+  const int my_id = live && lane < k ? expert_of(t * k + lane) : 0;
+  __shared__ int outside;
+  if (GIVEN && threadIdx.x == 0) outside = 0;
   static_assert(WAVES * MOE_WAVE >= PLACE_EXPERTS && CHUNK % WAVES == 0, "a thread an expert");
   if (threadIdx.x < PLACE_EXPERTS) below[threadIdx.x] = total[threadIdx.x] = 0, asked[threadIdx.x] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < CHUNK * k; i += blockDim.x) {
     const int r = chunk * CHUNK * k + i;
-    if (r < T * k) atomicOr(&asked[ids[r]], 1u << (i / k));
+    if (r < T * k) atomicOr(&asked[expert_of(r)], 1u << (i / k));
+  }
+  if (GIVEN && blockIdx.x == 0) {
+    int n = 0;
+    for (int c = threadIdx.x; c < chunks; c += blockDim.x) n += bad[c];
+    if (n) atomicAdd(&outside, n);
   }
   // two 16-bit sums a register: no expert has more rows than there are tokens
   const int w = threadIdx.x & ((1 << shift) - 1), step = blockDim.x >> shift;
@@ -129,7 +167,7 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     if (lane < E) counts[lane] = n0, offs[lane] = upto0 - n0;
     if (MOE_WAVE + lane < E) counts[MOE_WAVE + lane] = n1, offs[MOE_WAVE + lane] = upto1 - n1;
     if (lane == 0) offs[E] = T * k;
-    if (lane == 0 && bad_ids) *bad_ids = 0;  // (a selection asks for no other experts)
+    if (lane == 0 && bad_ids) *bad_ids = GIVEN ? outside : 0;  // (a selection asks for no other experts)
   }
   const int first0 = __shfl(upto0 - n0, my_id & 63, MOE_WAVE), first1 = __shfl(upto1 - n1, my_id & 63, MOE_WAVE);
   int pos = 0;
@@ -181,22 +219,45 @@ int moe_select_count(const void* logits, int logits_dtype, const float* bias, in
   return E <= MOE_WAVE ? go(One{}, float{}) : go(Two{}, float{});
 }
 
+// Row by row there is least else to do, and what the general path launches more is soon less than a table read by every workgroup: whole
+// training passes of rows, us, there and here: 1123 rows of 24 experts, 272 <-> 176, 69 -> 65; 4392 of 64, 264 <-> 264, 89 -> 81; 9085 of
+// 16, 512 <-> 448, 137 -> 129; 18747 of 32, 1280 <-> 192, 287 -> 290; 32768 of 16, 4096 <-> 1536, 3682 -> 3708.
+bool moe_count_ok(int64_t T, int64_t E, int64_t k) { return k == 1 && T <= 16384 && moe_place_ok(T, E, k); }
+int64_t moe_count_bytes(int64_t T, int64_t E) { return moe_place_bytes(T, E) + (T + CHUNK - 1) / CHUNK * 4; }
+
+int moe_count_ids(const int64_t* ids64, int32_t* ids, int64_t T, int64_t E, void* table, void* stream) {
+  uint32_t* bad = (uint32_t*)((char*)table + moe_place_bytes(T, E));
+  const dim3 grid((unsigned)((T + 255) / 256)), block(256);
+  if (ids64)
+    hipLaunchKernelGGL(count_ids_kernel<int64_t>, grid, block, 0, (hipStream_t)stream, ids64, (int)T, (int)E, ids,
+                       (uint32_t*)table, bad);
+  else
+    hipLaunchKernelGGL(count_ids_kernel<int32_t>, grid, block, 0, (hipStream_t)stream, ids, (int)T, (int)E, nullptr,
+                       (uint32_t*)table, bad);
+  return moe_launch_status();
+}
+
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
                    int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
-                   void* xp, int xp_dtype, void* stream) {
+                   void* xp, int xp_dtype, bool counted, void* stream) {
   if (H <= 0 || H % 8 != 0) return MOE_ERR_SHAPE;
   if (H > 65536) return MOE_ERR_LIMIT;
   if (x_dtype == MOE_DT_BF16 && xp_dtype != MOE_DT_BF16) return MOE_ERR_DTYPE;
   hipStream_t s = (hipStream_t)stream;
+  const uint32_t* bad = counted ? (const uint32_t*)((const char*)table + moe_place_bytes(T, E)) : nullptr;
   int shift = 0;
   while ((1 << shift) < words_of(E)) ++shift;
   const auto go = [&](auto xt, auto ot, auto waves) {
     using XT = decltype(xt);
     using OT = decltype(ot);
     constexpr int WAVES = decltype(waves)::value;
-    hipLaunchKernelGGL((place_rows_kernel<XT, OT, WAVES>), dim3((unsigned)((T + WAVES - 1) / WAVES)),
-                       dim3(WAVES * MOE_WAVE), 0, s, (const XT*)x, ids, (const uint32_t*)table, (int)T, (int)E, (int)k,
-                       (int)H, shift, counts, offs, pos_to_row, row_to_pos, bad_ids, (OT*)xp);
+    const auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)((T + WAVES - 1) / WAVES)), dim3(WAVES * MOE_WAVE), 0, s, (const XT*)x, ids,
+                         (const uint32_t*)table, (int)T, (int)E, (int)k, (int)H, shift, counts, offs, pos_to_row, row_to_pos,
+                         bad_ids, (OT*)xp, bad);
+    };
+    if (counted) launch(place_rows_kernel<XT, OT, WAVES, true>);
+    else launch(place_rows_kernel<XT, OT, WAVES, false>);
     return moe_launch_status();
   };
   const auto of = [&](auto waves) {
