@@ -91,3 +91,34 @@ def test_one_infinite_activation_makes_infinite_outputs(pkg, lib, H, k, I):
         with torch.no_grad():
             out = pkg.moe_ffn(x.cuda().to(bf), logits, *(w.cuda().to(bf) for w in (w1, w3, w2)), k)
         assert torch.isposinf(out).all(), (i, out.isnan().sum().item(), out.isfinite().sum().item())
+
+
+@pytest.mark.parametrize("T,E,k,H,I,x_dt,given", [
+    (2, 1, 1, 8, 8, torch.bfloat16, torch.bfloat16),       # one expert, all of both tokens
+    (5, 65, 7, 40, 24, torch.float32, torch.float32),      # one expert more than lanes in a wave; logits in fp32
+    (64, 4, 3, 136, 120, torch.bfloat16, torch.float32),   # more tokens than workgroups; more rows than 32 an expert
+    (33, 16, 16, 72, 40, torch.float32, torch.bfloat16),   # every token asks for every expert
+    (13, 128, 2, 264, 56, torch.bfloat16, torch.bfloat16),  # turns of four tokens and one, the most experts (2048 turns)
+    (17, 128, 2, 264, 56, torch.bfloat16, torch.bfloat16),  # ... past them: the launch of its own
+])
+def test_selection_inside_gate_up(pkg, lib, T, E, k, H, I, x_dt, given):
+    """Which rows an expert has, from the logits themselves: ties, a bias, infinities and a NaN, as the selection's own launch
+    (which the oracle stands for) decides them."""
+    print("selection inside gate/up", T, E, k, H, I, x_dt, given, flush=True)
+    g = torch.Generator().manual_seed(T + E)
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(torch.bfloat16)
+    x, w1, w3, w2 = r(T, H), r(E, I, H, std=0.05), r(E, I, H, std=0.05), r(E, H, I, std=0.05)
+    lg = torch.randn(T, E, generator=g).round(decimals=1).to(given)
+    if E > k:
+        lg[1, 0] = -float("inf")
+    bias = torch.randn(E, generator=g).round(decimals=1) if T % 2 else None
+    sel = lg.float() + bias if bias is not None else lg.float()
+    f = O.moe_forward(x, torch.zeros(E, H), w1, w3, w2, k, logits=sel)
+    fe = O.moe_forward(x, torch.zeros(E, H), w1, w3, w2, k, logits=sel, emulate_bf16=True)
+    ws = [w.cuda() for w in (w1, w3, w2)]
+    call = lambda logits: pkg.moe_ffn(x.cuda().to(x_dt), logits.cuda(), *ws, k, bias=None if bias is None else bias.cuda())
+    out = call(lg)
+    check("out", out, f["out"], fe["out"])
+    lg[0, E - 1] = float("nan")  # (its expert comes first and its token's gates are NaN; the others stay as they are)
+    bad = call(lg)
+    assert bad[0].isnan().all() and torch.equal(bad[1:], out[1:])

@@ -282,7 +282,7 @@ __device__ __forceinline__ void few_columns_16(const AT* __restrict__ A, int div
   else few_columns<AT, NB, 1, 8, 0>(A, div, w, e, n0, nblk, N, K, rows, n, part, C);
 }
 
-// The selection of a single token, made by every wave for itself (128 experts: in about the time its ids would take to
+// The selection, made where it is needed.  A single token's by every wave for itself (128 experts: in about the time its ids would take to
 // arrive, where a launch of its own costs more: 64 experts, 2048 <-> 1024, 33.5 -> 32.1 us a
 // token; 128 experts, 1024 <-> 256, 28.2 -> 25.0).
 struct Selection {
@@ -292,9 +292,43 @@ struct Selection {
   float* gates;
   int logits_f32, k;
 };
+template <int VPL>
+__device__ __forceinline__ void token_keys(const Selection& sel, int t, int E, uint32_t (&key)[VPL]) {
+  if (sel.logits_f32) moe_topk_keys<VPL>((const float*)sel.logits + (size_t)t * E, sel.bias, E, lane_id(), key);
+  else moe_topk_keys<VPL>((const uint16_t*)sel.logits + (size_t)t * E, sel.bias, E, lane_id(), key);
+}
+// The rows of expert e from the logits of T tokens, as list_rows makes them from the ids: a token asks for it if fewer than k of its
+// experts come before e, and that many is the slot.  A wave a token, a comparison and a ballot each, so that
+// the selection of a few tokens is no launch of its own (moe_gateup_few_selects has the line).
+template <int VPL>
+__device__ __forceinline__ int list_selected_rows(const Selection& sel, int T, int E, int e, int* rows, int* count) {
+  constexpr int AHEAD = 4;
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE)), waves = blockDim.x / MOE_WAVE;
+  if (threadIdx.x == 0) *count = 0;
+  __syncthreads();
+  for (int t0 = wv; t0 < T; t0 += AHEAD * waves) {
+    uint32_t key[AHEAD][VPL];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (t0 + i * waves < T) token_keys<VPL>(sel, t0 + i * waves, E, key[i]);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int t = t0 + i * waves;
+      if (t >= T) break;
+      const uint32_t own = e < MOE_WAVE ? read_lane(key[i][0], e) : read_lane(key[i][VPL - 1], e - MOE_WAVE);
+      int before = 0;
+#pragma unroll
+      for (int v = 0; v < VPL; ++v)
+        before += __popcll(__ballot(key[i][v] > own || (key[i][v] == own && v * MOE_WAVE + lane < e)));
+      if (before < sel.k && lane == 0) rows[atomicAdd(count, 1)] = t * sel.k + before;
+    }
+  }
+  __syncthreads();
+  return *count;
+}
 
-// ONE: a single token; block row j takes its j-th expert and no list is needed.  VPL > 0: which one that is comes from
-// the logits of at most 64 * VPL experts, not from ids.
+// ONE: a single token; block row j takes its j-th expert and no list is needed.  VPL > 0: which one that is, and else which rows
+// an expert has, comes from the logits of at most 64 * VPL experts, not from ids.
 template <typename AT, int NB, bool ONE, int VPL = 0>
 __global__ __launch_bounds__(256, 2) void few_kernel(const AT* __restrict__ A, int div, const int32_t* __restrict__ ids,
                                                     int R, const uint16_t* __restrict__ w0,
@@ -332,11 +366,35 @@ __global__ __launch_bounds__(256, 2) void few_kernel(const AT* __restrict__ A, i
     few_columns_16<AT, NB>(A, div, w, e, n0, nb, N, K, rows, 1, part, C);
   } else {
     const int e = blockIdx.y;
-    const int n = list_rows(ids, R, E, e, rows, &count);
-    if (n == 0) return;
-    if (n <= 16) few_columns_16<AT, NB>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
-    else if (n <= 32) few_columns<AT, NB, 2, 4, 0>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
-    else few_columns<AT, NB, 4, 2, 0>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
+    int n;
+    if constexpr (VPL > 0) {
+      const int T = R / sel.k;
+      n = list_selected_rows<VPL>(sel, T, E, e, rows, &count);
+    } else {
+      n = list_rows(ids, R, E, e, rows, &count);
+    }
+    if (n > 0) {
+      if (n <= 16) few_columns_16<AT, NB>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
+      else if (n <= 32) few_columns<AT, NB, 2, 4, 0>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
+      else few_columns<AT, NB, 4, 2, 0>(A, div, w, e, n0, nb, N, K, rows, n, part, C);
+    }
+    if constexpr (VPL > 0) {  // the launches that follow read ids and gates: the first workgroups leave a token's each, at their end
+      const int T = R / sel.k;
+      if (threadIdx.x < MOE_WAVE) {
+        const int lane = lane_id();
+        for (int t = blockIdx.y * gridDim.x + blockIdx.x; t < T; t += gridDim.x * gridDim.y) {
+          uint32_t key[VPL];
+          token_keys<VPL>(sel, t, E, key);
+          int id;
+          float gate;
+          moe_topk_softmax_wave<VPL>(key, sel.k, lane, id, gate);
+          if (lane < sel.k) {
+            sel.ids[(size_t)t * sel.k + lane] = id;
+            sel.gates[(size_t)t * sel.k + lane] = gate;
+          }
+        }
+      }
+    }
   }
 }
 
@@ -481,6 +539,33 @@ int moe_gateup_few(const void* x, int x_dtype, const int32_t* ids, const uint16_
   };
   if (x_dtype == MOE_DT_BF16) return T == 1 ? go(std::true_type{}, uint16_t{}) : go(std::false_type{}, uint16_t{});
   return T == 1 ? go(std::true_type{}, float{}) : go(std::false_type{}, float{});
+}
+
+// Every workgroup of gate/up goes through all tokens, four at a time: up to 2048 such turns in all they cost less than the
+// launch they save.  A whole call, us, with the launch and without: 2 tokens, 6 of 24 experts, 448 <-> 192 (288 turns) 32 -> 29; 5, 3
+// of 64, 320 <-> 192 (1536) 33 -> 29; 13, 1 of 4, 832 <-> 448 (448) 34 -> 30; 11, 8 of 64, 1088 <-> 192 (2304, not taken) 37 -> 37; 27, 6 of 64,
+// 896 <-> 384 (10752) 43 -> 47; 48, 8 of 64, 2048 <-> 1024 (12288) 164 -> 165.5.
+bool moe_gateup_few_selects(int64_t T, int64_t E, int64_t I, int64_t k) {
+  const int64_t nblk = few_blocks(I, T * k < E ? T * k : E);
+  return T > 1 && E <= 2 * MOE_WAVE && ((I + 15) / 16 + nblk - 1) / nblk * E * ((T + 3) / 4) <= 2048;
+}
+
+int moe_gateup_few_select(const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias, const uint16_t* w1,
+                          const uint16_t* w3, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int32_t* ids, float* gates,
+                          uint16_t* act, hipStream_t s) {
+  const int nblk = few_blocks(I, T * k < E ? T * k : E);
+  const dim3 grid((unsigned)(((I + 15) / 16 + nblk - 1) / nblk), (unsigned)E), block(256);
+  const Selection sel{logits, bias, ids, gates, logits_dtype == MOE_DT_F32, (int)k};
+  const auto go = [&](auto vpl, auto xt) {
+    using XT = decltype(xt);
+    hipLaunchKernelGGL((few_kernel<XT, 2, false, decltype(vpl)::value>), grid, block, 0, s, (const XT*)x, (int)k, nullptr,
+                       (int)(T * k), w1, w3, (int)E, (int)I, (int)H, nblk, act, sel);
+    return moe_launch_status();
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  if (x_dtype == MOE_DT_BF16) return E <= MOE_WAVE ? go(One{}, uint16_t{}) : go(Two{}, uint16_t{});
+  return E <= MOE_WAVE ? go(One{}, float{}) : go(Two{}, float{});
 }
 
 int moe_down_few(const uint16_t* act, const int32_t* ids, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I,

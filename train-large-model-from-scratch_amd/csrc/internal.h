@@ -81,6 +81,11 @@ int moe_router_few(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, 
 bool moe_few_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int x_dtype);
 int moe_gateup_few(const void* x, int x_dtype, const int32_t* ids, const uint16_t* w1, const uint16_t* w3, int64_t T,
                    int64_t H, int64_t E, int64_t I, int64_t k, uint16_t* act, hipStream_t s);
+// The same from the logits, the selection with it: ids and gates [T*k] are results.
+bool moe_gateup_few_selects(int64_t T, int64_t E, int64_t I, int64_t k);
+int moe_gateup_few_select(const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias, const uint16_t* w1,
+                          const uint16_t* w3, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int32_t* ids, float* gates,
+                          uint16_t* act, hipStream_t s);
 // The same for one token, its selection with it: ids and gates [k] are results.
 bool moe_gateup_one_ok(int64_t T, int64_t E, int64_t k);
 int moe_gateup_one(const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias, const uint16_t* w1,

@@ -130,12 +130,17 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
     return 0;
   }
   const bool few = moe_few_ok(T, H, E, I, k, x_dtype), place = !few && moe_place_ok(T, E, k);
+  const bool selects = few && moe_gateup_few_selects(T, E, I, k);  // gate/up does the selection
   if (place)
     MOE_STEP("moe_select_count", moe_select_count(logits, logits_dtype, bias, T, E, k, ids, gates, ws + c.dispatch, stream));
-  else
+  else if (!selects)
     MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream));
   if (few) {  // rows stay in routed order: no dispatch, no gather
-    MOE_STEP("moe_gateup_few", moe_gateup_few(x, x_dtype, ids, w1, w3, T, H, E, I, k, act, st));
+    if (selects)
+      MOE_STEP("moe_gateup_few", moe_gateup_few_select(x, x_dtype, logits, logits_dtype, bias, w1, w3, T, H, E, I, k,
+                                                              ids, gates, act, st));
+    else
+      MOE_STEP("moe_gateup_few", moe_gateup_few(x, x_dtype, ids, w1, w3, T, H, E, I, k, act, st));
     if (moe_down_one_ok(T, k)) {
       MOE_STEP("moe_down_one", moe_down_one(act, ids, gates, w2, H, E, I, k, out, out_dtype, st));
       return 0;
