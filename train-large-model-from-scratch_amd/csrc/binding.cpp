@@ -266,9 +266,14 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
         // time for the router, the logits are selected on before they leave the chip
         logits = empty({T, E}, at::kBFloat16, x);
         if (moe_place_ok(T, E, k)) table = empty({moe_place_bytes(T, E)}, at::kByte, x);
-        CALL(moe_rmsnorm_router_count, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, bf(f.wrb), T, H,
-             E, k, (uint16_t*)f.xn.data_ptr(), f.rstd.data_ptr<float>(), (uint16_t*)logits.data_ptr(),
-             r.part(f.routing, Routing::IDS), (float*)r.part(f.routing, Routing::GATES), ptr(table), s);
+        const char* name = "moe_rmsnorm_router_fwd";  // (the entry that callers know; this one leaves the table too)
+        moe_observe(name, 0);
+        const int rc = moe_rmsnorm_router_count(x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, bf(f.wrb), T, H, E, k,
+                                                (uint16_t*)f.xn.data_ptr(), f.rstd.data_ptr<float>(), (uint16_t*)logits.data_ptr(),
+                                                r.part(f.routing, Routing::IDS), (float*)r.part(f.routing, Routing::GATES),
+                                                ptr(table), s);
+        moe_observe(name, 1);
+        check(rc, name);
         selected = true;
       } else {
         CALL(moe_rmsnorm_fwd, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, T, H,
