@@ -434,8 +434,8 @@ def module_config3(P, torch, dev, steps, warmup):
             "entry": "MoE.forward", **out}
 
 
-# a product in fp32 is made of three fp16 ones, whose dense rate is that of bf16 (the fp32 matrix instruction: 157.3)
-MFMA_F32_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 3
+# a product in fp32 is made of six bf16 ones (the fp32 matrix instruction: 157.3)
+MFMA_F32_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 6
 
 
 def fp32_config3(P, torch, dev, steps=3, warmup=1):

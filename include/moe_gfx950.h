@@ -466,7 +466,7 @@ int moe_f32_gemm_wgrads(const float* dg, const float* du, const float* dyp, cons
                         const float* act, const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I,
                         float* dw1, float* dw3, float* dw2, void* stream);
 /* Test hook (no counterpart in the reference): the fp32 GEMM entries choose 64 x 64 or 128 x 128
- * output tiles of fp32 products, or tiles whose products are made of fp16 ones, from the shapes; 64,
+ * output tiles of fp32 products, or tiles whose products are made of bf16 ones, from the shapes; 64,
  * 128 or 1 forces one of the three, 0 restores the choice.  Returns the previous setting.  Process-wide, not synchronised. */
 int moe_f32_gemm_force_tile(int t);
 

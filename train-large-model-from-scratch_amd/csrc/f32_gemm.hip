@@ -1,13 +1,16 @@
 // Grouped (per-expert, ragged) GEMMs of the fp32 path on the matrix cores, and what is fused into them: large ones in
-// three fp16 products for one of fp32 (f32_split.h), the others with v_mfma_f32_32x32x2_f32 (fp32 operands, fp32 accumulation).
+// six bf16 products for one of fp32 (f32_split.h says what bounds those), the others with v_mfma_f32_32x32x2_f32 (fp32 operands,
+// fp32 accumulation).
 //
 // An fp32 MFMA takes 64 cycles for 2048 multiply-adds, sixteen times as long per flop as a bf16 one, so
-// that neither LDS nor HBM bounds these kernels: what does is how evenly the chip's matrix pipes are
+// that neither LDS nor HBM bounds the kernels of fp32 products: what does is how evenly the chip's matrix pipes are
 // loaded and how much of the time they wait for a wave's own loads, barriers and address arithmetic.
 // Hence small workgroups (four waves), several of them on a compute unit, k-tiles requested at least two
 // iterations before their use, one barrier per iteration that leaves global loads in flight, output tiles of a quarter
 // of the size where the last round of tiles would leave compute units empty, and few launches: gate and up share
 // one (and with it their tiles), the two halves of the input gradient another, the three weight gradients a third.
+#include <cmath>
+
 #include "f32_split.h"
 
 namespace {
@@ -247,9 +250,10 @@ __device__ __forceinline__ Job job_of(int tiles, int cus, int most, int chunk = 
 // Workgroups for at most `tiles` tiles: each XCD may round its two shares up.
 unsigned grid_of(int64_t tiles, int64_t cus) { return (unsigned)((tiles + 3 * (cus * 3 / 4) + 7) / 8 * 8 + 16); }
 
-// How many quarters the split tiles' last round may be cut into: one workgroup is resident on a compute unit, a whole tile takes
-// 9 + 0.03 k us and a quarter 9 + 0.009 k (k: length of the contraction), so that two rounds of quarters pay from 700 on.
-__device__ __forceinline__ int split_cut(int k, int cus) { return k > 700 ? 2 * cus : cus; }
+// How many quarters the split tiles' last round may be cut into: one workgroup is resident on a compute unit, and two rounds of quarters
+// take less time than one of whole tiles for contractions past about 900 (128 tiles, operands by turns k-contiguous and not:
+// 640 29 us whole; 768 33 to 36 in quarters, where whole tiles would take 33; 1024 40 to 44, and 42 to 43; 2048 69 to 73, and 78).
+__host__ __device__ __forceinline__ int split_cut(int k, int cus) { return k > 900 ? 2 * cus : cus; }
 
 template <int MODE>
 constexpr bool b_kcont = MODE == PLAIN_T || MODE == GATEUP;
@@ -358,7 +362,7 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& p, float* lds, int e, 
   }
 }
 
-// The same on the fp16 matrix cores (f32_split.h)
+// The same on the bf16 matrix cores (f32_split.h)
 template <int MODE, typename S>
 using SplitB = typename std::conditional<b_kcont<MODE>, SplitInner<S::BN, S::TK, S::NT>, SplitOuter<S::BN, S::TK, S::NT>>::type;
 template <int MODE, typename S>
@@ -409,13 +413,14 @@ __device__ __forceinline__ void split_rows_tile(const RowsArgs& p, char* lds, in
     }
   };
   const int l32 = lane & 31, lh = lane >> 5;
-  const auto again = [&](int r0, int c0, f32x16& acc) {  // the block of rows r0.., columns c0.. of the tile
+  const auto again = [&](int r0, int c0, int share, f32x16& acc) {  // the block of rows r0.., columns c0.. of the tile
+    const int quarter = p.K / 4, k1 = share == 3 ? p.K : (share + 1) * quarter;
     const int c = c0 + l32, col = DUAL ? c / 32 * 16 + (c & 15) : c;
     for (int seg = 0; seg < (MODE == GATEUP_BWD ? 2 : 1); ++seg) {
       const float *A = seg ? A1 : A0, *B = seg || (DUAL && (c & 16)) ? B1 : B0;
-      for (int k = 0; k < p.K; k += 2)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(OpB::value(B, ldb, p.N - n0, p.K, col, k + lh),
-                                                   OpA::value(A, p.K, row_end - row0, p.K, r0 + l32, k + lh), acc, 0, 0, 0);
+      for (int k = share * quarter; k < k1; k += 2)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(OpB::value(B, ldb, p.N - n0, k1, col, k + lh),
+                                                   OpA::value(A, p.K, row_end - row0, k1, r0 + l32, k + lh), acc, 0, 0, 0);
     }
   };
   typename L::Out out;
@@ -588,10 +593,11 @@ __device__ __forceinline__ void split_wgrad_tile(const F32Stack& s, char* lds, i
       for (int h = 0; h < 2; ++h) st.v[OpA::CH + c][h] = opB.load(c, h, rb, left);
   };
   const int l32 = lane & 31, lh = lane >> 5;
-  const auto again = [&](int r0, int c0, f32x16& acc) {
-    for (int k = 0; k < end - b; k += 2)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(OpB::value(B, s.N, s.N - n0, end - b, c0 + l32, k + lh),
-                                                 OpA::value(A, s.M, s.M - m0, end - b, r0 + l32, k + lh), acc, 0, 0, 0);
+  const auto again = [&](int r0, int c0, int share, f32x16& acc) {
+    const int quarter = (end - b) / 4, k1 = share == 3 ? end - b : (share + 1) * quarter;
+    for (int k = share * quarter; k < k1; k += 2)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(OpB::value(B, s.N, s.N - n0, k1, c0 + l32, k + lh),
+                                                 OpA::value(A, s.M, s.M - m0, k1, r0 + l32, k + lh), acc, 0, 0, 0);
   };
   typename L::Out out;
   const int n = (end - b + S::TK - 1) / S::TK;  // (without rows: one k-tile of zeros)
@@ -747,23 +753,33 @@ bool large_tiles(int64_t tiles128) {
   return tiles128 >= 8 * (int64_t)moe_compute_units();
 }
 
-// Split tiles (f32_split.h) keep a whole compute unit busy for 9 us and 0.03 us for each of the contraction's values: they take
-// launches with work for the chip and experts that fill a tile at least half (weight gradients: that have some length).  The
-// fused launches, where the second operand or the epilogue takes a tile longer, also need tiles for most compute units, by the
-// bound on their number.  The rules below are within 1.1 % (weight gradients 2.1 %) of the best of the three tiles in the mean
-// over 1040 row launches and 260 of weight gradients: 4 to 128 experts, 64 to 32768 rows, widths 256 to 4096 and 128 to 2048.
-// 4096 rows of 8 experts, 1024 <-> 512, the five launches, fp32 tiles and these: 77, 43, 46, 76, 108 and 56, 34, 40,
-// 54, 71 us; 256 rows: 67 and 85 us in all.  Contractions of 256 to 384 (taken) gain less: 13992 rows of 12 experts, 2368 <-> 256,
-// down 164 -> 132; 21996 of 32, 768 <-> 256, 84 -> 72.  Few tiles (not taken): 1492 rows of 12, 1920 <-> 448, dgrad-down, 48 to 92
-// tiles, 45 and 62.
+// Split tiles (f32_split.h) keep a whole compute unit busy; fp32 ones of 64 x 64 share it.  Both launches' times follow, to 8 %, from
+// their tiles and the contraction's length k, us: a round of split tiles `start` + 0.038 k, one of quarters 7 + 0.0115 k; fp32
+// tiles 5 + 0.0025 k and, of 256 compute units, `each` + 0.0645 k a thousand.  Split where that is 5 % less, experts fill half a tile
+// (weight gradients: have some rows, and tiles for every compute unit, as one heavy expert's would keep few of them), half of what
+// is computed is wanted (weight gradients, which have no other remainder: 0.7), and there is work to gain by.  DOWN_BWD, whose
+// epilogue reads two more operands, needs more of it.  900 drawn layers, 4 to 128 experts, 64 to 32768 rows, even to skewed, widths
+// 256 to 4096 and 128 to 2048: of 4500 launches 1111 are taken, gate/up 1.26, down 1.22, down's input gradient 1.16, gate/up's
+// 1.19, weight gradients 1.22 times as fast as in fp32 tiles in the mean, 27 of them slower by more than 3 %.
 constexpr int SPLIT = 1;
-bool split_rows(int64_t E, int64_t R, int64_t N, int64_t K, int64_t tiles128, bool fused) {
-  if (forced_tile) return forced_tile == SPLIT;
-  return R >= 64 * E && K >= 256 && R * N >= ((int64_t)1 << 30) / K && (!fused || tiles128 * 8 >= 5 * (int64_t)moe_compute_units());
+bool split_pays(double tiles128, double tiles64, double k, double start, double each) {
+  const double cus = moe_compute_units(), whole = std::floor(tiles128 / cus), rest = tiles128 - whole * cus;
+  const bool cut = rest * 4 <= split_cut((int)k, (int)cus);
+  const double split = (cut ? whole : whole + 1) * (start + 0.038 * k) + (cut ? std::ceil(rest * 4 / cus) * (7 + 0.0115 * k) : 0);
+  return split < 0.95 * (5 + 0.0025 * k + tiles64 / 1000 * 256 / cus * (each + 0.0645 * k));
 }
-bool split_wgrad(int64_t E, int64_t R, int64_t elements) {
+bool split_rows(Mode mode, int64_t E, int64_t R, int64_t N, int64_t K) {
   if (forced_tile) return forced_tile == SPLIT;
-  return R >= 192 * E && elements >= ((int64_t)1 << 30) / R;
+  const auto tiles = [&](int t) { return moe_expected_tiles(R, E, t) * ((N + t - 1) / t); };
+  const bool bwd = mode == DOWN_BWD;
+  const double work = (double)R * N * K / (1 << 30);
+  return R >= 64 * E && K >= (bwd ? 512 : 256) && work >= (bwd ? 1.5 : 1) && R * N * 2 >= tiles(128) * 128 * 128 &&
+         split_pays(tiles(128), tiles(64), (double)K, bwd ? 14 : mode == GATEUP ? 8 : 6, bwd ? 11 : mode == GATEUP ? 4.7 : 2.5);
+}
+bool split_wgrad(int64_t E, int64_t R, int64_t elements, int64_t tiles128, int64_t tiles64) {  // elements, tiles: of all stacks
+  if (forced_tile) return forced_tile == SPLIT;
+  return R >= 224 * E && tiles128 >= moe_compute_units() && elements >= ((int64_t)1 << 30) / R && 10 * E * elements >= 7 * tiles128 * 128 * 128 &&
+         split_pays((double)tiles128, (double)tiles64, (double)R / E, 9, 3.4);
 }
 
 int check_rows(int64_t E, int64_t R, int64_t N, int64_t K) {
@@ -780,8 +796,7 @@ int launch_rows(RowsArgs a, int64_t E, int64_t R, int64_t N, int64_t K, hipStrea
   a.E = (int)E, a.R = (int)R, a.N = (int)N, a.K = (int)K;
   const int cus = moe_compute_units();
   const auto tiles = [&](int64_t t) { return (R / t + E) * ((N * (MODE == GATEUP ? 2 : 1) + t - 1) / t); };  // at most
-  constexpr bool FUSED = MODE == GATEUP || MODE == DOWN_BWD || MODE == GATEUP_BWD;
-  if (split_rows(E, R, N * (MODE == GATEUP ? 2 : 1), K * (MODE == GATEUP_BWD ? 2 : 1), tiles(128), FUSED)) {
+  if (split_rows((Mode)MODE, E, R, N * (MODE == GATEUP ? 2 : 1), K * (MODE == GATEUP_BWD ? 2 : 1))) {
     constexpr int LDS = larger(SplitRowsLoop<MODE, SplitTile>::LDS_BYTES, SplitRowsLoop<MODE, SplitQuarter>::LDS_BYTES);
     static bool done[MOE_MAX_DEVICES];
     const auto kern = f32_split_rows_kernel<MODE, SplitTile, SplitQuarter>;
@@ -881,7 +896,7 @@ static int wgrads(const F32Stack* s, int n, const int32_t* offs, int64_t E, int6
   const int cus = moe_compute_units();
   int64_t elements = 0;
   for (int i = 0; i < n; ++i) elements += s[i].M * (int64_t)s[i].N;
-  const bool large = large_tiles(tiles(128)), split = R > 0 && split_wgrad(E, R, elements);
+  const bool large = large_tiles(tiles(128)), split = R > 0 && split_wgrad(E, R, elements, tiles(128), tiles(64));
   const auto go = [&](auto deal) {
     constexpr bool DEAL = decltype(deal)::value;
     if (split) {

@@ -1,16 +1,15 @@
-// fp32 products on the fp16 matrix cores.  A value times a power of two is the sum of two fp16 values, x = h + l with h the
-// nearest one and l the nearest to what is left, to 2^-24 of it.  Of the four products of two such sums three are added
-// up in the matrix cores' fp32 accumulators (hl, lh, hh; ll is below 2^-24 of the product and mostly far below): three
-// instructions at sixteen times the rate of the fp32 one, and closer to the exact sum, since an accumulator is rounded 3 times for
-// every 16 products instead of 8 times.  Relative 2-norm error against fp64, normal operands, 64 / 256 / 1024 / 4096 products:
-// 1.2e-7 / 1.9e-7 / 3.6e-7 / 7.1e-7, the fp32 instruction 1.4e-7 / 2.9e-7 / 5.7e-7 / 1.1e-6 (16 products: 8.7e-8, 7.3e-8).
-// (Three bf16 parts need no scale, but six products: 2.3e-7 .. 1.0e-6, and 205 us where this takes 168.)
+// fp32 products on the bf16 matrix cores.  An fp32 value is the sum of three bf16 values, exactly: x = h + m + l, each the nearest to
+// what the ones before it leave (8 significant bits each: h leaves 16 at most, m then 7).  bf16 has the
+// exponents of fp32, so this holds for each value by itself, whatever the sizes of its neighbours.  Of the nine products of two
+// such sums six are added up in the matrix cores' fp32 accumulators, small ones first (lh, hl, mm, mh, hm, hh); the rest
+// (ml, lm, ll) is at most 2^-24 of the product, mostly far below.  Six instructions at sixteen times the rate of the fp32 one.
+// Relative 2-norm error against fp64, normal operands, 4 / 16 / 64 / 256 / 1024 / 4096 products: 3.2e-8 / 3.4e-8 / 5.5e-8 / 1.2e-7 /
+// 2.4e-7 / 5.0e-7 in quarters of a tile, the fp32 instruction 4.0e-8 / 6.0e-8 / 8.5e-8 / 1.5e-7 / 2.9e-7 / 5.7e-7 there.
+// (Two fp16 parts need half the products, and lose what a scale shared with larger neighbours takes from small values.)
 //
-// The power of two brings the largest value of the first two k-tiles to 2^12 .. 2^13, so that what is lost of smaller ones is
-// below 2^-37 of it: of a row where the operand is rows of activations or their gradients, of the tile where it is weights,
-// or the contraction is along rows.  A k-tile whose values no longer fit, or are all below 4, gets another one, and
-// what was added up so far is multiplied by the ratio: what is lost is always below 2^-27 of the k-tile's largest value.  Infinities and NaN give sums that are not finite: such a tile is computed again with the fp32
-// instruction, and every result is the one it gives.
+// Values are multiplied by 2^24 on the way, so that no part of one is denormal (the smallest fp32 bit, 2^-149, becomes 2^-125),
+// and sums by 2^-48 at the end.  What does not fit then (values from 2^104 on, sums from 2^80 on), infinities and NaN make
+// an element's sum infinite or NaN: such an element, and no other, is the fp32 instruction's.
 #pragma once
 #include "internal.h"
 #include "tile_ops.h"
@@ -29,9 +28,6 @@ __device__ __forceinline__ f32x4 window_load(__amdgpu_buffer_rsrc_t rs, unsigned
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
 }
 
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-
 // f(0), f(1), .. f(N - 1) with constants for arguments: what they index stays in registers, however long the code
 template <typename F, int... I>
 __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>) {
@@ -42,34 +38,15 @@ __device__ __forceinline__ void each(F&& f) {
   each_of(f, std::make_integer_sequence<int, N>{});
 }
 
-// Two values times `scale`, in their two parts, packed.
-__device__ __forceinline__ uint32_t high_parts(float x, float y, float scale) {
-  const f16x2 h = {(_Float16)(x * scale), (_Float16)(y * scale)};
-  uint32_t w = __builtin_bit_cast(uint32_t, h);
-  asm("" : "+v"(w));  // (the compiler would convert each once more on its own to have it unpacked)
-  return w;
-}
-__device__ __forceinline__ uint32_t low_parts(float x, float y, float scale, uint32_t high) {
-  const f16x2 h = __builtin_bit_cast(f16x2, high);
-  const f16x2 l = {(_Float16)__builtin_fmaf(x, scale, -(float)h[0]), (_Float16)__builtin_fmaf(y, scale, -(float)h[1])};
-  return __builtin_bit_cast(uint32_t, l);
-}
-// max(big, |x|, |y|), where a NaN counts for nothing (fmaxf would quiet every operand first)
-__device__ __forceinline__ void larger_of(float& big, float x, float y) {
-  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(big) : "v"(x), "v"(y));
-}
+constexpr float SPLIT_SCALE = 16777216.f;  // 2^24, and what undoes it twice
+constexpr int SPLIT_EXP = -48;
 
-// The largest of the wave's values >= 0, which integers order as floats (in the vector unit alone, as wave_inclusive).
-__device__ __forceinline__ float wave_largest(float f) {
-  int v = __builtin_bit_cast(int, f);
-  const auto larger = [&](int w) { v = v > w ? v : w; };
-  larger(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true));  // row_shr:1, 2, 4, 8: inside the rows of 16
-  larger(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true));
-  larger(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true));
-  larger(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true));
-  larger(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 to rows 1 and 3
-  larger(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 to rows 2 and 3
-  return __builtin_bit_cast(float, read_lane(v, MOE_WAVE - 1));
+// The next part of two values, packed; what it leaves of them.
+__device__ __forceinline__ uint32_t next_part(float& x, float& y) {
+  uint32_t w = pack_bf16x2(x, y);
+  asm("" : "+v"(w));  // (the compiler would convert each once more on its own to have it unpacked)
+  x -= bf16lo(w), y -= bf16hi(w);
+  return w;
 }
 
 // Operand tiles of ROWS x TK in LDS, one plane a part.  A thread moves chunks of eight values.
@@ -80,7 +57,6 @@ __device__ __forceinline__ float wave_largest(float f) {
 //             through the transposing read (see OpOuter).
 template <int ROWS, int TK, int NT>
 struct SplitInner {
-  static constexpr bool INNER = true;
   static constexpr int PLANE = ROWS * TK * 2, CPR = TK / 8, STEP = NT / CPR, CH = ROWS * CPR / NT;
   static_assert(ROWS * CPR % NT == 0 && (CPR == 4 || CPR == 8), "loader shape");
   unsigned voff[CH];
@@ -109,20 +85,8 @@ struct SplitInner {
     const int l = lane_id(), r = row0 + (l & 31);
     return Lane{r * TK * 2, (l >> 5) ^ swizzle(r)};
   }
-  static __device__ __forceinline__ f16x8 frag(const char* plane, const Lane& l, int rows, int ks) {
-    return *reinterpret_cast<const f16x8*>(plane + (l.at + rows * TK * 2 + ((l.chunk ^ (ks * 2)) << 4)));
-  }
-  // the largest value of a row's chunks (the lanes that hold them), which integers order as floats
-  static __device__ __forceinline__ float row_largest(float f) {
-    int v = __builtin_bit_cast(int, f), w = __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, true);  // quad_perm 1 0 3 2
-    v = v > w ? v : w;
-    w = __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, true);  // quad_perm 2 3 0 1
-    v = v > w ? v : w;
-    if constexpr (CPR == 8) {
-      w = __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true);  // row_half_mirror
-      v = v > w ? v : w;
-    }
-    return __builtin_bit_cast(float, v);
+  static __device__ __forceinline__ bf16x8 frag(const char* plane, const Lane& l, int rows, int ks) {
+    return *reinterpret_cast<const bf16x8*>(plane + (l.at + rows * TK * 2 + ((l.chunk ^ (ks * 2)) << 4)));
   }
   // one value, anywhere
   static __device__ __forceinline__ float value(const float* base, int ld, int rows, int k_end, int r, int k) {
@@ -131,7 +95,6 @@ struct SplitInner {
 };
 template <int ROWS, int TK, int NT>
 struct SplitOuter {
-  static constexpr bool INNER = false;
   static constexpr int PLANE = ROWS * TK * 2, CPL = ROWS / 8, STEP = NT / CPL, CH = TK * CPL / NT;
   static_assert(TK * CPL % NT == 0 && (ROWS == 64 || ROWS == 128), "loader shape");
   unsigned voff[CH];
@@ -161,13 +124,13 @@ struct SplitOuter {
     const int l = lane_id(), i = l & 15, b = l >> 4;
     return Lane{((b >> 1) * 8 + (i >> 2)) * ROWS * 2 + (i & 1) * 8, (row0 / 8 + 2 * (b & 1) + ((i & 3) >> 1)) ^ swizzle(i >> 2)};
   }
-  static __device__ __forceinline__ f16x8 frag(const char* plane, const Lane& l, int rows, int ks) {
+  static __device__ __forceinline__ bf16x8 frag(const char* plane, const Lane& l, int rows, int ks) {
     const char* at = plane + (l.at + ((l.chunk ^ (rows / 8)) << 4) + ks * 16 * ROWS * 2);
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * ROWS * 2));
     typedef __attribute__((ext_vector_type(8))) short s16x8;
     const s16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return __builtin_bit_cast(f16x8, r);
+    return __builtin_bit_cast(bf16x8, r);
   }
   static __device__ __forceinline__ float value(const float* base, int ld, int rows, int k_end, int r, int k) {
     return r < rows && k < k_end ? base[(long long)k * ld + r] : 0.f;
@@ -187,20 +150,16 @@ struct SplitShape {
 
 template <typename S, typename OpA, typename OpB>
 struct SplitLoop {
-  static constexpr int CH = OpA::CH + OpB::CH, STAGE = 2 * (OpA::PLANE + OpB::PLANE);
-  static constexpr int SWAP = S::WM * S::WN * S::ITEMS * (S::WK - 1) * 2048, WORDS = 128;
-  // An operand A that lies k-contiguous is scaled row by row: then no row's values matter to another one's result
-  static constexpr bool BY_ROW = OpA::INNER;
-  static constexpr int ROW_WORDS = BY_ROW ? 5 * S::BM * 4 : 0;
-  static_assert(!BY_ROW || OpA::CH == 1, "a thread's values of A are of one row");
-  static constexpr int LDS_BYTES = (2 * STAGE > SWAP ? 2 * STAGE : SWAP) + WORDS + ROW_WORDS;
+  static constexpr int CH = OpA::CH + OpB::CH, STAGE = 3 * (OpA::PLANE + OpB::PLANE);
+  static constexpr int SWAP = S::WM * S::WN * S::ITEMS * (S::WK - 1) * 2048;
+  static constexpr int LDS_BYTES = 2 * STAGE > SWAP ? 2 * STAGE : SWAP;
   static constexpr int PF = 4;  // k-tiles in registers on their way to LDS
   typedef f32x16 Acc[S::NM][S::NN];
   struct Stage {
     f32x4 v[CH][2];
   };
-  struct Frags {
-    f16x8 a[S::NM][2], b[S::NN][2];
+  struct Frags {  // of the parts h, m, l
+    bf16x8 a[S::NM][3], b[S::NN][3];
   };
   // What a wave ends up with: item i is the quads g and g + 2 of block (bm, bn), lane l row l % 32 of the block, columns
   // 8 * quad + 4 * (l / 32) .. + 3
@@ -212,12 +171,13 @@ struct SplitLoop {
   }
 
   // acc = A-tile x B-tile over `n` > 0 k-tiles.  While k-tile t is multiplied, the fragments of t + 1 are read, t + 2 is split and
-  // written to the LDS stage that t has left, and t + 6 is requested: one barrier a k-tile, and nothing between two of them that
-  // waits for one another.  16384 rows of 8 experts, 1024 -> 2 x 512, four tiles of 128 x 128 to a compute unit: 168 us (fp32 instruction: 285), where the
-  // products alone take 76 and a tile's start and end 35; each k-tile of 32 has 768 cycles of products, 470 of LDS
-  // writes (70 bytes a cycle; reads 240), 450 of vector work.  Splitting after the LDS instead (fp32 values straight
-  // from memory into the ring, twice the vector work) takes a tenth longer: vector and matrix work of two waves hardly overlap.
-  // `load(t, stage)` requests a k-tile, `again(row, column, acc)` computes a block with fp32 products.
+  // written to the LDS stage that t has left, and t + 2 + PF is requested: one barrier a k-tile, and nothing between two of them that
+  // waits for one another.  What bounds it is the matrix unit, at the clock that its power leaves, with little to spare: a k-tile of 32
+  // has 1536 cycles of products, 700 of LDS writes, 375 of reads and 830 of vector work.  16384 rows of 8 experts, 1024 -> 2 x 512,
+  // four tiles of 128 x 128 to a compute unit: 211 us (fp32 instruction: 281), where the products alone take 161 at the rate of a
+  // large bf16 product.  224 to 232 registers: h alone is in them twice (below), with all parts twice there would be none left.
+  // `load(t, stage)` requests a k-tile, `again(row, column, share, acc)` adds up a quarter of the fp32 products of a
+  // block.
   template <typename Load, typename Again>
   static __device__ __forceinline__ void run(char* lds, int n, int wv, Out& out, Load&& load, Again&& again) {
     const int wn = wv % S::WN, wm = wv / S::WN % S::WM, wk = wv / (S::WN * S::WM);
@@ -234,191 +194,82 @@ struct SplitLoop {
       f.a[x][p] = OpA::frag(lds + b * STAGE + p * OpA::PLANE, la, x * 32, wk);
     };
     const auto read_b = [&](int b, Frags& f, int x, int p) {
-      f.b[x][p] = OpB::frag(lds + b * STAGE + 2 * OpA::PLANE + p * OpB::PLANE, lb, x * 32, wk);
+      f.b[x][p] = OpB::frag(lds + b * STAGE + 3 * OpA::PLANE + p * OpB::PLANE, lb, x * 32, wk);
     };
-    u32x4 parts[2];
-    float scale_a, scale_b;  // powers of two: a row's (BY_ROW) or all threads', all threads'
+    u32x4 parts[3];
+    float x, y;
     // step i of chunk c: a part of two of its values; the last one also writes the chunk
     const auto put = [&](const Stage& s, int b, auto chunk, auto step) __attribute__((always_inline)) {
-      constexpr int c = decltype(chunk)::value, q = decltype(step)::value / 2, p = decltype(step)::value % 2;
-      const float x = s.v[c][q >> 1][(q & 1) * 2], y = s.v[c][q >> 1][(q & 1) * 2 + 1], scale = c < OpA::CH ? scale_a : scale_b;
-      if constexpr (p == 0) parts[0][q] = high_parts(x, y, scale);
-      else parts[1][q] = low_parts(x, y, scale, parts[0][q]);
-      if constexpr (q == 3 && p == 1) {
-        char* to = c < OpA::CH ? lds + b * STAGE + OpA::place(c) : lds + b * STAGE + 2 * OpA::PLANE + OpB::place(c - OpA::CH);
-        *reinterpret_cast<u32x4*>(to) = parts[0];
-        *reinterpret_cast<u32x4*>(to + (c < OpA::CH ? OpA::PLANE : OpB::PLANE)) = parts[1];
-      }
-    };
-    // the largest values of a k-tile's chunks
-    const auto largest = [&](const Stage& s, float& a, float& b) __attribute__((always_inline)) {
-      each<CH * 4>([&](auto i) __attribute__((always_inline)) {
-        constexpr int c = decltype(i)::value / 4, q = decltype(i)::value % 4;
-        larger_of(c < OpA::CH ? a : b, s.v[c][q >> 1][(q & 1) * 2], s.v[c][q >> 1][(q & 1) * 2 + 1]);
-      });
-    };
-    // [8][2] largest values; [2] "values do not fit"; [2][2] the last k-tile that was large enough
-    int* words = reinterpret_cast<int*>(lds + LDS_BYTES - WORDS - ROW_WORDS);
-    float* row_grown = reinterpret_cast<float*>(lds + LDS_BYTES - ROW_WORDS);  // [4][BM] for k-tile t % 4, as `grown`
-    int* row_exp = reinterpret_cast<int*>(row_grown + 4 * S::BM);               // [BM] at the end
-    const auto largest_of_all = [&](float& a, float& b) {  // (two barriers)
-      a = wave_largest(a), b = wave_largest(b);
-      if (lane_id() == 0) words[2 * wv] = __builtin_bit_cast(int, a), words[2 * wv + 1] = __builtin_bit_cast(int, b);
-      lds_barrier();
-      int ia = 0, ib = 0;  // (as integers: an infinity is the largest, a NaN was left out)
+      constexpr int c = decltype(chunk)::value, q = decltype(step)::value / 3, p = decltype(step)::value % 3;
+      if constexpr (p == 0) x = s.v[c][q >> 1][(q & 1) * 2] * SPLIT_SCALE, y = s.v[c][q >> 1][(q & 1) * 2 + 1] * SPLIT_SCALE;
+      if constexpr (p < 2) parts[p][q] = next_part(x, y);
+      else parts[p][q] = pack_bf16x2(x, y);
+      if constexpr (q == 3 && p == 2) {
+        char* to = c < OpA::CH ? lds + b * STAGE + OpA::place(c) : lds + b * STAGE + 3 * OpA::PLANE + OpB::place(c - OpA::CH);
 #pragma unroll
-      for (int w = 0; w < S::NT / 64; ++w) {
-        ia = ia > words[2 * w] ? ia : words[2 * w];
-        ib = ib > words[2 * w + 1] ? ib : words[2 * w + 1];
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4*>(to + i * (c < OpA::CH ? OpA::PLANE : OpB::PLANE)) = parts[i];
       }
-      a = __builtin_bit_cast(float, uniform(ia)), b = __builtin_bit_cast(float, uniform(ib));
-      lds_barrier();
     };
-    int exp_a, exp_b, least_a, least_b;  // least: the smallest so far
-    float limit_a, limit_b, low_a, low_b;
-    // What the sums are multiplied by before k-tile t, t + 1, t + 2 (BY_ROW: times row_grown; 0: nothing)
-    float grown[3] = {0.f, 0.f, 0.f};
-    // The largest of so many values becomes 2^12 to 2^13: 7 times more fits, and parts below 2^-38 of it are lost.
-    const auto exponent_for = [](float big) {
-      const int e = 12 + 127 - (__builtin_bit_cast(int, big) >> 23);
-      return e > 126 ? 126 : e < -114 ? -114 : e;
-    };
-    const auto power = [](int e) { return __builtin_bit_cast(float, (127 + e) << 23); };
-    const auto set_scales = [&](int ea, int eb) {
-      exp_a = ea, exp_b = eb;
-      scale_a = power(ea), scale_b = power(eb);
-      limit_a = 60000.f * power(-ea), limit_b = 60000.f * power(-eb);
-      low_a = 4.f * power(-ea), low_b = 4.f * power(-eb);
-    };
-    const auto too_large = [](float big, float limit) { return big > limit && big < __builtin_inff(); };
-    const auto too_small = [](float big, float low) { return big > 0.f && big < low; };
-    const auto report = [&](int t, int word, float a, float b) __attribute__((always_inline)) {  // the largest values of k-tile t
-      bool misfit = too_large(b, limit_b);
-      if constexpr (BY_ROW) {
-        a = OpA::row_largest(a);
-        misfit |= too_large(a, limit_a) | too_small(a, low_a);
-      } else {
-        misfit |= too_large(a, limit_a);
-        if (__ballot(a >= low_a)) words[18 + 2 * word] = t;
-      }
-      if (__ballot(misfit)) words[16 + word] = 1;
-      if (__ballot(b >= low_b)) words[19 + 2 * word] = t;
-    };
-    const auto rescale = [&](const Stage& s, int t, int word) {  // for k-tile t, which s holds
-      float a = 0.f, b = 0.f, all_a;
-      largest(s, a, b);
-      all_a = a;
-      largest_of_all(all_a, b);
-      if constexpr (BY_ROW) a = OpA::row_largest(a);
-      else a = all_a;
-      // (2^30 more than the least: the sums, below 2^42 then, stay finite)
-      const auto fitting = [&](float big, float low, float limit, int e, int least) {
-        const int want = too_large(big, limit) || too_small(big, low) ? exponent_for(big) : e;
-        return want < least + 30 ? want : least + 30;
-      };
-      const int ea = fitting(a, low_a, limit_a, exp_a, least_a), eb = fitting(b, low_b, limit_b, exp_b, least_b);
-      const auto ratio = [&](int d) { return power(d < -126 ? -126 : d); };  // (what is lost so is far below the rest)
-      grown[2] = ratio(eb - exp_b);
-      if constexpr (BY_ROW) {
-        if (threadIdx.x % OpA::CPR == 0) row_grown[(t & 3) * S::BM + OpA::row(0)] = ratio(ea - exp_a);
-      } else {
-        grown[2] = ratio(ea - exp_a + eb - exp_b);
-      }
-      least_a = least_a < ea ? least_a : ea, least_b = least_b < eb ? least_b : eb;
-      set_scales(ea, eb);
-      words[16 + word] = 0;
-    };
+    constexpr int STEPS = 12;  // of a chunk
     const auto put_all = [&](const Stage& s, int b) __attribute__((always_inline)) {
-      each<CH * 8>([&](auto q) __attribute__((always_inline)) {
-        put(s, b, std::integral_constant<int, decltype(q)::value / 8>{}, std::integral_constant<int, decltype(q)::value % 8>{});
+      each<CH * STEPS>([&](auto q) __attribute__((always_inline)) {
+        put(s, b, std::integral_constant<int, decltype(q)::value / STEPS>{}, std::integral_constant<int, decltype(q)::value % STEPS>{});
       });
     };
     Stage st[PF];
     Frags fr[2];
     const auto step = [&](int t, auto at) __attribute__((always_inline)) {  // at: t modulo PF
-      constexpr int b = decltype(at)::value & 1, held = (decltype(at)::value + 2) % PF, after = (decltype(at)::value + 3) % PF;
-      constexpr int READS = (S::NM + S::NN) * 2, BLOCKS = S::NM * S::NN, MFMAS = BLOCKS * 3, PUTS = CH * 8;
+      constexpr int b = decltype(at)::value & 1, held = (decltype(at)::value + 2) % PF;
+      constexpr int BLOCKS = S::NM * S::NN, MFMAS = BLOCKS * 6, READS = S::NM + S::NN;
+      constexpr int PART_A[6] = {2, 0, 1, 1, 0, 0}, PART_B[6] = {0, 2, 1, 0, 1, 0};
       const Frags& f = fr[b];
       Frags& next = fr[b ^ 1];
-      const int misfit = words[16 + b], large_a = BY_ROW ? t + 2 : words[18 + 2 * b], large_b = words[19 + 2 * b];  // of k-tile t + 2
-      if (grown[0] != 0.f) {
-#pragma unroll
-        for (int i = 0; i < S::NM; ++i) {
-          float by = grown[0];
-          if constexpr (BY_ROW) by *= row_grown[(t & 3) * S::BM + (wm * S::NM + i) * 32 + (lane_id() & 31)];
-#pragma unroll
-          for (int j = 0; j < S::NN; ++j) acc[i][j] *= by;
-        }
-      }
-      float seen_a = 0.f, seen_b = 0.f;  // of k-tile t + 3
       each<MFMAS>([&](auto slot) __attribute__((always_inline)) {
-        constexpr int s = decltype(slot)::value, term = s / BLOCKS, bm = s % BLOCKS / S::NN, bn = s % S::NN;  // small products first
-        acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[bn][term == 0], f.a[bm][term == 1], acc[bm][bn], 0, 0, 0);
-        constexpr auto upto = [](int at, int n, int begin, int end) {
-          const int v = (at - begin) * n / (end - begin);
-          return at < begin ? 0 : v < n ? v : n;
+        constexpr int s = decltype(slot)::value, term = s / BLOCKS, bm = s % BLOCKS / S::NN, bn = s % S::NN;
+        acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[bn][PART_B[term]], f.a[bm][PART_A[term]], acc[bm][bn], 0, 0, 0);
+        // n things done by slots begin .. end - 1: those of slot s
+        const auto share = [&](auto n_, auto begin_, auto end_, auto&& what) __attribute__((always_inline)) {
+          constexpr int n = decltype(n_)::value, begin = decltype(begin_)::value, end = decltype(end_)::value;
+          constexpr auto upto = [](int at) { return at < begin ? 0 : at >= end ? n : (at - begin) * n / (end - begin); };
+          constexpr int from = upto(s), to = upto(s + 1);
+          each<to - from>([&](auto i) __attribute__((always_inline)) { what(std::integral_constant<int, from + decltype(i)::value>{}); });
         };
-        constexpr int CHECK = MFMAS / 6, R0 = upto(s, READS, 0, MFMAS * 2 / 3), R1 = upto(s + 1, READS, 0, MFMAS * 2 / 3);
-        constexpr int Q0 = upto(s, PUTS, CHECK, MFMAS * 5 / 6), Q1 = upto(s + 1, PUTS, CHECK, MFMAS * 5 / 6);
-        if constexpr (s == CHECK) {
-          if (uniform(misfit | (large_a ^ (t + 2)) | (large_b ^ (t + 2))) && t + 2 < n) rescale(st[held], t + 2, b);
-          grown[0] = grown[1], grown[1] = grown[2], grown[2] = 0.f;
-        }
-        each<R1 - R0>([&](auto i) __attribute__((always_inline)) {
-          constexpr int r = R0 + decltype(i)::value, rb = r - S::NM * 2;
-          if constexpr (r < S::NM * 2) read_a(b ^ 1, next, r % S::NM, r / S::NM);
-          else read_b(b ^ 1, next, rb % S::NN, rb / S::NN);
-        });
-        each<Q1 - Q0>([&](auto i) __attribute__((always_inline)) {
-          constexpr int q = Q0 + decltype(i)::value;
-          put(st[held], b, std::integral_constant<int, q / 8>{}, std::integral_constant<int, q % 8>{});
-        });
-        constexpr int L0 = upto(s, CH * 4, MFMAS / 2, MFMAS), L1 = upto(s + 1, CH * 4, MFMAS / 2, MFMAS);
-        each<L1 - L0>([&](auto i) __attribute__((always_inline)) {
-          constexpr int l = L0 + decltype(i)::value, c = l / 4, q = l % 4;
-          larger_of(c < OpA::CH ? seen_a : seen_b, st[after].v[c][q >> 1][(q & 1) * 2], st[after].v[c][q >> 1][(q & 1) * 2 + 1]);
+        // The parts of t + 1, each where those of t have been used for the last time or soon will: h alone is there twice.
+        const auto read = [&](auto part, auto begin, auto end) __attribute__((always_inline)) {
+          share(std::integral_constant<int, READS>{}, begin, end, [&](auto i) __attribute__((always_inline)) {
+            constexpr int r = decltype(i)::value;
+            if constexpr (r < S::NM) read_a(b ^ 1, next, r, decltype(part)::value);
+            else read_b(b ^ 1, next, r - S::NM, decltype(part)::value);
+          });
+        };
+        using std::integral_constant;
+        read(integral_constant<int, 2>{}, integral_constant<int, 2 * BLOCKS>{}, integral_constant<int, 3 * BLOCKS>{});
+        read(integral_constant<int, 0>{}, integral_constant<int, 3 * BLOCKS>{}, integral_constant<int, 4 * BLOCKS>{});
+        read(integral_constant<int, 1>{}, integral_constant<int, 4 * BLOCKS>{}, integral_constant<int, 5 * BLOCKS + BLOCKS / 2>{});
+        share(integral_constant<int, CH * STEPS>{}, integral_constant<int, 0>{}, integral_constant<int, MFMAS * 5 / 6>{},
+              [&](auto q) __attribute__((always_inline)) {
+          put(st[held], b, integral_constant<int, decltype(q)::value / STEPS>{}, integral_constant<int, decltype(q)::value % STEPS>{});
         });
         if constexpr (s + 1 < MFMAS) __builtin_amdgcn_sched_barrier(0);
       });
       load(t + 2 + PF, st[held]);
-      report(t + 3, b ^ 1, seen_a, seen_b);
       lds_barrier();
     };
-    static_assert(PF == 4, "rounds of four");
-    if (threadIdx.x < 2) words[16 + threadIdx.x] = 0;
-    load(0, st[0]);
-    load(1, st[1]);
-    load(2, st[2]);
-    load(3, st[3]);
-    {
-      float a = 0.f, b = 0.f;
-      largest(st[0], a, b);
-      largest(st[1], a, b);
-      float all_a = a;
-      largest_of_all(all_a, b);
-      if constexpr (BY_ROW) a = OpA::row_largest(a);
-      else a = all_a;
-      set_scales(exponent_for(a), exponent_for(b));
-      least_a = exp_a, least_b = exp_b;
-    }
+    each<PF>([&](auto i) __attribute__((always_inline)) { load(decltype(i)::value, st[decltype(i)::value]); });
     put_all(st[0], 0);
     load(PF, st[0]);
     put_all(st[1], 1);
     load(PF + 1, st[1]);
-    {
-      float a = 0.f, b = 0.f;
-      largest(st[2], a, b);
-      report(2, 0, a, b);
-    }
     lds_barrier();
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
+    for (int p = 0; p < 3; ++p) {
 #pragma unroll
-      for (int x = 0; x < S::NM; ++x) read_a(0, fr[0], x, p);
+      for (int i = 0; i < S::NM; ++i) read_a(0, fr[0], i, p);
 #pragma unroll
-      for (int x = 0; x < S::NN; ++x) read_b(0, fr[0], x, p);
+      for (int i = 0; i < S::NN; ++i) read_b(0, fr[0], i, p);
     }
     lds_barrier();  // (k-tile 2 takes the place of k-tile 0)
+    static_assert(PF == 4, "rounds of four");
     for (int t = 0;; t += 4) {
       step(t, std::integral_constant<int, 0>{});
       if (t + 1 >= n) break;
@@ -430,20 +281,7 @@ struct SplitLoop {
       if (t + 4 >= n) break;
     }
 
-    // ---- the shares of the k-tiles are added up, in their order, and the tile's range is looked at
-    f32x4 zeros = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < S::NM; ++i)
-#pragma unroll
-      for (int j = 0; j < S::NN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) zeros[v & 3] = __builtin_fmaf(acc[i][j][v], 0.f, zeros[v & 3]);
-    const float zero = (zeros[0] + zeros[1]) + (zeros[2] + zeros[3]);
-    const bool finite = __ballot(zero != 0.f) == 0;
-    if (lane_id() == 0) words[wv] = !finite;
-    if constexpr (BY_ROW) {
-      if (threadIdx.x % OpA::CPR == 0) row_exp[OpA::row(0)] = exp_a;
-    }
+    // ---- the shares of the k-tiles are added up, in their order
     const int pos = wm * S::WN + wn;
     f32x4* swap = reinterpret_cast<f32x4*>(lds) + lane_id();
     const auto slot = [&](int item, int owner, int from) {
@@ -460,24 +298,6 @@ struct SplitLoop {
       }
     }
     lds_barrier();
-    int again_all = 0;
-#pragma unroll
-    for (int i = 0; i < S::NT / 64; ++i) again_all |= words[i];
-    if (uniform(again_all)) {
-      // (rare: not worth LDS.  A wave computes the blocks of its items.)
-#pragma unroll 1
-      for (int o = 0; o < S::OWN; ++o) {
-        const int item = wk * S::OWN + o, block = item / 2, g = item & 1;
-        f32x16 a;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) a[v] = 0.f;
-        again((wm * S::NM + block / S::NN) * 32, (wn * S::NN + block % S::NN) * 32, a);
-#pragma unroll
-        for (int k = 0; k < S::OWN; ++k)
-          if (k == o) out.lo[k] = g ? quad(a, 1) : quad(a, 0), out.hi[k] = g ? quad(a, 3) : quad(a, 2);
-      }
-      return;
-    }
 #pragma unroll
     for (int i = 0; i < S::ITEMS; ++i) {
       const int owner = i / S::OWN, g = i & 1;
@@ -490,13 +310,43 @@ struct SplitLoop {
           if (from == 0) lo = l, hi = h;
           else lo += l, hi += h;
         }
-        const int e = (BY_ROW ? row_exp[(wm * S::NM + i / 2 / S::NN) * 32 + (lane_id() & 31)] : exp_a) + exp_b;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          out.lo[i % S::OWN][c] = __builtin_ldexpf(lo[c], -e);
-          out.hi[i % S::OWN][c] = __builtin_ldexpf(hi[c], -e);
+          out.lo[i % S::OWN][c] = __builtin_ldexpf(lo[c], SPLIT_EXP);
+          out.hi[i % S::OWN][c] = __builtin_ldexpf(hi[c], SPLIT_EXP);
         }
       }
+    }
+    // Elements that are not finite.  (Rare: not worth LDS.  A wave computes the blocks of its items.)
+    const auto odd = [](float v) { return __builtin_fabsf(v) >= __builtin_inff() || v != v; };
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < S::OWN; ++k)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) any |= odd(out.lo[k][c]) || odd(out.hi[k][c]);
+    if (__ballot(any) == 0) return;
+#pragma unroll 1
+    for (int o = 0; o < S::OWN; ++o) {
+      const int item = wk * S::OWN + o, block = item / 2, g = item & 1;
+      f32x16 a;
+#pragma unroll 1
+      for (int share = 0; share < 4; ++share) {  // (as the smallest fp32 tiles have it)
+        f32x16 q;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) q[v] = 0.f;
+        again((wm * S::NM + block / S::NN) * 32, (wn * S::NN + block % S::NN) * 32, share, q);
+        a = share ? a + q : q;
+      }
+      const f32x4 lo = g ? quad(a, 1) : quad(a, 0), hi = g ? quad(a, 3) : quad(a, 2);
+#pragma unroll
+      for (int k = 0; k < S::OWN; ++k)
+        if (k == o) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            if (odd(out.lo[k][c])) out.lo[k][c] = lo[c];
+            if (odd(out.hi[k][c])) out.hi[k][c] = hi[c];
+          }
+        }
     }
   }
 };

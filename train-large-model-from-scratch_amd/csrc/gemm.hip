@@ -1113,7 +1113,7 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   const long long tiles = row_slots(a.R, a.E, ROW_TILE) * ((a.N + CfgMain::BN - 1) / CfgMain::BN);
   const bool small = forced_row_tile > RING_TILE ? forced_row_tile == CfgHalf::BM
                                                  : 2 * tiles < moe_compute_units() &&
-                                                       expected_tiles(a, CfgHalf::BM) * a.n_tiles <= moe_compute_units();
+                                                       moe_expected_tiles(a.R, a.E, CfgHalf::BM) * a.n_tiles <= moe_compute_units();
   if (small)
     return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK>, attr_done[0], a,
                                  a.n_tiles * row_slots(a.R, a.E, CfgHalf::BM), s);

@@ -45,12 +45,5 @@ __device__ __forceinline__ void swiglu_bwd(float dact, float g, float u, float& 
   dot += du * u;
 }
 
-// Tiles of bm rows that R rows of E experts come to where a router deals them: half a tile an expert more than R / bm, and one
-// each where its rows do not fill one.
-inline double expected_tiles(const GemmArgs& a, int bm) {
-  const double x = (double)a.R / a.E / bm;
-  return a.E * (x <= 0.6 ? 1 : x >= 1 ? x + 0.5 : 1 + (x - 0.6) * 1.25);
-}
-
 // Takes a row-ragged launch of few tiles (csrc/row_ring.hip): false where it does not.
 bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, bool forced, hipStream_t s, int* rc);

@@ -9,6 +9,13 @@ void moe_observe(const char* name, int after);
 // Compute units of the current GPU (asked of the runtime once).
 int moe_compute_units();
 
+// Tiles of bm rows that R rows of E experts come to where a router deals them: half a tile an expert more than R / bm, and one
+// each where its rows do not fill one.
+inline double moe_expected_tiles(int64_t R, int64_t E, int bm) {
+  const double x = (double)R / E / bm;
+  return E * (x <= 0.6 ? 1 : x >= 1 ? x + 0.5 : 1 + (x - 0.6) * 1.25);
+}
+
 // Gate gradients from the dgrad-down kernel's block sums, softmax Jacobian and scatter to the logits in
 // one kernel (route.hip).  dlogits [T, ld] with columns E..ld-1 zero; dsel fp32 [T*k] (may be NULL): the k
 // nonzero entries per token, rounded to dlogits' type.

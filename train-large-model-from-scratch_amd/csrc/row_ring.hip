@@ -120,8 +120,8 @@ bool choose(const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
   if (launch<MODE, BLK, 1>(a, slots, forced, s, rc)) return true;
   constexpr int COLS = RingTile<MODE, 1, 4>::BNC;
   const double cols = (a.N + COLS - 1) / COLS, k = (double)a.K * (MODE == DGRAD_GATEUP ? 2 : 1);
-  if (expected_tiles(a, 64) * cols <= slots) return launch<MODE, BLK, 1>(a, slots, true, s, rc);
-  const double half = expected_tiles(a, 128) * cols;
+  if (moe_expected_tiles(a.R, a.E, 64) * cols <= slots) return launch<MODE, BLK, 1>(a, slots, true, s, rc);
+  const double half = moe_expected_tiles(a.R, a.E, 128) * cols;
   if ((half <= slots && k <= (MODE == GATEUP ? 640 : 1280)) || (half <= 2 * slots && k <= 320 && MODE != DGRAD_GATEUP))
     return launch<MODE, BLK, 2>(a, slots, true, s, rc);
   if constexpr (MODE == DOWN || MODE == DGRAD_GATEUP)
