@@ -196,8 +196,8 @@ int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const uint16_t* 
  * their two input gradients) run on 256-row tiles, what is left after whole rounds of them on
  * 128-row tiles where that is shorter, and launches of few tiles on narrower 128-row or on 64-row tiles
  * (up to 128 experts, g and u blocked or not kept) throughout.
- * moe_gemm_force_row_tile(64, 128 or 256) forces one of them for every later
- * call (64: where there is such a tile), 0 restores the automatic choice; the previous setting is returned.  Process-wide and not
+ * moe_gemm_force_row_tile(64, 128 or 256) forces one of them for every later call, 1 the 64-row
+ * tiles' kernel with 128 rows a tile (64 and 1: where there is such a tile), 0 restores the automatic choice; the previous setting is returned.  Process-wide and not
  * synchronised with calls in flight on other host threads.  No result depends on the choice:
  * every output element is accumulated over k in the same order on all tile heights, so all
  * outputs (the gate gradients' block sums included) are the same bits either way. */

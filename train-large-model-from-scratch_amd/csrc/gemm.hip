@@ -1097,7 +1097,7 @@ long long row_slots(int64_t R, int64_t E, int tile) { return (R + tile - 1) / ti
 // synchronisation).  With fewer tiles than half the compute units, by the bound on their number, every one of them can be
 // halved, as long as the halves are one round (gate/up has twice the tiles for its columns; 10842 rows of 8 experts, 2496 <-> 320, 266
 // halves 69 us, whole tiles and quarters 50; 13653 of 12, 1984 <-> 192, 225 halves, 34 and 35.5); what csrc/row_ring.hip takes is done there.  `forced_row_tile` (0: automatic) is a test hook.
-constexpr int RING_TILE = 64;
+constexpr int RING_TILE = 64, RING_TALL = 1;  // (1: the ring's tiles of 128 rows)
 int forced_row_tile = 0;
 
 // A row-ragged launch with `cols` output columns to a tile.
@@ -1106,8 +1106,8 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   static_assert(lds_bytes<MODE, CfgHalf>() <= lds_bytes<MODE, CfgMain>(), "both row tiles fit");
   static bool attr_done[2][MOE_MAX_DEVICES];  // per GPU and instantiation
   int rc = 0;
-  if ((!forced_row_tile || forced_row_tile == RING_TILE) &&
-      moe_ring_rows((Mode)MODE, BLK, a, forced_row_tile == RING_TILE, s, &rc))
+  if (forced_row_tile <= RING_TILE &&
+      moe_ring_rows((Mode)MODE, BLK, a, forced_row_tile == RING_TALL ? 128 : forced_row_tile, s, &rc))
     return rc;
   a.n_tiles = (a.N + cols - 1) / cols;
   const long long tiles = row_slots(a.R, a.E, ROW_TILE) * ((a.N + CfgMain::BN - 1) / CfgMain::BN);
@@ -1188,12 +1188,12 @@ extern "C" int moe_gemm_down_fwd(const uint16_t* act, const uint16_t* w2, const 
   return launch_rows<DOWN>(a, CfgMain::BN, (hipStream_t)stream);
 }
 
-// Test hook: 0 lets every row-ragged launch choose its row-tile height (the default), 64, 128 or 256 forces it (64: of
-// the launches that have such tiles).  Process-wide and not synchronised: for tests that want every shape on every
+// Test hook: 0 lets every row-ragged launch choose its row-tile height (the default), 64, 128 or 256 forces it, 1
+// the ring's tiles of 128 rows (64 and 1: of the launches that have such tiles).  Process-wide and not synchronised: for tests that want every shape on every
 // tile configuration, not for production callers.  Returns the previous setting.
 extern "C" int moe_gemm_force_row_tile(int rows) {
   const int before = forced_row_tile;
-  if (rows == 0 || rows == RING_TILE || rows == CfgHalf::BM || rows == CfgMain::BM) forced_row_tile = rows;
+  if (rows == 0 || rows == RING_TILE || rows == RING_TALL || rows == CfgHalf::BM || rows == CfgMain::BM) forced_row_tile = rows;
   return before;
 }
 

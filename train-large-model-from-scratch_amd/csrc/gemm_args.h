@@ -45,5 +45,6 @@ __device__ __forceinline__ void swiglu_bwd(float dact, float g, float u, float& 
   dot += du * u;
 }
 
-// Takes a row-ragged launch of few tiles (csrc/row_ring.hip): false where it does not.
-bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, bool forced, hipStream_t s, int* rc);
+// Takes a row-ragged launch of few tiles (csrc/row_ring.hip): false where it does not.  `forced`: any launch, in tiles of 64 or
+// 128 rows (0: its own choice).
+bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, int forced, hipStream_t s, int* rc);

@@ -115,9 +115,10 @@ bool small_tiles_pay(const GemmArgs& a) {
 // elsewhere, 7 % faster in the mean, 34 of them slower by more than 3 %.  Whole passes of 96 more layers: 0.99 to 1.16 times as
 // fast.  What it gets wrong: 15407 rows of 96, 576 <-> 192, gate/up 23.8 -> 26.6; 30411 of 12, 1408 <-> 320, down, not taken.
 template <int MODE, bool BLK>
-bool choose(const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
+bool choose(const GemmArgs& a, int forced, hipStream_t s, int* rc) {
   const long long slots = 2ll * moe_compute_units();
-  if (launch<MODE, BLK, 1>(a, slots, forced, s, rc)) return true;
+  if (forced == 128) return launch<MODE, BLK, 2>(a, slots, true, s, rc);
+  if (launch<MODE, BLK, 1>(a, slots, forced != 0, s, rc)) return true;
   constexpr int COLS = RingTile<MODE, 1, 4>::BNC;
   const double cols = (a.N + COLS - 1) / COLS, k = (double)a.K * (MODE == DGRAD_GATEUP ? 2 : 1);
   if (moe_expected_tiles(a.R, a.E, 64) * cols <= slots) return launch<MODE, BLK, 1>(a, slots, true, s, rc);
@@ -131,7 +132,7 @@ bool choose(const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
 
 }  // namespace
 
-bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, bool forced, hipStream_t s, int* rc) {
+bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, int forced, hipStream_t s, int* rc) {
   if (a.E > MAX_E) return false;
   switch (mode) {
     case GATEUP:
