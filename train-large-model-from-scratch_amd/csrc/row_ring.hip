@@ -58,12 +58,18 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
   ring_tile<MODE, BLK, FM, 4>(p, ring, e, first, row_end, in % nt * BM, in / nt * O::BNC);
 }
 
+// Tiles side by side.  (dgrad-down's sums cover the columns in steps of 256)
+template <int MODE>
+int columns(int N) {
+  constexpr int BNC = RingTile<MODE, 1, 4>::BNC;
+  return MODE == DGRAD_DOWN ? (N + 255) / 256 * 2 : (N + BNC - 1) / BNC;
+}
+
 // Launches of at most `most` tiles (by the bound that R and E give), or of any number.
 template <int MODE, bool BLK, int FM>
 bool launch(GemmArgs a, long long most, bool any, hipStream_t s, int* rc) {
   using O = RingTile<MODE, FM, 4>;
-  // (dgrad-down's sums cover the columns in steps of 256)
-  a.n_tiles = MODE == DGRAD_DOWN ? (a.N + 255) / 256 * 2 : (a.N + O::BNC - 1) / O::BNC;
+  a.n_tiles = columns<MODE>(a.N);
   const long long tiles = ((a.R + O::BM - 1) / O::BM + (long long)a.E) * a.n_tiles;
   if (tiles > (any ? 0x7fffff00ll : most)) return false;
   const auto kern = ring_rows_kernel<MODE, BLK, FM>;
@@ -106,27 +112,32 @@ bool small_tiles_pay(const GemmArgs& a) {
 // Down and dgrad-gate/up, whose epilogues are short, have tiles of 128 rows and two stages for what is too much for 64
 // rows (tiles of 128 rows; down and dgrad-gate/up us: 320 12.4, 19.8 -> 11.2, 17.6; 440 14.5, 22.6 -> 12.5, 19.6; 576
 // 19.0, 29.2 -> 19.5, 31.8).
-// The bound has a tile too many for every other expert.  Past it, launches that are expected to fit are taken all the same, and
-// in tiles of 128 rows where the contraction is at most 1280 (gate/up 640: longer ones are bound by LDS, where the larger kernels'
-// tiles of 128 x 256 have less traffic; 1024: 18.6 -> 16.8 us by itself, but a forward pass of 2048 tokens of 8 experts 45.3 -> 46.2),
-// or at most 320 and two rounds: there a tile's end is as long as its contraction, and two workgroups to a compute unit cover
-// each other's.  Before -> this, us: 6492 rows of 8 experts, 256 <-> 576, gate/up 16.2 -> 9.8; 18388 of 64, 576 <-> 192, down 18.4 ->
-// 12.1; 3784 of 16, 384 <-> 896, dgrad-down 16.3 -> 12.0 (in tiles of 64).  Of 2000 launches of 500 drawn layers 220 go
-// elsewhere, 7 % faster in the mean, 34 of them slower by more than 3 %.  Whole passes of 96 more layers: 0.99 to 1.16 times as
-// fast.  What it gets wrong: 15407 rows of 96, 576 <-> 192, gate/up 23.8 -> 26.6; 30411 of 12, 1408 <-> 320, down, not taken.
+// The bound has a tile too many for every other expert.  Past it, gate/up and dgrad-down are taken all the same where their tiles
+// are expected to fit (with room for a twentieth more: unless a router deals evenly there are more, and a second round of a few tiles
+// takes as long as the first); so are, where experts have 64 rows, launches in tiles of 128 whose contraction is at most 1280, gate/up's,
+// whose larger kernels have less LDS traffic in tiles of 128 x 256, 640 (1024: 18.6 -> 16.8 us by itself, but a forward pass of 2048
+// tokens of 8 experts 45.3 -> 46.2), dgrad-down's, whose narrow results larger tiles pad no more, 768 (17836 rows of 12, 1024 <-> 192,
+// not taken, 24.9 -> 26.5), or at most 320 and two rounds: there a tile's end is as long as its contraction, and two workgroups to a
+// compute unit cover each other's.  With fewer rows an expert the rule behind is the better one (240 rows of 64, 320 <-> 1664,
+// dgrad-down, 8.0 -> 11.1).  Before -> this, us: 6492 rows of 8 experts, 256 <-> 576, gate/up 16.2 -> 9.8; 18388 of 64, 576 <->
+// 192, down 18.4 -> 12.1; 3784 of 16, 384 <-> 896, dgrad-down 16.3 -> 12.0 (in tiles of 64).  Of 472 launches of 300 drawn layers
+// with a launch past the bound, weights cold, gate/up take 0.94, down 0.955, dgrad-down 0.96 and dgrad-gate/up 0.985 of the time in the
+// mean, one in thirty is slower by more than 3 % (up to 1.10, by heavy experts).
 template <int MODE, bool BLK>
 bool choose(const GemmArgs& a, int forced, hipStream_t s, int* rc) {
   const long long slots = 2ll * moe_compute_units();
   if (forced == 128) return launch<MODE, BLK, 2>(a, slots, true, s, rc);
   if (launch<MODE, BLK, 1>(a, slots, forced != 0, s, rc)) return true;
-  constexpr int COLS = RingTile<MODE, 1, 4>::BNC;
-  const double cols = (a.N + COLS - 1) / COLS, k = (double)a.K * (MODE == DGRAD_GATEUP ? 2 : 1);
-  if (moe_expected_tiles(a.R, a.E, 64) * cols <= slots) return launch<MODE, BLK, 1>(a, slots, true, s, rc);
-  const double half = moe_expected_tiles(a.R, a.E, 128) * cols;
-  if ((half <= slots && k <= (MODE == GATEUP ? 640 : 1280)) || (half <= 2 * slots && k <= 320 && MODE != DGRAD_GATEUP))
+  constexpr bool FUSED = MODE == GATEUP || MODE == DGRAD_DOWN;
+  if (!FUSED && launch<MODE, BLK, 2>(a, slots, false, s, rc)) return true;
+  constexpr int LONGEST = MODE == GATEUP ? 640 : MODE == DGRAD_DOWN ? 768 : 1280;
+  const double cols = columns<MODE>(a.N), k = (double)a.K * (MODE == DGRAD_GATEUP ? 2 : 1);
+  const double most = 0.95 * slots;
+  if (FUSED && moe_expected_tiles(a.R, a.E, 64) * cols <= most) return launch<MODE, BLK, 1>(a, slots, true, s, rc);
+  const double tall = moe_expected_tiles(a.R, a.E, 128) * cols;
+  if (a.R >= 64ll * a.E &&
+      ((tall <= most && k <= LONGEST) || (tall <= 2 * most && k <= 320 && MODE != DGRAD_GATEUP)))
     return launch<MODE, BLK, 2>(a, slots, true, s, rc);
-  if constexpr (MODE == DOWN || MODE == DGRAD_GATEUP)
-    if (launch<MODE, BLK, 2>(a, slots, false, s, rc)) return true;
   return small_tiles_pay<MODE>(a) && launch<MODE, BLK, 1>(a, slots, true, s, rc);
 }
 
