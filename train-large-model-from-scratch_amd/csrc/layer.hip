@@ -226,8 +226,8 @@ struct FwdScratch {
 // of an expert, another 4.4 with fp32 results.  (64 tiles, Zipf: a step of 8192 tokens 406 -> 362 us; 216 tiles: 401 -> 395; 512
 // tiles, 6 rounds against 8: 494 -> 514, not taken.  2006 tokens of 8 experts, 3136 <-> 704, 312 tiles, 6 rounds against 4.7: 326 -> 289;
 // 3959 tokens, 4 of 128 by Zipf's shares, 384 <-> 448, 6 against 6, 378 -> 223; 3390 of 64, 360 <-> 768, 5 against 4.5, 301 ->
-// 227.  150 drawn layers of one to eight rounds: 68 taken, steps 1.03 times as fast in the mean, four slower by 2 to 5 % (969
-// tokens, 6 of 128, 768 <-> 384, 9 against 9: 316 -> 331).)
+// 227.  Of 250 drawn layers of one to four rounds 131 are taken, their steps 1.13 times as fast in the mean where all three gradients
+// are wanted, 1.03 to 1.08 where one or two are, for which the rounds are counted as if all were; four are slower by 2 to 3 %.)
 constexpr int64_t WTILE = 256;
 constexpr int64_t MULTI_ROUNDS = 4;
 bool wgrad_multi(int64_t E, int64_t M, int64_t N, int64_t R) {
