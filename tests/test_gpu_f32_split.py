@@ -253,3 +253,21 @@ def test_at_the_lines_of_the_rule(pkg, lib, forced, E, R, N, K):
     size = torch.cat([p @ w.double().abs().t() for p, w in zip(sizes, b)])
     # (either tile: at most a rounding for every product of the contraction, and the parts that the split leaves out)
     assert ((got.cpu().double() - ref).abs() <= (K + 1) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("E,R,M,N", [
+    (8, 1792, 1024, 1024),   # weight gradients: the fewest rows an expert that split tiles take
+    (8, 1791, 1024, 1024),   # ... a row less
+    (4, 3584, 1024, 1028),   # columns past the tiles
+    (4, 3584, 1024, 960),    # fewer tiles than compute units
+])
+def test_at_the_lines_of_the_weight_gradients(pkg, lib, forced, E, R, M, N):
+    forced(0)
+    g = torch.Generator().manual_seed(R + N)
+    counts = [R // E + (e < R % E) for e in range(E)]
+    a, b = torch.randn(R, M, generator=g), torch.randn(R, N, generator=g)
+    got = pkg.ops.f32_gemm_wgrad(a.cuda(), b.cuda(), _offs(counts).cuda(), E)
+    parts = list(zip(a.double().split(counts), b.double().split(counts)))
+    ref = torch.stack([p.t() @ q for p, q in parts])
+    size = torch.stack([p.abs().t() @ q.abs() for p, q in parts])
+    assert ((got.cpu().double() - ref).abs() <= (max(counts) + 1) * 2.0 ** -24 * size).all()
