@@ -1,0 +1,62 @@
+"""Tiles that a workgroup of the tiled products does one after the other, each handing over to the next one's first k-tiles: odd
+and even numbers of k-tiles, one and two of them, ends past the contraction, tiles without rows for half of the waves, empty
+experts between others."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def experts(offs):
+    o = offs.tolist()
+    return [(e, slice(o[e], o[e + 1])) for e in range(len(o) - 1)]
+
+
+@pytest.mark.parametrize("K", [64, 128, 136, 192, 328])
+def test_rows(pkg, lib, K):
+    print("rows", K, flush=True)
+    ops, g = pkg.ops, torch.Generator(device="cuda").manual_seed(K)
+    counts = ([300, 129, 1, 0, 256, 65] * 47)[:280]  # 370 row tiles, two or four column tiles: at least three a workgroup
+    E, R, N = len(counts), sum(counts), 512
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    x, x2, gate, up, down, dw1, dw3 = r(R, K), r(R, K), r(E, N, K), r(E, N, K), r(E, N, K), r(E, K, N), r(E, K, N)
+
+    def products(height):
+        force = ops._lib.load().cdll.moe_gemm_force_row_tile
+        try:
+            force(height)
+            gu, a = ops.gemm_gateup_blocked(x, gate, up, offs)
+            d = ops.gemm_dgrad_down_blocked(x2, dw1, gu, offs, dgate_blocks=True)
+            return [a, ops.gemm_gateup(x, gate, up, offs, False)[2], ops.gemm_down(x, down, offs), *d,
+                    ops.gemm_dgrad_gateup(x, x2, dw1, dw3, offs)]
+        finally:
+            force(0)
+
+    want = products(64)  # (a kernel of its own, a tile to a workgroup)
+    for height in (256, 128):
+        for n, (a, b) in enumerate(zip(products(height), want)):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (height, n)
+    # a rounding to bf16, and sums of K products of unit variance in fp32 on both sides
+    ref = torch.cat([x[s].float() @ down[e].float().T for e, s in experts(offs)])
+    assert bool(((want[2].float() - ref).abs() <= ref.abs() * 2.0 ** -8 + 2.0 ** -22 * K * K ** 0.5).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts", [
+    [64, 65, 0, 1, 128, 129, 0, 0, 200, 63, 256, 300] * 2,  # 0 to 5 k-tiles in every order of odd and even
+    [64] * 24,                                              # one each
+    [130] * 23 + [1000],
+])
+def test_weight_gradients(pkg, lib, counts, dtype):
+    print("weight gradients", counts, dtype, flush=True)
+    ops, g = pkg.ops, torch.Generator(device="cuda").manual_seed(len(counts))
+    E, R, M, N = len(counts), sum(counts), 1016, 1280
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    a, b = (torch.randn(R, n, generator=g, device="cuda").to(torch.bfloat16) for n in (M, N))
+    got = ops.gemm_wgrad(a, b, offs, E, dtype)
+    K = max(counts)
+    for e, s in experts(offs):
+        ref = a[s].float().T @ b[s].float()
+        bound = ref.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0) + 2.0 ** -22 * K * K ** 0.5
+        assert bool(((got[e].float() - ref).abs() <= bound).all()), (e, counts[e])

@@ -364,22 +364,29 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   constexpr int CPRO = WTNC * OSZ / 16;  // 16-byte chunks per strip row
   constexpr int RPI = 64 / CPRO;         // rows covered by one wave-wide 16-byte access
   static_assert(64 % CPRO == 0 && 32 % RPI == 0, "strip shape");
-  // Where they fit, the strips take the second LDS stage only (half of the waves in its A
-  // part, half in its B part): the first stage is then free to receive the next tile's first
-  // k-tile while the results are still being written out.
-  // (the SwiGLU-backward epilogue needs the staging registers' room for its g/u rows: it sends
-  // the request during its last strip, when that room is free, and stages nothing -- moving the
-  // k-tile on into LDS at the end of that epilogue was measured 3 % slower)
+  // Where they fit, the strips take one LDS stage only (half of the waves in its A part, half in its B part): the
+  // one that the tile's last k-tile was read from.  The k-tiles of the next tile then follow this one's without a
+  // break: its first is asked for in the last but one iteration and moves to the other stage in the last one, which
+  // asks for its second.  A unit answers its loads and stores in order: loads sent between the stores of the strips
+  // wait behind them, and the stores behind the loads' trip to memory (65536 rows of 64 experts, 2048 <-> 1024, cycles
+  // of an epilogue with the next tile's loads in it and without: gate/up 11300, 6200; down 8600, 4000; weight
+  // gradients 9300, 4400, in fp32 17400, 8100; half of it comes back as a slower start of the next loop, and power takes
+  // its share: gate/up 528 -> 518 us, down 282 -> 272, weight gradients 786 -> 777, in fp32 925 -> 893; 32768 rows of 128,
+  // 1024 <-> 256: down 36.4 -> 35.1, dgrad-gate/up 53.4 -> 51.9).
+  // (the SwiGLU-backward epilogue needs the staging registers' room for its g/u rows: it sends the request during
+  // its last strip, when that room is free)
   constexpr bool EARLY_REQUEST = (MODE != DGRAD_DOWN);
   constexpr int HALF_WAVES = Cfg::WM * Cfg::WN / 2;
-  constexpr bool STAGE_EARLY = EARLY_REQUEST &&
-                               NSTRIP * SBYTES * HALF_WAVES <= StA::LDS_ELEMS * 2 &&
-                               NSTRIP * SBYTES * HALF_WAVES <= StB::LDS_ELEMS * 2;
+  constexpr bool STREAM = EARLY_REQUEST &&
+                          NSTRIP * SBYTES * HALF_WAVES <= StA::LDS_ELEMS * 2 &&
+                          NSTRIP * SBYTES * HALF_WAVES <= StB::LDS_ELEMS * 2;
   static_assert(NSTRIP * SBYTES * Cfg::WM * Cfg::WN <= lds_bytes<MODE, Cfg>(), "strips fit in the stages");
-  char* strip = STAGE_EARLY
-                    ? reinterpret_cast<char*>(wv < HALF_WAVES ? sA + StA::LDS_ELEMS : sB + StB::LDS_ELEMS) +
-                          (wv % HALF_WAVES) * (NSTRIP * SBYTES)
-                    : reinterpret_cast<char*>(smem) + wv * (NSTRIP * SBYTES);
+  const auto strip_in = [&](int stage) {
+    return STREAM ? reinterpret_cast<char*>(wv < HALF_WAVES ? sA + stage * StA::LDS_ELEMS : sB + stage * StB::LDS_ELEMS) +
+                        (wv % HALF_WAVES) * (NSTRIP * SBYTES)
+                  : reinterpret_cast<char*>(smem) + wv * (NSTRIP * SBYTES);
+  };
+  char* strip = strip_in(0);
   const int ldc = p.ld_c ? p.ld_c : p.N;  // outputs
   const int ldx = p.N;                    // epilogue inputs (g, u)
   // The accumulators of a strip are cleared for the next tile as soon as they are in LDS: the
@@ -403,9 +410,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   auto gu_block = [&](const void* base, const Tile& t, int rb, int cb, int ln) {
     return (char*)base + (((long long)t.block0 + rb) * n_cb + cb) * GU_BLOCK_BYTES + ln * 16;
   };
-  // `halfway` runs once, after the second of the FM strips; `last_rows_in` once the SwiGLU-backward
-  // epilogue has taken the last g/u rows out of their registers
-  auto epilogue = [&](const Tile& t, auto&& halfway, auto&& last_rows_in) {
+  // `last_rows_in` runs once the SwiGLU-backward epilogue has taken the last g/u rows out of their registers
+  auto epilogue = [&](const Tile& t, auto&& last_rows_in) {
     // Every per-lane address of the epilogue is derived from this copy of the lane index, which
     // the empty asm makes opaque: the compiler then recomputes them here, a handful of integer
     // operations per tile, instead of hoisting them out of the tile loop and holding a dozen
@@ -643,7 +649,6 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
         zero_row(i);
         store_rows(0, i, C0);
       }
-      if (i == (FM > 1 ? 1 : 0)) halfway();
     }
   };
 
@@ -663,7 +668,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   Tile cur;
   if (t_next >= t_hi || !locate(tile_at(t_next), cur)) return;
   request_first(cur);
-  bool staged = false;  // k-tile 0 of `cur` already sits in LDS stage 0, k-tile 1 is on its way
+  bool staged = false;  // k-tile 0 of `cur` already sits in LDS stage `s0`, k-tile 1 is on its way
+  int s0 = 0;           // the LDS stage of the tile's first k-tile; they alternate from there
 #pragma unroll
   for (int i = 0; i < FM; ++i) zero_row(i);  // later tiles find them cleared by the epilogue
   for (;;) {
@@ -690,21 +696,27 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     t_next += t_step;
     const bool more = t_next < t_hi && locate(tile_at(t_next), nxt);
     const int nkt = cur.nkt;
+    const bool stream = STREAM && more && nkt > 1 && nxt.nkt > 0;  // the k-tiles of the next tile follow this one's
+    // the k-tile two behind kt
+    auto request_ahead = [&](int kt) {
+      if (kt + 2 < nkt) load_tile(cur, kt + 2, stg);
+      else if (stream && kt + 2 - nkt < nxt.nkt) load_tile(nxt, kt + 2 - nkt, stg);
+    };
     if (nkt > 0) {
       if (!staged) {
+        s0 = 0;
         store_tile(stg, 0);
         if (1 < nkt) load_tile(cur, 1, stg);
         lds_barrier();
       }
-      if (!idle) f_read_all(0, 0, fr[0]);
+      if (!idle) f_read_all(s0, 0, fr[0]);
     }
     int kt = 0;
     if (idle) {
       for (; kt < nkt; ++kt) {
-        const bool has1 = kt + 1 < nkt, has2 = kt + 2 < nkt;
-        if (has1) {
-          store_tile(stg, (kt & 1) ^ 1);
-          if (has2) load_tile(cur, kt + 2, stg);
+        if (kt + 1 < nkt || stream) {
+          store_tile(stg, ((kt + s0) & 1) ^ 1);
+          request_ahead(kt);
           lds_barrier();
         }
       }
@@ -717,46 +729,36 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     while (kt < nkt) {
       int steady_end = nkt - 2;
       if (cur.need_mask) steady_end = (NSEG == 2 && kt + 2 < cur.kt_per_seg ? cur.kt_per_seg : nkt) - 3;
-      if (!(kt & 1)) {
+      if (!((kt + s0) & 1)) {
         for (; kt + 1 < steady_end; kt += 2) {
           body(integral_constant<int, 0>{}, cur, kt);
           body(integral_constant<int, 1>{}, cur, kt + 1);
         }
       }
-      const int buf = kt & 1;
-      const bool has1 = kt + 1 < nkt, has2 = kt + 2 < nkt;
+      const int buf = (kt + s0) & 1;
+      const bool has1 = kt + 1 < nkt;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         if (ks + 1 < KS) f_read_all(buf, ks + 1, fr[(ks + 1) & 1]);
-        if (ks == 0 && has1) {
+        if (ks == 0 && (has1 || stream)) {
           store_tile(stg, buf ^ 1);
-          if (has2) load_tile(cur, kt + 2, stg);
+          request_ahead(kt);
         }
-        if (ks == KS - 1 && has1) {
+        if (ks == KS - 1 && (has1 || stream)) {
           lds_barrier();
-          f_read_all(buf ^ 1, 0, fr[0]);
+          if (has1) f_read_all(buf ^ 1, 0, fr[0]);
         }
         mma_all(fr[ks & 1]);
       }
       ++kt;
     }
-    // the next tile's first k-tiles travel while this tile's results are written out
-    if (EARLY_REQUEST && more) request_first(nxt);
-    lds_barrier();  // every wave is done reading the operand stages
-    // Half-way through the epilogue the next tile's first k-tile has arrived: it moves on
-    // into LDS stage 0 (idle: the strips live in stage 1) and its registers fetch the second
-    // k-tile, so that the next main loop starts with both in place instead of waiting for
-    // a load it has only just issued.
-    staged = false;
-    auto stage_next = [&]() {
-      if constexpr (STAGE_EARLY) {
-        if (more && nxt.nkt > 0) {
-          store_tile(stg, 0);
-          if (1 < nxt.nkt) load_tile(nxt, 1, stg);
-          staged = true;
-        }
-      }
-    };
+    if (!stream) {
+      if (EARLY_REQUEST && more) request_first(nxt);
+      lds_barrier();  // every wave is done reading the operand stages
+    }
+    if (STREAM && nkt > 0) strip = strip_in((s0 + nkt - 1) & 1);
+    s0 = (s0 + nkt) & 1;
+    staged = stream;
     // Where the epilogue needs the staging registers' room for most of its length, the request
     // goes out as soon as that room is free: during the last of its strips.
     bool requested = EARLY_REQUEST;
@@ -766,8 +768,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
         requested = true;
       }
     };
-    if (idle) stage_next();
-    else epilogue(cur, stage_next, late_request);
+    if (!idle) epilogue(cur, late_request);
     if (!more) break;
     if (!requested) request_first(nxt);
     lds_barrier();  // every wave is done with its strip, and stage 0 is complete if staged
