@@ -466,6 +466,10 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
                            pack_bf16x2(bf16lo(v[2]) + bf16lo(o[2]), bf16hi(v[2]) + bf16hi(o[2])),
                            pack_bf16x2(bf16lo(v[3]) + bf16lo(o[3]), bf16hi(v[3]) + bf16hi(o[3]))};
             }
+          } else if (MODE == WGRAD && p.streaming) {
+            asm volatile("" ::: "memory");  // (without the two fences this store and the next become one, an ordinary one)
+            __builtin_nontemporal_store(v, dst);
+            asm volatile("" ::: "memory");
           } else {
             *dst = v;
           }
@@ -1126,6 +1130,13 @@ template <typename OutT>
 int launch_wgrad(GemmArgs& a, hipStream_t s) {
   a.n_tiles = (a.N + CfgMain::BN - 1) / CfgMain::BN;
   a.m_slots = (a.M + CfgMain::BM - 1) / CfgMain::BM;
+  // Nothing here reads the results again.  With few rows an expert they come as fast as the operands do, and as streaming
+  // stores they leave the operands' lines in L2 alone.  Rows an expert and time, streaming over ordinary, three results in
+  // turn so that none is still cached: 64 experts of 2048 <-> 1024, bf16 and fp32: 256, 0.86 and 0.83; 512, 0.93 and 0.91; 768, 1.01 and 1.04;
+  // 1024, 1.00 and 1.01; 2048, 1.00 and 1.00.  128 of 1024 <-> 256, 128 to 512 rows 0.93 to 0.96 and 0.84 to 0.92; 16 of 4096 <-> 1536, 1024 rows
+  // 0.95 and 0.95; by Zipf's shares, 500 rows of 64 1.00 and 0.85.
+  // (as for wgrad_multi_kernel: rows of whole pieces of 64 bytes)
+  a.streaming = a.R <= 512ll * a.E && a.N * (int)sizeof(OutT) % 64 == 0;
   static bool attr_done[MOE_MAX_DEVICES];
   return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT>, attr_done, a, (long long)a.n_tiles * a.m_slots * a.E, s);
 }

@@ -27,6 +27,7 @@ struct GemmArgs {
   int ld_c;     // row stride of the outputs C0/C1 in elements when it is not N (0: N)
   int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
   int whole_only;  // row-ragged modes: no half tiles (test hook)
+  int streaming;   // WGRAD: results that replace what is there leave with streaming stores
 };
 
 // sigmoid from the two hardware transcendentals (v_exp_f32, v_rcp_f32; about 1 ulp each):

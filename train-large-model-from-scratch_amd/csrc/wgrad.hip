@@ -235,6 +235,11 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   const long long MN = (long long)st.M * st.N;
   char* out = partial ? (char*)(st.part + sg.slot * MN) : (char*)st.out + sg.e * MN * (wide ? 4 : 2);
   const bool add = !partial && st.accumulate;
+  // (streaming stores of whole pieces of 64 bytes, a row's in one instruction: the operands' lines stay in L2.  Ordinary ones ->
+  // these, whole steps, us: 75 tokens, 3 of 96 experts, 384 <-> 1152, 234 -> 193; 2753 tokens, 24 experts, 1520 <-> 576, fp32, 276 -> 218; of
+  // 100 drawn steps of one or two rounds of jobs none is slower.  With ends inside such a piece, which memory then reads
+  // first, some are: 958 rows of 64, 3128 <-> 1064, 756 -> 1028 in the tiled kernel)
+  const bool stream = !partial && !st.accumulate && st.N * (wide ? 4 : 2) % 64 == 0;
 #pragma unroll
   for (int i = 0; i < WFM; ++i) {
 #pragma unroll
@@ -244,33 +249,48 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
         *reinterpret_cast<f32x4*>(strip + (lane & 31) * SS + j * 32 + 8 * q + 4 * (lane >> 5)) =
             f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
     // (a wave's strip is its own: its LDS accesses are in order)
+    if (wide) {  // 16 lanes a row, 4 columns a lane
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {  // 8 lanes a row, 8 columns a lane
-      const int r = it * 8 + (lane >> 3), c = (lane & 7) * 8;
-      const int m = m0 + wm * (WBM / 2) + i * 32 + r, n = n0 + wn * (WBN / 2) + c;
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(strip + r * SS + c);
-      const f32x4 hi = *reinterpret_cast<const f32x4*>(strip + r * SS + c + 4);
-      if (m < st.M && n < st.N) {
-        Row8 v;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) v.v[x] = lo[x], v.v[4 + x] = hi[x];
-        const long long at = (long long)m * st.N + n;
-        if (wide) {
-          float* dst = reinterpret_cast<float*>(out) + at;
-          if (add) {
-            const Row8 o = load8(dst);
-#pragma unroll
-            for (int x = 0; x < 8; ++x) v.v[x] += o.v[x];
+      for (int it = 0; it < 8; ++it) {
+        const int r = it * 4 + (lane >> 4), c = (lane & 15) * 4;
+        const int m = m0 + wm * (WBM / 2) + i * 32 + r, n = n0 + wn * (WBN / 2) + c;
+        f32x4 v = *reinterpret_cast<const f32x4*>(strip + r * SS + c);
+        if (m < st.M && n < st.N) {
+          f32x4* dst = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) + (long long)m * st.N + n);
+          if (stream) {
+            asm volatile("" ::: "memory");
+            __builtin_nontemporal_store(v, dst);
+            asm volatile("" ::: "memory");
+          } else {
+            if (add) v += *dst;
+            *dst = v;
           }
-          store8(dst, v);
-        } else {
-          uint16_t* dst = reinterpret_cast<uint16_t*>(out) + at;
-          if (add) {  // (the product rounded first, as the tiled kernel adds it)
-            const Row8 o = load8(dst);
+        }
+      }
+    } else {
 #pragma unroll
-            for (int x = 0; x < 8; ++x) v.v[x] = bf16_to_f32(f32_to_bf16(v.v[x])) + o.v[x];
+      for (int it = 0; it < 4; ++it) {  // 8 lanes a row, 8 columns a lane
+        const int r = it * 8 + (lane >> 3), c = (lane & 7) * 8;
+        const int m = m0 + wm * (WBM / 2) + i * 32 + r, n = n0 + wn * (WBN / 2) + c;
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(strip + r * SS + c);
+        const f32x4 hi = *reinterpret_cast<const f32x4*>(strip + r * SS + c + 4);
+        if (m < st.M && n < st.N) {
+          Row8 v;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) v.v[x] = lo[x], v.v[4 + x] = hi[x];
+          uint16_t* dst = reinterpret_cast<uint16_t*>(out) + (long long)m * st.N + n;
+          if (stream) {
+            asm volatile("" ::: "memory");
+            store8_nt(dst, v);
+            asm volatile("" ::: "memory");
+          } else {
+            if (add) {  // (the product rounded first, as the tiled kernel adds it)
+              const Row8 o = load8(dst);
+#pragma unroll
+              for (int x = 0; x < 8; ++x) v.v[x] = bf16_to_f32(f32_to_bf16(v.v[x])) + o.v[x];
+            }
+            store8(dst, v);
           }
-          store8(dst, v);
         }
       }
     }
