@@ -373,12 +373,13 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   // gradients 9300, 4400, in fp32 17400, 8100; half of it comes back as a slower start of the next loop, and power takes
   // its share: gate/up 528 -> 518 us, down 282 -> 272, weight gradients 786 -> 777, in fp32 925 -> 893; 32768 rows of 128,
   // 1024 <-> 256: down 36.4 -> 35.1, dgrad-gate/up 53.4 -> 51.9).
-  // (the SwiGLU-backward epilogue needs the staging registers' room for its g/u rows: it sends the request during
-  // its last strip, when that room is free)
+  // (the SwiGLU-backward epilogue needs the staging registers' room for its g/u rows: the next tile's first k-tile
+  // moves to LDS all the same, and its second is asked for during the last strip, when that room is free.  With the first
+  // strip's g and u on their way behind the last products, dgrad-down of 131072 rows of 64 experts, 2048 <-> 1024, 610 -> 596 us;
+  // 65536 rows 333 -> 326; 32768 of 128, 1024 <-> 256, 44.7 -> 43.1; 30000 of 64, 512 <-> 1024, 71.4 -> 68.2)
   constexpr bool EARLY_REQUEST = (MODE != DGRAD_DOWN);
   constexpr int HALF_WAVES = Cfg::WM * Cfg::WN / 2;
-  constexpr bool STREAM = EARLY_REQUEST &&
-                          NSTRIP * SBYTES * HALF_WAVES <= StA::LDS_ELEMS * 2 &&
+  constexpr bool STREAM = NSTRIP * SBYTES * HALF_WAVES <= StA::LDS_ELEMS * 2 &&
                           NSTRIP * SBYTES * HALF_WAVES <= StB::LDS_ELEMS * 2;
   static_assert(NSTRIP * SBYTES * Cfg::WM * Cfg::WN <= lds_bytes<MODE, Cfg>(), "strips fit in the stages");
   const auto strip_in = [&](int stage) {
@@ -410,6 +411,24 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   auto gu_block = [&](const void* base, const Tile& t, int rb, int cb, int ln) {
     return (char*)base + (((long long)t.block0 + rb) * n_cb + cb) * GU_BLOCK_BYTES + ln * 16;
   };
+  // (BLK) the two 16-byte parts of g and of u for each of the strip's column blocks
+  struct BlkRegs {
+    u32x4 g[FNC][2], u[FNC][2];
+  };
+  auto request_block = [&](const Tile& t, int i, int j, BlkRegs& b, int ln) {
+    const int cb = (t.n0 + wn * WTNC + j * 32) / 32;
+    const u32x4 zero = u32x4{0, 0, 0, 0};
+    b.g[j][0] = b.g[j][1] = b.u[j][0] = b.u[j][1] = zero;
+    if (t.row0 + wm * WTM + i * 32 < t.row_end && cb < n_cb) {
+      const u32x4* rec = reinterpret_cast<const u32x4*>(gu_block(p.X0, t, wm * FM + i, cb, ln));
+      // (read exactly once: streamed past the L2 lines the operand panels live in)
+      b.g[j][0] = __builtin_nontemporal_load(rec + 0);
+      b.g[j][1] = __builtin_nontemporal_load(rec + 64);
+      b.u[j][0] = __builtin_nontemporal_load(rec + 128);
+      b.u[j][1] = __builtin_nontemporal_load(rec + 192);
+    }
+  };
+  BlkRegs blk_in;
   // `last_rows_in` runs once the SwiGLU-backward epilogue has taken the last g/u rows out of their registers
   auto epilogue = [&](const Tile& t, auto&& last_rows_in) {
     // Every per-lane address of the epilogue is derived from this copy of the lane index, which
@@ -504,31 +523,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
         *reinterpret_cast<u32x4*>(strip + 1 * SBYTES + rr * SSTRIDE + ch * 16) = rr_.u[it];
       }
     };
-    // (BLK) the two 16-byte parts of g and of u for each of the strip's column blocks
-    struct BlkRegs {
-      u32x4 g[FNC][2], u[FNC][2];
-    };
-    auto request_block = [&](int i, int j, BlkRegs& b) {
-      const int cb = (col_w0 + j * 32) / 32;
-      const u32x4 zero = u32x4{0, 0, 0, 0};
-      b.g[j][0] = b.g[j][1] = b.u[j][0] = b.u[j][1] = zero;
-      if (t.row0 + wm * WTM + i * 32 < t.row_end && cb < n_cb) {
-        const u32x4* rec = reinterpret_cast<const u32x4*>(gu_block(p.X0, t, wm * FM + i, cb, lane_e));
-        // (read exactly once: streamed past the L2 lines the operand panels live in)
-        b.g[j][0] = __builtin_nontemporal_load(rec + 0);
-        b.g[j][1] = __builtin_nontemporal_load(rec + 64);
-        b.u[j][0] = __builtin_nontemporal_load(rec + 128);
-        b.u[j][1] = __builtin_nontemporal_load(rec + 192);
-      }
-    };
     RowRegs rows_in;
-    BlkRegs blk_in;
-    if constexpr (MODE == DGRAD_DOWN && BLK) {
-#pragma unroll
-      for (int j = 0; j < FNC; ++j) request_block(0, j, blk_in);
-    } else if constexpr (MODE == DGRAD_DOWN) {
-      request_rows(0, rows_in);
-    }
+    if constexpr (MODE == DGRAD_DOWN && !BLK) request_rows(0, rows_in);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       if constexpr (MODE == GATEUP) {
@@ -597,7 +593,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
             asm volatile("" : "+v"(rowdot));
           }
           __builtin_amdgcn_sched_barrier(0);  // (the loads must not move up: their registers are in use)
-          if (i + 1 < FM) request_block(i + 1, j, blk_in);
+          if (i + 1 < FM) request_block(t, i + 1, j, blk_in, lane_e);
           __builtin_amdgcn_sched_barrier(0);
         }
         if (i + 1 == FM) last_rows_in();
@@ -659,9 +655,9 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   // ---- the tile loop
   // At the top of the loop the first k-tile of `cur` is already on its way into the staging
   // registers (requested before the previous tile's epilogue).
-  auto request_first = [&](const Tile& t) {
-    if (0 < t.nkt) {
-      load_tile(t, 0, stg);
+  auto request_k = [&](const Tile& t, int kt) {
+    if (kt < t.nkt) {
+      load_tile(t, kt, stg);
     } else {
       // (nothing will be read from the staging registers: say so, or they stay alive through the
       // epilogue on account of this path)
@@ -669,6 +665,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       for (int c = 0; c < NCH; ++c) asm volatile("" : "=v"(stg.v[c]));
     }
   };
+  auto request_first = [&](const Tile& t) { request_k(t, 0); };
   Tile cur;
   if (t_next >= t_hi || !locate(tile_at(t_next), cur)) return;
   request_first(cur);
@@ -704,7 +701,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     // the k-tile two behind kt
     auto request_ahead = [&](int kt) {
       if (kt + 2 < nkt) load_tile(cur, kt + 2, stg);
-      else if (stream && kt + 2 - nkt < nxt.nkt) load_tile(nxt, kt + 2 - nkt, stg);
+      else if (stream && kt + 2 - nkt < (EARLY_REQUEST ? nxt.nkt : 1)) load_tile(nxt, kt + 2 - nkt, stg);
     };
     if (nkt > 0) {
       if (!staged) {
@@ -730,15 +727,13 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     // columns past the end of a segment (to be cleared), take the loop around them: the same order of
     // events, conditions evaluated, no static schedule.  (Segments of 1416 and 568, 9999 rows of 12 experts, when any
     // tail sent every iteration there: gate/up 54.9 us, now 46.1; dgrad-gate/up 71.5, now 62.5.)
-    while (kt < nkt) {
-      int steady_end = nkt - 2;
-      if (cur.need_mask) steady_end = (NSEG == 2 && kt + 2 < cur.kt_per_seg ? cur.kt_per_seg : nkt) - 3;
-      if (!((kt + s0) & 1)) {
-        for (; kt + 1 < steady_end; kt += 2) {
-          body(integral_constant<int, 0>{}, cur, kt);
-          body(integral_constant<int, 1>{}, cur, kt + 1);
-        }
-      }
+    auto request_blocks = [&]() {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+#pragma unroll
+      for (int j = 0; j < FNC; ++j) request_block(cur, 0, j, blk_in, ln);
+    };
+    auto one = [&](int kt) {
       const int buf = (kt + s0) & 1;
       const bool has1 = kt + 1 < nkt;
 #pragma unroll
@@ -754,7 +749,46 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
         }
         mma_all(fr[ks & 1]);
       }
+    };
+    // The tile's last k-tile, behind whose products the first g and u are on their way, in the registers of the staging and
+    // of the second set of fragments.
+    auto last = [&](int kt) {
+      const int buf = (kt + s0) & 1;
+      if (stream) store_tile(stg, buf ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      request_blocks();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (ks > 0) f_read_all(buf, ks, fr[0]);
+        if (ks == KS - 1 && stream) lds_barrier();
+        mma_all(fr[0]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    constexpr bool PEEL = MODE == DGRAD_DOWN && BLK;
+    const int looped = PEEL ? nkt - 1 : nkt;
+    while (kt < looped) {
+      int steady_end = nkt - 2;
+      if (cur.need_mask) steady_end = (NSEG == 2 && kt + 2 < cur.kt_per_seg ? cur.kt_per_seg : nkt) - 3;
+      if (!((kt + s0) & 1)) {
+        for (; kt + 1 < steady_end; kt += 2) {
+          body(integral_constant<int, 0>{}, cur, kt);
+          body(integral_constant<int, 1>{}, cur, kt + 1);
+        }
+      }
+      one(kt);
       ++kt;
+    }
+    if constexpr (PEEL) {
+      if (kt < nkt) {
+        last(kt);
+      } else {  // (a wave without rows: it will not read them, or they stay alive on its account)
+#pragma unroll
+        for (int j = 0; j < FNC; ++j)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) asm volatile("" : "=v"(blk_in.g[j][h]), "=v"(blk_in.u[j][h]));
+      }
     }
     if (!stream) {
       if (EARLY_REQUEST && more) request_first(nxt);
@@ -766,15 +800,19 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     // Where the epilogue needs the staging registers' room for most of its length, the request
     // goes out as soon as that room is free: during the last of its strips.
     bool requested = EARLY_REQUEST;
+    auto request_next = [&]() {
+      if (!stream) request_first(nxt);
+      else request_k(nxt, 1);
+    };
     auto late_request = [&]() {
       if constexpr (!EARLY_REQUEST) {
-        if (more) request_first(nxt);
+        if (more) request_next();
         requested = true;
       }
     };
     if (!idle) epilogue(cur, late_request);
     if (!more) break;
-    if (!requested) request_first(nxt);
+    if (!requested) request_next();
     lds_barrier();  // every wave is done with its strip, and stage 0 is complete if staged
     cur = nxt;
   }
