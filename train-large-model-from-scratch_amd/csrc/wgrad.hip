@@ -33,8 +33,10 @@ struct MultiArgs {
   Stack router;           // one "expert" of T rows, cut into r_slices slices of r_rows
   const int32_t* offs;
   int E, L, n_stacks, tiles;   // tiles: of all stacks together
+  int many;                    // experts of more rows than this come first
   int T, r_rows, r_slices;
-  int each, e_each, r_each;  // tiles of a segment to an XCD, its jobs of all segments, its router jobs (which come last)
+  int each, e_each, r_each;  // tiles of a segment to an XCD, its jobs of all segments, its router jobs
+  int r_first;               // the router's jobs come first, or last
   float per_each, r_per_tiles;
 };
 // n / d of a wave-uniform n, 1 / d given (exact: n is far below 2^23)
@@ -44,7 +46,7 @@ __device__ __forceinline__ int quotient(int n, int d, float per_d) {
   return q + ((q + 1) * d <= n);
 }
 
-// A segment of the experts' rows: experts of more than L / 2 rows come first (so that the short jobs fill
+// A segment of the experts' rows: experts of many rows (more than L / 2) come first (so that the short jobs fill
 // the end), each cut into ceil(n / L) parts, an empty one still being a part.
 struct Segment {
   int e, row0, row_end, parts, slot;  // slot: of its partial sums, where the expert has several parts
@@ -77,12 +79,12 @@ __device__ __forceinline__ void part_rows(int lo, int rows, int j, Segment& s) {
   s.row_end = lo + (j + 1 < s.parts && from + size < rows ? from + size : rows);
 }
 // Segment `seg`; first and n: the first row and the number of rows of expert `lane`.
-__device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, int seg, int first, int n, Segment& s) {
+__device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, int many, int seg, int first, int n, Segment& s) {
   const int lane = lane_id();
   int carry = 0;
   if (E <= MOE_WAVE) {
     const int p = lane < E ? parts_of(n, L) : 0;
-    const bool big = 2 * n > L;
+    const bool big = n > many;
     const int ib = wave_inclusive(big ? p : 0);
     const int nbig = read_lane(ib, 63);
     const int is = nbig + wave_inclusive(big ? 0 : p);
@@ -100,7 +102,7 @@ __device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, 
   for (int pass = 0; pass < 2; ++pass)
     for (int b = 0; b < E; b += MOE_WAVE) {
       const int n = expert_rows(offs, b + lane, E);
-      const bool mine = b + lane < E && (2 * n > L) == (pass == 0);
+      const bool mine = b + lane < E && (n > many) == (pass == 0);
       const int p = mine ? parts_of(n, L) : 0;
       const int incl = wave_inclusive(p);
       const int total = read_lane(incl, MOE_WAVE - 1);
@@ -139,15 +141,15 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   // in its L2), so that all of them have the same list of segments, long ones first.  (64 consecutive tiles to an
   // XCD, Zipf: 1.30 workgroups a compute unit on average where it is 1.55 now, with two resident.)
   const int b = blockIdx.x, x = b & 7;
-  int job = b >> 3;
+  int job = (b >> 3) - (p.r_first ? p.r_each : 0);  // (the experts' from 0)
   Stack st;
   Segment sg;
   int tile;
   // (asked for first: on the way while the job's numbers are worked out)
-  const bool experts = job < p.e_each && lane < p.E;
+  const bool of_router = job < 0 || job >= p.e_each, experts = !of_router && lane < p.E;
   const int first = experts ? p.offs[lane] : 0, count = experts ? max(p.offs[lane + 1] - first, 0) : 0;
-  if (job >= p.e_each) {
-    job += x * p.r_each - p.e_each;
+  if (of_router) {
+    job += x * p.r_each + (p.r_first ? p.r_each : -p.e_each);
     if (job >= p.r_slices * p.router.tiles) return;
     st = p.router;
     const int sl = quotient(job, st.tiles, p.r_per_tiles);
@@ -155,12 +157,12 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
     sg.e = 0;
     sg.row0 = sl * p.r_rows;
     sg.row_end = sg.row0 + p.r_rows < p.T ? sg.row0 + p.r_rows : p.T;
-    sg.parts = 2;  // (its sums always go through the second kernel, which may have fewer rows to write)
+    sg.parts = p.r_slices;
     sg.slot = sl;
   } else {
     const int seg = quotient(job, p.each, p.per_each);
     tile = x * p.each + job - seg * p.each;
-    if (tile >= p.tiles || !find_segment(p.offs, p.E, p.L, seg, first, count, sg)) return;
+    if (tile >= p.tiles || !find_segment(p.offs, p.E, p.L, p.many, seg, first, count, sg)) return;
     const int t0 = p.s[0].tiles, t1 = t0 + p.s[1].tiles;
     st = tile < t0 ? p.s[0] : (tile < t1 ? p.s[1] : p.s[2]);
     tile -= tile < t0 ? 0 : (tile < t1 ? t0 : t1);
@@ -302,7 +304,7 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
 __global__ __launch_bounds__(256) void wgrad_multi_sum_kernel(const MultiArgs p) {
   const int lane = lane_id();
   int e = 0, parts = p.r_slices, slot = 0;
-  const bool router = p.r_slices > 0 && blockIdx.y == gridDim.y - 1;
+  const bool router = p.r_slices > 1 && blockIdx.y == gridDim.y - 1;
   if (!router) {
     int carry = 0, slots = 0;
     bool found = false;
@@ -404,26 +406,33 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
   a.E = (int)E;
   // (from the shapes alone, whichever stacks are wanted: the room for the partial sums was made for it)
   a.L = n_stacks ? (int)segment_rows(R, H, I) : 1;
+  a.many = a.L / 2;
+  if (T <= a.L) a.L = (int)(R > 1 ? R : 1);  // (no expert has more rows than there are tokens: nothing to cut)
   a.T = (int)T;
   if (router) {
     fill(a.router, *router);
     a.r_rows = (int)router_rows;
     a.r_slices = (int)router_slices;
+    // (one slice is written straight to its result, which may have fewer rows than the padded product, and is as long as
+    // any expert's jobs)
+    a.r_first = router_slices == 1;
+    if (router_slices == 1) a.router.M = (int)E;
   }
   a.each = a.tiles > 0 ? (a.tiles + 7) / 8 : 1, a.per_each = 1.f / a.each;
   a.r_each = (a.r_slices * a.router.tiles + 7) / 8, a.r_per_tiles = a.router.tiles ? 1.f / a.router.tiles : 0.f;
-  const long long segs = n_stacks ? R / a.L + E : 0;
+  const long long segs = n_stacks ? (R > a.L ? R / a.L : 0) + E : 0;
   const long long e_each = n_stacks ? segs * a.each : 0, jobs = 8 * (e_each + (long long)a.r_each);
   if (jobs <= 0) return 0;
   if (jobs > 0x7fffffffll) return MOE_ERR_LIMIT;
   a.e_each = (int)e_each;
   hipLaunchKernelGGL(wgrad_multi_kernel, dim3((unsigned)jobs), dim3(WNT), 0, s, a);
-  const long long cut = n_stacks ? R / a.L : 0;  // experts of more than L rows, at most
-  const long long ys = (cut < E ? cut : E) + (router ? 1 : 0);
+  const long long cut = n_stacks && R > a.L ? R / a.L : 0;  // experts of more than L rows, at most
+  const bool sliced = router && router_slices > 1;
+  const long long ys = (cut < E ? cut : E) + (sliced ? 1 : 0);
   if (ys > 0) {
     long long n8 = 0;
     for (int i = 0; i < n_stacks; ++i) n8 += (long long)a.s[i].M * a.s[i].N / 8;
-    const long long nr = router ? (long long)a.router.M * a.router.N / 8 : 0;
+    const long long nr = sliced ? (long long)a.router.M * a.router.N / 8 : 0;
     if (nr > n8) n8 = nr;
     long long bx = (n8 + 255) / 256;
     if (bx > 2048) bx = 2048;
