@@ -353,27 +353,74 @@ __global__ __launch_bounds__(256) void permute_fwd_scatter_kernel(const XT* __re
 // out[t,:] = sum_j gates[t*k+j] * y[row_to_pos[t*k+j],:]  (+ addend[t,:]); fp32, slot order.  IN_ORDER: the rows of
 // y are in routed order, there is no map.  (A question at run time parts the loads of the positions from each
 // other: 1531 tokens, k = 8, 2048 wide, 11.6 -> 12.6 us.)
-// ROUTER: + bf16(sum_j dsel[t*k+j] * wr[ids[t*k+j],:]), the router path's input gradient: a row of
-// dlogits has k nonzero entries, so that product is k rows of the router weight per token, which sit in
+// LT other than void: the router's backward with it.  The token's row of dlogits (bf16 or fp32) from the block sums that
+// dgrad-down leaves, in the arithmetic of router_bwd_from_blocks_kernel, and + bf16(sum_j dsel[j] * wr[ids[t*k+j],:]) with dsel
+// its k nonzero entries: the router path's input gradient, k rows of the router weight a token, which sit in
 // every XCD's L2 (at most 512 rows) -- instead of a library product over all E columns, its result in
-// memory and another read of it here.
+// memory and another read of it here.  (In one kernel instead
+// of two, us: 8192 tokens, 2 of 8 experts, 1024 wide, 4 blocks 18.1 -> 12.3; 4096, 8 of 128, 1024 wide, 4 blocks, 25.9 -> 22.1; 16384, 8 of 64, 2048
+// wide, 16 blocks 141 -> 126.)
 // Bound by memory; on small calls by the two trips it takes, positions and then rows.  One wave a token: positions,
 // gates and ids are the same for all of its lanes and come as scalars, eight at a time, and the rows of y and of wr
 // are on their way together.  (A lane a piece of any of four tokens, wr after y: 8192 tokens, k = 2, 1024 wide,
 // both directions 31.2 -> 23.2 us; 3333 tokens, k = 3, 1416 wide 32.4 -> 21.2; 16384 tokens, k = 8, 2048 wide 250 -> 227.)
-template <typename OT, typename AT, bool ROUTER, bool IN_ORDER>
+struct RouterGrad {
+  const float* part;   // [P][T*k], by position
+  int P;
+  const float* gates;
+  const int32_t* ids;
+  const uint16_t* wr;  // [E, H]
+  void* dlogits;       // [T, ld]
+  int ld;
+};
+template <typename OT, typename AT, typename LT, bool IN_ORDER>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __restrict__ y,
                                                          const float* __restrict__ gates,
                                                          const int32_t* __restrict__ row_to_pos,
                                                          const AT* __restrict__ addend, int T,
-                                                         int H8, int k, OT* __restrict__ out,
-                                                         const float* __restrict__ dsel,
-                                                         const int32_t* __restrict__ ids,
-                                                         const uint16_t* __restrict__ wr) {
+                                                         int H8, int k, OT* __restrict__ out, const RouterGrad rg) {
+  constexpr bool ROUTER = !std::is_void<LT>::value;
   const int H = H8 * 8;
   for (int t = blockIdx.x * ROWS_PER_BLOCK + uniform((int)(threadIdx.x / MOE_WAVE)); t < T;
        t += gridDim.x * ROWS_PER_BLOCK) {
     const int r0 = t * k;
+    int id = -1;       // of slot `lane`
+    float dsel = 0.f;
+    if constexpr (ROUTER) {
+      const int lane = lane_id();
+      float s = 0.f, g = 0.f;
+      if (lane < k) {
+        const float* src = rg.part + row_to_pos[r0 + lane];
+        id = rg.ids[r0 + lane];
+        g = rg.gates[r0 + lane];
+        const size_t R = (size_t)T * k;
+        int b = 0;
+        for (; b + 8 <= rg.P; b += 8) {  // (eight gathers in flight, added in ascending order)
+          float v[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = src[(size_t)(b + i) * R];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) s += v[i];
+        }
+        for (; b + 4 <= rg.P; b += 4) {
+          const float v0 = src[(size_t)b * R], v1 = src[(size_t)(b + 1) * R], v2 = src[(size_t)(b + 2) * R],
+                      v3 = src[(size_t)(b + 3) * R];
+          s = (((s + v0) + v1) + v2) + v3;
+        }
+        for (; b < rg.P; ++b) s += src[(size_t)b * R];
+      }
+      const float dg = g != 0.f ? s / g : 0.f;
+      float dot = 0.f;
+      for (int j = 0; j < k; ++j) dot += read_lane_f(g, j) * read_lane_f(dg, j);
+      dsel = g * (dg - dot);
+      if constexpr (ROUTER && sizeof(LT) == 2) dsel = bf16_to_f32(f32_to_bf16(dsel));
+      for (int e = lane; e < rg.ld; e += MOE_WAVE) {
+        float v = 0.f;
+        for (int j = 0; j < k; ++j) v = read_lane(id, j) == e ? read_lane_f(dsel, j) : v;
+        if constexpr (ROUTER && sizeof(LT) == 2) ((uint16_t*)rg.dlogits)[(size_t)t * rg.ld + e] = f32_to_bf16(v);
+        else ((float*)rg.dlogits)[(size_t)t * rg.ld + e] = v;
+      }
+    }
     for (int col = lane_id() * 8; col < H; col += MOE_WAVE * 8) {
       Row8 acc, d2;
 #pragma unroll
@@ -389,7 +436,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
         }
         if constexpr (ROUTER) {
 #pragma unroll
-          for (int q = 0; q < N; ++q) w[q] = *reinterpret_cast<const u32x4*>(wr + (size_t)ids[r0 + j + q] * H + col);
+          for (int q = 0; q < N; ++q) w[q] = *reinterpret_cast<const u32x4*>(rg.wr + (size_t)read_lane(id, j + q) * H + col);
         }
 #pragma unroll
         for (int q = 0; q < N; ++q) {
@@ -401,7 +448,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
         if constexpr (ROUTER) {
 #pragma unroll
           for (int q = 0; q < N; ++q) {
-            const float ds = dsel[r0 + j + q];
+            const float ds = read_lane_f(dsel, j + q);
             const Row8 row = row8_from_bits(w[q]);
 #pragma unroll
             for (int i = 0; i < 8; ++i) d2.v[i] += ds * row.v[i];
@@ -753,14 +800,14 @@ static int combine_like(const uint16_t* y, const float* gates, const int32_t* ro
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
   if (out_dtype == MOE_DT_BF16 && addend_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false, false>), grid, block, 0, s, y, gates, row_to_pos,
-                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (uint16_t*)out, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, void, false>), grid, block, 0, s, y, gates, row_to_pos,
+                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (uint16_t*)out, RouterGrad{});
   else if (out_dtype == MOE_DT_F32 && addend_dtype == MOE_DT_F32)
-    hipLaunchKernelGGL((combine_fwd_kernel<float, float, false, false>), grid, block, 0, s, y, gates, row_to_pos,
-                       (const float*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((combine_fwd_kernel<float, float, void, false>), grid, block, 0, s, y, gates, row_to_pos,
+                       (const float*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, RouterGrad{});
   else if (out_dtype == MOE_DT_F32 && addend_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false, false>), grid, block, 0, s, y, gates, row_to_pos,
-                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, void, false>), grid, block, 0, s, y, gates, row_to_pos,
+                       (const uint16_t*)addend, (int)T, (int)(H / 8), (int)k, (float*)out, RouterGrad{});
   else
     return MOE_ERR_DTYPE;
   return moe_launch_status();
@@ -1060,25 +1107,26 @@ int moe_combine_in_order(const uint16_t* y, const float* gates, int64_t T, int64
   const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
   const uint16_t* none = nullptr;
   if (out_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, false, true>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
-                       (int)(H / 8), (int)k, (uint16_t*)out, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, void, true>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
+                       (int)(H / 8), (int)k, (uint16_t*)out, RouterGrad{});
   else
-    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, false, true>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
-                       (int)(H / 8), (int)k, (float*)out, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, void, true>), grid, block, 0, s, y, gates, nullptr, none, (int)T,
+                       (int)(H / 8), (int)k, (float*)out, RouterGrad{});
   return moe_launch_status();
 }
 
-int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const float* dsel, const int32_t* ids,
-                           const uint16_t* wr, int64_t T, int64_t H, int64_t k, void* dx, int dx_dtype,
-                           hipStream_t s) {
-  const dim3 grid(mover_grid(T, ROWS_PER_BLOCK)), block(256);
-  if (dx_dtype == MOE_DT_BF16)
-    hipLaunchKernelGGL((combine_fwd_kernel<uint16_t, uint16_t, true, false>), grid, block, 0, s, dxp, nullptr, row_to_pos,
-                       nullptr, (int)T, (int)(H / 8), (int)k, (uint16_t*)dx, dsel, ids, wr);
-  else
-    hipLaunchKernelGGL((combine_fwd_kernel<float, uint16_t, true, false>), grid, block, 0, s, dxp, nullptr, row_to_pos,
-                       nullptr, (int)T, (int)(H / 8), (int)k, (float*)dx, dsel, ids, wr);
-  return moe_launch_status();
+int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const float* part, int64_t P, const float* gates,
+                           const int32_t* ids, const uint16_t* wr, int64_t T, int64_t H, int64_t k, int64_t ld, void* dlogits,
+                           int dlogits_dtype, void* dx, int dx_dtype, hipStream_t s) {
+  const RouterGrad rg{part, (int)P, gates, ids, wr, dlogits, (int)ld};
+  const auto go = [&](auto out, auto logit) {
+    using OT = decltype(out);
+    hipLaunchKernelGGL((combine_fwd_kernel<OT, uint16_t, decltype(logit), false>), dim3(mover_grid(T, ROWS_PER_BLOCK)), dim3(256), 0,
+                       s, dxp, nullptr, row_to_pos, nullptr, (int)T, (int)(H / 8), (int)k, (OT*)dx, rg);
+    return moe_launch_status();
+  };
+  if (dlogits_dtype == MOE_DT_BF16) return dx_dtype == MOE_DT_BF16 ? go(uint16_t{}, uint16_t{}) : go(float{}, uint16_t{});
+  return dx_dtype == MOE_DT_BF16 ? go(uint16_t{}, float{}) : go(float{}, float{});
 }
 
 namespace {

@@ -17,17 +17,16 @@ inline double moe_expected_tiles(int64_t R, int64_t E, int bm) {
 }
 
 // Gate gradients from the dgrad-down kernel's block sums, softmax Jacobian and scatter to the logits in
-// one kernel (route.hip).  dlogits [T, ld] with columns E..ld-1 zero; dsel fp32 [T*k] (may be NULL): the k
-// nonzero entries per token, rounded to dlogits' type.
+// one kernel (route.hip).  dlogits [T, ld] with columns E..ld-1 zero.
 int moe_router_bwd_from_blocks(const float* part, int64_t P, const float* gates, const int32_t* ids,
                                const int32_t* row_to_pos, int64_t T, int64_t E, int64_t k, int64_t ld,
-                               void* dlogits, int dlogits_dtype, float* dsel, hipStream_t s);
+                               void* dlogits, int dlogits_dtype, hipStream_t s);
 
-// moe_permute_bwd with the router path's input gradient in the same pass: dx[t] = sum_j dxp[pos(t,j)]
-// + bf16(sum_j dsel[t,j] * wr[ids[t,j]]) (dispatch.hip).
-int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const float* dsel, const int32_t* ids,
-                           const uint16_t* wr, int64_t T, int64_t H, int64_t k, void* dx, int dx_dtype,
-                           hipStream_t s);
+// moe_permute_bwd with the router path's input gradient and what moe_router_bwd_from_blocks does in the same pass: dx[t] =
+// sum_j dxp[pos(t,j)] + bf16(sum_j dsel[t,j] * wr[ids[t,j]]), dsel the k nonzero entries of a row of dlogits (dispatch.hip).
+int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const float* part, int64_t P, const float* gates,
+                           const int32_t* ids, const uint16_t* wr, int64_t T, int64_t H, int64_t k, int64_t ld, void* dlogits,
+                           int dlogits_dtype, void* dx, int dx_dtype, hipStream_t s);
 
 // fp32 to bf16, two tensors of multiples of 8 elements in one launch (dispatch.hip).
 int moe_cast_two(const float* a, uint16_t* to_a, int64_t na, const float* b, uint16_t* to_b, int64_t nb, void* stream);

@@ -263,7 +263,7 @@ RouterSlices router_slices(int64_t T, int64_t H, int64_t E) {
 
 struct BwdScratch {
   uint16_t *dyp, *dg, *dxp;
-  float *part, *dsel, *wpart[3], *rpart;
+  float *part, *wpart[3], *rpart;
   uint16_t* dlogits;
   BwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
     const int64_t R = T * k;
@@ -271,7 +271,6 @@ struct BwdScratch {
     dg = (uint16_t*)s.take(R * I * 4);
     dxp = (uint16_t*)s.take(R * H * 2);
     part = (float*)s.take(moe_dgate_blocks(I) * R * 4);
-    dsel = (float*)s.take(R * 4);
     const RouterSlices rs = router_slices(T, H, E);
     dlogits = (uint16_t*)s.take(T * rs.Ep * 4);
     rpart = (float*)s.take(rs.slices * rs.Ep * H * 4);
@@ -447,20 +446,29 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     MOE_STEP("moe_dgates_from_blocks_by_pos", moe_dgates_from_blocks_by_pos(part, moe_dgate_blocks(I), a->gates,
                                                                             a->pos_to_row, R, a->dgates, stream));
   const RouterSlices rs = router_slices(T, H, E);
-  if (to_logits && R > 0) {
-    // (for the router's weight gradient the rows of dlogits are padded to a multiple of 8 columns)
-    const bool own = !a->dlogits;
-    MOE_STEP("moe_router_bwd_from_blocks",
-             moe_router_bwd_from_blocks(part, moe_dgate_blocks(I), a->gates, a->ids, a->row_to_pos, T, E, k,
-                                        own ? rs.Ep : E, own ? ws.dlogits : a->dlogits,
-                                        own ? MOE_DT_BF16 : (int)a->dlogits_dtype, router ? ws.dsel : nullptr, st));
-  }
+  // (for the router's weight gradient the rows of dlogits are padded to a multiple of 8 columns)
+  const bool own = !a->dlogits, with_dx = router && a->dx;
+  void* dlogits = own ? ws.dlogits : a->dlogits;
+  const int64_t ld = own ? rs.Ep : E;
+  const int dlogits_dtype = own ? MOE_DT_BF16 : (int)a->dlogits_dtype;
+  if (to_logits && !with_dx && R > 0)
+    MOE_STEP("moe_router_bwd_from_blocks", moe_router_bwd_from_blocks(part, moe_dgate_blocks(I), a->gates, a->ids, a->row_to_pos, T,
+                                                                      E, k, ld, dlogits, dlogits_dtype, st));
   if (a->dx || a->dxp) {
     if (pair)
       MOE_STEP("moe_gemm_dgrad_gateup_packed",
                moe_gemm_dgrad_gateup_packed(dg, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
     else
       MOE_STEP("moe_gemm_dgrad_gateup", moe_gemm_dgrad_gateup(dg, du, a->w1, a->w3, a->offs, E, R, H, I, dxp, stream));
+  }
+  if (a->dx && T > 0) {  // (before the weight gradients: the router's reads dlogits)
+    if (router && to_logits)
+      MOE_STEP("moe_permute_bwd_router",
+               moe_permute_bwd_router(dxp, a->row_to_pos, part, moe_dgate_blocks(I), a->gates, a->ids, a->wr, T, H, k, ld, dlogits,
+                                      dlogits_dtype, a->dx, (int)a->dx_dtype, st));
+    else
+      MOE_STEP("moe_permute_bwd",
+               moe_permute_bwd(dxp, a->row_to_pos, nullptr, T, H, k, a->dx, (int)a->dx_dtype, stream));
   }
   const bool router_dw = router && to_logits && a->dwr;
   if (router_dw && a->dlogits) return MOE_ERR_SHAPE;  // one or the other: the caller's dlogits are not padded
@@ -503,14 +511,6 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     if (router_dw)
       MOE_STEP("moe_router_wgrad",
                moe_wgrad_multi(stacks, 0, &rstack, a->offs, E, R, H, I, T, rs.slices, rs.rows, st));
-  }
-  if (a->dx && T > 0) {
-    if (router && to_logits)
-      MOE_STEP("moe_permute_bwd_router",
-               moe_permute_bwd_router(dxp, a->row_to_pos, ws.dsel, a->ids, a->wr, T, H, k, a->dx, (int)a->dx_dtype, st));
-    else
-      MOE_STEP("moe_permute_bwd",
-               moe_permute_bwd(dxp, a->row_to_pos, nullptr, T, H, k, a->dx, (int)a->dx_dtype, stream));
   }
   return 0;
 }

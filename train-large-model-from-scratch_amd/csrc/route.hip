@@ -78,8 +78,7 @@ constexpr int RB_PAIRS = 512;  // (token, slot) pairs per block at most
 template <typename DT>
 __global__ __launch_bounds__(256) void router_bwd_from_blocks_kernel(
     const float* __restrict__ part, int P, const float* __restrict__ gates, const int32_t* __restrict__ ids,
-    const int32_t* __restrict__ row_to_pos, int T, int E, int k, int TB, int ld, DT* __restrict__ dlogits,
-    float* __restrict__ dsel_out) {
+    const int32_t* __restrict__ row_to_pos, int T, int E, int k, int TB, int ld, DT* __restrict__ dlogits) {
   __shared__ float sg[RB_PAIRS], sdg[RB_PAIRS], ssel[RB_PAIRS];
   __shared__ int sid[RB_PAIRS];
   const int t0 = blockIdx.x * TB, nt = T - t0 < TB ? T - t0 : TB, n = nt * k;
@@ -107,7 +106,6 @@ __global__ __launch_bounds__(256) void router_bwd_from_blocks_kernel(
     float v = sg[i] * (sdg[i] - dot);
     if constexpr (sizeof(DT) == 2) v = bf16_to_f32(f32_to_bf16(v));
     ssel[i] = v;
-    if (dsel_out) dsel_out[r0 + i] = v;
   }
   __syncthreads();
   for (int i = threadIdx.x; i < nt * ld; i += blockDim.x) {
@@ -175,7 +173,7 @@ extern "C" int moe_router_topk_bwd(const float* gates, const float* dgates, cons
 
 int moe_router_bwd_from_blocks(const float* part, int64_t P, const float* gates, const int32_t* ids,
                                const int32_t* row_to_pos, int64_t T, int64_t E, int64_t k, int64_t ld,
-                               void* dlogits, int dlogits_dtype, float* dsel, hipStream_t s) {
+                               void* dlogits, int dlogits_dtype, hipStream_t s) {
   // tokens per block: about a pair per thread, and enough blocks for the chip
   int64_t TB = 256 / k;
   if (TB < 1) TB = 1;
@@ -183,9 +181,9 @@ int moe_router_bwd_from_blocks(const float* part, int64_t P, const float* gates,
   const dim3 grid((unsigned)((T + TB - 1) / TB)), block(256);
   if (dlogits_dtype == MOE_DT_BF16)
     hipLaunchKernelGGL(router_bwd_from_blocks_kernel<uint16_t>, grid, block, 0, s, part, (int)P, gates, ids,
-                       row_to_pos, (int)T, (int)E, (int)k, (int)TB, (int)ld, (uint16_t*)dlogits, dsel);
+                       row_to_pos, (int)T, (int)E, (int)k, (int)TB, (int)ld, (uint16_t*)dlogits);
   else
     hipLaunchKernelGGL(router_bwd_from_blocks_kernel<float>, grid, block, 0, s, part, (int)P, gates, ids, row_to_pos,
-                       (int)T, (int)E, (int)k, (int)TB, (int)ld, (float*)dlogits, dsel);
+                       (int)T, (int)E, (int)k, (int)TB, (int)ld, (float*)dlogits);
   return moe_launch_status();
 }
