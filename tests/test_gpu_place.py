@@ -148,3 +148,49 @@ def test_places_of_given_experts(pkg, lib, T, E, H, dtype):
         assert np.array_equal(rt[name].cpu().numpy().reshape(-1), want.astype(np.int32)), name
     sorted_out = pkg.experts_rows(x[torch.tensor(order, device="cuda")], torch.tensor(flat[order], device="cuda"), *ws)
     assert torch.equal(out[torch.tensor(order, device="cuda")], sorted_out)
+
+
+@pytest.mark.parametrize("T,E,k", [
+    (65, 8, 8),       # every expert asked for
+    (511, 4, 1),      # a lane short of a workgroup's
+    (513, 4, 4),      # one token in its second turn
+    (682, 8, 3),      # the most rows
+    (1024, 8, 2),
+    (1024, 4, 2),
+    (1025, 8, 1),     # past it: two launches
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("unaligned", [False, True])  # logits of which a lane cannot read a row at once: two launches
+def test_selection_and_places_in_one_launch(pkg, lib, T, E, k, dtype, unaligned):
+    print("one launch", T, E, k, dtype, unaligned, flush=True)
+    g = torch.Generator().manual_seed(T + E)
+    logits = torch.randn(T, E, generator=g).round(decimals=1).to(dtype)  # (ties)
+    logits[::7, 0], logits[::5, E - 1] = -float("inf"), float("inf")
+    logits[3, 1], logits[4, :] = float("nan"), -float("inf")
+    bias = torch.randn(E, generator=g).round(decimals=1)
+    x, ws = torch.randn(T, 64, generator=g), [torch.randn(*s, generator=g) * 0.1 for s in ((E, 8, 64), (E, 8, 64), (E, 64, 8))]
+    lg = torch.empty(T * E + 1, dtype=dtype, device="cuda")[1:].view(T, E) if unaligned else torch.empty(T, E, dtype=dtype, device="cuda")
+    lg.copy_(logits)
+    ops, dev = pkg.ops, lambda t: t.to(torch.bfloat16).cuda()
+    i32 = lambda n: torch.empty(n, dtype=torch.int32, device="cuda")
+    ids, gates, counts, offs, p2r, r2p = i32(T * k), i32(T * k), i32(E), i32(E + 1), i32(T * k), i32(T * k)
+    xd, wd, bd, out = dev(x), [dev(w) for w in ws], bias.cuda(), torch.empty(T, 64, dtype=torch.bfloat16, device="cuda")
+    xp, act = torch.empty(T * k, 64, dtype=torch.bfloat16, device="cuda"), torch.empty(T * k, 8, dtype=torch.bfloat16, device="cuda")
+    scratch = torch.empty(max(lib.cdll.moe_layer_scratch_bytes(T, 64, E, 8, k, 0), 256), dtype=torch.uint8, device="cuda")
+    p, bf16 = lambda t: t.data_ptr(), pkg.lib.DT_BF16
+    lib.call_layer("moe_layer_forward", ops._FORWARD_ARGS.pack(
+        T, 64, E, 8, k, p(xd), bf16, p(lg), bf16 if dtype == torch.bfloat16 else pkg.lib.DT_F32, p(bd), 0, p(wd[0]), p(wd[1]), p(wd[2]),
+        0, p(out), bf16, p(ids), p(gates), p(counts), p(offs), p(p2r), p(r2p), 0, p(xp), 0, p(act), p(scratch),
+        scratch.numel()), ops._stream())
+    want, _ = O.topk_select(logits.float() + bias, k)
+    flat = want.reshape(-1)
+    order = np.argsort(flat, kind="stable")
+    inverse = np.empty_like(order)
+    inverse[order] = np.arange(T * k)
+    n = np.bincount(flat, minlength=E)
+    for name, got, ref in (("ids", ids, flat), ("counts", counts, n), ("offs", offs, np.concatenate([[0], n.cumsum()])),
+                           ("pos_to_row", p2r, order), ("row_to_pos", r2p, inverse)):
+        assert np.array_equal(got.cpu().numpy(), ref.astype(np.int32)), name
+    assert torch.equal(xp.cpu(), xd.cpu()[torch.tensor(order) // k])
+    ids_ref, gates_ref = ops.router_topk(lg.clone(), k, bd)  # (the selection by itself)
+    assert torch.equal(ids.view(-1), ids_ref.view(-1)) and torch.equal(gates, gates_ref.reshape(-1).view(torch.int32))

@@ -30,6 +30,10 @@ int moe_select_count(const void* logits, int logits_dtype, const float* bias, in
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
                    int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
                    void* xp, int xp_dtype, bool counted, void* stream);
+bool moe_select_place_ok(const void* logits, int64_t T, int64_t E, int64_t k);
+int moe_select_place(const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t H,
+                     int64_t E, int64_t k, int32_t* ids, float* gates, int32_t* counts, int32_t* offs, int32_t* pos_to_row,
+                     int32_t* row_to_pos, int32_t* bad_ids, void* xp, int xp_dtype, void* stream);
 int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, float eps, const uint16_t* router_weight,
                              int64_t T, int64_t H, int64_t E, int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
                              int32_t* ids, float* gates, void* table, void* stream);
@@ -653,7 +657,10 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
     if (bias.defined()) b = dense(bias);
     gates = (float*)r.part(f.routing, Routing::GATES);
   }
-  if (place) {
+  if (place && moe_select_place_ok(logits.data_ptr(), T, E, k)) {
+    CALL(moe_select_place, x.data_ptr<float>(), MOE_DT_F32, logits.data_ptr(), (int)dt(logits), (const float*)ptr(b), T, H, E, k, ids,
+         gates, counts, offs, p2r, r2p, nullptr, xp, MOE_DT_F32, s);
+  } else if (place) {
     CALL(moe_select_count, logits.data_ptr(), (int)dt(logits), (const float*)ptr(b), T, E, k, ids, gates, ws.data_ptr(), s);
     CALL(moe_place_rows, x.data_ptr<float>(), MOE_DT_F32, ids, ws.data_ptr(), T, H, E, k, counts, offs, p2r, r2p,
          nullptr, xp, MOE_DT_F32, false, s);

@@ -63,6 +63,11 @@ int moe_select_count(const void* logits, int logits_dtype, const float* bias, in
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
                    int64_t k, int32_t* counts, int32_t* offs, int32_t* pos_to_row, int32_t* row_to_pos, int32_t* bad_ids,
                    void* xp, int xp_dtype, bool counted, void* stream);
+// Both in one launch, for few logits.
+bool moe_select_place_ok(const void* logits, int64_t T, int64_t E, int64_t k);
+int moe_select_place(const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t H,
+                     int64_t E, int64_t k, int32_t* ids, float* gates, int32_t* counts, int32_t* offs, int32_t* pos_to_row,
+                     int32_t* row_to_pos, int32_t* bad_ids, void* xp, int xp_dtype, void* stream);
 // The table where the experts are given, one a row (`counted` above), and how many of them are outside [0, E) behind it:
 // sizes it takes, bytes of both, and the launch.  ids64, unless NULL, are left in `ids` in 32 bits, else `ids` are given.
 bool moe_count_ok(int64_t T, int64_t E, int64_t k);

@@ -131,7 +131,11 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   }
   const bool few = moe_few_ok(T, H, E, I, k, x_dtype), place = !few && moe_place_ok(T, E, k);
   const bool selects = few && moe_gateup_few_selects(T, E, I, k);  // gate/up does the selection
-  if (place)
+  const bool at_once = place && moe_select_place_ok(logits, T, E, k);
+  if (at_once)
+    MOE_STEP("moe_select_place", moe_select_place(x, x_dtype, logits, logits_dtype, bias, T, H, E, k, ids, gates, counts, offs,
+                                                  pos_to_row, row_to_pos, nullptr, xp, MOE_DT_BF16, stream));
+  else if (place)
     MOE_STEP("moe_select_count", moe_select_count(logits, logits_dtype, bias, T, E, k, ids, gates, ws + c.dispatch, stream));
   else if (!selects)
     MOE_STEP("moe_router_topk_fwd", moe_router_topk_fwd(logits, logits_dtype, bias, T, E, k, ids, gates, stream));
@@ -149,10 +153,10 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
     MOE_STEP("moe_combine_in_order", moe_combine_in_order(y, gates, T, H, k, out, out_dtype, st));
     return 0;
   }
-  if (place) {
+  if (place && !at_once) {
     MOE_STEP("moe_place_rows", moe_place_rows(x, x_dtype, ids, ws + c.dispatch, T, H, E, k, counts, offs, pos_to_row,
                                               row_to_pos, nullptr, xp, MOE_DT_BF16, false, stream));
-  } else {
+  } else if (!place) {
     MOE_STEP("moe_histogram_scan_checked",
              moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
                                 moe_dispatch_workspace_bytes(R, E), stream));
@@ -341,7 +345,11 @@ static int layer_forward(const moe_layer_forward_args* a, const void* table, voi
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
   const FwdScratch ws(s, T, H, E, k);
   if (!s.fits()) return MOE_ERR_WORKSPACE;
-  if ((a->logits || table) && moe_place_ok(T, E, k)) {
+  if (a->logits && !table && moe_select_place_ok(a->logits, T, E, k)) {
+    MOE_STEP("moe_select_place", moe_select_place(a->x, (int)a->x_dtype, a->logits, (int)a->logits_dtype, a->bias, T, H, E, k, a->ids,
+                                                  a->gates, a->counts, a->offs, a->pos_to_row, a->row_to_pos, a->bad_ids, a->xp,
+                                                  MOE_DT_BF16, stream));
+  } else if ((a->logits || table) && moe_place_ok(T, E, k)) {
     if (!table)
       MOE_STEP("moe_select_count", moe_select_count(a->logits, (int)a->logits_dtype, a->bias, T, E, k, a->ids, a->gates,
                                                     ws.dispatch, stream));

@@ -85,13 +85,59 @@ __global__ __launch_bounds__(256) void count_ids_kernel(const IT* __restrict__ i
   for (int i = threadIdx.x; i < n; i += 256) table[(size_t)blockIdx.x * CHUNKS * words + i] = counts[i / words][i % words];
 }
 
+// The experts of E that a token asks for as bits, worked out by one lane from its logits: what moe_topk_softmax_wave selects.
+template <int E, typename LT>
+struct LaneLogits {
+  u32x2 w[E * sizeof(LT) / 8];
+  __device__ __forceinline__ void request(const LT* __restrict__ logits) {
+#pragma unroll
+    for (int i = 0; i < (int)(E * sizeof(LT) / 8); ++i) w[i] = reinterpret_cast<const u32x2*>(logits)[i];
+  }
+  __device__ __forceinline__ uint32_t selected(const float* __restrict__ bias, int k) const {
+    uint32_t key[E], bits = 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      constexpr int PER = 4 / sizeof(LT);
+      const uint32_t word = w[e / PER / 2][e / PER % 2];
+      float v = sizeof(LT) == 4 ? __builtin_bit_cast(float, word) : e & 1 ? bf16hi(word) : bf16lo(word);
+      if (bias) v += bias[e];
+      key[e] = moe_orderable(v);
+    }
+    for (int j = 0; j < k; ++j) {
+      uint32_t best = key[0], has = 0;
+#pragma unroll
+      for (int e = 1; e < E; ++e) best = key[e] > best ? key[e] : best;
+#pragma unroll
+      for (int e = 0; e < E; ++e) has |= key[e] == best ? 1u << e : 0;
+      has &= -has;  // the first that has it
+      bits |= has;
+#pragma unroll
+      for (int e = 0; e < E; ++e) key[e] = has & (1u << e) ? 0 : key[e];  // (which no logit maps to)
+    }
+    return bits;
+  }
+};
+
+// Where a token's experts come from: a selection's table, the caller (they may lie outside [0, E)), or the logits.
+enum Experts { TABLE, GIVEN_IDS, LOGITS };
+template <typename LT>
+struct Selection {  // LOGITS
+  const LT* logits;
+  const float* bias;
+  int32_t* ids;
+  float* gates;
+};
+
 // WAVES tokens of a chunk, one a wave.  `shift`: 2^shift words hold a chunk's counts.
-// GIVEN: the experts are, and may lie outside [0, E).
-template <typename XT, typename OT, int WAVES, bool GIVEN>
+// From the logits (of NE experts) every workgroup selects for all tokens, a lane a token, to count them, and leaves ids and gates of
+// its own.
+template <typename XT, typename OT, int WAVES, Experts FROM, int NE = 8, typename LT = float>
 __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     const XT* __restrict__ x, const int32_t* __restrict__ ids, const uint32_t* __restrict__ table, int T, int E, int k,
     int H, int shift, int32_t* __restrict__ counts, int32_t* __restrict__ offs, int32_t* __restrict__ pos_to_row,
-    int32_t* __restrict__ row_to_pos, int32_t* __restrict__ bad_ids, OT* __restrict__ xp, const uint32_t* __restrict__ bad) {
+    int32_t* __restrict__ row_to_pos, int32_t* __restrict__ bad_ids, OT* __restrict__ xp, const uint32_t* __restrict__ bad,
+    const Selection<LT> sel) {
+  constexpr bool GIVEN = FROM == GIVEN_IDS;
   __shared__ int below[PLACE_EXPERTS], total[PLACE_EXPERTS];  // of earlier chunks, of all
   __shared__ uint32_t asked[PLACE_EXPERTS];
   constexpr int AHEAD = 4;  // 8-element pieces of the row requested at once
@@ -115,50 +161,89 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     const int e = ids[r];
     return !GIVEN ? e : e < 0 ? 0 : e >= E ? E - 1 : e;
   };
-  const int my_id = live && lane < k ? expert_of(t * k + lane) : 0;
+  int my_id = 0;
+  if constexpr (FROM == LOGITS) {
+    if (live) {
+      uint32_t key[1];
+      float gate;
+      moe_topk_keys<1>(sel.logits + (size_t)t * E, sel.bias, E, lane, key);
+      moe_topk_softmax_wave<1>(key, k, lane, my_id, gate);
+      if (lane < k) {
+        sel.ids[(size_t)t * k + lane] = my_id;
+        sel.gates[(size_t)t * k + lane] = gate;
+      }
+    }
+  } else {
+    my_id = live && lane < k ? expert_of(t * k + lane) : 0;
+  }
   __shared__ int outside;
   if (GIVEN && threadIdx.x == 0) outside = 0;
   static_assert(WAVES * MOE_WAVE >= PLACE_EXPERTS && CHUNK % WAVES == 0, "a thread an expert");
   if (threadIdx.x < PLACE_EXPERTS) below[threadIdx.x] = total[threadIdx.x] = 0, asked[threadIdx.x] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < CHUNK * k; i += blockDim.x) {
-    const int r = chunk * CHUNK * k + i;
-    if (r < T * k) atomicOr(&asked[expert_of(r)], 1u << (i / k));
-  }
-  if (GIVEN && blockIdx.x == 0) {
-    int n = 0;
-    for (int c = threadIdx.x; c < chunks; c += blockDim.x) n += bad[c];
-    if (n) atomicAdd(&outside, n);
-  }
-  // two 16-bit sums a register: no expert has more rows than there are tokens
-  const int w = threadIdx.x & ((1 << shift) - 1), step = blockDim.x >> shift;
-  uint32_t all02 = 0, all13 = 0, low02 = 0, low13 = 0;
-  if (w < words) {
-#pragma unroll 4
-    for (int c = threadIdx.x >> shift; c < chunks; c += step) {
-      const uint32_t v = table[(size_t)c * words + w];
-      const uint32_t v02 = v & 0x00ff00ffu, v13 = (v >> 8) & 0x00ff00ffu;
-      all02 += v02;
-      all13 += v13;
-      low02 += c < chunk ? v02 : 0;
-      low13 += c < chunk ? v13 : 0;
+  if constexpr (FROM == LOGITS) {
+    if (live && lane < k) atomicOr(&asked[my_id], 1u << wv);
+    const int t0 = blockIdx.x * WAVES;
+    int all = 0, low = 0;  // of expert `lane`
+    for (int base = wv * MOE_WAVE; base < T; base += WAVES * MOE_WAVE) {
+      uint32_t bits = 0;
+      if (base + lane < T) {
+        LaneLogits<NE, LT> row;
+        row.request(sel.logits + (size_t)(base + lane) * NE);
+        bits = row.selected(sel.bias, k);
+      }
+      const unsigned long long before = t0 <= base ? 0 : t0 - base >= MOE_WAVE ? ~0ull : (1ull << (t0 - base)) - 1;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const unsigned long long who = __ballot(bits >> e & 1);
+        all += lane == e ? __popcll(who) : 0;
+        low += lane == e ? __popcll(who & before) : 0;
+      }
     }
-  }
-  for (int off = MOE_WAVE / 2; off >= 1 << shift; off >>= 1) {
-    all02 += __shfl_xor(all02, off, MOE_WAVE);
-    all13 += __shfl_xor(all13, off, MOE_WAVE);
-    low02 += __shfl_xor(low02, off, MOE_WAVE);
-    low13 += __shfl_xor(low13, off, MOE_WAVE);
-  }
-  if (w < words && lane < (1 << shift)) {
-    atomicAdd(&total[4 * w + 0], (int)(all02 & 0xffff));
-    atomicAdd(&total[4 * w + 1], (int)(all13 & 0xffff));
-    atomicAdd(&total[4 * w + 2], (int)(all02 >> 16));
-    atomicAdd(&total[4 * w + 3], (int)(all13 >> 16));
-    atomicAdd(&below[4 * w + 0], (int)(low02 & 0xffff));
-    atomicAdd(&below[4 * w + 1], (int)(low13 & 0xffff));
-    atomicAdd(&below[4 * w + 2], (int)(low02 >> 16));
-    atomicAdd(&below[4 * w + 3], (int)(low13 >> 16));
+    if (lane < E) {
+      atomicAdd(&total[lane], all);
+      atomicAdd(&below[lane], low);
+    }
+  } else {
+    for (int i = threadIdx.x; i < CHUNK * k; i += blockDim.x) {
+      const int r = chunk * CHUNK * k + i;
+      if (r < T * k) atomicOr(&asked[expert_of(r)], 1u << (i / k));
+    }
+    if (GIVEN && blockIdx.x == 0) {
+      int n = 0;
+      for (int c = threadIdx.x; c < chunks; c += blockDim.x) n += bad[c];
+      if (n) atomicAdd(&outside, n);
+    }
+    // two 16-bit sums a register: no expert has more rows than there are tokens
+    const int w = threadIdx.x & ((1 << shift) - 1), step = blockDim.x >> shift;
+    uint32_t all02 = 0, all13 = 0, low02 = 0, low13 = 0;
+    if (w < words) {
+  #pragma unroll 4
+      for (int c = threadIdx.x >> shift; c < chunks; c += step) {
+        const uint32_t v = table[(size_t)c * words + w];
+        const uint32_t v02 = v & 0x00ff00ffu, v13 = (v >> 8) & 0x00ff00ffu;
+        all02 += v02;
+        all13 += v13;
+        low02 += c < chunk ? v02 : 0;
+        low13 += c < chunk ? v13 : 0;
+      }
+    }
+    for (int off = MOE_WAVE / 2; off >= 1 << shift; off >>= 1) {
+      all02 += __shfl_xor(all02, off, MOE_WAVE);
+      all13 += __shfl_xor(all13, off, MOE_WAVE);
+      low02 += __shfl_xor(low02, off, MOE_WAVE);
+      low13 += __shfl_xor(low13, off, MOE_WAVE);
+    }
+    if (w < words && lane < (1 << shift)) {
+      atomicAdd(&total[4 * w + 0], (int)(all02 & 0xffff));
+      atomicAdd(&total[4 * w + 1], (int)(all13 & 0xffff));
+      atomicAdd(&total[4 * w + 2], (int)(all02 >> 16));
+      atomicAdd(&total[4 * w + 3], (int)(all13 >> 16));
+      atomicAdd(&below[4 * w + 0], (int)(low02 & 0xffff));
+      atomicAdd(&below[4 * w + 1], (int)(low13 & 0xffff));
+      atomicAdd(&below[4 * w + 2], (int)(low02 >> 16));
+      atomicAdd(&below[4 * w + 3], (int)(low13 >> 16));
+    }
   }
   __syncthreads();
   const int n0 = total[lane], n1 = total[MOE_WAVE + lane];
@@ -172,7 +257,7 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
   const int first0 = __shfl(upto0 - n0, my_id & 63, MOE_WAVE), first1 = __shfl(upto1 - n1, my_id & 63, MOE_WAVE);
   int pos = 0;
   if (live && lane < k) {
-    const uint32_t earlier = asked[my_id] & ((1u << (t % CHUNK)) - 1);
+    const uint32_t earlier = asked[my_id] & ((1u << (FROM == LOGITS ? wv : t % CHUNK)) - 1);
     pos = (my_id < MOE_WAVE ? first0 : first1) + below[my_id] + __popc(earlier);
     const int r = t * k + lane;
     row_to_pos[r] = pos;
@@ -254,10 +339,10 @@ int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* t
     const auto launch = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3((unsigned)((T + WAVES - 1) / WAVES)), dim3(WAVES * MOE_WAVE), 0, s, (const XT*)x, ids,
                          (const uint32_t*)table, (int)T, (int)E, (int)k, (int)H, shift, counts, offs, pos_to_row, row_to_pos,
-                         bad_ids, (OT*)xp, bad);
+                         bad_ids, (OT*)xp, bad, Selection<float>{});
     };
-    if (counted) launch(place_rows_kernel<XT, OT, WAVES, true>);
-    else launch(place_rows_kernel<XT, OT, WAVES, false>);
+    if (counted) launch(place_rows_kernel<XT, OT, WAVES, GIVEN_IDS>);
+    else launch(place_rows_kernel<XT, OT, WAVES, TABLE>);
     return moe_launch_status();
   };
   const auto of = [&](auto waves) {
@@ -267,4 +352,38 @@ int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* t
   // (fewer workgroups to read a large table: 4096 tokens, 128 experts 18.1 us, with 8 waves 20.0; 8192 tokens, 8 experts,
   // 4 KB 11.1 and 10.7)
   return moe_place_bytes(T, E) > 16 * 1024 ? of(std::integral_constant<int, 16>{}) : of(std::integral_constant<int, 8>{});
+}
+
+// A launch fewer, as long as the selection of all tokens costs a workgroup less than that: 128 / 512 / 1024 tokens, us, two launches
+// and here: 2 of 8 experts 7.3, 5.2 / 7.8, 5.4 / 8.6, 7.5 (2048: 9.6, 11.4); 1 of 4 7.1, 5.2 / 7.3, 5.2 / 7.5, 6.5.  (2 of 16 7.0, 6.4 /
+// 7.7, 7.0 / 8.6, 10.3, 8 of 16 from the first on slower: not taken.)
+bool moe_select_place_ok(const void* logits, int64_t T, int64_t E, int64_t k) {
+  return moe_place_ok(T, E, k) && (E == 4 || E == 8) && T <= 1024 && T * k <= 2048 && (reinterpret_cast<uintptr_t>(logits) & 7) == 0;
+}
+
+int moe_select_place(const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t H,
+                     int64_t E, int64_t k, int32_t* ids, float* gates, int32_t* counts, int32_t* offs, int32_t* pos_to_row,
+                     int32_t* row_to_pos, int32_t* bad_ids, void* xp, int xp_dtype, void* stream) {
+  if (H <= 0 || H % 8 != 0) return MOE_ERR_SHAPE;
+  if (H > 65536) return MOE_ERR_LIMIT;
+  if (x_dtype == MOE_DT_BF16 && xp_dtype != MOE_DT_BF16) return MOE_ERR_DTYPE;
+  constexpr int WAVES = 8;
+  const auto go = [&](auto xt, auto ot, auto lt, auto ne) {
+    using XT = decltype(xt);
+    using OT = decltype(ot);
+    using LT = decltype(lt);
+    hipLaunchKernelGGL((place_rows_kernel<XT, OT, WAVES, LOGITS, decltype(ne)::value, LT>), dim3((unsigned)((T + WAVES - 1) / WAVES)),
+                       dim3(WAVES * MOE_WAVE), 0, (hipStream_t)stream, (const XT*)x, nullptr, nullptr, (int)T, (int)E, (int)k, (int)H,
+                       0, counts, offs, pos_to_row, row_to_pos, bad_ids, (OT*)xp, nullptr,
+                       Selection<LT>{(const LT*)logits, bias, ids, gates});
+    return moe_launch_status();
+  };
+  const auto of = [&](auto lt, auto ne) {
+    if (x_dtype == MOE_DT_BF16) return go(uint16_t{}, uint16_t{}, lt, ne);
+    return xp_dtype == MOE_DT_BF16 ? go(float{}, uint16_t{}, lt, ne) : go(float{}, float{}, lt, ne);
+  };
+  using Four = std::integral_constant<int, 4>;
+  using Eight = std::integral_constant<int, 8>;
+  if (logits_dtype == MOE_DT_BF16) return E == 4 ? of(uint16_t{}, Four{}) : of(uint16_t{}, Eight{});
+  return E == 4 ? of(float{}, Four{}) : of(float{}, Eight{});
 }
