@@ -68,10 +68,12 @@ constexpr int ROW_TILE = 256;     // rows of a tile of the row-ragged modes
 // The kernel's tile walk: the tiles at positions t_next, t_next + t_step, .. below t_hi of the launch's tile
 // list, or of `list` where one is given.  The rows of a row-ragged launch are numbered in tiles of UNIT rows; where
 // the configuration's are half as high, a list entry is 2 * tile + half.  (tile_start and, there, offs: in LDS.)
-template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE>
+// TO (DOWN and DGRAD_GATEUP only): the rows leave to where p.row_map says.
+template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE, bool TO = false>
 __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, const int* tile_start, const int* offs,
                                            const uint32_t* list, int t_next, const int t_hi, const int t_step) {
   static_assert(!BLK || MODE == GATEUP || MODE == DGRAD_DOWN, "only g and u have the blocked layout");
+  static_assert(!TO || MODE == DOWN || MODE == DGRAD_GATEUP, "only y and dxp are rows that somebody else has a place for");
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, KS = Cfg::KS;
   constexpr int FM = Cfg::FM, FN = Cfg::FN, WTM = Cfg::WTM, WTN = Cfg::WTN;
   constexpr bool DUAL = (MODE == GATEUP);
@@ -429,6 +431,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     }
   };
   BlkRegs blk_in;
+  // (TO) where the wave's rows go, a lane a row: asked for at the top of the tile, there when its contraction is done
+  int row_to[TO ? (WTM + MOE_WAVE - 1) / MOE_WAVE : 1];
   // `last_rows_in` runs once the SwiGLU-backward epilogue has taken the last g/u rows out of their registers
   auto epilogue = [&](const Tile& t, auto&& last_rows_in) {
     // Every per-lane address of the epilogue is derived from this copy of the lane index, which
@@ -472,8 +476,10 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
         const int rr = it * RPI + row_in_pass, ch = chunk_in_row;
         const u32x4 v = *reinterpret_cast<const u32x4*>(strip + plane * SBYTES + rr * SSTRIDE + ch * 16);
         const int r = rbase + rr, c = col_w0 + ch * (16 / OSZ);
+        int to = r - m_shift;
+        if constexpr (TO) to = __shfl(row_to[i / 2], (i & 1) * 32 + rr, MOE_WAVE);
         if (r < row_lim && c < p.N) {
-          u32x4* dst = reinterpret_cast<u32x4*>(gbase + ((long long)(r - m_shift) * ldc + c) * OSZ);
+          u32x4* dst = reinterpret_cast<u32x4*>(gbase + ((long long)to * ldc + c) * OSZ);
           if (MODE == WGRAD && p.accumulate) {
             const u32x4 o = *dst;
             if constexpr (OSZ == 4) {
@@ -696,6 +702,13 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     Tile nxt;
     t_next += t_step;
     const bool more = t_next < t_hi && locate(tile_at(t_next), nxt);
+    if constexpr (TO) {
+#pragma unroll
+      for (int h = 0; h < (WTM + MOE_WAVE - 1) / MOE_WAVE; ++h) {
+        const int r = cur.row0 + wm * WTM + h * MOE_WAVE + lane;
+        row_to[h] = r < cur.row_end ? p.row_map[r] : 0;
+      }
+    }
     const int nkt = cur.nkt;
     const bool stream = STREAM && more && nkt > 1 && nxt.nkt > 0;  // the k-tiles of the next tile follow this one's
     // the k-tile two behind kt
@@ -879,7 +892,7 @@ __device__ __forceinline__ Sweep sweep_of(int n) {
 // fast, 0.94 to 1.25.  (The same quarters with the staging registers of the other tiles: two thirds of that.)  Dgrad-down is
 // 0.79 times as fast in quarters where they are all there is, and 0.94 after whole rounds (577 rows of 24 experts, 4096 <->
 // 1536, 60 -> 96 us; 8641 rows of 48 193 -> 225), never more than 1.05.
-template <int MODE, typename OutT, bool BLK>
+template <int MODE, typename OutT, bool BLK, bool TO>
 __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gemm_kernel(const GemmArgs p) {
   static_assert(CfgHalf::NT == CfgMain::NT, "one workgroup runs both");
   constexpr int WAVES = CfgMain::NT / MOE_WAVE;
@@ -958,7 +971,7 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
       for (int h = 0; h < n; ++h) half_list[at + h - skip] = 2u * (uint32_t)tile + h;
   }
   const Sweep s = sweep_of(whole);
-  walk_tiles<MODE, CfgMain, OutT, BLK>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
+  walk_tiles<MODE, CfgMain, OutT, BLK, ROW_TILE, TO>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
   if (halves == 0) return;
   __syncthreads();  // (the operand stages are free, the list is complete)
   const Sweep h = sweep_of(halves);
@@ -977,24 +990,24 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
         e = __builtin_amdgcn_readfirstlane(e);
         const int first = __builtin_amdgcn_readfirstlane(offs[e]), end = __builtin_amdgcn_readfirstlane(offs[e + 1]);
         const int row = (slot - __builtin_amdgcn_readfirstlane(tile_start[e])) * ROW_TILE + (entry & 3) * Quarter::BM;
-        ring_tile<MODE, BLK, 1, WAVES>(p, (char*)smem, e, first, end, row, tile % p.n_tiles * Quarter::BNC);
+        ring_tile<MODE, BLK, 1, WAVES, TO>(p, (char*)smem, e, first, end, row, tile % p.n_tiles * Quarter::BNC);
         __syncthreads();
       }
       return;
     }
   }
-  walk_tiles<MODE, CfgHalf, OutT, BLK>(p, smem, tile_start, offs, half_list, h.first, h.end, h.step);
+  walk_tiles<MODE, CfgHalf, OutT, BLK, ROW_TILE, TO>(p, smem, tile_start, offs, half_list, h.first, h.end, h.step);
 }
 
 // All in half tiles: launches of so few tiles that there is nothing to decide and that csrc/row_ring.hip does not take (4096 rows
 // of 8 experts, 1024 <-> 512, gate/up 19.5 us; in ring tiles of 64 rows, a few more than fit at once, 23.3).
-template <int MODE, typename OutT, bool BLK>
+template <int MODE, typename OutT, bool BLK, bool TO>
 __global__ __launch_bounds__(CfgHalf::NT, CfgHalf::WAVES_PER_SIMD) void small_rows_gemm_kernel(const GemmArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   __shared__ int tile_start[GEMM_MAX_E + 1], offs[GEMM_MAX_E + 1];
   number_tiles<CfgHalf::BM>(p, tile_start, offs);
   const Sweep s = sweep_of(__builtin_amdgcn_readfirstlane(tile_start[p.E]) * p.n_tiles);
-  walk_tiles<MODE, CfgHalf, OutT, BLK, CfgHalf::BM>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
+  walk_tiles<MODE, CfgHalf, OutT, BLK, CfgHalf::BM, TO>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
 }
 
 // Weight gradients.
@@ -1144,7 +1157,7 @@ constexpr int RING_TILE = 64, RING_TALL = 1;  // (1: the ring's tiles of 128 row
 int forced_row_tile = 0;
 
 // A row-ragged launch with `cols` output columns to a tile.
-template <int MODE, bool BLK = false>
+template <int MODE, bool BLK = false, bool TO = false>
 int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   static_assert(lds_bytes<MODE, CfgHalf>() <= lds_bytes<MODE, CfgMain>(), "both row tiles fit");
   static bool attr_done[2][MOE_MAX_DEVICES];  // per GPU and instantiation
@@ -1158,10 +1171,10 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
                                                  : 2 * tiles < moe_compute_units() &&
                                                        moe_expected_tiles(a.R, a.E, CfgHalf::BM) * a.n_tiles <= moe_compute_units();
   if (small)
-    return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK>, attr_done[0], a,
+    return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK, TO>, attr_done[0], a,
                                  a.n_tiles * row_slots(a.R, a.E, CfgHalf::BM), s);
   a.whole_only = forced_row_tile == ROW_TILE;
-  return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK>, attr_done[1], a,
+  return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK, TO>, attr_done[1], a,
                                2 * a.n_tiles * row_slots(a.R, a.E, ROW_TILE), s);
 }
 template <typename OutT>
@@ -1226,16 +1239,22 @@ extern "C" int moe_gemm_gateup_swiglu_fwd_blocked(const uint16_t* xp, const uint
   return launch_rows<GATEUP, true>(a, CfgMain::BN / 2, (hipStream_t)stream);
 }
 
-extern "C" int moe_gemm_down_fwd(const uint16_t* act, const uint16_t* w2, const int32_t* offs,
-                                 int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* y,
-                                 void* stream) {
+int moe_gemm_down_to(const uint16_t* act, const uint16_t* w2, const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I,
+                     uint16_t* y, const int32_t* row_map, void* stream) {
   if (int rc = check_common(offs, E, R, H, I)) return rc;
   if (R == 0) return 0;
   MOE_CHECK_PTR(act); MOE_CHECK_PTR(w2); MOE_CHECK_PTR(y);
   GemmArgs a{};
   a.A0 = act; a.B0 = w2; a.C0 = y; a.offs = offs;
-  a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I;
+  a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I; a.row_map = row_map;
+  if (row_map) return launch_rows<DOWN, false, true>(a, CfgMain::BN, (hipStream_t)stream);
   return launch_rows<DOWN>(a, CfgMain::BN, (hipStream_t)stream);
+}
+
+extern "C" int moe_gemm_down_fwd(const uint16_t* act, const uint16_t* w2, const int32_t* offs,
+                                 int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* y,
+                                 void* stream) {
+  return moe_gemm_down_to(act, w2, offs, E, R, H, I, y, nullptr, stream);
 }
 
 // Test hook: 0 lets every row-ragged launch choose its row-tile height (the default), 64, 128 or 256 forces it, 1
@@ -1310,15 +1329,16 @@ extern "C" int moe_gemm_dgrad_down_swiglu_bwd_packed(const uint16_t* dyp, const 
   return dgrad_down_impl(dyp, w2, g, u, offs, E, R, H, I, dgu, dgu ? dgu + I : nullptr, dgate_part, stream, 2 * I);
 }
 
-static int dgrad_gateup_impl(const uint16_t* dg, const uint16_t* du, int64_t ld_in, const uint16_t* w1,
-                             const uint16_t* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
-                             int64_t I, uint16_t* dxp, void* stream) {
+int moe_gemm_dgrad_gateup_to(const uint16_t* dg, const uint16_t* du, int64_t ld_in, const uint16_t* w1, const uint16_t* w3,
+                             const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* dxp,
+                             const int32_t* row_map, void* stream) {
   if (int rc = check_common(offs, E, R, H, I)) return rc;
   if (R == 0) return 0;
   MOE_CHECK_PTR(dg); MOE_CHECK_PTR(du); MOE_CHECK_PTR(w1); MOE_CHECK_PTR(w3); MOE_CHECK_PTR(dxp);
   GemmArgs a{};
   a.A0 = dg; a.A1 = du; a.B0 = w1; a.B1 = w3; a.C0 = dxp; a.offs = offs; a.ld_a = (int)ld_in;
-  a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I;
+  a.E = (int)E; a.R = (int)R; a.N = (int)H; a.K = (int)I; a.row_map = row_map;
+  if (row_map) return launch_rows<DGRAD_GATEUP, false, true>(a, CfgMain::BN, (hipStream_t)stream);
   return launch_rows<DGRAD_GATEUP>(a, CfgMain::BN, (hipStream_t)stream);
 }
 
@@ -1326,7 +1346,7 @@ extern "C" int moe_gemm_dgrad_gateup_packed(const uint16_t* dgu, const uint16_t*
                                             const int32_t* offs, int64_t E, int64_t R, int64_t H,
                                             int64_t I, uint16_t* dxp, void* stream) {
   if (R > 0 && !dgu) return MOE_ERR_NULL;
-  return dgrad_gateup_impl(dgu, dgu ? dgu + I : nullptr, 2 * I, w1, w3, offs, E, R, H, I, dxp, stream);
+  return moe_gemm_dgrad_gateup_to(dgu, dgu ? dgu + I : nullptr, 2 * I, w1, w3, offs, E, R, H, I, dxp, nullptr, stream);
 }
 
 extern "C" int moe_gemm_wgrad_pair(const uint16_t* dgu, const uint16_t* xp, const int32_t* offs, int64_t E,
@@ -1348,7 +1368,7 @@ extern "C" int moe_gemm_wgrad_pair(const uint16_t* dgu, const uint16_t* xp, cons
 extern "C" int moe_gemm_dgrad_gateup(const uint16_t* dg, const uint16_t* du, const uint16_t* w1,
                                      const uint16_t* w3, const int32_t* offs, int64_t E, int64_t R,
                                      int64_t H, int64_t I, uint16_t* dxp, void* stream) {
-  return dgrad_gateup_impl(dg, du, 0, w1, w3, offs, E, R, H, I, dxp, stream);
+  return moe_gemm_dgrad_gateup_to(dg, du, 0, w1, w3, offs, E, R, H, I, dxp, nullptr, stream);
 }
 
 extern "C" int moe_gemm_wgrad(const uint16_t* a_, const uint16_t* b_, const int32_t* offs, int64_t E,

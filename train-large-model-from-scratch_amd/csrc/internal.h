@@ -79,6 +79,15 @@ int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, fl
                              int64_t T, int64_t H, int64_t E, int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
                              int32_t* ids, float* gates, void* table, void* stream);
 
+// ---- grouped products (gemm.hip) ----
+// moe_gemm_down_fwd and moe_gemm_dgrad_gateup (ld_in: 0, or the row stride of dg and du) whose result's row of position p is row
+// row_map[p] (a permutation of the R rows; NULL: row p).
+int moe_gemm_down_to(const uint16_t* act, const uint16_t* w2, const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I,
+                     uint16_t* y, const int32_t* row_map, void* stream);
+int moe_gemm_dgrad_gateup_to(const uint16_t* dg, const uint16_t* du, int64_t ld_in, const uint16_t* w1, const uint16_t* w3,
+                             const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* dxp,
+                             const int32_t* row_map, void* stream);
+
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;
 constexpr int FEW_MAX_EXPERTS = 128;

@@ -22,8 +22,9 @@ struct RingTile {
 };
 
 // The tile of expert e, whose rows are first .. row_end, at its row `row` and column n0.  By the whole workgroup; `ring`: LDS bytes
-// of LDS that nobody else uses.  BLK: g and u are kept in blocks, as the kernels of larger tiles keep them (see there).
-template <int MODE, bool BLK, int FM, int WAVES>
+// of LDS that nobody else uses.  BLK: g and u are kept in blocks, as the kernels of larger tiles keep them; TO: the result's rows
+// go where p.row_map says (see there).
+template <int MODE, bool BLK, int FM, int WAVES, bool TO = false>
 __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, int first, int row_end, int row, int n0) {
   using O = RingTile<MODE, FM, WAVES>;
   using OpA = typename O::OpA;
@@ -55,6 +56,13 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
     if (p.K % 2048 == 0) ask_k = ((e * 13) & 31) * BK;
   }
   uint32_t ask_at = 0, at = 0;
+  // (TO) a lane a row of the wave's; asked for before the k-tiles, so that it has arrived when the first of them have
+  static_assert(!TO || FM <= 2, "a lane a row");
+  int row_to = 0;
+  if constexpr (TO) {
+    const int r = row0 + wm * 32 * FM + lane;
+    if (lane < 32 * FM && r < row_end) row_to = p.row_map[r];
+  }
   const auto ask = [&](bool live) {
     const int seg = NSEG == 2 && ask_seg, left = p.K - ask_k;
     opA.load(ring0 + ask_at, wv, ring_rsrc(vA[seg], (long long)ask_k * 2, live), left);
@@ -150,8 +158,8 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
     for (int it = 0; it < 32 / RPS; ++it) {
       const int rr = it * RPS + lane / CPS, ch = lane % CPS, col = col_w0 + ch * 8;
       const u32x4 v = *reinterpret_cast<const u32x4*>(strip + rr * STRIDE + perm(rr, ch) * 16);
-      if (strip_row + rr < rows && col < p.N)
-        *reinterpret_cast<u32x4*>((char*)base + ((long long)(row_w0 + strip_row + rr) * ldc + col) * 2) = v;
+      const int to = TO ? __shfl(row_to, strip_row + rr, MOE_WAVE) : row_w0 + strip_row + rr;
+      if (strip_row + rr < rows && col < p.N) *reinterpret_cast<u32x4*>((char*)base + ((long long)to * ldc + col) * 2) = v;
     }
   };
   if constexpr (MODE == GATEUP) {
