@@ -84,7 +84,7 @@ _GEMM_RHI = {"moe_gemm_gateup_swiglu_fwd": 4, "moe_gemm_gateup_swiglu_fwd_blocke
              "moe_gemm_dgrad_down_swiglu_bwd_dgate": 2, "moe_gemm_dgrad_down_swiglu_bwd_packed": 2,
              "moe_gemm_dgrad_down_swiglu_bwd_blocked": 2,
              "moe_gemm_dgrad_gateup": 4, "moe_gemm_dgrad_gateup_packed": 4, "moe_gemm_wgrad_pair": 4,
-             "moe_gemm_wgrad": 2, "moe_wgrad_multi": 6}
+             "moe_gemm_wgrad": 2, "moe_gemm_wgrad_all": 6, "moe_wgrad_multi": 6}
 
 
 def _launches_in_step(torch, P, step, steps, RHI, flops):

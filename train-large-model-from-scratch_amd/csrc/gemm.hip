@@ -1010,108 +1010,126 @@ __global__ __launch_bounds__(CfgHalf::NT, CfgHalf::WAVES_PER_SIMD) void small_ro
   walk_tiles<MODE, CfgHalf, OutT, BLK, CfgHalf::BM, TO>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
 }
 
-// Weight gradients.
+// Weight gradients: of up to three problems that share their experts' rows, one's tiles behind the other's without a launch
+// between them.  (What a launch's end, in which workgroups wait for the last ones, and the next one's start cost.  Whole steps, us,
+// a launch a problem and one: 9000 rows of 64 experts, 1024 <-> 1024, by Dirichlet's shares 443 -> 428; 4096 tokens, 8 of 128, 1024 <->
+// 256 459 -> 452; 450, 3 of 96, 3584 <-> 296 (three problems) 628 -> 616; 1558, 8 of 64 by Zipf's shares, 1792 <-> 1152 1014 -> 959; steps of a
+// few ms 1.00 to 1.02; of 24 layers one is slower by more than the noise, 160 tokens, 1 of 12, 3952 <-> 1936, 579 -> 581.)
+constexpr int WGRAD_PROBLEMS = 3;
+struct WgradArgs {
+  GemmArgs p[WGRAD_PROBLEMS];
+  int n;
+};
+// ---- which tiles a workgroup computes
+// The kernel is persistent: the grid has one workgroup per compute unit and each walks a
+// list of tiles.  Hardware hands workgroup b to XCD b % 8 (each XCD has its own L2).
+// With more tiles than workgroups: a tile of expert e contracts over that expert's rows,
+// so under skewed routing tiles differ in cost by orders of magnitude and a contiguous range is
+// all heavy or all light.  The (expert-major) list is dealt in groups of as many consecutive
+// tiles as an XCD has workgroups, group g to XCD g % 8, one tile to each of its workgroups: the
+// workgroups of an XCD stay on one expert (or two) and walk its rows together, and every XCD
+// sees every part of the list.  With at most 64 experts, whole groups per expert and skewed
+// routing (the largest expert above 1.25 times the mean) the groups are not dealt round-robin
+// but longest first: experts in descending order of their rows, each group to the XCD with the
+// least work so far; every workgroup works that out for itself from the offsets, the same way,
+// and keeps its own tiles' numbers in LDS.  (A generated power-law skew over 16 experts: 10-12 %
+// faster dealt in groups than with contiguous ranges of equal work, another 9-10 % longest
+// first; near-uniform routing: the same in all three.)  A tile of an expert costs the same in every problem: the next one's
+// groups are dealt on from where the last one's left the XCDs.
 template <typename OutT>
-__global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_gemm_kernel(const GemmArgs p) {
+__global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_gemm_kernel(const WgradArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   const int lane = threadIdx.x & 63;
-  // ---- which tiles this workgroup computes
-  // The kernel is persistent: the grid has one workgroup per compute unit and each walks a
-  // list of tiles.  Hardware hands workgroup b to XCD b % 8 (each XCD has its own L2).
-  // With more tiles than workgroups: a tile of expert e contracts over that expert's rows,
-  // so under skewed routing tiles differ in cost by orders of magnitude and a contiguous range is
-  // all heavy or all light.  The (expert-major) list is dealt in groups of as many consecutive
-  // tiles as an XCD has workgroups, group g to XCD g % 8, one tile to each of its workgroups: the
-  // workgroups of an XCD stay on one expert (or two) and walk its rows together, and every XCD
-  // sees every part of the list.  With at most 64 experts, whole groups per expert and skewed
-  // routing (the largest expert above 1.25 times the mean) the groups are not dealt round-robin
-  // but longest first: experts in descending order of their rows, each group to the XCD with the
-  // least work so far; every workgroup works that out for itself from the offsets, the same way,
-  // and keeps its own tiles' numbers in LDS.  (A generated power-law skew over 16 experts: 10-12 %
-  // faster dealt in groups than with contiguous ranges of equal work, another 9-10 % longest
-  // first; near-uniform routing: the same in all three.)
   constexpr int MAX_GROUPS = 512;
-  __shared__ uint32_t glist[MAX_GROUPS];
-  __shared__ int gcount;
-  int t_next, t_hi, t_step;
-  const uint32_t* list = nullptr;  // (given: positions in it, else tile numbers)
-  {
-    const int nb = gridDim.x, x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int nx = nb < 8 ? nb : 8;
-    t_step = (nb >> 3) + (x < (nb & 7) ? 1 : 0);
-    int lo;
-    if (p.E * p.m_slots * p.n_tiles > nb && (nb & 7) == 0) {
-      const int wgs = nb >> 3, TP = p.m_slots * p.n_tiles;
-      lo = x * wgs;
-      t_hi = p.E * TP;
-      t_step = nb;
-      if (p.E <= MOE_WAVE && TP % wgs == 0 && p.E * (TP / wgs) <= MAX_GROUPS) {
-        if (threadIdx.x < MOE_WAVE) {
-          const int gpe = TP / wgs;  // groups per expert
-          constexpr long long FIXED = 4 * CfgMain::BK;  // fill, tile switch and epilogue, in rows' worth
-          int rows = 0;
-          if (lane < p.E) {
-            rows = p.offs[lane + 1] - p.offs[lane];
-            rows = rows < 0 ? 0 : rows;
-          }
-          const long long cost = rows + FIXED;
-          // (only worth it when the routing is skewed: with near-equal experts the plain dealing is
-          // as balanced and keeps neighbouring experts on neighbouring XCDs)
-          int mx = rows, sum = rows;
+  __shared__ uint32_t glist[MAX_GROUPS];   // this XCD's groups, problem by problem
+  __shared__ int gcount[WGRAD_PROBLEMS];   // up to the end of each; -1: dealt round-robin
+  const int nb = gridDim.x, x = blockIdx.x & 7, j = blockIdx.x >> 3, wgs = nb >> 3;
+  const int E = a.p[0].E;
+  const auto tiles_of = [&](int w) { return a.p[w].m_slots * a.p[w].n_tiles; };  // of an expert
+  bool dealt = (nb & 7) == 0, ranked = E <= MOE_WAVE;
+  int groups = 0;
+  for (int w = 0; w < a.n; ++w) {
+    const int n = tiles_of(w);
+    dealt = dealt && E * n > nb;
+    ranked = ranked && dealt && n % wgs == 0;
+    if (ranked) groups += E * (n / wgs);
+  }
+  ranked = ranked && groups <= MAX_GROUPS;
+  if (ranked) {
+    if (threadIdx.x < MOE_WAVE) {
+      constexpr long long FIXED = 4 * CfgMain::BK;  // fill, tile switch and epilogue, in rows' worth
+      int rows = 0;
+      if (lane < E) {
+        rows = a.p[0].offs[lane + 1] - a.p[0].offs[lane];
+        rows = rows < 0 ? 0 : rows;
+      }
+      const long long cost = rows + FIXED;
+      // (only worth it when the routing is skewed: with near-equal experts the plain dealing is
+      // as balanced and keeps neighbouring experts on neighbouring XCDs)
+      int mx = rows, sum = rows;
 #pragma unroll
-          for (int off = MOE_WAVE / 2; off > 0; off >>= 1) {
-            const int om = __shfl_xor(mx, off, MOE_WAVE);
-            mx = om > mx ? om : mx;
-            sum += __shfl_xor(sum, off, MOE_WAVE);
-          }
-          const bool skewed = 4ll * mx * p.E > 5ll * sum;
-          int rank = 0;  // position of expert `lane` in descending order of cost (ties: lower index first)
-          for (int o = 0; o < p.E; ++o) {
-            const long long co = __shfl(cost, o, MOE_WAVE);
-            rank += (co > cost || (co == cost && o < lane)) ? 1 : 0;
-          }
-          if (lane >= p.E) rank = -1;
-          // lanes 0..7 carry the XCDs' loads, packed with the XCD index for the arg-min
-          long long load = 0;
-          int cnt = 0;
-          for (int s_ = 0; skewed && s_ < p.E; ++s_) {
-            const int e = __builtin_ctzll(__ballot(rank == s_));
-            const long long ce = __shfl(cost, e, MOE_WAVE);
-            for (int gi = 0; gi < gpe; ++gi) {
-              long long key = lane < 8 ? ((load << 3) | lane) : 0x7fffffffffffffffll;
+      for (int off = MOE_WAVE / 2; off > 0; off >>= 1) {
+        const int om = __shfl_xor(mx, off, MOE_WAVE);
+        mx = om > mx ? om : mx;
+        sum += __shfl_xor(sum, off, MOE_WAVE);
+      }
+      const bool skewed = 4ll * mx * E > 5ll * sum;
+      int rank = 0;  // position of expert `lane` in descending order of cost (ties: lower index first)
+      for (int o = 0; o < E; ++o) {
+        const long long co = __shfl(cost, o, MOE_WAVE);
+        rank += (co > cost || (co == cost && o < lane)) ? 1 : 0;
+      }
+      if (lane >= E) rank = -1;
+      // lanes 0..7 carry the XCDs' loads, packed with the XCD index for the arg-min
+      long long load = 0;
+      int cnt = 0;
+      for (int w = 0; skewed && w < a.n; ++w) {
+        const int gpe = tiles_of(w) / wgs;  // groups per expert
+        for (int s_ = 0; s_ < E; ++s_) {
+          const int e = __builtin_ctzll(__ballot(rank == s_));
+          const long long ce = __shfl(cost, e, MOE_WAVE);
+          for (int gi = 0; gi < gpe; ++gi) {
+            long long key = lane < 8 ? ((load << 3) | lane) : 0x7fffffffffffffffll;
 #pragma unroll
-              for (int off = 1; off < 8; off <<= 1) {
-                const long long other = __shfl_xor(key, off, MOE_WAVE);
-                key = other < key ? other : key;
-              }
-              const int xmin = (int)(__shfl(key, 0, MOE_WAVE) & 7);
-              if (lane == xmin) load += ce;
-              if (xmin == x) {
-                if (lane == 0) glist[cnt] = (e * gpe + gi) * wgs + j;
-                ++cnt;
-              }
+            for (int off = 1; off < 8; off <<= 1) {
+              const long long other = __shfl_xor(key, off, MOE_WAVE);
+              key = other < key ? other : key;
+            }
+            const int xmin = (int)(__shfl(key, 0, MOE_WAVE) & 7);
+            if (lane == xmin) load += ce;
+            if (xmin == x) {
+              if (lane == 0) glist[cnt] = (e * gpe + gi) * wgs + j;
+              ++cnt;
             }
           }
-          if (lane == 0) gcount = skewed ? cnt : -1;
         }
-        __syncthreads();
-        const int cnt = gcount;
-        if (cnt >= 0) {
-          t_hi = cnt;
-          lo = -j;
-          t_step = 1;
-          list = glist;
-        }
+        if (lane == 0) gcount[w] = cnt;
       }
-    } else {
-      const int total = p.E * p.m_slots * p.n_tiles;
-      const int q = total / nx, r = total % nx;
-      lo = x * q + (x < r ? x : r);
-      t_hi = lo + q + (x < r ? 1 : 0);
+      if (lane == 0 && !skewed) gcount[0] = -1;
     }
-    t_next = lo + j;
+    __syncthreads();
+    ranked = gcount[0] >= 0;
   }
-  walk_tiles<WGRAD, CfgMain, OutT, false>(p, smem, nullptr, p.offs, list, t_next, t_hi, t_step);
+  int done = 0;  // tiles of the problems before
+#pragma unroll 1
+  for (int w = 0; w < a.n; ++w) {
+    const GemmArgs p = a.p[w];  // (in registers: read where it is used, a tile of one k-tile is 1 % longer)
+    const int total = E * tiles_of(w);
+    int first, end, step;
+    if (ranked) {
+      first = w ? gcount[w - 1] : 0, end = gcount[w], step = 1;
+    } else if (dealt) {
+      // (a problem begins with the workgroups, in whole XCDs, that have one tile less of those before)
+      const int skip = done % nb / wgs * wgs, at = x * wgs + j;
+      first = at >= skip ? at - skip : at - skip + nb, end = total, step = nb;
+    } else {
+      const int nx = nb < 8 ? nb : 8, q = total / nx, r = total % nx, lo = x * q + (x < r ? x : r);
+      first = lo + j, end = lo + q + (x < r ? 1 : 0), step = (nb >> 3) + (x < (nb & 7) ? 1 : 0);
+    }
+    if (w) __syncthreads();  // (the operand stages are free)
+    walk_tiles<WGRAD, CfgMain, OutT, false>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
+    done += total;
+  }
 }
 
 }  // namespace
@@ -1131,8 +1149,8 @@ namespace {
 
 
 // As many workgroups as are resident at once (one per compute unit), or as there are jobs.
-template <int MODE, typename Cfg>
-int launch(void (*kern)(GemmArgs), bool (&attr_done)[MOE_MAX_DEVICES], const GemmArgs& a, long long jobs, hipStream_t s) {
+template <int MODE, typename Cfg, typename Args>
+int launch(void (*kern)(Args), bool (&attr_done)[MOE_MAX_DEVICES], const Args& a, long long jobs, hipStream_t s) {
   if (jobs <= 0) return 0;
   constexpr int LDS = lds_bytes<MODE, Cfg>();
   const int dev = moe_current_device();
@@ -1177,19 +1195,26 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK, TO>, attr_done[1], a,
                                2 * a.n_tiles * row_slots(a.R, a.E, ROW_TILE), s);
 }
+// Nothing here reads the results again.  With few rows an expert they come as fast as the operands do, and as streaming
+// stores they leave the operands' lines in L2 alone.  Rows an expert and time, streaming over ordinary, three results in
+// turn so that none is still cached: 64 experts of 2048 <-> 1024, bf16 and fp32: 256, 0.86 and 0.83; 512, 0.93 and 0.91; 768, 1.01 and 1.04;
+// 1024, 1.00 and 1.01; 2048, 1.00 and 1.00.  128 of 1024 <-> 256, 128 to 512 rows 0.93 to 0.96 and 0.84 to 0.92; 16 of 4096 <-> 1536, 1024 rows
+// 0.95 and 0.95; by Zipf's shares, 500 rows of 64 1.00 and 0.85.
+// (as for wgrad_multi_kernel: rows of whole pieces of 64 bytes)
 template <typename OutT>
-int launch_wgrad(GemmArgs& a, hipStream_t s) {
-  a.n_tiles = (a.N + CfgMain::BN - 1) / CfgMain::BN;
-  a.m_slots = (a.M + CfgMain::BM - 1) / CfgMain::BM;
-  // Nothing here reads the results again.  With few rows an expert they come as fast as the operands do, and as streaming
-  // stores they leave the operands' lines in L2 alone.  Rows an expert and time, streaming over ordinary, three results in
-  // turn so that none is still cached: 64 experts of 2048 <-> 1024, bf16 and fp32: 256, 0.86 and 0.83; 512, 0.93 and 0.91; 768, 1.01 and 1.04;
-  // 1024, 1.00 and 1.01; 2048, 1.00 and 1.00.  128 of 1024 <-> 256, 128 to 512 rows 0.93 to 0.96 and 0.84 to 0.92; 16 of 4096 <-> 1536, 1024 rows
-  // 0.95 and 0.95; by Zipf's shares, 500 rows of 64 1.00 and 0.85.
-  // (as for wgrad_multi_kernel: rows of whole pieces of 64 bytes)
-  a.streaming = a.R <= 512ll * a.E && a.N * (int)sizeof(OutT) % 64 == 0;
+int launch_wgrad(const WgradArgs& args, hipStream_t s) {
+  WgradArgs w = args;
+  long long tiles = 0;
+  for (int i = 0; i < w.n; ++i) {
+    GemmArgs& a = w.p[i];
+    a.n_tiles = (a.N + CfgMain::BN - 1) / CfgMain::BN;
+    a.m_slots = (a.M + CfgMain::BM - 1) / CfgMain::BM;
+    a.streaming = a.R <= 512ll * a.E && a.N * (int)sizeof(OutT) % 64 == 0;
+    const long long n = (long long)a.n_tiles * a.m_slots * a.E;
+    tiles = tiles > n ? tiles : n;
+  }
   static bool attr_done[MOE_MAX_DEVICES];
-  return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT>, attr_done, a, (long long)a.n_tiles * a.m_slots * a.E, s);
+  return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT>, attr_done, w, tiles, s);
 }
 
 int check_common(const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I) {
@@ -1349,20 +1374,56 @@ extern "C" int moe_gemm_dgrad_gateup_packed(const uint16_t* dgu, const uint16_t*
   return moe_gemm_dgrad_gateup_to(dgu, dgu ? dgu + I : nullptr, 2 * I, w1, w3, offs, E, R, H, I, dxp, nullptr, stream);
 }
 
-extern "C" int moe_gemm_wgrad_pair(const uint16_t* dgu, const uint16_t* xp, const int32_t* offs, int64_t E,
-                                   int64_t R, int64_t I, int64_t H, void* dw1, void* dw3, int dw_dtype,
-                                   int accumulate, void* stream) {
+static int wgrad_pair_args(GemmArgs& a, const uint16_t* dgu, const uint16_t* xp, const int32_t* offs, int64_t E, int64_t R,
+                           int64_t I, int64_t H, void* dw1, void* dw3, int dw_dtype, int accumulate) {
   if (int rc = check_common(offs, E, R, I, H)) return rc;  // (the stacked result has 2*I <= 131072 rows)
   // a 256-row tile of the stacked result must not straddle the two halves
   if ((I % CfgMain::BM) != 0) return MOE_ERR_SHAPE;
   MOE_CHECK_PTR(dw1); MOE_CHECK_PTR(dw3);
   if (R > 0) { MOE_CHECK_PTR(dgu); MOE_CHECK_PTR(xp); }
   if (dw_dtype != MOE_DT_BF16 && dw_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
-  GemmArgs a{};
+  a = {};
   a.A0 = dgu; a.B0 = xp; a.C0 = dw1; a.C1 = dw3; a.offs = offs; a.m_split = (int)I;
   a.E = (int)E; a.R = (int)R; a.M = (int)(2 * I); a.N = (int)H; a.accumulate = accumulate;
-  return dw_dtype == MOE_DT_F32 ? launch_wgrad<float>(a, (hipStream_t)stream)
-                                : launch_wgrad<uint16_t>(a, (hipStream_t)stream);
+  return 0;
+}
+
+static int wgrad_args(GemmArgs& a, const uint16_t* a_, const uint16_t* b_, const int32_t* offs, int64_t E, int64_t R, int64_t M,
+                      int64_t N, void* dw, int dw_dtype, int accumulate) {
+  if (int rc = check_common(offs, E, R, M, N)) return rc;
+  MOE_CHECK_PTR(dw);
+  if (R > 0) { MOE_CHECK_PTR(a_); MOE_CHECK_PTR(b_); }
+  if (dw_dtype != MOE_DT_BF16 && dw_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
+  a = {};
+  a.A0 = a_; a.B0 = b_; a.C0 = dw; a.offs = offs;
+  a.E = (int)E; a.R = (int)R; a.M = (int)M; a.N = (int)N; a.accumulate = accumulate;
+  return 0;
+}
+
+static int run_wgrad(const WgradArgs& w, int dw_dtype, void* stream) {
+  return dw_dtype == MOE_DT_F32 ? launch_wgrad<float>(w, (hipStream_t)stream) : launch_wgrad<uint16_t>(w, (hipStream_t)stream);
+}
+
+extern "C" int moe_gemm_wgrad_pair(const uint16_t* dgu, const uint16_t* xp, const int32_t* offs, int64_t E,
+                                   int64_t R, int64_t I, int64_t H, void* dw1, void* dw3, int dw_dtype,
+                                   int accumulate, void* stream) {
+  WgradArgs w{};
+  w.n = 1;
+  if (int rc = wgrad_pair_args(w.p[0], dgu, xp, offs, E, R, I, H, dw1, dw3, dw_dtype, accumulate)) return rc;
+  return run_wgrad(w, dw_dtype, stream);
+}
+
+int moe_gemm_wgrad_all(const MoeWgradStack* stacks, int n, const int32_t* offs, int64_t E, int64_t R, void* stream) {
+  WgradArgs w{};
+  if (n < 1 || n > WGRAD_PROBLEMS) return MOE_ERR_LIMIT;
+  for (; w.n < n; ++w.n) {
+    const MoeWgradStack& m = stacks[w.n];
+    if (m.dtype != stacks[0].dtype) return MOE_ERR_DTYPE;
+    const int rc = m.out2 ? wgrad_pair_args(w.p[w.n], m.a, m.b, offs, E, R, m.M / 2, m.N, m.out, m.out2, m.dtype, m.accumulate)
+                          : wgrad_args(w.p[w.n], m.a, m.b, offs, E, R, m.M, m.N, m.out, m.dtype, m.accumulate);
+    if (rc) return rc;
+  }
+  return run_wgrad(w, stacks[0].dtype, stream);
 }
 
 extern "C" int moe_gemm_dgrad_gateup(const uint16_t* dg, const uint16_t* du, const uint16_t* w1,
@@ -1374,13 +1435,8 @@ extern "C" int moe_gemm_dgrad_gateup(const uint16_t* dg, const uint16_t* du, con
 extern "C" int moe_gemm_wgrad(const uint16_t* a_, const uint16_t* b_, const int32_t* offs, int64_t E,
                               int64_t R, int64_t M, int64_t N, void* dw, int dw_dtype,
                               int accumulate, void* stream) {
-  if (int rc = check_common(offs, E, R, M, N)) return rc;
-  MOE_CHECK_PTR(dw);
-  if (R > 0) { MOE_CHECK_PTR(a_); MOE_CHECK_PTR(b_); }
-  if (dw_dtype != MOE_DT_BF16 && dw_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
-  GemmArgs a{};
-  a.A0 = a_; a.B0 = b_; a.C0 = dw; a.offs = offs;
-  a.E = (int)E; a.R = (int)R; a.M = (int)M; a.N = (int)N; a.accumulate = accumulate;
-  return dw_dtype == MOE_DT_F32 ? launch_wgrad<float>(a, (hipStream_t)stream)
-                                : launch_wgrad<uint16_t>(a, (hipStream_t)stream);
+  WgradArgs w{};
+  w.n = 1;
+  if (int rc = wgrad_args(w.p[0], a_, b_, offs, E, R, M, N, dw, dw_dtype, accumulate)) return rc;
+  return run_wgrad(w, dw_dtype, stream);
 }

@@ -42,7 +42,10 @@ struct MoeWgradStack {
   float* part;
   int64_t lda, ldb, M, N;
   int dtype, accumulate;
+  void* out2;  // moe_gemm_wgrad_all: an expert's rows M / 2 .. M - 1 go here (NULL: all to out)
 };
+// moe_gemm_wgrad, and moe_gemm_wgrad_pair where there is an out2, of up to three stacks with results of one kind in one launch.
+int moe_gemm_wgrad_all(const MoeWgradStack* stacks, int n, const int32_t* offs, int64_t E, int64_t R, void* stream);
 // Bytes of each stack's part for R rows.
 int64_t moe_wgrad_multi_part_bytes(int64_t R, int64_t H, int64_t I);
 // The stacks (the first n_stacks, all of the size I x H or H x I; without any, offs may be NULL) and, unless NULL, the router: a [T, M >= E] and b
@@ -87,7 +90,6 @@ int moe_gemm_down_to(const uint16_t* act, const uint16_t* w2, const int32_t* off
 int moe_gemm_dgrad_gateup_to(const uint16_t* dg, const uint16_t* du, int64_t ld_in, const uint16_t* w1, const uint16_t* w3,
                              const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* dxp,
                              const int32_t* row_map, void* stream);
-
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;
 constexpr int FEW_MAX_EXPERTS = 128;

@@ -487,7 +487,7 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
   const bool router_dw = router && to_logits && a->dwr;
   if (router_dw && a->dlogits) return MOE_ERR_SHAPE;  // one or the other: the caller's dlogits are not padded
   // weight gradients, down projection first: [dyp | act], [dg | xp], [du | xp]
-  MoeWgradStack stacks[3], rstack{};
+  MoeWgradStack stacks[3]{}, rstack{};
   int n_stacks = 0;
   for (int w : {2, 0, 1}) {
     if (!a->dw[w]) continue;
@@ -501,6 +501,11 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     m.part = ws.wpart[w];
     m.dtype = (int)a->dw_dtype[w];
     m.accumulate = a->dw_accumulate[w] ? 1 : 0;
+    if (pair && w == 0) {  // the up stack's rows are the ones behind
+      m.M = m.lda = 2 * I;
+      m.out2 = a->dw[1];
+      break;
+    }
   }
   if (router_dw) {
     rstack.a = ws.dlogits, rstack.b = a->xn, rstack.out = a->dwr, rstack.part = ws.rpart;
@@ -512,15 +517,14 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
       MOE_STEP("moe_wgrad_multi", moe_wgrad_multi(stacks, n_stacks, router_dw ? &rstack : nullptr, a->offs, E, R, H, I, T,
                                                   rs.slices, rs.rows, st));
   } else {
-    for (int i = 0; i < n_stacks; ++i) {
-      const MoeWgradStack& m = stacks[i];
-      if (pair && m.out == a->dw[0]) {
-        MOE_STEP("moe_gemm_wgrad_pair", moe_gemm_wgrad_pair(dg, a->xp, a->offs, E, R, I, H, a->dw[0], a->dw[1], m.dtype,
-                                                            m.accumulate, stream));
-        ++i;  // the up stack's came with it
-        continue;
-      }
-      MOE_STEP("moe_gemm_wgrad", moe_gemm_wgrad(m.a, m.b, a->offs, E, R, m.M, m.N, m.out, m.dtype, m.accumulate, stream));
+    bool one_kind = true;
+    for (int i = 1; i < n_stacks; ++i) one_kind = one_kind && stacks[i].dtype == stacks[0].dtype;
+    if (one_kind && n_stacks > 1) {
+      MOE_STEP("moe_gemm_wgrad_all", moe_gemm_wgrad_all(stacks, n_stacks, a->offs, E, R, stream));
+    } else {
+      for (int i = 0; i < n_stacks; ++i)
+        MOE_STEP(stacks[i].out2 ? "moe_gemm_wgrad_pair" : "moe_gemm_wgrad",
+                 moe_gemm_wgrad_all(stacks + i, 1, a->offs, E, R, stream));
     }
     if (router_dw)
       MOE_STEP("moe_router_wgrad",
