@@ -58,6 +58,18 @@ constexpr int lds_bytes() {
 constexpr int GEMM_MAX_E = 1024;  // per-expert tile prefix lives in LDS
 constexpr int ROW_TILE = 256;     // rows of a tile of the row-ragged modes
 
+// The expert of a row-tile slot, the last e with tile_start[e] <= slot (which skips those without rows), by a whole wave for a slot
+// that its lanes share: a count over the lanes and one trip to LDS, two past 64 experts, where a search takes seven, one after the
+// other.  (tile_start as number_tiles leaves it.  With number_tiles' single trip and the divisions by multiplication, us: a training pass of
+// 4096 tokens, 8 of 128 experts, 1024 <-> 256, 419.1 -> 412.0; 8192, 2 of 8, 1024 <-> 512, 303.4 -> 300.1; a prefill of 1531, 8 of 64, 238.7 -> 237.2.)
+__device__ __forceinline__ int expert_of(const int* tile_start, int slot, int E) {
+  const int lane = lane_id();
+  int n = 0;
+#pragma unroll 2
+  for (int b = 0; b < E; b += MOE_WAVE) n += __popcll(__ballot(tile_start[b + lane] <= slot));
+  return n - 1;
+}
+
 // BLK (GATEUP and DGRAD_DOWN only): g and u, which nothing but the SwiGLU backward reads, are kept
 // in a layout private to the library instead of as [R, I] rows: one 4 KB record per 32 x 32 block
 // of a row tile, holding the block exactly as the matrix cores leave it in a wave's accumulators
@@ -116,26 +128,19 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   // Every lane computes the same thing from the same LDS words / scalar loads.
   auto locate = [&](uint32_t entry, Tile& t) -> bool {
     constexpr bool HALF = MODE != WGRAD && BM < UNIT;
-    const uint32_t logical = HALF ? entry >> 1 : entry;
-    const int n_tile = (int)(logical % (uint32_t)p.n_tiles);
-    const int slot = (int)(logical / (uint32_t)p.n_tiles);
+    const int logical = (int)(HALF ? entry >> 1 : entry);
+    const int slot = p.by_n_tiles(logical), n_tile = logical - slot * p.n_tiles;
     t.m0 = 0;
     if constexpr (MODE == WGRAD) {
-      t.e = slot / p.m_slots;
-      t.m0 = (slot % p.m_slots) * BM;
+      t.e = p.by_m_slots(slot);
+      t.m0 = (slot - t.e * p.m_slots) * BM;
       t.row0 = offs[t.e];
       t.row_end = offs[t.e + 1];
     } else {
       if (slot >= tile_start[p.E]) return false;
-      int lo = 0, hi = p.E;  // largest e with tile_start[e] <= slot (skips empty experts)
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (tile_start[mid] <= slot) lo = mid;
-        else hi = mid;
-      }
-      t.e = __builtin_amdgcn_readfirstlane(lo);
+      t.e = expert_of(tile_start, slot, p.E);
       const int off = __builtin_amdgcn_readfirstlane(offs[t.e]);
-      int in_expert = (slot - __builtin_amdgcn_readfirstlane(tile_start[lo])) * UNIT;
+      int in_expert = (slot - __builtin_amdgcn_readfirstlane(tile_start[t.e])) * UNIT;
       if (HALF) in_expert += (int)(entry & 1) * BM;
       t.row0 = off + in_expert;
       t.row_end = __builtin_amdgcn_readfirstlane(offs[t.e + 1]);
@@ -835,28 +840,32 @@ using CfgMain = TileCfg<ROW_TILE, 256, 64, 2, 4>;
 // Row tiles of half the height (the eight waves 64 x 64 each), at 0.65 to 0.7 of a tile's cost.
 using CfgHalf = TileCfg<ROW_TILE / 2, 256, 64, 2, 4>;
 
-// tile_start[e] = number of tiles of UNIT rows of the experts before e, offs = p.offs, both in LDS (wave 0 scans).
+// tile_start[e] = number of tiles of UNIT rows of the experts before e (and of all from E up to the next multiple of 64 on), offs =
+// p.offs, both in LDS (wave 0 scans, two experts a lane: past 64 of them one trip to memory instead of two, 2.2 -> 1.3 us
+// from the kernel's start).
 template <int UNIT>
 __device__ __forceinline__ void number_tiles(const GemmArgs& p, int* tile_start, int* offs) {
   const int lane = threadIdx.x & 63;
   if (threadIdx.x < MOE_WAVE) {
     int carry = 0;
-    for (int b = 0; b < p.E; b += MOE_WAVE) {
-      const int e = b + lane;
-      const int first = e < p.E ? p.offs[e] : 0, end = e < p.E ? p.offs[e + 1] : 0;
-      const int nt = (end - first + UNIT - 1) / UNIT;
-      int incl = nt;
+    for (int b = 0; b < p.E; b += 2 * MOE_WAVE) {
+      int first[2], end[2];
 #pragma unroll
-      for (int off = 1; off < MOE_WAVE; off <<= 1) {
-        const int o = __shfl_up(incl, off, MOE_WAVE);
-        if (lane >= off) incl += o;
+      for (int h = 0; h < 2; ++h) {
+        const int e = b + h * MOE_WAVE + lane;
+        first[h] = e < p.E ? p.offs[e] : 0, end[h] = e < p.E ? p.offs[e + 1] : 0;
       }
-      if (e < p.E) {
-        tile_start[e] = carry + incl - nt;
-        offs[e] = first;
-        if (e == p.E - 1) offs[p.E] = end;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int e = b + h * MOE_WAVE + lane;
+        const int nt = (end[h] - first[h] + UNIT - 1) / UNIT, incl = wave_inclusive(nt);
+        if (e < GEMM_MAX_E) tile_start[e] = carry + incl - nt;
+        if (e < p.E) {
+          offs[e] = first[h];
+          if (e == p.E - 1) offs[p.E] = end[h];
+        }
+        carry += read_lane(incl, MOE_WAVE - 1);
       }
-      carry += __shfl(incl, MOE_WAVE - 1, MOE_WAVE);
     }
     if (lane == 0) tile_start[p.E] = carry;
   }
@@ -916,7 +925,7 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
     const bool last = tile >= total - left;
     int n = 0, n4 = 0;  // this tile's halves and quarters with rows
     if (tile < total) {
-      const int slot = tile / p.n_tiles;
+      const int slot = p.by_n_tiles(tile);
       int e = 0, hi = p.E;
       while (hi - e > 1) {
         const int mid = (e + hi) >> 1;
@@ -980,17 +989,11 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
       using Quarter = RingTile<MODE, 1, CfgMain::NT / MOE_WAVE>;
       static_assert(Quarter::LDS <= lds_bytes<MODE, CfgMain>() && Quarter::BM * 4 == ROW_TILE, "fits");
       for (int at = h.first; at < h.end; at += h.step) {
-        const int entry = __builtin_amdgcn_readfirstlane((int)half_list[at]), tile = entry >> 2, slot = tile / p.n_tiles;
-        int e = 0, hi = p.E;
-        while (hi - e > 1) {
-          const int mid = (e + hi) >> 1;
-          if (tile_start[mid] <= slot) e = mid;
-          else hi = mid;
-        }
-        e = __builtin_amdgcn_readfirstlane(e);
+        const int entry = __builtin_amdgcn_readfirstlane((int)half_list[at]), tile = entry >> 2, slot = p.by_n_tiles(tile);
+        const int e = expert_of(tile_start, slot, p.E);
         const int first = __builtin_amdgcn_readfirstlane(offs[e]), end = __builtin_amdgcn_readfirstlane(offs[e + 1]);
         const int row = (slot - __builtin_amdgcn_readfirstlane(tile_start[e])) * ROW_TILE + (entry & 3) * Quarter::BM;
-        ring_tile<MODE, BLK, 1, WAVES, TO>(p, (char*)smem, e, first, end, row, tile % p.n_tiles * Quarter::BNC);
+        ring_tile<MODE, BLK, 1, WAVES, TO>(p, (char*)smem, e, first, end, row, (tile - slot * p.n_tiles) * Quarter::BNC);
         __syncthreads();
       }
       return;
@@ -1184,6 +1187,7 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
       moe_ring_rows((Mode)MODE, BLK, a, forced_row_tile == RING_TALL ? 128 : forced_row_tile, s, &rc))
     return rc;
   a.n_tiles = (a.N + cols - 1) / cols;
+  a.by_n_tiles.set(a.n_tiles);
   const long long tiles = row_slots(a.R, a.E, ROW_TILE) * ((a.N + CfgMain::BN - 1) / CfgMain::BN);
   const bool small = forced_row_tile > RING_TILE ? forced_row_tile == CfgHalf::BM
                                                  : 2 * tiles < moe_compute_units() &&
@@ -1209,6 +1213,7 @@ int launch_wgrad(const WgradArgs& args, hipStream_t s) {
     GemmArgs& a = w.p[i];
     a.n_tiles = (a.N + CfgMain::BN - 1) / CfgMain::BN;
     a.m_slots = (a.M + CfgMain::BM - 1) / CfgMain::BM;
+    a.by_n_tiles.set(a.n_tiles), a.by_m_slots.set(a.m_slots);
     a.streaming = a.R <= 512ll * a.E && a.N * (int)sizeof(OutT) % 64 == 0;
     const long long n = (long long)a.n_tiles * a.m_slots * a.E;
     tiles = tiles > n ? tiles : n;

@@ -4,6 +4,19 @@
 
 enum Mode { GATEUP = 0, DOWN = 1, DGRAD_DOWN = 2, DGRAD_GATEUP = 3, WGRAD = 4 };
 
+// Division of 0 <= n < 2^31 by a divisor that the host knows, n * m >> s: m = floor(2^s / d) + 1 with s = 31 + ceil(log2 d) is exact there
+// (Granlund and Montgomery), as n * (m * d - 2^s) < 2^s.  A dozen cycles where the general one takes a few hundred.
+struct Divisor {
+  uint32_t m;
+  int s;
+  void set(uint32_t d) {
+    s = 31;
+    while ((1ull << (s - 31)) < d) ++s;
+    m = (uint32_t)((1ull << s) / d + 1);
+  }
+  __device__ __forceinline__ int operator()(int n) const { return (int)(((unsigned long long)(uint32_t)n * m) >> s); }
+};
+
 struct GemmArgs {
   const uint16_t* A0;
   const uint16_t* A1;
@@ -22,6 +35,7 @@ struct GemmArgs {
   int K;        // contraction length per segment (not used by WGRAD)
   int n_tiles;  // tiles along N
   int m_slots;  // row-tile slots (ragged modes) or tiles along M (WGRAD)
+  Divisor by_n_tiles, by_m_slots;  // (gemm.hip; m_slots: WGRAD only)
   int accumulate;
   int ld_a;     // row stride of A0/A1 in elements when it is not the contraction length (0: K)
   int ld_c;     // row stride of the outputs C0/C1 in elements when it is not N (0: N)
