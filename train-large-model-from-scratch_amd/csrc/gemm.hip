@@ -59,14 +59,16 @@ constexpr int GEMM_MAX_E = 1024;  // per-expert tile prefix lives in LDS
 constexpr int ROW_TILE = 256;     // rows of a tile of the row-ragged modes
 
 // The expert of a row-tile slot, the last e with tile_start[e] <= slot (which skips those without rows), by a whole wave for a slot
-// that its lanes share: a count over the lanes and one trip to LDS, two past 64 experts, where a search takes seven, one after the
+// that its lanes share: a count over the lanes and one trip to LDS for 128 experts, where a search takes seven, one after the
 // other.  (tile_start as number_tiles leaves it.  With number_tiles' single trip and the divisions by multiplication, us: a training pass of
 // 4096 tokens, 8 of 128 experts, 1024 <-> 256, 419.1 -> 412.0; 8192, 2 of 8, 1024 <-> 512, 303.4 -> 300.1; a prefill of 1531, 8 of 64, 238.7 -> 237.2.)
 __device__ __forceinline__ int expert_of(const int* tile_start, int slot, int E) {
   const int lane = lane_id();
   int n = 0;
-#pragma unroll 2
-  for (int b = 0; b < E; b += MOE_WAVE) n += __popcll(__ballot(tile_start[b + lane] <= slot));
+  for (int b = 0; b < E; b += 2 * MOE_WAVE) {
+    const int first = tile_start[b + lane], second = tile_start[b + MOE_WAVE + lane];
+    n += __popcll(__ballot(first <= slot)) + __popcll(__ballot(second <= slot));
+  }
   return n - 1;
 }
 
@@ -840,7 +842,7 @@ using CfgMain = TileCfg<ROW_TILE, 256, 64, 2, 4>;
 // Row tiles of half the height (the eight waves 64 x 64 each), at 0.65 to 0.7 of a tile's cost.
 using CfgHalf = TileCfg<ROW_TILE / 2, 256, 64, 2, 4>;
 
-// tile_start[e] = number of tiles of UNIT rows of the experts before e (and of all from E up to the next multiple of 64 on), offs =
+// tile_start[e] = number of tiles of UNIT rows of the experts before e (and of all from E up to the next multiple of 128 on), offs =
 // p.offs, both in LDS (wave 0 scans, two experts a lane: past 64 of them one trip to memory instead of two, 2.2 -> 1.3 us
 // from the kernel's start).
 template <int UNIT>
