@@ -40,6 +40,12 @@ int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, fl
 int moe_selected_layer_forward(const moe_layer_forward_args* a, const void* table, void* stream);
 int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
                    int64_t I, float* g, float* u, float* act, void* stream);
+int moe_f32_permute_bwd_router(const float* dxp, const int32_t* row_to_pos, const float* gates, const float* dgates,
+                               const int32_t* ids, const float* wr, int64_t T, int64_t H, int64_t k, float* dsel, float* dx,
+                               void* stream);
+int moe_f32_router_wgrad_slices(int64_t R, int64_t H, int64_t E);
+int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs, int64_t R, int64_t H, int64_t E, float* part,
+                         float* dwr, void* stream);
 int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
                    int64_t E, int64_t R, int64_t H, int64_t I, float* dw1, float* dw3, float* dw2, void* stream);
 int moe_routed_forward(const uint16_t* x, const uint16_t* wr, uint16_t* logits, const float* bias, const uint16_t* w1,
@@ -618,11 +624,11 @@ struct KeptF32 {
 };
 
 struct OutputsF32 {
-  Tensor out, routing, kept, w[3];
+  Tensor out, routing, kept, w[3], logits;
 };
 
-OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, const Tensor& w1, const Tensor& w3,
-                       const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
+OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& wr, const Tensor& logits_, const Tensor& w1,
+                       const Tensor& w3, const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
   OutputsF32 f;
   need_gpu(x_);
   TORCH_CHECK(x_.dim() == 2 && w1.dim() == 3, "the layer takes x [tokens, hidden] and weights [experts, ., .]");
@@ -630,9 +636,22 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
   TORCH_CHECK(w3.size(0) == E && w2.size(0) == E && w1.size(2) == H && w3.size(2) == H && w3.size(1) == I &&
                   w2.size(1) == H && w2.size(2) == I,
               "the weights' shapes do not belong together");
+  if (wr.defined()) {
+    need_gpu(wr);
+    TORCH_CHECK(wr.dim() == 2 && wr.size(0) == E && wr.size(1) == H, "the router weight has shape ", wr.sizes(), ", x ", x_.sizes(),
+                " and there are ", E, " experts");
+    TORCH_CHECK(wr.device() == x_.device(), "the router weight is on ", wr.device(), ", x on ", x_.device());
+    TORCH_CHECK_TYPE(wr.scalar_type() == at::kFloat && x_.scalar_type() == at::kFloat, "x and the router weight must be fp32");
+  }
   check_logits(logits_, bias, x_, E);
   const c10::DeviceGuard guard(x_.device());
   const Tensor x = dense(x_);
+  if (wr.defined()) {
+    const NoAutocast off;
+    f.logits = at::mm(x, wr.t());
+  } else {
+    f.logits = logits_;
+  }
   f.w[0] = dense(w1), f.w[1] = dense(w3), f.w[2] = dense(w2);
   void* s = stream_of(x);
   const Routing r(R, E);
@@ -643,7 +662,7 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
   float* base = f.kept.data_ptr<float>();
   float *xp = base, *g = base + kept.g, *u = base + kept.u, *act = base + kept.act, *y = base + kept.y;
   float* gates = nullptr;
-  const bool place = logits_.defined() && H % 8 == 0 && moe_place_ok(T, E, k);
+  const bool place = f.logits.defined() && H % 8 == 0 && moe_place_ok(T, E, k);
   const int64_t wsb = std::max<int64_t>(place ? moe_place_bytes(T, E) : moe_dispatch_workspace_bytes(R, E), 16);
   const Tensor ws = empty({wsb}, at::kByte, x);
   int32_t* counts = r.part(f.routing, Routing::COUNTS);
@@ -652,8 +671,8 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
   int32_t* r2p = r.part(f.routing, Routing::ROW_TO_POS);
   int32_t* ids = r.part(f.routing, Routing::IDS);
   Tensor logits, b;
-  if (logits_.defined()) {
-    logits = dense(logits_);
+  if (f.logits.defined()) {
+    logits = dense(f.logits);
     if (bias.defined()) b = dense(bias);
     gates = (float*)r.part(f.routing, Routing::GATES);
   }
@@ -688,33 +707,52 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, 
 }
 
 struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
-  enum Input { X, LOGITS, W1, W3, W2, BIAS, IDS, OPTIONS, INPUTS };
+  enum Input { X, WR, LOGITS, W1, W3, W2, BIAS, IDS, OPTIONS, INPUTS };
 
-  static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& logits_, const Tensor& w1,
-                               const Tensor& w3, const Tensor& w2, const OptTensor& bias_, const OptTensor& ids_,
-                               const Layer& o) {
-    const Tensor &logits = value(logits_), &bias = value(bias_), &ids = value(ids_);
-    const OutputsF32 f = forward_f32(o, x, logits, w1, w3, w2, bias, ids);
-    ctx->save_for_backward({f.kept, f.routing, f.w[0], f.w[1], f.w[2]});
-    ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), o.k, logits.defined(),
-                                                Present{true, logits.defined(), true, true, true, bias.defined(),
-                                                        ids.defined()}.mask};
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const OptTensor& wr_, const OptTensor& logits_,
+                               const Tensor& w1, const Tensor& w3, const Tensor& w2, const OptTensor& bias_,
+                               const OptTensor& ids_, const Layer& o) {
+    const Tensor &wr = value(wr_), &logits = value(logits_), &bias = value(bias_), &ids = value(ids_);
+    const OutputsF32 f = forward_f32(o, x, wr, logits, w1, w3, w2, bias, ids);
+    ctx->save_for_backward({f.kept, f.routing, f.w[0], f.w[1], f.w[2], wr.defined() ? x : Tensor(), wr});
+    ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), o.k, f.logits.defined(),
+                                                Present{true, wr.defined(), logits.defined(), true, true, true,
+                                                        bias.defined(), ids.defined()}.mask};
     ctx->set_materialize_grads(false);
+    if (wr.defined()) return {f.out, f.logits};
     return {f.out};
   }
 
+  // What a linear layer's backward gives the router's input and weight (in operations that can be differentiated again).
+  static void router_grads(const Tensor& dlogits, const Tensor& x, const Tensor& wr, bool want_x, bool want_wr, Tensor& dx,
+                           Tensor& dwr) {
+    const NoAutocast off;
+    if (want_wr) dwr = at::mm(dlogits.t(), x);
+    if (want_x) dx = dx.defined() ? dx + at::mm(dlogits, wr) : at::mm(dlogits, wr);
+  }
+
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    first_order_only();
     const variable_list saved = ctx->get_saved_variables();
-    const Tensor &kept_buf = saved[0], &routing = saved[1], &w1 = saved[2], &w3 = saved[3], &w2 = saved[4];
+    const Tensor &kept_buf = saved[0], &routing = saved[1], &w1 = saved[2], &w3 = saved[3], &w2 = saved[4], &x = saved[5],
+                 &wr = saved[6];
     const std::vector<int64_t> ints = ctx->saved_data["i"].toIntVector();
     const int64_t T = ints[0], k = ints[1], R = T * k, E = w1.size(0), I = w1.size(1), H = w1.size(2);
-    const bool routed = ints[2];
+    const bool routed = ints[2], has_router = wr.defined();
     const c10::DeviceGuard guard(kept_buf.device());
     Present present;
     present.mask = ints[3];
     const auto need = [&](Input i) { return present.wants_gradient(ctx, i); };
-    const bool want_gates = routed && (need(LOGITS) || need(BIAS));
+    const Tensor ext = has_router ? grads[1] : Tensor();
+    variable_list out(INPUTS);
+    if (has_router && !grads[0].defined()) {  // only the logits were used
+      if (ext.defined()) router_grads(ext, x, wr, need(X), need(WR), out[X], out[WR]);
+      return out;
+    }
+    first_order_only();
+    // (the logits' gradient has to be there by itself for a bias, and to be added to)
+    const bool by_hand = need(LOGITS) || need(BIAS) || (has_router && ext.defined());
+    const bool inside = has_router && !by_hand && (need(X) || need(WR));
+    const bool want_gates = routed && (by_hand || inside);
     const Tensor dout = grads[0].defined() ? dense(grads[0].to(at::kFloat)) : at::zeros({T, H}, kept_buf.options());
     const Routing r(R, E);
     const KeptF32 kept(R, H, I);
@@ -726,16 +764,27 @@ struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
     const int32_t* r2p = r.part(routing, Routing::ROW_TO_POS);
     void* s = stream_of(kept_buf);
     const int64_t rh = up(R * H, 64), ri = up(R * I, 64);
-    const Tensor scratch = empty({2 * rh + 2 * ri + up(R, 64) + 64}, at::kFloat, kept_buf);
+    const int slices = inside && need(WR) ? moe_f32_router_wgrad_slices(R, H, E) : 1;
+    const Tensor scratch = empty({2 * rh + 2 * ri + 2 * up(R, 64) + (slices > 1 ? slices * E * H : 0) + 64}, at::kFloat, kept_buf);
     float* dyp = scratch.data_ptr<float>();
-    float *dxp = dyp + rh, *dg = dxp + rh, *du = dg + ri, *dgates = du + ri;
+    float *dxp = dyp + rh, *dg = dxp + rh, *du = dg + ri, *dgates = du + ri, *dsel = dgates + up(R, 64), *part = dsel + up(R, 64);
     CALL(moe_f32_combine_bwd, dout.data_ptr<float>(), want_gates ? y : nullptr, gates, p2r, T, R, H, k, dyp,
          want_gates ? dgates : nullptr, s);
     CALL(moe_f32_gemm_down_swiglu_bwd, dyp, w2.data_ptr<float>(), g, u, offs, E, R, H, I, dg, du, s);
-    Tensor dx, dw1, dw3, dw2, dlogits, dbias;
+    Tensor dx, dwr, dw1, dw3, dw2, dlogits, dbias;
+    const int32_t* ids = r.part(routing, Routing::IDS);
     if (need(X)) {
       dx = empty({T, H}, at::kFloat, kept_buf);
       CALL(moe_f32_gemm_gateup_bwd, dg, du, w1.data_ptr<float>(), w3.data_ptr<float>(), offs, E, R, H, I, dxp, s);
+    }
+    if (inside) {
+      const Tensor wrd = dense(wr);
+      CALL(moe_f32_permute_bwd_router, dxp, r2p, gates, dgates, ids, wrd.data_ptr<float>(), T, H, k, dsel, (float*)ptr(dx), s);
+      if (need(WR)) {
+        dwr = empty({E, H}, at::kFloat, kept_buf);
+        CALL(moe_f32_router_wgrad, xp, dsel, offs, R, H, E, part, dwr.data_ptr<float>(), s);
+      }
+    } else if (need(X)) {
       CALL(moe_f32_permute_bwd, dxp, r2p, T, H, k, dx.data_ptr<float>(), s);
     }
     if (need(W1)) dw1 = empty({E, I, H}, at::kFloat, kept_buf);
@@ -743,38 +792,43 @@ struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
     if (need(W2)) dw2 = empty({E, H, I}, at::kFloat, kept_buf);
     CALL(moe_f32_wgrads, dg, du, dyp, xp, act, offs, E, R, H, I, (float*)ptr(dw1), (float*)ptr(dw3),
          (float*)ptr(dw2), s);
-    if (want_gates) {
+    if (by_hand) {
       dlogits = empty({T, E}, at::kFloat, kept_buf);
-      CALL(moe_router_topk_bwd, gates, dgates, r.part(routing, Routing::IDS), T, E, k, dlogits.data_ptr(), MOE_DT_F32, s);
+      CALL(moe_router_topk_bwd, gates, dgates, ids, T, E, k, dlogits.data_ptr(), MOE_DT_F32, s);
+      if (ext.defined()) dlogits = dlogits + ext;
       if (need(BIAS)) dbias = dlogits.sum(0);
+      if (has_router) router_grads(dlogits, x, wr, need(X), need(WR), dx, dwr);
       if (!need(LOGITS)) dlogits = Tensor();
     }
-    variable_list out(INPUTS);
-    out[X] = dx, out[LOGITS] = dlogits, out[W1] = dw1, out[W3] = dw3, out[W2] = dw2, out[BIAS] = dbias;
+    out[X] = dx, out[WR] = dwr, out[LOGITS] = dlogits, out[W1] = dw1, out[W3] = dw3, out[W2] = dw2, out[BIAS] = dbias;
     return out;
   }
 };
 
-// -> (out, routing words if asked for)
-std::tuple<Tensor, OptTensor> layer_f32(const Tensor& x, const OptTensor& logits, const OptTensor& ids, const Tensor& w1,
-                                        const Tensor& w3, const Tensor& w2, const OptTensor& bias, int64_t k,
-                                        bool want_routing) {
-  const Tensor &l = value(logits), &b = value(bias), &i = value(ids);
-  no_tangents({&x, &l, &w1, &w3, &w2, &b});
+// -> (out, logits if the router product is inside, routing words if asked for)
+std::tuple<Tensor, OptTensor, OptTensor> layer_f32(const Tensor& x, const OptTensor& wr, const OptTensor& logits,
+                                                   const OptTensor& ids, const Tensor& w1, const Tensor& w3, const Tensor& w2,
+                                                   const OptTensor& bias, int64_t k, bool want_routing) {
+  const Tensor &r = value(wr), &l = value(logits), &b = value(bias), &i = value(ids);
+  no_tangents({&x, &r, &l, &w1, &w3, &w2, &b});
   Layer o;
   o.k = k;
   Tensor routing;
   if (want_routing) o.routing_out = &routing;
   if (at::GradMode::is_enabled())
-    for (const Tensor* p : {&x, &l, &w1, &w3, &w2, &b}) o.train = o.train || (p->defined() && p->requires_grad());
-  Tensor out;
+    for (const Tensor* p : {&x, &r, &l, &w1, &w3, &w2, &b}) o.train = o.train || (p->defined() && p->requires_grad());
+  Tensor out, lg;
   if (o.train) {
-    out = LayerF32Node::apply(x, logits, w1, w3, w2, bias, ids, o)[0];
+    const variable_list v = LayerF32Node::apply(x, wr, logits, w1, w3, w2, bias, ids, o);
+    out = v[0];
+    if (v.size() > 1) lg = v[1];
   } else {
     const at::NoGradGuard off;
-    out = forward_f32(o, x, l, w1, w3, w2, b, i).out;
+    const OutputsF32 f = forward_f32(o, x, r, l, w1, w3, w2, b, i);
+    out = f.out;
+    if (r.defined()) lg = f.logits;
   }
-  return {out, want_routing ? OptTensor(routing) : std::nullopt};
+  return {out, lg.defined() ? OptTensor(lg) : std::nullopt, want_routing ? OptTensor(routing) : std::nullopt};
 }
 
 }  // namespace

@@ -4,6 +4,7 @@
 // dispatch kernels as the bf16 path; what differs is the row type of the expert-contiguous
 // buffers (fp32 [R,H] / [R,I]).  The products are in f32_gemm.hip.
 #include "common.h"
+#include "internal.h"
 
 namespace {
 
@@ -90,6 +91,88 @@ __global__ __launch_bounds__(256) void f32_permute_bwd_kernel(const float* __res
     }
     *reinterpret_cast<f32x4*>(dx + t * H + h) = acc;
   }
+}
+
+// The same with the router's backward in it, where the router product is part of the layer: from the gate gradients the softmax
+// Jacobian over the token's k winners (as router_topk_bwd_kernel, the k-term sum ascending), dsel = its k nonzero logit gradients,
+// left by position for the weight gradient, and dx += sum_j dsel[j] * wr[ids[t*k+j], :] (dx NULL: not wanted).  In its place were a
+// launch for the rows of dlogits, the library's product with them, and an addition of two [T, H].  Bound by memory, k rows of wr a token
+// from L2 on top of the other kernel's.  With the next kernel, whole passes, us: 2048 tokens, 2 of 8 experts, 1024 <-> 512, 381 -> 362; 4717,
+// 2 of 64, 768 <-> 384, 690 -> 624; 11981, 1 of 128, 320 <-> 1472, 1536 -> 1422; 939, 8 of 16, 3136 <-> 256, 1014 -> 1000; where the host bounds
+// them, two library products and two nodes less: 686, 2 of 4, 1136 <-> 160, 221 -> 161; 239, 3 of 64, 816 <-> 168, 227 -> 201.
+__global__ __launch_bounds__(256) void f32_permute_bwd_router_kernel(
+    const float* __restrict__ dxp, const int32_t* __restrict__ row_to_pos, const float* __restrict__ gates,
+    const float* __restrict__ dgates, const int32_t* __restrict__ ids, const float* __restrict__ wr, int R, int H, int k,
+    float* __restrict__ dsel_by_pos, float* __restrict__ dx) {
+  const long long t = blockIdx.x;
+  const int lane = lane_id();
+  float g = 0.f, dg = 0.f;
+  int id = 0, pos = -1;
+  if (lane < k) {
+    g = gates[t * k + lane];
+    dg = dgates[t * k + lane];
+    id = ids[t * k + lane];
+    pos = row_to_pos[t * k + lane];
+  }
+  float s = 0.f;
+  for (int j = 0; j < k; ++j) s += read_lane_f(g, j) * read_lane_f(dg, j);
+  const float dsel = g * (dg - s);
+  if (threadIdx.x < (unsigned)k && pos >= 0 && pos < R) dsel_by_pos[pos] = dsel;
+  if (!dx) return;
+  for (int h = threadIdx.x * 4; h < H; h += 256 * 4) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, router = {0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < k; ++j) {
+      const int p = read_lane(pos, j);
+      router += read_lane_f(dsel, j) * *reinterpret_cast<const f32x4*>(wr + (long long)read_lane(id, j) * H + h);
+      if (p < 0 || p >= R) continue;
+      acc += *reinterpret_cast<const f32x4*>(dxp + (long long)p * H + h);
+    }
+    *reinterpret_cast<f32x4*>(dx + t * H + h) = acc + router;
+  }
+}
+
+// dwr[e, :] = sum over the expert's rows of dsel * xp[row, :]: what dlogits^T x comes to, whose other entries are zero, in one
+// pass over the rows that the experts' products read anyway.  256 columns a workgroup, a row a wave, eight of them requested at
+// once, the waves' sums added in order; slice blockIdx.z of gridDim.z of the expert's rows, summed up by the next kernel.
+constexpr int RW_WAVES = 8, RW_COLS = 4 * MOE_WAVE;
+__global__ __launch_bounds__(RW_WAVES* MOE_WAVE) void f32_router_wgrad_kernel(const float* __restrict__ xp,
+                                                                            const float* __restrict__ dsel,
+                                                                            const int32_t* __restrict__ offs, int H,
+                                                                            float* __restrict__ out) {
+  constexpr int AHEAD = 8;
+  __shared__ f32x4 part[RW_WAVES][MOE_WAVE];
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE)), col = blockIdx.x * RW_COLS + lane * 4;
+  const int e = blockIdx.y, E = gridDim.y, first = offs[e];
+  const long long n = offs[e + 1] - first;
+  const int lo = first + (int)(n * blockIdx.z / gridDim.z), hi = first + (int)(n * (blockIdx.z + 1) / gridDim.z);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int r = lo + wv; r < hi; r += RW_WAVES * AHEAD) {
+    f32x4 v[AHEAD];
+    float d[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int row = r + i * RW_WAVES;
+      const bool in = row < hi;
+      d[i] = in ? dsel[row] : 0.f;
+      v[i] = in && col < H ? *reinterpret_cast<const f32x4*>(xp + (long long)row * H + col) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) acc += d[i] * v[i];
+  }
+  part[wv][lane] = acc;
+  __syncthreads();
+  if (wv || col >= H) return;
+#pragma unroll
+  for (int w = 1; w < RW_WAVES; ++w) acc += part[w][lane];
+  *reinterpret_cast<f32x4*>(out + ((long long)blockIdx.z * E + e) * H + col) = acc;
+}
+__global__ __launch_bounds__(256) void f32_sum_slices_kernel(const float* __restrict__ part, int slices, long long n4,
+                                                             float* __restrict__ out) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  f32x4 acc = reinterpret_cast<const f32x4*>(part)[i];
+  for (int s = 1; s < slices; ++s) acc += reinterpret_cast<const f32x4*>(part)[s * n4 + i];
+  reinterpret_cast<f32x4*>(out)[i] = acc;
 }
 
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.f / (1.f + expf(-x)); }
@@ -190,6 +273,52 @@ extern "C" int moe_f32_permute_bwd(const float* dxp, const int32_t* row_to_pos, 
   if (!row_to_pos) return MOE_ERR_NULL;
   hipLaunchKernelGGL(f32_permute_bwd_kernel, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream, dxp, row_to_pos,
                      (int)(T * k), (int)H, (int)k, dx);
+  return moe_launch_status();
+}
+
+int moe_f32_permute_bwd_router(const float* dxp, const int32_t* row_to_pos, const float* gates, const float* dgates,
+                               const int32_t* ids, const float* wr, int64_t T, int64_t H, int64_t k, float* dsel, float* dx,
+                               void* stream) {
+  if (int rc = check_rows(T, H)) return rc;
+  if (k <= 0) return MOE_ERR_SHAPE;
+  if (k > MOE_MAX_TOPK || T * k > (int64_t)1 << 30) return MOE_ERR_LIMIT;
+  if (T == 0) return 0;
+  if (dx) {
+    MOE_CHECK_PTR(dxp);
+    MOE_CHECK_PTR(wr);
+    MOE_CHECK_PTR(dx);
+  }
+  if (!row_to_pos || !gates || !dgates || !ids || !dsel) return MOE_ERR_NULL;
+  hipLaunchKernelGGL(f32_permute_bwd_router_kernel, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream, dxp, row_to_pos, gates,
+                     dgates, ids, wr, (int)(T * k), (int)H, (int)k, dsel, dx);
+  return moe_launch_status();
+}
+
+// Slices of an expert's rows: two workgroups for every compute unit, but eight rows for every wave where they are dealt evenly.
+int moe_f32_router_wgrad_slices(int64_t R, int64_t H, int64_t E) {
+  const int64_t blocks = E * ((H + RW_COLS - 1) / RW_COLS), want = 2 * (int64_t)moe_compute_units() / blocks;
+  const int64_t most = R / E / (8 * RW_WAVES), n = want < most ? want : most;
+  return (int)(n < 1 ? 1 : n > 64 ? 64 : n);
+}
+
+// `part`: the slices' results, slices * E * H floats, where there is more than one.
+int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs, int64_t R, int64_t H, int64_t E, float* part,
+                         float* dwr, void* stream) {
+  if (int rc = check_rows(R, H)) return rc;
+  if (E <= 0) return MOE_ERR_SHAPE;
+  if (E > MOE_MAX_EXPERTS) return MOE_ERR_LIMIT;
+  MOE_CHECK_PTR(xp);
+  MOE_CHECK_PTR(dwr);
+  if (!dsel || !offs) return MOE_ERR_NULL;
+  const int slices = moe_f32_router_wgrad_slices(R, H, E);
+  if (slices > 1) MOE_CHECK_PTR(part);
+  const hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(f32_router_wgrad_kernel, dim3((unsigned)((H + RW_COLS - 1) / RW_COLS), (unsigned)E, (unsigned)slices),
+                     dim3(RW_WAVES * MOE_WAVE), 0, s, xp, dsel, offs, (int)H, slices > 1 ? part : dwr);
+  if (slices == 1) return moe_launch_status();
+  if (const int rc = moe_launch_status()) return rc;
+  const long long n4 = (long long)E * H / 4;
+  hipLaunchKernelGGL(f32_sum_slices_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, part, slices, n4, dwr);
   return moe_launch_status();
 }
 

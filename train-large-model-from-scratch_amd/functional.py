@@ -131,8 +131,15 @@ def moe_ffn_f32(x: torch.Tensor, logits: torch.Tensor, w1: torch.Tensor, w3: tor
     for name, t in (("x", x), ("logits", logits), ("w1", w1), ("w3", w3), ("w2", w2)):
         if t.dtype != torch.float32:
             raise TypeError(f"moe_ffn_f32: {name} must be fp32, got {t.dtype}")
-    out, words = _lib.native().layer_f32(x, logits, None, w1, w3, w2, bias, k, return_routing)
+    out, _, words = _lib.native().layer_f32(x, None, logits, None, w1, w3, w2, bias, k, return_routing)
     return (out, _routing_dict(ops.Routing(words, x.shape[0] * k, w1.shape[0]))) if return_routing else out
+
+
+def routed_moe_f32(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor, w2: torch.Tensor, k: int):
+    """(MoE(x), router logits) for x [T,H], all fp32: `nn.Linear`'s product and `moe_ffn_f32` as one autograd node, whose
+    backward adds the router path's input gradient in the k-row-sum kernel."""
+    out, logits, _ = _lib.native().layer_f32(x, router_weight, None, None, w1, w3, w2, None, k, False)
+    return out, logits
 
 
 def prenorm_moe(x: torch.Tensor, norm_weight: torch.Tensor, router_weight: torch.Tensor,
@@ -175,7 +182,7 @@ def experts_rows_f32(rows: torch.Tensor, ids: torch.Tensor, w1, w3, w2, return_r
         if t.dtype != torch.float32:
             raise TypeError(f"experts_rows_f32: {name} must be fp32, got {t.dtype}")
     want = check_ids or return_routing
-    out, words = _lib.native().layer_f32(rows, None, ids, w1, w3, w2, None, 1, want)
+    out, _, words = _lib.native().layer_f32(rows, None, None, ids, w1, w3, w2, None, 1, want)
     routing = ops.Routing(words, rows.shape[0], w1.shape[0]) if want else None
     if check_ids:
         _check_ids("experts_rows_f32", routing, ids.numel(), w1.shape[0])

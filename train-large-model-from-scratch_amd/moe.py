@@ -9,10 +9,11 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 from torch.optim.optimizer import register_optimizer_step_post_hook
 
 from . import ops, parallel_state, traced
-from .functional import moe_ffn, moe_ffn_f32, prenorm_moe, routed_moe, router_linear
+from .functional import moe_ffn, moe_ffn_f32, prenorm_moe, routed_moe, routed_moe_f32, router_linear
 
 
 # Number of optimizer steps taken in this process, counted by a global post-step hook of
@@ -168,6 +169,12 @@ class MoE(nn.Module):
         r = self.router
         return bool(r._forward_hooks or r._forward_pre_hooks or r._backward_hooks or r._backward_pre_hooks)
 
+    def _router_is_plain(self) -> bool:
+        """Whether calling `self.router` is the product with its weight and nothing else."""
+        r = self.router
+        return (type(r) is nn.Linear and r.bias is None and "forward" not in r.__dict__ and not self._router_has_hooks()
+                and not _has_any_global_hook())
+
     def _router_in_bf16(self, x: torch.Tensor) -> bool:
         """Whether `self.router(x)` would be a bf16 product anyway (bf16 autocast, or bf16
         tensors): then router and experts run as one autograd node."""
@@ -191,9 +198,17 @@ class MoE(nn.Module):
     def _experts_f32(x2d, logits2d, w1, w3, w2, k) -> torch.Tensor:
         return moe_ffn_f32(x2d, logits2d, w1, w3, w2, k)
 
+    @torch._dynamo.disable
+    def _layer_f32(self, x2d: torch.Tensor):
+        return routed_moe_f32(x2d, self.router.weight, self.experts_gate_weights, self.experts_up_weights,
+                              self.experts_down_weights, self.top_k)
+
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         B, T, D = x.size()
         if self._runs_in_fp32(x):
+            if not torch.compiler.is_compiling() and self._router_is_plain():
+                out, gate_logits = self._layer_f32(x.reshape(B * T, D))
+                return out.reshape(B, T, D), gate_logits.reshape(B, T, self.num_experts)
             gate_logits = self.router(x)  # fp32 product and fp32 gradients, as nn.Linear gives them
             ffn = traced.moe_ffn_f32 if torch.compiler.is_compiling() else self._experts_f32
             out = ffn(x.reshape(B * T, D), gate_logits.reshape(B * T, self.num_experts),
