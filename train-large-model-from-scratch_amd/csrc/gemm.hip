@@ -212,36 +212,43 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     u32x4 v[NCH];
   };
   Stage stg;
+  // Where a k-tile lies: the windows of the operands from it on (DUAL: three of them).
+  constexpr int NOP = DUAL ? 3 : 2;
   struct TileSrc {
-    __amdgpu_buffer_rsrc_t a, b0, b1;
+    Window w[NOP];
     int k_left;
   };
-  auto tile_src = [&](const Tile& t, int kt) {
-    const int seg = (NSEG == 2) ? kt / t.kt_per_seg : 0;
-    int k0 = (kt - seg * t.kt_per_seg) * BK;
+  auto k_of = [&](const Tile& t, int kt) {  // (of its segment)
     if constexpr (MODE == GATEUP || MODE == DOWN) {
       const int at = kt + t.kt0;
-      k0 = (at >= t.nkt ? at - t.nkt : at) * BK;
-    }
-    TileSrc ts;
-    ts.a = view_rsrc((NSEG == 2 && seg) ? t.vA1 : t.vA0, StA::k_bytes(k0, lda));
-    if constexpr (DUAL) {
-      ts.b0 = view_rsrc(t.vB0, StBh::k_bytes(k0, ldb));
-      ts.b1 = view_rsrc(t.vB1, StBh::k_bytes(k0, ldb));
+      return (at >= t.nkt ? at - t.nkt : at) * BK;
     } else {
-      ts.b0 = view_rsrc((NSEG == 2 && seg) ? t.vB1 : t.vB0, StB::k_bytes(k0, ldb));
-      ts.b1 = ts.b0;
+      return (NSEG == 2 && kt >= t.kt_per_seg ? kt - t.kt_per_seg : kt) * BK;
     }
-    ts.k_left = t.Kseg - k0;
+  };
+  auto operand_src = [&](const Tile& t, int kt, int op) {
+    const int k0 = k_of(t, kt);
+    const bool second = NSEG == 2 && kt >= t.kt_per_seg;
+    if (op == 0) return window(second ? t.vA1 : t.vA0, StA::k_bytes(k0, lda));
+    if constexpr (DUAL) return window(op == 1 ? t.vB0 : t.vB1, StBh::k_bytes(k0, ldb));
+    else return window(second ? t.vB1 : t.vB0, StB::k_bytes(k0, ldb));
+  };
+  auto tile_src = [&](const Tile& t, int kt) {
+    TileSrc ts;
+#pragma unroll
+    for (int op = 0; op < NOP; ++op) ts.w[op] = operand_src(t, kt, op);
+    ts.k_left = t.Kseg - k_of(t, kt);
     return ts;
   };
+  constexpr auto operand_of = [](int c) { return c < CHA ? 0 : DUAL && c >= CHA + CHB ? 2 : 1; };  // a chunk's
   auto load_chunk = [&](int c, Stage& st, const TileSrc& ts) {
-    if (c < CHA) st.v[c] = opA.load_one(c, ts.a);
+    const __amdgpu_buffer_rsrc_t rs = ts.w[operand_of(c)].rsrc();
+    if (c < CHA) st.v[c] = opA.load_one(c, rs);
     else if constexpr (DUAL) {
-      if (c < CHA + CHB) st.v[c] = opB0.load_one(c - CHA, ts.b0);
-      else st.v[c] = opB1.load_one(c - CHA - CHB, ts.b1);
+      if (c < CHA + CHB) st.v[c] = opB0.load_one(c - CHA, rs);
+      else st.v[c] = opB1.load_one(c - CHA - CHB, rs);
     } else {
-      st.v[c] = opB.load_one(c - CHA, ts.b0);
+      st.v[c] = opB.load_one(c - CHA, rs);
     }
   };
   auto clear_past_k = [&](int c, Stage& st, int k_left) {
@@ -324,10 +331,13 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   //                   tile kt+2 requested | fragments of step s+1 read
   //   last phase      barrier (stage kt fully read, stage kt+1 fully written) | MFMAs of the
   //                   last step | first fragment reads of stage kt+1 hide behind them
-  auto body = [&](auto par_c, const Tile& t, int kt) {
+  // Where tile kt+3 lies is worked out behind the last request for an operand of kt+2, between two products: in front
+  // of the first one the forty scalar instructions, with six 64-bit comparisons in the vector unit among them, held up both waves of a
+  // SIMD, which come from the same barrier.  Whole passes, us: 1531 tokens, 8 of 64 experts, forward, 258.8 -> 254.6; 8192, 2 of 8, 1024 <-> 512,
+  // 308.5 -> 305.0; 13 smaller ones 1.01 to 1.03; 16384 tokens of 64, where power is the bound, 4946 -> 4944.
+  auto body = [&](auto par_c, const Tile& t, int kt, TileSrc& ts) {
     constexpr int buf = decltype(par_c)::value;  // LDS stage of k-tile kt == parity of kt
-    Stage& st = stg;                             // holds k-tile kt+1, refilled with kt+2
-    const TileSrc ts = tile_src(t, kt + 2);
+    Stage& st = stg;                             // holds k-tile kt+1, refilled with kt+2, which lies at `ts`
     constexpr int NSLOT = (KS - 1) * NMMA;  // MFMA slots before the barrier
 #pragma unroll
     for (int ks = 0; ks < KS - 1; ++ks) {
@@ -340,6 +350,13 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
           if (c * NSLOT / NCH == slot) {
             store_chunk(c, st, buf ^ 1);
             load_chunk(c, st, ts);
+            if (c + 1 == NCH || operand_of(c + 1) != operand_of(c)) {
+              Window& w = ts.w[operand_of(c)];
+              int ahead = kt + 3;
+              asm volatile("" : "+s"(ahead));  // (else most of it moves up in front of the first product all the same)
+              w = operand_src(t, ahead, operand_of(c));
+              w.stay_here();
+            }
           }
         }
         if (n < NFR) f_read_one(n, buf, ks + 1, fr[(ks + 1) & 1]);
@@ -792,9 +809,10 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       int steady_end = nkt - 2;
       if (cur.need_mask) steady_end = (NSEG == 2 && kt + 2 < cur.kt_per_seg ? cur.kt_per_seg : nkt) - 3;
       if (!((kt + s0) & 1)) {
+        TileSrc ts = tile_src(cur, kt + 2);
         for (; kt + 1 < steady_end; kt += 2) {
-          body(integral_constant<int, 0>{}, cur, kt);
-          body(integral_constant<int, 1>{}, cur, kt + 1);
+          body(integral_constant<int, 0>{}, cur, kt, ts);
+          body(integral_constant<int, 1>{}, cur, kt + 1, ts);
         }
       }
       one(kt);

@@ -9,11 +9,8 @@ namespace {
 
 // The window's resource from byte_off on; not `live`: empty, everything reads as zero.
 __device__ __forceinline__ u32x4 ring_rsrc(const View& w, long long byte_off, bool live) {
-  long long left = w.bytes - byte_off;
-  if (left < 0 || !live) left = 0;
-  if (left > 0xffffffffll) left = 0xffffffffll;
   const uint64_t at = (uint64_t)((const char*)w.base + byte_off);
-  return u32x4{(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, (uint32_t)left, 0x00020000u};
+  return u32x4{(uint32_t)at, (uint32_t)(at >> 32) & 0xffffu, live ? window_size(w.bytes - byte_off) : 0u, 0x00020000u};
 }
 // 16 bytes per lane from `off` into LDS at lds_byte + 16 * lane.  In assembly because the compiler would wait for every
 // such load before any LDS read that follows; the waits are ring_wait's.  The load takes its LDS address from m0, which is

@@ -20,12 +20,25 @@ struct View {
 __device__ __forceinline__ View make_view(const uint16_t* base, long long valid_elems) {
   return View{base, valid_elems > 0 ? valid_elems * 2 : 0};
 }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t view_rsrc(const View& w, long long byte_off) {
-  long long left = w.bytes - byte_off;
-  if (left < 0) left = 0;
-  if (left > 0xffffffffll) left = 0xffffffffll;
-  return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)w.base + byte_off), 0,
-                                           (int)(unsigned)left, 0x00020000);
+// What a window has left, as a resource's size: none past its end, and no more than the 32 bits hold.  In the scalar unit: there is no
+// 64-bit comparison there, and the vector unit's, whose results travel back, are what a k-tile's first products waited for.
+__device__ __forceinline__ uint32_t window_size(long long left) {
+  int high = (int)(left >> 32);
+  asm("" : "+s"(high));  // (or the two halves become one 64-bit comparison again)
+  return high < 0 ? 0u : high > 0 ? 0xffffffffu : (uint32_t)left;
+}
+// The window from a byte on, in scalar registers.
+struct Window {
+  const char* at;
+  uint32_t size;
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc() const {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, (int)size, 0x00020000);
+  }
+  // Worked out where the program says so, not where it is first needed.
+  __device__ __forceinline__ void stay_here() { asm volatile("" : "+s"(at), "+s"(size)); }
+};
+__device__ __forceinline__ Window window(const View& w, long long byte_off) {
+  return {(const char*)w.base + byte_off, window_size(w.bytes - byte_off)};
 }
 
 // ---- operand staging ----------------------------------------------------------------------
