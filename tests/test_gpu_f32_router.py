@@ -86,13 +86,140 @@ def test_no_tokens_and_logits_twice(pkg, lib):
         torch.autograd.grad(routed(*leaves)[0], leaves[0], dy, create_graph=True)
 
 
-def test_module_takes_it_unless_the_router_is_more_than_a_product(pkg, lib):
-    print("fp32 module, router with a hook", flush=True)
+@pytest.mark.parametrize("loss_on_logits", [False, True])
+@pytest.mark.parametrize("who", ["hook", "hook that changes it", "retain_grad", "asked for", "node", "product's node"])
+def test_the_logits_are_on_the_way_to_the_output(pkg, lib, who, loss_on_logits):
+    """Whoever looks at the logits' gradient sees the experts' share of it, and what a hook makes of it is what goes on."""
+    print("fp32 router, logits observed:", who, loss_on_logits, flush=True)
+    T, E, k, H, I = 150, 8, 2, 128, 64
+    leaves, dy, dl = inputs(T, E, H, I, 7)
+    leaves[0] = leaves[0].detach().view(3, 50, H).requires_grad_(True)
+    dy, dl = dy.view(3, 50, H), dl.view(3, 50, E)
+    routed = both(pkg, T, E, k, H, I)[0]
+
+    def apart(x, wr, w1, w3, w2):
+        logits = F.linear(x, wr)
+        return pkg.moe_ffn_f32(x.reshape(T, H), logits.reshape(T, E), w1, w3, w2, k).reshape(x.shape), logits
+
+    res = []
+    for call in (routed, apart):
+        out, logits = call(*leaves)
+        assert out.shape == (3, 50, H) and logits.shape == (3, 50, E) and not logits._is_view()
+        outs, given = ([out, logits], [dy, dl]) if loss_on_logits else ([out], [dy])
+        seen = []
+        if who == "hook":
+            logits.register_hook(lambda g: seen.append(g.clone()))
+        elif who == "hook that changes it":
+            logits.register_hook(lambda g: seen.append(g.clone()) or 3 * g)
+        elif who == "retain_grad":
+            logits.retain_grad()
+        elif who == "node":
+            logits.grad_fn.register_prehook(lambda g: seen.append(g[0].clone()))
+        elif who == "product's node":
+            node = logits.grad_fn
+            while len(node.next_functions) == 1:
+                node = node.next_functions[0][0]
+            node.register_prehook(lambda g: seen.append(g[0].clone().view(3, 50, E)))
+        want = leaves + ([logits] if who == "asked for" else [])
+        grads = list(torch.autograd.grad(outs, want, given))
+        if who == "retain_grad":
+            seen.append(logits.grad)
+        if seen:
+            grads.append(seen[0])
+        assert len(grads) == 6 and len(seen) == (who != "asked for")
+        res.append(grads)
+    for name, a, b in zip(("dx", "dwr", "dw1", "dw3", "dw2", "dlogits"), *res):
+        close(name, a, b)
+    assert bool(res[0][5].any())
+
+
+def test_logits_may_be_written_to(pkg, lib):
+    print("fp32 router, logits changed in place", flush=True)
+    T, E, k, H, I = 40, 8, 2, 64, 32
+    leaves, dy, dl = inputs(T, E, H, I, 3)
+    res = []
+    for call in both(pkg, T, E, k, H, I):
+        out, logits = call(*leaves)
+        logits.mul_(2)
+        res.append(torch.autograd.grad([out, logits], leaves, [dy, dl]))
+    for name, a, b in zip(("dx", "dwr", "dw1", "dw3", "dw2"), *res):
+        close(name, a, b)
+
+
+class Linear(torch.nn.Linear):
+    pass
+
+
+def global_hook(m):
+    h = torch.nn.modules.module.register_module_forward_hook(lambda mod, inp, o: None)
+    return h.remove
+
+
+def own_forward(m):
+    r = m.router
+    r.forward = lambda x: F.linear(x, r.weight)
+    return lambda: delattr(r, "forward")
+
+
+def other_router(make):
+    def change(m):
+        old, new = m.router, make(m.router)
+        with torch.no_grad():
+            new.weight.copy_(old.weight)
+        m.router = new
+        return lambda: setattr(m, "router", old)
+    return change
+
+
+def with_bias(r):
+    new = torch.nn.Linear(r.in_features, r.out_features, device="cuda")
+    torch.nn.init.zeros_(new.bias)
+    return new
+
+
+MORE_THAN_A_PRODUCT = {
+    "forward hook": lambda m: m.router.register_forward_hook(lambda mod, inp, o: None).remove,
+    "pre-hook": lambda m: m.router.register_forward_pre_hook(lambda mod, inp: None).remove,
+    "backward hook": lambda m: m.router.register_full_backward_hook(lambda mod, gi, go: None).remove,
+    "global hook": global_hook,
+    "bias": other_router(with_bias),
+    "subclass": other_router(lambda r: Linear(r.in_features, r.out_features, bias=False, device="cuda")),
+    "own forward": own_forward,
+}
+
+
+@pytest.mark.parametrize("what", ["plain"] + list(MORE_THAN_A_PRODUCT))
+def test_module_takes_it_unless_the_router_is_more_than_a_product(pkg, lib, what):
+    print("fp32 module, router:", what, flush=True)
     m = pkg.MoE(pkg.ModelConfig(hidden_size=128, num_experts=8, num_experts_per_tok=2, moe_intermediate_size=64, init_std=0.05), 2)
-    x = torch.randn(2, 50, 128, device="cuda")
-    out, logits = m(x)
-    seen = []
-    h = m.router.register_forward_hook(lambda mod, inp, o: seen.append(1))
-    out2, logits2 = m(x)
-    h.remove()
-    assert seen and torch.equal(out, out2) and torch.equal(logits, logits2)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x, dy = (torch.randn(2, 50, 128, generator=g, device="cuda") for _ in range(2))
+
+    def launches():
+        names = []
+
+        class Obs:
+            def before(self, name):
+                names.append(name)
+
+            def after(self, name):
+                pass
+
+        lib.observer = Obs()
+        try:
+            out, logits = m(x)
+            out.backward(dy)
+        finally:
+            lib.observer = None
+        return [out.detach(), logits.detach()], names.count("moe_f32_permute_bwd_router")
+
+    plain, times = launches()
+    assert times == 1
+    undo = MORE_THAN_A_PRODUCT.get(what, lambda m: lambda: None)(m)
+    try:
+        outs, times = launches()
+    finally:
+        undo()
+    assert times == (what == "plain")
+    for name, a, b in zip(("out", "logits"), plain, outs):
+        close(name, a, b)

@@ -9,6 +9,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/extension.h>
 
 #include <string>
@@ -202,8 +203,12 @@ struct Present {
     int i = 0;
     for (bool g : given) mask |= (int64_t)g << i++;
   }
+  int index(int input) const { return __builtin_popcountll(mask & ((1ll << input) - 1)); }
   bool wants_gradient(AutogradContext* ctx, int input) const {
-    return (mask >> input & 1) && ctx->needs_input_grad(__builtin_popcountll(mask & ((1ll << input) - 1)));
+    return (mask >> input & 1) && ctx->needs_input_grad(index(input));
+  }
+  torch::autograd::Node* next(const torch::autograd::Node& node, int input) const {
+    return node.next_edge(index(input)).function.get();
   }
 };
 
@@ -624,11 +629,11 @@ struct KeptF32 {
 };
 
 struct OutputsF32 {
-  Tensor out, routing, kept, w[3], logits;
+  Tensor out, routing, kept, w[3];
 };
 
-OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& wr, const Tensor& logits_, const Tensor& w1,
-                       const Tensor& w3, const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
+OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& logits_, const Tensor& w1, const Tensor& w3,
+                       const Tensor& w2, const Tensor& bias, const Tensor& ids_) {
   OutputsF32 f;
   need_gpu(x_);
   TORCH_CHECK(x_.dim() == 2 && w1.dim() == 3, "the layer takes x [tokens, hidden] and weights [experts, ., .]");
@@ -636,22 +641,9 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& wr, const
   TORCH_CHECK(w3.size(0) == E && w2.size(0) == E && w1.size(2) == H && w3.size(2) == H && w3.size(1) == I &&
                   w2.size(1) == H && w2.size(2) == I,
               "the weights' shapes do not belong together");
-  if (wr.defined()) {
-    need_gpu(wr);
-    TORCH_CHECK(wr.dim() == 2 && wr.size(0) == E && wr.size(1) == H, "the router weight has shape ", wr.sizes(), ", x ", x_.sizes(),
-                " and there are ", E, " experts");
-    TORCH_CHECK(wr.device() == x_.device(), "the router weight is on ", wr.device(), ", x on ", x_.device());
-    TORCH_CHECK_TYPE(wr.scalar_type() == at::kFloat && x_.scalar_type() == at::kFloat, "x and the router weight must be fp32");
-  }
   check_logits(logits_, bias, x_, E);
   const c10::DeviceGuard guard(x_.device());
   const Tensor x = dense(x_);
-  if (wr.defined()) {
-    const NoAutocast off;
-    f.logits = at::mm(x, wr.t());
-  } else {
-    f.logits = logits_;
-  }
   f.w[0] = dense(w1), f.w[1] = dense(w3), f.w[2] = dense(w2);
   void* s = stream_of(x);
   const Routing r(R, E);
@@ -662,7 +654,7 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& wr, const
   float* base = f.kept.data_ptr<float>();
   float *xp = base, *g = base + kept.g, *u = base + kept.u, *act = base + kept.act, *y = base + kept.y;
   float* gates = nullptr;
-  const bool place = f.logits.defined() && H % 8 == 0 && moe_place_ok(T, E, k);
+  const bool place = logits_.defined() && H % 8 == 0 && moe_place_ok(T, E, k);
   const int64_t wsb = std::max<int64_t>(place ? moe_place_bytes(T, E) : moe_dispatch_workspace_bytes(R, E), 16);
   const Tensor ws = empty({wsb}, at::kByte, x);
   int32_t* counts = r.part(f.routing, Routing::COUNTS);
@@ -671,8 +663,8 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& wr, const
   int32_t* r2p = r.part(f.routing, Routing::ROW_TO_POS);
   int32_t* ids = r.part(f.routing, Routing::IDS);
   Tensor logits, b;
-  if (f.logits.defined()) {
-    logits = dense(f.logits);
+  if (logits_.defined()) {
+    logits = dense(logits_);
     if (bias.defined()) b = dense(bias);
     gates = (float*)r.part(f.routing, Routing::GATES);
   }
@@ -706,6 +698,26 @@ OutputsF32 forward_f32(const Layer& o, const Tensor& x_, const Tensor& wr, const
   return f;
 }
 
+// Whether anything but the router's input and weight is there to see or to change the gradient that comes to `logits`, the
+// product of the two: a hook on it or on one of the nodes from it to the product, or a gradient asked for right there.
+bool logits_observed(torch::autograd::Node* node) {
+  const auto* info = torch::autograd::get_current_graph_task_exec_info();
+  for (; node; node = node->num_outputs() ? node->next_edge(0).function.get() : nullptr) {
+    if (!node->tensor_pre_hooks().empty() || !node->retains_grad_hooks().empty() || !node->pre_hooks().empty() ||
+        !node->post_hooks().empty())
+      return true;
+    if (info) {
+      const auto at = info->find(node);
+      if (at != info->end() && at->second.captures_) return true;
+    }
+    if (node->num_outputs() == 2) return false;  // the product
+  }
+  return true;
+}
+
+// Given the router weight too, `logits` are the fp32 product of x with it, made by the library in a graph of its own: the
+// layer hands their gradient on to it only where somebody observes it, and else works out what it comes to in x and in the
+// weight along with its own.
 struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
   enum Input { X, WR, LOGITS, W1, W3, W2, BIAS, IDS, OPTIONS, INPUTS };
 
@@ -713,45 +725,30 @@ struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
                                const Tensor& w1, const Tensor& w3, const Tensor& w2, const OptTensor& bias_,
                                const OptTensor& ids_, const Layer& o) {
     const Tensor &wr = value(wr_), &logits = value(logits_), &bias = value(bias_), &ids = value(ids_);
-    const OutputsF32 f = forward_f32(o, x, wr, logits, w1, w3, w2, bias, ids);
-    ctx->save_for_backward({f.kept, f.routing, f.w[0], f.w[1], f.w[2], wr.defined() ? x : Tensor(), wr});
-    ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), o.k, f.logits.defined(),
+    const OutputsF32 f = forward_f32(o, x, logits.defined() && logits.dim() != 2 ? logits.flatten(0, -2) : logits, w1, w3, w2, bias, ids);
+    ctx->save_for_backward({f.kept, f.routing, f.w[0], f.w[1], f.w[2], wr});
+    ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), o.k, logits.defined(),
                                                 Present{true, wr.defined(), logits.defined(), true, true, true,
                                                         bias.defined(), ids.defined()}.mask};
+    ctx->saved_data["shape"] = logits.defined() ? logits.sizes().vec() : std::vector<int64_t>();
     ctx->set_materialize_grads(false);
-    if (wr.defined()) return {f.out, f.logits};
     return {f.out};
   }
 
-  // What a linear layer's backward gives the router's input and weight (in operations that can be differentiated again).
-  static void router_grads(const Tensor& dlogits, const Tensor& x, const Tensor& wr, bool want_x, bool want_wr, Tensor& dx,
-                           Tensor& dwr) {
-    const NoAutocast off;
-    if (want_wr) dwr = at::mm(dlogits.t(), x);
-    if (want_x) dx = dx.defined() ? dx + at::mm(dlogits, wr) : at::mm(dlogits, wr);
-  }
-
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    first_order_only();
     const variable_list saved = ctx->get_saved_variables();
-    const Tensor &kept_buf = saved[0], &routing = saved[1], &w1 = saved[2], &w3 = saved[3], &w2 = saved[4], &x = saved[5],
-                 &wr = saved[6];
+    const Tensor &kept_buf = saved[0], &routing = saved[1], &w1 = saved[2], &w3 = saved[3], &w2 = saved[4], &wr = saved[5];
     const std::vector<int64_t> ints = ctx->saved_data["i"].toIntVector();
     const int64_t T = ints[0], k = ints[1], R = T * k, E = w1.size(0), I = w1.size(1), H = w1.size(2);
-    const bool routed = ints[2], has_router = wr.defined();
+    const bool routed = ints[2];
     const c10::DeviceGuard guard(kept_buf.device());
     Present present;
     present.mask = ints[3];
     const auto need = [&](Input i) { return present.wants_gradient(ctx, i); };
-    const Tensor ext = has_router ? grads[1] : Tensor();
-    variable_list out(INPUTS);
-    if (has_router && !grads[0].defined()) {  // only the logits were used
-      if (ext.defined()) router_grads(ext, x, wr, need(X), need(WR), out[X], out[WR]);
-      return out;
-    }
-    first_order_only();
-    // (the logits' gradient has to be there by itself for a bias, and to be added to)
-    const bool by_hand = need(LOGITS) || need(BIAS) || (has_router && ext.defined());
-    const bool inside = has_router && !by_hand && (need(X) || need(WR));
+    const auto node = torch::autograd::get_current_node();
+    const bool inside = wr.defined() && need(LOGITS) && node && !logits_observed(present.next(*node, LOGITS));
+    const bool by_hand = (need(LOGITS) && !inside) || need(BIAS);
     const bool want_gates = routed && (by_hand || inside);
     const Tensor dout = grads[0].defined() ? dense(grads[0].to(at::kFloat)) : at::zeros({T, H}, kept_buf.options());
     const Routing r(R, E);
@@ -795,40 +792,48 @@ struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
     if (by_hand) {
       dlogits = empty({T, E}, at::kFloat, kept_buf);
       CALL(moe_router_topk_bwd, gates, dgates, ids, T, E, k, dlogits.data_ptr(), MOE_DT_F32, s);
-      if (ext.defined()) dlogits = dlogits + ext;
       if (need(BIAS)) dbias = dlogits.sum(0);
-      if (has_router) router_grads(dlogits, x, wr, need(X), need(WR), dx, dwr);
-      if (!need(LOGITS)) dlogits = Tensor();
+      dlogits = need(LOGITS) ? dlogits.view(ctx->saved_data["shape"].toIntVector()) : Tensor();
     }
+    variable_list out(INPUTS);
     out[X] = dx, out[WR] = dwr, out[LOGITS] = dlogits, out[W1] = dw1, out[W3] = dw3, out[W2] = dw2, out[BIAS] = dbias;
     return out;
   }
 };
 
-// -> (out, logits if the router product is inside, routing words if asked for)
-std::tuple<Tensor, OptTensor, OptTensor> layer_f32(const Tensor& x, const OptTensor& wr, const OptTensor& logits,
+// -> (out [tokens, hidden], logits if the router weight is given, routing words if asked for); x: any number of leading
+// dimensions with a router weight, whose logits have them too.
+std::tuple<Tensor, OptTensor, OptTensor> layer_f32(const Tensor& x_, const OptTensor& wr, const OptTensor& logits,
                                                    const OptTensor& ids, const Tensor& w1, const Tensor& w3, const Tensor& w2,
                                                    const OptTensor& bias, int64_t k, bool want_routing) {
-  const Tensor &r = value(wr), &l = value(logits), &b = value(bias), &i = value(ids);
+  const Tensor &r = value(wr), &b = value(bias), &i = value(ids);
+  Tensor x = x_, l = value(logits);
   no_tangents({&x, &r, &l, &w1, &w3, &w2, &b});
   Layer o;
   o.k = k;
   Tensor routing;
   if (want_routing) o.routing_out = &routing;
+  if (r.defined()) {
+    need_gpu(x);
+    need_gpu(r);
+    TORCH_CHECK(x.dim() >= 2 && w1.dim() == 3 && r.dim() == 2 && r.size(0) == w1.size(0) && r.size(1) == x.size(-1),
+                "the router weight has shape ", r.sizes(), ", x ", x.sizes(), " and the experts' ", w1.sizes());
+    TORCH_CHECK(r.device() == x.device(), "the router weight is on ", r.device(), ", x on ", x.device());
+    TORCH_CHECK_TYPE(r.scalar_type() == at::kFloat && x.scalar_type() == at::kFloat, "x and the router weight must be fp32");
+    const NoAutocast off;
+    l = at::linear(x, r);
+    if (x.dim() != 2) x = x.flatten(0, -2);
+  }
   if (at::GradMode::is_enabled())
-    for (const Tensor* p : {&x, &r, &l, &w1, &w3, &w2, &b}) o.train = o.train || (p->defined() && p->requires_grad());
-  Tensor out, lg;
+    for (const Tensor* p : std::initializer_list<const Tensor*>{&x, &r, &l, &w1, &w3, &w2, &b}) o.train = o.train || (p->defined() && p->requires_grad());
+  Tensor out;
   if (o.train) {
-    const variable_list v = LayerF32Node::apply(x, wr, logits, w1, w3, w2, bias, ids, o);
-    out = v[0];
-    if (v.size() > 1) lg = v[1];
+    out = LayerF32Node::apply(x, wr, l.defined() ? OptTensor(l) : std::nullopt, w1, w3, w2, bias, ids, o)[0];
   } else {
     const at::NoGradGuard off;
-    const OutputsF32 f = forward_f32(o, x, r, l, w1, w3, w2, b, i);
-    out = f.out;
-    if (r.defined()) lg = f.logits;
+    out = forward_f32(o, x, l.defined() && l.dim() != 2 ? l.flatten(0, -2) : l, w1, w3, w2, b, i).out;
   }
-  return {out, lg.defined() ? OptTensor(lg) : std::nullopt, want_routing ? OptTensor(routing) : std::nullopt};
+  return {out, r.defined() ? OptTensor(l) : std::nullopt, want_routing ? OptTensor(routing) : std::nullopt};
 }
 
 }  // namespace

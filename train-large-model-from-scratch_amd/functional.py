@@ -136,10 +136,11 @@ def moe_ffn_f32(x: torch.Tensor, logits: torch.Tensor, w1: torch.Tensor, w3: tor
 
 
 def routed_moe_f32(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor, w2: torch.Tensor, k: int):
-    """(MoE(x), router logits) for x [T,H], all fp32: `nn.Linear`'s product and `moe_ffn_f32` as one autograd node, whose
-    backward adds the router path's input gradient in the k-row-sum kernel."""
+    """(MoE(x), router logits) for x [..., H], all fp32: `nn.Linear`'s product and `moe_ffn_f32`, the router path's gradients
+    worked out along with the experts'.  The logits are between the two as if they were called one after the other: where a hook
+    is on them, their gradient is retained or asked for, it is handed to the product's own backward instead."""
     out, logits, _ = _lib.native().layer_f32(x, router_weight, None, None, w1, w3, w2, None, k, False)
-    return out, logits
+    return out.reshape(x.shape), logits
 
 
 def prenorm_moe(x: torch.Tensor, norm_weight: torch.Tensor, router_weight: torch.Tensor,

@@ -199,16 +199,15 @@ class MoE(nn.Module):
         return moe_ffn_f32(x2d, logits2d, w1, w3, w2, k)
 
     @torch._dynamo.disable
-    def _layer_f32(self, x2d: torch.Tensor):
-        return routed_moe_f32(x2d, self.router.weight, self.experts_gate_weights, self.experts_up_weights,
+    def _layer_f32(self, x: torch.Tensor):
+        return routed_moe_f32(x, self.router.weight, self.experts_gate_weights, self.experts_up_weights,
                               self.experts_down_weights, self.top_k)
 
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         B, T, D = x.size()
         if self._runs_in_fp32(x):
             if not torch.compiler.is_compiling() and self._router_is_plain():
-                out, gate_logits = self._layer_f32(x.reshape(B * T, D))
-                return out.reshape(B, T, D), gate_logits.reshape(B, T, self.num_experts)
+                return self._layer_f32(x)
             gate_logits = self.router(x)  # fp32 product and fp32 gradients, as nn.Linear gives them
             ffn = traced.moe_ffn_f32 if torch.compiler.is_compiling() else self._experts_f32
             out = ffn(x.reshape(B * T, D), gate_logits.reshape(B * T, self.num_experts),
