@@ -57,6 +57,29 @@ def test_gradients(pkg, lib, T, E, k, H, I, outs):
         close(name, a, b)
 
 
+@pytest.mark.parametrize("T,E,k,H", [(3001, 64, 2, 260), (2500, 128, 3, 1024), (63, 64, 2, 128), (65, 128, 2, 64), (9000, 512, 2, 32)])
+@pytest.mark.parametrize("share", ["all", "falling"])
+def test_router_weight_gradient_of_skewed_routing(pkg, lib, T, E, k, H, share):
+    """All tokens with the same k experts, which lie apart, or most with a few: parts of an expert's rows and experts without any."""
+    print("fp32 router, skewed", T, E, k, H, share, flush=True)
+    (x, wr, w1, w3, w2), dy, _ = inputs(T, E, H, 16, T + E)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    order = torch.randperm(E, generator=g, device="cuda").float()
+    bias = -4.0 * order if share == "all" else -1.5 * torch.log1p(order)
+    with torch.no_grad():  # (the last column of x is one)
+        x[:, -1] = 1.0
+        wr[:, -1] = bias
+    leaves = [x, wr, w1, w3, w2]
+    res = []
+    for call in both(pkg, T, E, k, H, 16):
+        out, logits = call(*leaves)
+        res.append(torch.autograd.grad(out, leaves[1], dy)[0])
+    rows = torch.bincount(logits.topk(k, -1).indices.flatten(), minlength=E)
+    assert share != "all" or int((rows == T).sum()) >= 1
+    close("dwr", *res)
+    assert not bool(res[0][rows == 0].any())
+
+
 @pytest.mark.parametrize("wanted", [(0,), (1,), (0, 1), (2, 4), (1, 3)])
 def test_some_gradients(pkg, lib, wanted):
     T, E, k, H, I = 200, 8, 2, 128, 64

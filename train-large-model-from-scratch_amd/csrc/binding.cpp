@@ -44,8 +44,8 @@ int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int3
 int moe_f32_permute_bwd_router(const float* dxp, const int32_t* row_to_pos, const float* gates, const float* dgates,
                                const int32_t* ids, const float* wr, int64_t T, int64_t H, int64_t k, float* dsel, float* dx,
                                void* stream);
-int moe_f32_router_wgrad_slices(int64_t R, int64_t H, int64_t E);
-int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs, int64_t R, int64_t H, int64_t E, float* part,
+int64_t moe_f32_router_wgrad_floats(int64_t R, int64_t H, int64_t E);
+int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs, int64_t R, int64_t H, int64_t E, float* partial,
                          float* dwr, void* stream);
 int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
                    int64_t E, int64_t R, int64_t H, int64_t I, float* dw1, float* dw3, float* dw2, void* stream);
@@ -761,8 +761,8 @@ struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
     const int32_t* r2p = r.part(routing, Routing::ROW_TO_POS);
     void* s = stream_of(kept_buf);
     const int64_t rh = up(R * H, 64), ri = up(R * I, 64);
-    const int slices = inside && need(WR) ? moe_f32_router_wgrad_slices(R, H, E) : 1;
-    const Tensor scratch = empty({2 * rh + 2 * ri + 2 * up(R, 64) + (slices > 1 ? slices * E * H : 0) + 64}, at::kFloat, kept_buf);
+    const int64_t partial = inside && need(WR) ? moe_f32_router_wgrad_floats(R, H, E) : 0;
+    const Tensor scratch = empty({2 * rh + 2 * ri + 2 * up(R, 64) + partial + 64}, at::kFloat, kept_buf);
     float* dyp = scratch.data_ptr<float>();
     float *dxp = dyp + rh, *dg = dxp + rh, *du = dg + ri, *dgates = du + ri, *dsel = dgates + up(R, 64), *part = dsel + up(R, 64);
     CALL(moe_f32_combine_bwd, dout.data_ptr<float>(), want_gates ? y : nullptr, gates, p2r, T, R, H, k, dyp,

@@ -133,18 +133,48 @@ __global__ __launch_bounds__(256) void f32_permute_bwd_router_kernel(
 
 // dwr[e, :] = sum over the expert's rows of dsel * xp[row, :]: what dlogits^T x comes to, whose other entries are zero, in one
 // pass over the rows that the experts' products read anyway.  256 columns a workgroup, a row a wave, eight of them requested at
-// once, the waves' sums added in order; slice blockIdx.z of gridDim.z of the expert's rows, summed up by the next kernel.
+// once, the waves' sums added in order.  Workgroup y of a column is segment y of the rows: an expert of more than L rows is cut into
+// parts, whose sums the next kernel adds up.
 constexpr int RW_WAVES = 8, RW_COLS = 4 * MOE_WAVE;
+struct RowCut {
+  const int32_t* offs;
+  int E, L;
+  // (an expert without rows is a part too: its gradient is zero)
+  __device__ __forceinline__ int parts(int rows) const { return rows <= L ? 1 : (int)(((long long)rows + L - 1) / L); }
+  __device__ __forceinline__ int rows(int e) const { return e < E ? offs[e + 1] - offs[e] : 0; }
+  // Number of segments of the experts before e, by a whole wave; e past the last: those of all.
+  __device__ __forceinline__ int before(int e) const {
+    int n = 0;
+    for (int b = 0; b < e; b += MOE_WAVE) {
+      const int at = b + lane_id();
+      n += read_lane(wave_inclusive(at < e ? parts(rows(at)) : 0), MOE_WAVE - 1);
+    }
+    return n;
+  }
+};
 __global__ __launch_bounds__(RW_WAVES* MOE_WAVE) void f32_router_wgrad_kernel(const float* __restrict__ xp,
-                                                                            const float* __restrict__ dsel,
-                                                                            const int32_t* __restrict__ offs, int H,
-                                                                            float* __restrict__ out) {
+                                                                            const float* __restrict__ dsel, const RowCut cut,
+                                                                            int H, float* __restrict__ partial,
+                                                                            float* __restrict__ dwr) {
   constexpr int AHEAD = 8;
   __shared__ f32x4 part[RW_WAVES][MOE_WAVE];
   const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE)), col = blockIdx.x * RW_COLS + lane * 4;
-  const int e = blockIdx.y, E = gridDim.y, first = offs[e];
-  const long long n = offs[e + 1] - first;
-  const int lo = first + (int)(n * blockIdx.z / gridDim.z), hi = first + (int)(n * (blockIdx.z + 1) / gridDim.z);
+  const int seg = blockIdx.y;
+  int e = -1, parts = 0, j = 0;
+  for (int b = 0, carry = 0; b < cut.E; b += MOE_WAVE) {
+    const int p = b + lane < cut.E ? cut.parts(cut.rows(b + lane)) : 0, upto = carry + wave_inclusive(p);
+    const unsigned long long past = __ballot(upto > seg);
+    if (past) {
+      const int f = __builtin_ctzll(past);
+      e = b + f, parts = read_lane(p, f), j = seg - (read_lane(upto, f) - parts);
+      break;
+    }
+    carry = read_lane(upto, MOE_WAVE - 1);
+  }
+  if (e < 0) return;
+  const int first = cut.offs[e];
+  const long long n = cut.offs[e + 1] - first;
+  const int lo = first + (int)(n * j / parts), hi = first + (int)(n * (j + 1) / parts);
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int r = lo + wv; r < hi; r += RW_WAVES * AHEAD) {
     f32x4 v[AHEAD];
@@ -164,15 +194,30 @@ __global__ __launch_bounds__(RW_WAVES* MOE_WAVE) void f32_router_wgrad_kernel(co
   if (wv || col >= H) return;
 #pragma unroll
   for (int w = 1; w < RW_WAVES; ++w) acc += part[w][lane];
-  *reinterpret_cast<f32x4*>(out + ((long long)blockIdx.z * E + e) * H + col) = acc;
+  float* out = parts > 1 ? partial + (long long)seg * H : dwr + (long long)e * H;
+  *reinterpret_cast<f32x4*>(out + col) = acc;
 }
-__global__ __launch_bounds__(256) void f32_sum_slices_kernel(const float* __restrict__ part, int slices, long long n4,
-                                                             float* __restrict__ out) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n4) return;
-  f32x4 acc = reinterpret_cast<const f32x4*>(part)[i];
-  for (int s = 1; s < slices; ++s) acc += reinterpret_cast<const f32x4*>(part)[s * n4 + i];
-  reinterpret_cast<f32x4*>(out)[i] = acc;
+// dwr[e, :] of the experts that were cut: four waves, each every fourth part in ascending order, and the four sums in order.
+constexpr int RS_WAVES = 4;
+__global__ __launch_bounds__(RS_WAVES* MOE_WAVE) void f32_router_wgrad_sum_kernel(const float* __restrict__ partial,
+                                                                                const RowCut cut, int H,
+                                                                                float* __restrict__ dwr) {
+  __shared__ f32x4 part[RS_WAVES][MOE_WAVE];
+  const int e = blockIdx.y, parts = uniform(cut.parts(cut.rows(e)));
+  if (parts == 1) return;
+  const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE)), col = blockIdx.x * RW_COLS + lane * 4;
+  const float* from = partial + (long long)cut.before(e) * H + col;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  if (col < H) {
+#pragma unroll 8
+    for (int j = wv; j < parts; j += RS_WAVES) acc += *reinterpret_cast<const f32x4*>(from + (long long)j * H);
+  }
+  part[wv][lane] = acc;
+  __syncthreads();
+  if (wv || col >= H) return;
+#pragma unroll
+  for (int w = 1; w < RS_WAVES; ++w) acc += part[w][lane];
+  *reinterpret_cast<f32x4*>(dwr + (long long)e * H + col) = acc;
 }
 
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.f / (1.f + expf(-x)); }
@@ -294,15 +339,25 @@ int moe_f32_permute_bwd_router(const float* dxp, const int32_t* row_to_pos, cons
   return moe_launch_status();
 }
 
-// Slices of an expert's rows: two workgroups for every compute unit, but eight rows for every wave where they are dealt evenly.
-int moe_f32_router_wgrad_slices(int64_t R, int64_t H, int64_t E) {
-  const int64_t blocks = E * ((H + RW_COLS - 1) / RW_COLS), want = 2 * (int64_t)moe_compute_units() / blocks;
-  const int64_t most = R / E / (8 * RW_WAVES), n = want < most ? want : most;
-  return (int)(n < 1 ? 1 : n > 64 ? 64 : n);
+// The most rows of a segment: two workgroups for every compute unit, but eight rows for every wave.  (By rows, not so many parts
+// an expert: the longest expert's rows are what a workgroup walks one after the other.  Every expert cut alike by the mean, and here, whole
+// passes, us: 16384 tokens all with 1 of 128 experts, 1024 <-> 64, 1688 -> 1413; evenly 512 -> 507; 8192 all with 2 of 64, 2048 <-> 128, 1208 ->
+// 1097; 4717, 2 of 64, 768 <-> 384, two thirds with two, 877 -> 843, evenly 622 and 629, the same kernels' times.)
+static int router_segment_rows(int64_t R, int64_t H, int64_t E) {
+  const int64_t cols = (H + RW_COLS - 1) / RW_COLS, cus = moe_compute_units();
+  const int64_t want = 2 * cus / cols > 0 ? 2 * cus / cols : 1;
+  int64_t L = (R + want - 1) / want;
+  if (E * cols >= cus && L < 2 * (R / E)) L = 2 * (R / E);  // (the experts alone are enough workgroups: none of about the mean is cut)
+  return (int)(L < 8 * RW_WAVES ? 8 * RW_WAVES : L);
 }
 
-// `part`: the slices' results, slices * E * H floats, where there is more than one.
-int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs, int64_t R, int64_t H, int64_t E, float* part,
+int64_t moe_f32_router_wgrad_floats(int64_t R, int64_t H, int64_t E) {
+  const int64_t L = router_segment_rows(R, H, E);
+  return R > L ? (R / L + E) * H : 0;
+}
+
+// `partial`: moe_f32_router_wgrad_floats floats.
+int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs, int64_t R, int64_t H, int64_t E, float* partial,
                          float* dwr, void* stream) {
   if (int rc = check_rows(R, H)) return rc;
   if (E <= 0) return MOE_ERR_SHAPE;
@@ -310,15 +365,16 @@ int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs
   MOE_CHECK_PTR(xp);
   MOE_CHECK_PTR(dwr);
   if (!dsel || !offs) return MOE_ERR_NULL;
-  const int slices = moe_f32_router_wgrad_slices(R, H, E);
-  if (slices > 1) MOE_CHECK_PTR(part);
+  const RowCut cut{offs, (int)E, router_segment_rows(R, H, E)};
+  const bool any = R > cut.L;  // (else no expert can have more)
+  if (any) MOE_CHECK_PTR(partial);
   const hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(f32_router_wgrad_kernel, dim3((unsigned)((H + RW_COLS - 1) / RW_COLS), (unsigned)E, (unsigned)slices),
-                     dim3(RW_WAVES * MOE_WAVE), 0, s, xp, dsel, offs, (int)H, slices > 1 ? part : dwr);
-  if (slices == 1) return moe_launch_status();
+  const unsigned cols = (unsigned)((H + RW_COLS - 1) / RW_COLS);
+  hipLaunchKernelGGL(f32_router_wgrad_kernel, dim3(cols, (unsigned)(R / cut.L + E)), dim3(RW_WAVES * MOE_WAVE), 0, s, xp, dsel, cut,
+                     (int)H, partial, dwr);
+  if (!any) return moe_launch_status();
   if (const int rc = moe_launch_status()) return rc;
-  const long long n4 = (long long)E * H / 4;
-  hipLaunchKernelGGL(f32_sum_slices_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, part, slices, n4, dwr);
+  hipLaunchKernelGGL(f32_router_wgrad_sum_kernel, dim3(cols, (unsigned)E), dim3(RS_WAVES * MOE_WAVE), 0, s, partial, cut, (int)H, dwr);
   return moe_launch_status();
 }
 
