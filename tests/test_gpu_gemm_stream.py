@@ -61,3 +61,34 @@ def test_weight_gradients(pkg, lib, counts, dtype, N):
         ref = a[s].float().T @ b[s].float()
         bound = ref.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0) + 2.0 ** -22 * K * K ** 0.5
         assert bool(((got[e].float() - ref).abs() <= bound).all()), (e, counts[e])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("E,H,I", [
+    (61, 1024, 88), (65, 1024, 88), (65, 1016, 88),   # small launches: bf16 results of 32.8, 34.9 and 34.6 MB, around the line and rows of no whole pieces
+    (24, 2048, 256), (3, 264, 264),                   # ... of 75 and 1.3 MB
+    (33, 1024, 1024), (512, 520, 8),                  # tiled ones: 208 and 12.8 MB
+])
+def test_results_on_both_sides_of_the_streaming_line(pkg, lib, E, H, I, dtype):
+    print("weight gradients, streaming", E, H, I, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(E)
+    counts = torch.randint(0, 60, (E,), generator=torch.Generator().manual_seed(E))
+    ids = torch.arange(E).repeat_interleave(counts).cuda()
+    R = len(ids)
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).to(torch.bfloat16)
+    x, dy = r(R, H), r(R, H)
+    ws = [w.to(dtype).requires_grad_(True) for w in (r(E, I, H, std=0.05), r(E, I, H, std=0.05), r(E, H, I, std=0.05))]
+    pkg.experts_rows(x, ids, *ws).backward(dy)
+    both = [w.detach().clone().requires_grad_(True) for w in ws]
+    for w in both:  # (added to zeros: ordinary stores)
+        w.grad = torch.zeros_like(w)
+    pkg.experts_rows(x, ids, *both, accumulate_into_grad=True).backward(dy)
+    for n, (a, b) in enumerate(zip(ws, both)):
+        assert torch.equal(a.grad, b.grad), n
+    one = 7 % E  # one expert's against fp32 products of its rows
+    s = ids == one
+    xe, de, w1, w3, w2 = x[s].float(), dy[s].float(), *[w.detach()[one].float() for w in ws]
+    gate, up = xe @ w1.T, xe @ w3.T
+    act = (torch.nn.functional.silu(gate) * up).to(torch.bfloat16).float()
+    ref = de.T @ act
+    assert (ws[2].grad[one].float() - ref).norm() <= 1e-2 * ref.norm()  # (act and the result each rounded to bf16)

@@ -1219,8 +1219,8 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK, TO>, attr_done[1], a,
                                2 * a.n_tiles * row_slots(a.R, a.E, ROW_TILE), s);
 }
-// Nothing here reads the results again.  With few rows an expert they come as fast as the operands do, and as streaming
-// stores they leave the operands' lines in L2 alone.  Rows an expert and time, streaming over ordinary, three results in
+// With few rows an expert the results come as fast as the operands do, and as streaming stores they leave the operands' lines in L2
+// alone; what reads small ones afterwards would miss them (MOE_STREAMED_RESULTS).  Rows an expert and time, streaming over ordinary, three results in
 // turn so that none is still cached: 64 experts of 2048 <-> 1024, bf16 and fp32: 256, 0.86 and 0.83; 512, 0.93 and 0.91; 768, 1.01 and 1.04;
 // 1024, 1.00 and 1.01; 2048, 1.00 and 1.00.  128 of 1024 <-> 256, 128 to 512 rows 0.93 to 0.96 and 0.84 to 0.92; 16 of 4096 <-> 1536, 1024 rows
 // 0.95 and 0.95; by Zipf's shares, 500 rows of 64 1.00 and 0.85.
@@ -1228,13 +1228,14 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
 template <typename OutT>
 int launch_wgrad(const WgradArgs& args, hipStream_t s) {
   WgradArgs w = args;
-  long long tiles = 0;
+  long long tiles = 0, bytes = 0;
+  for (int i = 0; i < w.n; ++i) bytes += (long long)w.p[i].E * w.p[i].M * w.p[i].N * (int)sizeof(OutT);
   for (int i = 0; i < w.n; ++i) {
     GemmArgs& a = w.p[i];
     a.n_tiles = (a.N + CfgMain::BN - 1) / CfgMain::BN;
     a.m_slots = (a.M + CfgMain::BM - 1) / CfgMain::BM;
     a.by_n_tiles.set(a.n_tiles), a.by_m_slots.set(a.m_slots);
-    a.streaming = a.R <= 512ll * a.E && a.N * (int)sizeof(OutT) % 64 == 0;
+    a.streaming = bytes >= MOE_STREAMED_RESULTS && a.R <= 512ll * a.E && a.N * (int)sizeof(OutT) % 64 == 0;
     const long long n = (long long)a.n_tiles * a.m_slots * a.E;
     tiles = tiles > n ? tiles : n;
   }

@@ -44,6 +44,12 @@ struct MoeWgradStack {
   int dtype, accumulate;
   void* out2;  // moe_gemm_wgrad_all: an expert's rows M / 2 .. M - 1 go here (NULL: all to out)
 };
+// Weight gradients leave with streaming stores from so many bytes of results in a launch on, an eighth of the memory-side cache: a
+// model of a few such layers finds smaller ones there when it adds them up, clips them or steps.  Pass, pass with its gradients added
+// to another's, and pass with their norms taken, us, ordinary stores -> streaming: 1.5 MB 49 -> 49, 99 -> 100, 66 -> 70; 25 MB 128 -> 128, 256 ->
+// 257, 138 -> 143, and 298 -> 296, 608 -> 605, 311 -> 319; 48 MB 157 -> 154, 326 -> 325, 181 -> 192; 96 MB 204 -> 191, 465 -> 452, 234 -> 249;
+// 144 MB 183 -> 166, 461 -> 432, 268 -> 255; 192 MB 361 -> 331, 821 -> 767, 423 -> 403; 240 MB 405 -> 369, 943 -> 869, 495 -> 474.
+constexpr int64_t MOE_STREAMED_RESULTS = 32 << 20;
 // moe_gemm_wgrad, and moe_gemm_wgrad_pair where there is an out2, of up to three stacks with results of one kind in one launch.
 int moe_gemm_wgrad_all(const MoeWgradStack* stacks, int n, const int32_t* offs, int64_t E, int64_t R, void* stream);
 // Bytes of each stack's part for R rows.

@@ -37,6 +37,7 @@ struct MultiArgs {
   int T, r_rows, r_slices;
   int each, e_each, r_each;  // tiles of a segment to an XCD, its jobs of all segments, its router jobs
   int r_first;               // the router's jobs come first, or last
+  int streaming;             // results that replace what is there leave with streaming stores, where rows allow it
   float per_each, r_per_tiles;
 };
 // n / d of a wave-uniform n, 1 / d given (exact: n is far below 2^23)
@@ -237,11 +238,11 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   const long long MN = (long long)st.M * st.N;
   char* out = partial ? (char*)(st.part + sg.slot * MN) : (char*)st.out + sg.e * MN * (wide ? 4 : 2);
   const bool add = !partial && st.accumulate;
-  // (streaming stores of whole pieces of 64 bytes, a row's in one instruction: the operands' lines stay in L2.  Ordinary ones ->
+  // (large results: streaming stores of whole pieces of 64 bytes, a row's in one instruction: the operands' lines stay in L2.  Ordinary ones ->
   // these, whole steps, us: 75 tokens, 3 of 96 experts, 384 <-> 1152, 234 -> 193; 2753 tokens, 24 experts, 1520 <-> 576, fp32, 276 -> 218; of
   // 100 drawn steps of one or two rounds of jobs none is slower.  With ends inside such a piece, which memory then reads
   // first, some are: 958 rows of 64, 3128 <-> 1064, 756 -> 1028 in the tiled kernel)
-  const bool stream = !partial && !st.accumulate && st.N * (wide ? 4 : 2) % 64 == 0;
+  const bool stream = p.streaming && !partial && !st.accumulate && st.N * (wide ? 4 : 2) % 64 == 0;
 #pragma unroll
   for (int i = 0; i < WFM; ++i) {
 #pragma unroll
@@ -401,6 +402,9 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
     fill(a.s[i], stacks[i]);
     a.tiles += a.s[i].tiles;
   }
+  int64_t bytes = 0;
+  for (int i = 0; i < n_stacks; ++i) bytes += E * stacks[i].M * stacks[i].N * (a.s[i].out_f32 ? 4 : 2);
+  a.streaming = bytes >= MOE_STREAMED_RESULTS;
   a.n_stacks = n_stacks;
   a.offs = offs;
   a.E = (int)E;
