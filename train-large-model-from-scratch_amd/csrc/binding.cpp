@@ -715,6 +715,9 @@ bool logits_observed(torch::autograd::Node* node) {
   return true;
 }
 
+// The logits of the layer's own product, whose leading dimensions are x's, as a matrix; those that a caller brings as they are.
+Tensor flat(const Tensor& logits, const Tensor& wr) { return wr.defined() && logits.dim() != 2 ? logits.flatten(0, -2) : logits; }
+
 // Given the router weight too, `logits` are the fp32 product of x with it, made by the library in a graph of its own: the
 // layer hands their gradient on to it only where somebody observes it, and else works out what it comes to in x and in the
 // weight along with its own.
@@ -725,7 +728,7 @@ struct LayerF32Node : torch::autograd::Function<LayerF32Node> {
                                const Tensor& w1, const Tensor& w3, const Tensor& w2, const OptTensor& bias_,
                                const OptTensor& ids_, const Layer& o) {
     const Tensor &wr = value(wr_), &logits = value(logits_), &bias = value(bias_), &ids = value(ids_);
-    const OutputsF32 f = forward_f32(o, x, logits.defined() && logits.dim() != 2 ? logits.flatten(0, -2) : logits, w1, w3, w2, bias, ids);
+    const OutputsF32 f = forward_f32(o, x, flat(logits, wr), w1, w3, w2, bias, ids);
     ctx->save_for_backward({f.kept, f.routing, f.w[0], f.w[1], f.w[2], wr});
     ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), o.k, logits.defined(),
                                                 Present{true, wr.defined(), logits.defined(), true, true, true,
@@ -831,7 +834,7 @@ std::tuple<Tensor, OptTensor, OptTensor> layer_f32(const Tensor& x_, const OptTe
     out = LayerF32Node::apply(x, wr, l.defined() ? OptTensor(l) : std::nullopt, w1, w3, w2, bias, ids, o)[0];
   } else {
     const at::NoGradGuard off;
-    out = forward_f32(o, x, l.defined() && l.dim() != 2 ? l.flatten(0, -2) : l, w1, w3, w2, b, i).out;
+    out = forward_f32(o, x, flat(l, r), w1, w3, w2, b, i).out;
   }
   return {out, r.defined() ? OptTensor(l) : std::nullopt, want_routing ? OptTensor(routing) : std::nullopt};
 }
