@@ -38,3 +38,23 @@ def test_rows_go_where_they_came_from(pkg, counts, H, I):
     for height in (0, 1, 64, 128, 256):
         for a, b in zip(passed(torch.bfloat16, height), want):
             assert torch.equal(a, b), height
+
+
+def test_no_room_is_held_for_rows_that_stay_in_place(pkg, lib):
+    """Besides the results a direction holds one buffer of the size of the rows: those by expert, and the output's gradient by expert."""
+    print("rows in place, memory", flush=True)
+    R, E, H, I = 8192, 4, 2048, 8
+    r = lambda *s: torch.randn(*s, device="cuda").to(torch.bfloat16)
+    x, dy, ws, ids = r(R, H).requires_grad_(True), r(R, H), [r(E, I, H), r(E, I, H), r(E, H, I)], torch.randint(0, E, (R,), device="cuda")
+    rows = R * H * 2
+
+    def held(call):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        result = call()
+        return result, torch.cuda.max_memory_allocated() - before
+
+    out, forward = held(lambda: pkg.experts_rows(x, ids, *ws))
+    _, backward = held(lambda: out.backward(dy))
+    assert forward < 2.5 * rows and backward < 2.5 * rows, (forward / rows, backward / rows)

@@ -39,6 +39,8 @@ int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, fl
                              int64_t T, int64_t H, int64_t E, int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
                              int32_t* ids, float* gates, void* table, void* stream);
 int moe_selected_layer_forward(const moe_layer_forward_args* a, const void* table, void* stream);
+int64_t moe_forward_scratch(const moe_layer_forward_args* a);
+int64_t moe_backward_scratch(const moe_layer_backward_args* a);
 int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
                    int64_t I, float* g, float* u, float* act, void* stream);
 int moe_f32_permute_bwd_router(const float* dxp, const int32_t* row_to_pos, const float* gates, const float* dgates,
@@ -331,8 +333,6 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   const Kept kept(R, H, E, I, o.train);
   f.kept = empty({kept.total}, at::kByte, x);
   char* base = (char*)f.kept.data_ptr();
-  const int64_t bytes = std::max<int64_t>(moe_layer_scratch_bytes(T, H, E, I, k, 0), 256);
-  const Tensor scratch = empty({bytes}, at::kByte, x);
   Tensor ids = ids_;
   moe_layer_forward_args a{};
   a.T = T, a.H = H, a.E = E, a.I = I, a.k = k;
@@ -357,6 +357,8 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   a.xp = (uint16_t*)base;
   a.gu = o.train ? base + kept.gu : nullptr;
   a.act = (uint16_t*)(base + kept.act);
+  const int64_t bytes = std::max<int64_t>(moe_forward_scratch(&a), 256);
+  const Tensor scratch = empty({bytes}, at::kByte, x);
   a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
   check(moe_selected_layer_forward(&a, ptr(table), s), "moe_layer_forward");
   if (o.routing_out) *o.routing_out = f.routing;
@@ -484,8 +486,6 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
     const Routing r(R, E);
     const Kept kept(R, H, E, I, true);
     const char* base = (const char*)kept_buf.data_ptr();
-    const int64_t bytes = std::max<int64_t>(moe_layer_scratch_bytes(T, H, E, I, k, 1), 256);
-    const Tensor scratch = empty({bytes}, at::kByte, kept_buf);
     void* s = stream_of(kept_buf);
     moe_layer_backward_args a{};
     a.T = T, a.H = H, a.E = E, a.I = I, a.k = k;
@@ -508,6 +508,8 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
     if (dwr.defined()) a.dwr = dwr.data_ptr(), a.dwr_dtype = dt(dwr);
     if (dx.defined()) a.dx = dx.data_ptr(), a.dx_dtype = dt(dx);
     a.dxp = (uint16_t*)ptr(dxp);
+    const int64_t bytes = std::max<int64_t>(moe_backward_scratch(&a), 256);
+    const Tensor scratch = empty({bytes}, at::kByte, kept_buf);
     a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
     check(moe_layer_backward(&a, s), "moe_layer_backward");
     for (int i = 0; i < 3; ++i)

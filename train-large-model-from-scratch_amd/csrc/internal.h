@@ -28,6 +28,11 @@ int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const
                            const int32_t* ids, const uint16_t* wr, int64_t T, int64_t H, int64_t k, int64_t ld, void* dlogits,
                            int dlogits_dtype, void* dx, int dx_dtype, hipStream_t s);
 
+// Bytes of scratch that a call with these arguments (all but the scratch filled in) uses, no more than moe_layer_scratch_bytes says:
+// rows that stay in place need no buffer for them (layer.hip).
+int64_t moe_forward_scratch(const moe_layer_forward_args* a);
+int64_t moe_backward_scratch(const moe_layer_backward_args* a);
+
 // fp32 to bf16, two tensors of multiples of 8 elements in one launch (dispatch.hip).
 int moe_cast_two(const float* a, uint16_t* to_a, int64_t na, const float* b, uint16_t* to_b, int64_t nb, void* stream);
 

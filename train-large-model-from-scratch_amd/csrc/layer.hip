@@ -217,8 +217,8 @@ struct Scratch {
 struct FwdScratch {
   uint16_t* y;
   void* dispatch;
-  FwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t k) {
-    y = (uint16_t*)s.take(T * k * H * 2);
+  FwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t k, bool with_y = true) {
+    y = (uint16_t*)s.take(with_y ? T * k * H * 2 : 0);
     dispatch = s.take(order_bytes(T, E, k));
   }
 };
@@ -269,11 +269,11 @@ struct BwdScratch {
   uint16_t *dyp, *dg, *dxp;
   float *part, *wpart[3], *rpart;
   uint16_t* dlogits;
-  BwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
+  BwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, bool with_dxp = true) {
     const int64_t R = T * k;
     dyp = (uint16_t*)s.take(R * H * 2);
     dg = (uint16_t*)s.take(R * I * 4);
-    dxp = (uint16_t*)s.take(R * H * 2);
+    dxp = (uint16_t*)s.take(with_dxp ? R * H * 2 : 0);
     part = (float*)s.take(moe_dgate_blocks(I) * R * 4);
     const RouterSlices rs = router_slices(T, H, E);
     dlogits = (uint16_t*)s.take(T * rs.Ep * 4);
@@ -281,6 +281,16 @@ struct BwdScratch {
     for (float*& w : wpart) w = (float*)s.take(wgrad_multi(E, I, H, R) ? moe_wgrad_multi_part_bytes(R, H, I) : 0);
   }
 };
+
+// Rows of one slot without a gate: down leaves them where they came from, and there is nothing to combine.  (That pass, and
+// its counterpart behind the gate/up input gradient, each move every row in and out: 32768 rows of 16 experts, 4096 wide, 82 us
+// of 3700 either way; a step of 24 drawn sizes, 288 to 46000 rows, 1.05 to 1.15 times as fast without the two.)
+bool out_in_place(const moe_layer_forward_args& a) { return a.k == 1 && !a.gates && !a.residual && a.out_dtype == MOE_DT_BF16; }
+// (dxp is dx but for the order, and nothing else is to be added)
+bool dx_in_place(const moe_layer_backward_args& a) {
+  const bool router = a.wr && !a.dgates;
+  return a.k == 1 && a.dx && !a.dxp && !router && a.dx_dtype == MOE_DT_BF16;
+}
 
 bool dtype_ok(int64_t d) { return d == MOE_DT_BF16 || d == MOE_DT_F32; }
 
@@ -318,6 +328,20 @@ extern "C" int64_t moe_layer_scratch_bytes(int64_t T, int64_t H, int64_t E, int6
   return s.at;
 }
 
+int64_t moe_forward_scratch(const moe_layer_forward_args* a) {
+  if (!sizes_ok(a->T, a->H, a->E, a->I, a->k)) return 0;
+  Scratch s{nullptr, 0, 0};
+  FwdScratch(s, a->T, a->H, a->E, a->k, !out_in_place(*a));
+  return s.at;
+}
+
+int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
+  if (!sizes_ok(a->T, a->H, a->E, a->I, a->k)) return 0;
+  Scratch s{nullptr, 0, 0};
+  BwdScratch(s, a->T, a->H, a->E, a->I, a->k, a->dx && !a->dxp && !dx_in_place(*a));
+  return s.at;
+}
+
 // With `table` the selection is done, ids and gates are there, and so are its counts (moe_rmsnorm_router_count).
 static int layer_forward(const moe_layer_forward_args* a, const void* table, void* stream) {
   if (!a) return MOE_ERR_NULL;
@@ -343,7 +367,7 @@ static int layer_forward(const moe_layer_forward_args* a, const void* table, voi
   }
   if (a->logits && !a->gates) return MOE_ERR_NULL;
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
-  const FwdScratch ws(s, T, H, E, k);
+  const FwdScratch ws(s, T, H, E, k, !out_in_place(*a));
   if (!s.fits()) return MOE_ERR_WORKSPACE;
   if (a->logits && !table && moe_select_place_ok(a->logits, T, E, k)) {
     MOE_STEP("moe_select_place", moe_select_place(a->x, (int)a->x_dtype, a->logits, (int)a->logits_dtype, a->bias, T, H, E, k, a->ids,
@@ -380,10 +404,7 @@ static int layer_forward(const moe_layer_forward_args* a, const void* table, voi
   else
     MOE_STEP("moe_gemm_gateup_swiglu_fwd",
              moe_gemm_gateup_swiglu_fwd(a->xp, a->w1, a->w3, a->offs, E, R, H, I, nullptr, nullptr, a->act, stream));
-  // Rows of one slot without a gate: down leaves them where they came from, and there is nothing to combine.  (That pass, and
-  // its counterpart behind the gate/up input gradient, each move every row in and out: 32768 rows of 16 experts, 4096 wide, 82 us
-  // of 3700 either way; a step of 24 drawn sizes, 288 to 46000 rows, 1.05 to 1.15 times as fast without the two.)
-  if (k == 1 && !a->gates && !a->residual && a->out_dtype == MOE_DT_BF16) {
+  if (out_in_place(*a)) {
     MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_to(a->act, a->w2, a->offs, E, R, H, I, (uint16_t*)a->out, a->pos_to_row, stream));
     return 0;
   }
@@ -434,7 +455,7 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     if (a->dwr && (!router || !a->xn)) return MOE_ERR_NULL;
   }
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
-  const BwdScratch ws(s, T, H, E, I, k);
+  const BwdScratch ws(s, T, H, E, I, k, a->dx && !a->dxp && !dx_in_place(*a));
   if (!s.fits()) return MOE_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   uint16_t* dxp = a->dxp ? a->dxp : ws.dxp;
@@ -469,8 +490,7 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
   if (to_logits && !with_dx && R > 0)
     MOE_STEP("moe_router_bwd_from_blocks", moe_router_bwd_from_blocks(part, moe_dgate_blocks(I), a->gates, a->ids, a->row_to_pos, T,
                                                                       E, k, ld, dlogits, dlogits_dtype, st));
-  // (rows of one slot: dxp is dx but for the order, and nothing else is to be added)
-  const bool in_place = k == 1 && a->dx && !a->dxp && !(router && to_logits) && a->dx_dtype == MOE_DT_BF16;
+  const bool in_place = dx_in_place(*a);
   if (a->dx || a->dxp)
     MOE_STEP(pair ? "moe_gemm_dgrad_gateup_packed" : "moe_gemm_dgrad_gateup",
              moe_gemm_dgrad_gateup_to(dg, du, pair ? 2 * I : 0, a->w1, a->w3, a->offs, E, R, H, I,
