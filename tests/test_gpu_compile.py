@@ -141,9 +141,10 @@ def test_compiled_module_on_the_bf16_cores_for_fp32_calls(pkg, lib):
 
 
 def test_compiled_fp32_call_takes_the_fp32_operators(pkg, lib):
-    """fp32 parameters and input, no autocast: the compiled module stays one graph, runs the
-    fp32 pair of operators and gives the bits of the eager fp32 call (same kernels, same order;
-    the router product is the module's own nn.Linear in both)."""
+    """fp32 parameters and input, no autocast: the compiled module stays one graph, runs the fp32 pair of operators behind
+    its own nn.Linear and gives the bits of the eager fp32 call in the outputs and the experts' gradients.  The router path's
+    gradients are nn.Linear's there and worked out along with the experts' here: those of its weight and of x agree to
+    rounding, and to the bit with an eager call that hands the logits' gradient on."""
     traced = importlib.import_module(pkg.__name__ + ".traced")
     m, x, dy = _case(pkg, torch.float32)
     x2 = x.reshape(-1, 256).requires_grad_(True)
@@ -152,22 +153,25 @@ def test_compiled_fp32_call_takes_the_fp32_operators(pkg, lib):
     torch.library.opcheck(traced.ffn_f32_fwd, args,
                           test_utils=("test_schema", "test_faketensor", "test_autograd_registration"))
 
-    def run(mod):
+    def run(mod, observe=False):
         m.zero_grad(set_to_none=True)
         xi = x.clone().requires_grad_(True)
         out, lg = mod(xi)
+        if observe:
+            lg.retain_grad()
         out.backward(dy)
         return [out.detach(), lg.detach(), xi.grad] + [p.grad.clone() for p in m.parameters()]
 
-    eager = run(m)
+    eager, observed = run(m), run(m, observe=True)
     compiled = run(torch.compile(m, backend="aot_eager", fullgraph=True))
     names = ["out", "gate_logits", "dx"] + [n for n, _ in m.named_parameters()]
-    for n, a, b in zip(names, eager, compiled):
+    for n, a, b, o in zip(names, eager, compiled, observed):
         assert a.dtype == torch.float32 and b.dtype == torch.float32 and a.shape == b.shape, n
         rel = ((a - b).norm() / a.norm().clamp_min(1e-30)).item()
-        _say(f"  {n}: rel diff compiled vs eager {rel:.2e}")
+        _say(f"  {n}: rel diff compiled vs eager {rel:.2e}, vs eager and observed {(o - b).abs().max().item():.2e}")
         assert rel < 1e-5, (n, rel)
-    assert torch.equal(eager[0], compiled[0])
+        assert torch.equal(a, b) or n in ("dx", "router.weight"), n
+        assert torch.equal(o, b), n
 
 
 @pytest.mark.parametrize("loss_on_logits", [False, True])

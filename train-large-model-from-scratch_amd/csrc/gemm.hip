@@ -333,8 +333,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   //                   last step | first fragment reads of stage kt+1 hide behind them
   // Where tile kt+3 lies is worked out behind the last request for an operand of kt+2, between two products: in front
   // of the first one the forty scalar instructions, with six 64-bit comparisons in the vector unit among them, held up both waves of a
-  // SIMD, which come from the same barrier.  Whole passes, us: 1531 tokens, 8 of 64 experts, forward, 258.8 -> 254.6; 8192, 2 of 8, 1024 <-> 512,
-  // 308.5 -> 305.0; 13 smaller ones 1.01 to 1.03; 16384 tokens of 64, where power is the bound, 4946 -> 4944.
+  // SIMD, which come from the same barrier.  Whole passes, us, in turn on one GPU: 1531 tokens, 8 of 64 experts, forward, 265.4 -> 262.6; 8192, 2 of
+  // 8, 1024 <-> 512, 317.7 -> 313.7; smaller ones 1.00 to 1.02; 16384 tokens of 64, where power is the bound, equal.
   auto body = [&](auto par_c, const Tile& t, int kt, TileSrc& ts) {
     constexpr int buf = decltype(par_c)::value;  // LDS stage of k-tile kt == parity of kt
     Stage& st = stg;                             // holds k-tile kt+1, refilled with kt+2, which lies at `ts`
@@ -394,11 +394,10 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   // one that the tile's last k-tile was read from.  The k-tiles of the next tile then follow this one's without a
   // break: its first is asked for in the last but one iteration and moves to the other stage in the last one, which
   // asks for its second.  A unit answers its loads and stores in order: loads sent between the stores of the strips
-  // wait behind them, and the stores behind the loads' trip to memory (65536 rows of 64 experts, 2048 <-> 1024, cycles
-  // of an epilogue with the next tile's loads in it and without: gate/up 11300, 6200; down 8600, 4000; weight
-  // gradients 9300, 4400, in fp32 17400, 8100; half of it comes back as a slower start of the next loop, and power takes
-  // its share: gate/up 528 -> 518 us, down 282 -> 272, weight gradients 786 -> 777, in fp32 925 -> 893; 32768 rows of 128,
-  // 1024 <-> 256: down 36.4 -> 35.1, dgrad-gate/up 53.4 -> 51.9).
+  // wait behind them, and the stores behind the loads' trip to memory (65536 rows of 64 experts, 2048 <-> 1024, with the next
+  // tile's loads in the epilogue and without: an epilogue takes half as long, half of that comes back as a slower start of the next
+  // loop, and power takes its share: gate/up 528 -> 518 us, down 282 -> 272, weight gradients 786 -> 777, in fp32 925 -> 893; 32768
+  // rows of 128, 1024 <-> 256: down 36.4 -> 35.1, dgrad-gate/up 53.4 -> 51.9).
   // (the SwiGLU-backward epilogue needs the staging registers' room for its g/u rows: the next tile's first k-tile
   // moves to LDS all the same, and its second is asked for during the last strip, when that room is free.  With the first
   // strip's g and u on their way behind the last products, dgrad-down of 131072 rows of 64 experts, 2048 <-> 1024, 610 -> 596 us;
@@ -683,8 +682,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   };
 
   // ---- the tile loop
-  // At the top of the loop the first k-tile of `cur` is already on its way into the staging
-  // registers (requested before the previous tile's epilogue).
+  // At the top of the loop the first k-tile of `cur` has been asked for: with `staged` it sits in LDS stage s0 and the second
+  // is on its way into the staging registers, else the first is.
   auto request_k = [&](const Tile& t, int kt) {
     if (kt < t.nkt) {
       load_tile(t, kt, stg);
@@ -699,7 +698,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   Tile cur;
   if (t_next >= t_hi || !locate(tile_at(t_next), cur)) return;
   request_first(cur);
-  bool staged = false;  // k-tile 0 of `cur` already sits in LDS stage `s0`, k-tile 1 is on its way
+  bool staged = false;
   int s0 = 0;           // the LDS stage of the tile's first k-tile; they alternate from there
 #pragma unroll
   for (int i = 0; i < FM; ++i) zero_row(i);  // later tiles find them cleared by the epilogue
@@ -721,7 +720,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     }
     const bool idle =
         (MODE != WGRAD) && __builtin_amdgcn_readfirstlane((int)(wm * WTM >= cur.row_end - cur.row0)) != 0;
-    // where the next tile lies is worked out now (a binary search in LDS and some address
+    // where the next tile lies is worked out now (a count over the lanes, a trip to LDS and some address
     // arithmetic), in the shadow of this tile's first MFMAs, not between the tiles
     Tile nxt;
     t_next += t_step;
@@ -851,7 +850,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     if (!idle) epilogue(cur, late_request);
     if (!more) break;
     if (!requested) request_next();
-    lds_barrier();  // every wave is done with its strip, and stage 0 is complete if staged
+    lds_barrier();  // every wave is done with its strip, and stage s0 is complete if staged
     cur = nxt;
   }
 }

@@ -225,13 +225,13 @@ struct FwdScratch {
 
 // Whether the weight gradients go to the kernel that takes all stacks at once (wgrad.hip).  Decided from shapes alone: where
 // one stack's 256 x 256 tiles are at most one for every compute unit, and up to four where its launch of 128 x 128 tiles, three to
-// a compute unit, comes to no more rounds than the tiled kernel's launches do (one for w2's stack, one or two for the others),
-// each of which ends in a partial round and pads the matrices to 256.  A round of either takes about as long: 4 us and 0.03 for each row
-// of an expert, another 4.4 with fp32 results.  (64 tiles, Zipf: a step of 8192 tokens 406 -> 362 us; 216 tiles: 401 -> 395; 512
-// tiles, 6 rounds against 8: 494 -> 514, not taken.  2006 tokens of 8 experts, 3136 <-> 704, 312 tiles, 6 rounds against 4.7: 326 -> 289;
-// 3959 tokens, 4 of 128 by Zipf's shares, 384 <-> 448, 6 against 6, 378 -> 223; 3390 of 64, 360 <-> 768, 5 against 4.5, 301 ->
-// 227.  Of 250 drawn layers of one to four rounds 131 are taken, their steps 1.13 times as fast in the mean where all three gradients
-// are wanted, 1.03 to 1.08 where one or two are, for which the rounds are counted as if all were; four are slower by 2 to 3 %.)
+// a compute unit, comes to no more rounds than tiles of 256 x 256 do where every problem (w2's stack, and one or two for the others) begins
+// a round of its own.  (The tiled kernel runs its problems in one launch, so it has fewer partial rounds than are counted here; it still pads
+// the matrices to 256 and has no part of an expert's rows to deal.  Where the line lies was measured with one launch on either side, whole
+// steps of 90 drawn layers, bf16 and fp32 results, tiled kernel -> small one, us: the 69 taken are 1.07 times as fast in the mean, most of all by
+// skewed shares (5953 tokens, 4 of 128, 336 <-> 536, 565 -> 312; 56149 rows of 8, 2688 <-> 704, 4230 -> 2345), 15 of them slower, seven by
+// more than 3 % (1392 rows of 128, 384 <-> 192, 67 -> 75; 9269 tokens, 6 of 24, 2912 <-> 432, 2107 -> 2268); the 21 past the line come
+// to 1.005, from 0.91 to 1.09, but for one by Zipf's shares (15833 tokens, 2 of 128, 960 <-> 256, 679 -> 434).)
 constexpr int64_t WTILE = 256;
 constexpr int64_t MULTI_ROUNDS = 4;
 bool wgrad_multi(int64_t E, int64_t M, int64_t N, int64_t R) {

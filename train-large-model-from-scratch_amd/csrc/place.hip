@@ -354,9 +354,11 @@ int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* t
   return moe_place_bytes(T, E) > 16 * 1024 ? of(std::integral_constant<int, 16>{}) : of(std::integral_constant<int, 8>{});
 }
 
-// A launch fewer, as long as the selection of all tokens costs a workgroup less than that: 128 / 512 / 1024 tokens, us, two launches
-// and here: 2 of 8 experts 7.3, 5.2 / 7.8, 5.4 / 8.6, 7.5 (2048: 9.6, 11.4); 1 of 4 7.1, 5.2 / 7.3, 5.2 / 7.5, 6.5.  (2 of 16 7.0, 6.4 /
-// 7.7, 7.0 / 8.6, 10.3, 8 of 16 from the first on slower: not taken.)
+// A launch fewer, as long as the selection of all tokens costs a workgroup less than that: 128 / 512 / 1024 tokens, bf16, 1024 wide, us, two
+// launches' own times and here: 2 of 8 experts 7.3, 4.7 / 7.5, 5.2 / 8.6, 7.2 (2048: 9.6, 11.4); 1 of 4 7.1, 4.0 / 7.3, 4.2 / 7.4, 5.1; 512
+// tokens, 4 of 8 9.0, 6.8, 4 of 4 9.0, 6.1; 256, 8 of 8 9.9, 8.0.  (2 of 16 7.0, 6.4 / 7.7, 7.0 / 8.6, 10.3, 8 of 16 from the first on slower: not
+// taken.  A lane holds a token's logits in registers, their number is the kernel's own: 4 and 8 are what the kernel is made for; counts
+// that are not multiples of 4 have bf16 rows that do not come in whole words of 8 bytes, and 12 lies next to 16.)
 bool moe_select_place_ok(const void* logits, int64_t T, int64_t E, int64_t k) {
   return moe_place_ok(T, E, k) && (E == 4 || E == 8) && T <= 1024 && T * k <= 2048 && (reinterpret_cast<uintptr_t>(logits) & 7) == 0;
 }
