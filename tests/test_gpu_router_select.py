@@ -1,0 +1,75 @@
+"""The router product and the selection in one launch: logits of the bits that the library's product has, the selection that
+`moe_ffn` makes on them, and the same rest of the layer; at the edges of the sizes that it takes."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+@pytest.mark.parametrize("T,E,k,H,taken", [
+    (65, 2, 1, 64, True), (65, 64, 8, 2048, True), (66, 128, 8, 1024, True), (70, 33, 3, 72, True),  # the fewest tokens; ends of slices
+    (256, 8, 2, 1016, True), (257, 8, 2, 1016, True), (257, 12, 3, 128, True), (300, 16, 16, 320, True),  # one chain and four, to 16 experts
+    (2048, 12, 4, 256, True), (3200, 16, 2, 512, True), (3333, 12, 3, 1416, True), (12288, 8, 2, 1024, True), (8192, 3, 3, 2048, True),
+    (4081, 32, 4, 1032, True), (4096, 32, 32, 1032, True), (2048, 64, 6, 1600, True), (4096, 64, 8, 2048, True),
+    (1360, 96, 6, 1360, True), (1361, 96, 6, 1360, True), (1031, 77, 5, 1208, True), (1009, 128, 8, 1000, True), (4091, 100, 7, 1000, True),
+    (64, 8, 2, 1024, False), (4097, 64, 8, 1024, False), (8193, 8, 2, 2048, False), (1531, 24, 4, 1024, False), (700, 128, 8, 1032, False),
+])
+@pytest.mark.parametrize("x_type,w_type", [(BF16, BF16), (F32, F32)])
+def test_bits_of_the_two_calls(pkg, lib, T, E, k, H, taken, x_type, w_type):
+    print("router select", T, E, k, H, x_type, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + E + H)
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g, device="cuda") * std
+    I = 8
+    x, wr = r(T, H).to(x_type), r(E, H, std=0.05).to(w_type)
+    w1, w3, w2 = (r(*s, std=0.05).to(BF16) for s in ((E, I, H), (E, I, H), (E, H, I)))
+    bias = r(E) if k % 2 else None
+    want = F.linear(x.to(BF16), wr.to(BF16))
+    names = []
+
+    class Obs:
+        before = staticmethod(names.append)
+        after = staticmethod(lambda name: None)
+
+    lib.observer = Obs()
+    try:
+        out, lg = pkg.routed_moe(x, wr, w1, w3, w2, k, bias=bias)   # nothing to differentiate: one call for the pass
+    finally:
+        lib.observer = None
+    assert ("moe_router_select" in names) == taken, names
+    if T <= 64:
+        return  # (the kernels for few tokens sum up in an order of their own)
+    assert torch.equal(lg, want)
+    ref, routing = pkg.moe_ffn(x, want, w1, w3, w2, k, bias=bias, return_routing=True)
+    assert torch.equal(out, ref)
+    ws = [t.clone().requires_grad_(True) for t in (wr, w1, w3, w2)]
+    out, lg, kept = pkg.routed_moe(x, *ws, k, bias=bias, return_routing=True)
+    assert torch.equal(lg, want) and torch.equal(out, ref)
+    for name in ("ids", "gates", "counts", "offs", "pos_to_row", "row_to_pos"):
+        assert torch.equal(kept[name], routing[name]), name
+    # what the backward pass reads: the router's weight and x in bf16
+    dy = r(T, H).to(x_type)
+    out.backward(dy)
+    xr, wd = x.to(BF16).float(), ws[0].grad.float()
+    lr = want.clone().requires_grad_(True)
+    pkg.moe_ffn(x, lr, w1, w3, w2, k, bias=bias).backward(dy)
+    ref_w = lr.grad.float().T @ xr
+    # (roundings of dlogits and of the result to bf16, sums of T products in fp32)
+    assert (wd - ref_w).norm() <= 2.0 ** -7 * ref_w.norm() + 1e-6
+
+
+def test_values_that_are_not_finite(pkg):
+    print("router select, not finite", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    r = lambda *s: (torch.randn(*s, generator=g, device="cuda") * 0.1).to(BF16)
+    for T, E, k, H in ((130, 8, 2, 256), (130, 64, 8, 1536), (130, 128, 8, 512)):
+        x, wr = r(T, H), r(E, H)
+        x[3, 5], x[64, 7], wr[1, 2] = float("nan"), float("inf"), float("-inf")
+        w1, w3, w2 = r(E, 8, H), r(E, 8, H), r(E, H, 8)
+        _, lg = pkg.routed_moe(x, wr, w1, w3, w2, k)
+        want = F.linear(x, wr)
+        assert torch.equal(lg.isnan(), want.isnan())
+        ok = ~want.isnan()
+        assert torch.equal(lg[ok], want[ok])

@@ -12,7 +12,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libmoe_gfx950.so")
 NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
-SOURCES = ("route.hip", "dispatch.hip", "place.hip", "norm.hip", "gemm.hip", "row_ring.hip", "f32.hip", "f32_gemm.hip", "few.hip", "wgrad.hip", "layer.hip")
+SOURCES = ("route.hip", "dispatch.hip", "place.hip", "norm.hip", "gemm.hip", "row_ring.hip", "f32.hip", "f32_gemm.hip", "few.hip", "router.hip", "wgrad.hip", "layer.hip")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "moe_gfx950.h"
+#include "router.h"
 
 // (from internal.h and layer.hip, which only device code can include)
 void moe_observe(const char* name, int after);
@@ -38,7 +39,6 @@ int moe_select_place(const void* x, int x_dtype, const void* logits, int logits_
 int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, float eps, const uint16_t* router_weight,
                              int64_t T, int64_t H, int64_t E, int64_t k, uint16_t* xn, float* rstd, uint16_t* logits,
                              int32_t* ids, float* gates, void* table, void* stream);
-int moe_selected_layer_forward(const moe_layer_forward_args* a, const void* table, void* stream);
 int64_t moe_forward_scratch(const moe_layer_forward_args* a);
 int64_t moe_backward_scratch(const moe_layer_backward_args* a);
 int moe_f32_gateup(const float* xp, const float* w1, const float* w3, const int32_t* offs, int64_t E, int64_t R, int64_t H,
@@ -51,9 +51,6 @@ int moe_f32_router_wgrad(const float* xp, const float* dsel, const int32_t* offs
                          float* dwr, void* stream);
 int moe_f32_wgrads(const float* dg, const float* du, const float* dyp, const float* xp, const float* act, const int32_t* offs,
                    int64_t E, int64_t R, int64_t H, int64_t I, float* dw1, float* dw3, float* dw2, void* stream);
-int moe_routed_forward(const uint16_t* x, const uint16_t* wr, uint16_t* logits, const float* bias, const uint16_t* w1,
-                       const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k,
-                       void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
 using at::Tensor;
 using torch::autograd::AutogradContext;
@@ -260,13 +257,26 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   Tensor logits;
   Tensor table;  // of the selection's counts, where it is done and they are wanted
   bool selected = false, inside = false;  // selection done; the forward-only call makes the logits itself
+  MoeRouter router{};                     // its product is part of the layer's call where `own` says so
+  bool own = false;
   const Tensor b = bias.defined() ? dense(bias) : Tensor();
   if (o.train || o.routing_out || !(wr.defined() || logits_.defined()) || norm_w.defined() || T == 0)
     f.routing = empty({r.at[Routing::PARTS]}, at::kInt, x);
   if (wr.defined()) {
     const Tensor wrd = dense(wr.detach());
-    const bool both = !norm_w.defined() && x_type == at::kFloat && wrd.scalar_type() == at::kFloat && H % 8 == 0 && T > 0;
-    if (both) {  // (a launch each took 4.7 us for the router's weight and 7.7 for 4096 tokens, 1024 wide; together 8.8)
+    own = !norm_w.defined() && moe_router_select_ok(T, H, E, k) && (wrd.scalar_type() == at::kFloat || wrd.scalar_type() == at::kBFloat16);
+    const bool both = !own && !norm_w.defined() && x_type == at::kFloat && wrd.scalar_type() == at::kFloat && H % 8 == 0 && T > 0;
+    if (own) {  // (what is to be rounded to bf16 is rounded on the way)
+      const bool x_as_is = x_type == at::kBFloat16, wr_as_is = wrd.scalar_type() == at::kBFloat16;
+      f.xn = x_as_is ? x : empty(x.sizes(), at::kBFloat16, x);
+      f.wrb = wr_as_is || !o.train ? wrd : empty(wrd.sizes(), at::kBFloat16, x);
+      logits = empty({T, E}, at::kBFloat16, x);
+      router.x = x.data_ptr(), router.x_dtype = (int)dt(x), router.wr = wrd.data_ptr(), router.wr_dtype = (int)dt(wrd);
+      router.xn = x_as_is ? nullptr : (uint16_t*)f.xn.data_ptr();
+      router.wrb = wr_as_is || !o.train ? nullptr : (uint16_t*)f.wrb.data_ptr();
+      router.bias = (const float*)ptr(b), router.logits = (uint16_t*)logits.data_ptr();
+      inside = !f.routing.defined(), selected = true;
+    } else if (both) {  // (a launch each took 4.7 us for the router's weight and 7.7 for 4096 tokens, 1024 wide; together 8.8)
       f.wrb = empty(wrd.sizes(), at::kBFloat16, x);
       f.xn = empty(x.sizes(), at::kBFloat16, x);
       CALL(moe_cast_two, x.data_ptr<float>(), (uint16_t*)f.xn.data_ptr(), x.numel(), wrd.data_ptr<float>(),
@@ -296,15 +306,19 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
         CALL(moe_rmsnorm_fwd, x.data_ptr(), (int)dt(x), f.nw.data_ptr<float>(), (float)o.eps, T, H,
              (uint16_t*)f.xn.data_ptr(), f.rstd.data_ptr<float>(), s);
       }
-    } else if (!both) {
+    } else if (!both && !own) {
       f.xn = cast_bf16(x);
     }
     rows = f.xn;
     if (!selected && moe_router_few_ok(T, H, E, k)) {
       logits = empty({T, E}, at::kBFloat16, x);
       inside = !f.routing.defined();
-      if (!inside)
+      if (inside) {
+        router.x = f.xn.data_ptr(), router.wr = f.wrb.data_ptr(), router.x_dtype = router.wr_dtype = MOE_DT_BF16;
+        router.bias = (const float*)ptr(b), router.logits = (uint16_t*)logits.data_ptr();
+      } else {
         check(moe_router_logits(bf(f.xn), bf(f.wrb), T, H, E, (uint16_t*)logits.data_ptr(), s), "moe_router_few");
+      }
     } else if (!selected) {
       const NoAutocast off;
       logits = at::mm(f.xn, f.wrb.t());
@@ -319,9 +333,8 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
     const Tensor ws = empty({std::max<int64_t>(bytes, 256)}, at::kByte, x);
     // (it tells the observer about its launches itself, as do the two calls of a training step)
     if (inside)
-      check(moe_routed_forward(bf(rows), bf(f.wrb), (uint16_t*)logits.data_ptr(), (const float*)ptr(b), bf(f.w.w1),
-                               bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(), (int)dt(x_type), ws.data_ptr(),
-                               ws.numel(), s),
+      check(moe_routed_forward(router, bf(rows), bf(f.w.w1), bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(),
+                               (int)dt(x_type), ws.data_ptr(), ws.numel(), s),
             "moe_routed_forward");
     else check(moe_ffn_forward(rows.data_ptr(), (int)dt(rows), logits.data_ptr(), (int)dt(logits), (const float*)ptr(b),
                           bf(f.w.w1), bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(), (int)dt(x_type),
@@ -360,7 +373,7 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   const int64_t bytes = std::max<int64_t>(moe_forward_scratch(&a), 256);
   const Tensor scratch = empty({bytes}, at::kByte, x);
   a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
-  check(moe_selected_layer_forward(&a, ptr(table), s), "moe_layer_forward");
+  check(moe_selected_layer_forward(&a, own ? &router : nullptr, ptr(table), s), "moe_layer_forward");
   if (o.routing_out) *o.routing_out = f.routing;
   return f;
 }

@@ -2,6 +2,7 @@
 // checked by the entry points that reach them.
 #pragma once
 #include "common.h"
+#include "router.h"
 
 // Tells the installed launch observer, if any, about one launch (layer.hip).
 void moe_observe(const char* name, int after);
@@ -87,6 +88,10 @@ int moe_select_place(const void* x, int x_dtype, const void* logits, int logits_
 bool moe_count_ok(int64_t T, int64_t E, int64_t k);
 int64_t moe_count_bytes(int64_t T, int64_t E);
 int moe_count_ids(const int64_t* ids64, int32_t* ids, int64_t T, int64_t E, void* table, void* stream);
+
+// The router's product, the selection and its table of counts (NULL: not wanted) in one launch (router.hip).
+int moe_router_select(const MoeRouter& r, int64_t T, int64_t H, int64_t E, int64_t k, int32_t* ids, float* gates, void* table,
+                      hipStream_t s);
 
 // moe_rmsnorm_router_fwd that leaves the table too, unless it is NULL (norm.hip).
 int moe_rmsnorm_router_count(const void* x, int x_dtype, const float* weight, float eps, const uint16_t* router_weight,

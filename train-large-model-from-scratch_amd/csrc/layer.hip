@@ -79,11 +79,9 @@ extern "C" int64_t moe_ffn_forward_workspace_bytes(int64_t T, int64_t H, int64_t
   return carve(T, H, E, I, k).total;
 }
 
-// The pass itself.  With `wr` the router product is part of it (logits are written to logits_out; shapes
-// that moe_router_few_ok takes), without it the logits are given.
-static int forward_only(const void* x, int x_dtype, const void* logits, int logits_dtype, const uint16_t* wr,
-                        uint16_t* logits_out, const float* bias, const uint16_t* w1, const uint16_t* w3,
-                        const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
+// The pass itself.  With `router` its product is part of it (see router.h), without it the logits are given.
+static int forward_only(const void* x, int x_dtype, const void* logits, int logits_dtype, const MoeRouter* router,
+                        const float* bias, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
                         int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
   if (!sizes_ok(T, H, E, I, k)) return MOE_ERR_LIMIT;
@@ -92,11 +90,12 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   if (out_dtype != MOE_DT_BF16 && out_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
   if (T == 0) return 0;
   MOE_CHECK_PTR(x);
-  if (wr) {
-    MOE_CHECK_PTR(wr);
-    MOE_CHECK_PTR(logits_out);
-    if (x_dtype != MOE_DT_BF16) return MOE_ERR_DTYPE;
-    if (!moe_router_few_ok(T, H, E, k)) return MOE_ERR_LIMIT;
+  const bool few_logits = router && moe_router_few_ok(T, H, E, k);
+  if (router) {
+    MOE_CHECK_PTR(router->wr);
+    MOE_CHECK_PTR(router->logits);
+    if (few_logits ? x_dtype != MOE_DT_BF16 || router->wr_dtype != MOE_DT_BF16 : !moe_router_select_ok(T, H, E, k))
+      return few_logits ? MOE_ERR_DTYPE : MOE_ERR_LIMIT;
   } else {
     MOE_CHECK_PTR(logits);
   }
@@ -119,10 +118,11 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   uint16_t* act = (uint16_t*)(ws + c.act);
   uint16_t* y = (uint16_t*)(ws + c.y);
   hipStream_t st = (hipStream_t)stream;
-  if (wr) {
-    MOE_STEP("moe_router_few", moe_router_few((const uint16_t*)x, wr, T, H, E, logits_out, st));
-    logits = logits_out;
+  if (few_logits) MOE_STEP("moe_router_few", moe_router_few((const uint16_t*)x, (const uint16_t*)router->wr, T, H, E, router->logits, st));
+  if (router) {
+    logits = router->logits;
     logits_dtype = MOE_DT_BF16;
+    bias = router->bias;
   }
   if (moe_gateup_one_ok(T, E, k)) {
     MOE_STEP("moe_gateup_one", moe_gateup_one(x, x_dtype, logits, logits_dtype, bias, w1, w3, H, E, I, k, ids, gates, act, st));
@@ -131,8 +131,10 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   }
   const bool few = moe_few_ok(T, H, E, I, k, x_dtype), place = !few && moe_place_ok(T, E, k);
   const bool selects = few && moe_gateup_few_selects(T, E, I, k);  // gate/up does the selection
-  const bool at_once = place && moe_select_place_ok(logits, T, E, k);
-  if (at_once)
+  const bool selected = router && !few_logits, at_once = place && !selected && moe_select_place_ok(logits, T, E, k);
+  if (selected)
+    MOE_STEP("moe_router_select", moe_router_select(*router, T, H, E, k, ids, gates, place ? ws + c.dispatch : nullptr, st));
+  else if (at_once)
     MOE_STEP("moe_select_place", moe_select_place(x, x_dtype, logits, logits_dtype, bias, T, H, E, k, ids, gates, counts, offs,
                                                   pos_to_row, row_to_pos, nullptr, xp, MOE_DT_BF16, stream));
   else if (place)
@@ -175,15 +177,14 @@ extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, i
                                const float* bias, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
                                int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
                                int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
-  return forward_only(x, x_dtype, logits, logits_dtype, nullptr, nullptr, bias, w1, w3, w2, T, H, E, I, k, out,
+  return forward_only(x, x_dtype, logits, logits_dtype, nullptr, bias, w1, w3, w2, T, H, E, I, k, out,
                       out_dtype, workspace, workspace_bytes, stream);
 }
 
-int moe_routed_forward(const uint16_t* x, const uint16_t* wr, uint16_t* logits, const float* bias, const uint16_t* w1,
-                       const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k,
-                       void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
-  if (!wr) return MOE_ERR_NULL;
-  return forward_only(x, MOE_DT_BF16, nullptr, MOE_DT_BF16, wr, logits, bias, w1, w3, w2, T, H, E, I, k, out, out_dtype,
+int moe_routed_forward(const MoeRouter& router, const uint16_t* x, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
+                       int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out, int out_dtype, void* workspace,
+                       int64_t workspace_bytes, void* stream) {
+  return forward_only(x, MOE_DT_BF16, nullptr, MOE_DT_BF16, &router, nullptr, w1, w3, w2, T, H, E, I, k, out, out_dtype,
                       workspace, workspace_bytes, stream);
 }
 
@@ -342,8 +343,8 @@ int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
   return s.at;
 }
 
-// With `table` the selection is done, ids and gates are there, and so are its counts (moe_rmsnorm_router_count).
-static int layer_forward(const moe_layer_forward_args* a, const void* table, void* stream) {
+// (`router` and `table`: see router.h)
+static int layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream) {
   if (!a) return MOE_ERR_NULL;
   const int64_t T = a->T, H = a->H, E = a->E, I = a->I, k = a->k, R = T * k;
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
@@ -369,6 +370,12 @@ static int layer_forward(const moe_layer_forward_args* a, const void* table, voi
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
   const FwdScratch ws(s, T, H, E, k, !out_in_place(*a));
   if (!s.fits()) return MOE_ERR_WORKSPACE;
+  if (router && T > 0) {
+    if (!a->gates) return MOE_ERR_NULL;
+    if (moe_place_ok(T, E, k)) table = ws.dispatch;
+    MOE_STEP("moe_router_select", moe_router_select(*router, T, H, E, k, a->ids, a->gates, moe_place_ok(T, E, k) ? ws.dispatch : nullptr,
+                                                    (hipStream_t)stream));
+  }
   if (a->logits && !table && moe_select_place_ok(a->logits, T, E, k)) {
     MOE_STEP("moe_select_place", moe_select_place(a->x, (int)a->x_dtype, a->logits, (int)a->logits_dtype, a->bias, T, H, E, k, a->ids,
                                                   a->gates, a->counts, a->offs, a->pos_to_row, a->row_to_pos, a->bad_ids, a->xp,
@@ -419,10 +426,10 @@ static int layer_forward(const moe_layer_forward_args* a, const void* table, voi
   return 0;
 }
 
-extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) { return layer_forward(a, nullptr, stream); }
+extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) { return layer_forward(a, nullptr, nullptr, stream); }
 
-int moe_selected_layer_forward(const moe_layer_forward_args* a, const void* table, void* stream) {
-  return layer_forward(a, table, stream);
+int moe_selected_layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream) {
+  return layer_forward(a, router, table, stream);
 }
 
 extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream) {

@@ -1,0 +1,23 @@
+// What the router's product is made of, and the layer calls that it is part of (declared for host code too, which internal.h is not).
+#pragma once
+#include <stdint.h>
+
+#include "moe_gfx950.h"
+
+struct MoeRouter {
+  const void *x, *wr;  // [T,H] and [E,H], each bf16 or fp32
+  int x_dtype, wr_dtype;
+  const float* bias;   // [E] or NULL: added to the logits for the selection
+  uint16_t *xn, *wrb;  // where bf16 copies of an fp32 x and wr are left (NULL: they are not wanted)
+  uint16_t* logits;    // [T,E]
+};
+
+// Sizes for which product and selection are one launch (router.hip).
+bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k);
+// moe_ffn_forward, and moe_layer_forward (x: the bf16 rows), with the router's product part of it: sizes that moe_router_few_ok (x and
+// wr in bf16) or moe_router_select_ok takes, the latter alone in training.  moe_selected_layer_forward: with a `table` instead the
+// selection is done, ids and gates are there, and so are its counts; with neither it is moe_layer_forward.
+int moe_routed_forward(const MoeRouter& router, const uint16_t* x, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
+                       int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out, int out_dtype, void* workspace,
+                       int64_t workspace_bytes, void* stream);
+int moe_selected_layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream);

@@ -38,6 +38,19 @@ __device__ __forceinline__ float moe_wave_sum_f32(float v) {
   return v;
 }
 
+// The same where only the first 16 lanes have something other than zero, for them: the same pairs in the same order, on the vector
+// ALU's own data path.
+__device__ __forceinline__ float moe_row_sum_f32(float v) {
+#define MOE_SUM_STEP(n) \
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + n, 0xf, 0xf, false));
+  MOE_SUM_STEP(8)  // row_ror
+  MOE_SUM_STEP(4)
+  MOE_SUM_STEP(2)
+  MOE_SUM_STEP(1)
+#undef MOE_SUM_STEP
+  return v;
+}
+
 // The keys of one token's E logits, plus the experts' biases unless NULL: the larger the logit, the larger the key; 0
 // (which no logit maps to) marks what is taken or absent.
 template <int VPL, typename LT>
@@ -89,6 +102,6 @@ __device__ __forceinline__ void moe_topk_softmax_wave(uint32_t (&key)[VPL], int 
     }
   }
   const float p = lane < k ? expf(my_val - vmax) : 0.f;
-  const float s = moe_wave_sum_f32(p);
+  const float s = k <= 16 ? moe_row_sum_f32(p) : moe_wave_sum_f32(p);
   my_gate = p / s;
 }
