@@ -42,7 +42,7 @@ struct GemmArgs {
   int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
   int whole_only;  // row-ragged modes: no half tiles (test hook)
   const int32_t* row_map;  // row-ragged modes, DOWN and DGRAD_GATEUP: where a row of the result goes (NULL: rows stay in order)
-  int streaming;   // WGRAD: results that replace what is there leave with streaming stores
+  int streaming;   // WGRAD: results that replace what is there leave with streaming stores; GATEUP: act does
 };
 
 // sigmoid from the two hardware transcendentals (v_exp_f32, v_rcp_f32; about 1 ulp each):
