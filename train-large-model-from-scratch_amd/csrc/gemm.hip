@@ -82,11 +82,12 @@ __device__ __forceinline__ int expert_of(const int* tile_start, int slot, int E)
 // The kernel's tile walk: the tiles at positions t_next, t_next + t_step, .. below t_hi of the launch's tile
 // list, or of `list` where one is given.  The rows of a row-ragged launch are numbered in tiles of UNIT rows; where
 // the configuration's are half as high, a list entry is 2 * tile + half.  (tile_start and, there, offs: in LDS.)
-// TO (DOWN and DGRAD_GATEUP only): the rows leave to where p.row_map says.
-template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE, bool TO = false>
+// TO (DOWN and DGRAD_GATEUP only): the rows leave to where p.row_map says.  FROM (GATEUP only): A's rows come from where p.row_from says.
+template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE, bool TO = false, bool FROM = false>
 __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, const int* tile_start, const int* offs,
                                            const uint32_t* list, int t_next, const int t_hi, const int t_step) {
   static_assert(!BLK || MODE == GATEUP || MODE == DGRAD_DOWN, "only g and u have the blocked layout");
+  static_assert(!FROM || MODE == GATEUP, "only x is read where the caller has it");
   static_assert(!TO || MODE == DOWN || MODE == DGRAD_GATEUP, "only y and dxp are rows that somebody else has a place for");
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, KS = Cfg::KS;
   constexpr int FM = Cfg::FM, FN = Cfg::FN, WTM = Cfg::WTM, WTN = Cfg::WTN;
@@ -170,7 +171,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       if (p.K % 2048 == 0) t.kt0 = (t.e * 13) & 31;  // (32 k-tiles to 4 KB)
     }
     if constexpr (MODE == GATEUP) {
-      t.vA0 = make_view(p.A0 + (long long)t.row0 * lda, rows * lda);
+      t.vA0 = FROM ? View{p.A0, p.from_bytes} : make_view(p.A0 + (long long)t.row0 * lda, rows * lda);
       const long long wofs = ((long long)t.e * p.N + t.n0) * p.K;
       const long long wvalid = (long long)(p.N - t.n0) * p.K;
       t.vB0 = make_view(p.B0 + wofs, wvalid);
@@ -204,6 +205,18 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   } else {
     opB.init(ldb);
   }
+  // (FROM) A lane has the place of one of the rows that its wave requests: asked for a tile ahead, worked out and dealt to the lanes
+  // that request the row where the first k-tile of its tile is asked for.
+  int row_from = 0;
+  auto ask_rows = [&](const Tile& t) {
+    if constexpr (FROM) {
+      const int r = t.row0 + StA::own_row(wv, lane);
+      row_from = r < t.row_end ? p.row_from[r] : -1;
+    }
+  };
+  auto set_rows = [&]() {
+    if constexpr (FROM) opA.set_rows(row_from < 0 ? NO_ROW : (uint32_t)p.by_k(row_from) * (uint32_t)(lda * 2));
+  };
   // One set of registers carries a k-tile from HBM to LDS: it is requested one iteration
   // before it is written to LDS, which is what hides the latency of a load that misses L2.
   constexpr int CHA = StA::CH, CHB = DUAL ? StBh::CH : StB::CH;
@@ -697,6 +710,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   auto request_first = [&](const Tile& t) { request_k(t, 0); };
   Tile cur;
   if (t_next >= t_hi || !locate(tile_at(t_next), cur)) return;
+  ask_rows(cur);
+  set_rows();
   request_first(cur);
   bool staged = false;
   int s0 = 0;           // the LDS stage of the tile's first k-tile; they alternate from there
@@ -725,6 +740,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     Tile nxt;
     t_next += t_step;
     const bool more = t_next < t_hi && locate(tile_at(t_next), nxt);
+    if (more) ask_rows(nxt);
     if constexpr (TO) {
 #pragma unroll
       for (int h = 0; h < (WTM + MOE_WAVE - 1) / MOE_WAVE; ++h) {
@@ -737,7 +753,10 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     // the k-tile two behind kt
     auto request_ahead = [&](int kt) {
       if (kt + 2 < nkt) load_tile(cur, kt + 2, stg);
-      else if (stream && kt + 2 - nkt < (EARLY_REQUEST ? nxt.nkt : 1)) load_tile(nxt, kt + 2 - nkt, stg);
+      else if (stream && kt + 2 - nkt < (EARLY_REQUEST ? nxt.nkt : 1)) {
+        if (kt + 2 == nkt) set_rows();
+        load_tile(nxt, kt + 2 - nkt, stg);
+      }
     };
     if (nkt > 0) {
       if (!staged) {
@@ -828,7 +847,10 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       }
     }
     if (!stream) {
-      if (EARLY_REQUEST && more) request_first(nxt);
+      if (EARLY_REQUEST && more) {
+        set_rows();
+        request_first(nxt);
+      }
       lds_barrier();  // every wave is done reading the operand stages
     }
     if (STREAM && nkt > 0) strip = strip_in((s0 + nkt - 1) & 1);
@@ -920,7 +942,7 @@ __device__ __forceinline__ Sweep sweep_of(int n) {
 // fast, 0.94 to 1.25.  (The same quarters with the staging registers of the other tiles: two thirds of that.)  Dgrad-down is
 // 0.79 times as fast in quarters where they are all there is, and 0.94 after whole rounds (577 rows of 24 experts, 4096 <->
 // 1536, 60 -> 96 us; 8641 rows of 48 193 -> 225), never more than 1.05.
-template <int MODE, typename OutT, bool BLK, bool TO>
+template <int MODE, typename OutT, bool BLK, bool TO, bool FROM>
 __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gemm_kernel(const GemmArgs p) {
   static_assert(CfgHalf::NT == CfgMain::NT, "one workgroup runs both");
   constexpr int WAVES = CfgMain::NT / MOE_WAVE;
@@ -999,7 +1021,7 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
       for (int h = 0; h < n; ++h) half_list[at + h - skip] = 2u * (uint32_t)tile + h;
   }
   const Sweep s = sweep_of(whole);
-  walk_tiles<MODE, CfgMain, OutT, BLK, ROW_TILE, TO>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
+  walk_tiles<MODE, CfgMain, OutT, BLK, ROW_TILE, TO, FROM>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
   if (halves == 0) return;
   __syncthreads();  // (the operand stages are free, the list is complete)
   const Sweep h = sweep_of(halves);
@@ -1012,24 +1034,24 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void rows_gem
         const int e = expert_of(tile_start, slot, p.E);
         const int first = __builtin_amdgcn_readfirstlane(offs[e]), end = __builtin_amdgcn_readfirstlane(offs[e + 1]);
         const int row = (slot - __builtin_amdgcn_readfirstlane(tile_start[e])) * ROW_TILE + (entry & 3) * Quarter::BM;
-        ring_tile<MODE, BLK, 1, WAVES, TO>(p, (char*)smem, e, first, end, row, (tile - slot * p.n_tiles) * Quarter::BNC);
+        ring_tile<MODE, BLK, 1, WAVES, TO, FROM>(p, (char*)smem, e, first, end, row, (tile - slot * p.n_tiles) * Quarter::BNC);
         __syncthreads();
       }
       return;
     }
   }
-  walk_tiles<MODE, CfgHalf, OutT, BLK, ROW_TILE, TO>(p, smem, tile_start, offs, half_list, h.first, h.end, h.step);
+  walk_tiles<MODE, CfgHalf, OutT, BLK, ROW_TILE, TO, FROM>(p, smem, tile_start, offs, half_list, h.first, h.end, h.step);
 }
 
 // All in half tiles: launches of so few tiles that there is nothing to decide and that csrc/row_ring.hip does not take (4096 rows
 // of 8 experts, 1024 <-> 512, gate/up 19.5 us; in ring tiles of 64 rows, a few more than fit at once, 23.3).
-template <int MODE, typename OutT, bool BLK, bool TO>
+template <int MODE, typename OutT, bool BLK, bool TO, bool FROM>
 __global__ __launch_bounds__(CfgHalf::NT, CfgHalf::WAVES_PER_SIMD) void small_rows_gemm_kernel(const GemmArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   __shared__ int tile_start[GEMM_MAX_E + 1], offs[GEMM_MAX_E + 1];
   number_tiles<CfgHalf::BM>(p, tile_start, offs);
   const Sweep s = sweep_of(__builtin_amdgcn_readfirstlane(tile_start[p.E]) * p.n_tiles);
-  walk_tiles<MODE, CfgHalf, OutT, BLK, CfgHalf::BM, TO>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
+  walk_tiles<MODE, CfgHalf, OutT, BLK, CfgHalf::BM, TO, FROM>(p, smem, tile_start, offs, nullptr, s.first, s.end, s.step);
 }
 
 // Weight gradients: of up to three problems that share their experts' rows, one's tiles behind the other's without a launch
@@ -1197,7 +1219,7 @@ constexpr int RING_TILE = 64, RING_TALL = 1;  // (1: the ring's tiles of 128 row
 int forced_row_tile = 0;
 
 // A row-ragged launch with `cols` output columns to a tile.
-template <int MODE, bool BLK = false, bool TO = false>
+template <int MODE, bool BLK = false, bool TO = false, bool FROM = false>
 int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   static_assert(lds_bytes<MODE, CfgHalf>() <= lds_bytes<MODE, CfgMain>(), "both row tiles fit");
   static bool attr_done[2][MOE_MAX_DEVICES];  // per GPU and instantiation
@@ -1212,7 +1234,7 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
                                                  : 2 * tiles < moe_compute_units() &&
                                                        moe_expected_tiles(a.R, a.E, CfgHalf::BM) * a.n_tiles <= moe_compute_units();
   if (small)
-    return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK, TO>, attr_done[0], a,
+    return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK, TO, FROM>, attr_done[0], a,
                                  a.n_tiles * row_slots(a.R, a.E, CfgHalf::BM), s);
   a.whole_only = forced_row_tile == ROW_TILE;
   // With few rows an expert gate/up is bound by its weights, whose way through L2 a streamed act leaves free.  Ordinary -> streaming, forward
@@ -1220,7 +1242,7 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
   // 395.4; 12 of 4096 <-> 2048, 150 rows 181.0 -> 177.1; 96 of 1536 <-> 640, 94 rows 172.1 -> 170.5; 48 of 3072 <-> 896, 208 rows, not taken,
   // 276.4 -> 280.1; 8 of 2048 <-> 1024, 1500 rows 195.6 -> 198.0.  (y and the gradients so too: 0.97 to 1.00 times as fast.)
   a.streaming = MODE == GATEUP && a.R <= 200ll * a.E;
-  return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK, TO>, attr_done[1], a,
+  return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK, TO, FROM>, attr_done[1], a,
                                2 * a.n_tiles * row_slots(a.R, a.E, ROW_TILE), s);
 }
 // With few rows an expert the results come as fast as the operands do, and as streaming stores they leave the operands' lines in L2
@@ -1260,6 +1282,28 @@ int check_common(const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I
 }
 
 }  // namespace
+
+// A's rows where the tokens are.  The copies in expert order are a pass that writes k rows a token and a gate/up that reads them from memory,
+// where the tokens' own rows stay in the caches; a lane's offset a row instead of a constant one costs the loop nothing (the offsets are in registers
+// either way, 253 of them with the next tile's row).  Forward passes, us, copies -> this, the same bits: 64 experts, 2048 <-> 1024, 8 a token, 257 / 700
+// / 1531 / 4000 / 16384 tokens 166 -> 163, 187 -> 180, 245 -> 230, 496 -> 469, 1742 -> 1639; 8192 of 128, 1024 <-> 256, 232 -> 204; 2048 of 8, 1024 <->
+// 512, 42.6 -> 40.3; 3333 of 12, 1416 <-> 568, 99 -> 92; 16000, 1 of 4, 512 <-> 256, 60.6 -> 57.1; no size of 16 slower.  A lane's
+// offset and a window's size have 32 bits, and one of them marks rows that there are none of: hence the limit.
+bool moe_gateup_from_ok(int64_t T, int64_t H) { return T * H < (int64_t)1 << 30; }
+
+int moe_gemm_gateup_from(const uint16_t* x, const int32_t* pos_to_row, int64_t T, int64_t k, const uint16_t* w1, const uint16_t* w3,
+                         const int32_t* offs, int64_t E, int64_t H, int64_t I, uint16_t* act, void* stream) {
+  const int64_t R = T * k;
+  if (int rc = check_common(offs, E, R, H, I)) return rc;
+  if (R == 0) return 0;
+  if (!moe_gateup_from_ok(T, H)) return MOE_ERR_LIMIT;
+  MOE_CHECK_PTR(x); MOE_CHECK_PTR(w1); MOE_CHECK_PTR(w3); MOE_CHECK_PTR(act); MOE_CHECK_PTR(pos_to_row);
+  GemmArgs a{};
+  a.A0 = x; a.B0 = w1; a.B1 = w3; a.C2 = act; a.offs = offs;
+  a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H;
+  a.row_from = pos_to_row; a.by_k.set((uint32_t)k); a.from_bytes = T * H * 2;
+  return launch_rows<GATEUP, false, false, true>(a, CfgMain::BN / 2, (hipStream_t)stream);
+}
 
 extern "C" int moe_gemm_gateup_swiglu_fwd(const uint16_t* xp, const uint16_t* w1, const uint16_t* w3,
                                           const int32_t* offs, int64_t E, int64_t R, int64_t H,

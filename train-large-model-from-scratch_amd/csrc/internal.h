@@ -72,7 +72,7 @@ constexpr int MOE_PLACE_CHUNK = 16;
 bool moe_place_ok(int64_t T, int64_t E, int64_t k);
 int64_t moe_place_bytes(int64_t T, int64_t E);
 // moe_router_topk_fwd that leaves the table, and from it the results of moe_histogram_scan and moe_permute_fwd (fp32 rows
-// where x is fp32 and xp_dtype says so); *bad_ids, unless NULL, becomes 0.
+// where x is fp32 and xp_dtype says so; xp NULL: no rows); *bad_ids, unless NULL, becomes 0.
 int moe_select_count(const void* logits, int logits_dtype, const float* bias, int64_t T, int64_t E, int64_t k,
                      int32_t* ids, float* gates, void* table, void* stream);
 int moe_place_rows(const void* x, int x_dtype, const int32_t* ids, const void* table, int64_t T, int64_t H, int64_t E,
@@ -106,6 +106,10 @@ int moe_gemm_down_to(const uint16_t* act, const uint16_t* w2, const int32_t* off
 int moe_gemm_dgrad_gateup_to(const uint16_t* dg, const uint16_t* du, int64_t ld_in, const uint16_t* w1, const uint16_t* w3,
                              const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* dxp,
                              const int32_t* row_map, void* stream);
+// moe_gemm_gateup_swiglu_fwd without g and u whose row p of xp is x[pos_to_row[p] / k], for x [T,H] of sizes that it takes.
+bool moe_gateup_from_ok(int64_t T, int64_t H);
+int moe_gemm_gateup_from(const uint16_t* x, const int32_t* pos_to_row, int64_t T, int64_t k, const uint16_t* w1, const uint16_t* w3,
+                         const int32_t* offs, int64_t E, int64_t H, int64_t I, uint16_t* act, void* stream);
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;
 constexpr int FEW_MAX_EXPERTS = 128;

@@ -131,12 +131,15 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   }
   const bool few = moe_few_ok(T, H, E, I, k, x_dtype), place = !few && moe_place_ok(T, E, k);
   const bool selects = few && moe_gateup_few_selects(T, E, I, k);  // gate/up does the selection
+  // gate/up reads a token's row where it is, k times, and nobody else wants the copies in expert order
+  const bool in_place = !few && x_dtype == MOE_DT_BF16 && moe_gateup_from_ok(T, H);
+  uint16_t* rows = in_place ? nullptr : xp;
   const bool selected = router && !few_logits, at_once = place && !selected && moe_select_place_ok(logits, T, E, k);
   if (selected)
     MOE_STEP("moe_router_select", moe_router_select(*router, T, H, E, k, ids, gates, place ? ws + c.dispatch : nullptr, st));
   else if (at_once)
     MOE_STEP("moe_select_place", moe_select_place(x, x_dtype, logits, logits_dtype, bias, T, H, E, k, ids, gates, counts, offs,
-                                                  pos_to_row, row_to_pos, nullptr, xp, MOE_DT_BF16, stream));
+                                                  pos_to_row, row_to_pos, nullptr, rows, MOE_DT_BF16, stream));
   else if (place)
     MOE_STEP("moe_select_count", moe_select_count(logits, logits_dtype, bias, T, E, k, ids, gates, ws + c.dispatch, stream));
   else if (!selects)
@@ -157,17 +160,19 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   }
   if (place && !at_once) {
     MOE_STEP("moe_place_rows", moe_place_rows(x, x_dtype, ids, ws + c.dispatch, T, H, E, k, counts, offs, pos_to_row,
-                                              row_to_pos, nullptr, xp, MOE_DT_BF16, false, stream));
+                                              row_to_pos, nullptr, rows, MOE_DT_BF16, false, stream));
   } else if (!place) {
     MOE_STEP("moe_histogram_scan_checked",
              moe_histogram_scan(ids, R, E, counts, offs, pos_to_row, row_to_pos, ws + c.dispatch,
                                 moe_dispatch_workspace_bytes(R, E), stream));
-    MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
-             k > 1 ? moe_permute_fwd_scatter(x, x_dtype, row_to_pos, T, H, k, xp, stream)
-                   : moe_permute_fwd(x, x_dtype, pos_to_row, R, H, k, xp, stream));
+    if (!in_place)
+      MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
+               k > 1 ? moe_permute_fwd_scatter(x, x_dtype, row_to_pos, T, H, k, xp, stream)
+                     : moe_permute_fwd(x, x_dtype, pos_to_row, R, H, k, xp, stream));
   }
   MOE_STEP("moe_gemm_gateup_swiglu_fwd",
-           moe_gemm_gateup_swiglu_fwd(xp, w1, w3, offs, E, R, H, I, nullptr, nullptr, act, stream));
+           in_place ? moe_gemm_gateup_from((const uint16_t*)x, pos_to_row, T, k, w1, w3, offs, E, H, I, act, stream)
+                    : moe_gemm_gateup_swiglu_fwd(xp, w1, w3, offs, E, R, H, I, nullptr, nullptr, act, stream));
   MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_fwd(act, w2, offs, E, R, H, I, y, stream));
   MOE_STEP("moe_combine_fwd", moe_combine_fwd(y, gates, row_to_pos, T, H, k, out, out_dtype, stream));
   return 0;

@@ -144,13 +144,13 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
   const int lane = lane_id(), wv = uniform((int)(threadIdx.x / MOE_WAVE));
   const int chunk = blockIdx.x / (CHUNK / WAVES), chunks = (T + CHUNK - 1) / CHUNK, words = (E + 3) / 4;
   const int t = blockIdx.x * WAVES + wv;
-  const bool live = t < T;
+  const bool live = t < T, with_rows = xp != nullptr;
   typename std::conditional<sizeof(XT) == 2, u32x4, Row8>::type row[AHEAD];
   const auto request = [&](int base) {
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i) {
       const int col = base + (i * MOE_WAVE + lane) * 8;
-      if (live && col < H) {
+      if (live && with_rows && col < H) {
         if constexpr (sizeof(XT) == 2) row[i] = *reinterpret_cast<const u32x4*>(x + (size_t)t * H + col);
         else row[i] = load8(x + (size_t)t * H + col);
       }
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(WAVES* MOE_WAVE) void place_rows_kernel(
     row_to_pos[r] = pos;
     pos_to_row[pos] = r;
   }
-  if (!live) return;
+  if (!live || !with_rows) return;
   for (int base = 0; base < H; base += AHEAD * MOE_WAVE * 8) {
     if (base > 0) request(base);
     for (int j = 0; j < k; ++j) {

@@ -51,6 +51,12 @@ struct RingInner {
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) off[i] = (uint32_t)(((i * WAVES + wv) * RPP + r) * ld + kc) * 2;
   }
+  // Rows from anywhere: at(r) is the byte offset of the tile's row r.
+  template <typename At>
+  __device__ __forceinline__ void set_rows(int wv, At at) {
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) off[i] = at((i * WAVES + wv) * RPP + lane_id() / CPR) + (uint32_t)kc * 2;
+  }
   // k past the end of the contraction lies in the next row: such chunks get an offset past any view (k_left: valid k)
   __device__ __forceinline__ void load(uint32_t stage, int wv, u32x4 rsrc, int k_left) const {
     const uint32_t past = kc >= k_left ? 0xffffffffu : 0u;

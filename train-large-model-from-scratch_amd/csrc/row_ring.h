@@ -23,8 +23,8 @@ struct RingTile {
 
 // The tile of expert e, whose rows are first .. row_end, at its row `row` and column n0.  By the whole workgroup; `ring`: LDS bytes
 // of LDS that nobody else uses.  BLK: g and u are kept in blocks, as the kernels of larger tiles keep them; TO: the result's rows
-// go where p.row_map says (see there).
-template <int MODE, bool BLK, int FM, int WAVES, bool TO = false>
+// go where p.row_map says, FROM: A's come from where p.row_from says (see there).
+template <int MODE, bool BLK, int FM, int WAVES, bool TO = false, bool FROM = false>
 __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, int first, int row_end, int row, int n0) {
   using O = RingTile<MODE, FM, WAVES>;
   using OpA = typename O::OpA;
@@ -38,7 +38,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
   const long long a_at = (long long)row0 * lda, a_valid = (long long)(row_end - row0) * lda;
   const long long b_at = (long long)e * p.K * p.N + (long long)n0 * (B_OUTER ? 1 : p.K);
   const long long b_valid = (long long)p.K * p.N - (long long)n0 * (B_OUTER ? 1 : p.K);
-  vA[0] = make_view(p.A0 + a_at, a_valid);
+  vA[0] = FROM ? View{p.A0, p.from_bytes} : make_view(p.A0 + a_at, a_valid);
   vB[0] = make_view(p.B0 + b_at, b_valid);
   if constexpr (NSEG == 2) vA[1] = make_view(p.A1 + a_at, a_valid);
   if constexpr (NSEG == 2 || DUAL) vB[1] = make_view(p.B1 + b_at, b_valid);
@@ -49,6 +49,8 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, char* ring, int e, 
   OpA opA;
   OpB opB;
   opA.init(lda, wv);
+  if constexpr (FROM)
+    opA.set_rows(wv, [&](int r) { return row0 + r < row_end ? (uint32_t)p.by_k(p.row_from[row0 + r]) * (uint32_t)(lda * 2) : NO_ROW; });
   opB.init(ldb, wv);
   const uint32_t ring0 = lds_address(ring);
   int ask_seg = 0, ask_k = 0;

@@ -36,7 +36,7 @@ struct Experts {
   }
 };
 
-template <int MODE, bool BLK, int FM, bool TO>
+template <int MODE, bool BLK, int FM, bool TO, bool FROM>
 __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
   using O = RingTile<MODE, FM, 4>;
   constexpr int BM = O::BM;
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256, 2) void ring_rows_kernel(const GemmArgs p) {
   const int first = read_lane(high ? ex.first[1] : ex.first[0], l), row_end = read_lane(high ? ex.end[1] : ex.end[0], l);
   const int nt = (row_end - first + BM - 1) / BM;
   const int in = tile - (read_lane(high ? ex.upto[1] : ex.upto[0], l) - nt) * p.n_tiles;
-  ring_tile<MODE, BLK, FM, 4, TO>(p, ring, e, first, row_end, in % nt * BM, in / nt * O::BNC);
+  ring_tile<MODE, BLK, FM, 4, TO, FROM>(p, ring, e, first, row_end, in % nt * BM, in / nt * O::BNC);
 }
 
 // Tiles side by side.  (dgrad-down's sums cover the columns in steps of 256)
@@ -66,13 +66,13 @@ int columns(int N) {
 }
 
 // Launches of at most `most` tiles (by the bound that R and E give), or of any number.
-template <int MODE, bool BLK, int FM, bool TO>
+template <int MODE, bool BLK, int FM, bool TO, bool FROM>
 bool launch(GemmArgs a, long long most, bool any, hipStream_t s, int* rc) {
   using O = RingTile<MODE, FM, 4>;
   a.n_tiles = columns<MODE>(a.N);
   const long long tiles = ((a.R + O::BM - 1) / O::BM + (long long)a.E) * a.n_tiles;
   if (tiles > (any ? 0x7fffff00ll : most)) return false;
-  const auto kern = ring_rows_kernel<MODE, BLK, FM, TO>;
+  const auto kern = ring_rows_kernel<MODE, BLK, FM, TO, FROM>;
   static bool attr_done[MOE_MAX_DEVICES];
   const int dev = moe_current_device();
   if (!attr_done[dev]) {
@@ -123,22 +123,22 @@ bool small_tiles_pay(const GemmArgs& a) {
 // 192, down 18.4 -> 12.1; 3784 of 16, 384 <-> 896, dgrad-down 16.3 -> 12.0 (in tiles of 64).  Of 472 launches of 300 drawn layers
 // with a launch past the bound, weights cold, gate/up take 0.94, down 0.955, dgrad-down 0.96 and dgrad-gate/up 0.985 of the time in the
 // mean, one in thirty is slower by more than 3 % (up to 1.10, by heavy experts).
-template <int MODE, bool BLK, bool TO = false>
+template <int MODE, bool BLK, bool TO = false, bool FROM = false>
 bool choose(const GemmArgs& a, int forced, hipStream_t s, int* rc) {
   const long long slots = 2ll * moe_compute_units();
-  if (forced == 128) return launch<MODE, BLK, 2, TO>(a, slots, true, s, rc);
-  if (launch<MODE, BLK, 1, TO>(a, slots, forced != 0, s, rc)) return true;
+  if (forced == 128) return launch<MODE, BLK, 2, TO, FROM>(a, slots, true, s, rc);
+  if (launch<MODE, BLK, 1, TO, FROM>(a, slots, forced != 0, s, rc)) return true;
   constexpr bool FUSED = MODE == GATEUP || MODE == DGRAD_DOWN;
-  if (!FUSED && launch<MODE, BLK, 2, TO>(a, slots, false, s, rc)) return true;
+  if (!FUSED && launch<MODE, BLK, 2, TO, FROM>(a, slots, false, s, rc)) return true;
   constexpr int LONGEST = MODE == GATEUP ? 640 : MODE == DGRAD_DOWN ? 768 : 1280;
   const double cols = columns<MODE>(a.N), k = (double)a.K * (MODE == DGRAD_GATEUP ? 2 : 1);
   const double most = 0.95 * slots;
-  if (FUSED && moe_expected_tiles(a.R, a.E, 64) * cols <= most) return launch<MODE, BLK, 1, TO>(a, slots, true, s, rc);
+  if (FUSED && moe_expected_tiles(a.R, a.E, 64) * cols <= most) return launch<MODE, BLK, 1, TO, FROM>(a, slots, true, s, rc);
   const double tall = moe_expected_tiles(a.R, a.E, 128) * cols;
   if (a.R >= 64ll * a.E &&
       ((tall <= most && k <= LONGEST) || (tall <= 2 * most && k <= 320 && MODE != DGRAD_GATEUP)))
-    return launch<MODE, BLK, 2, TO>(a, slots, true, s, rc);
-  return small_tiles_pay<MODE>(a) && launch<MODE, BLK, 1, TO>(a, slots, true, s, rc);
+    return launch<MODE, BLK, 2, TO, FROM>(a, slots, true, s, rc);
+  return small_tiles_pay<MODE>(a) && launch<MODE, BLK, 1, TO, FROM>(a, slots, true, s, rc);
 }
 
 }  // namespace
@@ -148,7 +148,8 @@ bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, int forced, hipSt
   switch (mode) {
     case GATEUP:
       if (blocked) return choose<GATEUP, true>(a, forced, s, rc);
-      return !a.C0 && choose<GATEUP, false>(a, forced, s, rc);  // (g and u in rows: not here)
+      if (a.C0) return false;  // (g and u in rows: not here)
+      return a.row_from ? choose<GATEUP, false, false, true>(a, forced, s, rc) : choose<GATEUP, false>(a, forced, s, rc);
     case DOWN: return a.row_map ? choose<DOWN, false, true>(a, forced, s, rc) : choose<DOWN, false>(a, forced, s, rc);
     case DGRAD_DOWN: return blocked && choose<DGRAD_DOWN, true>(a, forced, s, rc);
     default: return a.row_map ? choose<DGRAD_GATEUP, false, true>(a, forced, s, rc) : choose<DGRAD_GATEUP, false>(a, forced, s, rc);

@@ -41,6 +41,9 @@ __device__ __forceinline__ Window window(const View& w, long long byte_off) {
   return {(const char*)w.base + byte_off, window_size(w.bytes - byte_off)};
 }
 
+// A byte offset outside any window that rows are read from anywhere of (less than 2 GB).
+constexpr uint32_t NO_ROW = 1u << 31;
+
 // ---- operand staging ----------------------------------------------------------------------
 // Two LDS layouts, one per memory order of the operand, each with the fragment read that
 // hands an MFMA lane its 8 consecutive k values for row (lane % 32):
@@ -72,6 +75,14 @@ struct OpInner {
 #pragma unroll
     for (int i = 0; i < CH; ++i) voff[i] = ((r + i * RSTEP) * ld + kc) * 2;
     lds_w = r * LDK + kc;
+  }
+  // Rows from anywhere: lane l has the byte offset of row own_row(l), of which the wave's lanes read CH * RPW.
+  static constexpr int RPW = MOE_WAVE / CPR;  // rows of a wave's chunk
+  static_assert(CH * RPW <= MOE_WAVE, "a lane a row");
+  static __device__ __forceinline__ int own_row(int wv, int lane) { return wv * RPW + lane % RPW + lane / RPW * RSTEP; }
+  __device__ __forceinline__ void set_rows(uint32_t at) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) voff[i] = (int)(__shfl(at, lane_id() / CPR + i * RPW, MOE_WAVE) + (uint32_t)kc * 2);
   }
   static __device__ __forceinline__ long long k_bytes(int k0, int /*ld*/) { return (long long)k0 * 2; }
   __device__ __forceinline__ u32x4 load_one(int i, __amdgpu_buffer_rsrc_t rs) const {
