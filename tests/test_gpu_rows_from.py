@@ -1,0 +1,56 @@
+"""A layer with its router keeps no rows in expert order where its weight gradients are tiled: gate/up and the gradients of its weights read
+the tokens' rows.  With the logits given it keeps them: the same bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,H,E,I,k,skew", [
+    (2600, 1024, 128, 256, 8, 0.6),   # two stacks in one result; experts of one k-tile to a dozen
+    (1800, 2040, 64, 520, 6, 0.5),    # three problems, columns that end in the middle
+    (5200, 2048, 64, 1024, 2, 2.0),   # dealt longest first; experts with a row or two and without any
+    (10400, 1992, 64, 1000, 1, 1.0),
+    (9216, 1536, 48, 768, 1, -1.0),   # 192 rows each: whole k-tiles
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])  # of the weights and their gradients
+def test_training_reads_the_tokens(pkg, T, H, E, I, k, skew, dtype):
+    print("rows from the tokens, training", T, H, E, I, k, skew, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    x, dy, ws = r(T, H), r(T, H), [w.to(dtype) for w in (r(E, I, H), r(E, I, H), r(E, H, I))]
+    wr = r(E, H) * 0.02
+    bias = -skew * torch.arange(E, device="cuda", dtype=torch.float32).log1p()
+    if skew < 0:  # every expert in turn
+        wr = wr * 0
+        x[:, :E] = 0
+        x[torch.arange(T, device="cuda"), torch.arange(T, device="cuda") % E] = 1
+        wr[torch.arange(E, device="cuda"), torch.arange(E, device="cuda")] = 1
+        bias = None
+    calls = []
+
+    class Obs:
+        def before(self, name):
+            calls.append(name)
+
+        def after(self, name):
+            pass
+
+    def passed(layer):
+        leaves = [w.detach().requires_grad_(True) for w in ws]
+        lib.observer = Obs()
+        try:
+            out, logits = layer(*leaves)
+            out.backward(dy)
+        finally:
+            lib.observer = None
+        return out.detach(), logits.detach(), [w.grad for w in leaves]
+
+    lib = pkg.ops._lib.load()
+    xr = x.detach().requires_grad_(True)
+    out, logits, grads = passed(lambda a, b, c: pkg.routed_moe(xr, wr, a, b, c, k, bias=bias))
+    assert "moe_gemm_wgrad_all" in calls
+    want, _, want_grads = passed(lambda a, b, c: (pkg.moe_ffn(x, logits, a, b, c, k, bias=bias), logits))
+    assert torch.equal(out, want)
+    for i, (a, b) in enumerate(zip(grads, want_grads)):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), i

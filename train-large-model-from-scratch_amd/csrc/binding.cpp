@@ -138,7 +138,7 @@ int64_t up(int64_t n, int64_t to) { return (n + to - 1) / to * to; }
 
 // What a forward pass leaves for the backward pass besides its inputs: the routing (int32 words, parts in
 // this order: ids, gates, counts, offs, pos_to_row, row_to_pos, bad ids) and the expert-ordered rows xp
-// with gu and act behind them.
+// (unless the experts read x where it is) with gu and act behind them.
 struct Routing {
   enum Part { IDS, GATES, COUNTS, OFFS, POS_TO_ROW, ROW_TO_POS, BAD, PARTS };
   int64_t at[PARTS + 1];
@@ -152,8 +152,8 @@ struct Routing {
 
 struct Kept {
   int64_t gu, act, total;
-  Kept(int64_t R, int64_t H, int64_t E, int64_t I, bool with_gu) {
-    gu = up(R * H * 2, 256);
+  Kept(int64_t R, int64_t H, int64_t E, int64_t I, bool with_gu, bool with_xp) {
+    gu = with_xp ? up(R * H * 2, 256) : 0;
     act = gu + (with_gu ? up(moe_gu_blocked_bytes(R, E, I), 256) : 0);
     total = act + up(R * I * 2, 256);
     if (total == 0) total = 256;
@@ -222,6 +222,7 @@ struct Layer {  // the arguments of one call
 struct Outputs {
   Tensor out, logits, routing, kept, xn, wrb, nw, rstd;
   Weights w;
+  bool in_place = false;  // no rows in expert order are kept: xn is read instead
 };
 
 Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Tensor& wr, const Tensor& logits_,
@@ -343,7 +344,9 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
     return f;
   }
   f.out = empty({T, H}, x_type, x);
-  const Kept kept(R, H, E, I, o.train);
+  // (only where xn is saved whatever happens: with given logits or experts the caller may change x after the call)
+  f.in_place = o.train && f.xn.defined() && moe_layer_rows_from_ok(T, H, E, I, k);
+  const Kept kept(R, H, E, I, o.train, !f.in_place);
   f.kept = empty({kept.total}, at::kByte, x);
   char* base = (char*)f.kept.data_ptr();
   Tensor ids = ids_;
@@ -367,7 +370,7 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   a.w1 = bf(f.w.w1), a.w3 = bf(f.w.w3), a.w2 = bf(f.w.w2);
   a.residual = o.add_residual ? x.data_ptr() : nullptr;
   a.out = f.out.data_ptr(), a.out_dtype = dt(x_type);
-  a.xp = (uint16_t*)base;
+  a.xp = f.in_place ? nullptr : (uint16_t*)base;
   a.gu = o.train ? base + kept.gu : nullptr;
   a.act = (uint16_t*)(base + kept.act);
   const int64_t bytes = std::max<int64_t>(moe_forward_scratch(&a), 256);
@@ -444,7 +447,7 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
     ctx->saved_data["i"] = std::vector<int64_t>{x.size(0), x.size(1), o.k, o.add_residual, type(x), type(norm_w),
                                                 type(wr), type(logits), type(w1),
                                                 Present{true, norm_w.defined(), wr.defined(), logits.defined(), true, true,
-                                                        true, bias.defined(), ids.defined()}.mask};
+                                                        true, bias.defined(), ids.defined()}.mask, f.in_place};
     if (o.accumulate) {
       std::vector<Tensor> params;
       for (const Tensor* w : {&w1, &w3, &w2}) params.push_back(w->requires_grad() && w->is_leaf() ? *w : Tensor());
@@ -497,7 +500,8 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
     if (!by_hand && want_logits) dlogits = empty({T, E}, type(7), kept_buf);
 
     const Routing r(R, E);
-    const Kept kept(R, H, E, I, true);
+    const bool in_place = ints[10];
+    const Kept kept(R, H, E, I, true, !in_place);
     const char* base = (const char*)kept_buf.data_ptr();
     void* s = stream_of(kept_buf);
     moe_layer_backward_args a{};
@@ -508,7 +512,7 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
     a.gates = gates, a.ids = ids;
     a.offs = r.part(routing, Routing::OFFS);
     a.pos_to_row = r.part(routing, Routing::POS_TO_ROW), a.row_to_pos = r.part(routing, Routing::ROW_TO_POS);
-    a.xp = (const uint16_t*)base, a.gu = base + kept.gu, a.act = (const uint16_t*)(base + kept.act);
+    a.xp = in_place ? nullptr : (const uint16_t*)base, a.gu = base + kept.gu, a.act = (const uint16_t*)(base + kept.act);
     a.w1 = bf(w[0]), a.w3 = bf(w[1]), a.w2 = bf(w[2]);
     for (int i = 0; i < 3; ++i) {
       a.dw[i] = ptr(wg.into[i]);
@@ -524,7 +528,7 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
     const int64_t bytes = std::max<int64_t>(moe_backward_scratch(&a), 256);
     const Tensor scratch = empty({bytes}, at::kByte, kept_buf);
     a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
-    check(moe_layer_backward(&a, s), "moe_layer_backward");
+    check(in_place ? moe_in_place_layer_backward(&a, s) : moe_layer_backward(&a, s), "moe_layer_backward");
     for (int i = 0; i < 3; ++i)
       if (wg.fresh[i].defined()) params[i].mutable_grad() = wg.fresh[i];
     if (dwr.defined() && !wr_direct) dwr = dwr.to(type(6));

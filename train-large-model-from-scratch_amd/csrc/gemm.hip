@@ -82,12 +82,14 @@ __device__ __forceinline__ int expert_of(const int* tile_start, int slot, int E)
 // The kernel's tile walk: the tiles at positions t_next, t_next + t_step, .. below t_hi of the launch's tile
 // list, or of `list` where one is given.  The rows of a row-ragged launch are numbered in tiles of UNIT rows; where
 // the configuration's are half as high, a list entry is 2 * tile + half.  (tile_start and, there, offs: in LDS.)
-// TO (DOWN and DGRAD_GATEUP only): the rows leave to where p.row_map says.  FROM (GATEUP only): A's rows come from where p.row_from says.
+// TO (DOWN and DGRAD_GATEUP only): the rows leave to where p.row_map says.  FROM (GATEUP: A's rows; WGRAD: B's lines): they
+// come from where p.row_from says.
 template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE, bool TO = false, bool FROM = false>
 __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, const int* tile_start, const int* offs,
                                            const uint32_t* list, int t_next, const int t_hi, const int t_step) {
   static_assert(!BLK || MODE == GATEUP || MODE == DGRAD_DOWN, "only g and u have the blocked layout");
-  static_assert(!FROM || MODE == GATEUP, "only x is read where the caller has it");
+  static_assert(!FROM || MODE == GATEUP || MODE == WGRAD, "only x is read where the caller has it");
+  constexpr bool ROWS_FROM = FROM && MODE == GATEUP, LINES_FROM = FROM && MODE == WGRAD;
   static_assert(!TO || MODE == DOWN || MODE == DGRAD_GATEUP, "only y and dxp are rows that somebody else has a place for");
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, KS = Cfg::KS;
   constexpr int FM = Cfg::FM, FN = Cfg::FN, WTM = Cfg::WTM, WTN = Cfg::WTN;
@@ -189,7 +191,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       }
     } else {  // WGRAD: A = a [R,M] as [k][m]; B = b [R,N] as [k][n]; k = rows of expert e
       t.vA0 = make_view(p.A0 + (long long)t.row0 * lda + t.m0, rows * lda - t.m0);
-      t.vB0 = make_view(p.B0 + (long long)t.row0 * ldb + t.n0, rows * ldb - t.n0);
+      t.vB0 = LINES_FROM ? View{p.B0 + t.n0, p.from_bytes - t.n0 * 2}
+                         : make_view(p.B0 + (long long)t.row0 * ldb + t.n0, rows * ldb - t.n0);
     }
     return true;
   };
@@ -209,13 +212,27 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   // that request the row where the first k-tile of its tile is asked for.
   int row_from = 0;
   auto ask_rows = [&](const Tile& t) {
-    if constexpr (FROM) {
+    if constexpr (ROWS_FROM) {
       const int r = t.row0 + StA::own_row(wv, lane);
       row_from = r < t.row_end ? p.row_from[r] : -1;
     }
   };
   auto set_rows = [&]() {
-    if constexpr (FROM) opA.set_rows(row_from < 0 ? NO_ROW : (uint32_t)p.by_k(row_from) * (uint32_t)(lda * 2));
+    if constexpr (ROWS_FROM) opA.set_rows(row_from < 0 ? NO_ROW : (uint32_t)p.by_k(row_from) * (uint32_t)(lda * 2));
+  };
+  // (WGRAD: the lines of a k-tile, asked for while the k-tile before is requested.  `lines_left`: how many of them the expert has.)
+  int lines_left = 0;
+  auto ask_lines = [&](int first, int end) {
+    if constexpr (LINES_FROM) {
+      lines_left = end - first;
+      const __amdgpu_buffer_rsrc_t rs =
+          __builtin_amdgcn_make_buffer_rsrc((void*)(p.row_from + first), 0, lines_left > 0 ? lines_left * 4 : 0, 0x00020000);
+      row_from = __builtin_amdgcn_raw_buffer_load_b32(rs, StB::own_line(wv, lane) * 4, 0, 0);
+    }
+  };
+  auto set_lines = [&]() {
+    if constexpr (LINES_FROM)
+      opB.set_lines(StB::own_line(wv, lane) < lines_left ? (uint32_t)p.by_k(row_from) * (uint32_t)(ldb * 2) : NO_ROW);
   };
   // One set of registers carries a k-tile from HBM to LDS: it is requested one iteration
   // before it is written to LDS, which is what hides the latency of a load that misses L2.
@@ -244,7 +261,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     const bool second = NSEG == 2 && kt >= t.kt_per_seg;
     if (op == 0) return window(second ? t.vA1 : t.vA0, StA::k_bytes(k0, lda));
     if constexpr (DUAL) return window(op == 1 ? t.vB0 : t.vB1, StBh::k_bytes(k0, ldb));
-    else return window(second ? t.vB1 : t.vB0, StB::k_bytes(k0, ldb));
+    else return window(second ? t.vB1 : t.vB0, LINES_FROM ? 0 : StB::k_bytes(k0, ldb));
   };
   auto tile_src = [&](const Tile& t, int kt) {
     TileSrc ts;
@@ -282,6 +299,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   };
   auto load_tile = [&](const Tile& t, int kt, Stage& st) {
     const TileSrc ts = tile_src(t, kt);
+    set_lines();
 #pragma unroll
     for (int c = 0; c < NCH; ++c) load_chunk(c, st, ts);
     if (t.need_mask && ts.k_left < BK) {
@@ -348,7 +366,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   // of the first one the forty scalar instructions, with six 64-bit comparisons in the vector unit among them, held up both waves of a
   // SIMD, which come from the same barrier.  Whole passes, us, in turn on one GPU: 1531 tokens, 8 of 64 experts, forward, 265.4 -> 262.6; 8192, 2 of
   // 8, 1024 <-> 512, 317.7 -> 313.7; smaller ones 1.00 to 1.02; 16384 tokens of 64, where power is the bound, equal.
-  auto body = [&](auto par_c, const Tile& t, int kt, TileSrc& ts) {
+  auto body = [&](auto par_c, const Tile& t, int kt, TileSrc& ts, auto&& lines_behind) {
     constexpr int buf = decltype(par_c)::value;  // LDS stage of k-tile kt == parity of kt
     Stage& st = stg;                             // holds k-tile kt+1, refilled with kt+2, which lies at `ts`
     constexpr int NSLOT = (KS - 1) * NMMA;  // MFMA slots before the barrier
@@ -362,6 +380,10 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
         for (int c = 0; c < NCH; ++c) {
           if (c * NSLOT / NCH == slot) {
             store_chunk(c, st, buf ^ 1);
+            if (LINES_FROM && c == 0) {
+              set_lines();
+              lines_behind(kt + 2);
+            }
             load_chunk(c, st, ts);
             if (c + 1 == NCH || operand_of(c + 1) != operand_of(c)) {
               Window& w = ts.w[operand_of(c)];
@@ -707,7 +729,11 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       for (int c = 0; c < NCH; ++c) asm volatile("" : "=v"(stg.v[c]));
     }
   };
-  auto request_first = [&](const Tile& t) { request_k(t, 0); };
+  auto request_first = [&](const Tile& t) {
+    ask_lines(t.row0, t.row_end);
+    request_k(t, 0);
+    ask_lines(t.row0 + BK, t.row_end);
+  };
   Tile cur;
   if (t_next >= t_hi || !locate(tile_at(t_next), cur)) return;
   ask_rows(cur);
@@ -749,20 +775,37 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       }
     }
     const int nkt = cur.nkt;
-    const bool stream = STREAM && more && nkt > 1 && nxt.nkt > 0;  // the k-tiles of the next tile follow this one's
+    // the k-tiles of the next tile follow this one's.  (Lines from anywhere: unless this tile would request all of them, and the lines of
+    // a tile behind it would have to be asked for, which is not known yet; the registers for asking at one place more are not there.)
+    const bool stream = STREAM && more && nkt > 1 && nxt.nkt > (LINES_FROM ? 2 : 0);
+    // the lines of the k-tile behind kt
+    auto lines_behind = [&](int kt) {
+      if constexpr (LINES_FROM) {
+        const int next = kt + 1;
+        const bool here = next < nkt;
+        ask_lines(here ? cur.row0 + next * BK : stream ? nxt.row0 + (next - nkt) * BK : 0, here ? cur.row_end : stream ? nxt.row_end : 0);
+      }
+    };
     // the k-tile two behind kt
     auto request_ahead = [&](int kt) {
-      if (kt + 2 < nkt) load_tile(cur, kt + 2, stg);
+      if (kt + 2 < nkt) {
+        load_tile(cur, kt + 2, stg);
+        lines_behind(kt + 2);
+      }
       else if (stream && kt + 2 - nkt < (EARLY_REQUEST ? nxt.nkt : 1)) {
         if (kt + 2 == nkt) set_rows();
         load_tile(nxt, kt + 2 - nkt, stg);
+        lines_behind(kt + 2);
       }
     };
     if (nkt > 0) {
       if (!staged) {
         s0 = 0;
         store_tile(stg, 0);
-        if (1 < nkt) load_tile(cur, 1, stg);
+        if (1 < nkt) {
+          load_tile(cur, 1, stg);
+          lines_behind(1);
+        }
         lds_barrier();
       }
       if (!idle) f_read_all(s0, 0, fr[0]);
@@ -829,8 +872,8 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       if (!((kt + s0) & 1)) {
         TileSrc ts = tile_src(cur, kt + 2);
         for (; kt + 1 < steady_end; kt += 2) {
-          body(integral_constant<int, 0>{}, cur, kt, ts);
-          body(integral_constant<int, 1>{}, cur, kt + 1, ts);
+          body(integral_constant<int, 0>{}, cur, kt, ts, lines_behind);
+          body(integral_constant<int, 1>{}, cur, kt + 1, ts, lines_behind);
         }
       }
       one(kt);
@@ -1080,7 +1123,7 @@ struct WgradArgs {
 // faster dealt in groups than with contiguous ranges of equal work, another 9-10 % longest
 // first; near-uniform routing: the same in all three.)  A tile of an expert costs the same in every problem: the next one's
 // groups are dealt on from where the last one's left the XCDs.
-template <typename OutT>
+template <typename OutT, bool FROM>
 __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_gemm_kernel(const WgradArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   const int lane = threadIdx.x & 63;
@@ -1171,7 +1214,9 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_ge
       first = lo + j, end = lo + q + (x < r ? 1 : 0), step = (nb >> 3) + (x < (nb & 7) ? 1 : 0);
     }
     if (w) __syncthreads();  // (the operand stages are free)
-    walk_tiles<WGRAD, CfgMain, OutT, false>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
+    if (FROM && p.row_from)
+      walk_tiles<WGRAD, CfgMain, OutT, false, ROW_TILE, false, FROM>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
+    else walk_tiles<WGRAD, CfgMain, OutT, false>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
     done += total;
   }
 }
@@ -1265,8 +1310,10 @@ int launch_wgrad(const WgradArgs& args, hipStream_t s) {
     const long long n = (long long)a.n_tiles * a.m_slots * a.E;
     tiles = tiles > n ? tiles : n;
   }
-  static bool attr_done[MOE_MAX_DEVICES];
-  return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT>, attr_done, w, tiles, s);
+  static bool attr_done[2][MOE_MAX_DEVICES];
+  for (int i = 0; i < w.n; ++i)
+    if (w.p[i].row_from) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, true>, attr_done[1], w, tiles, s);
+  return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, false>, attr_done[0], w, tiles, s);
 }
 
 int check_common(const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I) {
@@ -1289,19 +1336,23 @@ int check_common(const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I
 // / 1531 / 4000 / 16384 tokens 166 -> 163, 187 -> 180, 245 -> 230, 496 -> 469, 1742 -> 1639; 8192 of 128, 1024 <-> 256, 232 -> 204; 2048 of 8, 1024 <->
 // 512, 42.6 -> 40.3; 3333 of 12, 1416 <-> 568, 99 -> 92; 16000, 1 of 4, 512 <-> 256, 60.6 -> 57.1; no size of 16 slower.  A lane's
 // offset and a window's size have 32 bits, and one of them marks rows that there are none of: hence the limit.
-bool moe_gateup_from_ok(int64_t T, int64_t H) { return T * H < (int64_t)1 << 30; }
+bool moe_rows_from_ok(int64_t T, int64_t H) { return T * H < (int64_t)1 << 30; }
 
 int moe_gemm_gateup_from(const uint16_t* x, const int32_t* pos_to_row, int64_t T, int64_t k, const uint16_t* w1, const uint16_t* w3,
-                         const int32_t* offs, int64_t E, int64_t H, int64_t I, uint16_t* act, void* stream) {
+                         const int32_t* offs, int64_t E, int64_t H, int64_t I, void* gu_blocked, uint16_t* act, void* stream) {
   const int64_t R = T * k;
   if (int rc = check_common(offs, E, R, H, I)) return rc;
   if (R == 0) return 0;
-  if (!moe_gateup_from_ok(T, H)) return MOE_ERR_LIMIT;
+  if (!moe_rows_from_ok(T, H)) return MOE_ERR_LIMIT;
   MOE_CHECK_PTR(x); MOE_CHECK_PTR(w1); MOE_CHECK_PTR(w3); MOE_CHECK_PTR(act); MOE_CHECK_PTR(pos_to_row);
   GemmArgs a{};
-  a.A0 = x; a.B0 = w1; a.B1 = w3; a.C2 = act; a.offs = offs;
+  a.A0 = x; a.B0 = w1; a.B1 = w3; a.C0 = gu_blocked; a.C2 = act; a.offs = offs;
   a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H;
   a.row_from = pos_to_row; a.by_k.set((uint32_t)k); a.from_bytes = T * H * 2;
+  if (gu_blocked) {
+    MOE_CHECK_PTR(gu_blocked);
+    return launch_rows<GATEUP, true, false, true>(a, CfgMain::BN / 2, (hipStream_t)stream);
+  }
   return launch_rows<GATEUP, false, false, true>(a, CfgMain::BN / 2, (hipStream_t)stream);
 }
 
@@ -1496,6 +1547,10 @@ int moe_gemm_wgrad_all(const MoeWgradStack* stacks, int n, const int32_t* offs, 
     const int rc = m.out2 ? wgrad_pair_args(w.p[w.n], m.a, m.b, offs, E, R, m.M / 2, m.N, m.out, m.out2, m.dtype, m.accumulate)
                           : wgrad_args(w.p[w.n], m.a, m.b, offs, E, R, m.M, m.N, m.out, m.dtype, m.accumulate);
     if (rc) return rc;
+    if (m.row_from) {
+      if (!moe_rows_from_ok(m.from_rows, m.N)) return MOE_ERR_LIMIT;
+      w.p[w.n].row_from = m.row_from, w.p[w.n].by_k.set((uint32_t)m.from_k), w.p[w.n].from_bytes = m.from_rows * m.N * 2;
+    }
   }
   return run_wgrad(w, stacks[0].dtype, stream);
 }

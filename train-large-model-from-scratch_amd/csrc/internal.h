@@ -49,6 +49,8 @@ struct MoeWgradStack {
   int64_t lda, ldb, M, N;
   int dtype, accumulate;
   void* out2;  // moe_gemm_wgrad_all: an expert's rows M / 2 .. M - 1 go here (NULL: all to out)
+  const int32_t* row_from;  // moe_gemm_wgrad_all: row r of b is row row_from[r] / from_k of its from_rows (NULL: row r)
+  int64_t from_k, from_rows;
 };
 // Weight gradients leave with streaming stores from so many bytes of results in a launch on, an eighth of the memory-side cache: a
 // model of a few such layers finds smaller ones there when it adds them up, clips them or steps.  Pass, pass with its gradients added
@@ -106,10 +108,10 @@ int moe_gemm_down_to(const uint16_t* act, const uint16_t* w2, const int32_t* off
 int moe_gemm_dgrad_gateup_to(const uint16_t* dg, const uint16_t* du, int64_t ld_in, const uint16_t* w1, const uint16_t* w3,
                              const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* dxp,
                              const int32_t* row_map, void* stream);
-// moe_gemm_gateup_swiglu_fwd without g and u whose row p of xp is x[pos_to_row[p] / k], for x [T,H] of sizes that it takes.
-bool moe_gateup_from_ok(int64_t T, int64_t H);
+// moe_gemm_gateup_swiglu_fwd_blocked (gu_blocked NULL: moe_gemm_gateup_swiglu_fwd without g and u) whose row p of xp is x[pos_to_row[p] / k], for x [T,H] of sizes that it takes.
+bool moe_rows_from_ok(int64_t T, int64_t H);
 int moe_gemm_gateup_from(const uint16_t* x, const int32_t* pos_to_row, int64_t T, int64_t k, const uint16_t* w1, const uint16_t* w3,
-                         const int32_t* offs, int64_t E, int64_t H, int64_t I, uint16_t* act, void* stream);
+                         const int32_t* offs, int64_t E, int64_t H, int64_t I, void* gu_blocked, uint16_t* act, void* stream);
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;
 constexpr int FEW_MAX_EXPERTS = 128;

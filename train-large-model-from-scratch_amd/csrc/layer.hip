@@ -132,7 +132,7 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   const bool few = moe_few_ok(T, H, E, I, k, x_dtype), place = !few && moe_place_ok(T, E, k);
   const bool selects = few && moe_gateup_few_selects(T, E, I, k);  // gate/up does the selection
   // gate/up reads a token's row where it is, k times, and nobody else wants the copies in expert order
-  const bool in_place = !few && x_dtype == MOE_DT_BF16 && moe_gateup_from_ok(T, H);
+  const bool in_place = !few && x_dtype == MOE_DT_BF16 && moe_rows_from_ok(T, H);
   uint16_t* rows = in_place ? nullptr : xp;
   const bool selected = router && !few_logits, at_once = place && !selected && moe_select_place_ok(logits, T, E, k);
   if (selected)
@@ -171,7 +171,7 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
                      : moe_permute_fwd(x, x_dtype, pos_to_row, R, H, k, xp, stream));
   }
   MOE_STEP("moe_gemm_gateup_swiglu_fwd",
-           in_place ? moe_gemm_gateup_from((const uint16_t*)x, pos_to_row, T, k, w1, w3, offs, E, H, I, act, stream)
+           in_place ? moe_gemm_gateup_from((const uint16_t*)x, pos_to_row, T, k, w1, w3, offs, E, H, I, nullptr, act, stream)
                     : moe_gemm_gateup_swiglu_fwd(xp, w1, w3, offs, E, R, H, I, nullptr, nullptr, act, stream));
   MOE_STEP("moe_gemm_down_fwd", moe_gemm_down_fwd(act, w2, offs, E, R, H, I, y, stream));
   MOE_STEP("moe_combine_fwd", moe_combine_fwd(y, gates, row_to_pos, T, H, k, out, out_dtype, stream));
@@ -348,8 +348,19 @@ int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
   return s.at;
 }
 
-// (`router` and `table`: see router.h)
-static int layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream) {
+// Training steps in which nobody but gate/up and the tiled gradients of its weights would read rows in expert order: both read x where it
+// is, a lane's offset a row, those of a k-tile of the gradients asked for a k-tile ahead.  Besides the pass the copies (R x H x 2 bytes, a
+// step's largest buffer) go from memory's traffic and from what is held between the passes.  Steps with the copies and this one, the same bits, us:
+// 16384 tokens, 8 of 64 experts, 2048 <-> 1024, 4992 -> 4909; 8192 with norm and fp32 gradients 2933 -> 2906; 4096, 8 of 128, 1024 <-> 256, fp32
+// gradients, 409 -> 394; 9000, 4 of 64 by Zipf's shares, 1416 <-> 1000, 2116 -> 2091; 16000, 1 of 32, 2000 <-> 800, 980 -> 971; 8000, 8 of
+// 128, 256 <-> 640, 500 -> 500.  Tiles of one or two k-tiles have none to ask ahead in: rows an expert, 64 experts, 2048 <-> 1024, 250 947 -> 932;
+// 125 676 -> 687; 100 653 -> 675; 75 629 -> 651; 162 of 32 474 -> 472.
+bool moe_layer_rows_from_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
+  return T > 0 && sizes_ok(T, H, E, I, k) && moe_rows_from_ok(T, H) && T * k >= 160 * E && !wgrad_multi(E, I, H, T * k);
+}
+
+// (`router` and `table`: see router.h; `in_place`: no xp, x is in bf16)
+static int layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, bool in_place, void* stream) {
   if (!a) return MOE_ERR_NULL;
   const int64_t T = a->T, H = a->H, E = a->E, I = a->I, k = a->k, R = T * k;
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
@@ -368,7 +379,8 @@ static int layer_forward(const moe_layer_forward_args* a, const MoeRouter* route
     MOE_CHECK_PTR(a->ids);
     MOE_CHECK_PTR(a->pos_to_row);
     MOE_CHECK_PTR(a->row_to_pos);
-    MOE_CHECK_PTR(a->xp);
+    if (!in_place) MOE_CHECK_PTR(a->xp);
+    else if (a->x_dtype != MOE_DT_BF16) return MOE_ERR_DTYPE;
     MOE_CHECK_PTR(a->act);
   }
   if (a->logits && !a->gates) return MOE_ERR_NULL;
@@ -406,11 +418,15 @@ static int layer_forward(const moe_layer_forward_args* a, const MoeRouter* route
              moe_histogram_scan_checked(a->ids, R, E, a->counts, a->offs, a->pos_to_row, a->row_to_pos, a->bad_ids,
                                         ws.dispatch, moe_dispatch_workspace_bytes(R, E), stream));
     if (T == 0) return 0;
-    MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
-             k > 1 ? moe_permute_fwd_scatter(a->x, (int)a->x_dtype, a->row_to_pos, T, H, k, a->xp, stream)
-                   : moe_permute_fwd(a->x, (int)a->x_dtype, a->pos_to_row, R, H, k, a->xp, stream));
+    if (!in_place)
+      MOE_STEP(k > 1 ? "moe_permute_fwd_scatter" : "moe_permute_fwd",
+               k > 1 ? moe_permute_fwd_scatter(a->x, (int)a->x_dtype, a->row_to_pos, T, H, k, a->xp, stream)
+                     : moe_permute_fwd(a->x, (int)a->x_dtype, a->pos_to_row, R, H, k, a->xp, stream));
   }
-  if (a->gu)
+  if (in_place)
+    MOE_STEP(a->gu ? "moe_gemm_gateup_swiglu_fwd_blocked" : "moe_gemm_gateup_swiglu_fwd",
+             moe_gemm_gateup_from((const uint16_t*)a->x, a->pos_to_row, T, k, a->w1, a->w3, a->offs, E, H, I, a->gu, a->act, stream));
+  else if (a->gu)
     MOE_STEP("moe_gemm_gateup_swiglu_fwd_blocked",
              moe_gemm_gateup_swiglu_fwd_blocked(a->xp, a->w1, a->w3, a->offs, E, R, H, I, a->gu, a->act, stream));
   else
@@ -431,13 +447,16 @@ static int layer_forward(const moe_layer_forward_args* a, const MoeRouter* route
   return 0;
 }
 
-extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) { return layer_forward(a, nullptr, nullptr, stream); }
-
-int moe_selected_layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream) {
-  return layer_forward(a, router, table, stream);
+extern "C" int moe_layer_forward(const moe_layer_forward_args* a, void* stream) {
+  return layer_forward(a, nullptr, nullptr, false, stream);
 }
 
-extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream) {
+int moe_selected_layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream) {
+  return layer_forward(a, router, table, a && !a->xp, stream);
+}
+
+// (`in_place`: no xp, its rows are xn's)
+static int layer_backward(const moe_layer_backward_args* a, bool in_place, void* stream) {
   if (!a) return MOE_ERR_NULL;
   const int64_t T = a->T, H = a->H, E = a->E, I = a->I, k = a->k, R = T * k;
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
@@ -457,7 +476,7 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     MOE_CHECK_PTR(a->dout);
     MOE_CHECK_PTR(a->pos_to_row);
     MOE_CHECK_PTR(a->row_to_pos);
-    MOE_CHECK_PTR(a->xp);
+    MOE_CHECK_PTR(in_place ? a->xn : a->xp);
     MOE_CHECK_PTR(a->gu);
     MOE_CHECK_PTR(a->act);
     MOE_CHECK_PTR(a->w1);
@@ -466,6 +485,7 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     if ((to_logits || a->dgates) && (!a->gates || !a->ids)) return MOE_ERR_NULL;
     if (a->dwr && (!router || !a->xn)) return MOE_ERR_NULL;
   }
+  if (in_place && !moe_layer_rows_from_ok(T, H, E, I, k)) return MOE_ERR_LIMIT;
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
   const BwdScratch ws(s, T, H, E, I, k, a->dx && !a->dxp && !dx_in_place(*a));
   if (!s.fits()) return MOE_ERR_WORKSPACE;
@@ -502,12 +522,12 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
   if (to_logits && !with_dx && R > 0)
     MOE_STEP("moe_router_bwd_from_blocks", moe_router_bwd_from_blocks(part, moe_dgate_blocks(I), a->gates, a->ids, a->row_to_pos, T,
                                                                       E, k, ld, dlogits, dlogits_dtype, st));
-  const bool in_place = dx_in_place(*a);
+  const bool dx_stays = dx_in_place(*a);
   if (a->dx || a->dxp)
     MOE_STEP(pair ? "moe_gemm_dgrad_gateup_packed" : "moe_gemm_dgrad_gateup",
              moe_gemm_dgrad_gateup_to(dg, du, pair ? 2 * I : 0, a->w1, a->w3, a->offs, E, R, H, I,
-                                      in_place ? (uint16_t*)a->dx : dxp, in_place ? a->pos_to_row : nullptr, stream));
-  if (a->dx && T > 0 && !in_place) {  // (before the weight gradients: the router's reads dlogits)
+                                      dx_stays ? (uint16_t*)a->dx : dxp, dx_stays ? a->pos_to_row : nullptr, stream));
+  if (a->dx && T > 0 && !dx_stays) {  // (before the weight gradients: the router's reads dlogits)
     if (router && to_logits)
       MOE_STEP("moe_permute_bwd_router",
                moe_permute_bwd_router(dxp, a->row_to_pos, part, moe_dgate_blocks(I), a->gates, a->ids, a->wr, T, H, k, ld, dlogits,
@@ -525,7 +545,8 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
     if (!a->dw[w]) continue;
     MoeWgradStack& m = stacks[n_stacks++];
     m.a = w == 2 ? ws.dyp : w == 0 ? dg : du;
-    m.b = w == 2 ? a->act : a->xp;
+    m.b = w == 2 ? a->act : in_place ? a->xn : a->xp;
+    if (in_place && w != 2) m.row_from = a->pos_to_row, m.from_k = k, m.from_rows = T;
     m.M = w == 2 ? H : I;
     m.N = w == 2 ? I : H;
     m.lda = m.M, m.ldb = m.N;
@@ -564,3 +585,7 @@ extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream
   }
   return 0;
 }
+
+extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream) { return layer_backward(a, false, stream); }
+
+int moe_in_place_layer_backward(const moe_layer_backward_args* a, void* stream) { return layer_backward(a, true, stream); }

@@ -20,4 +20,8 @@ bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k);
 int moe_routed_forward(const MoeRouter& router, const uint16_t* x, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
                        int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out, int out_dtype, void* workspace,
                        int64_t workspace_bytes, void* stream);
+// Without xp the experts read x where it is (then in bf16), for sizes that moe_layer_rows_from_ok takes; the backward pass is then
+// moe_in_place_layer_backward, which has x as xn.
+bool moe_layer_rows_from_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k);
+int moe_in_place_layer_backward(const moe_layer_backward_args* a, void* stream);
 int moe_selected_layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream);

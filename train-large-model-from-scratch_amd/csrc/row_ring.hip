@@ -147,7 +147,7 @@ bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, int forced, hipSt
   if (a.E > MAX_E) return false;
   switch (mode) {
     case GATEUP:
-      if (blocked) return choose<GATEUP, true>(a, forced, s, rc);
+      if (blocked) return a.row_from ? choose<GATEUP, true, false, true>(a, forced, s, rc) : choose<GATEUP, true>(a, forced, s, rc);
       if (a.C0) return false;  // (g and u in rows: not here)
       return a.row_from ? choose<GATEUP, false, false, true>(a, forced, s, rc) : choose<GATEUP, false>(a, forced, s, rc);
     case DOWN: return a.row_map ? choose<DOWN, false, true>(a, forced, s, rc) : choose<DOWN, false>(a, forced, s, rc);

@@ -117,6 +117,15 @@ struct OpOuter {
     for (int i = 0; i < CH; ++i) voff[i] = ((kk + i * KSTEP) * ld + rc) * 2;
     lds_w = kk * LDN + rc;
   }
+  // Lines from anywhere: lane l has the byte offset of line own_line(l), of which the wave's lanes read CH * LPW.
+  static constexpr int LPW = MOE_WAVE / CPK;  // lines of a wave's chunk
+  static_assert(LPW > 0 && CH * LPW <= MOE_WAVE, "a lane a line");
+  static __device__ __forceinline__ int own_line(int wv, int lane) { return wv * LPW + lane % LPW + lane / LPW % CH * KSTEP; }
+  __device__ __forceinline__ void set_lines(uint32_t at) {
+    const uint32_t rc = threadIdx.x % CPK * 16;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) voff[i] = (int)(__shfl(at, lane_id() / CPK + i * LPW, MOE_WAVE) + rc);
+  }
   static __device__ __forceinline__ long long k_bytes(int k0, int ld) { return (long long)k0 * ld * 2; }
   __device__ __forceinline__ u32x4 load_one(int i, __amdgpu_buffer_rsrc_t rs) const {
     return __builtin_amdgcn_raw_buffer_load_b128(rs, voff[i], 0, 0);
