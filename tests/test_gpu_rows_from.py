@@ -54,3 +54,37 @@ def test_training_reads_the_tokens(pkg, T, H, E, I, k, skew, dtype):
     assert torch.equal(out, want)
     for i, (a, b) in enumerate(zip(grads, want_grads)):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), i
+
+
+@pytest.mark.parametrize("counts,H,I", [
+    ([160] * 64, 2048, 1024),                          # two and a half k-tiles each
+    ([0, 1, 63, 64, 65, 127, 128, 129, 900] * 8, 2040, 520),  # three problems; all numbers of k-tiles around one and two
+    ([40, 30] * 31 + [9000, 0], 2048, 1024),           # longest first
+    ([250, 0, 130, 400] * 12, 1536, 768),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_gradient_is_read_where_it_is(pkg, counts, H, I, dtype):
+    """In fp32 the output's gradient is rounded and put in order by a pass of its own."""
+    E, R = len(counts), sum(counts)
+    assert R >= 160 * E
+    g = torch.Generator(device="cuda").manual_seed(R)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    x, dy, ws = r(R, H), r(R, H), [w.to(dtype) for w in (r(E, I, H), r(E, I, H), r(E, H, I))]
+    ids = torch.arange(E, device="cuda").repeat_interleave(torch.tensor(counts, device="cuda"))
+    ids = ids[torch.randperm(R, generator=g, device="cuda")]
+    force = pkg.ops._lib.load().cdll.moe_gemm_force_row_tile
+
+    def passed(kind, height):
+        print("rows, gradient in place", E, R, H, I, dtype, kind, height, flush=True)
+        leaf, leaves = x.to(kind, copy=True).requires_grad_(True), [w.detach().requires_grad_(True) for w in ws]
+        try:
+            force(height)
+            pkg.experts_rows(leaf, ids, *leaves).backward(dy.to(kind))
+        finally:
+            force(0)
+        return [leaf.grad.bfloat16()] + [w.grad for w in leaves]
+
+    want = passed(torch.float32, 0)
+    for height in (0, 1, 64, 128, 256):
+        for i, (a, b) in enumerate(zip(passed(torch.bfloat16, height), want)):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (height, i)

@@ -57,6 +57,7 @@ constexpr int lds_bytes() {
 
 constexpr int GEMM_MAX_E = 1024;  // per-expert tile prefix lives in LDS
 constexpr int ROW_TILE = 256;     // rows of a tile of the row-ragged modes
+constexpr int FROM_A = 1, FROM_B = 2;
 
 // The expert of a row-tile slot, the last e with tile_start[e] <= slot (which skips those without rows), by a whole wave for a slot
 // that its lanes share: a count over the lanes and one trip to LDS for 128 experts, where a search takes seven, one after the
@@ -82,14 +83,14 @@ __device__ __forceinline__ int expert_of(const int* tile_start, int slot, int E)
 // The kernel's tile walk: the tiles at positions t_next, t_next + t_step, .. below t_hi of the launch's tile
 // list, or of `list` where one is given.  The rows of a row-ragged launch are numbered in tiles of UNIT rows; where
 // the configuration's are half as high, a list entry is 2 * tile + half.  (tile_start and, there, offs: in LDS.)
-// TO (DOWN and DGRAD_GATEUP only): the rows leave to where p.row_map says.  FROM (GATEUP: A's rows; WGRAD: B's lines): they
-// come from where p.row_from says.
-template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE, bool TO = false, bool FROM = false>
+// TO (DOWN and DGRAD_GATEUP only): the rows leave to where p.row_map says.  FROM (GATEUP and DGRAD_DOWN:
+// A's rows; WGRAD: A's lines, FROM_A, or B's, FROM_B): they come from where p.row_from says.
+template <int MODE, typename Cfg, typename OutT, bool BLK, int UNIT = ROW_TILE, bool TO = false, int FROM = 0>
 __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, const int* tile_start, const int* offs,
                                            const uint32_t* list, int t_next, const int t_hi, const int t_step) {
   static_assert(!BLK || MODE == GATEUP || MODE == DGRAD_DOWN, "only g and u have the blocked layout");
-  static_assert(!FROM || MODE == GATEUP || MODE == WGRAD, "only x is read where the caller has it");
-  constexpr bool ROWS_FROM = FROM && MODE == GATEUP, LINES_FROM = FROM && MODE == WGRAD;
+  static_assert(!FROM || MODE == GATEUP || MODE == DGRAD_DOWN || MODE == WGRAD, "only x and dy are read where the caller has them");
+  constexpr bool ROWS_FROM = FROM && MODE != WGRAD, LINES_FROM = FROM && MODE == WGRAD, A_LINES = LINES_FROM && FROM == FROM_A;
   static_assert(!TO || MODE == DOWN || MODE == DGRAD_GATEUP, "only y and dxp are rows that somebody else has a place for");
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT, KS = Cfg::KS;
   constexpr int FM = Cfg::FM, FN = Cfg::FN, WTM = Cfg::WTM, WTN = Cfg::WTN;
@@ -173,7 +174,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       if (p.K % 2048 == 0) t.kt0 = (t.e * 13) & 31;  // (32 k-tiles to 4 KB)
     }
     if constexpr (MODE == GATEUP) {
-      t.vA0 = FROM ? View{p.A0, p.from_bytes} : make_view(p.A0 + (long long)t.row0 * lda, rows * lda);
+      t.vA0 = ROWS_FROM ? View{p.A0, p.from_bytes} : make_view(p.A0 + (long long)t.row0 * lda, rows * lda);
       const long long wofs = ((long long)t.e * p.N + t.n0) * p.K;
       const long long wvalid = (long long)(p.N - t.n0) * p.K;
       t.vB0 = make_view(p.B0 + wofs, wvalid);
@@ -183,15 +184,15 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
       t.vB0 = make_view(p.B0 + ((long long)t.e * p.N + t.n0) * p.K, (long long)(p.N - t.n0) * p.K);
     } else if constexpr (MODE == DGRAD_DOWN || MODE == DGRAD_GATEUP) {
       // A = dy [R,K] (or dg|du [R,K]); B = W[e] as [K][N]
-      t.vA0 = make_view(p.A0 + (long long)t.row0 * lda, rows * lda);
+      t.vA0 = ROWS_FROM ? View{p.A0, p.from_bytes} : make_view(p.A0 + (long long)t.row0 * lda, rows * lda);
       t.vB0 = make_view(p.B0 + (long long)t.e * p.K * p.N + t.n0, (long long)p.K * p.N - t.n0);
       if constexpr (MODE == DGRAD_GATEUP) {
         t.vA1 = make_view(p.A1 + (long long)t.row0 * lda, rows * lda);
         t.vB1 = make_view(p.B1 + (long long)t.e * p.K * p.N + t.n0, (long long)p.K * p.N - t.n0);
       }
     } else {  // WGRAD: A = a [R,M] as [k][m]; B = b [R,N] as [k][n]; k = rows of expert e
-      t.vA0 = make_view(p.A0 + (long long)t.row0 * lda + t.m0, rows * lda - t.m0);
-      t.vB0 = LINES_FROM ? View{p.B0 + t.n0, p.from_bytes - t.n0 * 2}
+      t.vA0 = A_LINES ? View{p.A0 + t.m0, p.from_bytes - t.m0 * 2} : make_view(p.A0 + (long long)t.row0 * lda + t.m0, rows * lda - t.m0);
+      t.vB0 = LINES_FROM && !A_LINES ? View{p.B0 + t.n0, p.from_bytes - t.n0 * 2}
                          : make_view(p.B0 + (long long)t.row0 * ldb + t.n0, rows * ldb - t.n0);
     }
     return true;
@@ -222,17 +223,25 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   };
   // (WGRAD: the lines of a k-tile, asked for while the k-tile before is requested.  `lines_left`: how many of them the expert has.)
   int lines_left = 0;
+  const auto own_line = [&]() {
+    if constexpr (A_LINES) return StA::own_line(wv, lane);
+    else if constexpr (LINES_FROM) return StB::own_line(wv, lane);
+    else return 0;
+  };
   auto ask_lines = [&](int first, int end) {
     if constexpr (LINES_FROM) {
       lines_left = end - first;
       const __amdgpu_buffer_rsrc_t rs =
           __builtin_amdgcn_make_buffer_rsrc((void*)(p.row_from + first), 0, lines_left > 0 ? lines_left * 4 : 0, 0x00020000);
-      row_from = __builtin_amdgcn_raw_buffer_load_b32(rs, StB::own_line(wv, lane) * 4, 0, 0);
+      row_from = __builtin_amdgcn_raw_buffer_load_b32(rs, own_line() * 4, 0, 0);
     }
   };
   auto set_lines = [&]() {
-    if constexpr (LINES_FROM)
-      opB.set_lines(StB::own_line(wv, lane) < lines_left ? (uint32_t)p.by_k(row_from) * (uint32_t)(ldb * 2) : NO_ROW);
+    if constexpr (LINES_FROM) {
+      const uint32_t at = own_line() < lines_left ? (uint32_t)p.by_k(row_from) * (uint32_t)((A_LINES ? lda : ldb) * 2) : NO_ROW;
+      if constexpr (A_LINES) opA.set_lines(at);
+      else opB.set_lines(at);
+    }
   };
   // One set of registers carries a k-tile from HBM to LDS: it is requested one iteration
   // before it is written to LDS, which is what hides the latency of a load that misses L2.
@@ -259,9 +268,9 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
   auto operand_src = [&](const Tile& t, int kt, int op) {
     const int k0 = k_of(t, kt);
     const bool second = NSEG == 2 && kt >= t.kt_per_seg;
-    if (op == 0) return window(second ? t.vA1 : t.vA0, StA::k_bytes(k0, lda));
+    if (op == 0) return window(second ? t.vA1 : t.vA0, A_LINES ? 0 : StA::k_bytes(k0, lda));
     if constexpr (DUAL) return window(op == 1 ? t.vB0 : t.vB1, StBh::k_bytes(k0, ldb));
-    else return window(second ? t.vB1 : t.vB0, LINES_FROM ? 0 : StB::k_bytes(k0, ldb));
+    else return window(second ? t.vB1 : t.vB0, LINES_FROM && !A_LINES ? 0 : StB::k_bytes(k0, ldb));
   };
   auto tile_src = [&](const Tile& t, int kt) {
     TileSrc ts;
@@ -903,8 +912,12 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
     // goes out as soon as that room is free: during the last of its strips.
     bool requested = EARLY_REQUEST;
     auto request_next = [&]() {
-      if (!stream) request_first(nxt);
-      else request_k(nxt, 1);
+      if (!stream) {
+        set_rows();
+        request_first(nxt);
+      } else {
+        request_k(nxt, 1);
+      }
     };
     auto late_request = [&]() {
       if constexpr (!EARLY_REQUEST) {
@@ -1123,7 +1136,7 @@ struct WgradArgs {
 // faster dealt in groups than with contiguous ranges of equal work, another 9-10 % longest
 // first; near-uniform routing: the same in all three.)  A tile of an expert costs the same in every problem: the next one's
 // groups are dealt on from where the last one's left the XCDs.
-template <typename OutT, bool FROM>
+template <typename OutT, int FROM>
 __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_gemm_kernel(const WgradArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   const int lane = threadIdx.x & 63;
@@ -1214,8 +1227,10 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_ge
       first = lo + j, end = lo + q + (x < r ? 1 : 0), step = (nb >> 3) + (x < (nb & 7) ? 1 : 0);
     }
     if (w) __syncthreads();  // (the operand stages are free)
-    if (FROM && p.row_from)
-      walk_tiles<WGRAD, CfgMain, OutT, false, ROW_TILE, false, FROM>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
+    if ((FROM & FROM_A) && p.row_from && p.from_a)
+      walk_tiles<WGRAD, CfgMain, OutT, false, ROW_TILE, false, FROM_A>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
+    else if ((FROM & FROM_B) && p.row_from)
+      walk_tiles<WGRAD, CfgMain, OutT, false, ROW_TILE, false, FROM_B>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
     else walk_tiles<WGRAD, CfgMain, OutT, false>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
     done += total;
   }
@@ -1310,10 +1325,14 @@ int launch_wgrad(const WgradArgs& args, hipStream_t s) {
     const long long n = (long long)a.n_tiles * a.m_slots * a.E;
     tiles = tiles > n ? tiles : n;
   }
-  static bool attr_done[2][MOE_MAX_DEVICES];
+  static bool attr_done[4][MOE_MAX_DEVICES];
+  int from = 0;
   for (int i = 0; i < w.n; ++i)
-    if (w.p[i].row_from) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, true>, attr_done[1], w, tiles, s);
-  return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, false>, attr_done[0], w, tiles, s);
+    if (w.p[i].row_from) from |= w.p[i].from_a ? FROM_A : FROM_B;
+  if (from == FROM_A) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, FROM_A>, attr_done[1], w, tiles, s);
+  if (from == FROM_B) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, FROM_B>, attr_done[2], w, tiles, s);
+  if (from) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, FROM_A | FROM_B>, attr_done[3], w, tiles, s);
+  return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, 0>, attr_done[0], w, tiles, s);
 }
 
 int check_common(const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I) {
@@ -1451,11 +1470,10 @@ extern "C" int moe_gemm_dgrad_down_swiglu_bwd_dgate(const uint16_t* dyp, const u
   return dgrad_down_impl(dyp, w2, g, u, offs, E, R, H, I, dg, du, dgate_part, stream);
 }
 
-extern "C" int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const uint16_t* w2,
-                                                      const void* gu_blocked, const int32_t* offs, int64_t E,
-                                                      int64_t R, int64_t H, int64_t I, uint16_t* dg,
-                                                      uint16_t* du, int64_t ld_out, float* dgate_part,
-                                                      void* stream) {
+// dyp: row p is row p of it, or with pos_to_row row pos_to_row[p] / k of its `from_rows`
+static int dgrad_down_blocked(const uint16_t* dyp, const int32_t* pos_to_row, int64_t from_rows, int64_t k, const uint16_t* w2,
+                              const void* gu_blocked, const int32_t* offs, int64_t E, int64_t R, int64_t H, int64_t I, uint16_t* dg,
+                              uint16_t* du, int64_t ld_out, float* dgate_part, void* stream) {
   if (int rc = check_common(offs, E, R, H, I)) return rc;
   if (R == 0) return 0;
   MOE_CHECK_PTR(dyp); MOE_CHECK_PTR(w2); MOE_CHECK_PTR(gu_blocked); MOE_CHECK_PTR(dg); MOE_CHECK_PTR(du);
@@ -1464,7 +1482,25 @@ extern "C" int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const
   a.C2 = dgate_part;
   a.A0 = dyp; a.B0 = w2; a.X0 = (const uint16_t*)gu_blocked; a.C0 = dg; a.C1 = du; a.offs = offs;
   a.E = (int)E; a.R = (int)R; a.N = (int)I; a.K = (int)H; a.ld_c = (int)ld_out;
-  return launch_rows<DGRAD_DOWN, true>(a, CfgMain::BN, (hipStream_t)stream);
+  if (!pos_to_row) return launch_rows<DGRAD_DOWN, true>(a, CfgMain::BN, (hipStream_t)stream);
+  if (!moe_rows_from_ok(from_rows, H)) return MOE_ERR_LIMIT;
+  a.row_from = pos_to_row; a.by_k.set((uint32_t)k); a.from_bytes = from_rows * H * 2;
+  return launch_rows<DGRAD_DOWN, true, false, true>(a, CfgMain::BN, (hipStream_t)stream);
+}
+
+extern "C" int moe_gemm_dgrad_down_swiglu_bwd_blocked(const uint16_t* dyp, const uint16_t* w2,
+                                                      const void* gu_blocked, const int32_t* offs, int64_t E,
+                                                      int64_t R, int64_t H, int64_t I, uint16_t* dg,
+                                                      uint16_t* du, int64_t ld_out, float* dgate_part,
+                                                      void* stream) {
+  return dgrad_down_blocked(dyp, nullptr, R, 1, w2, gu_blocked, offs, E, R, H, I, dg, du, ld_out, dgate_part, stream);
+}
+
+int moe_gemm_dgrad_down_from(const uint16_t* dy, const int32_t* pos_to_row, int64_t T, int64_t k, const uint16_t* w2,
+                             const void* gu_blocked, const int32_t* offs, int64_t E, int64_t H, int64_t I, uint16_t* dg, uint16_t* du,
+                             int64_t ld_out, float* dgate_part, void* stream) {
+  if (!pos_to_row) return MOE_ERR_NULL;
+  return dgrad_down_blocked(dy, pos_to_row, T, k, w2, gu_blocked, offs, E, T * k, H, I, dg, du, ld_out, dgate_part, stream);
 }
 
 // The two row gradients side by side in one buffer: dgu [R, 2I], row = [dg row | du row].  The
@@ -1548,8 +1584,10 @@ int moe_gemm_wgrad_all(const MoeWgradStack* stacks, int n, const int32_t* offs, 
                           : wgrad_args(w.p[w.n], m.a, m.b, offs, E, R, m.M, m.N, m.out, m.dtype, m.accumulate);
     if (rc) return rc;
     if (m.row_from) {
-      if (!moe_rows_from_ok(m.from_rows, m.N)) return MOE_ERR_LIMIT;
-      w.p[w.n].row_from = m.row_from, w.p[w.n].by_k.set((uint32_t)m.from_k), w.p[w.n].from_bytes = m.from_rows * m.N * 2;
+      const int64_t wide = m.from_a ? m.M : m.N;
+      if (!moe_rows_from_ok(m.from_rows, wide) || (m.from_a && m.out2)) return MOE_ERR_LIMIT;
+      w.p[w.n].row_from = m.row_from, w.p[w.n].by_k.set((uint32_t)m.from_k), w.p[w.n].from_bytes = m.from_rows * wide * 2;
+      w.p[w.n].from_a = m.from_a;
     }
   }
   return run_wgrad(w, stacks[0].dtype, stream);

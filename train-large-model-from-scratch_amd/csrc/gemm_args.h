@@ -42,7 +42,9 @@ struct GemmArgs {
   int m_split;  // WGRAD: rows m >= m_split of an expert's result go to C1 (as its rows m - m_split); 0: all to C0
   int whole_only;  // row-ragged modes: no half tiles (test hook)
   const int32_t* row_map;  // row-ragged modes, DOWN and DGRAD_GATEUP: where a row of the result goes (NULL: rows stay in order)
-  const int32_t* row_from;  // GATEUP: row r of A0, WGRAD: of B0, is row by_k(row_from[r]) of it, which has from_bytes bytes (NULL: row r)
+  // GATEUP and DGRAD_DOWN: row r of A0, WGRAD: of A0 or B0, is row by_k(row_from[r]) of it, which has from_bytes bytes (NULL: row r)
+  const int32_t* row_from;
+  bool from_a;
   Divisor by_k;
   long long from_bytes;  // < 2^31
   int streaming;   // WGRAD: results that replace what is there leave with streaming stores; GATEUP: act does

@@ -49,8 +49,10 @@ struct MoeWgradStack {
   int64_t lda, ldb, M, N;
   int dtype, accumulate;
   void* out2;  // moe_gemm_wgrad_all: an expert's rows M / 2 .. M - 1 go here (NULL: all to out)
-  const int32_t* row_from;  // moe_gemm_wgrad_all: row r of b is row row_from[r] / from_k of its from_rows (NULL: row r)
+  // moe_gemm_wgrad_all: row r of b, or with from_a of a, is row row_from[r] / from_k of its from_rows (NULL: row r)
+  const int32_t* row_from;
   int64_t from_k, from_rows;
+  bool from_a;
 };
 // Weight gradients leave with streaming stores from so many bytes of results in a launch on, an eighth of the memory-side cache: a
 // model of a few such layers finds smaller ones there when it adds them up, clips them or steps.  Pass, pass with its gradients added
@@ -112,6 +114,10 @@ int moe_gemm_dgrad_gateup_to(const uint16_t* dg, const uint16_t* du, int64_t ld_
 bool moe_rows_from_ok(int64_t T, int64_t H);
 int moe_gemm_gateup_from(const uint16_t* x, const int32_t* pos_to_row, int64_t T, int64_t k, const uint16_t* w1, const uint16_t* w3,
                          const int32_t* offs, int64_t E, int64_t H, int64_t I, void* gu_blocked, uint16_t* act, void* stream);
+// moe_gemm_dgrad_down_swiglu_bwd_blocked whose row p of dyp is dy[pos_to_row[p] / k], for dy [T,H] of sizes that moe_rows_from_ok takes.
+int moe_gemm_dgrad_down_from(const uint16_t* dy, const int32_t* pos_to_row, int64_t T, int64_t k, const uint16_t* w2,
+                             const void* gu_blocked, const int32_t* offs, int64_t E, int64_t H, int64_t I, uint16_t* dg, uint16_t* du,
+                             int64_t ld_out, float* dgate_part, void* stream);
 // ---- few tokens (few.hip) ----
 constexpr int FEW_MAX_TOKENS = 64;
 constexpr int FEW_MAX_EXPERTS = 128;

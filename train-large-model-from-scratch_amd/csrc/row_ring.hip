@@ -151,7 +151,9 @@ bool moe_ring_rows(Mode mode, bool blocked, const GemmArgs& a, int forced, hipSt
       if (a.C0) return false;  // (g and u in rows: not here)
       return a.row_from ? choose<GATEUP, false, false, true>(a, forced, s, rc) : choose<GATEUP, false>(a, forced, s, rc);
     case DOWN: return a.row_map ? choose<DOWN, false, true>(a, forced, s, rc) : choose<DOWN, false>(a, forced, s, rc);
-    case DGRAD_DOWN: return blocked && choose<DGRAD_DOWN, true>(a, forced, s, rc);
+    case DGRAD_DOWN:
+      if (!blocked) return false;
+      return a.row_from ? choose<DGRAD_DOWN, true, false, true>(a, forced, s, rc) : choose<DGRAD_DOWN, true>(a, forced, s, rc);
     default: return a.row_map ? choose<DGRAD_GATEUP, false, true>(a, forced, s, rc) : choose<DGRAD_GATEUP, false>(a, forced, s, rc);
   }
 }
