@@ -282,3 +282,53 @@ def test_norm_router_unsupported_shapes_fall_back(pkg, lib):
                                torch.zeros(16, 72, dtype=torch.bfloat16, device="cuda"), 2)
     # prenorm_moe on such a shape takes the separate kernels and still matches (covered by
     # test_prenorm_moe_odd_shapes: H = 72 and 520, E = 3 and 6)
+
+
+@pytest.mark.parametrize("T,H,E,I,k,x_dt", [
+    (1, 256, 16, 64, 1, torch.float32),          # one row, one wave of columns
+    (37, 2048, 16, 64, 3, torch.float32),
+    (1100, 768, 64, 128, 6, torch.float32),      # more rows than partial sums
+    (300, 1024, 32, 64, 8, torch.bfloat16),      # the gradient in between is rounded
+    (129, 2080, 16, 64, 5, torch.bfloat16),      # columns that end in a wave's second piece
+    (65, 4104, 8, 64, 2, torch.float32),         # four pieces a thread
+    (700, 1400, 48, 600, 4, torch.float32),
+])
+@pytest.mark.parametrize("add_residual", [True, False])
+def test_rows_summed_in_the_norms_backward(pkg, T, H, E, I, k, x_dt, add_residual):
+    """The k-row sum with the router's share and the norm's backward in one pass hold the bits of the two."""
+    ops = pkg.ops
+    _say("rows in the norm's backward", T, H, E, I, k, x_dt, add_residual)
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, dout, nw = (r(T, H) * 1.5).to(x_dt).requires_grad_(True), r(T, H).to(x_dt), (1 + 0.2 * r(H)).requires_grad_(True)
+    wr = (r(E, H) * 0.02).bfloat16().requires_grad_(True)
+    ws = [(r(*s) * 0.05).bfloat16() for s in ((E, I, H), (E, I, H), (E, H, I))]
+    names = []
+
+    class Obs:
+        def before(self, name):
+            names.append(name)
+
+        def after(self, name):
+            pass
+
+    L = ops._lib.load()
+    out, logits = pkg.functional.prenorm_moe(x, nw, wr, *ws, k, eps=EPS, add_residual=add_residual)
+    L.observer = Obs()
+    try:
+        out.backward(dout)
+    finally:
+        L.observer = None
+    assert "moe_rmsnorm_bwd_rows" in names and "moe_rmsnorm_bwd" not in names
+    xd, logits = x.detach(), logits.detach()
+    if ops.rmsnorm_router_supported(H, E, k):
+        xn, rstd = ops.rmsnorm_router_fwd(xd, nw.detach(), EPS, wr.detach(), k)[:2]
+    else:
+        xn, rstd = ops.rmsnorm_fwd(xd, nw.detach(), EPS)
+    _, rt, xp, gu, act = ops.layer_forward(xn, logits, *ws, k, train=True)
+    d1, dwr = torch.empty_like(xd), torch.empty_like(wr)
+    ops.layer_backward(dout, k, rt.gates, rt.ids, rt.offs, rt.pos_to_row, rt.row_to_pos, xp, gu, act, *ws, (None, None, None),
+                       wr=wr.detach(), xn=xn, dwr=dwr, dx=d1)
+    dx, dnw = ops.rmsnorm_bwd(xd, nw.detach(), rstd, d1, None, dout if add_residual else None)
+    for name, got, want in (("dx", x.grad, dx), ("dnw", nw.grad, dnw), ("dwr", wr.grad, dwr)):
+        assert torch.equal(got, want), name

@@ -528,7 +528,18 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
     const int64_t bytes = std::max<int64_t>(moe_backward_scratch(&a), 256);
     const Tensor scratch = empty({bytes}, at::kByte, kept_buf);
     a.scratch = scratch.data_ptr(), a.scratch_bytes = bytes;
-    check(in_place ? moe_in_place_layer_backward(&a, s) : moe_layer_backward(&a, s), "moe_layer_backward");
+    // (the norm's backward in the pass that adds the rows up)
+    const bool norm_inside = has_norm && has_router && want_dx && !by_hand && moe_norm_rows_ok(T, H);
+    if (norm_inside) {
+      const int64_t nb = std::max<int64_t>(moe_rmsnorm_bwd_workspace_bytes(T, H), 16);
+      const Tensor ws = empty({nb}, at::kByte, kept_buf);
+      dnw = empty({H}, at::kFloat, kept_buf);
+      const MoeNormBackward norm{x.data_ptr(), (int)dt(x), nw.data_ptr<float>(), rstd.data_ptr<float>(),
+                                 add_residual ? dout.data_ptr() : nullptr, dnw.data_ptr<float>(), ws.data_ptr(), nb};
+      check(moe_norm_layer_backward(&a, norm, s), "moe_layer_backward");
+    } else {
+      check(in_place ? moe_in_place_layer_backward(&a, s) : moe_layer_backward(&a, s), "moe_layer_backward");
+    }
     for (int i = 0; i < 3; ++i)
       if (wg.fresh[i].defined()) params[i].mutable_grad() = wg.fresh[i];
     if (dwr.defined() && !wr_direct) dwr = dwr.to(type(6));
@@ -567,7 +578,9 @@ struct LayerNode : torch::autograd::Function<LayerNode> {
       }
       if (!want_logits) dlogits = Tensor();
     }
-    if (want_dx && has_norm) {
+    if (norm_inside) {
+      dnw = need(NORM) ? dnw.to(type(5)) : Tensor();
+    } else if (want_dx && has_norm) {
       const int64_t nb = std::max<int64_t>(moe_rmsnorm_bwd_workspace_bytes(T, H), 16);
       const Tensor ws = empty({nb}, at::kByte, kept_buf);
       const Tensor d1 = dx;

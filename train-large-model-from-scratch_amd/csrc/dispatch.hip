@@ -15,6 +15,7 @@
 
 #include "common.h"
 #include "internal.h"
+#include "row_sum.h"
 
 namespace {
 
@@ -364,15 +365,6 @@ __global__ __launch_bounds__(256) void permute_fwd_scatter_kernel(const XT* __re
 // gates and ids are the same for all of its lanes and come as scalars, eight at a time, and the rows of y and of wr
 // are on their way together.  (A lane a piece of any of four tokens, wr after y: 8192 tokens, k = 2, 1024 wide,
 // both directions 31.2 -> 23.2 us; 3333 tokens, k = 3, 1416 wide 32.4 -> 21.2; 16384 tokens, k = 8, 2048 wide 250 -> 227.)
-struct RouterGrad {
-  const float* part;   // [P][T*k], by position
-  int P;
-  const float* gates;
-  const int32_t* ids;
-  const uint16_t* wr;  // [E, H]
-  void* dlogits;       // [T, ld]
-  int ld;
-};
 template <typename OT, typename AT, typename LT, bool IN_ORDER>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __restrict__ y,
                                                          const float* __restrict__ gates,
@@ -386,80 +378,10 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(const uint16_t* __rest
     const int r0 = t * k;
     int id = -1;       // of slot `lane`
     float dsel = 0.f;
-    if constexpr (ROUTER) {
-      const int lane = lane_id();
-      float s = 0.f, g = 0.f;
-      if (lane < k) {
-        const float* src = rg.part + row_to_pos[r0 + lane];
-        id = rg.ids[r0 + lane];
-        g = rg.gates[r0 + lane];
-        const size_t R = (size_t)T * k;
-        int b = 0;
-        for (; b + 8 <= rg.P; b += 8) {  // (eight gathers in flight, added in ascending order)
-          float v[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) v[i] = src[(size_t)(b + i) * R];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) s += v[i];
-        }
-        for (; b + 4 <= rg.P; b += 4) {
-          const float v0 = src[(size_t)b * R], v1 = src[(size_t)(b + 1) * R], v2 = src[(size_t)(b + 2) * R],
-                      v3 = src[(size_t)(b + 3) * R];
-          s = (((s + v0) + v1) + v2) + v3;
-        }
-        for (; b < rg.P; ++b) s += src[(size_t)b * R];
-      }
-      const float dg = g != 0.f ? s / g : 0.f;
-      float dot = 0.f;
-      for (int j = 0; j < k; ++j) dot += read_lane_f(g, j) * read_lane_f(dg, j);
-      dsel = g * (dg - dot);
-      if constexpr (ROUTER && sizeof(LT) == 2) dsel = bf16_to_f32(f32_to_bf16(dsel));
-      for (int e = lane; e < rg.ld; e += MOE_WAVE) {
-        float v = 0.f;
-        for (int j = 0; j < k; ++j) v = read_lane(id, j) == e ? read_lane_f(dsel, j) : v;
-        if constexpr (ROUTER && sizeof(LT) == 2) ((uint16_t*)rg.dlogits)[(size_t)t * rg.ld + e] = f32_to_bf16(v);
-        else ((float*)rg.dlogits)[(size_t)t * rg.ld + e] = v;
-      }
-    }
+    if constexpr (ROUTER) dsel = router_dsel<LT>(rg, row_to_pos, T, k, t, true, id);
     for (int col = lane_id() * 8; col < H; col += MOE_WAVE * 8) {
       Row8 acc, d2;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc.v[i] = 0.f, d2.v[i] = 0.f;
-      // the next N rows, all in flight; summed in slot order
-      const auto add = [&](int j, auto n) {
-        constexpr int N = decltype(n)::value;
-        u32x4 v[N], w[ROUTER ? N : 1];
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
-          const int pos = IN_ORDER ? r0 + j + q : row_to_pos[r0 + j + q];
-          v[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(y + (size_t)pos * H + col));
-        }
-        if constexpr (ROUTER) {
-#pragma unroll
-          for (int q = 0; q < N; ++q) w[q] = *reinterpret_cast<const u32x4*>(rg.wr + (size_t)read_lane(id, j + q) * H + col);
-        }
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
-          const float gt = gates ? gates[r0 + j + q] : 1.f;
-          const Row8 row = row8_from_bits(v[q]);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc.v[i] += gt * row.v[i];
-        }
-        if constexpr (ROUTER) {
-#pragma unroll
-          for (int q = 0; q < N; ++q) {
-            const float ds = read_lane_f(dsel, j + q);
-            const Row8 row = row8_from_bits(w[q]);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) d2.v[i] += ds * row.v[i];
-          }
-        }
-      };
-      int j = 0;
-      for (; j + 8 <= k; j += 8) add(j, std::integral_constant<int, 8>{});
-      if (j + 4 <= k) add(j, std::integral_constant<int, 4>{}), j += 4;
-      if (j + 2 <= k) add(j, std::integral_constant<int, 2>{}), j += 2;
-      if (j < k) add(j, std::integral_constant<int, 1>{});
+      sum_rows<ROUTER, IN_ORDER>(y, gates, row_to_pos, rg, id, dsel, r0, k, H, col, acc, d2);
       if (addend) {
         const Row8 a = load8(addend + (size_t)t * H + col);
 #pragma unroll

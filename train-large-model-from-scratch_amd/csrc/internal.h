@@ -29,6 +29,11 @@ int moe_permute_bwd_router(const uint16_t* dxp, const int32_t* row_to_pos, const
                            const int32_t* ids, const uint16_t* wr, int64_t T, int64_t H, int64_t k, int64_t ld, void* dlogits,
                            int dlogits_dtype, void* dx, int dx_dtype, hipStream_t s);
 
+// moe_permute_bwd_router and moe_rmsnorm_bwd in one pass, without what one hands on to the other (norm.hip).
+int moe_rmsnorm_bwd_rows(const MoeNormBackward& n, const uint16_t* dxp, const int32_t* row_to_pos, const float* part, int64_t P,
+                         const float* gates, const int32_t* ids, const uint16_t* wr, int64_t T, int64_t H, int64_t k, int64_t ld,
+                         uint16_t* dlogits, void* dx, hipStream_t s);
+
 // Bytes of scratch that a call with these arguments (all but the scratch filled in) uses, no more than moe_layer_scratch_bytes says:
 // rows that stay in place need no buffer for them (layer.hip).
 int64_t moe_forward_scratch(const moe_layer_forward_args* a);

@@ -463,8 +463,8 @@ int moe_selected_layer_forward(const moe_layer_forward_args* a, const MoeRouter*
   return layer_forward(a, router, table, a && !a->xp, stream);
 }
 
-// (`in_place`: no xp, its rows are xn's)
-static int layer_backward(const moe_layer_backward_args* a, bool in_place, void* stream) {
+// (`in_place`: no xp, its rows are xn's; `norm`: see router.h)
+static int layer_backward(const moe_layer_backward_args* a, bool in_place, const MoeNormBackward* norm, void* stream) {
   if (!a) return MOE_ERR_NULL;
   const int64_t T = a->T, H = a->H, E = a->E, I = a->I, k = a->k, R = T * k;
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
@@ -494,6 +494,7 @@ static int layer_backward(const moe_layer_backward_args* a, bool in_place, void*
     if (a->dwr && (!router || !a->xn)) return MOE_ERR_NULL;
   }
   if (in_place && !moe_layer_rows_from_ok(T, H, E, I, k)) return MOE_ERR_LIMIT;
+  if (norm && (!router || !to_logits || !a->dx || a->dxp || a->dlogits || !moe_norm_rows_ok(T, H))) return MOE_ERR_SHAPE;
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
   const bool dout_stays = dout_in_place(*a);
   const BwdScratch ws(s, T, H, E, I, k, a->dx && !a->dxp && !dx_in_place(*a), !dout_stays);
@@ -540,7 +541,11 @@ static int layer_backward(const moe_layer_backward_args* a, bool in_place, void*
              moe_gemm_dgrad_gateup_to(dg, du, pair ? 2 * I : 0, a->w1, a->w3, a->offs, E, R, H, I,
                                       dx_stays ? (uint16_t*)a->dx : dxp, dx_stays ? a->pos_to_row : nullptr, stream));
   if (a->dx && T > 0 && !dx_stays) {  // (before the weight gradients: the router's reads dlogits)
-    if (router && to_logits)
+    if (norm)
+      MOE_STEP("moe_rmsnorm_bwd_rows",
+               moe_rmsnorm_bwd_rows(*norm, dxp, a->row_to_pos, part, moe_dgate_blocks(I), a->gates, a->ids, a->wr, T, H, k, ld,
+                                    ws.dlogits, a->dx, st));
+    else if (router && to_logits)
       MOE_STEP("moe_permute_bwd_router",
                moe_permute_bwd_router(dxp, a->row_to_pos, part, moe_dgate_blocks(I), a->gates, a->ids, a->wr, T, H, k, ld, dlogits,
                                       dlogits_dtype, a->dx, (int)a->dx_dtype, st));
@@ -599,6 +604,12 @@ static int layer_backward(const moe_layer_backward_args* a, bool in_place, void*
   return 0;
 }
 
-extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream) { return layer_backward(a, false, stream); }
+extern "C" int moe_layer_backward(const moe_layer_backward_args* a, void* stream) { return layer_backward(a, false, nullptr, stream); }
 
-int moe_in_place_layer_backward(const moe_layer_backward_args* a, void* stream) { return layer_backward(a, true, stream); }
+int moe_in_place_layer_backward(const moe_layer_backward_args* a, void* stream) {
+  return layer_backward(a, true, nullptr, stream);
+}
+
+int moe_norm_layer_backward(const moe_layer_backward_args* a, const MoeNormBackward& norm, void* stream) {
+  return layer_backward(a, a && !a->xp, &norm, stream);
+}

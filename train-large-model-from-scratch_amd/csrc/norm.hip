@@ -14,6 +14,7 @@
 #include "common.h"
 #include "internal.h"
 #include "topk_core.h"
+#include "row_sum.h"
 
 namespace {
 
@@ -352,6 +353,78 @@ __global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(
   }
 }
 
+// rmsnorm_bwd_kernel with d1 = what moe_permute_bwd_router makes of the rows of dxp, in x's type, in the arithmetic of both.
+// Two passes write d1 and read it, a launch apart.  Whole steps, fp32 x, us, two passes -> this, the same bits: 8192 tokens, 8 of 64 experts, 2048
+// wide, 2877 -> 2855; 2 of 16 639 -> 611; 12000, 1 of 8, 1024 wide, 288 -> 273; 3000, 8 of 24, 4096 wide, 893 -> 852; 700, 4 of 48, 1400 wide, 355 ->
+// 354; 64, 2 of 16, 1024 wide, 165 -> 159.  A block a token, as the norm's mean has it (the rows by themselves have a wave a token): narrow
+// rows leave its waves without columns, which is less than the launch only while tokens are few: 640 wide, 3000 / 16000 tokens 199 -> 194, 532 ->
+// 534; 512 wide, 2000 / 8000 170 -> 167, 407 -> 417; 256 wide, 4000 / 16000 200 -> 197, 255 -> 262; 768 wide, 16000 444 -> 439.
+template <typename XT, int NV>
+__global__ __launch_bounds__(NT, NV == 1 ? 4 : 2) void rmsnorm_bwd_rows_kernel(
+    const XT* __restrict__ x, const float* __restrict__ w, const float* __restrict__ rstd, const uint16_t* __restrict__ dxp,
+    const int32_t* __restrict__ row_to_pos, const RouterGrad rg, const XT* __restrict__ dres, int T, int H8, int k,
+    XT* __restrict__ dx, float* __restrict__ part) {
+  __shared__ float red[NW];
+  const int H = H8 * 8;
+  const bool first_wave = uniform((int)(threadIdx.x / MOE_WAVE)) == 0;
+  Row8 wv[NV], dwv[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = threadIdx.x + i * NT;
+    if (c < H8) wv[i] = load8(w + c * 8);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) dwv[i].v[j] = 0.f;
+  }
+  for (int t = blockIdx.x; t < T; t += gridDim.x) {
+    const float r = rstd[t];
+    int id;
+    const float dsel = router_dsel<uint16_t>(rg, row_to_pos, T, k, t, first_wave, id);
+    Row8 xh[NV], gw[NV];
+    float dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + i * NT;
+      if (c < H8) {
+        xh[i] = load8(x + (size_t)t * H + c * 8);
+        Row8 g, d2;
+        sum_rows<true, false>(dxp, nullptr, row_to_pos, rg, id, dsel, t * k, k, H, c * 8, g, d2);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          g.v[j] += bf16_to_f32(f32_to_bf16(d2.v[j]));
+          if (sizeof(XT) == 2) g.v[j] = bf16_to_f32(f32_to_bf16(g.v[j]));
+          xh[i].v[j] *= r;
+          dwv[i].v[j] += g.v[j] * xh[i].v[j];
+          gw[i].v[j] = g.v[j] * wv[i].v[j];
+          dot += gw[i].v[j] * xh[i].v[j];
+        }
+      }
+    }
+    dot = block_sum(dot, red);
+    const float m = dot / (float)H;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + i * NT;
+      if (c < H8) {
+        const size_t at = (size_t)t * H + c * 8;
+        Row8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o.v[j] = r * (gw[i].v[j] - xh[i].v[j] * m);
+        if (dres) {
+          const Row8 a = load8(dres + at);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) o.v[j] += a.v[j];
+        }
+        store8(dx + at, o);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = threadIdx.x + i * NT;
+    if (c < H8) store8(part + (size_t)blockIdx.x * H + c * 8, dwv[i]);
+  }
+}
+
 // dw[c] = sum_b part[b][c], b ascending within each of CG row groups, groups combined in ascending order:
 // one fixed order whatever the launch.  A block owns 64 columns, a wave a group of rows: the launch has
 // few blocks (32 at H = 2048), so what bounds it is the length of a wave's chain of loads; with 16 groups
@@ -550,5 +623,40 @@ extern "C" int moe_rmsnorm_bwd(const void* x, int x_dtype, const float* weight, 
   if (rc) return rc;
   hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + MOE_WAVE - 1) / MOE_WAVE)), dim3(CG * MOE_WAVE), 0, s,
                      (const float*)part, bwd_blocks(T), (int)H, dweight);
+  return moe_launch_status();
+}
+
+bool moe_norm_rows_ok(int64_t T, int64_t H) {
+  return T > 0 && T <= (int64_t)1 << 30 && H % 8 == 0 && pick_nv(H) != 0 && (H >= 768 || T <= 4096);
+}
+
+int moe_rmsnorm_bwd_rows(const MoeNormBackward& n, const uint16_t* dxp, const int32_t* row_to_pos, const float* part, int64_t P,
+                         const float* gates, const int32_t* ids, const uint16_t* wr, int64_t T, int64_t H, int64_t k, int64_t ld,
+                         uint16_t* dlogits, void* dx, hipStream_t s) {
+  if (int rc = check_norm(T, H)) return rc;
+  if (T == 0) return MOE_ERR_SHAPE;
+  for (const void* q : {n.x, (const void*)n.weight, (const void*)n.dweight, (const void*)n.workspace, (const void*)dxp, (const void*)wr,
+                        (const void*)dx})
+    MOE_CHECK_PTR(q);
+  if (!n.rstd || !part || !gates || !ids || !dlogits || !row_to_pos) return MOE_ERR_NULL;
+  if (!aligned16(n.dres)) return MOE_ERR_ALIGN;
+  if (n.workspace_bytes < moe_rmsnorm_bwd_workspace_bytes(T, H)) return MOE_ERR_WORKSPACE;
+  const RouterGrad rg{part, (int)P, gates, ids, wr, dlogits, (int)ld};
+  const auto go = [&](auto xt, auto nv) {
+    using XT = decltype(xt);
+    hipLaunchKernelGGL((rmsnorm_bwd_rows_kernel<XT, decltype(nv)::value>), dim3((unsigned)bwd_blocks(T)), dim3(NT), 0, s,
+                       (const XT*)n.x, n.weight, n.rstd, dxp, row_to_pos, rg, (const XT*)n.dres, (int)T, (int)(H / 8), (int)k, (XT*)dx,
+                       (float*)n.workspace);
+    return moe_launch_status();
+  };
+  const auto of = [&](auto xt) {
+    const int nv = pick_nv(H);
+    return nv == 1 ? go(xt, std::integral_constant<int, 1>{}) : nv == 2 ? go(xt, std::integral_constant<int, 2>{})
+                                                                       : go(xt, std::integral_constant<int, 4>{});
+  };
+  if (n.x_dtype != MOE_DT_BF16 && n.x_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
+  if (const int rc = n.x_dtype == MOE_DT_BF16 ? of(uint16_t{}) : of(float{})) return rc;
+  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((H + MOE_WAVE - 1) / MOE_WAVE)), dim3(CG * MOE_WAVE), 0, s, (const float*)n.workspace,
+                     bwd_blocks(T), (int)H, n.dweight);
   return moe_launch_status();
 }

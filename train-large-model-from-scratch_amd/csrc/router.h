@@ -24,4 +24,17 @@ int moe_routed_forward(const MoeRouter& router, const uint16_t* x, const uint16_
 // moe_in_place_layer_backward, which has x as xn.
 bool moe_layer_rows_from_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k);
 int moe_in_place_layer_backward(const moe_layer_backward_args* a, void* stream);
+// moe_layer_backward, or moe_in_place_layer_backward where there is no xp, with the backward pass of the norm in front of the layer: dx is the
+// gradient of the norm's input, of its type.  For a router whose gradients are worked out in the call, and sizes that moe_norm_rows_ok takes.
+struct MoeNormBackward {
+  const void* x;        // the norm's input [T,H]
+  int x_dtype;
+  const float *weight, *rstd;
+  const void* dres;     // gradient of a residual branch, of x's type (NULL: there is none)
+  float* dweight;       // [H]
+  void* workspace;      // of moe_rmsnorm_bwd_workspace_bytes
+  int64_t workspace_bytes;
+};
+bool moe_norm_rows_ok(int64_t T, int64_t H);
+int moe_norm_layer_backward(const moe_layer_backward_args* a, const MoeNormBackward& norm, void* stream);
 int moe_selected_layer_forward(const moe_layer_forward_args* a, const MoeRouter* router, const void* table, void* stream);
