@@ -12,6 +12,12 @@ pytestmark = pytest.mark.gpu
     (5200, 2048, 64, 1024, 2, 2.0),   # dealt longest first; experts with a row or two and without any
     (10400, 1992, 64, 1000, 1, 1.0),
     (9216, 1536, 48, 768, 1, -1.0),   # 192 rows each: whole k-tiles
+    # ... and in the kernel for small launches: a step or two, ends inside a step, experts cut into segments, more experts than lanes
+    (5, 72, 4, 24, 2, 0.0),
+    (130, 264, 16, 136, 4, 0.5),
+    (3333, 1416, 12, 568, 3, 0.3),
+    (8192, 1024, 8, 512, 2, 1.5),
+    (900, 512, 96, 192, 4, 0.4),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])  # of the weights and their gradients
 def test_training_reads_the_tokens(pkg, T, H, E, I, k, skew, dtype):
@@ -49,7 +55,7 @@ def test_training_reads_the_tokens(pkg, T, H, E, I, k, skew, dtype):
     lib = pkg.ops._lib.load()
     xr = x.detach().requires_grad_(True)
     out, logits, grads = passed(lambda a, b, c: pkg.routed_moe(xr, wr, a, b, c, k, bias=bias))
-    assert "moe_gemm_wgrad_all" in calls
+    assert ("moe_gemm_wgrad_all" if E >= 48 and H > 1000 else "moe_wgrad_multi") in calls
     want, _, want_grads = passed(lambda a, b, c: (pkg.moe_ffn(x, logits, a, b, c, k, bias=bias), logits))
     assert torch.equal(out, want)
     for i, (a, b) in enumerate(zip(grads, want_grads)):

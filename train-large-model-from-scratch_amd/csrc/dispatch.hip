@@ -470,7 +470,7 @@ template <typename DT, int NV>
 __global__ __launch_bounds__(256) void combine_bwd_token_kernel(
     const DT* __restrict__ dy, const uint16_t* __restrict__ y, const float* __restrict__ gates,
     const int32_t* __restrict__ row_to_pos, int T, int H8, int k, uint16_t* __restrict__ dyp,
-    float* __restrict__ dgates) {
+    float* __restrict__ dgates, uint32_t* __restrict__ row_at) {
   const int H = H8 * 8, lane = lane_id();
   const int wpb = blockDim.x / MOE_WAVE;
   for (int t = blockIdx.x * wpb + uniform((int)(threadIdx.x / MOE_WAVE)); t < T; t += gridDim.x * wpb) {
@@ -480,6 +480,7 @@ __global__ __launch_bounds__(256) void combine_bwd_token_kernel(
       const int c = lane + i * MOE_WAVE;
       if (c < H8) d[i] = load8(dy + (size_t)t * H + c * 8);
     }
+    if (row_at && lane < k) row_at[row_to_pos[t * k + lane]] = (uint32_t)t * (uint32_t)(H * 2);
     for (int j = 0; j < k; ++j) {
       const int r = t * k + j;
       const int pos = row_to_pos[r];
@@ -789,12 +790,12 @@ extern "C" int moe_combine_bwd(const void* dy, int dy_dtype, const uint16_t* y, 
 template <typename DT>
 static int launch_combine_bwd_token(const void* dy, const uint16_t* y, const float* gates,
                                     const int32_t* row_to_pos, int64_t T, int64_t H, int64_t k,
-                                    uint16_t* dyp, float* dgates, hipStream_t s) {
+                                    uint16_t* dyp, float* dgates, hipStream_t s, uint32_t* row_at = nullptr) {
   const dim3 grid(mover_grid(T, 4)), block(256);
   const int64_t nv = (H / 8 + MOE_WAVE - 1) / MOE_WAVE;
 #define MOE_CBT(NV)                                                                               \
   hipLaunchKernelGGL((combine_bwd_token_kernel<DT, NV>), grid, block, 0, s, (const DT*)dy, y, gates, \
-                     row_to_pos, (int)T, (int)(H / 8), (int)k, dyp, dgates)
+                     row_to_pos, (int)T, (int)(H / 8), (int)k, dyp, dgates, row_at)
   if (nv <= 1) MOE_CBT(1);
   else if (nv <= 2) MOE_CBT(2);
   else if (nv <= 4) MOE_CBT(4);
@@ -1066,4 +1067,12 @@ __global__ __launch_bounds__(256) void narrow_ids_kernel(const int64_t* __restri
 int moe_narrow_ids(const int64_t* ids, int64_t R, int32_t* out, hipStream_t s) {
   hipLaunchKernelGGL(narrow_ids_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, s, ids, (int)R, out);
   return moe_launch_status();
+}
+
+int moe_combine_bwd_places(const void* dy, int dy_dtype, const float* gates, const int32_t* row_to_pos, int64_t T, int64_t H, int64_t k,
+                           uint16_t* dyp, uint32_t* row_at, hipStream_t s) {
+  if (dy_dtype != MOE_DT_BF16 && dy_dtype != MOE_DT_F32) return MOE_ERR_DTYPE;
+  if (H > 2048 || k > MOE_WAVE || !row_at) return MOE_ERR_LIMIT;
+  if (dy_dtype == MOE_DT_BF16) return launch_combine_bwd_token<uint16_t>(dy, nullptr, gates, row_to_pos, T, H, k, dyp, nullptr, s, row_at);
+  return launch_combine_bwd_token<float>(dy, nullptr, gates, row_to_pos, T, H, k, dyp, nullptr, s, row_at);
 }

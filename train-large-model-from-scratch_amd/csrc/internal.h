@@ -34,8 +34,12 @@ int moe_rmsnorm_bwd_rows(const MoeNormBackward& n, const uint16_t* dxp, const in
                          const float* gates, const int32_t* ids, const uint16_t* wr, int64_t T, int64_t H, int64_t k, int64_t ld,
                          uint16_t* dlogits, void* dx, hipStream_t s);
 
-// Bytes of scratch that a call with these arguments (all but the scratch filled in) uses, no more than moe_layer_scratch_bytes says:
-// rows that stay in place need no buffer for them (layer.hip).
+// moe_combine_bwd_by_token without y, which also leaves where a position's token is, in bytes of rows of H elements of bf16 (dispatch.hip).
+int moe_combine_bwd_places(const void* dy, int dy_dtype, const float* gates, const int32_t* row_to_pos, int64_t T, int64_t H, int64_t k,
+                           uint16_t* dyp, uint32_t* row_at, hipStream_t s);
+
+// Bytes of scratch that a call with these arguments (all but the scratch filled in) uses: rows that stay in place need no
+// buffer for them (layer.hip), and it is no more than moe_layer_scratch_bytes says but for the list of where they are, without xp.
 int64_t moe_forward_scratch(const moe_layer_forward_args* a);
 int64_t moe_backward_scratch(const moe_layer_backward_args* a);
 
@@ -57,6 +61,8 @@ struct MoeWgradStack {
   // moe_gemm_wgrad_all: row r of b, or with from_a of a, is row row_from[r] / from_k of its from_rows (NULL: row r)
   const int32_t* row_from;
   int64_t from_k, from_rows;
+  // moe_wgrad_multi: row r of b, of from_rows rows, is row_at[r] bytes from its beginning (NULL: row r); 32 words behind the last are read.
+  const uint32_t* row_at;
   bool from_a;
 };
 // Weight gradients leave with streaming stores from so many bytes of results in a launch on, an eighth of the memory-side cache: a

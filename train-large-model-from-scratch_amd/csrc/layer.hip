@@ -273,9 +273,11 @@ RouterSlices router_slices(int64_t T, int64_t H, int64_t E) {
 
 struct BwdScratch {
   uint16_t *dyp, *dg, *dxp;
+  uint32_t* row_at;
   float *part, *wpart[3], *rpart;
   uint16_t* dlogits;
-  BwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, bool with_dxp = true, bool with_dyp = true) {
+  BwdScratch(Scratch& s, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, bool with_dxp = true, bool with_dyp = true,
+             bool with_places = false) {
     const int64_t R = T * k;
     dyp = (uint16_t*)s.take(with_dyp ? R * H * 2 : 0);
     dg = (uint16_t*)s.take(R * I * 4);
@@ -285,6 +287,7 @@ struct BwdScratch {
     dlogits = (uint16_t*)s.take(T * rs.Ep * 4);
     rpart = (float*)s.take(rs.slices * rs.Ep * H * 4);
     for (float*& w : wpart) w = (float*)s.take(wgrad_multi(E, I, H, R) ? moe_wgrad_multi_part_bytes(R, H, I) : 0);
+    row_at = with_places ? (uint32_t*)s.take((R + 32) * 4) : nullptr;
   }
 };
 
@@ -303,7 +306,8 @@ bool dx_in_place(const moe_layer_backward_args& a) {
 // and by Dirichlet's shares 3483 -> 3407 and 3458 -> 3378; 12000 of 64, 2048 <-> 1024, 743 -> 725; 30000 of 32, 1000 <-> 1000, 728 -> 711; 60000 of 128 by
 // Dirichlet's shares, 768 <-> 256, 610 -> 578; 50000 of 96, 512 <-> 640, 542 -> 542.
 bool dout_in_place(const moe_layer_backward_args& a) {
-  return a.k == 1 && !a.gates && a.dout_dtype == MOE_DT_BF16 && moe_layer_rows_from_ok(a.T, a.H, a.E, a.I, a.k);
+  return a.k == 1 && !a.gates && a.dout_dtype == MOE_DT_BF16 && moe_layer_rows_from_ok(a.T, a.H, a.E, a.I, a.k) &&
+         !wgrad_multi(a.E, a.I, a.H, a.T);
 }
 
 bool dtype_ok(int64_t d) { return d == MOE_DT_BF16 || d == MOE_DT_F32; }
@@ -352,19 +356,25 @@ int64_t moe_forward_scratch(const moe_layer_forward_args* a) {
 int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
   if (!sizes_ok(a->T, a->H, a->E, a->I, a->k)) return 0;
   Scratch s{nullptr, 0, 0};
-  BwdScratch(s, a->T, a->H, a->E, a->I, a->k, a->dx && !a->dxp && !dx_in_place(*a), !dout_in_place(*a));
+  BwdScratch(s, a->T, a->H, a->E, a->I, a->k, a->dx && !a->dxp && !dx_in_place(*a), !dout_in_place(*a),
+             !a->xp && wgrad_multi(a->E, a->I, a->H, a->T * a->k));
   return s.at;
 }
 
-// Training steps in which nobody but gate/up and the tiled gradients of its weights would read rows in expert order: both read x where it
+// Training steps in which nobody but gate/up and the gradients of its weights would read rows in expert order: both read x where it
 // is, a lane's offset a row, those of a k-tile of the gradients asked for a k-tile ahead.  Besides the pass the copies (R x H x 2 bytes, a
 // step's largest buffer) go from memory's traffic and from what is held between the passes.  Steps with the copies and this one, the same bits, us:
 // 16384 tokens, 8 of 64 experts, 2048 <-> 1024, 4992 -> 4909; 8192 with norm and fp32 gradients 2933 -> 2906; 4096, 8 of 128, 1024 <-> 256, fp32
 // gradients, 409 -> 394; 9000, 4 of 64 by Zipf's shares, 1416 <-> 1000, 2116 -> 2091; 16000, 1 of 32, 2000 <-> 800, 980 -> 971; 8000, 8 of
 // 128, 256 <-> 640, 500 -> 500.  Tiles of one or two k-tiles have none to ask ahead in: rows an expert, 64 experts, 2048 <-> 1024, 250 947 -> 932;
 // 125 676 -> 687; 100 653 -> 675; 75 629 -> 651; 162 of 32 474 -> 472.
+// The kernel for small weight gradients finds where its rows are in a list that the pass over the output's gradient leaves (which is by token where k > 1
+// and rows are at most 2048 long): 8192, 2 of 8 by Zipf's shares, 1024 <-> 512, 291 -> 282; 3333, 3 of 12, 1416 <-> 568, 288 -> 286; 8000, 4 of 16, 768 <->
+// 768, 525 -> 515; 15000, 2 of 8, 256 <-> 2048, 563 -> 557; 2000, 8 of 64, 320 <-> 256, 118 -> 116; with the division by k in the kernel instead 298 ->
+// 291, 295 -> 297, 541 -> 550.
 bool moe_layer_rows_from_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
-  return T > 0 && sizes_ok(T, H, E, I, k) && moe_rows_from_ok(T, H) && T * k >= 160 * E && !wgrad_multi(E, I, H, T * k);
+  return T > 0 && sizes_ok(T, H, E, I, k) && moe_rows_from_ok(T, H) && 
+         (wgrad_multi(E, I, H, T * k) ? k > 1 && k <= MOE_WAVE && H <= 2048 : T * k >= 160 * E);
 }
 
 // (`router` and `table`: see router.h; `in_place`: no xp, x is in bf16)
@@ -497,20 +507,23 @@ static int layer_backward(const moe_layer_backward_args* a, bool in_place, const
   if (norm && (!router || !to_logits || !a->dx || a->dxp || a->dlogits || !moe_norm_rows_ok(T, H))) return MOE_ERR_SHAPE;
   Scratch s{(char*)a->scratch, 0, a->scratch_bytes};
   const bool dout_stays = dout_in_place(*a);
-  const BwdScratch ws(s, T, H, E, I, k, a->dx && !a->dxp && !dx_in_place(*a), !dout_stays);
+  const bool multi = wgrad_multi(E, I, H, R);
+  const BwdScratch ws(s, T, H, E, I, k, a->dx && !a->dxp && !dx_in_place(*a), !dout_stays, in_place && multi);
   if (!s.fits()) return MOE_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   uint16_t* dxp = a->dxp ? a->dxp : ws.dxp;
   const uint16_t* dyp = dout_stays ? (const uint16_t*)a->dout : ws.dyp;
   if (R > 0 && !dout_stays) {
-    if (k > 1 && H <= 2048)
+    if (in_place && multi)
+      MOE_STEP("moe_combine_bwd_by_token", moe_combine_bwd_places(a->dout, (int)a->dout_dtype, a->gates, a->row_to_pos, T, H, k, ws.dyp,
+                                                                  ws.row_at, st));
+    else if (k > 1 && H <= 2048)
       MOE_STEP("moe_combine_bwd_by_token", moe_combine_bwd_by_token(a->dout, (int)a->dout_dtype, nullptr, a->gates,
                                                                     a->row_to_pos, T, H, k, ws.dyp, nullptr, stream));
     else
       MOE_STEP("moe_combine_bwd", moe_combine_bwd(a->dout, (int)a->dout_dtype, nullptr, a->gates, a->pos_to_row, R, H,
                                                   k, ws.dyp, nullptr, stream));
   }
-  const bool multi = wgrad_multi(E, I, H, R);
   // dg and du side by side where their two weight gradients can come out of one launch of the tiled kernel: both
   // wanted into results of one kind, no 256-row tile of the stacked result across the halves
   const bool pair = R > 0 && a->dw[0] && a->dw[1] && I % WTILE == 0 && !multi && a->dw_dtype[0] == a->dw_dtype[1] &&
@@ -564,7 +577,11 @@ static int layer_backward(const moe_layer_backward_args* a, bool in_place, const
     m.a = w == 2 ? dyp : w == 0 ? dg : du;
     m.b = w == 2 ? a->act : in_place ? a->xn : a->xp;
     if (dout_stays && w == 2) m.row_from = a->pos_to_row, m.from_k = k, m.from_rows = T, m.from_a = true;
-    if (in_place && w != 2) m.row_from = a->pos_to_row, m.from_k = k, m.from_rows = T;
+    if (in_place && w != 2) {
+      m.from_k = k, m.from_rows = T;
+      if (multi) m.row_at = ws.row_at;
+      else m.row_from = a->pos_to_row;
+    }
     m.M = w == 2 ? H : I;
     m.N = w == 2 ? I : H;
     m.lda = m.M, m.ldb = m.N;

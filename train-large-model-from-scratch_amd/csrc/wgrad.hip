@@ -26,6 +26,7 @@ struct Stack {
   void* out;              // [E, M, N]
   float* part;            // partial sums [slot][M][N]
   int lda, ldb, M, N, n_tiles, tiles, out_f32, accumulate;
+  int from;               // row r of b is where row_at[r] says
   float per_n;            // 1 / n_tiles
 };
 struct MultiArgs {
@@ -39,6 +40,8 @@ struct MultiArgs {
   int r_first;               // the router's jobs come first, or last
   int streaming;             // results that replace what is there leave with streaming stores, where rows allow it
   float per_each, r_per_tiles;
+  const uint32_t* row_at;    // bytes from b's beginning (32 words behind the last can be read)
+  long long from_bytes;      // of a `from` stack's b, less than 2^31
 };
 // n / d of a wave-uniform n, 1 / d given (exact: n is far below 2^23)
 __device__ __forceinline__ int quotient(int n, int d, float per_d) {
@@ -176,14 +179,48 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   opA.init(st.lda, wv);
   opB.init(st.ldb, wv);
   const View vA = make_view(st.a + (long long)sg.row0 * st.lda + m0, (long long)rows * st.lda - m0);
-  const View vB = make_view(st.b + (long long)sg.row0 * st.ldb + n0, (long long)rows * st.ldb - n0);
+  const View vB = st.from ? View{st.b + n0, p.from_bytes - n0 * 2}
+                          : make_view(st.b + (long long)sg.row0 * st.ldb + n0, (long long)rows * st.ldb - n0);
   const int steps = (rows + WK - 1) / WK;
   const uint32_t stages = lds_address(sm);
   long long askA = 0, askB = 0;
   uint32_t ask_at = 0;
+  // (b's lines from anywhere: where a step's rows are comes through the scalar cache, asked for a step ahead, as a vector load, in order with those of
+  // the ring, would have to be waited for with them; a lane has its line's)
+  static_assert(WOpB::PER_WAVE == 2 && WOpB::LPP == 4, "a wave's lines");
+  const int q = lane / WOpB::CPL;
+  const uint32_t piece = ((lane % WOpB::CPL) ^ WOpB::swizzle(q)) * 16;
+  uint32_t from[2][4];  // of the step asked for next
+  int ask_row = 0;
+  const auto fetch = [&](int row) {
+    typedef const __attribute__((address_space(4))) uint32_t* Scalar;
+    const Scalar at = (Scalar)(p.row_at + sg.row0 + row + wv * 4);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) from[i][j] = at[i * 16 + j];
+  };
+  if (st.from && rows > 0) fetch(0);
+  const auto ask_lines = [&](uint32_t stage, bool live) {
+    const u32x4 window = ring_rsrc(vB, 0, live);
+    const bool whole = ask_row + WK <= rows;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint32_t line = from[i][0];
+      asm("" : "+v"(line));  // (or the four choices become an array in memory)
+      line = q == 1 ? from[i][1] : line;
+      line = q == 2 ? from[i][2] : line;
+      line = (q == 3 ? from[i][3] : line) + piece;
+      if (!whole) line = ask_row + (i * 4 + wv) * 4 + q < rows ? line : NO_ROW;
+      ring_load(stage + (i * 4 + wv) * 1024, window, line);
+    }
+    ask_row += WK;
+    if (ask_row < rows) fetch(ask_row);
+  };
   const auto ask = [&](bool live) {  // (past the last step: empty loads, which the counting of loads relies on)
     opA.load(stages + ask_at, wv, ring_rsrc(vA, askA, live));
-    opB.load(stages + ask_at + WOpA::BYTES, wv, ring_rsrc(vB, askB, live));
+    if (st.from) ask_lines(stages + ask_at + WOpA::BYTES, live);
+    else opB.load(stages + ask_at + WOpA::BYTES, wv, ring_rsrc(vB, askB, live));
     askA += (long long)st.lda * (WK * 2);
     askB += (long long)st.ldb * (WK * 2);
     ask_at = ask_at == (WSTAGES - 1) * WSTAGE ? 0 : ask_at + WSTAGE;
@@ -401,6 +438,11 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
   for (int i = 0; i < n_stacks; ++i) {
     fill(a.s[i], stacks[i]);
     a.tiles += a.s[i].tiles;
+    if (const MoeWgradStack& m = stacks[i]; m.row_at) {  // (the same of all that have one)
+      if (!moe_rows_from_ok(m.from_rows, m.N)) return MOE_ERR_LIMIT;
+      a.s[i].from = 1;
+      a.row_at = m.row_at, a.from_bytes = m.from_rows * m.N * 2;
+    }
   }
   int64_t bytes = 0;
   for (int i = 0; i < n_stacks; ++i) bytes += E * stacks[i].M * stacks[i].N * (a.s[i].out_f32 ? 4 : 2);
