@@ -373,7 +373,7 @@ typedef struct {
 
 typedef struct {
   int64_t T, H, E, I, k;
-  const void* dout;       /* [T,H] */
+  const void* dout;       /* [T,H]; results may lie over it */
   int64_t dout_dtype;
   const float* gates;     /* as the forward call left them, from here to w2 (bf16) */
   const int32_t *ids, *offs, *pos_to_row, *row_to_pos;

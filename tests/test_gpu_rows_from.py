@@ -94,3 +94,32 @@ def test_rows_gradient_is_read_where_it_is(pkg, counts, H, I, dtype):
     for height in (0, 1, 64, 128, 256):
         for i, (a, b) in enumerate(zip(passed(torch.bfloat16, height), want)):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (height, i)
+
+
+@pytest.mark.parametrize("over", ["dx", "dxp", "dw1", "dw2"])
+def test_a_result_over_the_outputs_gradient(pkg, over):
+    """Through the C interface a result may take the place of dout; dout is then read before anything is written there."""
+    ops = pkg.ops
+    E, R, H, I = 128, 20480, 1024, 256
+    print("rows, a result over the gradient", over, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(R)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    x, dy, ws = r(R, H), r(R, H), (r(E, I, H), r(E, I, H), r(E, H, I))
+    _, rt, xp, gu, act = ops.layer_forward(x, r(R, E), *ws, 1, train=True)
+
+    def passed(name):
+        room = torch.empty(max(R * H, E * I * H), dtype=torch.bfloat16, device="cuda")
+        dout = room[:R * H].view(R, H).copy_(dy)
+        t = {n: torch.empty_like(w) for n, w in zip(("dw1", "dw3", "dw2"), ws)}
+        t["dx"] = torch.empty_like(x)
+        if name == "dxp" or over == "dxp":
+            t["dxp"] = torch.empty_like(x)
+        if name:
+            t[name] = room[:t[name].numel()].view(t[name].shape)
+        ops.layer_backward(dout, 1, None, rt.ids, rt.offs, rt.pos_to_row, rt.row_to_pos, xp, gu, act, *ws,
+                           (t["dw1"], t["dw3"], t["dw2"]), dx=t["dx"], dxp=t.get("dxp"))
+        return t
+
+    want, got = passed(None), passed(over)
+    for name in want:
+        assert torch.equal(got[name].view(torch.uint8), want[name].view(torch.uint8)), name

@@ -305,9 +305,20 @@ bool dx_in_place(const moe_layer_backward_args& a) {
 // pass that put it in order goes with its buffer.  Steps with the pass and without, the same bits, us: 32768 rows of 16 experts, 4096 <-> 1536, even
 // and by Dirichlet's shares 3483 -> 3407 and 3458 -> 3378; 12000 of 64, 2048 <-> 1024, 743 -> 725; 30000 of 32, 1000 <-> 1000, 728 -> 711; 60000 of 128 by
 // Dirichlet's shares, 768 <-> 256, 610 -> 578; 50000 of 96, 512 <-> 640, 542 -> 542.
+// A result that lies over it would be there before the last of the two has read it: then it is copied first, as everywhere else.
+bool over(const void* p, int64_t bytes, const void* q, int64_t q_bytes) {
+  const uintptr_t at = (uintptr_t)p, other = (uintptr_t)q;
+  return q && at < other + q_bytes && other < at + bytes;
+}
 bool dout_in_place(const moe_layer_backward_args& a) {
-  return a.k == 1 && !a.gates && a.dout_dtype == MOE_DT_BF16 && moe_layer_rows_from_ok(a.T, a.H, a.E, a.I, a.k) &&
-         !wgrad_multi(a.E, a.I, a.H, a.T);
+  if (a.k != 1 || a.gates || a.dout_dtype != MOE_DT_BF16 || !moe_layer_rows_from_ok(a.T, a.H, a.E, a.I, a.k) ||
+      wgrad_multi(a.E, a.I, a.H, a.T))
+    return false;
+  const int64_t rows = a.T * a.H, bytes = rows * 2;
+  const auto size = [](int64_t n, int64_t dtype) { return n * (dtype == MOE_DT_F32 ? 4 : 2); };
+  bool apart = !over(a.dout, bytes, a.dx, size(rows, a.dx_dtype)) && !over(a.dout, bytes, a.dxp, bytes);
+  for (int i = 0; i < 3; ++i) apart = apart && !over(a.dout, bytes, a.dw[i], size(a.E * a.I * a.H, a.dw_dtype[i]));
+  return apart;
 }
 
 bool dtype_ok(int64_t d) { return d == MOE_DT_BF16 || d == MOE_DT_F32; }
