@@ -136,6 +136,10 @@ __device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, 
 // 95 us; this one 79 and 81, and with 16 slices of the router's tokens, at the end of the list, instead of 32 at its start
 // 72 and 82.  Two workgroups with two stages of 64 rows or four of 32: 84 and 92, 80 and 93; two with 256 x 128 tiles
 // and three stages: 99 and 103; four with two stages of 32 rows 77 and 85 where this one takes 72 and 82.
+// FROM: some stack's rows are where row_at says.  (With the question asked in the loop of every launch, those that have none such pay for it too;
+// asked there -> not asked, us: 16936 rows of 128, 320 <-> 512, 61 -> 57 to 65 -> 60; 10065, 1 of 12, 536 <-> 504, 36.8 -> 35.2; 2317, 2 of 8,
+// 2304 <-> 832, 84 -> 79; whole steps 226.6 -> 221.5, 174.3 -> 172.7, 301.6 -> 298.9.)
+template <bool FROM>
 __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) {
   constexpr int KS = WK / 16, LOADS = WOpA::PER_WAVE + WOpB::PER_WAVE;
   __shared__ __attribute__((aligned(1024))) char sm[WSTAGES * WSTAGE];
@@ -179,7 +183,8 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   opA.init(st.lda, wv);
   opB.init(st.ldb, wv);
   const View vA = make_view(st.a + (long long)sg.row0 * st.lda + m0, (long long)rows * st.lda - m0);
-  const View vB = st.from ? View{st.b + n0, p.from_bytes - n0 * 2}
+  const bool from_list = FROM && st.from;
+  const View vB = from_list ? View{st.b + n0, p.from_bytes - n0 * 2}
                           : make_view(st.b + (long long)sg.row0 * st.ldb + n0, (long long)rows * st.ldb - n0);
   const int steps = (rows + WK - 1) / WK;
   const uint32_t stages = lds_address(sm);
@@ -200,7 +205,7 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
 #pragma unroll
       for (int j = 0; j < 4; ++j) from[i][j] = at[i * 16 + j];
   };
-  if (st.from && rows > 0) fetch(0);
+  if (from_list && rows > 0) fetch(0);
   const auto ask_lines = [&](uint32_t stage, bool live) {
     const u32x4 window = ring_rsrc(vB, 0, live);
     const bool whole = ask_row + WK <= rows;
@@ -219,7 +224,7 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   };
   const auto ask = [&](bool live) {  // (past the last step: empty loads, which the counting of loads relies on)
     opA.load(stages + ask_at, wv, ring_rsrc(vA, askA, live));
-    if (st.from) ask_lines(stages + ask_at + WOpA::BYTES, live);
+    if (from_list) ask_lines(stages + ask_at + WOpA::BYTES, live);
     else opB.load(stages + ask_at + WOpA::BYTES, wv, ring_rsrc(vB, askB, live));
     askA += (long long)st.lda * (WK * 2);
     askB += (long long)st.ldb * (WK * 2);
@@ -471,7 +476,8 @@ int moe_wgrad_multi(const MoeWgradStack (&stacks)[3], int n_stacks, const MoeWgr
   if (jobs <= 0) return 0;
   if (jobs > 0x7fffffffll) return MOE_ERR_LIMIT;
   a.e_each = (int)e_each;
-  hipLaunchKernelGGL(wgrad_multi_kernel, dim3((unsigned)jobs), dim3(WNT), 0, s, a);
+  if (a.row_at) hipLaunchKernelGGL(wgrad_multi_kernel<true>, dim3((unsigned)jobs), dim3(WNT), 0, s, a);
+  else hipLaunchKernelGGL(wgrad_multi_kernel<false>, dim3((unsigned)jobs), dim3(WNT), 0, s, a);
   const long long cut = n_stacks && R > a.L ? R / a.L : 0;  // experts of more than L rows, at most
   const bool sliced = router && router_slices > 1;
   const long long ys = (cut < E ? cut : E) + (sliced ? 1 : 0);
