@@ -558,7 +558,7 @@ __device__ __forceinline__ void walk_tiles(const GemmArgs& p, uint16_t* smem, co
                            pack_bf16x2(bf16lo(v[2]) + bf16lo(o[2]), bf16hi(v[2]) + bf16hi(o[2])),
                            pack_bf16x2(bf16lo(v[3]) + bf16lo(o[3]), bf16hi(v[3]) + bf16hi(o[3]))};
             }
-          } else if ((MODE == WGRAD || MODE == GATEUP) && p.streaming) {
+          } else if (MODE == WGRAD && p.streaming) {
             asm volatile("" ::: "memory");  // (without the two fences this store and the next become one, an ordinary one)
             __builtin_nontemporal_store(v, dst);
             asm volatile("" ::: "memory");
@@ -1297,11 +1297,9 @@ int launch_rows(GemmArgs& a, int cols, hipStream_t s) {
     return launch<MODE, CfgHalf>(small_rows_gemm_kernel<MODE, uint16_t, BLK, TO, FROM>, attr_done[0], a,
                                  a.n_tiles * row_slots(a.R, a.E, CfgHalf::BM), s);
   a.whole_only = forced_row_tile == ROW_TILE;
-  // With few rows an expert gate/up is bound by its weights, whose way through L2 a streamed act leaves free.  Ordinary -> streaming, forward
-  // passes, us: 64 experts, 2048 <-> 1024, 75 / 125 / 191 / 250 / 400 rows an expert 184.4 -> 184.1, 203.6 -> 200.4, 236.0 -> 230.0, 301.1 -> 299.2, 394.6 ->
-  // 395.4; 12 of 4096 <-> 2048, 150 rows 181.0 -> 177.1; 96 of 1536 <-> 640, 94 rows 172.1 -> 170.5; 48 of 3072 <-> 896, 208 rows, not taken,
-  // 276.4 -> 280.1; 8 of 2048 <-> 1024, 1500 rows 195.6 -> 198.0.  (y and the gradients so too: 0.97 to 1.00 times as fast.)
-  a.streaming = MODE == GATEUP && a.R <= 200ll * a.E;
+  // (act streamed past the caches where rows an expert are few, as it takes the weights' place in L2, gains nothing for certain: at 40 to 195 rows
+  // an expert, 14 layers, ordinary -> streaming, forward passes 0.95 to 1.08 times as fast, 1.00 in the mean (1280 tokens of 32, 2624 <-> 1792,
+  // 260 -> 273 us; 1280 of 64, 2048 <-> 1024, 230 -> 214), training 0.96 to 1.03, as down and the weight gradients read it next.)
   return launch<MODE, CfgMain>(rows_gemm_kernel<MODE, uint16_t, BLK, TO, FROM>, attr_done[1], a,
                                2 * a.n_tiles * row_slots(a.R, a.E, ROW_TILE), s);
 }

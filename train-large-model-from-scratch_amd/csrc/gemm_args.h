@@ -47,7 +47,7 @@ struct GemmArgs {
   bool from_a;
   Divisor by_k;
   long long from_bytes;  // < 2^31
-  int streaming;   // WGRAD: results that replace what is there leave with streaming stores; GATEUP: act does
+  int streaming;   // WGRAD: results that replace what is there leave with streaming stores
 };
 
 // sigmoid from the two hardware transcendentals (v_exp_f32, v_rcp_f32; about 1 ulp each):
