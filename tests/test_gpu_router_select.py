@@ -60,6 +60,33 @@ def test_bits_of_the_two_calls(pkg, lib, T, E, k, H, taken, x_type, w_type):
     assert (wd - ref_w).norm() <= 2.0 ** -7 * ref_w.norm() + 1e-6
 
 
+@pytest.mark.parametrize("T,E,k,H,w_type,taken", [
+    (1024, 96, 6, 1360, F32, False), (1024, 96, 6, 1360, BF16, True), (1025, 96, 6, 1360, F32, True), (70, 65, 3, 1032, F32, False),
+    (70, 64, 3, 1032, F32, True), (70, 65, 3, 1024, F32, True),
+])
+def test_long_rows_of_fp32_weights(pkg, lib, T, E, k, H, w_type, taken):
+    """Few tokens and long router rows in fp32: the product stays with the library.  The same bits either way."""
+    print("router select, long rows", T, E, k, H, w_type, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + E + H)
+    x, wr = torch.randn(T, H, generator=g, device="cuda"), (torch.randn(E, H, generator=g, device="cuda") * 0.05).to(w_type)
+    ws = [(torch.randn(*s, generator=g, device="cuda") * 0.05).to(BF16) for s in ((E, 8, H), (E, 8, H), (E, H, 8))]
+    names = []
+
+    class Obs:
+        before = staticmethod(names.append)
+        after = staticmethod(lambda name: None)
+
+    lib.observer = Obs()
+    try:
+        out, lg = pkg.routed_moe(x, wr, *ws, k)
+    finally:
+        lib.observer = None
+    assert ("moe_router_select" in names) == taken, names
+    want = F.linear(x.to(BF16), wr.to(BF16))
+    assert torch.equal(lg, want)
+    assert torch.equal(out, pkg.moe_ffn(x, want, *ws, k))
+
+
 def test_values_that_are_not_finite(pkg):
     print("router select, not finite", flush=True)
     g = torch.Generator(device="cuda").manual_seed(3)

@@ -265,7 +265,8 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
     f.routing = empty({r.at[Routing::PARTS]}, at::kInt, x);
   if (wr.defined()) {
     const Tensor wrd = dense(wr.detach());
-    own = !norm_w.defined() && moe_router_select_ok(T, H, E, k) && (wrd.scalar_type() == at::kFloat || wrd.scalar_type() == at::kBFloat16);
+    own = !norm_w.defined() && (wrd.scalar_type() == at::kFloat || wrd.scalar_type() == at::kBFloat16) &&
+          moe_router_select_ok(T, H, E, k, (int)dt(wrd));
     const bool both = !own && !norm_w.defined() && x_type == at::kFloat && wrd.scalar_type() == at::kFloat && H % 8 == 0 && T > 0;
     if (own) {  // (what is to be rounded to bf16 is rounded on the way)
       const bool x_as_is = x_type == at::kBFloat16, wr_as_is = wrd.scalar_type() == at::kBFloat16;

@@ -94,7 +94,7 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   if (router) {
     MOE_CHECK_PTR(router->wr);
     MOE_CHECK_PTR(router->logits);
-    if (few_logits ? x_dtype != MOE_DT_BF16 || router->wr_dtype != MOE_DT_BF16 : !moe_router_select_ok(T, H, E, k))
+    if (few_logits ? x_dtype != MOE_DT_BF16 || router->wr_dtype != MOE_DT_BF16 : !moe_router_select_ok(T, H, E, k, router->wr_dtype))
       return few_logits ? MOE_ERR_DTYPE : MOE_ERR_LIMIT;
   } else {
     MOE_CHECK_PTR(logits);

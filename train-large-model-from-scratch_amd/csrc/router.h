@@ -13,7 +13,7 @@ struct MoeRouter {
 };
 
 // Sizes for which product and selection are one launch (router.hip).
-bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k);
+bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k, int wr_dtype);
 // moe_ffn_forward, and moe_layer_forward (x: the bf16 rows), with the router's product part of it: sizes that moe_router_few_ok (x and
 // wr in bf16) or moe_router_select_ok takes, the latter alone in training.  moe_selected_layer_forward: with a `table` instead the
 // selection is done, ids and gates are there, and so are its counts; with neither it is moe_layer_forward.

@@ -330,15 +330,24 @@ int router_chains(int64_t T, int64_t H, int64_t E) {
 // 12288 tokens 5.0, 5.3, 7.5, 8.6 and 7.2, 7.4, 10.2, 12.1; 2048 wide, 8192 / 12288 tokens 11.3, 16.4 and 12.7, 15.4; 8 of 64, 1024 wide, 1024 / 4096 /
 // 8192 tokens 8.2, 9.2, 17.5 and 10.2, 12.7, 14.5; 2048 wide, 1024 / 2048 / 4096 tokens 10.4, 11.6, 13.9 and 9.2, 12.8, 13.6; 8 of 128, 1024 wide, 256 /
 // 2048 / 4096 tokens 9.9, 10.4, 11.7 and 9.5, 12.7, 13.8; 2048 wide, not taken, 2048 tokens 15.5 and 13.2; fp32, 8 of 128, 1024 wide, 4096 tokens
-// 17.4 and 21.7.  The host has 15 us less to do, which small training steps take: 512 tokens, 2 of 8 experts, 256 <-> 128, 128 -> 104 us.
-bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k) {
-  const bool pays = E <= 16 ? T <= (H <= 1024 ? 12288 : 8192) : T <= TOKENS * moe_compute_units() && E * H <= 128 * 1024;
+// 17.4 and 21.7.  Where the kernel is the longer one of the two by a microsecond the launch that goes is worth more: whole forward passes of the
+// layer, 256 inside, bf16, without -> with it: 64 experts, 2048 wide, 1024 / 4096 tokens 87.6 -> 85.4, 183.5 -> 181.5; 128, 1024 wide, 256 / 4096 tokens
+// 67.4 -> 65.6, 121.8 -> 118; 96, 1360 wide, 128 / 1024 / 4096 tokens 74.7 -> 75.4, 95.1 -> 94.2, 164.7 -> 156; of 70 sizes, 32 to 128 experts, none slower.  The host
+// has 15 us less to do, which small steps take: training, 512 tokens, 2 of 8 experts, 256 <-> 128, 128 -> 104 us.
+// Router rows in fp32 are twice the bytes a workgroup; with more than 64 experts and 1024 columns (two pieces a thread and slice, more than eight slices)
+// that is the longer way while few tokens leave most compute units without a workgroup: with it -> without, 96, 1360 wide, forward, 70 / 512 / 1024 / 1531
+// tokens 79.3 -> 75.0, 87.6 -> 83.0, 101.4 -> 97.9, 111.0 -> 111.0, training, 70 / 256 / 1024 227.9 -> 223.2, 236.5 -> 233.3, 315 -> 312; 80, 1536 wide, 70 / 1024
+// 71.1 -> 67.0, 88.5 -> 83.3.  (Not so, or by no more than a GPU differs from the next: 64, 2048 wide, forward, 70 / 1024 tokens 69.5 -> 66 to 70, 93 -> 90 to 94,
+// training, 70 / 512 213.5 -> 211.8, 256.1 -> 255.0; 128, 1024 wide, forward 66.6 -> 66 to 70, 78.6 -> 76 to 81, training 200 -> 202, 223 -> 230.)
+bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k, int wr_dtype) {
+  const bool long_rows = wr_dtype == MOE_DT_F32 && E > 64 && H > 1024 && T <= 1024;
+  const bool pays = E <= 16 ? T <= (H <= 1024 ? 12288 : 8192) : T <= TOKENS * moe_compute_units() && E * H <= 128 * 1024 && !long_rows;
   return pays && router_chains(T, H, E) != 0 && k > 0 && k <= E && k <= MOE_MAX_TOPK;
 }
 
 int moe_router_select(const MoeRouter& r, int64_t T, int64_t H, int64_t E, int64_t k, int32_t* ids, float* gates, void* table,
                       hipStream_t s) {
-  if (!moe_router_select_ok(T, H, E, k)) return MOE_ERR_LIMIT;
+  if (!moe_router_select_ok(T, H, E, k, r.wr_dtype)) return MOE_ERR_LIMIT;
   for (int d : {r.x_dtype, r.wr_dtype})
     if (d != MOE_DT_BF16 && d != MOE_DT_F32) return MOE_ERR_DTYPE;
   MOE_CHECK_PTR(r.x);
