@@ -61,7 +61,7 @@ struct MoeWgradStack {
   // moe_gemm_wgrad_all: row r of b, or with from_a of a, is row row_from[r] / from_k of its from_rows (NULL: row r)
   const int32_t* row_from;
   int64_t from_k, from_rows;
-  // moe_wgrad_multi: row r of b, of from_rows rows, is row_at[r] bytes from its beginning (NULL: row r); 32 words behind the last are read.
+  // moe_wgrad_multi: row r of b, of from_rows rows, is row_at[r] bytes from its beginning (NULL: row r).
   const uint32_t* row_at;
   bool from_a;
 };

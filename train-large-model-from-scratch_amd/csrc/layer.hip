@@ -287,7 +287,7 @@ struct BwdScratch {
     dlogits = (uint16_t*)s.take(T * rs.Ep * 4);
     rpart = (float*)s.take(rs.slices * rs.Ep * H * 4);
     for (float*& w : wpart) w = (float*)s.take(wgrad_multi(E, I, H, R) ? moe_wgrad_multi_part_bytes(R, H, I) : 0);
-    row_at = with_places ? (uint32_t*)s.take((R + 32) * 4) : nullptr;
+    row_at = with_places ? (uint32_t*)s.take(R * 4) : nullptr;
   }
 };
 
@@ -380,12 +380,13 @@ int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
 // 128, 256 <-> 640, 500 -> 500.  Tiles of one or two k-tiles have none to ask ahead in: rows an expert, 64 experts, 2048 <-> 1024, 250 947 -> 932;
 // 125 676 -> 687; 100 653 -> 675; 75 629 -> 651; 162 of 32 474 -> 472.
 // The kernel for small weight gradients finds where its rows are in a list that the pass over the output's gradient leaves (which is by token where k > 1
-// and rows are at most 2048 long): 8192, 2 of 8 by Zipf's shares, 1024 <-> 512, 291 -> 282; 3333, 3 of 12, 1416 <-> 568, 288 -> 286; 8000, 4 of 16, 768 <->
-// 768, 525 -> 515; 15000, 2 of 8, 256 <-> 2048, 563 -> 557; 2000, 8 of 64, 320 <-> 256, 118 -> 116; with the division by k in the kernel instead 298 ->
-// 291, 295 -> 297, 541 -> 550.
+// and rows are at most 2048 long): 8192, 2 of 8 by Zipf's shares, 1024 <-> 512, 299 -> 282; 3333, 3 of 12, 1416 <-> 568, 294 -> 287; 8000, 4 of 16, 768 <->
+// 768, 515 -> 502; 10892, 6 of 12, 448 <-> 192, 371 -> 336; 2000, 8 of 64, 320 <-> 256, 121 -> 116; 10342, 2 of 4, 832 <-> 704, fp32 gradients, 421 -> 419; of 94
+// sizes drawn, those apart that the host bounds, 1.025 in the mean.  What the copies cost goes with k H, what lines from anywhere cost in the products with I:
+// 2 of 4, 960 <-> 1856, 462 -> 473, 1024 <-> 1152, 496 -> 506, 2 of 64, 352 <-> 1416, 280 -> 285, 4 of 16, 512 <-> 1152, 310 -> 314, not taken.
 bool moe_layer_rows_from_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
-  return T > 0 && sizes_ok(T, H, E, I, k) && moe_rows_from_ok(T, H) && 
-         (wgrad_multi(E, I, H, T * k) ? k > 1 && k <= MOE_WAVE && H <= 2048 : T * k >= 160 * E);
+  return T > 0 && sizes_ok(T, H, E, I, k) && moe_rows_from_ok(T, H) &&
+         (wgrad_multi(E, I, H, T * k) ? k > 1 && k <= MOE_WAVE && H <= 2048 && 2 * I <= k * H : T * k >= 160 * E);
 }
 
 // (`router` and `table`: see router.h; `in_place`: no xp, x is in bf16)

@@ -21,6 +21,10 @@ __device__ __forceinline__ void ring_load(uint32_t lds_byte, u32x4 rsrc, uint32_
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds_byte)
                : "m0");
 }
+// 4 bytes per lane, to lds_byte + 4 * lane.
+__device__ __forceinline__ void ring_load_word(uint32_t lds_byte, u32x4 rsrc, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds_byte) : "m0");
+}
 #pragma clang diagnostic pop
 // All but the wave's N youngest loads have arrived and its LDS reads are done; then meet the other waves, for whose loads
 // and reads the same holds.

@@ -11,6 +11,8 @@
 #include "internal.h"
 #include "ring.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int WBM = 128, WBN = 128;            // tile
@@ -40,7 +42,7 @@ struct MultiArgs {
   int r_first;               // the router's jobs come first, or last
   int streaming;             // results that replace what is there leave with streaming stores, where rows allow it
   float per_each, r_per_tiles;
-  const uint32_t* row_at;    // bytes from b's beginning (32 words behind the last can be read)
+  const uint32_t* row_at;    // bytes from b's beginning
   long long from_bytes;      // of a `from` stack's b, less than 2^31
 };
 // n / d of a wave-uniform n, 1 / d given (exact: n is far below 2^23)
@@ -136,13 +138,14 @@ __device__ __forceinline__ bool find_segment(const int32_t* offs, int E, int L, 
 // 95 us; this one 79 and 81, and with 16 slices of the router's tokens, at the end of the list, instead of 32 at its start
 // 72 and 82.  Two workgroups with two stages of 64 rows or four of 32: 84 and 92, 80 and 93; two with 256 x 128 tiles
 // and three stages: 99 and 103; four with two stages of 32 rows 77 and 85 where this one takes 72 and 82.
-// FROM: some stack's rows are where row_at says.  (With the question asked in the loop of every launch, those that have none such pay for it too;
-// asked there -> not asked, us: 16936 rows of 128, 320 <-> 512, 61 -> 57 to 65 -> 60; 10065, 1 of 12, 536 <-> 504, 36.8 -> 35.2; 2317, 2 of 8,
+// FROM: some stack's rows are where row_at says; each kind of stack has a loop of its own.  (With the question asked in one loop, launches that have none
+// such pay for it too; asked -> not asked, us: 16936 rows of 128, 320 <-> 512, 61 -> 57 to 65 -> 60; 10065, 1 of 12, 536 <-> 504, 36.8 -> 35.2; 2317, 2 of 8,
 // 2304 <-> 832, 84 -> 79; whole steps 226.6 -> 221.5, 174.3 -> 172.7, 301.6 -> 298.9.)
 template <bool FROM>
 __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) {
-  constexpr int KS = WK / 16, LOADS = WOpA::PER_WAVE + WOpB::PER_WAVE;
-  __shared__ __attribute__((aligned(1024))) char sm[WSTAGES * WSTAGE];
+  constexpr int KS = WK / 16;
+  constexpr int PLACES = MOE_WAVE * 4;  // bytes a wave and stage
+  __shared__ __attribute__((aligned(1024))) char sm[WSTAGES * (WSTAGE + (FROM ? 4 * PLACES : 0))];
   const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MOE_WAVE));
   const int wm = wv >> 1, wn = wv & 1;
   // Workgroup b runs on XCD b % 8.  Every XCD takes an eighth of each segment's tiles (neighbours, which share operands
@@ -178,60 +181,9 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
   const int tm = quotient(tile, st.n_tiles, st.per_n);
   const int m0 = tm * WBM, n0 = (tile - tm * st.n_tiles) * WBN;
   const int rows = uniform(sg.row_end - sg.row0);
-  WOpA opA;
-  WOpB opB;
-  opA.init(st.lda, wv);
-  opB.init(st.ldb, wv);
   const View vA = make_view(st.a + (long long)sg.row0 * st.lda + m0, (long long)rows * st.lda - m0);
-  const bool from_list = FROM && st.from;
-  const View vB = from_list ? View{st.b + n0, p.from_bytes - n0 * 2}
-                          : make_view(st.b + (long long)sg.row0 * st.ldb + n0, (long long)rows * st.ldb - n0);
   const int steps = (rows + WK - 1) / WK;
   const uint32_t stages = lds_address(sm);
-  long long askA = 0, askB = 0;
-  uint32_t ask_at = 0;
-  // (b's lines from anywhere: where a step's rows are comes through the scalar cache, asked for a step ahead, as a vector load, in order with those of
-  // the ring, would have to be waited for with them; a lane has its line's)
-  static_assert(WOpB::PER_WAVE == 2 && WOpB::LPP == 4, "a wave's lines");
-  const int q = lane / WOpB::CPL;
-  const uint32_t piece = ((lane % WOpB::CPL) ^ WOpB::swizzle(q)) * 16;
-  uint32_t from[2][4];  // of the step asked for next
-  int ask_row = 0;
-  const auto fetch = [&](int row) {
-    typedef const __attribute__((address_space(4))) uint32_t* Scalar;
-    const Scalar at = (Scalar)(p.row_at + sg.row0 + row + wv * 4);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) from[i][j] = at[i * 16 + j];
-  };
-  if (from_list && rows > 0) fetch(0);
-  const auto ask_lines = [&](uint32_t stage, bool live) {
-    const u32x4 window = ring_rsrc(vB, 0, live);
-    const bool whole = ask_row + WK <= rows;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      uint32_t line = from[i][0];
-      asm("" : "+v"(line));  // (or the four choices become an array in memory)
-      line = q == 1 ? from[i][1] : line;
-      line = q == 2 ? from[i][2] : line;
-      line = (q == 3 ? from[i][3] : line) + piece;
-      if (!whole) line = ask_row + (i * 4 + wv) * 4 + q < rows ? line : NO_ROW;
-      ring_load(stage + (i * 4 + wv) * 1024, window, line);
-    }
-    ask_row += WK;
-    if (ask_row < rows) fetch(ask_row);
-  };
-  const auto ask = [&](bool live) {  // (past the last step: empty loads, which the counting of loads relies on)
-    opA.load(stages + ask_at, wv, ring_rsrc(vA, askA, live));
-    if (from_list) ask_lines(stages + ask_at + WOpA::BYTES, live);
-    else opB.load(stages + ask_at + WOpA::BYTES, wv, ring_rsrc(vB, askB, live));
-    askA += (long long)st.lda * (WK * 2);
-    askB += (long long)st.ldb * (WK * 2);
-    ask_at = ask_at == (WSTAGES - 1) * WSTAGE ? 0 : ask_at + WSTAGE;
-  };
-#pragma unroll
-  for (int i = 0; i < WSTAGES - 1; ++i) ask(i < steps);
   f32x16 acc[WFM][WFN];
 #pragma unroll
   for (int i = 0; i < WFM; ++i)
@@ -239,36 +191,101 @@ __global__ __launch_bounds__(WNT, 3) void wgrad_multi_kernel(const MultiArgs p) 
     for (int j = 0; j < WFN; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  const WOpA::Place inA = WOpA::place(wm * (WBM / 2));
-  const WOpB::Place inB = WOpB::place(wn * (WBN / 2));
-  uint32_t at = 0;
-  for (int s = 0; s < steps; ++s) {
-    ring_wait<(WSTAGES - 2) * LOADS>();
-    const char *sA = sm + at, *sB = sA + WOpA::BYTES;
-    bf16x8 fa[2][WFM], fb[2][WFN];
-    const auto read_one = [&](int u, int ks) {  // in the order the products need them
-      if (u == 0) fa[ks & 1][0] = WOpA::frag(sA, inA, 0, ks);
-      else if (u <= WFN) fb[ks & 1][u - 1] = WOpB::frag(sB, inB, (u - 1) * 32, ks);
-      else fa[ks & 1][u - WFN] = WOpA::frag(sA, inA, (u - WFN) * 32, ks);
-    };
+  const auto products = [&](auto lines_c) __attribute__((always_inline)) {
+    constexpr bool LINES = decltype(lines_c)::value;  // b's lines are where row_at says
+    constexpr int LOADS = WOpA::PER_WAVE + WOpB::PER_WAVE + (LINES ? 1 : 0);
+    const View vB = LINES ? View{st.b + n0, p.from_bytes - n0 * 2}
+                          : make_view(st.b + (long long)sg.row0 * st.ldb + n0, (long long)rows * st.ldb - n0);
+    WOpA opA;
+    WOpB opB;
+    opA.init(st.lda, wv);
+    if constexpr (!LINES) opB.init(st.ldb, wv);
+    long long askA = 0, askB = 0;
+    uint32_t ask_at = 0;
+    // (LINES: where a step's lines are comes through LDS, with the stage two steps before; a wave has its own eight.  As vector loads they would have
+    // to be waited for with the ring's behind them.  Through the scalar cache, whose loads come in any order and are counted with the LDS reads, a step
+    // stood behind them before its first product: 10342 tokens, 2 of 4 experts, 832 <-> 704, 131 us, so and from copies 106.)
+    static_assert(WOpB::PER_WAVE == 2 && WOpB::LPP == 4, "a wave's lines");
+    const int q = lane / WOpB::CPL;
+    const uint32_t piece = ((lane % WOpB::CPL) ^ WOpB::swizzle(q)) * 16;
+    const uint32_t places = stages + WSTAGES * WSTAGE + wv * PLACES;  // of step 0; a step's 4 * PLACES further
+    uint32_t places_from = lane < 8 ? (((lane >> 2) * 4 + wv) * 4 + (lane & 3) + (WSTAGES - 1) * WK) * 4 : NO_ROW;
+    const u32x4 list = ring_rsrc(View{(const uint16_t*)(p.row_at + sg.row0), (long long)rows * 4}, 0, true);
+    uint32_t line[2];
+    int ask_row = q + wv * 4;
+    const auto ask = [&](bool live) {  // (past the last step: empty loads, which the counting of loads relies on)
+      opA.load(stages + ask_at, wv, ring_rsrc(vA, askA, live));
+      if constexpr (LINES) {
+        const u32x4 window = ring_rsrc(vB, 0, live);
 #pragma unroll
-    for (int u = 0; u < WFM + WFN; ++u) read_one(u, 0);
-    // (the stage of the step before is free; the requests go out while the first fragments are on their way, and the
-    // fences keep the compiler from clumping the other reads in front of their use)
-    __builtin_amdgcn_sched_barrier(0);
-    ask(s + WSTAGES - 1 < steps);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int n = 0; n < WFM * WFN; ++n) {
-        const int i = n / WFN, j = (i & 1) ? WFN - 1 - n % WFN : n % WFN;  // neighbours share an operand
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks & 1][j], fa[ks & 1][i], acc[i][j], 0, 0, 0);
-        if (ks + 1 < KS && n < WFM + WFN) read_one(n, ks + 1);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 2; ++i)
+          ring_load(stages + ask_at + WOpA::BYTES + (i * 4 + wv) * 1024, window, ask_row + i * 16 < rows ? line[i] + piece : NO_ROW);
+        const uint32_t slot = ask_at == 0 ? WSTAGES - 1 : ask_at == WSTAGE ? 0 : 1;  // of two steps on
+        ring_load_word(places + slot * (4 * PLACES), list, places_from);
+        places_from += WK * 4;
+        ask_row += WK;
+      } else {
+        opB.load(stages + ask_at + WOpA::BYTES, wv, ring_rsrc(vB, askB, live));
+        askB += (long long)st.ldb * (WK * 2);
       }
-    at = at == (WSTAGES - 1) * WSTAGE ? 0 : at + WSTAGE;
-  }
+      askA += (long long)st.lda * (WK * 2);
+      ask_at = ask_at == (WSTAGES - 1) * WSTAGE ? 0 : ask_at + WSTAGE;
+    };
+    if constexpr (LINES) {
+      const __amdgpu_buffer_rsrc_t first_lines = __builtin_amdgcn_make_buffer_rsrc((void*)(p.row_at + sg.row0), 0, rows * 4, 0x00020000);
+      uint32_t at[WSTAGES - 1][2];
+#pragma unroll
+      for (int i = 0; i < (WSTAGES - 1) * 2; ++i)
+        at[i / 2][i & 1] = __builtin_amdgcn_raw_buffer_load_b32(first_lines, (ask_row + i * 16) * 4, 0, 0);
+      asm volatile("" : "+v"(at[0][0]), "+v"(at[0][1]), "+v"(at[1][0]), "+v"(at[1][1]));  // (waited for here, not behind the ring's first loads)
+#pragma unroll
+      for (int i = 0; i < WSTAGES - 1; ++i) {
+        line[0] = at[i][0], line[1] = at[i][1];
+        ask(i < steps);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < WSTAGES - 1; ++i) ask(i < steps);
+    }
+    const WOpA::Place inA = WOpA::place(wm * (WBM / 2));
+    const WOpB::Place inB = WOpB::place(wn * (WBN / 2));
+    uint32_t at = 0;
+    for (int s = 0; s < steps; ++s) {
+      ring_wait<(WSTAGES - 2) * LOADS>();
+      const char *sA = sm + at, *sB = sA + WOpA::BYTES;
+      bf16x8 fa[2][WFM], fb[2][WFN];
+      const auto read_one = [&](int u, int ks) {  // in the order the products need them
+        if (u == 0) fa[ks & 1][0] = WOpA::frag(sA, inA, 0, ks);
+        else if (u <= WFN) fb[ks & 1][u - 1] = WOpB::frag(sB, inB, (u - 1) * 32, ks);
+        else fa[ks & 1][u - WFN] = WOpA::frag(sA, inA, (u - WFN) * 32, ks);
+      };
+      if constexpr (LINES) {
+        const uint32_t slot = ask_at == 0 ? 0 : ask_at == WSTAGE ? 1 : WSTAGES - 1;  // of the step asked for
+        const char* here = sm + WSTAGES * WSTAGE + slot * (4 * PLACES) + wv * PLACES + q * 4;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) line[i] = *reinterpret_cast<const uint32_t*>(here + i * 16);
+      }
+#pragma unroll
+      for (int u = 0; u < WFM + WFN; ++u) read_one(u, 0);
+      // (the stage of the step before is free; the requests go out while the first fragments are on their way, and the
+      // fences keep the compiler from clumping the other reads in front of their use)
+      __builtin_amdgcn_sched_barrier(0);
+      ask(s + WSTAGES - 1 < steps);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int n = 0; n < WFM * WFN; ++n) {
+          const int i = n / WFN, j = (i & 1) ? WFN - 1 - n % WFN : n % WFN;  // neighbours share an operand
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks & 1][j], fa[ks & 1][i], acc[i][j], 0, 0, 0);
+          if (ks + 1 < KS && n < WFM + WFN) read_one(n, ks + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      at = at == (WSTAGES - 1) * WSTAGE ? 0 : at + WSTAGE;
+    }
+  };
+  if (FROM && st.from) products(std::true_type{});
+  else products(std::false_type{});
   ring_wait<0>();
   // results leave through LDS in strips of 32 rows x 64 columns, fp32: a wave's accumulators hold row l % 32 and
   // columns 8 q + 4 (l / 32) .. + 3 of each block
