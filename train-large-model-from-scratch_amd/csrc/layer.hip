@@ -301,18 +301,18 @@ bool dx_in_place(const moe_layer_backward_args& a) {
   return a.k == 1 && a.dx && !a.dxp && !router && a.dx_dtype == MOE_DT_BF16;
 }
 
+bool over(const void* p, int64_t bytes, const void* q, int64_t q_bytes) {
+  const uintptr_t at = (uintptr_t)p, other = (uintptr_t)q;
+  return q && at < other + q_bytes && other < at + bytes;
+}
+
 // The output's gradient is theirs too but for the order.  Where the weight gradients are tiled both of its products read it where it is, and the
 // pass that put it in order goes with its buffer.  Steps with the pass and without, the same bits, us: 32768 rows of 16 experts, 4096 <-> 1536, even
 // and by Dirichlet's shares 3483 -> 3407 and 3458 -> 3378; 12000 of 64, 2048 <-> 1024, 743 -> 725; 30000 of 32, 1000 <-> 1000, 728 -> 711; 60000 of 128 by
 // Dirichlet's shares, 768 <-> 256, 610 -> 578; 50000 of 96, 512 <-> 640, 542 -> 542.
 // A result that lies over it would be there before the last of the two has read it: then it is copied first, as everywhere else.
-bool over(const void* p, int64_t bytes, const void* q, int64_t q_bytes) {
-  const uintptr_t at = (uintptr_t)p, other = (uintptr_t)q;
-  return q && at < other + q_bytes && other < at + bytes;
-}
 bool dout_in_place(const moe_layer_backward_args& a) {
-  if (a.k != 1 || a.gates || a.dout_dtype != MOE_DT_BF16 || !moe_layer_rows_from_ok(a.T, a.H, a.E, a.I, a.k) ||
-      wgrad_multi(a.E, a.I, a.H, a.T))
+  if (a.k != 1 || a.gates || a.dout_dtype != MOE_DT_BF16 || !moe_rows_from_ok(a.T, a.H) || a.T < 160 * a.E || wgrad_multi(a.E, a.I, a.H, a.T))
     return false;
   const int64_t rows = a.T * a.H, bytes = rows * 2;
   const auto size = [](int64_t n, int64_t dtype) { return n * (dtype == MOE_DT_F32 ? 4 : 2); };
@@ -378,7 +378,8 @@ int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
 // 16384 tokens, 8 of 64 experts, 2048 <-> 1024, 4992 -> 4909; 8192 with norm and fp32 gradients 2933 -> 2906; 4096, 8 of 128, 1024 <-> 256, fp32
 // gradients, 409 -> 394; 9000, 4 of 64 by Zipf's shares, 1416 <-> 1000, 2116 -> 2091; 16000, 1 of 32, 2000 <-> 800, 980 -> 971; 8000, 8 of
 // 128, 256 <-> 640, 500 -> 500.  Tiles of one or two k-tiles have none to ask ahead in: rows an expert, 64 experts, 2048 <-> 1024, 250 947 -> 932;
-// 125 676 -> 687; 100 653 -> 675; 75 629 -> 651; 162 of 32 474 -> 472.
+// 125 676 -> 687; 100 653 -> 675; 75 629 -> 651; 162 of 32 474 -> 472.  Nor are they for rows that are short beside the products: of 50 sizes drawn,
+// 1.016 in the mean, those with I past 2 H 0.999: 8126, 4 of 128 by Zipf's shares, 384 <-> 1600, 1181 -> 1224; 7824, 4 of 96, 448 <-> 1152, 626 -> 630.
 // The kernel for small weight gradients finds where its rows are in a list that the pass over the output's gradient leaves (which is by token where k > 1
 // and rows are at most 2048 long): 8192, 2 of 8 by Zipf's shares, 1024 <-> 512, 299 -> 282; 3333, 3 of 12, 1416 <-> 568, 294 -> 287; 8000, 4 of 16, 768 <->
 // 768, 515 -> 502; 10892, 6 of 12, 448 <-> 192, 371 -> 336; 2000, 8 of 64, 320 <-> 256, 121 -> 116; 10342, 2 of 4, 832 <-> 704, fp32 gradients, 421 -> 419; of 94
@@ -386,7 +387,7 @@ int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
 // 2 of 4, 960 <-> 1856, 462 -> 473, 1024 <-> 1152, 496 -> 506, 2 of 64, 352 <-> 1416, 280 -> 285, 4 of 16, 512 <-> 1152, 310 -> 314, not taken.
 bool moe_layer_rows_from_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
   return T > 0 && sizes_ok(T, H, E, I, k) && moe_rows_from_ok(T, H) &&
-         (wgrad_multi(E, I, H, T * k) ? k > 1 && k <= MOE_WAVE && H <= 2048 && 2 * I <= k * H : T * k >= 160 * E);
+         (wgrad_multi(E, I, H, T * k) ? k > 1 && k <= MOE_WAVE && H <= 2048 && 2 * I <= k * H : I <= 2 * H && T * k >= 160 * E);
 }
 
 // (`router` and `table`: see router.h; `in_place`: no xp, x is in bf16)
