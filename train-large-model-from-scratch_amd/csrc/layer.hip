@@ -379,7 +379,8 @@ int64_t moe_backward_scratch(const moe_layer_backward_args* a) {
 // gradients, 409 -> 394; 9000, 4 of 64 by Zipf's shares, 1416 <-> 1000, 2116 -> 2091; 16000, 1 of 32, 2000 <-> 800, 980 -> 971; 8000, 8 of
 // 128, 256 <-> 640, 500 -> 500.  Tiles of one or two k-tiles have none to ask ahead in: rows an expert, 64 experts, 2048 <-> 1024, 250 947 -> 932;
 // 125 676 -> 687; 100 653 -> 675; 75 629 -> 651; 162 of 32 474 -> 472.  Nor are they for rows that are short beside the products: of 50 sizes drawn,
-// 1.016 in the mean, those with I past 2 H 0.999: 8126, 4 of 128 by Zipf's shares, 384 <-> 1600, 1181 -> 1224; 7824, 4 of 96, 448 <-> 1152, 626 -> 630.
+// 1.016 in the mean, those with I past 2 H 0.999: 8126, 4 of 128 by Zipf's shares, 384 <-> 1600, 1181 -> 1224; 7824, 4 of 96, 448 <-> 1152, 626 -> 630.  (Most of 128 experts by
+// Zipf's shares have few rows where the mean is 160: 1024 <-> 256, 165 / 200 / 250 rows 352 -> 358, 404 -> 412, 488 -> 485, even 307 -> 302, 339 -> 324, 393 -> 376.)
 // The kernel for small weight gradients finds where its rows are in a list that the pass over the output's gradient leaves (which is by token where k > 1
 // and rows are at most 2048 long): 8192, 2 of 8 by Zipf's shares, 1024 <-> 512, 299 -> 282; 3333, 3 of 12, 1416 <-> 568, 294 -> 287; 8000, 4 of 16, 768 <->
 // 768, 515 -> 502; 10892, 6 of 12, 448 <-> 192, 371 -> 336; 2000, 8 of 64, 320 <-> 256, 121 -> 116; 10342, 2 of 4, 832 <-> 704, fp32 gradients, 421 -> 419; of 94

@@ -357,8 +357,9 @@ __global__ __launch_bounds__(NT) void rmsnorm_bwd_kernel(
 // Two passes write d1 and read it, a launch apart.  Whole steps, fp32 x, us, two passes -> this, the same bits: 8192 tokens, 8 of 64 experts, 2048
 // wide, 2877 -> 2855; 2 of 16 639 -> 611; 12000, 1 of 8, 1024 wide, 288 -> 273; 3000, 8 of 24, 4096 wide, 893 -> 852; 700, 4 of 48, 1400 wide, 355 ->
 // 354; 64, 2 of 16, 1024 wide, 165 -> 159.  A block a token, as the norm's mean has it (the rows by themselves have a wave a token): narrow
-// rows leave its waves without columns, which is less than the launch only while tokens are few: 640 wide, 3000 / 16000 tokens 199 -> 194, 532 ->
-// 534; 512 wide, 2000 / 8000 170 -> 167, 407 -> 417; 256 wide, 4000 / 16000 200 -> 197, 255 -> 262; 768 wide, 16000 444 -> 439.
+// rows leave its waves without columns, which is less than the launch only while tokens are few: 832 wide, 9312 tokens 446 -> 438 without; below 4096 tokens
+// steps that the host bounds gain 2 % (384 wide, 2563 tokens 174 -> 169; 704 wide, 2188 212 -> 208.5), others are within 1 % (576 wide, 3929 tokens 511 -> 516; 448
+// wide, 2837 196 -> 195).  From 1024 columns on none of 25 drawn sizes is slower by more than 0.6 %, 1.013 in the mean.
 template <typename XT, int NV>
 __global__ __launch_bounds__(NT, NV == 1 ? 4 : 2) void rmsnorm_bwd_rows_kernel(
     const XT* __restrict__ x, const float* __restrict__ w, const float* __restrict__ rstd, const uint16_t* __restrict__ dxp,
@@ -627,7 +628,7 @@ extern "C" int moe_rmsnorm_bwd(const void* x, int x_dtype, const float* weight, 
 }
 
 bool moe_norm_rows_ok(int64_t T, int64_t H) {
-  return T > 0 && T <= (int64_t)1 << 30 && H % 8 == 0 && pick_nv(H) != 0 && (H >= 768 || T <= 4096);
+  return T > 0 && T <= (int64_t)1 << 30 && H % 8 == 0 && pick_nv(H) != 0 && (H >= 1024 || T <= 4096);
 }
 
 int moe_rmsnorm_bwd_rows(const MoeNormBackward& n, const uint16_t* dxp, const int32_t* row_to_pos, const float* part, int64_t P,
