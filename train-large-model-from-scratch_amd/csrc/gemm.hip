@@ -1227,10 +1227,8 @@ __global__ __launch_bounds__(CfgMain::NT, CfgMain::WAVES_PER_SIMD) void wgrad_ge
       first = lo + j, end = lo + q + (x < r ? 1 : 0), step = (nb >> 3) + (x < (nb & 7) ? 1 : 0);
     }
     if (w) __syncthreads();  // (the operand stages are free)
-    if ((FROM & FROM_A) && p.row_from && p.from_a)
-      walk_tiles<WGRAD, CfgMain, OutT, false, ROW_TILE, false, FROM_A>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
-    else if ((FROM & FROM_B) && p.row_from)
-      walk_tiles<WGRAD, CfgMain, OutT, false, ROW_TILE, false, FROM_B>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
+    if (FROM && p.row_from)
+      walk_tiles<WGRAD, CfgMain, OutT, false, ROW_TILE, false, FROM>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
     else walk_tiles<WGRAD, CfgMain, OutT, false>(p, smem, nullptr, p.offs, ranked ? glist : nullptr, first, end, step);
     done += total;
   }
@@ -1323,13 +1321,15 @@ int launch_wgrad(const WgradArgs& args, hipStream_t s) {
     const long long n = (long long)a.n_tiles * a.m_slots * a.E;
     tiles = tiles > n ? tiles : n;
   }
-  static bool attr_done[4][MOE_MAX_DEVICES];
-  int from = 0;
-  for (int i = 0; i < w.n; ++i)
-    if (w.p[i].row_from) from |= w.p[i].from_a ? FROM_A : FROM_B;
+  static bool attr_done[3][MOE_MAX_DEVICES];
+  int from = 0;  // (a's lines are where the caller has them where the experts are given, b's where the router is part of the call)
+  for (int i = 0; i < w.n; ++i) {
+    const int of = w.p[i].row_from ? (w.p[i].from_a ? FROM_A : FROM_B) : 0;
+    if (of && from && of != from) return MOE_ERR_LIMIT;
+    from |= of;
+  }
   if (from == FROM_A) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, FROM_A>, attr_done[1], w, tiles, s);
   if (from == FROM_B) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, FROM_B>, attr_done[2], w, tiles, s);
-  if (from) return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, FROM_A | FROM_B>, attr_done[3], w, tiles, s);
   return launch<WGRAD, CfgMain>(wgrad_gemm_kernel<OutT, 0>, attr_done[0], w, tiles, s);
 }
 

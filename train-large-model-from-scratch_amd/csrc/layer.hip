@@ -456,7 +456,7 @@ static int layer_forward(const moe_layer_forward_args* a, const MoeRouter* route
                      : moe_permute_fwd(a->x, (int)a->x_dtype, a->pos_to_row, R, H, k, a->xp, stream));
   }
   if (in_place)
-    MOE_STEP(a->gu ? "moe_gemm_gateup_swiglu_fwd_blocked" : "moe_gemm_gateup_swiglu_fwd",
+    MOE_STEP("moe_gemm_gateup_swiglu_fwd_blocked",
              moe_gemm_gateup_from((const uint16_t*)a->x, a->pos_to_row, T, k, a->w1, a->w3, a->offs, E, H, I, a->gu, a->act, stream));
   else if (a->gu)
     MOE_STEP("moe_gemm_gateup_swiglu_fwd_blocked",
