@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
     (4321, 640, 130, 328, 6),    # past the sizes that have a table of counts
 ])
 def test_rows_from_the_tokens(pkg, T, H, E, I, k):
-    ops, force = pkg.ops, pkg.ops._lib.load().cdll.moe_gemm_force_row_tile
+    ops, cdll = pkg.ops, pkg.ops._lib.load().cdll
+    force, workspace = cdll.moe_gemm_force_row_tile, cdll.moe_ffn_forward_workspace_bytes
     g = torch.Generator(device="cuda").manual_seed(T + H)
     r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
     x, logits, w1, w3, w2 = r(T, H), r(T, E), r(E, I, H), r(E, I, H), r(E, H, I)
@@ -27,10 +28,15 @@ def test_rows_from_the_tokens(pkg, T, H, E, I, k):
     want = ops.combine_fwd(ops.gemm_down(act, w2, offs), gates, row_to_pos, T, k, torch.bfloat16)
     for height in (0, 1, 64, 128, 256):
         print("rows from the tokens", T, H, E, I, k, height, flush=True)
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_stats()["requested_bytes.all.current"]
         try:
             force(height)
             with torch.no_grad():
                 out = pkg.moe_ffn(x, logits, w1, w3, w2, k)
         finally:
             force(0)
+        held = torch.cuda.memory_stats()["requested_bytes.all.peak"] - before
         assert torch.equal(out, want), height
+        # (no room for copies, of which the documented workspace has some; parts of it begin at multiples of 256 bytes)
+        assert held <= workspace(T, H, E, I, k) - T * k * H * 2 + out.numel() * 2 + 256, held

@@ -331,17 +331,13 @@ Outputs forward(const Layer& o, const Tensor& x_, const Tensor& norm_w, const Te
   f.logits = logits;
   if (!f.routing.defined()) {  // nothing is kept and nobody asks for the routing
     f.out = empty({T, H}, x_type, x);
-    const int64_t bytes = moe_ffn_forward_workspace_bytes(T, H, E, I, k);
+    const int64_t bytes = moe_forward_only_scratch(T, H, E, I, k, (int)dt(rows));
     const Tensor ws = empty({std::max<int64_t>(bytes, 256)}, at::kByte, x);
     // (it tells the observer about its launches itself, as do the two calls of a training step)
-    if (inside)
-      check(moe_routed_forward(router, bf(rows), bf(f.w.w1), bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(),
-                               (int)dt(x_type), ws.data_ptr(), ws.numel(), s),
-            "moe_routed_forward");
-    else check(moe_ffn_forward(rows.data_ptr(), (int)dt(rows), logits.data_ptr(), (int)dt(logits), (const float*)ptr(b),
-                          bf(f.w.w1), bf(f.w.w3), bf(f.w.w2), T, H, E, I, k, f.out.data_ptr(), (int)dt(x_type),
-                          ws.data_ptr(), ws.numel(), s),
-          "moe_ffn_forward");
+    check(moe_forward_only(inside ? &router : nullptr, rows.data_ptr(), (int)dt(rows), inside ? nullptr : logits.data_ptr(),
+                           inside ? MOE_DT_BF16 : (int)dt(logits), (const float*)ptr(b), bf(f.w.w1), bf(f.w.w3), bf(f.w.w2), T, H, E, I, k,
+                           f.out.data_ptr(), (int)dt(x_type), ws.data_ptr(), ws.numel(), s),
+          inside ? "moe_routed_forward" : "moe_ffn_forward");
     return f;
   }
   f.out = empty({T, H}, x_type, x);

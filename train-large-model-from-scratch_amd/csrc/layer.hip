@@ -44,7 +44,7 @@ int64_t order_bytes(int64_t T, int64_t E, int64_t k) {
   return place > general ? place : general;
 }
 
-Carve carve(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
+Carve carve(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, bool with_xp = true) {
   const int64_t R = T * k;
   Carve c;
   int64_t at = 0;
@@ -59,7 +59,7 @@ Carve carve(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
   c.offs = take((E + 1) * 4);
   c.pos_to_row = take(R * 4);
   c.row_to_pos = take(R * 4);
-  c.xp = take(R * H * 2);
+  c.xp = take(with_xp ? R * H * 2 : 0);
   c.act = take(R * I * 2);
   c.y = take(R * H * 2);
   c.dispatch = take(order_bytes(T, E, k));
@@ -72,15 +72,24 @@ bool sizes_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
          H <= 65536 && I <= 65536 && T <= ((int64_t)1 << 30) / k;
 }
 
+// Gate/up reads a token's row where it is, k times, and nobody else wants copies in expert order.
+bool forward_in_place(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int x_dtype) {
+  return !moe_few_ok(T, H, E, I, k, x_dtype) && x_dtype == MOE_DT_BF16 && moe_rows_from_ok(T, H);
+}
+
 }  // namespace
 
 extern "C" int64_t moe_ffn_forward_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k) {
   if (!sizes_ok(T, H, E, I, k)) return 0;
   return carve(T, H, E, I, k).total;
 }
+int64_t moe_forward_only_scratch(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int x_dtype) {
+  if (!sizes_ok(T, H, E, I, k)) return 0;
+  return carve(T, H, E, I, k, !forward_in_place(T, H, E, I, k, x_dtype)).total;
+}
 
-// The pass itself.  With `router` its product is part of it (see router.h), without it the logits are given.
-static int forward_only(const void* x, int x_dtype, const void* logits, int logits_dtype, const MoeRouter* router,
+// The pass itself.  With `router` its product is part of it (see router.h), without it the logits are given.  `room`: what the workspace has to have.
+static int forward_only(int64_t room, const void* x, int x_dtype, const void* logits, int logits_dtype, const MoeRouter* router,
                         const float* bias, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
                         int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   if (T < 0 || H <= 0 || E <= 0 || I <= 0 || k <= 0 || H % 8 != 0 || I % 8 != 0) return MOE_ERR_SHAPE;
@@ -104,8 +113,9 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   MOE_CHECK_PTR(w2);
   MOE_CHECK_PTR(out);
   MOE_CHECK_PTR(workspace);
-  const Carve c = carve(T, H, E, I, k);
-  if (workspace_bytes < c.total) return MOE_ERR_WORKSPACE;
+  const bool in_place = forward_in_place(T, H, E, I, k, x_dtype);
+  const Carve c = carve(T, H, E, I, k, !in_place);
+  if (workspace_bytes < room || workspace_bytes < c.total) return MOE_ERR_WORKSPACE;
   char* ws = (char*)workspace;
   const int64_t R = T * k;
   int32_t* ids = (int32_t*)(ws + c.ids);
@@ -131,8 +141,6 @@ static int forward_only(const void* x, int x_dtype, const void* logits, int logi
   }
   const bool few = moe_few_ok(T, H, E, I, k, x_dtype), place = !few && moe_place_ok(T, E, k);
   const bool selects = few && moe_gateup_few_selects(T, E, I, k);  // gate/up does the selection
-  // gate/up reads a token's row where it is, k times, and nobody else wants the copies in expert order
-  const bool in_place = !few && x_dtype == MOE_DT_BF16 && moe_rows_from_ok(T, H);
   uint16_t* rows = in_place ? nullptr : xp;
   const bool selected = router && !few_logits, at_once = place && !selected && moe_select_place_ok(logits, T, E, k);
   if (selected)
@@ -182,15 +190,15 @@ extern "C" int moe_ffn_forward(const void* x, int x_dtype, const void* logits, i
                                const float* bias, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
                                int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out,
                                int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
-  return forward_only(x, x_dtype, logits, logits_dtype, nullptr, bias, w1, w3, w2, T, H, E, I, k, out,
-                      out_dtype, workspace, workspace_bytes, stream);
+  return forward_only(moe_ffn_forward_workspace_bytes(T, H, E, I, k), x, x_dtype, logits, logits_dtype, nullptr, bias, w1, w3, w2, T, H, E, I, k,
+                      out, out_dtype, workspace, workspace_bytes, stream);
 }
 
-int moe_routed_forward(const MoeRouter& router, const uint16_t* x, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
-                       int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out, int out_dtype, void* workspace,
-                       int64_t workspace_bytes, void* stream) {
-  return forward_only(x, MOE_DT_BF16, nullptr, MOE_DT_BF16, &router, nullptr, w1, w3, w2, T, H, E, I, k, out, out_dtype,
-                      workspace, workspace_bytes, stream);
+int moe_forward_only(const MoeRouter* router, const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias,
+                     const uint16_t* w1, const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k,
+                     void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  return forward_only(0, x, x_dtype, logits, logits_dtype, router, bias, w1, w3, w2, T, H, E, I, k, out, out_dtype, workspace,
+                      workspace_bytes, stream);
 }
 
 int moe_router_logits(const uint16_t* x, const uint16_t* wr, int64_t T, int64_t H, int64_t E, uint16_t* logits,

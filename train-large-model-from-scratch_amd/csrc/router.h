@@ -17,9 +17,11 @@ bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k, int wr_dty
 // moe_ffn_forward, and moe_layer_forward (x: the bf16 rows), with the router's product part of it: sizes that moe_router_few_ok (x and
 // wr in bf16) or moe_router_select_ok takes, the latter alone in training.  moe_selected_layer_forward: with a `table` instead the
 // selection is done, ids and gates are there, and so are its counts; with neither it is moe_layer_forward.
-int moe_routed_forward(const MoeRouter& router, const uint16_t* x, const uint16_t* w1, const uint16_t* w3, const uint16_t* w2,
-                       int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, void* out, int out_dtype, void* workspace,
-                       int64_t workspace_bytes, void* stream);
+// moe_forward_only without a router is moe_ffn_forward, in a workspace without room for copies that are not made.
+int64_t moe_forward_only_scratch(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k, int x_dtype);
+int moe_forward_only(const MoeRouter* router, const void* x, int x_dtype, const void* logits, int logits_dtype, const float* bias,
+                     const uint16_t* w1, const uint16_t* w3, const uint16_t* w2, int64_t T, int64_t H, int64_t E, int64_t I, int64_t k,
+                     void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 // Without xp the experts read x where it is (then in bf16), for sizes that moe_layer_rows_from_ok takes; the backward pass is then
 // moe_in_place_layer_backward, which has x as xn.
 bool moe_layer_rows_from_ok(int64_t T, int64_t H, int64_t E, int64_t I, int64_t k);

@@ -341,8 +341,9 @@ int router_chains(int64_t T, int64_t H, int64_t E) {
 // training, 70 / 512 213.5 -> 211.8, 256.1 -> 255.0; 128, 1024 wide, forward 66.6 -> 66 to 70, 78.6 -> 76 to 81, training 200 -> 202, 223 -> 230.)
 bool moe_router_select_ok(int64_t T, int64_t H, int64_t E, int64_t k, int wr_dtype) {
   const bool long_rows = wr_dtype == MOE_DT_F32 && E > 64 && H > 1024 && T <= 1024;
+  if (router_chains(T, H, E) == 0) return false;
   const bool pays = E <= 16 ? T <= (H <= 1024 ? 12288 : 8192) : T <= TOKENS * moe_compute_units() && E * H <= 128 * 1024 && !long_rows;
-  return pays && router_chains(T, H, E) != 0 && k > 0 && k <= E && k <= MOE_MAX_TOPK;
+  return pays && k > 0 && k <= E && k <= MOE_MAX_TOPK;
 }
 
 int moe_router_select(const MoeRouter& r, int64_t T, int64_t H, int64_t E, int64_t k, int32_t* ids, float* gates, void* table,
