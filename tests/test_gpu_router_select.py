@@ -1,5 +1,8 @@
 """The router product and the selection in one launch: logits of the bits that the library's product has, the selection that
 `moe_ffn` makes on them, and the same rest of the layer; at the edges of the sizes that it takes."""
+import math
+import random
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -85,6 +88,47 @@ def test_long_rows_of_fp32_weights(pkg, lib, T, E, k, H, w_type, taken):
     want = F.linear(x.to(BF16), wr.to(BF16))
     assert torch.equal(lg, want)
     assert torch.equal(out, pkg.moe_ffn(x, want, *ws, k))
+
+
+def edges():
+    """Sizes on both sides of the lines where the order of a logit's sum changes, or the launch that makes it."""
+    few = [(T, E, H) for T in (65, 256, 257, 2048, 2049, 3200, 3201) for E in (2, 12, 13, 16)
+           for H in (64, 120, 128, 312, 320, 504, 512, 1016, 1024, 2048)]
+    few += [(T, E, H) for T in (8192, 8193, 12288, 12289) for E in (2, 16) for H in (1016, 1024, 1032)]
+    many = [(T, E, H) for E in (17, 31, 32, 48, 49, 64, 65, 80, 112, 113, 128) for H in (64, 1024, 1032, 1536, 2048)
+            for T in {t + d for n in (512, 1024) for t in (16 * (n // -(-E // 16)),) for d in (0, 1)} | {65, 4096, 4097}]
+    return few + many
+
+
+def test_bits_at_the_lines_and_over_the_ranges(pkg, lib):
+    """Whichever launch makes a logit, it has the bits that nn.Linear gives it: at every line of the rule, and for 300 sizes drawn."""
+    rng = random.Random(7)
+    log = lambda lo, hi: int(math.exp(rng.uniform(math.log(lo), math.log(hi))))
+    sizes = edges() + [(log(65, 12288), rng.choice([log(2, 16), log(32, 128)]), log(8, 256) * 8) for _ in range(300)]
+    names, taken = [], 0
+
+    class Obs:
+        before = staticmethod(names.append)
+        after = staticmethod(lambda name: None)
+
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x_all = torch.randn(12289 * 2048, generator=g, device="cuda").to(BF16)
+    wr_all = (torch.randn(128 * 2048, generator=g, device="cuda") * 0.05).to(BF16)
+    w_all = torch.zeros(128 * 2048 * 8, dtype=BF16, device="cuda")
+    for i, (T, E, H) in enumerate(sizes):
+        if i % 100 == 0:
+            print("router select, sizes from", i, "of", len(sizes), flush=True)
+        x, wr = x_all[:T * H].view(T, H), wr_all[:E * H].view(E, H)
+        w1, w2 = w_all[:E * H * 8].view(E, 8, H), w_all[:E * H * 8].view(E, H, 8)
+        names.clear()
+        lib.observer = Obs()
+        try:
+            _, lg = pkg.routed_moe(x, wr, w1, w1, w2, min(E, 2))
+        finally:
+            lib.observer = None
+        taken += "moe_router_select" in names
+        assert torch.equal(lg, F.linear(x, wr)), (T, E, H)
+    assert 3 * taken >= len(sizes)
 
 
 def test_values_that_are_not_finite(pkg):

@@ -304,8 +304,10 @@ int launch(const RouterArgs& a, hipStream_t s) {
   return moe_launch_status();
 }
 
-// Chains that the library's product sums a logit in (0: not known).  Found by comparing bits, 900000 sizes: of 65 to 30000 tokens, 1 to 128
-// experts, widths of 64 to 2048 in steps of 8, all that this names agree in every logit.  (Wider ones have more kinds of sums.)
+// Chains that the library's product sums a logit in (0: not known): what the matrix library that PyTorch 2.10 for ROCm 7 calls does on 256 compute
+// units, found by comparing results.  Sizes on both sides of every line here, and drawn ones, are compared to the bit in tests/test_gpu_router_select.py; another
+// build of that library may sum in another order, and then a logit made here and nn.Linear's may differ in their last bit.  (Wider ones than MAX_H have more kinds
+// of sums.)
 int router_chains(int64_t T, int64_t H, int64_t E) {
   if (T <= 64 || H < 64 || H > MAX_H || H % 8 != 0 || E < 2 || E > MAX_E) return 0;
   if (E <= 16) {
@@ -317,6 +319,7 @@ int router_chains(int64_t T, int64_t H, int64_t E) {
   if (E < 32 || T > 30000) return 0;
   if (H <= 1024) return 1;
   const int64_t groups = (E + 15) / 16, tiles = (T + 15) / 16 * groups;
+  if (tiles == 511) return 0;  // (one short of two full rounds: not four chains)
   if (tiles <= 512) return 4;
   if (tiles > 1024) return 1;
   return groups % 2 ? 0 : E == 64 ? 4 : 1;
